@@ -36,11 +36,8 @@ from inference_gateway_amd.engine.models.batch import ForwardBatch
 PAGE = 16
 DEVICE = "cuda"
 BIVATAR = "bivatar-4k"
+MIXTRAL = "mixtral-8x7b"
 LLAMAS = ("llama-3-8b", "llama-3.1-8b", "phi-3-medium")
-# random router logits are so close that rounding picks the experts, and an
-# error of one bf16 step before the router would be compared as a large one
-# behind it.  A router that has learned something prefers its experts clearly.
-ROUTER_GAIN = 4.0
 
 
 def _step(name, model, layers, prompts=0, rows=0, prefix=0, decodes=0,
@@ -72,10 +69,10 @@ def listed():
         _step("chunk-and-decode", "llama-3.1-8b", 4, prompts=1, rows=2000,
               prefix=6000, decodes=33, context=3000, ragged=90),
         # a few users of a mixture-of-experts model
-        _step("moe-decode-5", "mixtral-8x7b", 1, decodes=5, context=1500,
+        _step("moe-decode-5", MIXTRAL, 1, decodes=5, context=1500,
               ragged=50),
         # its prompts
-        _step("moe-prefill-3x700", "mixtral-8x7b", 1, prompts=3, rows=700,
+        _step("moe-prefill-3x700", MIXTRAL, 1, prompts=3, rows=700,
               ragged=20),
         # per-layer design: prompts beyond its window
         _step("layered-prefill-2x3000", BIVATAR, 4, prompts=2, rows=3000,
@@ -109,7 +106,7 @@ def draw(rng):
         return _step(None, BIVATAR, 4, decodes=_spread(rng, 1, 128),
                      context=_spread(rng, 100, 4000),
                      ragged=rng.randint(0, 95))
-    model, layers = (("mixtral-8x7b", 1) if rng.random() < 0.2
+    model, layers = ((MIXTRAL, 1) if rng.random() < 0.2
                      else (rng.choice(LLAMAS), 4))
     longest = min(16000, MODEL_PRESETS[model].max_position)
     if what == "decode":
@@ -239,6 +236,22 @@ def _batch(case, tokens, table, with_sequences):
     return fb
 
 
+def _preferring(embed, router):
+    """Embedding and router of a model whose tokens prefer their experts.
+    Random weights leave a mixture-of-experts model without a preference:
+    router logits lie so close that rounding picks the experts, and one bf16
+    step before the router would be compared as another expert's output.
+    Here a token's row of about unit width points to its two experts, which
+    get about 0.7 and 0.3 of it, as in a trained model."""
+    token = torch.arange(embed.shape[0], device=embed.device)
+    E = router.shape[0]
+    first = token % E
+    second = (first + 1 + token // E % (E - 1)) % E
+    to = F.normalize(router.float(), dim=1)
+    embed = 50.0 * embed.float() + 60.0 * to[first] + 48.0 * to[second]
+    return embed.to(torch.bfloat16), (0.1 * router.float()).to(torch.bfloat16)
+
+
 def prepare(case, seed):
     if case["kind"] == "sample":
         return _prepare_sample(case, seed)
@@ -250,9 +263,12 @@ def prepare(case, seed):
         max_model_len=max(p + n for p, n in seqs) + PAGE,
         use_hip_graphs=False, enforce_eager=True), device="cuda:0")
     model, caches = engine.model, engine.kv_caches
-    for name, p in model.named_parameters():
-        if name.endswith("router.weight"):
-            p.mul_(ROUTER_GAIN)
+    if case["model"] == MIXTRAL:
+        named = dict(model.named_parameters())
+        router = [n for n in named if n.endswith("router.weight")]
+        for n, w in zip(["embed"] + router, _preferring(
+                named["embed"], *(named[n] for n in router))):
+            named[n].copy_(w)
     for t in _tensors(caches):
         _fill(t, g)
     fb = _batch(case, tokens, table, getattr(model, "needs_seq_meta", False))
@@ -396,7 +412,7 @@ def tolerance(case):
         # lies on an edge
         return {"differ": 0.01}
     # bf16 activations: measured 0.015 to 0.020 against 64 bits after four
-    # Llama layers and 0.006 after four of the layers with an fp32 residual;
+    # Llama layers, 0.006 after four of the layers with an fp32 residual;
     # two correct implementations lie as far apart
     if case["model"] == BIVATAR:
         return {"rel": 0.02, "max": 0.5}
@@ -506,7 +522,11 @@ def _exact_llama(cfg, case, tokens, table, g):
                    cfg.num_kv_heads)
     pos, slots, _, cu, _ = _rows(case, table)
     inv = _llama_frequencies(cfg)
-    x = _weight((cfg.vocab_size, D), "embed")[tokens]
+    x = _weight((cfg.vocab_size, D), "embed")
+    if cfg.num_experts:
+        x, router = (w.double() for w in _preferring(
+            x, _weight((cfg.num_experts, D), "l0.router")))
+    x = x[tokens]
     caches = []
     for i in range(cfg.num_layers):
         caches += [_new_cache(case, g, G, PAGE, hd),
@@ -535,7 +555,6 @@ def _exact_llama(cfg, case, tokens, table, g):
         if not cfg.num_experts:
             x = x + swiglu(h, f"l{i}")
             continue
-        router = _weight((cfg.num_experts, D), f"l{i}.router") * ROUTER_GAIN
         w, chosen = (h @ router.t()).topk(cfg.num_experts_per_tok, -1)
         w = w.softmax(-1)
         for e in range(cfg.num_experts):
