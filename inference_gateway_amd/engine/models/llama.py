@@ -95,8 +95,7 @@ class LlamaAttention(nn.Module):
             if fb.prefix_lens is not None:
                 # prefix-cache hit in the batch: q rows are suffixes;
                 # cached prefix + the just-appended suffix K/V are read
-                # back from the paged cache (ops/csrc/flash_prefill.hip,
-                # flash_prefill_paged_kernel)
+                # back from the paged cache (ops/csrc/flash_prefill.hip)
                 o = ops.flash_prefill_paged(
                     qv[:P], kc, vc, fb.block_table,
                     fb.prefix_lens, fb.cu_seqlens, fb.seq_lens, self.scale)

@@ -166,12 +166,7 @@ def flash_prefill(q, k, v, cu_seqlens, seq_lens, scale: float):
     if q.is_cuda:
         _require_kernels()
         out = torch.empty_like(q)
-        tile_seq, tile_off = torch_ref.make_prefill_tiles(
-            seq_lens, tile_m=64, device=q.device
-        )
-        _kernels.flash_prefill(
-            out, q, k, v, cu_seqlens, tile_seq, tile_off, scale
-        )
+        _kernels.flash_prefill(out, q, k, v, cu_seqlens, seq_lens, scale)
         return out
     return torch_ref.flash_prefill_ref(q, k, v, cu_seqlens, scale)
 
@@ -186,12 +181,9 @@ def flash_prefill_paged(q, kcache, vcache, block_table, prefix_lens,
     if q.is_cuda:
         _require_kernels()
         out = torch.empty_like(q)
-        tile_seq, tile_off = torch_ref.make_prefill_tiles(
-            seq_lens, tile_m=64, device=q.device
-        )
         _kernels.flash_prefill_paged(
             out, q, kcache, vcache, block_table, prefix_lens, cu_seqlens,
-            tile_seq, tile_off, scale
+            seq_lens, scale
         )
         return out
     return torch_ref.flash_prefill_paged_ref(

@@ -23,13 +23,12 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
                        double scale);
 void flash_prefill(torch::Tensor out, torch::Tensor q, torch::Tensor k,
                    torch::Tensor v, torch::Tensor cu_seqlens,
-                   torch::Tensor tile_seq, torch::Tensor tile_off,
-                   double scale);
+                   std::vector<int64_t> seq_lens, double scale);
 void flash_prefill_paged(torch::Tensor out, torch::Tensor q,
                          torch::Tensor kcache, torch::Tensor vcache,
                          torch::Tensor block_table, torch::Tensor prefix_lens,
-                         torch::Tensor cu_seqlens, torch::Tensor tile_seq,
-                         torch::Tensor tile_off, double scale);
+                         torch::Tensor cu_seqlens,
+                         std::vector<int64_t> seq_lens, double scale);
 void sample(torch::Tensor out, torch::Tensor logits, torch::Tensor temperature,
             torch::Tensor top_k, torch::Tensor top_p, torch::Tensor uniforms);
 void silu_mul(torch::Tensor out, torch::Tensor gate_up);

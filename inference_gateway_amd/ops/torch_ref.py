@@ -185,7 +185,7 @@ def flash_prefill_paged_ref(q, kcache, vcache, block_table, prefix_lens,
 
 
 def make_prefill_tiles(seq_lens, tile_m: int = 64, device="cpu"):
-    """Host-side tile map for flash_prefill: (tile_seq, tile_off) int32."""
+    """Host-side tile map of prompt portions: (tile_seq, tile_off) int32."""
     tseq, toff = [], []
     for i, L in enumerate(seq_lens):
         for off in range(0, int(L), tile_m):

@@ -326,6 +326,85 @@ def test_flash_prefill_paged_vs_ref(chunks):
                                atol=3e-2, rtol=3e-2)
 
 
+def _attention_bound(v):
+    """|error| <= bound + |value| 2^-8: probabilities rounded to bf16 move
+    the weighted mean by at most 2^-9 of the largest value, the result and
+    the reference's are rounded once each; the rest (32-bit sums and the
+    exponential) is far below the other half of the bound."""
+    return 2.0 ** -8 * float(v.float().abs().max())
+
+
+@pytest.mark.parametrize("seq_lens,nq,nkv,gain,scale", [
+    # rows at the edges of the 128-row tiles and the 64-key tiles
+    ([127, 128, 129], 8, 2, 1.0, 128 ** -0.5),
+    ([1, 32, 33, 191, 192, 193, 257], 8, 8, 1.0, 128 ** -0.5),
+    # heads that do not divide over the chiplets; a wide group
+    ([130, 5], 12, 4, 1.0, 128 ** -0.5),
+    ([70, 300], 40, 10, 1.0, 128 ** -0.5),
+    ([65], 9, 1, 1.0, 128 ** -0.5),
+    # more sequences than one step of the tile search takes
+    ([3, 1, 2] * 30, 8, 1, 1.0, 128 ** -0.5),
+    # scores that outgrow the running maximum by far; other signs of scale
+    ([400], 8, 2, 12.0, 128 ** -0.5),
+    ([200], 8, 2, 3.0, -0.125),
+    ([100], 8, 2, 1.0, 0.0),
+])
+def test_flash_prefill_edges(seq_lens, nq, nkv, gain, scale):
+    g = torch.Generator().manual_seed(sum(seq_lens))
+    T, hd = sum(seq_lens), 128
+    # views into one fused projection, as the model passes them
+    qkv = (torch.randn(T, (nq + 2 * nkv) * hd, generator=g) * gain).to(
+        torch.bfloat16)
+    cu = torch.tensor([0] + torch.tensor(seq_lens).cumsum(0).tolist(),
+                      dtype=torch.int32)
+
+    def split(x):
+        q, k, v = x.split([nq * hd, nkv * hd, nkv * hd], -1)
+        return (q.view(T, nq, hd), k.view(T, nkv, hd), v.view(T, nkv, hd))
+
+    q, k, v = split(qkv)
+    ref = torch_ref.flash_prefill_ref(q, k, v, cu, scale)
+    out = ops.flash_prefill(*split(qkv.cuda()), cu.cuda(), seq_lens, scale)
+    torch.testing.assert_close(out.float().cpu(), ref.float(),
+                               atol=_attention_bound(v), rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("chunks,nq,nkv", [
+    # prefixes and rows at page, key-tile and row-tile edges
+    ([(15, 1), (16, 1), (17, 128), (63, 129)], 8, 2),
+    ([(64, 64), (0, 127), (129, 3)], 16, 16),
+    ([(200, 130)], 12, 4),
+])
+def test_flash_prefill_paged_edges(chunks, nq, nkv):
+    g = torch.Generator().manual_seed(len(chunks))
+    hd, bs = 128, 16
+    need = [-(-(p + n) // bs) for p, n in chunks]
+    order = torch.randperm(sum(need), generator=g).to(torch.int32) + 1
+    kc, vc = (torch.randn(sum(need) + 1, nkv, bs, hd, generator=g).to(
+        torch.bfloat16) for _ in range(2))
+    # slots past a sequence's end must not be read
+    bt = torch.zeros(len(chunks), max(need) + 1, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        bt[i, :n] = order[at:at + n]
+        at += n
+        used = (sum(chunks[i]) - 1) % bs + 1
+        kc[bt[i, n - 1], :, used:] = float("nan")
+        vc[bt[i, n - 1], :, used:] = float("nan")
+    rows = [n for _, n in chunks]
+    q = torch.randn(sum(rows), nq, hd, generator=g).to(torch.bfloat16)
+    cu = torch.tensor([0] + torch.tensor(rows).cumsum(0).tolist(),
+                      dtype=torch.int32)
+    prefix = torch.tensor([p for p, _ in chunks], dtype=torch.int32)
+    args = (q, kc, vc, bt, prefix, cu)
+    ref = torch_ref.flash_prefill_paged_ref(*args, hd ** -0.5)
+    out = ops.flash_prefill_paged(*(t.cuda() for t in args), rows,
+                                  hd ** -0.5)
+    torch.testing.assert_close(out.float().cpu(), ref.float(),
+                               atol=_attention_bound(vc.nan_to_num()),
+                               rtol=2.0 ** -8)
+
+
 def test_zz_chunked_prefill_engine_matches_unchunked():
     # placed in this (alphabetically last) file, and named to sort last,
     # so the driver's -x run covers everything else first
