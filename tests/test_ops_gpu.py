@@ -405,6 +405,97 @@ def test_flash_prefill_paged_edges(chunks, nq, nkv):
                                rtol=2.0 ** -8)
 
 
+def _check_draw(row, temp, k, p, u, got):
+    """The token drawn for one row, against 64 bits: it is kept, and u lies
+    in its share of the kept mass.  Sums of 32-bit exponentials are good to
+    about 1e-6 of the total; 1e-5 is allowed."""
+    V = row.numel()
+    assert 0 <= got < V
+    x = row.double()
+    if temp <= 0:
+        assert got == int((x == x.max()).nonzero()[0])
+        return
+    w = torch.exp((x - x.max()) / temp)
+    if 0 < k < V:
+        assert x[got] >= x.sort(descending=True).values[k - 1]
+    if p < 1:
+        assert w[x > x[got]].sum() < (p + 1e-5) * w.sum()
+    tau = -float("inf")
+    if 0 < k < V:
+        tau = float(x.sort(descending=True).values[k - 1])
+    if p < 1:
+        v, i = x.sort(descending=True)
+        cum = w[i].cumsum(0)
+        tau_p = float(v[min(V - 1, int((cum < p * w.sum()).sum()))])
+        if tau_p > tau:
+            # a mass within rounding of p keeps one value more or less
+            edge = (cum / w.sum() - p).abs().min() < 1e-5
+            if edge:
+                return
+            tau = tau_p
+    w = torch.where(x >= tau, w, torch.zeros_like(w))
+    cdf = w.cumsum(0) / w.sum()
+    assert w[got] > 0
+    assert cdf[got] >= u - 1e-5
+    assert got == 0 or cdf[got - 1] <= u + 1e-5
+
+
+@pytest.mark.parametrize("V", [
+    1, 7, 8, 9, 4095, 4096, 4097,          # chunks and their tails
+    32767, 32768, 32769,                   # 8 chunks, the first of 16
+    65536, 65537, 128256, 131072, 131073,  # 16 and 32 chunks
+    163840, 163841])                       # 40 chunks; the kernel beyond
+def test_sample_bf16_sizes(V):
+    g = torch.Generator().manual_seed(V)
+    settings = [(0.8, 50, 0.95), (0.0, 0, 1.0), (1.0, 0, 0.9), (0.7, 40, 1.0),
+                (1.0, 0, 1.0), (1.3, V, 0.3), (0.5, 1, 0.5)]
+    B = len(settings)
+    logits = (torch.randn(B, V, generator=g) * 1.3).to(torch.bfloat16)
+    temp, k, p = (torch.tensor(c) for c in zip(*settings))
+    u = torch.rand(B, generator=g)
+    out = ops.sample(logits.cuda(), temp.float().cuda(),
+                     k.to(torch.int32).cuda(), p.float().cuda(), u.cuda())
+    for i, got in enumerate(out.tolist()):
+        _check_draw(logits[i], *settings[i], float(u[i]), got)
+
+
+@pytest.mark.parametrize("kind", ["ties", "zeros", "negative", "masked",
+                                  "wide", "one", "tiny"])
+def test_sample_bf16_values(kind):
+    """Logits whose thresholds lie outside the first windows or on values
+    that compare equal."""
+    g = torch.Generator().manual_seed(len(kind))
+    V, B = 5000, 8
+    x = torch.randn(B, V, generator=g)
+    if kind == "ties":
+        x = x.round()
+    elif kind == "zeros":      # both zeros, nothing above
+        x = -x.abs() * (torch.rand(B, V, generator=g) < 0.5)
+    elif kind == "negative":   # the maximum is far below zero
+        x = x - 40
+    elif kind == "masked":
+        x = x.masked_fill(torch.rand(B, V, generator=g) < 0.999,
+                          -float("inf"))
+        x[:, 77] = 0.5
+    elif kind == "wide":       # spread over all exponents
+        x = x * torch.exp(torch.randn(B, V, generator=g) * 20)
+        x = x.clamp(-1e4, 20)
+    elif kind == "one":
+        x[:, 4321] = 300.0
+    elif kind == "tiny":       # nearly flat, all exponents below one
+        x = x * 1e-3
+    logits = x.to(torch.bfloat16)
+    settings = [(1.0, 3000, 1.0), (1.0, 0, 0.99), (2.0, 4000, 0.97),
+                (0.8, 50, 0.95), (0.0, 0, 1.0), (1.0, 0, 1.0),
+                (0.3, 4999, 0.999), (1.0, 2, 1.0)]
+    temp, k, p = (torch.tensor(c) for c in zip(*settings))
+    u = torch.tensor([0.5, 0.999999, 1e-6, 0.3, 0.5, 0.7, 0.2, 0.9])
+    out = ops.sample(logits.cuda(), temp.float().cuda(),
+                     k.to(torch.int32).cuda(), p.float().cuda(), u.cuda())
+    for i, got in enumerate(out.tolist()):
+        _check_draw(logits[i], *settings[i], float(u[i]), got)
+
+
 def test_zz_chunked_prefill_engine_matches_unchunked():
     # placed in this (alphabetically last) file, and named to sort last,
     # so the driver's -x run covers everything else first
