@@ -20,7 +20,12 @@
 //   * V pass: 16 lanes x 8 contiguous dims (b128 reads), 4 token subgroups,
 //     partials folded with 2 shfl_xor at the end;
 //   * waves stripe over cache blocks and merge via LDS once at the end
-//     (flash-decoding style rescale).
+//     (flash-decoding style rescale);
+//   * a sequence's pages are split over up to nsplit workgroups when
+//     sequences x key/value heads alone do not fill the chip.  The split is
+//     by the sequence's own length (read on the device, so a captured launch
+//     stays right as contexts grow); the parts' unnormalised sums (fp32) are
+//     merged by a second kernel.
 //
 // Wavefront-64 throughout; no CUDA-isms, no Triton.
 
@@ -50,6 +55,19 @@ DEVINLINE float token_reduce_sum(float x) {
   return x;
 }
 
+// How a sequence of ctx tokens is cut for nsplit workgroups: `count` parts of
+// `blocks` pages, a part no shorter than DECODE_MIN_BLOCKS pages.
+constexpr int DECODE_MIN_BLOCKS = 4;
+struct DecodeSplit {
+  int blocks, count;
+  DEVINLINE DecodeSplit(int ctx, int nsplit) {
+    const int n = (ctx + 15) / 16;
+    blocks = max((n + nsplit - 1) / nsplit, DECODE_MIN_BLOCKS);
+    if (nsplit == 1) blocks = max(n, 1);
+    count = max((n + blocks - 1) / blocks, 1);
+  }
+};
+
 template <int HD, int G, int NWAVES>
 __global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
     uint16_t* __restrict__ out,          // [B, NQ, HD]
@@ -58,7 +76,10 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
     const uint16_t* __restrict__ vcache, // [NB, NKV, BS, HD]
     const int32_t* __restrict__ block_table, // [B, max_blocks]
     const int32_t* __restrict__ ctx_lens,    // [B]
-    int max_blocks, int nkv, float scale, int q_rs) {
+    int max_blocks, int nkv, float scale, int q_rs,
+    float* __restrict__ part_o,   // [B, NQ, nsplit, HD] when nsplit > 1
+    float* __restrict__ part_ml,  // [B, NQ, nsplit, 2]: maximum, sum
+    int nsplit) {
   // q_rs: q row stride in elements (q may be a view into the fused QKV
   // GEMM output — no .contiguous() copy on the decode hot path)
   constexpr int BS = 16;  // tokens per cache block
@@ -66,11 +87,15 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
   const int seq = blockIdx.y;
   const int nq = nkv * G;
   const int ctx = ctx_lens[seq];
-  const int nblocks = (ctx + BS - 1) / BS;
+  const int split = blockIdx.z;
+  const DecodeSplit part(ctx, nsplit);
+  if (split >= part.count) return;
+  const int block0 = split * part.blocks;
+  const int nblocks = min((ctx + BS - 1) / BS, block0 + part.blocks);
 
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE_SIZE - 1);
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
   __shared__ uint16_t q_lds[G][HD];
   __shared__ float m_lds[NWAVES][G];
@@ -107,15 +132,27 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
   // raw (unconverted) K tile registers for the current block
   ushort8 kraw[4];
 
+  // page numbers of this wave's next 64 pages, one per lane: a K address
+  // does not wait for a table entry, and its base is in scalar registers
+  const int b0 = block0 + wave;
+  int ids = 0;
+  auto load_ids = [&](int b) {
+    const int i = b + lane * NWAVES;
+    ids = i < nblocks ? bt_row[i] : 0;
+  };
+  auto page_of = [&](int b) {
+    return (int64_t)__builtin_amdgcn_readlane(ids, ((b - b0) / NWAVES) & 63);
+  };
+  load_ids(b0);
+
   auto load_k = [&](int b, ushort8* dst) {
-    const uint16_t* kp = kcache + ((int64_t)bt_row[b] * nkv) * BS * HD +
-                         head_off + tok * HD + seg;
+    const uint16_t* kp = kcache + page_of(b) * nkv * BS * HD + head_off +
+                         (tok * HD + seg);
 #pragma unroll
     for (int c = 0; c < 4; ++c)
       dst[c] = *reinterpret_cast<const ushort8*>(kp + c * 8);
   };
 
-  const int b0 = wave;
   if (b0 < nblocks) load_k(b0, kraw);
 
   for (int b = b0; b < nblocks; b += NWAVES) {
@@ -154,8 +191,8 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
     //      softmax + V-accumulate phase of flight time ----
     const int tlimit = min(BS, ctx - b * BS);
     ushort8 vraw[4];
-    const uint16_t* vp = vcache + ((int64_t)bt_row[b] * nkv) * BS * HD +
-                         head_off + vlane * 8;
+    const uint16_t* vp =
+        vcache + page_of(b) * nkv * BS * HD + head_off + vlane * 8;
     if (tlimit == BS) {
 #pragma unroll
       for (int t4 = 0; t4 < 4; ++t4)
@@ -168,7 +205,10 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
           vraw[t4] = *reinterpret_cast<const ushort8*>(
               vp + (vtok + 4 * t4) * HD);
     }
-    if (b + NWAVES < nblocks) load_k(b + NWAVES, kraw);
+    if (b + NWAVES < nblocks) {
+      if ((((b - b0) / NWAVES + 1) & 63) == 0) load_ids(b + NWAVES);
+      load_k(b + NWAVES, kraw);
+    }
 
     // ---- finish scores: pairwise dot reduce + mask ----
     const bool valid = (b * BS + tok) < ctx;
@@ -270,8 +310,65 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
       L = fmaf(f, l_lds[w][j], L);
       o = fmaf(f, acc_lds[w][j][d], o);
     }
-    out[((int64_t)seq * nq + kvh * G + j) * HD + d] = f32_to_bf16(o / L);
+    const int64_t head = (int64_t)seq * nq + kvh * G + j;
+    if (part.count == 1) {
+      out[head * HD + d] = f32_to_bf16(o / L);
+    } else {
+      part_o[(head * nsplit + split) * HD + d] = o;
+      if (d == 0) {
+        part_ml[(head * nsplit + split) * 2] = M;
+        part_ml[(head * nsplit + split) * 2 + 1] = L;
+      }
+    }
   }
+}
+
+// Merges the parts of every (sequence, head) that has more than one: one
+// workgroup of HD threads each.  The threads first weigh the parts side by
+// side (a loop over them would wait for memory at every step), then each sums
+// one dim over the parts, 8 loads in flight.
+template <int HD>
+__global__ __launch_bounds__(HD) void paged_attn_merge_kernel(
+    uint16_t* __restrict__ out, const float* __restrict__ part_o,
+    const float* __restrict__ part_ml, const int32_t* __restrict__ ctx_lens,
+    int nq, int nsplit) {
+  constexpr int NW = HD / WAVE_SIZE;
+  __shared__ float red[NW];
+  __shared__ float weight[HD];
+  const int seq = blockIdx.y, tid = threadIdx.x;
+  const DecodeSplit part(ctx_lens[seq], nsplit);
+  if (part.count == 1) return;
+  const int64_t head = (int64_t)seq * nq + blockIdx.x;
+  const float2* ml = reinterpret_cast<const float2*>(part_ml) + head * nsplit;
+  const float* po = part_o + head * nsplit * HD + tid;
+  float M = -INFINITY;
+  for (int s = tid; s < part.count; s += HD) M = fmaxf(M, ml[s].x);
+  M = wave_reduce_max(M);
+  if ((tid & 63) == 0) red[tid >> 6] = M;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NW; ++w) M = fmaxf(M, red[w]);
+  float L = 0.0f, o = 0.0f;
+  for (int s0 = 0; s0 < part.count; s0 += HD) {
+    const int n = min(HD, part.count - s0);
+    __syncthreads();   // weight (and red) were read by everybody
+    float l = 0.0f;
+    if (tid < n) {
+      const float2 v = ml[s0 + tid];
+      const float f = v.x == -INFINITY ? 0.0f : __expf(v.x - M);
+      weight[tid] = f;
+      l = f * v.y;
+    }
+    l = wave_reduce_sum(l);
+    if ((tid & 63) == 0) red[tid >> 6] = l;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < NW; ++w) L += red[w];
+#pragma unroll 8
+    for (int s = 0; s < n; ++s)
+      o = fmaf(weight[s], po[(int64_t)(s0 + s) * HD], o);
+  }
+  out[head * HD + tid] = f32_to_bf16(o / L);
 }
 
 template <int G>
@@ -283,18 +380,46 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
                           hipStream_t stream) {
   const int B = q.size(0);
   const int nkv = kcache.size(1);
-  constexpr int NWAVES = 4;
-  dim3 grid(nkv, B);
-  hipLaunchKernelGGL((paged_attn_decode_kernel<128, G, NWAVES>), grid,
-                     dim3(NWAVES * WAVE_SIZE), 0, stream,
+  constexpr int NWAVES = 4, HD = 128;
+  const int nq = q.size(1);
+  const int max_blocks = block_table.size(1);
+  // The chip holds 1024 of these workgroups (four per compute unit, by their
+  // registers).  Where sequences x heads are fewer, aim for two rounds, so
+  // that parts of ragged lengths even out; a part has at least a page per
+  // wave.  Measured with 8 heads, whole against split: 1 sequence of 700
+  // tokens 25.8 and 9.8 us, 1 of 8000 268 and 22, 61 of 200 to 4000 177 and
+  // 137; with 1024 workgroups it only adds the merge (128 of 100 to 2000
+  // tokens: 155 and 160).
+  const int whole = std::max(1, B * nkv);
+  const int nsplit =
+      whole >= 1024
+          ? 1
+          : std::max(1, std::min(2048 / whole,
+                                 (max_blocks + DECODE_MIN_BLOCKS - 1) /
+                                     DECODE_MIN_BLOCKS));
+  torch::Tensor part;
+  float *part_o = nullptr, *part_ml = nullptr;
+  if (nsplit > 1) {
+    const int64_t n = (int64_t)B * nq * nsplit;
+    part = torch::empty({n * (HD + 2)}, q.options().dtype(torch::kFloat32));
+    part_o = part.data_ptr<float>();
+    part_ml = part_o + n * HD;
+  }
+  hipLaunchKernelGGL((paged_attn_decode_kernel<HD, G, NWAVES>),
+                     dim3(nkv, B, nsplit), dim3(NWAVES * WAVE_SIZE), 0, stream,
                      (uint16_t*)out.data_ptr(), (const uint16_t*)q.data_ptr(),
                      (const uint16_t*)kcache.data_ptr(),
                      (const uint16_t*)vcache.data_ptr(),
                      (const int32_t*)block_table.data_ptr(),
-                     (const int32_t*)ctx_lens.data_ptr(),
-                     (int)block_table.size(1), nkv, scale,
-                     (int)q.stride(0));
+                     (const int32_t*)ctx_lens.data_ptr(), max_blocks, nkv,
+                     scale, (int)q.stride(0), part_o, part_ml, nsplit);
   HIP_CHECK_KERNEL();
+  if (nsplit > 1) {
+    hipLaunchKernelGGL((paged_attn_merge_kernel<HD>), dim3(nq, B), dim3(HD), 0,
+                       stream, (uint16_t*)out.data_ptr(), part_o, part_ml,
+                       (const int32_t*)ctx_lens.data_ptr(), nq, nsplit);
+    HIP_CHECK_KERNEL();
+  }
 }
 
 void paged_attn_decode(torch::Tensor out, torch::Tensor q,

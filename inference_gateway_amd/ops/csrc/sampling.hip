@@ -597,8 +597,9 @@ __global__ __launch_bounds__(BLOCK) void sample_bf16_kernel(
 // about as long again, mostly for the exponentials of Z; one row per compute
 // unit at a time.  Each of the four passes of sample_bf16_kernel reads the row
 // again and updates LDS bins for all elements: 1024 rows of 128256 took 945
-// us, here 198 us (temperature, top-k and top-p on most rows; greedy rows 62).  Rows of more than 8 * 512 * 40 logits keep that
-// kernel: they would not leave registers for the arithmetic.
+// us, here 198 us (temperature, top-k and top-p on most rows; greedy rows
+// 62).  Rows of more than 8 * 512 * 40 logits keep that kernel: they would
+// not leave registers for the arithmetic.
 // ---------------------------------------------------------------------------
 constexpr int SR_THREADS = 512;
 constexpr int SR_WAVES = SR_THREADS / WAVE_SIZE;

@@ -98,6 +98,38 @@ def test_paged_attn_decode(G):
     _assert_close_bf16(out, ref)
 
 
+@pytest.mark.parametrize("nq,nkv,ctx", [
+    (4, 1, [1, 15, 16, 17, 63, 64, 65]),   # parts of four pages, and less
+    (8, 8, [4096 + 7]),                    # a part per four pages
+    (8, 1, [9000, 1]),                     # more parts than merge threads
+    (16, 4, [700, 2000, 64, 65] * 3),
+    (64, 8, [1000, 129] * 40),             # parts longer than four pages
+    (32, 8, [40] * 256),                   # not split
+])
+def test_paged_attn_decode_split(nq, nkv, ctx):
+    """Contexts cut over several workgroups; the probabilities and sums are
+    32 bits, so only the rounding of the result (and of the reference's) to
+    bf16 is allowed, and the exponential's 2^-20 or so of the values."""
+    g = torch.Generator().manual_seed(nq + len(ctx))
+    hd, bs, B = 128, 16, len(ctx)
+    need = [-(-c // bs) for c in ctx]
+    kc, vc = (torch.randn(sum(need) + 1, nkv, bs, hd, generator=g).to(
+        torch.bfloat16) for _ in range(2))
+    order = torch.randperm(sum(need), generator=g).to(torch.int32) + 1
+    bt = torch.zeros(B, max(need) + 3, dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    q = torch.randn(B, nq, hd, generator=g).to(torch.bfloat16)
+    ctx = torch.tensor(ctx, dtype=torch.int32)
+    args = (q, kc, vc, bt, ctx)
+    ref = torch_ref.paged_attn_decode_ref(*args, hd ** -0.5)
+    out = ops.paged_attn_decode(*(t.cuda() for t in args), hd ** -0.5)
+    torch.testing.assert_close(out.float().cpu(), ref.float(), rtol=2.0 ** -7,
+                               atol=2.0 ** -14 * float(vc.abs().max()))
+
+
 @pytest.mark.parametrize(
     "seq_lens", [[64], [1, 37, 64, 200], [128, 1024], [63, 65, 129]]
 )
