@@ -779,19 +779,6 @@ def append_paged_kv(k, v, kcache, vcache, slot_mapping):
 SOFTCAP_ATTENTION_MFMA = True
 
 
-@functools.lru_cache(maxsize=256)
-def _softcap_tiles(seq_lens: tuple, num_seqs: int, device):
-    """Tile map of the MFMA attention kernel: prompt portions (the first
-    len(seq_lens) sequences of the batch) cut into runs of its tile rows,
-    and the sequences that bring one decoded row.  Cached: serving
-    repeats the same batch shapes."""
-    tq = int(_shared_ext("softcap_attention_tile_rows")())
-    tseq, toff = torch_ref.make_prefill_tiles(seq_lens, tq, device)
-    dec = torch.arange(len(seq_lens), num_seqs, dtype=torch.int32,
-                       device=device)
-    return tseq, toff, dec
-
-
 def softcap_attention(q, kcache, vcache, block_table, row_seq, positions,
                       scale: float, softcap: float = 0.0,
                       temp_coef: float = 0.0, temp_every: int = 1,
@@ -822,12 +809,10 @@ def softcap_attention(q, kcache, vcache, block_table, row_seq, positions,
                           device=q.device)
         if (q.dtype == torch.bfloat16 and SOFTCAP_ATTENTION_MFMA
                 and seq_cu is not None and seq_start is not None):
-            lens = tuple(prefill_seq_lens or ()) if num_prefill_rows else ()
-            tseq, toff, dec = _softcap_tiles(lens, seq_start.shape[0],
-                                             q.device)
+            lens = list(prefill_seq_lens or ()) if num_prefill_rows else []
             if _shared_ext("softcap_attention_mfma")(
                     out, q, kcache, vcache, block_table, seq_cu, seq_start,
-                    tseq, toff, dec, scale, softcap, temp_coef, temp_every,
+                    lens, scale, softcap, temp_coef, temp_every,
                     window, slopes, chunk, sinks, gate, keep):
                 return out
         _shared_ext("softcap_attention")(

@@ -1,0 +1,437 @@
+// Prompt attention on MFMA tiles (gfx950, bf16): the part that the engine's
+// prompt attentions share.  A workgroup of four waves owns 128 query rows of
+// one head, 32 per wave, and walks the keys they can see 64 at a time.
+//
+// What bounds it: per score NK + NV MFMA multiply-adds, and on the vector
+// units one max, one multiply-add, one exponential (quarter rate), one add
+// and half a conversion, at NK = NV = 128 about as many cycles as the MFMAs
+// take.  The design keeps everything else off those two units:
+//
+//   * S^T = K Q^T with mfma_f32_32x32x16_bf16: a lane then holds 16 keys of
+//     ONE query row per tile, so row maxima and sums are in-lane, with one
+//     exchange between lane halves per 64 keys (the sums only at the end);
+//   * O^T += V^T P^T: the C layout of S^T (keys 8a + 4h + 0..3 of lane half
+//     h) is fed to the B operand as it is, the key order inside the
+//     contraction being free as long as V^T is read in the same order, so
+//     the probabilities never leave their registers;
+//   * V stays row-major in LDS, ds_read_b64_tr_b16 transposes 4 keys x 16
+//     dims on the way to the A operand (no transposing stores);
+//   * K and V tiles go from global memory straight to LDS, the next tile
+//     being fetched while this one is used: two buffers, one barrier a tile,
+//     four LDS objects so that the reads of one buffer do not wait for the
+//     writes to the other;
+//   * 16-byte chunks are XOR-swizzled by row (on the global side, a DMA
+//     writes LDS linearly): K by row & 7 against the 32 rows of a fragment,
+//     V by the rows that one transposing read spreads over its lanes;
+//   * the running maximum is raised, and the accumulators rescaled, only
+//     when a row outgrows it by more than 2^8 (exact: every term carries
+//     the same factor, which the division by the sum takes out again);
+//   * masks are evaluated only in tiles that some row of the wave sees in
+//     part, and a wave skips tiles that none of its rows sees.
+//
+// Two waves per SIMD (256 registers, up to 80 KB of LDS per workgroup) let
+// one wave's softmax run beside the other's MFMAs.
+#pragma once
+
+#include "common.h"
+
+namespace igw {
+
+typedef __attribute__((ext_vector_type(4))) short ft_short4;
+typedef __attribute__((ext_vector_type(2))) __bf16 ft_bf16x2;
+typedef __attribute__((ext_vector_type(8))) __bf16 ft_bf16x8;
+typedef __attribute__((ext_vector_type(16))) float ft_f32x16;
+
+constexpr int FT_BN = 64;    // keys per tile
+constexpr int FT_WAVES = 4;  // waves per workgroup, 32 query rows each
+constexpr int FT_BM = 32 * FT_WAVES;
+constexpr float FT_LOG2E = 1.44269504088896340736f;
+
+// two floats -> packed bf16 pair, round to nearest even
+DEVINLINE uint32_t ft_pack_bf16(float a, float b) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+  const f32x2_t v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, ft_bf16x2));
+}
+
+// x of lane i and of lane i ^ 32, in both lanes: a = lower half's value, b =
+// upper half's.  Written out because the compiler folds the builtin's two
+// results into one when its operands are equal; the s_nop is the wait that
+// the swap needs behind the instruction that wrote its operands.
+DEVINLINE void ft_both_halves(float x, float& a, float& b) {
+  a = b = x;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 0" : "+v"(a), "+v"(b));
+}
+
+// Head and tile of a workgroup in a grid of ntiles * heads.  Ids go
+// round-robin over the 8 XCDs: heads are dealt to id % 8, so heads that share
+// keys run on one XCD, the tiles of a head follow each other there, the last
+// (longest) tiles of each prompt first.
+DEVINLINE void ft_head_and_tile(int heads, int ntiles, int* head, int* tile) {
+  const int id = blockIdx.x;
+  if (heads % 8 == 0) {
+    const int hp = heads >> 3, local = id >> 3;
+    *head = (id & 7) * hp + local % hp;
+    *tile = ntiles - 1 - local / hp;
+  } else {
+    *head = id % heads;
+    *tile = ntiles - 1 - id / heads;
+  }
+}
+
+// Sequence and row offset of tile t when each of the B sequences of cu takes
+// ceil(rows / BM) tiles (found here: a tile map made on the host costs copies
+// that wait for the stream).  One step per 64 sequences; false when there is
+// no such tile.
+template <int BM>
+DEVINLINE bool ft_find_tile(const int32_t* cu, int B, int t, int* seq,
+                            int* off) {
+  const int lane = threadIdx.x & 63;
+  int before = 0;
+  for (int base = 0; base < B; base += 64) {
+    const int i = base + lane;
+    const int n = i < B ? (cu[i + 1] - cu[i] + BM - 1) / BM : 0;
+    int sum = n;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(sum, d, 64);
+      if (lane >= d) sum += up;
+    }
+    const uint64_t past = __ballot(before + sum > t);
+    if (past) {
+      const int w = __builtin_ctzll(past);
+      *seq = __builtin_amdgcn_readfirstlane(base + w);
+      *off = __builtin_amdgcn_readfirstlane(
+          (t - before - __shfl(sum - n, w, 64)) * BM);
+      return true;
+    }
+    before += __builtin_amdgcn_readfirstlane(__shfl(sum, 63, 64));
+  }
+  return false;
+}
+
+// The key tiles of a workgroup, in order: [0, kept), then [first, end).
+struct FlashSpan {
+  int kv_len;            // keys of the sequence
+  int kept, first, end;  // kept and first are multiples of FT_BN
+  DEVINLINE int begin() const { return kept > 0 ? 0 : first; }
+  DEVINLINE int next(int kb) const {
+    kb += FT_BN;
+    return kb >= kept && kb < first ? first : kb;
+  }
+};
+
+// Scores of this lane's query row.
+struct FlashScore {
+  int pos;         // its position; it sees keys lo .. pos and < keep
+  int lo, keep;
+  int wave_pos;    // position of the wave's first row
+  int wave_lo[2];  // lo of the wave's first and last row
+  float c;         // raw score -> log2 of the weight, > 0 when PLAIN
+  float cap;       // > 0: c * s goes through cap tanh(. / cap), in log2
+  float slope;     // per key of distance, in log2
+};
+
+// K and V rows of one sequence.  begin(kbase, wave) is called before the
+// addresses of a tile are asked for, with the wave (which moves the tile's
+// rows 16 wave .. + 15); rows past the last key repeat it (they are masked).
+// prefetch(kbase, wave) is called one tile ahead.
+
+// In pages of any size; with 16 a wave's rows lie in one page, whose number
+// was asked for one tile ahead, and the address is a scalar base and a small
+// lane offset.
+struct PagedRows {
+  const uint16_t *k, *v;   // [pages, heads, size, width]
+  const int32_t* table;    // the sequence's pages
+  int head, heads, size, kw, vw, kv_len;
+  int page = 0, last = 0, tile = 0;
+  int64_t base = 0;
+  DEVINLINE void prefetch(int kbase, int wave) {
+    if (size == 16) page = table[min((kbase >> 4) + wave, (kv_len - 1) >> 4)];
+  }
+  DEVINLINE void begin(int kbase, int wave) {
+    tile = kbase;
+    if (size != 16) return;
+    last = kv_len - 1 - (min((kbase >> 4) + wave, (kv_len - 1) >> 4) << 4);
+    base = ((int64_t)__builtin_amdgcn_readfirstlane(page) * heads + head) * 16;
+  }
+  DEVINLINE const uint16_t* at(const uint16_t* p, int w, int r, int c) const {
+    // a chunk past the width repeats the first one: the other operand is zero
+    const int d = c * 8 < w ? c * 8 : 0;
+    if (size == 16)
+      return p + base * w + (uint32_t)(min(r & 15, last) * w + d);
+    const int pos = min(tile + r, kv_len - 1);
+    return p + (((int64_t)table[pos / size] * heads + head) * size +
+                pos % size) * w + d;
+  }
+  DEVINLINE const uint16_t* kp(int r, int c) const { return at(k, kw, r, c); }
+  DEVINLINE const uint16_t* vp(int r, int c) const { return at(v, vw, r, c); }
+};
+
+// Dense: k and v point to the sequence's first row, this head.  A tile's rows
+// are 32-bit offsets from its first.
+struct DenseRows {
+  const uint16_t *k, *v;
+  int k_rs, v_rs;
+  int kv_len;
+  const uint16_t *kt = nullptr, *vt = nullptr;
+  int last = 0;
+  DEVINLINE void prefetch(int, int) {}
+  DEVINLINE void begin(int kbase, int) {
+    kt = k + (int64_t)kbase * k_rs;
+    vt = v + (int64_t)kbase * v_rs;
+    last = kv_len - 1 - kbase;
+  }
+  DEVINLINE const uint16_t* kp(int r, int c) const {
+    return kt + (uint32_t)(min(r, last) * k_rs + c * 8);
+  }
+  DEVINLINE const uint16_t* vp(int r, int c) const {
+    return vt + (uint32_t)(min(r, last) * v_rs + c * 8);
+  }
+};
+
+// Swizzle of V's 16-byte chunks in row r.
+template <int NV>
+DEVINLINE int ft_vswz(int r) {
+  return NV >= 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2;
+}
+
+// Walks the tiles.  qf: the query row as B operand (dims 16 s + 8 half);
+// k0 .. v1: LDS of FT_BN rows of NK (NV) bf16.  Out: o[dt][i] is dim 32 dt +
+// 8 (i / 4) + 4 half + i % 4 of the lane's row, unnormalised; l the row's sum
+// and m its reference, in log2 (both lane halves alike).
+// PLAIN: causal only, the maximum is of raw scores.
+template <int NK, int NV, bool PLAIN, class Rows>
+DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
+                           const FlashScore& sc,
+                           const ft_bf16x8 (&qf)[NK / 16], uint8_t* k0,
+                           uint8_t* k1, uint8_t* v0, uint8_t* v1,
+                           ft_f32x16 (&o)[NV / 32], float& m, float& l) {
+  constexpr int BN = FT_BN, CK = NK / 8, CV = NV / 8;
+  constexpr int RW = BN / FT_WAVES;   // rows that a wave moves
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int half = lane >> 5, col = lane & 31;
+
+  auto stage = [&](int kbase, uint8_t* kd, uint8_t* vd) {
+    rows.begin(kbase, wave);
+#pragma unroll
+    for (int i = 0; i < CK / 4; ++i) {
+      const int r = wave * RW + (i * 64 + lane) / CK;
+      const int c = ((i * 64 + lane) % CK) ^ (r & 7);
+      __builtin_amdgcn_global_load_lds(
+          reinterpret_cast<const uint32_t*>(rows.kp(r, c)),
+          reinterpret_cast<uint32_t*>(kd + (wave * (CK / 4) + i) * 1024), 16,
+          0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < CV / 4; ++i) {
+      const int r = wave * RW + (i * 64 + lane) / CV;
+      const int c = ((i * 64 + lane) % CV) ^ ft_vswz<NV>(r);
+      __builtin_amdgcn_global_load_lds(
+          reinterpret_cast<const uint32_t*>(rows.vp(r, c)),
+          reinterpret_cast<uint32_t*>(vd + (wave * (CV / 4) + i) * 1024), 16,
+          0, 0);
+    }
+    rows.prefetch(span.next(kbase), wave);
+  };
+
+  // LDS offsets of this lane's fragments
+  int koff[NK / 16];  // K row `col` (+ 32 per sub-tile), dims 16 s + 8 half
+#pragma unroll
+  for (int s = 0; s < NK / 16; ++s)
+    koff[s] = col * (NK * 2) + (((2 * s + half) ^ (col & 7)) << 4);
+  int voff[NV / 32][2];  // V^T: dims 32 dt + 16 (lane bit 4), keys 4 half + 8 e
+#pragma unroll
+  for (int dt = 0; dt < NV / 32; ++dt)
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int i = lane & 15, r = 4 * half + 8 * e + (i >> 2);
+      const int c = 4 * dt + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
+      voff[dt][e] =
+          r * (NV * 2) + ((c ^ ft_vswz<NV>(r)) << 4) + 8 * (i & 1);
+    }
+
+  const ft_bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
+  m = -INFINITY;
+  l = 0.0f;  // this lane half's keys, until the end
+#pragma unroll
+  for (int dt = 0; dt < NV / 32; ++dt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
+  // tanh by exp2: cap - 2 cap / (1 + 2^(cap_k s))
+  const float cap_k = sc.cap > 0.0f ? 2.0f * FT_LOG2E * sc.c / sc.cap : 0.0f;
+
+  auto step = [&](int kbase, int knext, uint8_t* kb, uint8_t* vb, uint8_t* kn,
+                  uint8_t* vn) {
+    // this wave's loads of the tile have arrived; behind the barrier all
+    // have, and nobody reads the other buffer any more
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (knext < span.end) stage(knext, kn, vn);
+    if (kbase > sc.wave_pos + 31) return;
+    if (!PLAIN && kbase + BN <= sc.wave_lo[0] && kbase >= sc.keep) return;
+
+    ft_f32x16 s[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s[t][i] = 0.0f;
+#pragma unroll
+    for (int d = 0; d < NK / 16; ++d)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const ft_bf16x8 kf = *reinterpret_cast<const ft_bf16x8*>(
+            kb + koff[d] + t * 32 * NK * 2);
+        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[d], s[t], 0, 0,
+                                                       0);
+      }
+
+    if (!PLAIN) {
+      if (sc.cap > 0.0f) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            s[t][i] = fmaf(-2.0f * sc.cap,
+                           __builtin_amdgcn_rcpf(
+                               1.0f + __builtin_amdgcn_exp2f(s[t][i] * cap_k)),
+                           sc.cap);
+      } else {
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) s[t][i] *= sc.c;
+      }
+      if (sc.slope != 0.0f) {
+        const float base = (float)(kbase + 4 * half - sc.pos) * sc.slope;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            s[t][i] += fmaf(sc.slope, (float)(32 * t + (i & 3) + 8 * (i >> 2)),
+                            base);
+      }
+    }
+    bool partly = kbase + BN - 1 > sc.wave_pos;
+    if (!PLAIN) partly |= kbase < sc.wave_lo[1] && kbase + BN > sc.keep;
+    if (partly) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const int kpos = kbase + 32 * t + (i & 3) + 8 * (i >> 2) + 4 * half;
+          bool hide = kpos > sc.pos || kpos >= span.kv_len;
+          if (!PLAIN) hide |= kpos < sc.lo && kpos >= sc.keep;
+          if (hide) s[t][i] = -INFINITY;
+        }
+    }
+
+    float mx = s[0][0];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) mx = fmaxf(mx, s[t][i]);
+    {
+      float lo, hi;
+      ft_both_halves(mx, lo, hi);
+      mx = fmaxf(lo, hi);
+    }
+    const float c = PLAIN ? sc.c : 1.0f;
+    // grown by at most 2^8 for all rows of the wave: keep the old maximum
+    if (__any((mx - m) * c > 8.0f)) {
+      const float mn = fmaxf(m, mx);
+      const float alpha =
+          m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m - mn) * c);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < NV / 32; ++dt)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
+    }
+    const float mc = m == -INFINITY ? 0.0f : m * c;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        s[t][i] = __builtin_amdgcn_exp2f(PLAIN ? fmaf(s[t][i], c, -mc)
+                                               : s[t][i] - mc);
+
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks) {
+        union {
+          uint32_t u[4];
+          ft_bf16x8 v;
+        } pf;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          pf.u[e] = ft_pack_bf16(s[t][8 * ks + 2 * e],
+                                 s[t][8 * ks + 2 * e + 1]);
+          // the sum is of the rounded weights, the ones that V meets: their
+          // rounding then cancels in the quotient, and it is one dot
+          // product per pair
+          l = __builtin_amdgcn_fdot2_f32_bf16(
+              __builtin_bit_cast(ft_bf16x2, pf.u[e]), ones, l, false);
+        }
+#pragma unroll
+        for (int dt = 0; dt < NV / 32; ++dt) {
+          typedef __attribute__((address_space(3))) ft_short4 lds_short4;
+          union {
+            ft_short4 h[2];
+            ft_bf16x8 v;
+          } vf;
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            vf.h[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (lds_short4*)(vb + voff[dt][e] + (32 * t + 16 * ks) * NV * 2));
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf.v, o[dt],
+                                                          0, 0, 0);
+        }
+      }
+  };
+
+  int kb = span.begin();
+  if (kb < span.end) {
+    rows.prefetch(kb, wave);
+    stage(kb, k0, v0);
+    while (true) {
+      int kn = span.next(kb);
+      step(kb, kn, k0, v0, k1, v1);
+      if (kn >= span.end) break;
+      kb = kn;
+      kn = span.next(kb);
+      step(kb, kn, k1, v1, k0, v0);
+      if (kn >= span.end) break;
+      kb = kn;
+    }
+  }
+  float lo, hi;
+  ft_both_halves(l, lo, hi);
+  l = lo + hi;
+  if (PLAIN) m *= sc.c;
+}
+
+// Stores the lane's dims d of an output row times f(d), 4 dims at a time; P
+// is the row's real width.
+template <int NV, class F>
+DEVINLINE void flash_store(uint16_t* row, const ft_f32x16 (&o)[NV / 32], int P,
+                           int half, F f) {
+#pragma unroll
+  for (int dt = 0; dt < NV / 32; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d = 32 * dt + 8 * g + 4 * half;
+      if (d < P) {
+        uint2 w;
+        w.x = ft_pack_bf16(o[dt][4 * g] * f(d), o[dt][4 * g + 1] * f(d + 1));
+        w.y = ft_pack_bf16(o[dt][4 * g + 2] * f(d + 2),
+                           o[dt][4 * g + 3] * f(d + 3));
+        *reinterpret_cast<uint2*>(row + d) = w;
+      }
+    }
+}
+
+}  // namespace igw

@@ -55,14 +55,13 @@ void softcap_attention(torch::Tensor out, torch::Tensor q, torch::Tensor kcache,
 bool softcap_attention_mfma(torch::Tensor out, torch::Tensor q,
                             torch::Tensor kcache, torch::Tensor vcache,
                             torch::Tensor block_table, torch::Tensor seq_cu,
-                            torch::Tensor seq_start, torch::Tensor tile_seq,
-                            torch::Tensor tile_off, torch::Tensor dec_seq,
-                            double scale, double softcap, double temp_coef,
+                            torch::Tensor seq_start,
+                            std::vector<int64_t> prompt_rows, double scale,
+                            double softcap, double temp_coef,
                             int64_t temp_every, int64_t window,
                             c10::optional<torch::Tensor> slopes,
                             int64_t chunk, c10::optional<torch::Tensor> sinks,
                             c10::optional<torch::Tensor> gate, int64_t keep);
-int64_t softcap_attention_tile_rows();
 void delta_scan(torch::Tensor out, torch::Tensor q, torch::Tensor k,
                 torch::Tensor v, torch::Tensor decay, torch::Tensor beta,
                 torch::Tensor state, torch::Tensor seq_cu,
@@ -125,8 +124,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("softcap_attention_mfma", &igw::softcap_attention_mfma,
         "capped softmax attention on MFMA tiles (bf16); false = sizes do "
         "not fit, use softcap_attention");
-  m.def("softcap_attention_tile_rows", &igw::softcap_attention_tile_rows,
-        "query rows per MFMA tile");
   m.def("add_rmsnorm_pair", &igw::add_rmsnorm_pair,
         "fp32 residual += two deltas; one RMS statistic, two weighted outputs");
   m.def("relu2", &igw::relu2, "squared ReLU activation");

@@ -1,9 +1,6 @@
 // Causal softmax attention with a score cap on MFMA tiles (gfx950, bf16):
-// the serving path of softcap_attention.  Same tiling as the engine's
-// paged flash-attention prefill (64 query rows x 64 keys per step, 4
-// waves of 16 rows, mfma_f32_16x16x32_bf16 for Q.K^T and P.V, K staged
-// row-major and V transposed in swizzled LDS, probabilities through a
-// per-wave LDS tile, online softmax in fp32 registers), generalised to
+// the serving path of softcap_attention, generalised over the engine's prompt
+// attention by
 //
 //   * key width N and value width P of their own, each padded with zeros
 //     to the template's NP / PP (N, P multiples of 8);
@@ -15,16 +12,28 @@
 //     positions, an optional linear distance bias per head
 //     (slope * (row position - key position) is taken off the score), an
 //     optional sink term per head in the softmax denominator and an
-//     optional sigmoid output gate (per value entry or per head);
-//   * two row maps.  Prompt tiles: rows are 64 consecutive tokens of one
-//     head (grid = tiles x heads).  Decoded rows (HEADS_ROWS): the rows of
-//     a tile are the query heads that share one key/value head, so every
-//     K/V page is staged once per group instead of once per head
-//     (grid = decoded rows x key/value heads).
+//     optional sigmoid output gate (per value entry or per head).
+//
+// Prompt rows with P <= 128 run the tile walk of flash_tile.h
+// (softcap_prompt_kernel: 128 rows of one head).  Decoded rows, and prompt
+// rows of wider values, whose accumulators do not fit two waves per SIMD
+// there, run softcap_attention_mfma_kernel: 64 rows x 64 keys, 4 waves of 16
+// rows, mfma_f32_16x16x32_bf16, K staged row-major and V transposed in
+// swizzled LDS, probabilities through a per-wave LDS tile.  Its row maps:
+// prompt tiles (64 consecutive tokens of one head), and decoded rows
+// (HEADS_ROWS), where the rows of a tile are the query heads that share one
+// key/value head, so every K/V page is staged once per group instead of once
+// per head (grid = decoded rows x key/value heads).
+//
+// Measured (32 heads on 8, N = P = 128), 64-row tiles for all and the tile
+// walk: prompts of 3000 and 2790 tokens, window 1024 with 16 kept tokens,
+// distance bias and head gate 563 and 198 us; 4 prompts of 2048, causal, with
+// a sink 1293 and 261 us, with a score cap 1412 and 285 us.
 //
 // Everything is read from the paged cache; a row's own key is already
 // appended.  Sequence s has rows [seq_cu[s], seq_cu[s+1]) whose first sits
-// at position seq_start[s].
+// at position seq_start[s]; the first sequences are the prompt portions.
+#include "../csrc/flash_tile.h"
 #include "../csrc_hybrid/act_types.h"
 
 namespace igw {
@@ -61,8 +70,8 @@ __global__ __launch_bounds__(256, 2) void softcap_attention_mfma_kernel(
     const uint16_t* __restrict__ kcache, const uint16_t* __restrict__ vcache,
     const int32_t* __restrict__ block_table, int max_blocks,
     const int32_t* __restrict__ seq_cu, const int32_t* __restrict__ seq_start,
-    const int32_t* __restrict__ tile_seq, const int32_t* __restrict__ tile_off,
-    int H, int G, int N, int P, int BS, float scale, float softcap,
+    int nprompt, int H, int G, int N, int P, int BS, float scale,
+    float softcap,
     float temp_coef, int temp_every, int window,
     const float* __restrict__ slopes, int chunk, int keep,
     const float* __restrict__ sinks, const uint16_t* __restrict__ gate,
@@ -76,13 +85,13 @@ __global__ __launch_bounds__(256, 2) void softcap_attention_mfma_kernel(
   uint16_t* vt_s = smem + BN * NP;
   uint16_t* p_s = vt_s + PP * BN;
 
-  const int tile = blockIdx.x;
-  const int seq = tile_seq[tile];
+  int seq = nprompt + blockIdx.x, qoff = 0;
+  if (!HEADS_ROWS && !ft_find_tile<BM>(seq_cu, nprompt, blockIdx.x, &seq, &qoff))
+    return;
   const int q0 = seq_cu[seq];
   const int Lq = HEADS_ROWS ? 1 : seq_cu[seq + 1] - q0;
   const int P0 = seq_start[seq];
   const int KVL = P0 + Lq;
-  const int qoff = HEADS_ROWS ? 0 : tile_off[tile];
   const int rep = H / G;
   const int kvh = HEADS_ROWS ? blockIdx.y : blockIdx.y / rep;
   const int nrows = HEADS_ROWS ? rep : min(BM, Lq - qoff);  // valid rows
@@ -334,17 +343,109 @@ __global__ __launch_bounds__(256, 2) void softcap_attention_mfma_kernel(
   }
 }
 
-int64_t softcap_attention_tile_rows() { return SA_BM; }
+struct SoftcapArgs {
+  uint16_t* out;             // [T, H * P]
+  const uint16_t* q;         // [T, H * N], row stride q_rs
+  int64_t q_rs;
+  const uint16_t *kcache, *vcache;
+  const int32_t *block_table, *seq_cu, *seq_start;
+  int max_blocks, nprompt, ntiles, H, G, N, P, BS;
+  float scale, softcap, temp_coef;
+  int temp_every, window, chunk, keep;
+  const float *slopes, *sinks;
+  const uint16_t* gate;      // [T, H * gate_w], row stride gate_rs
+  int64_t gate_rs;
+  int gate_w;
+};
 
-// prompt tiles: (tile_seq, tile_off) over the first sequences of the
-// batch; decoded rows: dec_seq lists the sequences that bring one row.
-// Returns false when the sizes do not fit the tile kernel.
+template <int NP, int PP>
+__global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_prompt_kernel(
+    SoftcapArgs a) {
+  __shared__ __attribute__((aligned(1024))) uint8_t k_s0[FT_BN * NP * 2];
+  __shared__ __attribute__((aligned(1024))) uint8_t k_s1[FT_BN * NP * 2];
+  __shared__ __attribute__((aligned(1024))) uint8_t v_s0[FT_BN * PP * 2];
+  __shared__ __attribute__((aligned(1024))) uint8_t v_s1[FT_BN * PP * 2];
+  const int lane = threadIdx.x & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+  int head, tile, seq, qoff;
+  ft_head_and_tile(a.H, a.ntiles, &head, &tile);
+  if (!ft_find_tile<FT_BM>(a.seq_cu, a.nprompt, tile, &seq, &qoff)) return;
+  const int q0 = a.seq_cu[seq];
+  const int Lq = a.seq_cu[seq + 1] - q0;
+  const int P0 = a.seq_start[seq];
+  const int KVL = P0 + Lq;
+
+  const int row = qoff + wave * 32 + (lane & 31);
+  ft_bf16x8 qf[NP / 16];
+  const uint16_t* qp = a.q + (int64_t)(q0 + min(row, Lq - 1)) * a.q_rs +
+                       (int64_t)head * a.N;
+#pragma unroll
+  for (int s = 0; s < NP / 16; ++s) {
+    const int d = 16 * s + 8 * half;
+    ft_bf16x8 f{};
+    if (d < a.N) f = *reinterpret_cast<const ft_bf16x8*>(qp + d);
+    qf[s] = f;
+  }
+
+  auto first_key = [&](int pos) {   // window and position chunk
+    int lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+    return a.chunk > 0 ? max(lo, pos / a.chunk * a.chunk) : lo;
+  };
+  FlashScore sc{};
+  sc.pos = P0 + row;
+  sc.lo = first_key(sc.pos);
+  sc.keep = a.keep;
+  sc.wave_pos = P0 + qoff + wave * 32;
+  sc.wave_lo[0] = first_key(sc.wave_pos);
+  sc.wave_lo[1] = first_key(sc.wave_pos + 31);
+  sc.c = a.scale * FT_LOG2E *
+         (1.0f + a.temp_coef *
+                     logf((float)((sc.pos + 1) / a.temp_every) + 1.0f));
+  sc.cap = a.softcap > 0.0f ? a.softcap * FT_LOG2E : 0.0f;
+  sc.slope = a.slopes ? a.slopes[head] * FT_LOG2E : 0.0f;
+  FlashSpan span;
+  span.kv_len = KVL;
+  span.first = first_key(P0 + qoff) / FT_BN * FT_BN;
+  span.kept =
+      a.keep > 0 ? min((a.keep + FT_BN - 1) / FT_BN * FT_BN, span.first) : 0;
+  span.end = min(KVL, P0 + qoff + FT_BM);
+
+  PagedRows rows{a.kcache, a.vcache,
+                 a.block_table + (int64_t)seq * a.max_blocks,
+                 head / (a.H / a.G), a.G, a.BS, a.N, a.P, KVL};
+  ft_f32x16 o[PP / 32];
+  float m, l;
+  flash_tiles<NP, PP, false>(rows, span, sc, qf, k_s0, k_s1, v_s0, v_s1, o, m,
+                             l);
+  if (row >= Lq) return;
+  // the sink's term relative to the running maximum (an overflow to
+  // infinity gives the right limit, an all-zero row)
+  if (a.sinks)
+    l += __builtin_amdgcn_exp2f(fmaf(a.sinks[head], FT_LOG2E, -m));
+  const float inv = 1.0f / l;
+  const uint16_t* gt =
+      a.gate ? a.gate + (q0 + row) * a.gate_rs + head * a.gate_w : nullptr;
+  uint16_t* out = a.out + ((int64_t)(q0 + row) * a.H + head) * a.P;
+  if (gt && a.gate_w > 1)
+    flash_store<PP>(out, o, a.P, half, [&](int d) {
+      return inv * sigmoid_fast(bf16_to_f32(gt[d]));
+    });
+  else {
+    const float f = gt ? inv * sigmoid_fast(bf16_to_f32(gt[0])) : inv;
+    flash_store<PP>(out, o, a.P, half, [&](int) { return f; });
+  }
+}
+
+// prompt_rows: row counts of the first sequences of the batch; the other
+// sequences bring one decoded row each.  Returns false when the sizes do not
+// fit the tile kernels.
 bool softcap_attention_mfma(torch::Tensor out, torch::Tensor q,
                             torch::Tensor kcache, torch::Tensor vcache,
                             torch::Tensor block_table, torch::Tensor seq_cu,
-                            torch::Tensor seq_start, torch::Tensor tile_seq,
-                            torch::Tensor tile_off, torch::Tensor dec_seq,
-                            double scale, double softcap, double temp_coef,
+                            torch::Tensor seq_start,
+                            std::vector<int64_t> prompt_rows, double scale,
+                            double softcap, double temp_coef,
                             int64_t temp_every, int64_t window,
                             c10::optional<torch::Tensor> slopes,
                             int64_t chunk, c10::optional<torch::Tensor> sinks,
@@ -360,21 +461,21 @@ bool softcap_attention_mfma(torch::Tensor out, torch::Tensor q,
   const int H = q.size(1) / N;
   TORCH_CHECK(H % G == 0 && vcache.size(0) == kcache.size(0) &&
               vcache.size(1) == G && vcache.size(2) == BS);
-  const int ndec = dec_seq.numel(), ntile = tile_seq.numel();
+  const int S = seq_start.numel(), nprompt = prompt_rows.size();
+  TORCH_CHECK(nprompt <= S);
+  const int ndec = S - nprompt;
   if (N % 8 || P % 8 || N > 128 || P > 256 || q.stride(0) % 8 ||
       (reinterpret_cast<uintptr_t>(q.data_ptr()) & 15) ||
+      (reinterpret_cast<uintptr_t>(kcache.data_ptr()) & 15) ||
+      (reinterpret_cast<uintptr_t>(vcache.data_ptr()) & 15) ||
       (ndec > 0 && H / G > SA_BM))
     return false;
   TORCH_CHECK(out.is_contiguous() && out.dtype() == q.dtype() &&
               out.numel() == (int64_t)T * H * P);
   TORCH_CHECK(block_table.dtype() == torch::kInt32 &&
               block_table.is_contiguous() && block_table.dim() == 2);
-  const int S = seq_start.numel();
   TORCH_CHECK(seq_cu.dtype() == torch::kInt32 && seq_cu.numel() == S + 1 &&
               seq_start.dtype() == torch::kInt32 && block_table.size(0) >= S);
-  TORCH_CHECK(tile_seq.dtype() == torch::kInt32 &&
-              tile_off.dtype() == torch::kInt32 &&
-              tile_off.numel() == ntile && dec_seq.dtype() == torch::kInt32);
   TORCH_CHECK(temp_every >= 1 && chunk >= 0 && keep >= 0);
   if (slopes.has_value())
     TORCH_CHECK(slopes->dtype() == torch::kFloat32 &&
@@ -388,36 +489,55 @@ bool softcap_attention_mfma(torch::Tensor out, torch::Tensor q,
                 (gate->size(1) == (int64_t)H * P || gate->size(1) == H));
   const int gate_w = gate.has_value() ? (int)(gate->size(1) / H) : 1;
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
-#define LAUNCH_SA(NPV, PPV, HR, GRID, TSEQ)                                   \
+  auto tiles = [&](int bm) {
+    int64_t n = 0;
+    for (int64_t len : prompt_rows) n += (len + bm - 1) / bm;
+    return n;
+  };
+  SoftcapArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)q.data_ptr(),
+                q.stride(0), (const uint16_t*)kcache.data_ptr(),
+                (const uint16_t*)vcache.data_ptr(),
+                (const int32_t*)block_table.data_ptr(),
+                (const int32_t*)seq_cu.data_ptr(),
+                (const int32_t*)seq_start.data_ptr(),
+                (int)block_table.size(1), nprompt, (int)tiles(FT_BM), H, G, N,
+                P, BS, (float)scale, (float)softcap, (float)temp_coef,
+                (int)temp_every, (int)window, (int)chunk, (int)keep,
+                slopes.has_value() ? (const float*)slopes->data_ptr() : nullptr,
+                sinks.has_value() ? (const float*)sinks->data_ptr() : nullptr,
+                gate.has_value() ? (const uint16_t*)gate->data_ptr() : nullptr,
+                gate.has_value() ? (int64_t)gate->stride(0) : 0, gate_w};
+#define LAUNCH_SP(NPV, PPV)                                                   \
+  hipLaunchKernelGGL((softcap_prompt_kernel<NPV, PPV>),                       \
+                     dim3((int64_t)a.ntiles * H), dim3(64 * FT_WAVES), 0,     \
+                     stream, a)
+#define LAUNCH_SA(NPV, PPV, HR, GRID)                                         \
   hipLaunchKernelGGL(                                                         \
       (softcap_attention_mfma_kernel<NPV, PPV, HR>), GRID, dim3(256), 0,      \
-      stream, (uint16_t*)out.data_ptr(), (const uint16_t*)q.data_ptr(),       \
-      (int64_t)q.stride(0), (const uint16_t*)kcache.data_ptr(),               \
-      (const uint16_t*)vcache.data_ptr(),                                     \
-      (const int32_t*)block_table.data_ptr(), (int)block_table.size(1),       \
-      (const int32_t*)seq_cu.data_ptr(), (const int32_t*)seq_start.data_ptr(), \
-      (const int32_t*)TSEQ.data_ptr(), (const int32_t*)tile_off.data_ptr(),   \
-      H, G, N, P, BS, (float)scale, (float)softcap, (float)temp_coef,         \
-      (int)temp_every, (int)window,                                           \
-      slopes.has_value() ? (const float*)slopes->data_ptr() : nullptr,        \
-      (int)chunk, (int)keep,                                                  \
-      sinks.has_value() ? (const float*)sinks->data_ptr() : nullptr,          \
-      gate.has_value() ? (const uint16_t*)gate->data_ptr() : nullptr,         \
-      gate.has_value() ? (int64_t)gate->stride(0) : 0, gate_w)
-#define LAUNCH_SA_SIZES(HR, GRID, TSEQ)                                       \
-  do {                                                                        \
-    if (N <= 64 && P <= 64) LAUNCH_SA(64, 64, HR, GRID, TSEQ);                \
-    else if (N <= 64 && P <= 128) LAUNCH_SA(64, 128, HR, GRID, TSEQ);         \
-    else if (N <= 64) LAUNCH_SA(64, 256, HR, GRID, TSEQ);                     \
-    else if (P <= 64) LAUNCH_SA(128, 64, HR, GRID, TSEQ);                     \
-    else if (P <= 128) LAUNCH_SA(128, 128, HR, GRID, TSEQ);                   \
-    else LAUNCH_SA(128, 256, HR, GRID, TSEQ);                                 \
-  } while (0)
-  if (ntile > 0) LAUNCH_SA_SIZES(false, dim3(ntile, H), tile_seq);
-  if (ndec > 0) LAUNCH_SA_SIZES(true, dim3(ndec, G), dec_seq);
-#undef LAUNCH_SA_SIZES
+      stream, a.out, a.q, a.q_rs, a.kcache, a.vcache, a.block_table,          \
+      a.max_blocks, a.seq_cu, a.seq_start, nprompt, H, G, N, P, BS, a.scale,  \
+      a.softcap, a.temp_coef, a.temp_every, a.window, a.slopes, a.chunk,      \
+      a.keep, a.sinks, a.gate, a.gate_rs, gate_w)
+  if (a.ntiles > 0) {
+    if (N <= 64 && P <= 64) LAUNCH_SP(64, 64);
+    else if (N <= 64 && P <= 128) LAUNCH_SP(64, 128);
+    else if (P <= 64) LAUNCH_SP(128, 64);
+    else if (P <= 128) LAUNCH_SP(128, 128);
+    else if (N <= 64) LAUNCH_SA(64, 256, false, dim3(tiles(SA_BM), H));
+    else LAUNCH_SA(128, 256, false, dim3(tiles(SA_BM), H));
+    HIP_CHECK_KERNEL();
+  }
+  if (ndec > 0) {
+    if (N <= 64 && P <= 64) LAUNCH_SA(64, 64, true, dim3(ndec, G));
+    else if (N <= 64 && P <= 128) LAUNCH_SA(64, 128, true, dim3(ndec, G));
+    else if (N <= 64) LAUNCH_SA(64, 256, true, dim3(ndec, G));
+    else if (P <= 64) LAUNCH_SA(128, 64, true, dim3(ndec, G));
+    else if (P <= 128) LAUNCH_SA(128, 128, true, dim3(ndec, G));
+    else LAUNCH_SA(128, 256, true, dim3(ndec, G));
+    HIP_CHECK_KERNEL();
+  }
 #undef LAUNCH_SA
-  HIP_CHECK_KERNEL();
+#undef LAUNCH_SP
   return true;
 }
 

@@ -472,6 +472,70 @@ def _check_draw(row, temp, k, p, u, got):
     assert got == 0 or cdf[got - 1] <= u + 1e-5
 
 
+@pytest.mark.parametrize("rows,starts,H,G,N,P,bs,kw", [
+    # row and key tile edges; padded widths; heads over the chiplets
+    ([127, 128, 129], [0, 64, 1], 8, 2, 128, 128, 16, {}),
+    ([200, 3], [0, 61], 4, 2, 32, 16, 16, dict(sinks=True)),
+    ([130, 63], [0, 77], 4, 2, 24, 16, 4,
+     dict(window=20, keep=3, slopes=True, gate=1)),
+    ([257, 5], [0, 100], 8, 2, 128, 64, 16,
+     dict(softcap=20.0, temp_coef=0.25, temp_every=8)),
+    ([300], [0], 4, 4, 16, 24, 16, dict(chunk=50, slopes=True, gate=2)),
+    # a window that starts inside, at and before a wave's first tile
+    ([400, 190], [0, 300], 3, 1, 64, 72, 16, dict(window=64)),
+    ([320], [0], 2, 1, 64, 128, 32,
+     dict(window=33, keep=70, sinks=True, gate=1)),
+    # values too wide for the tile walk; decoded rows beside portions
+    ([150, 1, 1], [0, 40, 99], 6, 3, 96, 136, 16, dict(sinks=True, gate=2)),
+    ([70, 1, 1], [10, 0, 300], 8, 2, 128, 128, 16, dict(chunk=64)),
+    ([100], [0], 8, 8, 64, 64, 16, dict(scale=-0.2)),
+])
+def test_softcap_prompt_tiles(rows, starts, H, G, N, P, bs, kw):
+    """The tile kernels against the CPU rows, over the forms that reach
+    them."""
+    kw = dict(kw)
+    g = torch.Generator().manual_seed(sum(rows))
+    portions = [n for n in rows if n > 1]
+    T, need = sum(rows), [-(-(a + b) // bs) for a, b in zip(rows, starts)]
+    kc, vc = (torch.randn(sum(need) + 1, G, bs, w, generator=g).to(
+        torch.bfloat16) for w in (N, P))
+    order = torch.randperm(sum(need), generator=g).to(torch.int32) + 1
+    bt = torch.zeros(len(rows), max(need), dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    row_seq = torch.repeat_interleave(
+        torch.arange(len(rows)), torch.tensor(rows)).to(torch.int32)
+    pos = torch.cat([torch.arange(a, a + n) for n, a in zip(rows, starts)]
+                    ).to(torch.int32)
+    cu = torch.tensor([0] + torch.tensor(rows).cumsum(0).tolist(),
+                      dtype=torch.int32)
+    start = torch.tensor(starts, dtype=torch.int32)
+    q = torch.randn(T, H * N, generator=g).to(torch.bfloat16)
+    opt = dict(
+        slopes=torch.rand(H, generator=g) * 0.2
+        if kw.pop("slopes", False) else None,
+        sinks=torch.randn(H, generator=g)
+        if kw.pop("sinks", False) else None)
+    gate = kw.pop("gate", 0)
+    opt["gate"] = torch.randn(T, H * (P if gate == 2 else 1), generator=g).to(
+        torch.bfloat16) if gate else None
+    scale = kw.pop("scale", N ** -0.5)
+
+    def run(dev, **more):
+        a = [t.to(dev) for t in (q, kc, vc, bt, row_seq, pos)]
+        o = {k: None if v is None else v.to(dev) for k, v in opt.items()}
+        return ops.softcap_attention(*a, scale, **kw, **o, **more)
+
+    ref = run("cpu")
+    out = run("cuda", num_prefill_rows=sum(portions),
+              prefill_seq_lens=portions, seq_cu=cu.cuda(),
+              seq_start=start.cuda())
+    torch.testing.assert_close(out.float().cpu(), ref.float(),
+                               atol=_attention_bound(vc), rtol=2.0 ** -8)
+
+
 @pytest.mark.parametrize("V", [
     1, 7, 8, 9, 4095, 4096, 4097,          # chunks and their tails
     32767, 32768, 32769,                   # 8 chunks, the first of 16
