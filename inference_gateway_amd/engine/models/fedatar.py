@@ -48,6 +48,11 @@ def _rand(shape, device, dtype, name: str, scale: float = 1.0):
         scale).to(dtype)
 
 
+# prompt rows in a batch from which latent attention writes out its keys and
+# values
+EXPAND_FROM = 64
+
+
 class LayerNormParams(nn.Module):
     """Weight and bias of a LayerNorm, held in fp32 (the norm runs in
     fp32 on the fp32 residual — ops.add_layernorm)."""
@@ -149,6 +154,18 @@ class LatentAttention(nn.Module):
         self.inv_freq = _param(torch.tensor(
             freq, dtype=torch.float64).to(torch.float32).to(device))
 
+    def _expanded_rows(self, q, fb) -> int:
+        """Leading rows of the batch that run with keys and values written
+        out (ops.latent_prompt_attention): all prompt rows, if every portion
+        is a whole prompt (so the keys are the rows) and there are enough of
+        them to pay for the two up-projections; else 0."""
+        P = fb.num_chunk_rows
+        if not (q.is_cuda and fb.is_prefill and fb.prefix_lens is None
+                and P >= EXPAND_FROM and fb.cu_seqlens is not None):
+            return 0
+        return P if ops.latent_prompt_fits(q, self.spec.rot_dim,
+                                           self.spec.vdim) else 0
+
     def cache_width(self) -> int:
         return self.spec.cache_width
 
@@ -179,14 +196,33 @@ class LatentAttention(nn.Module):
             q = F.linear(cq, self.uq).view(T, H, dn + rd)
             ops.rope_pairs_(q, fb.positions, self.inv_freq, dn, sp.rot_half,
                             self.mag)
-        q_abs = torch.bmm(q[:, :, :dn].transpose(0, 1), self.uk)  # [H,T,R]
-        o_lat = ops.latent_attention(
-            q_abs.transpose(0, 1), q[:, :, dn:], cache, fb.seq_block_table,
-            fb.row_seq, fb.positions, self.sink, sp.scale, sp.window,
-            fb.num_chunk_rows, fb.seq_lens, fb.max_context, gate)
-        # the batched product writes head-major rows [T, H, vd] in place
         v = torch.empty((T, H, sp.vdim), dtype=h.dtype, device=h.device)
-        torch.bmm(o_lat.transpose(0, 1), self.uv_t, out=v.transpose(0, 1))
+        P = self._expanded_rows(q, fb)
+        if P:
+            # whole prompts: their keys and values written out (the rows'
+            # latents are in the cache already)
+            rows = cache.view(-1, sp.cache_width).index_select(
+                0, fb.slot_mapping[:P])
+            lat = rows[:, :sp.kv_rank]
+            ops.latent_prompt_attention(
+                q[:P], F.linear(lat, self.uk.view(H * dn, sp.kv_rank)),
+                rows[:, sp.kv_rank:],
+                torch.bmm(lat.expand(H, P, sp.kv_rank), self.uv_t),
+                fb.cu_seqlens, fb.seq_lens, self.sink, sp.scale, sp.window,
+                gate, out=v[:P])
+        if P < T:
+            whole = P == 0
+            q_abs = torch.bmm(q[P:, :, :dn].transpose(0, 1), self.uk)
+            o_lat = ops.latent_attention(
+                q_abs.transpose(0, 1), q[P:, :, dn:], cache,
+                fb.seq_block_table, fb.row_seq[P:], fb.positions[P:],
+                self.sink, sp.scale, sp.window,
+                fb.num_chunk_rows if whole else 0,
+                fb.seq_lens if whole else None, fb.max_context,
+                None if gate is None else gate[P:])
+            # the batched product writes head-major rows [T, H, vd] in place
+            torch.bmm(o_lat.transpose(0, 1), self.uv_t,
+                      out=v[P:].transpose(0, 1))
         return F.linear(v.view(T, H * sp.vdim), self.o)
 
 

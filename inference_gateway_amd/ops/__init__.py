@@ -467,6 +467,39 @@ def latent_attention(q_abs, q_rot, cache, block_table, row_seq, positions,
         window, gate)
 
 
+def latent_prompt_fits(q, rot_dim: int, vdim: int) -> bool:
+    """Whether latent_prompt_attention takes queries q [P, H, dim + rot_dim]
+    and values of vdim entries on their device."""
+    if not q.is_cuda:
+        return True
+    return q.dtype == torch.bfloat16 and LATENT_ATTENTION_MFMA and bool(
+        _shared_ext("latent_prompt_fits")(q.shape[2] - rot_dim, rot_dim,
+                                          vdim)) \
+        and q.stride(0) % 8 == 0 and q.stride(1) % 8 == 0 \
+        and q.data_ptr() % 16 == 0
+
+
+def latent_prompt_attention(q, k_heads, k_rot, v, cu_seqlens, seq_lens, sink,
+                            scale: float, window: int, gate=None, out=None):
+    """Attention of whole prompts (sequence i: rows cu[i] .. cu[i + 1] at
+    positions 0, 1, ...) whose keys are a part per head and a rotated part
+    that all heads share: q [P, H, dim + rot_dim] (strided ok), k_heads [P,
+    H * dim], k_rot [P, rot_dim] (strided rows ok), v [H, P, vdim]; window,
+    sink and gate as in latent_attention.  Returns [P, H, vdim] (`out` when
+    given)."""
+    if out is None:
+        out = torch.empty((q.shape[0], q.shape[1], v.shape[2]),
+                          dtype=q.dtype, device=q.device)
+    if q.is_cuda:
+        _shared_ext("latent_prompt")(out, q, k_heads, k_rot, v, cu_seqlens,
+                                     list(seq_lens), sink, scale, window,
+                                     gate)
+        return out
+    out.copy_(torch_ref.latent_prompt_attention_ref(
+        q, k_heads, k_rot, v, seq_lens, sink, scale, window, gate))
+    return out
+
+
 def xielu(z, pq):
     if z.is_cuda:
         _require_hybrid()

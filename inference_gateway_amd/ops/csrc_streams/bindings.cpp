@@ -58,6 +58,12 @@ bool latent_attention_mfma(torch::Tensor out, torch::Tensor q_abs,
                            int64_t window, int64_t max_keys,
                            c10::optional<torch::Tensor> gate);
 int64_t latent_attention_tile_rows(int64_t H);
+bool latent_prompt_fits(int64_t dn, int64_t rd, int64_t vd);
+void latent_prompt(torch::Tensor out, torch::Tensor q, torch::Tensor kn,
+                   torch::Tensor kr, torch::Tensor v, torch::Tensor cu,
+                   std::vector<int64_t> rows,
+                   c10::optional<torch::Tensor> sink, double scale,
+                   int64_t window, c10::optional<torch::Tensor> gate);
 void moe_topk_route(torch::Tensor weights, torch::Tensor idx,
                     torch::Tensor logits, c10::optional<torch::Tensor> dst,
                     c10::optional<torch::Tensor> counts, int64_t capacity,
@@ -123,6 +129,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("latent_attention_mfma", &igw::latent_attention_mfma,
         "absorbed latent attention on MFMA tiles (bf16); false = sizes do "
         "not fit, use latent_attention");
+  m.def("latent_prompt_fits", &igw::latent_prompt_fits,
+        "whether latent_prompt takes these head widths");
+  m.def("latent_prompt", &igw::latent_prompt,
+        "latent attention of whole prompts, keys and values written out");
   m.def("latent_attention_tile_rows", &igw::latent_attention_tile_rows,
         "token rows per MFMA tile for a head count");
   m.def("moe_topk_route", &igw::moe_topk_route,

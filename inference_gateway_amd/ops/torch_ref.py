@@ -411,6 +411,35 @@ def latent_down_post_ref(down, positions, slot_mapping, cache, qnorm_w,
     return cq.to(down.dtype), gate
 
 
+def latent_prompt_attention_ref(q, k_heads, k_rot, v, seq_lens, sink, scale,
+                                window, gate=None):
+    """Row t of head h of a prompt scores its keys j as (q[t,h] . (k_heads[j,h]
+    | k_rot[j])) * scale for t-window < j <= t (window 0: all j <= t); the
+    softmax denominator also holds exp(sink_h).  [P, H, vdim]."""
+    P, H, dk = q.shape
+    dn = dk - k_rot.shape[1]
+    out = torch.empty((P, H, v.shape[2]), dtype=torch.float32,
+                      device=q.device)
+    a = 0
+    for n in seq_lens:
+        rows = slice(a, a + n)
+        k = torch.cat([k_heads[rows].view(n, H, dn).float(),
+                       k_rot[rows].float()[:, None].expand(n, H, dk - dn)],
+                      -1).transpose(0, 1)
+        s = q[rows].float().transpose(0, 1) @ k.transpose(1, 2) * scale
+        i = torch.arange(n, device=q.device)
+        hide = i[None] > i[:, None]
+        if window > 0:
+            hide |= i[None] <= i[:, None] - window
+        s = s.masked_fill(hide, float("-inf"))
+        if sink is not None:
+            s = torch.cat([s, sink.float().view(H, 1, 1).expand(H, n, 1)], -1)
+        p = torch.softmax(s, -1)[..., :n]
+        out[rows] = (p @ v[:, rows].float()).transpose(0, 1)
+        a += n
+    return out if gate is None else out * gate[:P].unsqueeze(-1)
+
+
 def latent_attention_ref(q_abs, q_rot, cache, block_table, row_seq,
                          positions, sink, scale, window, gate=None):
     """Absorbed latent attention over the paged cache.  Row t of head h

@@ -536,6 +536,109 @@ def test_softcap_prompt_tiles(rows, starts, H, G, N, P, bs, kw):
                                atol=_attention_bound(vc), rtol=2.0 ** -8)
 
 
+@pytest.mark.parametrize("rows,H,dn,rd,vd,kw", [
+    ([127, 128, 129], 8, 128, 64, 128, {}),
+    ([64, 1, 65], 4, 128, 64, 128, dict(sink=True, gate=True)),
+    ([300], 3, 16, 8, 24, dict(window=70, gate=True)),
+    ([200, 130], 16, 64, 32, 64, dict(window=1, sink=True)),
+    ([90], 8, 184, 8, 8, dict(window=64)),
+])
+def test_latent_prompt_attention(rows, H, dn, rd, vd, kw):
+    g = torch.Generator().manual_seed(sum(rows))
+    P = sum(rows)
+
+    def t(*shape):
+        return torch.randn(*shape, generator=g).to(torch.bfloat16)
+
+    # queries and rotated keys as slices of wider rows
+    q = t(P, H, dn + rd + 8)[:, :, :dn + rd]
+    kn, kr, v = t(P, H * dn), t(P, rd + 8)[:, 8:], t(H, P, vd)
+    cu = torch.tensor([0] + torch.tensor(rows).cumsum(0).tolist(),
+                      dtype=torch.int32)
+    sink = torch.randn(H, generator=g) if kw.get("sink") else None
+    gate = torch.rand(P, H, generator=g) if kw.get("gate") else None
+    scale, window = (dn + rd) ** -0.5, kw.get("window", 0)
+    ref = torch_ref.latent_prompt_attention_ref(q, kn, kr, v, rows, sink,
+                                                scale, window, gate)
+    q, kr = t(P, H, dn + rd + 8).copy_(torch.nn.functional.pad(q, (0, 8))), \
+        torch.nn.functional.pad(kr, (8, 0))
+    out = ops.latent_prompt_attention(
+        q.cuda()[:, :, :dn + rd], kn.cuda(), kr.cuda()[:, 8:], v.cuda(),
+        cu.cuda(), rows, None if sink is None else sink.cuda(), scale,
+        window, None if gate is None else gate.cuda())
+    torch.testing.assert_close(out.float().cpu(), ref,
+                               atol=_attention_bound(v), rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("design", ["fedatar", "bivatar", "defosun"])
+def test_latent_written_out_matches_absorbed(design):
+    """A latent layer gives the same rows with its keys written out as in
+    absorbed form: whole prompts beside decoded tokens, where only the
+    prompts are written out, and a batch with a continued portion, where
+    nothing is."""
+    from inference_gateway_amd.engine.config import MODEL_PRESETS
+    from inference_gateway_amd.engine.models import fedatar as mod
+    from inference_gateway_amd.engine.models.batch import ForwardBatch
+
+    cfg = MODEL_PRESETS[f"tiny-{design}"]
+    spec = next(l.mixer for l in cfg.layers
+                if l.type in ("latent_attention", "attention")
+                and hasattr(l.mixer, "kv_rank"))
+    torch.manual_seed(3)
+    layer = mod.LatentAttention(cfg.hidden_size, spec, 1e-6, "t", "cuda",
+                                torch.bfloat16)
+    bs, rows, starts = 16, [70, 1, 33, 1, 1], [0, 0, 0, 50, 7]
+    T, need = sum(rows), [-(-(a + b) // bs) for a, b in zip(rows, starts)]
+    bt = torch.zeros(5, max(need), dtype=torch.int32)
+    at = 1
+    for i, n in enumerate(need):
+        bt[i, :n] = torch.arange(at, at + n)
+        at += n
+    seq = torch.repeat_interleave(torch.arange(5), torch.tensor(rows))
+    pos = torch.cat([torch.arange(a, a + n) for n, a in zip(rows, starts)])
+    slots = bt[seq, pos // bs] * bs + pos % bs
+    cu = torch.tensor([0] + torch.tensor(rows).cumsum(0).tolist(),
+                      dtype=torch.int32)
+    h = torch.randn(T, cfg.hidden_size).to(torch.bfloat16).cuda()
+    first = torch.randn(at, bs, spec.cache_width).to(torch.bfloat16).cuda()
+
+    def run(expand_from, portions, prefix):
+        i32 = dict(dtype=torch.int32, device="cuda")
+        fb = ForwardBatch(
+            token_ids=torch.zeros(T, dtype=torch.int64, device="cuda"),
+            positions=pos.to(**i32), slot_mapping=slots.to(**i32),
+            is_prefill=True, cu_seqlens=cu[:portions + 1].cuda(),
+            seq_lens=rows[:portions], seq_block_table=bt.cuda(),
+            row_seq=seq.to(**i32), num_chunk_rows=sum(rows[:portions]),
+            max_context=70)
+        if prefix:
+            fb.prefix_lens = torch.tensor(starts[:portions], **i32)
+        old, mod.EXPAND_FROM = mod.EXPAND_FROM, expand_from
+        try:
+            cache = first.clone()
+            assert (layer._expanded_rows(
+                torch.empty(T, spec.heads, spec.dim + spec.rot_dim,
+                            dtype=torch.bfloat16, device="cuda"), fb)
+                    == (sum(rows[:portions]) if expand_from == 1
+                        and not prefix else 0))
+            return layer.forward(h, fb, cache).float().cpu(), cache
+        finally:
+            mod.EXPAND_FROM = old
+
+    # three whole prompts (of 70, 1 and 33 rows) and two decoded tokens
+    a, ca = run(1, 3, False)
+    b, cb = run(10 ** 9, 3, False)
+    assert torch.equal(ca, cb)
+    # queries, keys, results and values are each rounded to bf16 once on
+    # either way: a few steps of 2^-8 of the rows' size
+    assert float((a - b).norm() / b.norm()) < 4 * 2.0 ** -8
+    assert torch.equal(a[104:], b[104:])
+    # a portion behind cached tokens
+    c, _ = run(1, 4, True)
+    d, _ = run(10 ** 9, 4, True)
+    assert torch.equal(c, d)
+
+
 @pytest.mark.parametrize("V", [
     1, 7, 8, 9, 4095, 4096, 4097,          # chunks and their tails
     32767, 32768, 32769,                   # 8 chunks, the first of 16
