@@ -19,7 +19,7 @@ with RMS norms and one multiplier m.  Mixers, chosen per layer:
 The feed-forward is GatedMLP (gelu-gated).  Everything a layer keeps
 between steps is paged and handed in by the engine (cache_specs), so
 portions of prompts, decoded tokens and mixed batches are one code path.
-GEMMs go through F.linear/bmm; everything between them is a gfx950 kernel
+GEMMs go through ops.linear/bmm; everything between them is a gfx950 kernel
 from ops, the residual update fused with its norm and the cast that the
 next GEMM reads.
 """
@@ -69,7 +69,7 @@ class WindowAttention(nn.Module):
     def forward(self, h: torch.Tensor, fb: ForwardBatch, cache):
         kc, vc = cache
         s = self.spec
-        proj = F.linear(h, self.qkvg)
+        proj = ops.linear(h, self.qkvg)
         q = ops.qk_norm_rope_append(
             proj, fb.positions, fb.slot_mapping, kc, vc, self.qnorm_w,
             self.knorm_w, None, 1.0, self.eps, s.heads, s.kv_heads, s.dim,
@@ -79,7 +79,7 @@ class WindowAttention(nn.Module):
             s.scale, 0.0, 0.0, 1, s.window, fb.num_chunk_rows, fb.seq_lens,
             fb.seq_cu, fb.seq_start, slopes=self.slopes,
             gate=proj[:, self.gate0:], keep=s.keep_first)
-        return F.linear(o, self.o)
+        return ops.linear(o, self.o)
 
 
 class GatedMLP(nn.Module):
@@ -96,7 +96,7 @@ class GatedMLP(nn.Module):
                        spec.ff)
 
     def forward(self, h: torch.Tensor, fb: ForwardBatch) -> torch.Tensor:
-        return F.linear(ops.gated_act(F.linear(h, self.gate_up), self.mode),
+        return ops.linear(ops.gated_act(ops.linear(h, self.gate_up), self.mode),
                         self.down)
 
 
@@ -186,4 +186,4 @@ class BivatarForCausalLM(nn.Module):
             self.dtype, cfg.residual_mult)
 
     def compute_logits(self, hidden_last: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden_last, self.head).float()
+        return ops.linear(hidden_last, self.head).float()

@@ -29,7 +29,7 @@ router that chooses inside the best expert groups.
 Everything a layer keeps between steps is paged K/V or a slot buffer
 handed in by the engine (cache_specs), so portions of prompts, decoded
 tokens and mixed batches are one code path.  GEMMs go through
-F.linear/bmm; the small projections that feed the recurrence's gates and
+ops.linear/bmm; the small projections that feed the recurrence's gates and
 the router run in fp32; everything between GEMMs is a gfx950 kernel from
 ops.
 """
@@ -92,7 +92,7 @@ class ChunkBiasAttention(nn.Module):
         """cache: this layer's (K, V) pages, or its source layer's."""
         kc, vc = cache
         s = self.spec
-        proj = F.linear(h, self.qkvg)
+        proj = ops.linear(h, self.qkvg)
         k0, v0 = self.nq, self.nq + self.nk
         if self.owns_kv:
             ops.append_paged_kv(proj[:, k0:v0], proj[:, v0:v0 + self.nv],
@@ -102,7 +102,7 @@ class ChunkBiasAttention(nn.Module):
             fb.positions, s.scale, 0.0, 0.0, 1, 0, fb.num_chunk_rows,
             fb.seq_lens, fb.seq_cu, fb.seq_start, slopes=self.slopes,
             chunk=s.chunk, gate=proj[:, v0 + self.nv:])
-        return F.linear(o, self.o)
+        return ops.linear(o, self.o)
 
 
 class SinkRotaryAttention(nn.Module):
@@ -152,7 +152,7 @@ class SinkRotaryAttention(nn.Module):
     def forward(self, h, fb: ForwardBatch, cache):
         (kc, vc), = cache
         s = self.spec
-        proj = F.linear(h, self.qkv, self.qkv_b)
+        proj = ops.linear(h, self.qkv, self.qkv_b)
         q = ops.qk_norm_rope_append(
             proj, fb.positions, fb.slot_mapping, kc, vc, self.qnorm_w,
             self.knorm_w, self.inv_freq, self.mag, self.eps, s.heads,
@@ -161,7 +161,7 @@ class SinkRotaryAttention(nn.Module):
             q, kc, vc, fb.seq_block_table, fb.row_seq, fb.positions,
             s.scale, 0.0, 0.0, 1, 0, fb.num_chunk_rows, fb.seq_lens,
             fb.seq_cu, fb.seq_start, sinks=self.sinks)
-        return F.linear(o, self.o, self.o_b)
+        return ops.linear(o, self.o, self.o_b)
 
 
 class GatedDeltaMixer(nn.Module):
@@ -205,9 +205,9 @@ class GatedDeltaMixer(nn.Module):
         s = self.spec
         H, G, N, P = s.heads, s.kv_heads, s.dim, s.vdim
         T, GN, CC = h.shape[0], G * N, s.conv_channels
-        proj = F.linear(h, self.qkvg)
+        proj = ops.linear(h, self.qkvg)
         decay, beta = ops.decay_beta_gates(
-            F.linear(h.float(), self.ab_w), self.a_log, self.dt_bias)
+            ops.linear(h.float(), self.ab_w), self.a_log, self.dt_bias)
         c = ops.causal_conv(proj[:, :CC], self.conv_w, None, conv_state,
                             fb.seq_cu, fb.seq_start, fb.seq_slots,
                             fb.row_seq, True)
@@ -218,7 +218,7 @@ class GatedDeltaMixer(nn.Module):
             float(N) ** -0.5)
         y = ops.head_norm_gate(o, proj[:, CC:], self.norm_w, self.eps, P,
                                ops.GATE_SILU, False, None, None, self.dtype)
-        return F.linear(y, self.o)
+        return ops.linear(y, self.o)
 
 
 class GroupRoutedMoE(nn.Module):
@@ -252,7 +252,7 @@ class GroupRoutedMoE(nn.Module):
     def forward(self, h: torch.Tensor, fb: ForwardBatch) -> torch.Tensor:
         sp = self.spec
         T = h.shape[0]
-        logits = F.linear(h.float(), self.router_w)
+        logits = ops.linear(h.float(), self.router_w)
         padded = T <= self.PADDED_MAX_ROWS
         C = (T + 63) // 64 * 64
         weights, idx, dst = ops.moe_group_route(
@@ -281,9 +281,9 @@ class TokenSideInput(nn.Module):
         self.norm_w = _norm_w(hidden, device, name + ".norm")
 
     def forward(self, x, table, token_ids):
-        g = ops.gelu_mul_rows(F.linear(x, self.gate), table, token_ids,
+        g = ops.gelu_mul_rows(ops.linear(x, self.gate), table, token_ids,
                               self.col0)
-        return F.linear(g, self.proj)
+        return ops.linear(g, self.proj)
 
 
 class BozolornLayer(nn.Module):
@@ -390,4 +390,4 @@ class BozolornForCausalLM(nn.Module):
                                       self.dtype)
 
     def compute_logits(self, hidden_last: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden_last, self.head).float()
+        return ops.linear(hidden_last, self.head).float()

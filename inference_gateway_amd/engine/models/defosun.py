@@ -70,7 +70,7 @@ class FixedDecayAttention(nn.Module):
         H, N, P = s.heads, s.dim, s.vdim
         T, k0, v0 = h.shape[0], H * N, 2 * H * N
         g0 = v0 + H * P
-        proj = F.linear(h, self.qkvg)
+        proj = ops.linear(h, self.qkvg)
         o = ops.fixed_decay_scan(
             proj[:, :k0].view(T, H, N), proj[:, k0:v0].view(T, H, N),
             proj[:, v0:g0].view(T, H, P), self.decay, mem, fb.seq_cu,
@@ -78,7 +78,7 @@ class FixedDecayAttention(nn.Module):
         y = ops.head_norm_gate(o, proj[:, g0:], self.norm_w, self.eps, H * P,
                                ops.GATE_SIGMOID, False, None, None,
                                self.dtype)
-        return F.linear(y, self.o)
+        return ops.linear(y, self.o)
 
 
 class SharedExpertMoE(nn.Module):
@@ -118,7 +118,7 @@ class SharedExpertMoE(nn.Module):
     def forward(self, h: torch.Tensor, fb: ForwardBatch) -> torch.Tensor:
         sp = self.spec
         T, E = h.shape[0], sp.experts
-        logits = F.linear(h.float(), self.router_w)
+        logits = ops.linear(h.float(), self.router_w)
         padded = T <= self.PADDED_MAX_ROWS
         C = (T + 63) // 64 * 64
         weights, idx, dst = ops.moe_topk_route(
@@ -127,8 +127,8 @@ class SharedExpertMoE(nn.Module):
             dst = moe_common.padded_rows(idx, E, C)
         shared = gate = None
         if self.shared_up is not None:
-            shared = F.linear(ops.gated_act(
-                F.linear(h, self.shared_up), ops.GATED_ACT_CLAMPED,
+            shared = ops.linear(ops.gated_act(
+                ops.linear(h, self.shared_up), ops.GATED_ACT_CLAMPED,
                 sp.shared_limit, self.ALPHA), self.shared_down)
             gate = logits[:, E]
         return moe_common.experts_combined(
@@ -256,4 +256,4 @@ class DefosunForCausalLM(nn.Module):
                                self.dtype)[1]
 
     def compute_logits(self, hidden_last: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden_last, self.head).float()
+        return ops.linear(hidden_last, self.head).float()

@@ -17,7 +17,7 @@ by the configuration:
 
 The mechanisms are separate modules with their constants as arguments so
 other designs can assemble them differently.  GEMMs go through
-F.linear/bmm (hipBLASLt / rocBLAS); everything between them is a gfx950
+ops.linear/bmm (hipBLASLt / rocBLAS); everything between them is a gfx950
 kernel from ops (fp32 math for norms, angles, softmax, gates and the
 recurrence; bf16 or fp32 activations).
 """
@@ -90,10 +90,10 @@ class MinGRUMixer(nn.Module):
 
     def forward(self, h: torch.Tensor, fb: ForwardBatch,
                 state: torch.Tensor) -> torch.Tensor:
-        zxg = F.linear(h, self.zxg, self.zxg_b)
+        zxg = ops.linear(h, self.zxg, self.zxg_b)
         y = ops.mingru_scan(zxg, state, fb.seq_cu, fb.seq_start,
                             fb.seq_slots, fb.seq_rows)
-        return F.linear(y, self.o)
+        return ops.linear(y, self.o)
 
 
 class LatentAttention(nn.Module):
@@ -179,7 +179,7 @@ class LatentAttention(nn.Module):
         sp = self.spec
         T = h.shape[0]
         H, dn, rd = sp.heads, sp.dim, sp.rot_dim
-        down = F.linear(h, self.down)
+        down = ops.linear(h, self.down)
         if self.direct:
             gate = None
             ops.latent_rope_append(
@@ -193,7 +193,7 @@ class LatentAttention(nn.Module):
                 cache if self.owns_kv else None, self.qnorm_w,
                 self.kvnorm_w, self.inv_freq, self.eps, sp.q_rank,
                 sp.kv_rank, rd, H, sp.rot_half, self.mag)
-            q = F.linear(cq, self.uq).view(T, H, dn + rd)
+            q = ops.linear(cq, self.uq).view(T, H, dn + rd)
             ops.rope_pairs_(q, fb.positions, self.inv_freq, dn, sp.rot_half,
                             self.mag)
         v = torch.empty((T, H, sp.vdim), dtype=h.dtype, device=h.device)
@@ -205,7 +205,7 @@ class LatentAttention(nn.Module):
                 0, fb.slot_mapping[:P])
             lat = rows[:, :sp.kv_rank]
             ops.latent_prompt_attention(
-                q[:P], F.linear(lat, self.uk.view(H * dn, sp.kv_rank)),
+                q[:P], ops.linear(lat, self.uk.view(H * dn, sp.kv_rank)),
                 rows[:, sp.kv_rank:],
                 torch.bmm(lat.expand(H, P, sp.kv_rank), self.uv_t),
                 fb.cu_seqlens, fb.seq_lens, self.sink, sp.scale, sp.window,
@@ -223,7 +223,7 @@ class LatentAttention(nn.Module):
             # the batched product writes head-major rows [T, H, vd] in place
             torch.bmm(o_lat.transpose(0, 1), self.uv_t,
                       out=v[P:].transpose(0, 1))
-        return F.linear(v.view(T, H * sp.vdim), self.o)
+        return ops.linear(v.view(T, H * sp.vdim), self.o)
 
 
 class XieluMLP(nn.Module):
@@ -241,7 +241,7 @@ class XieluMLP(nn.Module):
                                 name + ".act", 25.0))
 
     def forward(self, h: torch.Tensor, fb: ForwardBatch) -> torch.Tensor:
-        return F.linear(ops.xielu(F.linear(h, self.up), self.act),
+        return ops.linear(ops.xielu(ops.linear(h, self.up), self.act),
                         self.down)
 
 
@@ -284,7 +284,7 @@ class Relu2MoE(nn.Module):
     def forward(self, h: torch.Tensor, fb: ForwardBatch) -> torch.Tensor:
         T = h.shape[0]
         E, K = self.spec.experts, self.spec.top
-        logits = F.linear(h.float(), self.router_w, self.router_b)
+        logits = ops.linear(h.float(), self.router_w, self.router_b)
         padded = T <= self.PADDED_MAX_ROWS
         C = (T + 63) // 64 * 64
         weights, idx, dst = ops.moe_topk_route(logits, K, C if padded else 0)
@@ -297,7 +297,7 @@ class Relu2MoE(nn.Module):
             out = moe_common.experts_sorted(h, weights, idx, self.up_t,
                                             self.down_t, ops.relu2)
         if self.shared_up is not None:
-            out = out + F.linear(ops.relu2(F.linear(h, self.shared_up)),
+            out = out + ops.linear(ops.relu2(ops.linear(h, self.shared_up)),
                                  self.shared_down)
         return out
 
@@ -382,4 +382,4 @@ class FedatarForCausalLM(nn.Module):
                                  self.dtype)
 
     def compute_logits(self, hidden_last: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden_last, self.head).float()
+        return ops.linear(hidden_last, self.head).float()

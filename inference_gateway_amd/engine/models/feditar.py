@@ -21,7 +21,7 @@ a, c, k, q are made and the read-out's epilogue (ops.head_norm_gate).
 Everything a layer keeps between steps is a slot buffer or paged K/V
 handed in by the engine (cache_specs), so portions of prompts, decoded
 tokens and mixed batches are the same code path.  GEMMs go through
-F.linear/bmm; the small projections that feed gates, step sizes and
+ops.linear/bmm; the small projections that feed gates, step sizes and
 decays run in fp32.
 """
 from __future__ import annotations
@@ -83,8 +83,8 @@ class MLSTMMixer(nn.Module):
         s = self.spec
         H, N, P = s.heads, s.dim, s.vdim
         T = h.shape[0]
-        proj = F.linear(h, self.qkvg)
-        pre = F.linear(h.float(), self.gates_w, self.gates_b)
+        proj = ops.linear(h, self.qkvg)
+        pre = ops.linear(h.float(), self.gates_w, self.gates_b)
         decay, kscale, floor = ops.mlstm_gates(
             pre, s.gate_cap, m_state, fb.seq_cu, fb.seq_start, fb.seq_slots)
         o, den = ops.outer_scan(
@@ -97,7 +97,7 @@ class MLSTMMixer(nn.Module):
         y = ops.head_norm_gate(o, proj[:, 2 * H * N + H * P:], self.norm_w,
                                self.eps, P, ops.GATE_SIGMOID, False, den,
                                floor, self.dtype)
-        return F.linear(y, self.o)
+        return ops.linear(y, self.o)
 
 
 class Mamba2Mixer(nn.Module):
@@ -141,9 +141,9 @@ class Mamba2Mixer(nn.Module):
         s = self.spec
         H, P, N, G, inner = s.heads, s.vdim, s.state, s.groups, s.inner
         T = h.shape[0]
-        proj = F.linear(h, self.in_main)
+        proj = ops.linear(h, self.in_main)
         decay, dt = ops.ssm_gates(
-            F.linear(h.float(), self.dt_w, self.dt_b), self.a_log)
+            ops.linear(h.float(), self.dt_w, self.dt_b), self.a_log)
         xbc = ops.causal_conv(proj[:, inner:], self.conv_w, self.conv_b,
                               conv_state, fb.seq_cu, fb.seq_start,
                               fb.seq_slots, fb.row_seq, True)
@@ -156,7 +156,7 @@ class Mamba2Mixer(nn.Module):
         y = ops.head_norm_gate(o, proj[:, :inner], self.norm_w, self.eps,
                                inner // s.norm_groups, ops.GATE_SILU, True,
                                None, None, self.dtype)
-        return F.linear(y, self.o)
+        return ops.linear(y, self.o)
 
 
 class SoftcapAttention(nn.Module):
@@ -187,7 +187,7 @@ class SoftcapAttention(nn.Module):
         (kc, vc), conv_state = cache
         s = self.spec
         HN, GN = s.heads * s.dim, s.kv_heads * s.dim
-        c = F.linear(h, self.qkv)
+        c = ops.linear(h, self.qkv)
         if s.conv > 1:
             c = ops.causal_conv(c, self.conv_w, None, conv_state, fb.seq_cu,
                                 fb.seq_start, fb.seq_slots, fb.row_seq,
@@ -198,7 +198,7 @@ class SoftcapAttention(nn.Module):
             c[:, :HN], kc, vc, fb.seq_block_table, fb.row_seq, fb.positions,
             s.scale, s.softcap, s.temp_coef, s.temp_every, 0,
             fb.num_chunk_rows, fb.seq_lens, fb.seq_cu, fb.seq_start)
-        return F.linear(o, self.o)
+        return ops.linear(o, self.o)
 
 
 class DecayMemory(nn.Module):
@@ -244,7 +244,7 @@ class DecayMemory(nn.Module):
         mixes = ops.token_shift_mix(h, self.mu, prev_h, fb.seq_cu,
                                     fb.seq_start, fb.seq_slots, fb.row_seq)
         rkvg = torch.bmm(mixes[:4], self.rkvg_t)          # [4, T, H*N]
-        lw = F.linear(torch.tanh(F.linear(mixes[4].float(), self.w1)),
+        lw = ops.linear(torch.tanh(ops.linear(mixes[4].float(), self.w1)),
                       self.w2, self.w0)                    # fp32 [T, H*N]
         o, _ = ops.outer_scan(
             rkvg[0].view(T, H, N), rkvg[1].view(T, H, N),
@@ -253,7 +253,7 @@ class DecayMemory(nn.Module):
             ops.DECAY_EXP_NEG_EXP, False, 1.0)
         y = ops.head_norm_gate(o, rkvg[3], self.norm_w, self.eps, N,
                                ops.GATE_SILU, False, None, None, self.dtype)
-        return F.linear(y, self.o)
+        return ops.linear(y, self.o)
 
 
 class ParallelMixer(nn.Module):
@@ -293,7 +293,7 @@ class Relu2MLP(nn.Module):
         self.down = _w((hidden, ff), device, dtype, name + ".down", ff)
 
     def forward(self, h):
-        return F.linear(ops.relu2(F.linear(h, self.up)), self.down)
+        return ops.linear(ops.relu2(ops.linear(h, self.up)), self.down)
 
 
 class FeditarLayer(nn.Module):
@@ -390,4 +390,4 @@ class FeditarForCausalLM(nn.Module):
         return h
 
     def compute_logits(self, hidden_last: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden_last, self.embed).float()
+        return ops.linear(hidden_last, self.embed).float()

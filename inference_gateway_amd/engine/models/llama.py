@@ -1,7 +1,7 @@
 """Llama-family decoder (Llama-3 8B / 70B architectures) for the MI355X
 engine.
 
-Compute path (SURVEY.md §7 stage 3): GEMMs via F.linear (hipBLASLt on ROCm,
+Compute path (SURVEY.md §7 stage 3): GEMMs via ops.linear (hipBLASLt on ROCm,
 TP-sharded through parallel.layers); everything between them is a
 hand-written gfx950 kernel — fused add+RMSNorm, NeoX RoPE, paged-cache
 append, MFMA flash prefill / paged decode attention, fused SwiGLU. On CPU
@@ -79,7 +79,7 @@ class LlamaAttention(nn.Module):
                 kv_cache: Tuple[torch.Tensor, torch.Tensor],
                 cos_sin: torch.Tensor) -> torch.Tensor:
         T = x.shape[0]
-        qkv = F.linear(x, self.qkv, self.qkv_b)
+        qkv = ops.linear(x, self.qkv, self.qkv_b)
         # strided views into the fused QKV output — the HIP kernels take a
         # row stride, so there are no .contiguous() copies on the hot path
         q, k, v = qkv.split(
@@ -137,8 +137,7 @@ class LlamaMLP(nn.Module):
         del self.gate_proj, self.up_proj
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        gu = F.linear(x, self.gate_up)
-        return self.down_proj(ops.silu_mul(gu))
+        return self.down_proj(ops.linear_silu_mul(x, self.gate_up))
 
 
 class LlamaLayer(nn.Module):
@@ -207,5 +206,5 @@ class LlamaForCausalLM(nn.Module):
         """hidden_last: [B, hidden] -> bf16 logits [B, vocab] (the
         sampler's bf16 radix kernel consumes them directly)."""
         if self.lm_head is None:
-            return F.linear(hidden_last, self.embed)
+            return ops.linear(hidden_last, self.embed)
         return self.lm_head(hidden_last)

@@ -21,7 +21,7 @@ second, and both results are added back together:
                                  renormalised and scaled, SwiGLU experts
 
 The mechanisms are separate modules with their constants as arguments.
-GEMMs go through F.linear/bmm (hipBLASLt / rocBLAS); everything between
+GEMMs go through ops.linear/bmm (hipBLASLt / rocBLAS); everything between
 them is a gfx950 kernel from ops (fp32 math for norms, scores, weights,
 router; bf16 or fp32 activations).
 """
@@ -110,7 +110,7 @@ class SigmoidWindowAttention(nn.Module):
         is the first blending layer)."""
         sp = self.spec
         kcache, vcache = cache
-        proj = F.linear(h, self.qkvg)
+        proj = ops.linear(h, self.qkvg)
         q = ops.qk_norm_append(
             proj, fb.slot_mapping, kcache, vcache, self.qnorm_w,
             self.knorm_w, v_first, self.lam, self.eps, sp.heads,
@@ -120,7 +120,7 @@ class SigmoidWindowAttention(nn.Module):
             q, kcache, vcache, fb.seq_block_table, fb.row_seq, fb.positions,
             self.dist_bias, self.talk, proj[:, v0 + self.nv:], sp.scale,
             sp.window, fb.num_chunk_rows, fb.seq_lens, fb.max_context)
-        return F.linear(o, self.o), proj[:, v0:v0 + self.nv]
+        return ops.linear(o, self.o), proj[:, v0:v0 + self.nv]
 
 
 class ClampedGLUMLP(nn.Module):
@@ -140,9 +140,9 @@ class ClampedGLUMLP(nn.Module):
                                  name + ".down", spec.ff ** -0.5 / 0.02))
 
     def forward(self, h: torch.Tensor, fb: ForwardBatch) -> torch.Tensor:
-        a = ops.gated_act(F.linear(h, self.gate_up), ops.GATED_ACT_CLAMPED,
+        a = ops.gated_act(ops.linear(h, self.gate_up), ops.GATED_ACT_CLAMPED,
                           self.limit, self.ALPHA)
-        return F.linear(a, self.down)
+        return ops.linear(a, self.down)
 
 
 class RoutedGLUMoE(nn.Module):
@@ -175,7 +175,7 @@ class RoutedGLUMoE(nn.Module):
     def forward(self, h: torch.Tensor, fb: ForwardBatch) -> torch.Tensor:
         T = h.shape[0]
         E, K = self.spec.experts, self.spec.top
-        logits = F.linear(h.float(), self.router_w)
+        logits = ops.linear(h.float(), self.router_w)
         padded = T <= self.PADDED_MAX_ROWS
         C = (T + 63) // 64 * 64
         weights, idx, dst = ops.moe_topk_route(
@@ -276,7 +276,7 @@ class MekevikForCausalLM(nn.Module):
         return h
 
     def compute_logits(self, hidden_last: torch.Tensor) -> torch.Tensor:
-        logits = F.linear(hidden_last, self.head).float()
+        logits = ops.linear(hidden_last, self.head).float()
         if self.cfg.logit_scale != 1.0:
             logits.mul_(self.cfg.logit_scale)
         return logits

@@ -205,6 +205,41 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_mul_ref(gate_up)
 
 
+def _gemv_takes(x, w, swiglu: bool) -> bool:
+    return (x.is_cuda and HAS_KERNELS and x.dim() == 2 and w.dim() == 2
+            and x.shape[0] <= 8 and x.dtype == torch.bfloat16
+            and w.dtype == x.dtype and w.shape[1] == x.shape[1]
+            and _kernels.gemv_fits(x.shape[0], x.shape[1], swiglu)
+            and w.is_contiguous() and x.stride(1) == 1
+            and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and w.data_ptr() % 16 == 0
+            and not (torch.is_grad_enabled()
+                     and (x.requires_grad or w.requires_grad)))
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
+    """x W^T (+ bias).  A few rows of bf16 run the weight-streaming kernel
+    (ops/csrc/gemv.hip), everything else the library's product."""
+    if _gemv_takes(x, w, False) and (bias is None or (
+            bias.dtype == x.dtype and bias.is_contiguous())):
+        out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
+                          device=x.device)
+        _kernels.gemv(out, x, w, bias, False)
+        return out
+    return torch.nn.functional.linear(x, w, bias)
+
+
+def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """silu(x Wg^T) * (x Wu^T) with w = [Wg; Wu]: one kernel for a few rows
+    of bf16, else the product and silu_mul."""
+    if _gemv_takes(x, w, True) and w.shape[0] % 2 == 0:
+        out = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype,
+                          device=x.device)
+        _kernels.gemv(out, x, w, None, True)
+        return out
+    return silu_mul(torch.nn.functional.linear(x, w))
+
+
 def sample(logits, temperature, top_k, top_p, uniforms):
     """logits [B, V] fp32 -> sampled token ids [B] int32."""
     if logits.is_cuda:

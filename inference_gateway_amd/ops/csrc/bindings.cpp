@@ -29,6 +29,9 @@ void flash_prefill_paged(torch::Tensor out, torch::Tensor q,
                          torch::Tensor block_table, torch::Tensor prefix_lens,
                          torch::Tensor cu_seqlens,
                          std::vector<int64_t> seq_lens, double scale);
+void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+          c10::optional<torch::Tensor> bias, bool swiglu);
+bool gemv_fits(int64_t M, int64_t K, bool swiglu);
 void sample(torch::Tensor out, torch::Tensor logits, torch::Tensor temperature,
             torch::Tensor top_k, torch::Tensor top_p, torch::Tensor uniforms);
 void silu_mul(torch::Tensor out, torch::Tensor gate_up);
@@ -70,6 +73,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "GQA paged-attention decode (bf16, gfx950)");
   m.def("flash_prefill", &igw::flash_prefill,
         "varlen causal MFMA flash-attention prefill (bf16, gfx950)");
+  m.def("gemv", &igw::gemv,
+        "x W^T for a few rows of x, optional bias or SwiGLU");
+  m.def("gemv_fits", &igw::gemv_fits, "whether gemv takes these sizes");
   m.def("flash_prefill_paged", &igw::flash_prefill_paged,
         "paged-extend prefill: chunk queries over cached prefix+chunk K/V "
         "via block table (bf16, gfx950)");

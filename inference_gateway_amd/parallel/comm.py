@@ -31,6 +31,8 @@ from typing import Optional
 import torch
 import torch.distributed as dist
 
+from .. import ops
+
 _TP_SIZE = 1
 _TP_RANK = 0
 _ONESHOT = None            # OneShotAllReduce or None (ring fallback)
@@ -144,7 +146,7 @@ def row_parallel_matmul_allreduce(x: torch.Tensor,
     if (_TP_SIZE <= 1 or not torch.cuda.is_available()
             or x.shape[0] < _OVERLAP_MIN_ROWS
             or torch.cuda.is_current_stream_capturing()):
-        return tp_all_reduce(F.linear(x, weight))
+        return tp_all_reduce(ops.linear(x, weight))
     cs = comm_stream()
     cur = torch.cuda.current_stream()
     n = _OVERLAP_CHUNKS

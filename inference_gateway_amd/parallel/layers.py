@@ -2,15 +2,16 @@
 
 Megatron-style sharding adapted to the 8-GPU xGMI node:
 column-parallel layers keep their shard's activations local; row-parallel
-layers end in one RCCL all-reduce. GEMMs go through F.linear (hipBLASLt on
-ROCm); the fused hot ops around them are the hand-written gfx950 kernels.
+layers end in one RCCL all-reduce. GEMMs go through ops.linear (hipBLASLt on
+ROCm, a streaming kernel for a few rows); the fused hot ops around them are
+the hand-written gfx950 kernels.
 """
 from __future__ import annotations
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
+from .. import ops
 from .comm import row_parallel_matmul_allreduce, tp_all_reduce
 
 
@@ -40,7 +41,7 @@ class ColumnParallelLinear(nn.Module):
         self.weight = nn.Parameter(w, requires_grad=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight)
+        return ops.linear(x, self.weight)
 
 
 class RowParallelLinear(nn.Module):
@@ -70,4 +71,4 @@ class ReplicatedLinear(nn.Module):
         self.weight = nn.Parameter(w, requires_grad=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return F.linear(x, self.weight)
+        return ops.linear(x, self.weight)

@@ -695,6 +695,51 @@ def test_sample_bf16_values(kind):
         _check_draw(logits[i], *settings[i], float(u[i]), got)
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("N,K,bias", [
+    (1, 8, True),          # one output, one lane
+    (3, 520, False),       # a ragged row group, a ragged piece of K
+    (64, 512, True),
+    (2050, 4104, False),
+    (16, 8192, True),      # the largest x of 8 rows
+    (40, 14336, False),    # of 4 rows
+    (8, 65536, False),     # of one
+    (9000, 1024, False),   # several groups per wave
+])
+def test_linear_few_rows(M, N, K, bias):
+    """fp32 products and sums, one rounding: within 2^-8 of the result and
+    the fp32 sums' K 2^-24 of the sum of magnitudes."""
+    g = torch.Generator().manual_seed(M * K)
+    x = torch.randn(M, K + 8, generator=g).to(torch.bfloat16)[:, :K]
+    w = torch.randn(N, K, generator=g).to(torch.bfloat16)
+    b = torch.randn(N, generator=g).to(torch.bfloat16) if bias else None
+    xg = torch.nn.functional.pad(x, (0, 8)).cuda()[:, :K]
+    out = ops.linear(xg, w.cuda(), None if b is None else b.cuda())
+    ref = x.double() @ w.double().t()
+    if bias:
+        ref = ref + b.double()
+    mag = x.double().abs() @ w.double().abs().t()
+    err = (out.double().cpu() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * ref.abs()
+                 + max(K, 64) * 2.0 ** -24 * mag + 1e-6).all())
+
+
+@pytest.mark.parametrize("M,F,K", [(1, 1, 8), (4, 77, 520), (6, 512, 4096),
+                                   (8, 3000, 1024), (8, 64, 8192),
+                                   (9, 64, 512)])
+def test_linear_silu_mul_few_rows(M, F, K):
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(2 * F, K, generator=g) * K ** -0.5).to(torch.bfloat16)
+    out = ops.linear_silu_mul(x.cuda(), w.cuda())
+    y = x.double() @ w.double().t()
+    ref = torch.nn.functional.silu(y[:, :F]) * y[:, F:]
+    # the separate activation also rounds both halves (2^-9 each, silu's
+    # slope is below 1.1)
+    torch.testing.assert_close(out.double().cpu(), ref, rtol=2.0 ** -7,
+                               atol=2.0 ** -8 * float(y.abs().max()) * 0.5)
+
+
 def test_zz_chunked_prefill_engine_matches_unchunked():
     # placed in this (alphabetically last) file, and named to sort last,
     # so the driver's -x run covers everything else first
