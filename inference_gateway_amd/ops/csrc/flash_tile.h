@@ -110,11 +110,12 @@ DEVINLINE bool ft_find_tile(const int32_t* cu, int B, int t, int* seq,
   return false;
 }
 
-// The key tiles of a workgroup, in order: [0, kept), then [first, end).
+// The key tiles of a workgroup, in order: [kept_from, kept), then [first, end).
 struct FlashSpan {
   int kv_len;            // keys of the sequence
   int kept, first, end;  // kept and first are multiples of FT_BN
-  DEVINLINE int begin() const { return kept > 0 ? 0 : first; }
+  int kept_from = 0;
+  DEVINLINE int begin() const { return kept > kept_from ? kept_from : first; }
   DEVINLINE int next(int kb) const {
     kb += FT_BN;
     return kb >= kept && kb < first ? first : kb;
@@ -201,13 +202,19 @@ DEVINLINE int ft_vswz(int r) {
 // 8 (i / 4) + 4 half + i % 4 of the lane's row, unnormalised; l the row's sum
 // and m its reference, in log2 (both lane halves alike).
 // PLAIN: causal only, the maximum is of raw scores.
-template <int NK, int NV, bool PLAIN, class Rows>
+// VD < NV: the four waves have the SAME 32 query rows and each the VD value
+// dims from dim0 on (decoded rows: the heads that share keys).
+// SHARED: the values are the first entries of the key rows, v0 and v1 unused.
+template <int NK, int NV, bool PLAIN, class Rows, int VD = NV,
+          bool SHARED = false>
 DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
                            const FlashScore& sc,
                            const ft_bf16x8 (&qf)[NK / 16], uint8_t* k0,
                            uint8_t* k1, uint8_t* v0, uint8_t* v1,
-                           ft_f32x16 (&o)[NV / 32], float& m, float& l) {
-  constexpr int BN = FT_BN, CK = NK / 8, CV = NV / 8;
+                           ft_f32x16 (&o)[VD / 32], float& m, float& l,
+                           int dim0 = 0) {
+  constexpr int BN = FT_BN, CK = NK / 8, CV = SHARED ? 0 : NV / 8;
+  constexpr int VROW = SHARED ? NK * 2 : NV * 2;   // bytes of a V row
   constexpr int RW = BN / FT_WAVES;   // rows that a wave moves
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -226,8 +233,9 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
     }
 #pragma unroll
     for (int i = 0; i < CV / 4; ++i) {
-      const int r = wave * RW + (i * 64 + lane) / CV;
-      const int c = ((i * 64 + lane) % CV) ^ ft_vswz<NV>(r);
+      constexpr int C = CV > 0 ? CV : 1;
+      const int r = wave * RW + (i * 64 + lane) / C;
+      const int c = ((i * 64 + lane) % C) ^ ft_vswz<NV>(r);
       __builtin_amdgcn_global_load_lds(
           reinterpret_cast<const uint32_t*>(rows.vp(r, c)),
           reinterpret_cast<uint32_t*>(vd + (wave * (CV / 4) + i) * 1024), 16,
@@ -241,22 +249,24 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
 #pragma unroll
   for (int s = 0; s < NK / 16; ++s)
     koff[s] = col * (NK * 2) + (((2 * s + half) ^ (col & 7)) << 4);
-  int voff[NV / 32][2];  // V^T: dims 32 dt + 16 (lane bit 4), keys 4 half + 8 e
+  int voff[VD / 32][2];  // V^T: dims 32 dt + 16 (lane bit 4), keys 4 half + 8 e
 #pragma unroll
-  for (int dt = 0; dt < NV / 32; ++dt)
+  for (int dt = 0; dt < VD / 32; ++dt)
 #pragma unroll
     for (int e = 0; e < 2; ++e) {
       const int i = lane & 15, r = 4 * half + 8 * e + (i >> 2);
-      const int c = 4 * dt + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
-      voff[dt][e] =
-          r * (NV * 2) + ((c ^ ft_vswz<NV>(r)) << 4) + 8 * (i & 1);
+      const int c =
+          dim0 / 8 + 4 * dt + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
+      voff[dt][e] = r * VROW +
+                    ((c ^ (SHARED ? r & 7 : ft_vswz<NV>(r))) << 4) +
+                    8 * (i & 1);
     }
 
   const ft_bf16x2 ones = {(__bf16)1.0f, (__bf16)1.0f};
   m = -INFINITY;
   l = 0.0f;  // this lane half's keys, until the end
 #pragma unroll
-  for (int dt = 0; dt < NV / 32; ++dt)
+  for (int dt = 0; dt < VD / 32; ++dt)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[dt][i] = 0.0f;
   // tanh by exp2: cap - 2 cap / (1 + 2^(cap_k s))
@@ -346,7 +356,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
       m = mn;
       l *= alpha;
 #pragma unroll
-      for (int dt = 0; dt < NV / 32; ++dt)
+      for (int dt = 0; dt < VD / 32; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
     }
@@ -377,7 +387,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
               __builtin_bit_cast(ft_bf16x2, pf.u[e]), ones, l, false);
         }
 #pragma unroll
-        for (int dt = 0; dt < NV / 32; ++dt) {
+        for (int dt = 0; dt < VD / 32; ++dt) {
           typedef __attribute__((address_space(3))) ft_short4 lds_short4;
           union {
             ft_short4 h[2];
@@ -386,7 +396,8 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
 #pragma unroll
           for (int e = 0; e < 2; ++e)
             vf.h[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (lds_short4*)(vb + voff[dt][e] + (32 * t + 16 * ks) * NV * 2));
+                (lds_short4*)((SHARED ? kb : vb) + voff[dt][e] +
+                              (32 * t + 16 * ks) * VROW));
           o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf.v, o[dt],
                                                           0, 0, 0);
         }
@@ -414,6 +425,30 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
   if (PLAIN) m *= sc.c;
 }
 
+// Decoded rows: a sequence's key tiles are cut for `nsplit` workgroups, the
+// part's unnormalised fp32 sums are merged by flash_merge_kernel.  Part `split`
+// of the tiles of a span (whose kept tiles come first).
+DEVINLINE FlashSpan flash_part(FlashSpan s, int split, int nsplit) {
+  if (nsplit == 1) return s;
+  const int kept = s.kept / FT_BN;
+  const int n = kept + (s.end - s.first + FT_BN - 1) / FT_BN;
+  const int per = (n + nsplit - 1) / nsplit;
+  const int a = min(split * per, n), b = min(a + per, n);
+  FlashSpan p = s;
+  // tile t of the walk starts at key 64 t, or behind the kept ones at first
+  p.first = a > kept ? s.first + (a - kept) * FT_BN : s.first;
+  p.end = b > kept ? min(s.end, s.first + (b - kept) * FT_BN) : s.first;
+  p.kept = 0;
+  if (a < kept) {          // [64 a, min(kept, 64 b)), then the rest
+    p.kept_from = a * FT_BN;
+    p.kept = min(b, kept) * FT_BN;
+    if (b <= kept) p.end = p.first = p.kept;   // nothing behind them
+  } else if (a == b) {
+    p.end = p.first;
+  }
+  return p;
+}
+
 // Stores the lane's dims d of an output row times f(d), 4 dims at a time; P
 // is the row's real width.
 template <int NV, class F>
@@ -432,6 +467,94 @@ DEVINLINE void flash_store(uint16_t* row, const ft_f32x16 (&o)[NV / 32], int P,
         *reinterpret_cast<uint2*>(row + d) = w;
       }
     }
+}
+
+// The unnormalised sums of decoded rows, one slot per (row, head, part).
+struct FlashParts {
+  float* o;    // [rows, heads, nsplit, width]
+  float* ml;   // [rows, heads, nsplit, 2]: reference (log2) and sum
+  int nsplit;
+};
+
+// Dims dim0 .. of the lane's row to a part's slot.
+template <int VD>
+DEVINLINE void flash_store_part(const FlashParts& p, int64_t pair, int split,
+                                int width, const ft_f32x16 (&o)[VD / 32],
+                                int dim0, float m, float l, int half) {
+  const int64_t slot = pair * p.nsplit + split;
+#pragma unroll
+  for (int dt = 0; dt < VD / 32; ++dt)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int d = dim0 + 32 * dt + 8 * g + 4 * half;
+      if (d < width)
+        *reinterpret_cast<float4*>(p.o + slot * width + d) =
+            make_float4(o[dt][4 * g], o[dt][4 * g + 1], o[dt][4 * g + 2],
+                        o[dt][4 * g + 3]);
+    }
+  if (dim0 == 0 && half == 0) {
+    p.ml[2 * slot] = m;
+    p.ml[2 * slot + 1] = l;
+  }
+}
+
+// What closes a decoded row: sink and gate per head (fp32) or a sigmoid gate
+// from bf16 logits, per head or per value.
+struct FlashClose {
+  uint16_t* out;           // [tokens, heads, width]
+  int heads, width;
+  const float* sinks;      // [heads]
+  const float* gate;       // [tokens, heads]
+  const uint16_t* logits;  // [tokens, heads * logit_w], row stride logits_rs
+  int64_t logits_rs;
+  int logit_w;
+  DEVINLINE float sum(int head, float m, float l) const {
+    return sinks ? l + __builtin_amdgcn_exp2f(fmaf(sinks[head], FT_LOG2E, -m))
+                 : l;
+  }
+  DEVINLINE float factor(int64_t tok, int head, int d) const {
+    float f = gate ? gate[tok * heads + head] : 1.0f;
+    if (logits) {
+      const float x = bf16_to_f32(logits[tok * logits_rs + head * logit_w +
+                                         (logit_w > 1 ? d : 0)]);
+      f *= __frcp_rn(1.0f + __expf(-x));
+    }
+    return f;
+  }
+};
+
+// One workgroup of width / 4 threads per (row, head); row r is token first + r.
+static __global__ void flash_merge_kernel(FlashClose c, FlashParts p,
+                                          int64_t first) {
+  const int64_t pair = blockIdx.x;
+  const int head = pair % c.heads;
+  const int64_t tok = first + pair / c.heads;
+  const int d = threadIdx.x * 4;
+  const float2* ml =
+      reinterpret_cast<const float2*>(p.ml) + pair * p.nsplit;
+  float m = -INFINITY;
+  for (int s = 0; s < p.nsplit; ++s) m = fmaxf(m, ml[s].x);
+  float l = 0.0f;
+  float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll 4
+  for (int s = 0; s < p.nsplit; ++s) {
+    const float2 v = ml[s];
+    const float4 a = *reinterpret_cast<const float4*>(
+        p.o + (pair * p.nsplit + s) * c.width + d);
+    const float f = v.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(v.x - m);
+    l = fmaf(f, v.y, l);
+    o.x = fmaf(f, a.x, o.x);
+    o.y = fmaf(f, a.y, o.y);
+    o.z = fmaf(f, a.z, o.z);
+    o.w = fmaf(f, a.w, o.w);
+  }
+  const float inv = 1.0f / c.sum(head, m, l);
+  uint2 w;
+  w.x = ft_pack_bf16(o.x * inv * c.factor(tok, head, d),
+                     o.y * inv * c.factor(tok, head, d + 1));
+  w.y = ft_pack_bf16(o.z * inv * c.factor(tok, head, d + 2),
+                     o.w * inv * c.factor(tok, head, d + 3));
+  *reinterpret_cast<uint2*>(c.out + (tok * c.heads + head) * c.width + d) = w;
 }
 
 }  // namespace igw

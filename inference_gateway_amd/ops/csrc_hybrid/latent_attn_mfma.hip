@@ -330,6 +330,13 @@ int64_t latent_attention_tile_rows(int64_t H) {
   return 64 / HB > 0 ? 64 / HB : 1;
 }
 
+bool latent_decode(torch::Tensor out, torch::Tensor q_abs,
+                   torch::Tensor q_rot, torch::Tensor cache,
+                   torch::Tensor block_table, torch::Tensor row_seq,
+                   torch::Tensor positions, c10::optional<torch::Tensor> sink,
+                   double scale, int64_t window, int64_t max_keys,
+                   c10::optional<torch::Tensor> gate);
+
 // returns false when the sizes do not fit this kernel (the caller then
 // runs latent_attention_rows)
 bool latent_attention_mfma(torch::Tensor out, torch::Tensor q_abs,
@@ -361,6 +368,11 @@ bool latent_attention_mfma(torch::Tensor out, torch::Tensor q_abs,
               tile_nrows.dtype() == torch::kInt32 &&
               tile_nrows.numel() == ntiles);
   if (T == 0 || ntiles == 0) return true;
+  // single decoded tokens have a kernel of their own for the usual ranks
+  if (ntiles == T && latent_decode(out, q_abs, q_rot, cache, block_table,
+                                   row_seq, positions, sink, scale, window,
+                                   max_keys, gate))
+    return true;
   const int CW = R + RD;
   const int ks_n = (CW + 31) / 32, nt_n = (R + 15) / 16;
   if (ks_n > 18 || nt_n > 32) return false;

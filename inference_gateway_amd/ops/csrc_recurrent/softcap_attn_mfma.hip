@@ -14,11 +14,11 @@
 //     optional sink term per head in the softmax denominator and an
 //     optional sigmoid output gate (per value entry or per head).
 //
-// Prompt rows with P <= 128 run the tile walk of flash_tile.h
-// (softcap_prompt_kernel: 128 rows of one head).  Decoded rows, and prompt
-// rows of wider values, whose accumulators do not fit two waves per SIMD
-// there, run softcap_attention_mfma_kernel: 64 rows x 64 keys, 4 waves of 16
-// rows, mfma_f32_16x16x32_bf16, K staged row-major and V transposed in
+// Values of at most 128 entries run the tile walk of flash_tile.h
+// (softcap_prompt_kernel: 128 rows of one head; softcap_decode_kernel: the
+// heads that share a key/value head).  Wider ones, whose accumulators do not
+// fit two waves per SIMD there, run softcap_attention_mfma_kernel: 64 rows x
+// 64 keys, 4 waves of 16 rows, mfma_f32_16x16x32_bf16, K staged row-major and V transposed in
 // swizzled LDS, probabilities through a per-wave LDS tile.  Its row maps:
 // prompt tiles (64 consecutive tokens of one head), and decoded rows
 // (HEADS_ROWS), where the rows of a tile are the query heads that share one
@@ -27,8 +27,10 @@
 //
 // Measured (32 heads on 8, N = P = 128), 64-row tiles for all and the tile
 // walk: prompts of 3000 and 2790 tokens, window 1024 with 16 kept tokens,
-// distance bias and head gate 563 and 198 us; 4 prompts of 2048, causal, with
-// a sink 1293 and 261 us, with a score cap 1412 and 285 us.
+// distance bias and head gate 563 and 159 us; 4 prompts of 2048, causal, with
+// a sink 1293 and 207 us, with a score cap 1412 and 247 us; decoded, 256
+// tokens of 2048 keys 863 and 396 us (5.4 TB/s), 48 of 700 to 3500 with that
+// window 103 and 48, one of 3000 181 and 17 (split over workgroups).
 //
 // Everything is read from the paged cache; a row's own key is already
 // appended.  Sequence s has rows [seq_cu[s], seq_cu[s+1]) whose first sits
@@ -437,6 +439,73 @@ __global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_prompt_kernel(
   }
 }
 
+// Decoded rows: the heads that share a key/value head (32 of them at most per
+// workgroup) are the 32 query rows of all four waves, which take a quarter of
+// the value dims each; no probabilities are exchanged, and scoring four times
+// costs less than HBM takes to deliver the keys.
+template <int NP>
+__global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_decode_kernel(
+    SoftcapArgs a, FlashClose close, FlashParts parts) {
+  constexpr int PP = 128, VD = PP / FT_WAVES;
+  __shared__ __attribute__((aligned(1024))) uint8_t k_s0[FT_BN * NP * 2];
+  __shared__ __attribute__((aligned(1024))) uint8_t k_s1[FT_BN * NP * 2];
+  __shared__ __attribute__((aligned(1024))) uint8_t v_s0[FT_BN * PP * 2];
+  __shared__ __attribute__((aligned(1024))) uint8_t v_s1[FT_BN * PP * 2];
+  const int lane = threadIdx.x & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int seq = a.nprompt + blockIdx.x;
+  const int rep = a.H / a.G;
+  const int kvh = blockIdx.y % a.G;
+  const int in_group = blockIdx.y / a.G * 32 + (lane & 31);
+  const bool real = in_group < rep;
+  const int head = kvh * rep + (real ? in_group : 0);
+  const int64_t tok = a.seq_cu[seq];
+  const int pos = a.seq_start[seq];
+
+  ft_bf16x8 qf[NP / 16];
+  const uint16_t* qp = a.q + tok * a.q_rs + (int64_t)head * a.N;
+#pragma unroll
+  for (int s = 0; s < NP / 16; ++s) {
+    const int d = 16 * s + 8 * half;
+    ft_bf16x8 f{};
+    if (real && d < a.N) f = *reinterpret_cast<const ft_bf16x8*>(qp + d);
+    qf[s] = f;
+  }
+  FlashScore sc{};
+  sc.pos = sc.wave_pos = pos;
+  sc.lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  if (a.chunk > 0) sc.lo = max(sc.lo, pos / a.chunk * a.chunk);
+  sc.wave_lo[0] = sc.wave_lo[1] = sc.lo;
+  sc.keep = a.keep;
+  sc.c = a.scale * FT_LOG2E *
+         (1.0f +
+          a.temp_coef * logf((float)((pos + 1) / a.temp_every) + 1.0f));
+  sc.cap = a.softcap > 0.0f ? a.softcap * FT_LOG2E : 0.0f;
+  sc.slope = a.slopes ? a.slopes[head] * FT_LOG2E : 0.0f;
+  FlashSpan span{pos + 1, 0, sc.lo / FT_BN * FT_BN, pos + 1};
+  span.kept =
+      a.keep > 0 ? min((a.keep + FT_BN - 1) / FT_BN * FT_BN, span.first) : 0;
+  span = flash_part(span, blockIdx.z, parts.nsplit);
+  PagedRows rows{a.kcache, a.vcache,
+                 a.block_table + (int64_t)seq * a.max_blocks, kvh, a.G, a.BS,
+                 a.N, a.P, pos + 1};
+  ft_f32x16 o[VD / 32];
+  float m, l;
+  flash_tiles<NP, PP, false, PagedRows, VD>(rows, span, sc, qf, k_s0, k_s1,
+                                            v_s0, v_s1, o, m, l, wave * VD);
+  if (!real) return;
+  if (parts.nsplit > 1) {
+    flash_store_part<VD>(parts, (int64_t)blockIdx.x * a.H + head, blockIdx.z,
+                         a.P, o, wave * VD, m, l, half);
+    return;
+  }
+  const float inv = 1.0f / close.sum(head, m, l);
+  flash_store<VD>(a.out + (tok * a.H + head) * a.P + wave * VD, o,
+                  a.P - wave * VD, half, [&](int d) {
+                    return inv * close.factor(tok, head, wave * VD + d);
+                  });
+}
+
 // prompt_rows: row counts of the first sequences of the batch; the other
 // sequences bring one decoded row each.  Returns false when the sizes do not
 // fit the tile kernels.
@@ -527,12 +596,46 @@ bool softcap_attention_mfma(torch::Tensor out, torch::Tensor q,
     else LAUNCH_SA(128, 256, false, dim3(tiles(SA_BM), H));
     HIP_CHECK_KERNEL();
   }
-  if (ndec > 0) {
-    if (N <= 64 && P <= 64) LAUNCH_SA(64, 64, true, dim3(ndec, G));
-    else if (N <= 64 && P <= 128) LAUNCH_SA(64, 128, true, dim3(ndec, G));
-    else if (N <= 64) LAUNCH_SA(64, 256, true, dim3(ndec, G));
-    else if (P <= 64) LAUNCH_SA(128, 64, true, dim3(ndec, G));
-    else if (P <= 128) LAUNCH_SA(128, 128, true, dim3(ndec, G));
+  if (ndec > 0 && P <= 128) {
+    const int64_t groups = (int64_t)G * ((H / G + 31) / 32);
+    // two workgroups per compute unit; a part has at least four tiles of the
+    // longest context that the block table holds
+    const int64_t cus =
+        at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
+    const int64_t longest = (int64_t)a.max_blocks * BS;
+    const int64_t keys =
+        window > 0 ? std::min<int64_t>(longest, window + keep) : longest;
+    const int64_t nsplit = std::max<int64_t>(
+        1, std::min<int64_t>({32, 2 * cus / std::max<int64_t>(1, ndec * groups),
+                              keys / (4 * FT_BN)}));
+    const FlashClose close{a.out, H, P, a.sinks, nullptr, a.gate, a.gate_rs,
+                           gate_w};
+    FlashParts parts{nullptr, nullptr, (int)nsplit};
+    torch::Tensor part;
+    if (nsplit > 1) {
+      const int64_t slots = (int64_t)ndec * H * nsplit;
+      part = torch::empty({slots * (P + 2)},
+                          q.options().dtype(torch::kFloat32));
+      parts.o = part.data_ptr<float>();
+      parts.ml = parts.o + slots * P;
+    }
+    const dim3 grid(ndec, groups, nsplit), block(64 * FT_WAVES);
+    if (N <= 64)
+      hipLaunchKernelGGL(softcap_decode_kernel<64>, grid, block, 0, stream, a,
+                         close, parts);
+    else
+      hipLaunchKernelGGL(softcap_decode_kernel<128>, grid, block, 0, stream, a,
+                         close, parts);
+    HIP_CHECK_KERNEL();
+    if (nsplit > 1) {
+      // decoded rows are the last rows of the batch
+      hipLaunchKernelGGL(flash_merge_kernel, dim3((int64_t)ndec * H),
+                         dim3(P / 4), 0, stream, close, parts,
+                         (int64_t)(T - ndec));
+      HIP_CHECK_KERNEL();
+    }
+  } else if (ndec > 0) {
+    if (N <= 64) LAUNCH_SA(64, 256, true, dim3(ndec, G));
     else LAUNCH_SA(128, 256, true, dim3(ndec, G));
     HIP_CHECK_KERNEL();
   }

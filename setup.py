@@ -38,7 +38,8 @@ recurrent_sources = [str(REC / "bindings.cpp")] + _hip_sources(REC) + [str(HYB /
 PN = ROOT / "inference_gateway_amd" / "ops" / "csrc_postnorm"
 postnorm_sources = [str(PN / "bindings.cpp")] + [
     str(HYB / f) for f in ("hybrid_ops.hip", "latent_attn.hip",
-                           "latent_attn_mfma.hip", "latent_prompt.hip",
+                           "latent_attn_mfma.hip", "latent_decode.hip",
+                           "latent_prompt.hip",
                            "parallel_ops.hip")] + [
     str(REC / f) for f in ("qk_rope_append.hip", "sandwich_ops.hip",
                            "softcap_attn.hip", "softcap_attn_mfma.hip")]
@@ -48,7 +49,8 @@ postnorm_sources = [str(PN / "bindings.cpp")] + [
 STR = ROOT / "inference_gateway_amd" / "ops" / "csrc_streams"
 streams_sources = [str(STR / "bindings.cpp")] + _hip_sources(STR) + [
     str(HYB / f) for f in ("hybrid_ops.hip", "latent_attn.hip",
-                           "latent_attn_mfma.hip", "latent_prompt.hip",
+                           "latent_attn_mfma.hip", "latent_decode.hip",
+                           "latent_prompt.hip",
                            "parallel_ops.hip")] + [
     str(REC / f) for f in ("qk_rope_append.hip", "recurrent_ops.hip",
                            "softcap_attn.hip", "softcap_attn_mfma.hip")]

@@ -639,6 +639,90 @@ def test_latent_written_out_matches_absorbed(design):
     assert torch.equal(c, d)
 
 
+@pytest.mark.parametrize("ctx,H,R,rd,bs,kw", [
+    ([1, 63, 64, 65, 700], 32, 512, 64, 16, dict(gate=True)),
+    ([2000], 32, 512, 64, 16, {}),                  # cut into parts
+    ([300, 1500], 16, 256, 64, 16, dict(sink=True)),
+    ([130, 900], 40, 512, 32, 16, dict(window=100, sink=True, gate=True)),
+    ([400], 8, 256, 8, 4, dict(window=250)),
+    ([70] * 300, 4, 256, 64, 16, {}),               # not cut
+])
+def test_latent_decode(ctx, H, R, rd, bs, kw):
+    g = torch.Generator().manual_seed(sum(ctx))
+    T, need = len(ctx), [-(-c // bs) for c in ctx]
+
+    def t(*shape):
+        return torch.randn(*shape, generator=g).to(torch.bfloat16)
+
+    cache = t(sum(need) + 1, bs, R + rd)
+    order = torch.randperm(sum(need), generator=g).to(torch.int32) + 1
+    bt = torch.zeros(T, max(need), dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    # scores of about unit variance
+    qa, qr = t(H, T, R).transpose(0, 1), t(T, H, rd)
+    sink = torch.randn(H, generator=g) if kw.get("sink") else None
+    gate = torch.rand(T, H, generator=g) if kw.get("gate") else None
+    row_seq = torch.arange(T, dtype=torch.int32)
+    pos = torch.tensor(ctx, dtype=torch.int32) - 1
+    scale, window = (R + rd) ** -0.5, kw.get("window", 0)
+    ref = torch_ref.latent_attention_ref(qa, qr, cache, bt, row_seq, pos,
+                                         sink, scale, window, gate)
+    out = ops.latent_attention(
+        qa.cuda(), qr.cuda(), cache.cuda(), bt.cuda(), row_seq.cuda(),
+        pos.cuda(), None if sink is None else sink.cuda(), scale, window,
+        max_context=max(ctx), gate=None if gate is None else gate.cuda())
+    torch.testing.assert_close(out.float().cpu(), ref.float(),
+                               atol=_attention_bound(cache), rtol=2.0 ** -8)
+
+
+@pytest.mark.parametrize("ctx,H,G,N,P,bs,kw", [
+    ([1, 16, 64, 65, 333], 8, 2, 128, 128, 16, dict(sinks=True)),
+    ([3000], 8, 8, 64, 64, 16, dict(softcap=30.0)),           # cut
+    ([5000, 40], 4, 1, 128, 72, 16, dict(window=700, keep=130, slopes=True,
+                                         gate=1)),
+    ([900, 20], 4, 2, 24, 16, 4, dict(chunk=64, gate=2, sinks=True)),
+    ([200], 40, 1, 128, 128, 16, {}),                         # two head groups
+    ([700, 100], 6, 3, 96, 136, 16, dict(gate=2)),            # wide values
+    ([100] * 80, 16, 8, 128, 128, 16, {}),                    # not cut
+    ([2000] * 3, 8, 8, 128, 128, 16, dict(window=64, keep=1)),
+])
+def test_softcap_decode(ctx, H, G, N, P, bs, kw):
+    kw = dict(kw)
+    g = torch.Generator().manual_seed(sum(ctx))
+    T, need = len(ctx), [-(-c // bs) for c in ctx]
+    kc, vc = (torch.randn(sum(need) + 1, G, bs, w, generator=g).to(
+        torch.bfloat16) for w in (N, P))
+    order = torch.randperm(sum(need), generator=g).to(torch.int32) + 1
+    bt = torch.zeros(T, max(need), dtype=torch.int32)
+    at = 0
+    for i, n in enumerate(need):
+        bt[i, :n] = order[at:at + n]
+        at += n
+    q = torch.randn(T, H * N, generator=g).to(torch.bfloat16)
+    ar = torch.arange(T + 1, dtype=torch.int32)
+    pos = torch.tensor(ctx, dtype=torch.int32) - 1
+    opt = dict(slopes=torch.rand(H, generator=g) * 0.02
+               if kw.pop("slopes", False) else None,
+               sinks=torch.randn(H, generator=g)
+               if kw.pop("sinks", False) else None)
+    gate = kw.pop("gate", 0)
+    opt["gate"] = torch.randn(T, H * (P if gate == 2 else 1), generator=g).to(
+        torch.bfloat16) if gate else None
+
+    def run(dev, **more):
+        a = [t.to(dev) for t in (q, kc, vc, bt, ar[:T], pos)]
+        o = {k: None if v is None else v.to(dev) for k, v in opt.items()}
+        return ops.softcap_attention(*a, N ** -0.5, **kw, **o, **more)
+
+    ref = run("cpu")
+    out = run("cuda", seq_cu=ar.cuda(), seq_start=pos.cuda())
+    torch.testing.assert_close(out.float().cpu(), ref.float(),
+                               atol=_attention_bound(vc), rtol=2.0 ** -8)
+
+
 @pytest.mark.parametrize("V", [
     1, 7, 8, 9, 4095, 4096, 4097,          # chunks and their tails
     32767, 32768, 32769,                   # 8 chunks, the first of 16
