@@ -295,6 +295,37 @@ def moe_grouped_gemm(a: torch.Tensor, w: torch.Tensor,
     return torch_ref.moe_grouped_gemm_ref(a, w, counts, capacity)
 
 
+def moe_few_fits(x: torch.Tensor, gate_up: torch.Tensor,
+                 down: torch.Tensor, top_k: int) -> bool:
+    """Whether moe_few takes this step: a few bf16 tokens on the GPU, a top_k
+    that moe_route has."""
+    return (x.is_cuda and HAS_KERNELS and x.dim() == 2
+            and top_k in (1, 2, 4, 8)
+            and all(t.dtype == torch.bfloat16 and t.is_contiguous()
+                    and t.data_ptr() % 16 == 0 for t in (x, gate_up, down))
+            and bool(_kernels.moe_few_fits(x.shape[0], top_k, x.shape[1],
+                                           down.shape[2])))
+
+
+def moe_few(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor,
+            topk_idx: torch.Tensor, weights: torch.Tensor) -> torch.Tensor:
+    """SwiGLU experts of a few tokens, only the chosen ones read: x [T, D],
+    gate_up [E, 2 F, D], down [E, D, F], topk_idx int32 and weights fp32 [T,
+    K]; returns sum_k weights * expert(x) [T, D]."""
+    if x.is_cuda:
+        _require_kernels()
+        out = torch.empty_like(x)
+        _kernels.moe_few(out, x, gate_up, down, topk_idx, weights)
+        return out
+    out = torch.zeros(x.shape, dtype=torch.float32)
+    for t in range(x.shape[0]):
+        for e, w in zip(topk_idx[t].tolist(), weights[t].tolist()):
+            g, u = (gate_up[e].float() @ x[t].float()).chunk(2)
+            out[t] += w * (down[e].float()
+                           @ (torch.nn.functional.silu(g) * u))
+    return out.to(x.dtype)
+
+
 def silu_mul_grouped(gate_up: torch.Tensor, counts: torch.Tensor,
                      capacity: int) -> torch.Tensor:
     """SwiGLU over only the real rows of the padded dispatch buffer."""

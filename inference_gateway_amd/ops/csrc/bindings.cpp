@@ -32,6 +32,9 @@ void flash_prefill_paged(torch::Tensor out, torch::Tensor q,
 void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
           c10::optional<torch::Tensor> bias, bool swiglu);
 bool gemv_fits(int64_t M, int64_t K, bool swiglu);
+bool moe_few_fits(int64_t T, int64_t top_k, int64_t D, int64_t F);
+void moe_few(torch::Tensor out, torch::Tensor x, torch::Tensor gate_up,
+             torch::Tensor down, torch::Tensor idx, torch::Tensor weight);
 void sample(torch::Tensor out, torch::Tensor logits, torch::Tensor temperature,
             torch::Tensor top_k, torch::Tensor top_p, torch::Tensor uniforms);
 void silu_mul(torch::Tensor out, torch::Tensor gate_up);
@@ -75,6 +78,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "varlen causal MFMA flash-attention prefill (bf16, gfx950)");
   m.def("gemv", &igw::gemv,
         "x W^T for a few rows of x, optional bias or SwiGLU");
+  m.def("moe_few", &igw::moe_few, "SwiGLU experts of a few tokens");
+  m.def("moe_few_fits", &igw::moe_few_fits, "whether moe_few takes these");
   m.def("gemv_fits", &igw::gemv_fits, "whether gemv takes these sizes");
   m.def("flash_prefill_paged", &igw::flash_prefill_paged,
         "paged-extend prefill: chunk queries over cached prefix+chunk K/V "

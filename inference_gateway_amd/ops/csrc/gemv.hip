@@ -33,23 +33,22 @@ constexpr int GV_WAVES = 8;
 constexpr int GV_ROWS = 2;              // of W per wave (SWIGLU: gate and up)
 constexpr int64_t GV_MAX_X = 64 * 1024; // entries of x: 128 KB of LDS
 
-template <int M, int R, bool SWIGLU>
-__global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
-    uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
-    const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
-    int rows, int N, int K, int64_t x_rs) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t xs[];   // [M][K]
-  // 16-byte loads in flight per row and lane: what 128 registers leave room
-  // for (two workgroups per compute unit)
-  constexpr int GV_U = M <= 3 ? 8 : 4;
+// A wave's walk over the row groups first, first + stride, ... of W [N (or 2
+// N), K] against the M rows of x in LDS.  stage() puts x there, after the
+// first rows of W have been asked for; store(n, sums of W row n, of its up
+// row) is called by lane 0.
+// U is the 16-byte loads in flight per row and lane: what 128 registers leave
+// room for (two workgroups per compute unit).
+template <int M, int R, int U, bool SWIGLU, class Stage, class Store>
+DEVINLINE void gemv_walk(const uint16_t* xs, const uint16_t* __restrict__ w,
+                         int N, int K, int first, int stride, Stage stage,
+                         Store store) {
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int chunks = (K + 511) >> 9;
   constexpr int STEP = SWIGLU ? R / 2 : R;   // output columns per group
   const int groups = (N + STEP - 1) / STEP;
-  const int stride = gridDim.x * GV_WAVES;
 
-  uint4 buf[R][GV_U];
+  uint4 buf[R][U];
   auto load = [&](int grp, int c0) {
 #pragma unroll
     for (int t = 0; t < R; ++t) {
@@ -57,7 +56,7 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
       n = min(n, N - 1) + (SWIGLU && t >= STEP ? N : 0);
       const uint16_t* row = w + (int64_t)n * K;
 #pragma unroll
-      for (int u = 0; u < GV_U; ++u) {
+      for (int u = 0; u < U; ++u) {
         const int k = ((c0 + u) << 9) + lane * 8;
         uint4 v = {0, 0, 0, 0};
         if (k < K) {
@@ -70,33 +69,19 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
       }
     }
   };
-  // x to LDS, linearly, all of it in flight at once; a 1 KB piece may cross
-  // rows, lanes past the end repeat the last entries
-  const int total = M * K;
-  for (int base = wave * 512; base < total; base += GV_WAVES * 512) {
-    const int i = min(base + lane * 8, total - 8);
-    const int m = i / K;
-    __builtin_amdgcn_global_load_lds(
-        reinterpret_cast<const uint32_t*>(x + min(m, rows - 1) * x_rs +
-                                          (i - m * K)),
-        reinterpret_cast<uint32_t*>(xs + base), 16, 0, 0);
-  }
-  int grp = blockIdx.x * GV_WAVES + wave;
-  // the first rows of W are on their way meanwhile
-  if (grp < groups) load(grp, 0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
+  if (first < groups) load(first, 0);
+  stage();
 
-  for (; grp < groups; grp += stride) {
+  for (int grp = first; grp < groups; grp += stride) {
     float acc[R][M];
 #pragma unroll
     for (int t = 0; t < R; ++t)
 #pragma unroll
       for (int m = 0; m < M; ++m) acc[t][m] = 0.0f;
-    for (int c0 = 0; c0 < chunks; c0 += GV_U) {
-      if (!(c0 == 0 && grp < stride)) load(grp, c0);
+    for (int c0 = 0; c0 < chunks; c0 += U) {
+      if (c0 > 0 || grp > first) load(grp, c0);
 #pragma unroll
-      for (int u = 0; u < GV_U; ++u) {
+      for (int u = 0; u < U; ++u) {
         const int k = ((c0 + u) << 9) + lane * 8;
         if (((c0 + u) << 9) >= K) break;
         const int kx = k < K ? k : 0;   // W is zero there
@@ -120,21 +105,216 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
       for (int m = 0; m < M; ++m) acc[t][m] = wave_reduce_sum(acc[t][m]);
     if (lane == 0) {
 #pragma unroll
-      for (int t = 0; t < STEP; ++t) {
-        const int n = grp * STEP + t;
-        if (n < N) {
-#pragma unroll
-          for (int m = 0; m < M; ++m) {
-            if (m >= rows) break;
-            float y = acc[t][m];
-            if (SWIGLU) y = y / (1.0f + __expf(-y)) * acc[t + STEP][m];
-            else if (bias) y += bf16_to_f32(bias[n]);
-            out[(int64_t)m * N + n] = f32_to_bf16(y);
-          }
-        }
-      }
+      for (int t = 0; t < STEP; ++t)
+        if (grp * STEP + t < N)
+          store(grp * STEP + t, acc[t], acc[SWIGLU ? t + STEP : t]);
     }
   }
+}
+
+// Rows of x to LDS, linearly, all of it in flight at once; row(m) is the m-th
+// row.  A 1 KB piece may cross rows, lanes past the end repeat the last
+// entries.
+template <class Row>
+DEVINLINE void gemv_stage(uint16_t* xs, int total, int K, Row row) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (int base = wave * 512; base < total; base += GV_WAVES * 512) {
+    const int i = min(base + lane * 8, total - 8);
+    const int m = i / K;
+    __builtin_amdgcn_global_load_lds(
+        reinterpret_cast<const uint32_t*>(row(m) + (i - m * K)),
+        reinterpret_cast<uint32_t*>(xs + base), 16, 0, 0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+}
+
+template <int M, int R, bool SWIGLU>
+__global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
+    uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
+    const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
+    int rows, int N, int K, int64_t x_rs) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t xs[];   // [M][K]
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  gemv_walk<M, R, M <= 3 ? 8 : 4, SWIGLU>(
+      xs, w, N, K, blockIdx.x * GV_WAVES + wave, gridDim.x * GV_WAVES,
+      [&] {
+        gemv_stage(xs, M * K, K,
+                   [&](int m) { return x + min(m, rows - 1) * x_rs; });
+      },
+      [&](int n, const float* a, const float* up) {
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          if (m >= rows) break;
+          float y = a[m];
+          if (SWIGLU) y = y / (1.0f + __expf(-y)) * up[m];
+          else if (bias) y += bf16_to_f32(bias[n]);
+          out[(int64_t)m * N + n] = f32_to_bf16(y);
+        }
+      });
+}
+
+// ---------------------------------------------------------------------------
+// Experts of a small decode step.  Assignment a = t K + k sends token t to
+// expert idx[a]; blockIdx.y is the expert, an expert without a token is not
+// read (a batched product over all experts reads every one of them).  The
+// assignments of an expert are found from the list, in passes of as many rows
+// as LDS holds (more than one pass only where many tokens meet wide rows).
+//
+// SWIGLU: out [T K, N] bf16 = silu(x_t Wg^T) * (x_t Wu^T).  Otherwise: in is
+// [T K, K] and sums [T K, N] fp32 = weight_a * in_a W^T.
+//
+// Bound by streaming the chosen experts' weights.  Measured from the hidden
+// rows to the combined ones, 8 experts of 14336 x 4096 in bf16, two per token
+// (us; batched products over the padded rows of all experts, here): 1 token
+// 588 and 136, 2 589 and 259, 5 600 and 397 (six experts reached), 8 612 and
+// 489 (5.8 TB/s).
+constexpr int GV_ASSIGN = 64;   // assignments a step may have
+
+template <bool SWIGLU>
+__global__ __launch_bounds__(64 * GV_WAVES, 4) void expert_gemv_kernel(
+    uint16_t* __restrict__ out, float* __restrict__ sums,
+    const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
+    const int32_t* __restrict__ idx, const float* __restrict__ weight,
+    int assigned, int top_k, int N, int K, int64_t in_rs, int max_rows) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t xs[];
+  __shared__ int list[GV_ASSIGN];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int e = blockIdx.y;
+  const bool mine = lane < assigned && idx[lane] == e;
+  const uint64_t all = __ballot(mine);
+  if (all == 0) return;
+  const int count = __popcll(all);
+  if (wave == 0 && mine)
+    list[__popcll(all & ((1ull << lane) - 1))] = lane;
+  __syncthreads();
+  w += (int64_t)e * (SWIGLU ? 2 * N : N) * K;
+
+  for (int at = 0; at < count; at += max_rows) {
+    const int rows = min(max_rows, count - at);
+    auto pass = [&](auto m_) {
+      constexpr int M = decltype(m_)::value;
+      gemv_walk<M, GV_ROWS, 4, SWIGLU>(
+          xs, w, N, K, blockIdx.x * GV_WAVES + wave, gridDim.x * GV_WAVES,
+          [&] {
+            gemv_stage(xs, rows * K, K, [&](int m) {
+              const int a = list[at + m];
+              return in + (SWIGLU ? a / top_k : a) * in_rs;
+            });
+          },
+          [&](int n, const float* y, const float* up) {
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+              if (m >= rows) break;
+              const int64_t a = list[at + m];
+              if (SWIGLU)
+                out[a * N + n] =
+                    f32_to_bf16(y[m] / (1.0f + __expf(-y[m])) * up[m]);
+              else
+                sums[a * N + n] = weight[a] * y[m];
+            }
+          });
+    };
+    if (rows == 1) pass(std::integral_constant<int, 1>{});
+    else if (rows == 2) pass(std::integral_constant<int, 2>{});
+    else if (rows <= 4) pass(std::integral_constant<int, 4>{});
+    else pass(std::integral_constant<int, 8>{});
+    __syncthreads();   // x is replaced by the next pass
+  }
+}
+
+__global__ void expert_combine_kernel(uint16_t* __restrict__ out,
+                                      const float* __restrict__ sums, int N,
+                                      int top_k) {
+  const int64_t t = blockIdx.y;
+  const int n = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  if (n >= N) return;
+  float4 y = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int k = 0; k < top_k; ++k) {
+    const float4 v =
+        *reinterpret_cast<const float4*>(sums + (t * top_k + k) * N + n);
+    y.x += v.x;
+    y.y += v.y;
+    y.z += v.z;
+    y.w += v.w;
+  }
+  ushort4x o;
+  o.v[0] = f32_to_bf16(y.x);
+  o.v[1] = f32_to_bf16(y.y);
+  o.v[2] = f32_to_bf16(y.z);
+  o.v[3] = f32_to_bf16(y.w);
+  *reinterpret_cast<ushort4x*>(out + t * N + n) = o;
+}
+
+// Most tokens that moe_few takes.  With more of them the experts that many
+// tokens share are read once per pass: at 16 tokens 540 us against 594 where
+// the router spreads them and 714 where it does not, at 8 it is ahead either
+// way (409 to 489 against 612).
+constexpr int64_t GV_MOE_TOKENS = 8;
+
+bool moe_few_fits(int64_t T, int64_t top_k, int64_t D, int64_t F) {
+  return T >= 1 && T <= GV_MOE_TOKENS && T * top_k <= GV_ASSIGN &&
+         D >= 8 && F >= 8 && D % 8 == 0 && F % 8 == 0 && D <= GV_MAX_X &&
+         F <= GV_MAX_X;
+}
+
+// out [T, D] = sum over a token's experts of weight * down(silu(gate) * up):
+// x [T, D], gate_up [E, 2 F, D], down [E, D, F], idx and weight [T, K] (int32,
+// fp32).
+void moe_few(torch::Tensor out, torch::Tensor x, torch::Tensor gate_up,
+             torch::Tensor down, torch::Tensor idx, torch::Tensor weight) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() &&
+              gate_up.dim() == 3 && down.dim() == 3 && idx.dim() == 2);
+  for (auto* t : {&out, &x, &gate_up, &down})
+    TORCH_CHECK(t->dtype() == torch::kBFloat16 && t->is_contiguous() &&
+                (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) == 0);
+  const int64_t T = x.size(0), D = x.size(1), E = gate_up.size(0);
+  const int64_t F = down.size(2), top_k = idx.size(1);
+  TORCH_CHECK(moe_few_fits(T, top_k, D, F) && out.sizes() == x.sizes() &&
+              gate_up.size(1) == 2 * F && gate_up.size(2) == D &&
+              down.size(0) == E && down.size(1) == D && idx.size(0) == T);
+  TORCH_CHECK(idx.dtype() == torch::kInt32 && idx.is_contiguous() &&
+              weight.dtype() == torch::kFloat32 && weight.is_contiguous() &&
+              weight.numel() == T * top_k);
+  const int64_t n = T * top_k;
+  auto act = torch::empty({n, F}, x.options());
+  auto sums = torch::empty({n, D}, x.options().dtype(torch::kFloat32));
+  hipStream_t stream = at::cuda::getCurrentCUDAStream();
+  // two workgroups per compute unit for the experts that n draws are
+  // expected to reach
+  const double reached = E * (1.0 - std::pow(1.0 - 1.0 / E, (double)n));
+  const int64_t per = std::max<int64_t>(1, (int64_t)(512.0 / reached));
+  auto launch = [&](auto kern, int64_t K, int64_t cols, int64_t group,
+                    const torch::Tensor& in, const torch::Tensor& w) {
+    // a power of two, as the kernel rounds the rows of a pass up to one
+    int64_t rows = 1;
+    while (rows < std::min<int64_t>(T, 8) && 2 * rows * K <= GV_MAX_X)
+      rows *= 2;
+    const size_t shmem = (size_t)(rows * K + 511) / 512 * 1024;
+    if (shmem > 64 * 1024)
+      TORCH_CHECK(hipFuncSetAttribute(
+                      (const void*)kern,
+                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                      (int)shmem) == hipSuccess);
+    const int64_t need = (cols / group + GV_WAVES) / GV_WAVES;
+    hipLaunchKernelGGL(kern, dim3(std::min(per, need), E),
+                       dim3(64 * GV_WAVES), shmem, stream,
+                       (uint16_t*)act.data_ptr(), sums.data_ptr<float>(),
+                       (const uint16_t*)in.data_ptr(),
+                       (const uint16_t*)w.data_ptr(),
+                       (const int32_t*)idx.data_ptr(),
+                       (const float*)weight.data_ptr(), (int)n, (int)top_k,
+                       (int)cols, (int)K, K, (int)rows);
+    HIP_CHECK_KERNEL();
+  };
+  launch(expert_gemv_kernel<true>, D, F, GV_ROWS / 2, x, gate_up);
+  launch(expert_gemv_kernel<false>, F, D, GV_ROWS, act, down);
+  hipLaunchKernelGGL(expert_combine_kernel, dim3((D / 4 + 255) / 256, T),
+                     dim3(256), 0, stream, (uint16_t*)out.data_ptr(),
+                     sums.data_ptr<float>(), (int)D, (int)top_k);
+  HIP_CHECK_KERNEL();
 }
 
 // Whether gemv takes M rows of x with K entries against this many outputs.

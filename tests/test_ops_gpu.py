@@ -824,6 +824,40 @@ def test_linear_silu_mul_few_rows(M, F, K):
                                atol=2.0 ** -8 * float(y.abs().max()) * 0.5)
 
 
+@pytest.mark.parametrize("T,K,E,D,F,same", [
+    (1, 1, 1, 8, 8, False), (1, 2, 8, 4096, 14336, False),
+    (5, 2, 8, 520, 1000, False), (8, 2, 8, 512, 14336, True),
+    (8, 8, 64, 64, 136, False), (7, 4, 5, 16384, 24, True),
+    (3, 2, 2, 40, 65536, True)])
+def test_moe_few(T, K, E, D, F, same):
+    # same: every token picks the same experts, which takes several passes
+    # over their weights where the rows are wide
+    g = torch.Generator().manual_seed(T + D)
+    x = torch.randn(T, D, generator=g).to(torch.bfloat16)
+    gu = (torch.randn(E, 2 * F, D, generator=g) * D ** -0.5).to(torch.bfloat16)
+    dn = (torch.randn(E, D, F, generator=g) * F ** -0.5).to(torch.bfloat16)
+    if same:
+        idx = torch.randperm(E, generator=g)[:K].expand(T, K)
+    else:
+        idx = torch.stack([torch.randperm(E, generator=g)[:K]
+                           for _ in range(T)])
+    idx = idx.to(torch.int32).contiguous()
+    w = torch.rand(T, K, generator=g)
+    assert ops.moe_few_fits(x.cuda(), gu.cuda(), dn.cuda(), K)
+    out = ops.moe_few(x.cuda(), gu.cuda(), dn.cuda(), idx.cuda(), w.cuda())
+    ref = torch.zeros(T, D, dtype=torch.float64)
+    mag = torch.zeros_like(ref)
+    for t in range(T):
+        for e, c in zip(idx[t].tolist(), w[t].tolist()):
+            y = gu[e].double() @ x[t].double()
+            a = torch.nn.functional.silu(y[:F]) * y[F:]
+            ref[t] += c * (dn[e].double() @ a)
+            mag[t] += c * (dn[e].double().abs() @ a.abs())
+    # the result and each activation are rounded to bf16 (2^-9 each)
+    err = (out.double().cpu() - ref).abs()
+    assert bool((err <= 2.0 ** -8 * (ref.abs() + mag) + 1e-6).all())
+
+
 def test_zz_chunked_prefill_engine_matches_unchunked():
     # placed in this (alphabetically last) file, and named to sort last,
     # so the driver's -x run covers everything else first
