@@ -858,6 +858,32 @@ def test_moe_few(T, K, E, D, F, same):
     assert bool((err <= 2.0 ** -8 * (ref.abs() + mag) + 1e-6).all())
 
 
+@pytest.mark.parametrize("D", [4, 1020, 1024, 1028, 2052, 4096, 8188, 8192,
+                               8196, 4098])
+@pytest.mark.parametrize("dtype,pad", [(torch.bfloat16, 4),
+                                       (torch.bfloat16, 3),
+                                       (torch.float32, 8)])
+def test_add_normed_rmsnorm_rows(D, dtype, pad):
+    # rows kept in registers and rows read again: same formula, either side
+    # of the lengths and alignments where one takes over from the other
+    g = torch.Generator().manual_seed(D + pad)
+    res = torch.randn(3, D, generator=g) * 3
+    delta = (torch.randn(3, D + pad, generator=g) * 7).to(dtype)
+    wp, wn = torch.randn(D, generator=g), torch.randn(D, generator=g)
+    d = delta[:, :D].double()
+    r = res.double() + 0.5 * d * wp.double() / (
+        d.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    ref = r * wn.double() / (r.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+    x = res.cuda()
+    out = ops.add_normed_rmsnorm(x, delta.cuda()[:, :D], wp.cuda(), wn.cuda(),
+                                 1e-5, dtype, 0.5)
+    torch.testing.assert_close(x.double().cpu(), r, atol=2e-5, rtol=2e-5)
+    tol = 2e-5 if dtype == torch.float32 else 2.0 ** -8
+    torch.testing.assert_close(out.double().cpu(), ref, atol=2e-5, rtol=tol)
+    same = ops.add_normed_rmsnorm(x, None, None, None, 1e-5, torch.float32)
+    torch.testing.assert_close(same, x, atol=0, rtol=0)
+
+
 def test_zz_chunked_prefill_engine_matches_unchunked():
     # placed in this (alphabetically last) file, and named to sort last,
     # so the driver's -x run covers everything else first
