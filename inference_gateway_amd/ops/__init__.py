@@ -205,26 +205,36 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_mul_ref(gate_up)
 
 
-def _gemv_takes(x, w, swiglu: bool) -> bool:
-    return (x.is_cuda and HAS_KERNELS and x.dim() == 2 and w.dim() == 2
-            and x.shape[0] <= 8 and x.dtype == torch.bfloat16
+def _few_rows(x, w, swiglu: bool):
+    """The kernel for a few rows of bf16 against w, or None: gemv streams the
+    weights past one to eight rows (ops/csrc/gemv.hip), rows_gemm past tens
+    of them (ops/csrc/rows_gemm.hip); each says which sizes it takes."""
+    if not (x.is_cuda and HAS_KERNELS and x.dim() == 2 and w.dim() == 2
+            and x.shape[0] <= 64 and x.dtype == torch.bfloat16
             and w.dtype == x.dtype and w.shape[1] == x.shape[1]
-            and _kernels.gemv_fits(x.shape[0], x.shape[1], swiglu)
             and w.is_contiguous() and x.stride(1) == 1
             and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
             and w.data_ptr() % 16 == 0
             and not (torch.is_grad_enabled()
-                     and (x.requires_grad or w.requires_grad)))
+                     and (x.requires_grad or w.requires_grad))):
+        return None
+    M, K = x.shape
+    if _kernels.gemv_fits(M, K, swiglu):
+        return _kernels.gemv
+    N = w.shape[0] // 2 if swiglu else w.shape[0]
+    return (_kernels.rows_gemm
+            if _kernels.rows_gemm_splits(M, N, K, swiglu) else None)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
-    """x W^T (+ bias).  A few rows of bf16 run the weight-streaming kernel
-    (ops/csrc/gemv.hip), everything else the library's product."""
-    if _gemv_takes(x, w, False) and (bias is None or (
+    """x W^T (+ bias).  A few rows of bf16 run the weight-streaming kernels,
+    everything else the library's product."""
+    kernel = _few_rows(x, w, False)
+    if kernel and (bias is None or (
             bias.dtype == x.dtype and bias.is_contiguous())):
         out = torch.empty((x.shape[0], w.shape[0]), dtype=x.dtype,
                           device=x.device)
-        _kernels.gemv(out, x, w, bias, False)
+        kernel(out, x, w, bias, False)
         return out
     return torch.nn.functional.linear(x, w, bias)
 
@@ -232,10 +242,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T) with w = [Wg; Wu]: one kernel for a few rows
     of bf16, else the product and silu_mul."""
-    if _gemv_takes(x, w, True) and w.shape[0] % 2 == 0:
+    kernel = _few_rows(x, w, True) if w.shape[0] % 2 == 0 else None
+    if kernel:
         out = torch.empty((x.shape[0], w.shape[0] // 2), dtype=x.dtype,
                           device=x.device)
-        _kernels.gemv(out, x, w, None, True)
+        kernel(out, x, w, None, True)
         return out
     return silu_mul(torch.nn.functional.linear(x, w))
 

@@ -31,6 +31,9 @@ void flash_prefill_paged(torch::Tensor out, torch::Tensor q,
                          std::vector<int64_t> seq_lens, double scale);
 void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
           c10::optional<torch::Tensor> bias, bool swiglu);
+void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> bias, bool swiglu);
+int64_t rows_gemm_splits(int64_t M, int64_t N, int64_t K, bool swiglu);
 bool gemv_fits(int64_t M, int64_t K, bool swiglu);
 bool moe_few_fits(int64_t T, int64_t top_k, int64_t D, int64_t F);
 void moe_few(torch::Tensor out, torch::Tensor x, torch::Tensor gate_up,
@@ -80,6 +83,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "x W^T for a few rows of x, optional bias or SwiGLU");
   m.def("moe_few", &igw::moe_few, "SwiGLU experts of a few tokens");
   m.def("moe_few_fits", &igw::moe_few_fits, "whether moe_few takes these");
+  m.def("rows_gemm", &igw::rows_gemm, "x W^T of tens of rows");
+  m.def("rows_gemm_splits", &igw::rows_gemm_splits,
+        "parts of K that rows_gemm takes, 0: it does not");
   m.def("gemv_fits", &igw::gemv_fits, "whether gemv takes these sizes");
   m.def("flash_prefill_paged", &igw::flash_prefill_paged,
         "paged-extend prefill: chunk queries over cached prefix+chunk K/V "

@@ -884,6 +884,48 @@ def test_add_normed_rmsnorm_rows(D, dtype, pad):
     torch.testing.assert_close(same, x, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("N,K,splits", [(28000, 256, 1), (32764, 768, 1),
+                                        (128 * 224, 1280, 1), (4, 6144 * 64, 256),
+                                        (4096, 14336, 8), (1924, 25856, 16)])
+@pytest.mark.parametrize("M", [16, 17, 31, 33, 48, 49, 64, 65])
+def test_linear_tens_of_rows(M, N, K, splits):
+    # either side of the rows it takes; slices of K one to seven and more,
+    # uneven parts of a split K, outputs that end inside a wave's rows
+    g = torch.Generator().manual_seed(M + N)
+    buf = torch.randn(M, K + 8, generator=g).to(torch.bfloat16).cuda()
+    x = buf[:, :K]
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).cuda()
+    b = torch.randn(N, generator=g).to(torch.bfloat16).cuda()
+    takes = ops._kernels.rows_gemm_splits(M, N, K, False)
+    assert takes == (splits if 17 <= M <= 64 else 0)
+    out = ops.linear(x, w, b).double()
+    ref = x.double() @ w.double().t() + b.double()
+    mag = x.double().abs() @ w.double().abs().t()
+    assert bool(((out - ref).abs() <= 2.0 ** -8 * ref.abs()
+                 + K * 2.0 ** -24 * mag + 1e-6).all())
+
+
+@pytest.mark.parametrize("M,F,K", [(8, 14336, 512), (9, 14000, 256),
+                                   (17, 16380, 1024), (48, 14336, 768),
+                                   (64, 14336, 1280), (65, 14336, 512)])
+def test_linear_silu_mul_tens_of_rows(M, F, K):
+    g = torch.Generator().manual_seed(M)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).cuda()
+    w = (torch.randn(2 * F, K, generator=g) * K ** -0.5).to(
+        torch.bfloat16).cuda()
+    assert bool(ops._kernels.rows_gemm_splits(M, F, K, True)) == (9 <= M <= 64)
+    out = ops.linear_silu_mul(x, w).double()
+    y = x.double() @ w.double().t()
+    ref = torch.nn.functional.silu(y[:, :F]) * y[:, F:]
+    # bf16 rounds by at most 2^-8 of a value: once here, and on the library's
+    # side the up half, the gate (silu's relative slope is at most 1.3 above
+    # zero, below it the values are within atol) and the result
+    once = bool(ops._kernels.rows_gemm_splits(M, F, K, True)) or M <= 8
+    torch.testing.assert_close(out, ref, rtol=2.0 ** -8 * (1.1 if once
+                                                           else 3.4),
+                               atol=2.0 ** -9 * float(y.abs().max()))
+
+
 def test_zz_chunked_prefill_engine_matches_unchunked():
     # placed in this (alphabetically last) file, and named to sort last,
     # so the driver's -x run covers everything else first
