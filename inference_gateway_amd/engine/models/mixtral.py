@@ -8,9 +8,9 @@ of every expert), so dispatch stays local and the existing row-parallel
 all-reduce covers the combine — the right choice for the fully-connected
 xGMI topology at Mixtral's scale (8 experts / 8 GPUs would leave EP
 all-to-all bound by single-link bandwidth with no GEMM-shape benefit at
-decode batch sizes). Token routing/gather is done with index_select /
-index_add (hipBLASLt batched GEMMs per expert); a fused grouped-GEMM HIP
-kernel is the planned next optimization.
+decode batch sizes). Up to eight tokens read only the experts they chose
+(ops.moe_few); larger decode steps run batched GEMMs over padded rows, and
+prompts one GEMM per expert, with index_select / index_add around them.
 """
 from __future__ import annotations
 
