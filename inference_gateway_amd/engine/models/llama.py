@@ -84,11 +84,11 @@ class LlamaAttention(nn.Module):
         # row stride, so there are no .contiguous() copies on the hot path
         q, k, v = qkv.split(
             [self.nq * self.hd, self.nkv * self.hd, self.nkv * self.hd], dim=-1)
-        ops.rotary_embedding(fb.positions, q, k, self.hd, cos_sin)
         kc, vc = kv_cache
+        ops.rope_append(fb.positions, q, k, v, self.hd, cos_sin, kc, vc,
+                        fb.slot_mapping)
         k3 = k.view(T, self.nkv, self.hd)
         v3 = v.view(T, self.nkv, self.hd)
-        ops.append_kv_cache(k3, v3, kc, vc, fb.slot_mapping)
         if fb.is_prefill:
             P = fb.num_prefill_tokens if fb.is_mixed else T
             qv = q.view(T, self.nq, self.hd)

@@ -148,6 +148,20 @@ def append_kv_cache(k, v, kcache, vcache, slot_mapping):
     torch_ref.append_kv_cache_ref(k, v, kcache, vcache, slot_mapping)
 
 
+def rope_append(positions, q, k, v, head_dim: int, cos_sin_cache, kcache,
+                vcache, slot_mapping):
+    """rotary_embedding of q and k (in place), then append_kv_cache of k and
+    v [T, NKV*HD], in one launch on the GPU."""
+    if q.is_cuda:
+        _require_kernels()
+        _kernels.rope_append(positions, q, k, v, cos_sin_cache, kcache,
+                             vcache, slot_mapping)
+        return
+    rotary_embedding(positions, q, k, head_dim, cos_sin_cache)
+    rows = (k.shape[0], kcache.shape[1], head_dim)
+    append_kv_cache(k.view(rows), v.view(rows), kcache, vcache, slot_mapping)
+
+
 def paged_attn_decode(q, kcache, vcache, block_table, ctx_lens, scale: float):
     if q.is_cuda:
         _require_kernels()

@@ -15,6 +15,10 @@ void fused_add_rmsnorm(torch::Tensor x, torch::Tensor residual,
 void rotary_embedding(torch::Tensor positions, torch::Tensor q,
                       torch::Tensor k, int64_t head_dim,
                       torch::Tensor cos_sin_cache);
+void rope_append(torch::Tensor positions, torch::Tensor q, torch::Tensor k,
+                 torch::Tensor v, torch::Tensor cos_sin_cache,
+                 torch::Tensor kcache, torch::Tensor vcache,
+                 torch::Tensor slot_mapping);
 void append_kv_cache(torch::Tensor k, torch::Tensor v, torch::Tensor kcache,
                      torch::Tensor vcache, torch::Tensor slot_mapping);
 void paged_attn_decode(torch::Tensor out, torch::Tensor q,
@@ -73,6 +77,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "residual += x; x = rmsnorm(residual) (bf16, gfx950)");
   m.def("rotary_embedding", &igw::rotary_embedding,
         "NeoX-style RoPE in-place on q/k (bf16, gfx950)");
+  m.def("rope_append", &igw::rope_append,
+        "RoPE of q and k, k and v into the paged cache");
   m.def("append_kv_cache", &igw::append_kv_cache,
         "scatter step K/V into the paged cache (bf16, gfx950)");
   m.def("paged_attn_decode", &igw::paged_attn_decode,

@@ -2,9 +2,12 @@
 //
 // Part of the net-new local engine (SURVEY.md §7 stage 3b). Both ops are
 // memory-bound elementwise passes, fused as tightly as the call graph allows:
-// RoPE rotates Q and K in one launch; the cache append scatters K and V of
-// the current step into the paged cache ([num_blocks, n_kv_heads, block_size,
-// head_dim] layout chosen so the decode-attention kernel reads contiguous
+// RoPE rotates Q and K in one launch, and with APPEND the same launch writes
+// the rotated K and V into the paged cache: a launch is 4.0 us however few the
+// rows, so a decode step's layer has 4.0 us where the two launches had 8.0.
+// The cache append alone scatters K and V of the current step.  Cache layout
+// [num_blocks, n_kv_heads, block_size, head_dim], chosen so the
+// decode-attention kernel reads contiguous
 // [block_size, head_dim] tiles per (block, head)).
 
 #include <ATen/cuda/CUDAContext.h>
@@ -17,10 +20,17 @@ namespace igw {
 // GPT-NeoX-style rotate-half RoPE, in place on q and k.
 // q: [T, NQ*HD], k: [T, NKV*HD], cos_sin: [max_pos, HD] fp32
 // (cos in [0, HD/2), sin in [HD/2, HD)).
+// APPEND: v [T, NKV*HD] and the caches as for append_kv_kernel below.
+template <bool APPEND>
 __global__ void rope_kernel(uint16_t* __restrict__ q, uint16_t* __restrict__ k,
+                            const uint16_t* __restrict__ v,
                             const int32_t* __restrict__ positions,
-                            const float* __restrict__ cos_sin, int nq, int nkv,
-                            int hd, int qs, int ks) {
+                            const float* __restrict__ cos_sin,
+                            uint16_t* __restrict__ kcache,
+                            uint16_t* __restrict__ vcache,
+                            const int32_t* __restrict__ slot_mapping, int nq,
+                            int nkv, int hd, int block_size, int qs, int ks,
+                            int vs) {
   // qs/ks: row strides in elements — q/k may be views into a fused-QKV
   // GEMM output (no .contiguous() copies on the decode hot path).
   // Vectorized 8 pairs per thread: the rotate-half halves are each
@@ -32,6 +42,12 @@ __global__ void rope_kernel(uint16_t* __restrict__ q, uint16_t* __restrict__ k,
   const int half = hd / 2;
   const int nheads = nq + nkv;
   const int groups = half >> 3;       // 8 pairs per group (hd % 16 == 0)
+  const int slot = APPEND ? slot_mapping[t] : -1;
+  // (head 0, this row's offset) of the cache; a head is block_size rows on
+  const int64_t cell =
+      slot < 0 ? 0
+               : ((int64_t)(slot / block_size) * nkv * block_size +
+                  slot % block_size) * hd;
   for (int i = threadIdx.x; i < nheads * groups; i += blockDim.x) {
     const int h = i / groups;
     const int d0 = (i % groups) * 8;
@@ -55,6 +71,19 @@ __global__ void rope_kernel(uint16_t* __restrict__ q, uint16_t* __restrict__ k,
     }
     *reinterpret_cast<ushort8*>(base + d0) = o1;
     *reinterpret_cast<ushort8*>(base + half + d0) = o2;
+    if (APPEND && slot >= 0 && h >= nq) {
+      uint16_t* c = kcache + cell + (int64_t)(h - nq) * block_size * hd;
+      *reinterpret_cast<ushort8*>(c + d0) = o1;
+      *reinterpret_cast<ushort8*>(c + half + d0) = o2;
+    }
+  }
+  if (APPEND && slot >= 0) {
+    for (int i = threadIdx.x * 8; i < nkv * hd; i += blockDim.x * 8) {
+      const int h = i / hd;
+      *reinterpret_cast<ushort8*>(vcache + cell +
+                                  (int64_t)h * block_size * hd + i % hd) =
+          *reinterpret_cast<const ushort8*>(v + (int64_t)t * vs + i);
+    }
   }
 }
 
@@ -98,11 +127,46 @@ void rotary_embedding(torch::Tensor positions, torch::Tensor q, torch::Tensor k,
   const int nkv = k.size(-1) / hd;
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
   const int threads = 256;
-  hipLaunchKernelGGL(rope_kernel, dim3(T), dim3(threads), 0, stream,
+  hipLaunchKernelGGL(rope_kernel<false>, dim3(T), dim3(threads), 0, stream,
                      (uint16_t*)q.data_ptr(), (uint16_t*)k.data_ptr(),
+                     (const uint16_t*)nullptr,
                      (const int32_t*)positions.data_ptr(),
-                     (const float*)cos_sin_cache.data_ptr(), nq, nkv, hd,
-                     (int)q.stride(0), (int)k.stride(0));
+                     (const float*)cos_sin_cache.data_ptr(),
+                     (uint16_t*)nullptr, (uint16_t*)nullptr,
+                     (const int32_t*)nullptr, nq, nkv, hd, 1,
+                     (int)q.stride(0), (int)k.stride(0), 0);
+  HIP_CHECK_KERNEL();
+}
+
+// rotary_embedding of q and k [T, heads * HD], then append_kv_cache of k and v.
+void rope_append(torch::Tensor positions, torch::Tensor q, torch::Tensor k,
+                 torch::Tensor v, torch::Tensor cos_sin_cache,
+                 torch::Tensor kcache, torch::Tensor vcache,
+                 torch::Tensor slot_mapping) {
+  TORCH_CHECK(q.is_cuda() && q.dtype() == torch::kBFloat16 &&
+              k.dtype() == q.dtype() && v.dtype() == q.dtype());
+  TORCH_CHECK(positions.dtype() == torch::kInt32 &&
+              slot_mapping.dtype() == torch::kInt32);
+  TORCH_CHECK(cos_sin_cache.dtype() == torch::kFloat32);
+  TORCH_CHECK(q.stride(-1) == 1 && k.stride(-1) == 1 && v.stride(-1) == 1);
+  TORCH_CHECK(kcache.is_contiguous() && vcache.is_contiguous());
+  const int T = q.size(0);
+  const int nkv = kcache.size(1), block_size = kcache.size(2);
+  const int hd = kcache.size(3);
+  TORCH_CHECK(hd % 16 == 0, "rope: head_dim must be 16-aligned");
+  TORCH_CHECK(k.size(-1) == nkv * hd && v.size(-1) == nkv * hd &&
+              q.size(-1) % hd == 0);
+  hipStream_t stream = at::cuda::getCurrentCUDAStream();
+  hipLaunchKernelGGL(rope_kernel<true>, dim3(T), dim3(256), 0, stream,
+                     (uint16_t*)q.data_ptr(), (uint16_t*)k.data_ptr(),
+                     (const uint16_t*)v.data_ptr(),
+                     (const int32_t*)positions.data_ptr(),
+                     (const float*)cos_sin_cache.data_ptr(),
+                     (uint16_t*)kcache.data_ptr(),
+                     (uint16_t*)vcache.data_ptr(),
+                     (const int32_t*)slot_mapping.data_ptr(),
+                     (int)(q.size(-1) / hd), nkv, hd, block_size,
+                     (int)q.stride(0), (int)k.stride(0), (int)v.stride(0));
   HIP_CHECK_KERNEL();
 }
 

@@ -926,6 +926,37 @@ def test_linear_silu_mul_tens_of_rows(M, F, K):
                                atol=2.0 ** -9 * float(y.abs().max()))
 
 
+@pytest.mark.parametrize("T,nq,nkv,hd,bs", [(1, 32, 8, 128, 16),
+                                            (37, 5, 1, 64, 16),
+                                            (300, 40, 10, 128, 32),
+                                            (3, 2, 2, 16, 8)])
+def test_rope_append_is_the_two_launches(T, nq, nkv, hd, bs):
+    # a fused projection's views; some rows without a slot
+    g = torch.Generator().manual_seed(T)
+    nb = T // bs + 3
+    qkv = torch.randn(T, (nq + 2 * nkv) * hd, generator=g).to(
+        torch.bfloat16).cuda()
+    pos = torch.randint(0, 2048, (T,), dtype=torch.int32, device="cuda")
+    cs = torch_ref.build_cos_sin_cache(hd, 4096, device="cuda")
+    slots = torch.randperm(nb * bs, device="cuda")[:T].to(torch.int32)
+    slots[1::5] = -1
+    res = []
+    for fused in (False, True):
+        a = qkv.clone()
+        q, k, v = a.split([nq * hd, nkv * hd, nkv * hd], -1)
+        kc = torch.zeros(nb, nkv, bs, hd, dtype=torch.bfloat16, device="cuda")
+        vc = torch.zeros_like(kc)
+        if fused:
+            ops.rope_append(pos, q, k, v, hd, cs, kc, vc, slots)
+        else:
+            ops.rotary_embedding(pos, q, k, hd, cs)
+            ops.append_kv_cache(k.view(T, nkv, hd), v.view(T, nkv, hd), kc,
+                                vc, slots)
+        res.append((a, kc, vc))
+    for one, two in zip(*res):
+        assert torch.equal(one, two)
+
+
 def test_zz_chunked_prefill_engine_matches_unchunked():
     # placed in this (alphabetically last) file, and named to sort last,
     # so the driver's -x run covers everything else first
