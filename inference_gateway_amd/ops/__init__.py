@@ -221,10 +221,10 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_mul_ref(gate_up)
 
 
-def _few_rows(x, w, bias, swiglu: bool):
-    """x W^T of a few rows by the weight-streaming kernels (a few rows
-    ops/csrc/gemv.hip, tens of them ops/csrc/rows_gemm.hip), or None where
-    they do not take the call (ops/csrc/few_rows.hip says which)."""
+def _own_product(x, w, bias, swiglu: bool):
+    """x W^T by the kernels here (a few rows ops/csrc/gemv.hip, tens of them
+    ops/csrc/rows_gemm.hip, hundreds to thousands ops/csrc/wide_gemm.hip), or
+    None where they do not take the call (ops/csrc/few_rows.hip says which)."""
     if (has_torch_function_variadic(x, w) or torch.compiler.is_compiling()
             or not (x.is_cuda and HAS_KERNELS)):
         return None
@@ -233,15 +233,16 @@ def _few_rows(x, w, bias, swiglu: bool):
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     """x W^T (+ bias).  A few rows of bf16 run the weight-streaming kernels,
-    everything else the library's product."""
-    out = _few_rows(x, w, bias, False)
+    hundreds of them over a vocabulary's width the tiled one, everything else
+    the library's product."""
+    out = _own_product(x, w, bias, False)
     return torch.nn.functional.linear(x, w, bias) if out is None else out
 
 
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """silu(x Wg^T) * (x Wu^T) with w = [Wg; Wu]: one kernel for a few rows
-    of bf16, else the product and silu_mul."""
-    out = _few_rows(x, w, None, True)
+    """silu(x Wg^T) * (x Wu^T) with w = [Wg; Wu]: one kernel for bf16 rows
+    where it is ahead, else the product and silu_mul."""
+    out = _own_product(x, w, None, True)
     return (silu_mul(torch.nn.functional.linear(x, w)) if out is None
             else out)
 

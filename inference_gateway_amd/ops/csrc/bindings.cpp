@@ -38,6 +38,9 @@ void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
           c10::optional<torch::Tensor> bias, bool swiglu);
 void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias, bool swiglu);
+int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
+void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               bool swiglu, int64_t tile);
 int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
                        const c10::optional<torch::Tensor>& bias, bool swiglu,
                        bool anywhere);
@@ -93,12 +96,16 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash_prefill", &igw::flash_prefill,
         "varlen causal MFMA flash-attention prefill (bf16, gfx950)");
   m.def("few_rows", &igw::few_rows,
-        "x W^T of a few rows by gemv or rows_gemm, None: neither takes it");
+        "x W^T by gemv, rows_gemm or wide_gemm, None: none of them takes it");
   m.def("gemv", &igw::gemv,
         "x W^T for a few rows of x, optional bias or SwiGLU");
   m.def("rows_gemm", &igw::rows_gemm, "x W^T of tens of rows");
+  m.def("wide_gemm", &igw::wide_gemm,
+        "x W^T of hundreds to thousands of rows on a given tile");
+  m.def("wide_gemm_tile", &igw::wide_gemm_tile,
+        "its tile (16 MT + NT) for a product; 0: not ahead of the library");
   m.def("few_rows_takes", &igw::few_rows_takes,
-        "0: neither, 1: gemv, 2: rows_gemm");
+        "0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm");
   m.def("moe_few", &igw::moe_few, "SwiGLU experts of a few tokens");
   m.def("moe_few_takes", &igw::moe_few_takes, "whether moe_few takes a step");
   m.def("rows_gemm_splits", &igw::rows_gemm_splits,

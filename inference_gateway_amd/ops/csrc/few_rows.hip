@@ -1,5 +1,6 @@
 // Host side of ops.linear, ops.linear_silu_mul and ops.moe_few: which calls
-// the weight-streaming kernels take (gemv.hip, rows_gemm.hip).
+// the kernels for a few rows of x (gemv.hip, rows_gemm.hip) and for hundreds
+// and thousands of them (wide_gemm.hip) take.
 //
 // What they are handed is a pointer, so the tensors have to be what they seem:
 // plain dense bf16 on one GPU, in a call that nothing but the product has to
@@ -18,6 +19,10 @@ bool gemv_fits(int64_t M, int64_t K, bool swiglu);
 bool gemv_ahead(int64_t M, int64_t N, int64_t K, bool swiglu);
 int64_t rows_gemm_splits(int64_t M, int64_t N, int64_t K, bool swiglu);
 bool rows_gemm_ahead(int64_t M, int64_t S, int64_t K, bool swiglu);
+int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
+bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu);
+void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               bool swiglu, int64_t tile);
 bool moe_few_fits(int64_t T, int64_t top_k, int64_t D, int64_t F);
 void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
           c10::optional<torch::Tensor> bias, bool swiglu);
@@ -49,13 +54,13 @@ static bool by16(const torch::Tensor& t) {
   return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
 
-// 0: neither, 1: gemv, 2: rows_gemm.  `anywhere`: also off the GPU (the rule
+// 0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm.  `anywhere`: also off the GPU (the rule
 // alone, nothing is launched).
 int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
                        const c10::optional<torch::Tensor>& bias, bool swiglu,
                        bool anywhere) {
   if (!(anywhere || x.is_cuda()) || x.dim() != 2 || w.dim() != 2 ||
-      x.size(0) > 64 || !call_is_plain() || !plain_bf16(x, x.device()) ||
+      !call_is_plain() || !plain_bf16(x, x.device()) ||
       !plain_bf16(w, x.device()))
     return 0;
   const int64_t M = x.size(0), K = x.size(1);
@@ -67,12 +72,17 @@ int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
       !(!swiglu && plain_bf16(*bias, x.device()) && bias->dim() == 1 &&
         bias->size(0) == N && bias->is_contiguous()))
     return 0;
+  if (M > 64)
+    return !bias.has_value() && wide_gemm_tile(M, N, K, swiglu) > 0 &&
+                   wide_gemm_fits(x.stride(0), N, K, swiglu)
+               ? 3
+               : 0;
   if (gemv_fits(M, K, swiglu)) return gemv_ahead(M, w.size(0), K, swiglu);
   const int64_t S = rows_gemm_splits(M, N, K, swiglu);
   return S > 0 && rows_gemm_ahead(M, S, K, swiglu) ? 2 : 0;
 }
 
-// The product, or nothing when neither kernel takes it.
+// The product, or nothing when none of the kernels takes it.
 c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
                                       const torch::Tensor& w,
                                       const c10::optional<torch::Tensor>& bias,
@@ -81,7 +91,11 @@ c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
   if (which == 0) return c10::nullopt;
   auto out = torch::empty({x.size(0), swiglu ? w.size(0) / 2 : w.size(0)},
                           x.options());
-  (which == 1 ? gemv : rows_gemm)(out, x, w, bias, swiglu);
+  if (which == 3)
+    wide_gemm(out, x, w, swiglu,
+              wide_gemm_tile(x.size(0), out.size(1), x.size(1), swiglu));
+  else
+    (which == 1 ? gemv : rows_gemm)(out, x, w, bias, swiglu);
   return out;
 }
 

@@ -244,6 +244,49 @@ def test_few_rows_lines(M, N, K, swiglu, want):
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,swiglu,tile", [
+    # (rows of 16 in the tile, of W) for the library's side 0
+    (1024, 28672, 4096, True, (8, 7)), (16000, 28672, 4096, True, (8, 8)),
+    (256, 28672, 4096, True, (4, 8)), (333, 28672, 4096, True, (6, 8)),
+    (65, 35840, 5120, True, (4, 8)), (512, 35840, 5120, True, (8, 6)),
+    (128, 28672, 4096, True, 0), (512, 7168, 4096, True, 0),
+    (1536, 57344, 8192, True, (8, 7)), (1537, 57344, 8192, True, 0),
+    (1024, 28672, 4160, True, 0), (1024, 28680, 4096, True, 0),
+    (1024, 128256, 4096, False, (8, 8)), (256, 65536, 4096, False, (8, 8)),
+    (255, 128256, 4096, False, 0), (2049, 128256, 4096, False, 0),
+    (1024, 32000, 4096, False, 0), (1024, 128256, 256, False, 0),
+    # offsets of 32 bits
+    (256, 131072, 8192, True, 0)])
+def test_wide_gemm_lines(M, N, K, swiglu, tile):
+    x = torch.empty(M, K, dtype=torch.bfloat16)
+    want = tile and tile[0] * 16 + tile[1]
+    if (N, K) != (131072, 8192):
+        assert ops._kernels.wide_gemm_tile(
+            M, N // 2 if swiglu else N, K, swiglu) == want
+    w = torch.empty(N, K, dtype=torch.bfloat16)     # never touched
+    assert ops._kernels.few_rows_takes(x, w, None, swiglu, True) == (
+        3 if want else 0)
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+def test_wide_gemm_takes_plain_calls_only():
+    bf = torch.bfloat16
+    x, w = torch.empty(300, 520, dtype=bf), torch.empty(65536, 512, dtype=bf)
+
+    def takes(x, w, b=None):
+        return ops._kernels.few_rows_takes(x, w, b, False, True)
+
+    assert takes(x[:, :512], w) == 3
+    assert takes(x[:, :512], w, torch.empty(65536, dtype=bf)) == 0
+    assert takes(x[:, 1:513], w) == 0
+    assert takes(torch.empty(300, 515, dtype=bf)[:, :512], w) == 0
+    assert takes(x[:, :512].t().contiguous().t(), w) == 0
+    assert takes(x[:, :512].float(), w.float()) == 0
+    assert takes(x[:, :512].clone().requires_grad_(), w) == 0
+    assert takes(x[:, :512], w[:, :512].t().contiguous().t()) == 0
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 def test_moe_few_takes():
     bf = torch.bfloat16
     x, gu, dn = torch.randn(3, 64).to(bf), torch.randn(4, 96, 64).to(bf), \
