@@ -9,8 +9,9 @@ all-reduce covers the combine — the right choice for the fully-connected
 xGMI topology at Mixtral's scale (8 experts / 8 GPUs would leave EP
 all-to-all bound by single-link bandwidth with no GEMM-shape benefit at
 decode batch sizes). Up to eight tokens read only the experts they chose
-(ops.moe_few); larger decode steps run batched GEMMs over padded rows, and
-prompts one GEMM per expert, with index_select / index_add around them.
+(ops.moe_few); everything larger runs two products over rows sorted by expert
+(ops.moe_rows). Where those do not take the call, decode steps run batched
+GEMMs over padded rows, and prompts one GEMM per expert.
 """
 from __future__ import annotations
 
@@ -100,6 +101,9 @@ class MixtralMoE(nn.Module):
             weights, _dst, idx, _counts = ops.moe_route(
                 self.router(x).float(), self.top_k, 64)
             out = ops.moe_few(x, self.gate_up, self.down, idx, weights)
+        elif ops.moe_rows_fits(x, self.gate_up, self.down, self.top_k):
+            out = ops.moe_rows(x, self.router(x).contiguous(), self.gate_up,
+                               self.down, self.top_k)
         elif is_prefill and x.shape[0] > 1024:
             out = self._forward_sorted(x)
         else:

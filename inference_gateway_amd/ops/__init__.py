@@ -81,7 +81,7 @@ def _shared_ext(name: str):
     """An op that several extensions compile (same source file):
     whichever is built serves it, so a process that runs one model family
     needs one library."""
-    for ext in (_postnorm, _streams, _hybrid, _recurrent):
+    for ext in (_postnorm, _streams, _hybrid, _recurrent, _kernels):
         if ext is not None and hasattr(ext, name):
             return getattr(ext, name)
     raise RuntimeError(
@@ -320,6 +320,37 @@ def moe_few(x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor,
     out = torch.empty_like(x)
     _kernels.moe_few(out, x, gate_up, down, topk_idx, weights)
     return out
+
+
+def moe_rows_fits(x: torch.Tensor, gate_up: torch.Tensor,
+                  down: torch.Tensor, top_k: int) -> bool:
+    """Whether moe_rows takes this step: plain bf16 on the GPU, widths in
+    whole pairs of K steps, a top_k that the routing kernel has."""
+    return bool(x.is_cuda and HAS_KERNELS and _kernels.moe_rows_takes(
+        x, gate_up, down, top_k, False))
+
+
+def moe_rows(x: torch.Tensor, logits: torch.Tensor, gate_up: torch.Tensor,
+             down: torch.Tensor, top_k: int) -> torch.Tensor:
+    """SwiGLU experts of any number of tokens (on the GPU, where moe_rows_fits
+    says so): x [T, D], router logits [T, E] in bf16 or fp32, gate_up [E, 2 F,
+    D], down [E, D, F]; returns the sum of the top_k experts of each token,
+    weighted by the softmax over their logits, [T, D].  Rows are sorted by
+    expert on the device and no count goes to the host, so the step can be
+    captured."""
+    _require_kernels()
+    T, E = logits.shape
+    dev = x.device
+    weights = torch.empty((T, top_k), dtype=torch.float32, device=dev)
+    dst = torch.empty(T * top_k, dtype=torch.int64, device=dev)
+    start = torch.empty(E + 1, dtype=torch.int32, device=dev)
+    _kernels.moe_dispatch(weights, dst, start, logits)
+    rows = moe_scatter_rows(x, dst, T * top_k)
+    act = torch.empty((T * top_k, down.shape[2]), dtype=x.dtype, device=dev)
+    _kernels.grouped_gemm(act, rows, gate_up, start, True, 0)
+    # the scattered rows are read, their memory takes the result
+    _kernels.grouped_gemm(rows, act, down, start, False, 0)
+    return moe_combine(rows, dst, weights)
 
 
 def silu_mul_grouped(gate_up: torch.Tensor, counts: torch.Tensor,
@@ -1188,9 +1219,9 @@ def moe_scatter_rows(x, dst, rows: int):
     """[rows, D] buffer with buf[dst[t*K + k]] = x[t] (dst int64 [T*K]);
     rows that nothing is written to are left undefined."""
     if x.is_cuda:
-        _require_streams()
         buf = torch.empty((rows, x.shape[1]), dtype=x.dtype, device=x.device)
-        _streams.moe_scatter_rows(buf, x, dst, dst.numel() // x.shape[0])
+        _shared_ext("moe_scatter_rows")(buf, x, dst,
+                                        dst.numel() // x.shape[0])
         return buf
     buf = x.new_zeros((rows, x.shape[1]))
     buf[dst] = x.repeat_interleave(dst.numel() // x.shape[0], 0)
@@ -1202,10 +1233,9 @@ def moe_combine(y, dst, weights, shared=None, shared_gate=None):
     sigmoid(shared_gate[t]) * shared[t] (shared None: no such term), fp32
     sums; weights fp32 [T, K], shared_gate fp32 [T] (strided ok)."""
     if y.is_cuda:
-        _require_streams()
         out = torch.empty((weights.shape[0], y.shape[1]), dtype=y.dtype,
                           device=y.device)
-        _streams.moe_combine(out, y, dst, weights, shared, shared_gate)
+        _shared_ext("moe_combine")(out, y, dst, weights, shared, shared_gate)
         return out
     T, K = weights.shape
     out = (y[dst].view(T, K, -1).float() * weights[:, :, None]).sum(1)

@@ -50,6 +50,18 @@ c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
                                       bool swiglu);
 bool moe_few_takes(const torch::Tensor& x, const torch::Tensor& gate_up,
                    const torch::Tensor& down, int64_t top_k, bool anywhere);
+bool moe_rows_takes(const torch::Tensor& x, const torch::Tensor& gate_up,
+                    const torch::Tensor& down, int64_t top_k, bool anywhere);
+int64_t grouped_tile(int64_t rows, int64_t E, int64_t N, bool swiglu);
+void grouped_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                  torch::Tensor start, bool swiglu, int64_t tile);
+void moe_dispatch(torch::Tensor weights, torch::Tensor dst,
+                  torch::Tensor start, torch::Tensor logits);
+void moe_scatter_rows(torch::Tensor buf, torch::Tensor x, torch::Tensor dst,
+                      int64_t K);
+void moe_combine(torch::Tensor out, torch::Tensor y, torch::Tensor dst,
+                 torch::Tensor w, c10::optional<torch::Tensor> shared,
+                 c10::optional<torch::Tensor> g);
 void moe_few(torch::Tensor out, torch::Tensor x, torch::Tensor gate_up,
              torch::Tensor down, torch::Tensor idx, torch::Tensor weight);
 void sample(torch::Tensor out, torch::Tensor logits, torch::Tensor temperature,
@@ -107,6 +119,17 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("few_rows_takes", &igw::few_rows_takes,
         "0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm");
   m.def("moe_few", &igw::moe_few, "SwiGLU experts of a few tokens");
+  m.def("moe_rows_takes", &igw::moe_rows_takes,
+        "whether the grouped products take a step");
+  m.def("grouped_tile", &igw::grouped_tile, "grouped_gemm's tile (16 MT + NT)");
+  m.def("grouped_gemm", &igw::grouped_gemm,
+        "every expert's rows of x times its weights, optional SwiGLU");
+  m.def("moe_dispatch", &igw::moe_dispatch,
+        "top-k, softmax weights and rows sorted by expert");
+  m.def("moe_scatter_rows", &igw::moe_scatter_rows,
+        "buf[dst[t*K + k]] = x[t]");
+  m.def("moe_combine", &igw::moe_combine,
+        "out[t] = sum_k w[t, k] y[dst[t*K + k]] (+ gated shared rows)");
   m.def("moe_few_takes", &igw::moe_few_takes, "whether moe_few takes a step");
   m.def("rows_gemm_splits", &igw::rows_gemm_splits,
         "parts of K that rows_gemm takes, 0: it does not");

@@ -116,4 +116,24 @@ bool moe_few_takes(const torch::Tensor& x, const torch::Tensor& gate_up,
          moe_few_fits(x.size(0), top_k, D, F);
 }
 
+// Whether the grouped products take a step of any number of tokens.
+bool moe_rows_takes(const torch::Tensor& x, const torch::Tensor& gate_up,
+                    const torch::Tensor& down, int64_t top_k, bool anywhere) {
+  if (!(anywhere || x.is_cuda()) || x.dim() != 2 || gate_up.dim() != 3 ||
+      down.dim() != 3 ||
+      !(top_k == 1 || top_k == 2 || top_k == 4 || top_k == 8) ||
+      !call_is_plain())
+    return false;
+  for (const auto* t : {&x, &gate_up, &down})
+    if (!plain_bf16(*t, x.device()) || !t->is_contiguous() || !by16(*t))
+      return false;
+  const int64_t T = x.size(0), D = x.size(1), F = down.size(2),
+                E = gate_up.size(0);
+  return gate_up.size(1) == 2 * F && gate_up.size(2) == D &&
+         down.size(0) == E && down.size(1) == D && E >= top_k && E <= 64 &&
+         T >= 1 && T < (1 << 25) && D >= 384 && D % 128 == 0 && F >= 384 &&
+         F % 128 == 0 && wide_gemm_fits(D, F, D, true) &&
+         wide_gemm_fits(F, D, F, false);
+}
+
 }  // namespace igw

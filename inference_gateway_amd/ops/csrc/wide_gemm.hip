@@ -26,6 +26,7 @@
 #include <c10/cuda/CUDAGuard.h>
 #include <torch/extension.h>
 
+#include <cmath>
 #include <type_traits>
 
 #include "common.h"
@@ -46,6 +47,8 @@ struct WideArgs {
   const uint16_t* w;
   int M, N, K;
   int64_t x_rs;
+  const int32_t* start;  // [E + 1]: first row of every expert (GROUPED)
+  int E;
 };
 
 DEVINLINE uint32_t wg_pack(float a, float b) {
@@ -81,7 +84,9 @@ DEVINLINE void wg_dma(wg_u32x4 buf, int lane_off, int off, uint32_t at) {
 #define WG_INLINE __attribute__((always_inline))
 
 // MT, NT: 16-row tiles of x and of W of one of the 2 x 2 waves.
-template <int MT, int NT, bool SWIGLU>
+// GROUPED: rows start[e] .. start[e + 1] - 1 of x with the e-th of E <= 64
+// stacked W, known on the device only; an expert's tiles follow each other.
+template <int MT, int NT, bool SWIGLU, bool GROUPED>
 __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
   constexpr int XB = 32 * MT * WG_BK, WB = 32 * NT * WG_BK;  // of a K step
   constexpr int TM = 32 * MT, TN = SWIGLU ? 16 * NT : 32 * NT;
@@ -90,8 +95,26 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave >> 1, wc = wave & 1;
   const int r16 = lane & 15, quad = lane >> 4;
-  const int mt = (a.M + TM - 1) / TM, nt = (a.N + TN - 1) / TN;
-  const int tiles = mt * nt, steps = a.K / WG_BK;
+  const int nt = (a.N + TN - 1) / TN, steps = a.K / WG_BK;
+  // of this workgroup's tile: the matrix's first row in x and its row count; of
+  // expert `lane`: its tiles, those up to it, its first row, its rows
+  int base = 0, M = a.M, expert = 0;
+  int mine = 0, upto = 0, first = 0, count = 0;
+  if (GROUPED) {
+    if (lane < a.E) {
+      first = a.start[lane];
+      count = a.start[lane + 1] - first;
+      mine = (count + TM - 1) / TM * nt;
+    }
+    upto = mine;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int up = __shfl_up(upto, d, 64);
+      if (lane >= d) upto += up;
+    }
+  }
+  const int tiles = GROUPED ? __builtin_amdgcn_readlane(upto, 63)
+                            : (a.M + TM - 1) / TM * nt;
 
   // Tile of round r; -1: none.  A round's tiles are dealt to the XCDs in
   // stretches (ids go round-robin over the XCDs), and a stretch is a patch of
@@ -104,9 +127,15 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
     return slot < per && at < left ? r * WG_BLOCKS + at : -1;
   };
   auto origin = [&](int tile, int* m0, int* n0) WG_INLINE {
+    if (GROUPED) {
+      expert = __builtin_ctzll(__ballot(upto > tile));
+      tile -= __builtin_amdgcn_readlane(upto - mine, expert);
+      base = __builtin_amdgcn_readlane(first, expert);
+      M = __builtin_amdgcn_readlane(count, expert);
+    }
     constexpr int GM = 4;
     const int panel = tile / (GM * nt), in = tile - panel * (GM * nt);
-    const int gm = min(GM, mt - panel * GM);
+    const int gm = min(GM, (M + TM - 1) / TM - panel * GM);
     *m0 = (panel * GM + in % gm) * TM;
     *n0 = in / gm * TN;
   };
@@ -119,15 +148,16 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
   wg_u32x4 xbuf, wbuf;
   int xo[MT], wo[NT];
   auto x_from = [&](int m0) WG_INLINE {
-    xbuf = wg_buffer(a.x + m0 * a.x_rs,
-                     ((a.M - 1 - m0) * a.x_rs + a.K) * 2);
+    xbuf = wg_buffer(a.x + (base + m0) * a.x_rs,
+                     ((M - 1 - m0) * a.x_rs + a.K) * 2);
 #pragma unroll
     for (int i = 0; i < MT; ++i)
-      xo[i] = min(i * 32 + prow, a.M - 1 - m0) * ((int)a.x_rs * 2) + pbyte;
+      xo[i] = min(i * 32 + prow, M - 1 - m0) * ((int)a.x_rs * 2) + pbyte;
   };
   auto w_from = [&](int n0) WG_INLINE {
     const int rows = SWIGLU ? 2 * a.N : a.N;
-    wbuf = wg_buffer(a.w + (int64_t)n0 * a.K, (int64_t)(rows - n0) * a.K * 2);
+    wbuf = wg_buffer(a.w + ((int64_t)expert * rows + n0) * a.K,
+                     (int64_t)(rows - n0) * a.K * 2);
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const int r = i * 32 + prow, half = r >= 16 * NT, in = r - half * 16 * NT;
@@ -248,7 +278,8 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
     step(Yes{}, true, 0, XB, 256, 384);
     step(No{}, false, XB, 0, 384, 512);
     const int next = tile_of(++round);
-    const int mc = m0, nc = n0;
+    const int mc = m0, nc = n0, Mc = M;
+    uint16_t* const oc = a.out + (int64_t)base * a.N;
     origin(next < 0 ? tile : next, &m0, &n0);
     int k = 512;
     for (int t = 2; t < steps - 4; t += 2, k += 256) {
@@ -268,7 +299,7 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
       const int row = mc + (wr * MT + m) * 16 + r16;
-      uint16_t* out = a.out + (int64_t)row * a.N;
+      uint16_t* out = oc + (int64_t)row * a.N;
       if (SWIGLU) {
         auto act = [&](int t, int e) WG_INLINE {
           const float g = acc[m][t][e];
@@ -282,20 +313,20 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
         for (int t = 0; t < (NT & ~3); t += 4) {
           const wg_u32x4 y = {pair(t), pair(t + 1), pair(t + 2), pair(t + 3)};
           const int at = n + t * 8 + quad * 8;
-          if (row < a.M && at < a.N)
+          if (row < Mc && at < a.N)
             *reinterpret_cast<wg_u32x4*>(out + at) = y;
         }
         if (NT & 2) {
           constexpr int t = NT & ~3;
           const wg_u32x2 y = {pair(t), pair(t + 1)};
           const int at = n + t * 8 + quad * 4;
-          if (row < a.M && at < a.N)
+          if (row < Mc && at < a.N)
             *reinterpret_cast<wg_u32x2*>(out + at) = y;
         }
         if (NT & 1) {
           const uint32_t y = pair(NT - 1);
           const int at = n + (NT - 1) * 8 + quad * 2;
-          if (row < a.M && at < a.N) *reinterpret_cast<uint32_t*>(out + at) = y;
+          if (row < Mc && at < a.N) *reinterpret_cast<uint32_t*>(out + at) = y;
         }
       } else {
         const int n = nc + wc * 16 * NT;
@@ -307,13 +338,13 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
           const wg_u32x4 y = {pair(t, 0), pair(t, 2), pair(t + 1, 0),
                               pair(t + 1, 2)};
           const int at = n + t * 16 + quad * 8;
-          if (row < a.M && at < a.N)
+          if (row < Mc && at < a.N)
             *reinterpret_cast<wg_u32x4*>(out + at) = y;
         }
         if (NT & 1) {
           const wg_u32x2 y = {pair(NT - 1, 0), pair(NT - 1, 2)};
           const int at = n + (NT - 1) * 16 + quad * 4;
-          if (row < a.M && at < a.N)
+          if (row < Mc && at < a.N)
             *reinterpret_cast<wg_u32x2*>(out + at) = y;
         }
       }
@@ -393,15 +424,15 @@ void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
   const WideArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)x.data_ptr(),
                    (const uint16_t*)w.data_ptr(), (int)M, (int)N, (int)K,
-                   x.stride(0)};
+                   x.stride(0), nullptr, 0};
 #define LAUNCH_WIDE(MT, NT)                                                   \
   case MT * 16 + NT:                                                          \
     if (swiglu)                                                               \
-      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, true>), dim3(WG_BLOCKS),   \
-                         dim3(256), 0, stream, a);                            \
+      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, true, false>),             \
+                         dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
     else                                                                      \
-      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, false>), dim3(WG_BLOCKS),  \
-                         dim3(256), 0, stream, a);                            \
+      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, false, false>),            \
+                         dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
     break
   switch (tile) {
     LAUNCH_WIDE(8, 8);
@@ -412,6 +443,85 @@ void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     default: TORCH_CHECK(false, "no such tile: ", tile);
   }
 #undef LAUNCH_WIDE
+  HIP_CHECK_KERNEL();
+}
+
+// Tiles of a grouped product and what a round of them costs (hundredths of one
+// of 256 x 256 over many rounds: fewer columns or rows come cheaper there than
+// above, where the rounds are few).
+static constexpr WideTile grouped_tiles[] = {
+    {8, 8, 98}, {8, 7, 85}, {6, 8, 77}, {6, 7, 69}, {4, 8, 57}, {4, 6, 45}};
+
+// The tile for `rows` rows that E experts share.  How many each has is known on
+// the device only; they spread by about the root of the mean, and four points
+// of that spread stand for the tiles that whole rounds are counted for
+// (us, by 16-row tiles of x and W; eight experts of 4096 and 14336: 4200 rows,
+// up 88 1008, 87 962, 68 837, 67 836, 48 986, down 617 599 527 483 566; 2048
+// rows, up 621 590 670 674 551, down 342 340 310 475 387; 128 rows, up 435 386
+// 394 365 372 and 46 356, down 263 267 241 203 204 and 175).
+int64_t grouped_tile(int64_t rows, int64_t E, int64_t N, bool swiglu) {
+  const double r = (double)rows / (double)E, s = std::sqrt(r);
+  int64_t best = 0;
+  double least = 0.0;
+  for (const auto& c : grouped_tiles) {
+    const int64_t nt = (N + (swiglu ? 16 : 32) * c.NT - 1) /
+                       ((swiglu ? 16 : 32) * c.NT);
+    double m = 0.0;
+    for (const double at : {r - 1.5 * s, r - 0.5 * s, r + 0.5 * s, r + 1.5 * s})
+      m += std::max(1.0, std::ceil(at / (32 * c.MT))) / 4.0;
+    const double cost = std::ceil(m * (E * nt) / WG_BLOCKS) * c.cost;
+    if (best == 0 || cost < least) {
+      best = c.MT * 16 + c.NT;
+      least = cost;
+    }
+  }
+  return best;
+}
+
+// out[r] = x[r] W_e^T for the rows start[e] .. start[e + 1] - 1 of every expert
+// e, w [E, N or 2 N, K]; rows past start[E] are left alone.
+void grouped_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                  torch::Tensor start, bool swiglu, int64_t tile) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.is_contiguous() &&
+              x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
+              w.dim() == 3 && w.is_contiguous() && out.dim() == 2 &&
+              out.is_contiguous() && out.dtype() == x.dtype() &&
+              start.dtype() == torch::kInt32 && start.is_contiguous());
+  const int64_t R = x.size(0), K = x.size(1), N = out.size(1), E = w.size(0);
+  TORCH_CHECK(R >= 1 && E >= 1 && E <= 64 && start.numel() == E + 1 && N >= 8 &&
+              N % 8 == 0 && K >= 6 * WG_BK && K % (2 * WG_BK) == 0 &&
+              R < (1 << 30) && N < (1 << 30) && wide_gemm_fits(K, N, K, swiglu));
+  TORCH_CHECK(out.size(0) == R && w.size(2) == K &&
+              w.size(1) == (swiglu ? 2 * N : N));
+  TORCH_CHECK(w.device() == x.device() && out.device() == x.device() &&
+                  start.device() == x.device(),
+              "tensors on different devices");
+  for (const auto* t : {&out, &x, &w})
+    TORCH_CHECK((reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) == 0);
+  const at::cuda::CUDAGuard guard(x.device());
+  hipStream_t stream = at::cuda::getCurrentCUDAStream();
+  const WideArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)x.data_ptr(),
+                   (const uint16_t*)w.data_ptr(), (int)R, (int)N, (int)K, K,
+                   (const int32_t*)start.data_ptr(), (int)E};
+#define LAUNCH_GROUPED(MT, NT)                                                \
+  case MT * 16 + NT:                                                          \
+    if (swiglu)                                                               \
+      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, true, true>),              \
+                         dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
+    else                                                                      \
+      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, false, true>),             \
+                         dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
+    break
+  switch (tile > 0 ? tile : grouped_tile(R, E, N, swiglu)) {
+    LAUNCH_GROUPED(8, 8);
+    LAUNCH_GROUPED(8, 7);
+    LAUNCH_GROUPED(6, 8);
+    LAUNCH_GROUPED(6, 7);
+    LAUNCH_GROUPED(4, 8);
+    LAUNCH_GROUPED(4, 6);
+    default: TORCH_CHECK(false, "no such tile: ", tile);
+  }
+#undef LAUNCH_GROUPED
   HIP_CHECK_KERNEL();
 }
 

@@ -24,7 +24,10 @@ def _hip_sources(d):
                   if not p.name.endswith("_hip.hip"))
 
 
-sources = [str(CSRC / "bindings.cpp")] + _hip_sources(CSRC)
+STR = ROOT / "inference_gateway_amd" / "ops" / "csrc_streams"
+# the dispatch and combine kernels of the mixture-of-experts layers are shared
+sources = ([str(CSRC / "bindings.cpp")] + _hip_sources(CSRC)
+           + [str(STR / "stream_ops.hip")])
 HYB = ROOT / "inference_gateway_amd" / "ops" / "csrc_hybrid"
 hybrid_sources = [str(HYB / "bindings.cpp")] + _hip_sources(HYB)
 
@@ -46,7 +49,6 @@ postnorm_sources = [str(PN / "bindings.cpp")] + [
 
 # the multi-stream extension: its own kernels plus the attention, row and
 # router kernels its models launch
-STR = ROOT / "inference_gateway_amd" / "ops" / "csrc_streams"
 streams_sources = [str(STR / "bindings.cpp")] + _hip_sources(STR) + [
     str(HYB / f) for f in ("hybrid_ops.hip", "latent_attn.hip",
                            "latent_attn_mfma.hip", "latent_decode.hip",

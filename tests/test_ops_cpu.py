@@ -306,6 +306,34 @@ def test_moe_few_takes():
     assert not takes(torch.randn(9, 64).to(bf), gu, dn)
 
 
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+def test_moe_rows_takes():
+    bf = torch.bfloat16
+    x, gu, dn = (torch.empty(*s, dtype=bf) for s in (
+        (30, 512), (4, 768, 512), (4, 512, 384)))
+
+    def takes(x, gu, dn, k=2):
+        return ops._kernels.moe_rows_takes(x, gu, dn, k, True)
+
+    assert takes(x, gu, dn) and takes(x, gu, dn, 4) and takes(x[:1], gu, dn)
+    assert not takes(x, gu, dn, 3)
+    assert not takes(x, gu, dn, 8)                  # more than there are
+    assert not takes(x[:0], gu, dn)
+    assert not takes(x, gu.to("meta"), dn)
+    assert not takes(x, gu, dn.to("meta"))
+    assert not takes(x.float(), gu.float(), dn.float())
+    assert not takes(x, gu, dn.clone().requires_grad_())
+    assert not takes(x[:, :256], gu[:, :, :256].contiguous(), dn[:, :256]
+                     .contiguous())                 # too short a K
+    assert not takes(torch.empty(30, 576, dtype=bf), torch.empty(
+        4, 768, 576, dtype=bf), torch.empty(4, 576, 384, dtype=bf))
+    assert not takes(torch.empty(30, 520, dtype=bf)[:, :512], gu, dn)
+    assert not takes(x, gu[:3], dn)
+    assert not takes(x, gu[:, :760], dn)
+    assert not takes(x, torch.empty(65, 768, 512, dtype=bf),
+                     torch.empty(65, 512, 384, dtype=bf))
+
+
 def test_linear_is_the_library_under_a_symbolic_trace():
     class M(torch.nn.Module):
         def __init__(self):
