@@ -6,12 +6,10 @@
 // the q rows are a chunk behind `prefix` cached tokens and row r sits at
 // position prefix + r; the chunk's own keys are already appended).
 //
-// Measured with 32 heads on 8: one prompt of 16000 tokens 2145 us, 978
-// TFLOP/s (64 x 64 tiles of 16x16x32 MFMAs with V transposed by the stores
-// and P through LDS: 12518 us); 16 prompts of 512 82 us (416); 2000 rows
-// behind 6000 cached ones 277 us, 828 TFLOP/s (1552).  With a maximum raised
-// only when it is outgrown, and sums of rounded weights, 2070, 81 and 266, at
-// a larger error.
+// Measured with 32 heads on 8 (cards differ by 10 %): one prompt of 16000
+// tokens 1948 us, 1077 TFLOP/s (64 x 64 tiles of 16x16x32 MFMAs with V
+// transposed by the stores and P through LDS: 12518 us); 16 prompts of 512 70
+// us, 490 TFLOP/s; 2000 rows behind 6000 cached ones 256 us, 900 TFLOP/s.
 
 #include <ATen/cuda/CUDAContext.h>
 #include <torch/extension.h>

@@ -22,8 +22,9 @@
 //     four LDS objects so that the reads of one buffer do not wait for the
 //     writes to the other;
 //   * 16-byte chunks are XOR-swizzled by row (on the global side, a DMA
-//     writes LDS linearly): K by row & 7 against the 32 rows of a fragment,
-//     V by the rows that one transposing read spreads over its lanes;
+//     writes LDS linearly): K so that the 16 rows that the LDS serves at a time
+//     of a fragment's 32 (0-3, 12-15, 20-27, and the rest) lie in different
+//     banks, V by the rows that one transposing read spreads over its lanes;
 //   * the accumulators are rescaled only where a row of the wave has a new
 //     maximum, which gets rare along the keys (raising it only when it is
 //     outgrown by 2^8 leaves the largest weight another value than one and
@@ -32,7 +33,14 @@
 //     part, and a wave skips tiles that none of its rows sees.
 //
 // Two waves per SIMD (256 registers, up to 80 KB of LDS per workgroup) let
-// one wave's softmax run beside the other's MFMAs.
+// one wave's softmax run beside the other's MFMAs.  A wave waits a fifth of its
+// time (for LDS reads and its workgroup), so what it can it has under way: K
+// fragments four products ahead, V one step, the weights of the second 32 keys
+// between the products of the first.  Next to nothing is left of the addresses
+// of tiles that lie whole in one sequence.  One prompt of 16000 tokens, 32
+// heads on 8, before and after these: 2290 and 2148 us, of 4000 178 and 157,
+// 16 of 512 77 and 70, 2000 rows behind 6000 277 and 256.  Computing the next
+// tile's scores beside this one's weights wants more registers than there are.
 #pragma once
 
 #include <climits>
@@ -50,6 +58,9 @@ typedef __attribute__((ext_vector_type(16))) float ft_f32x16;
 constexpr int FT_BN = 64;    // keys per tile
 constexpr int FT_WAVES = 4;  // waves per workgroup, 32 query rows each
 constexpr int FT_BM = 32 * FT_WAVES;
+#define FT_INLINE __attribute__((always_inline))
+// classes of instructions, as __builtin_amdgcn_sched_group_barrier names them
+constexpr int FT_VALU = 0x2, FT_MFMA = 0x8, FT_DS_READ = 0x100;
 constexpr float FT_LOG2E = 1.44269504088896340736f;
 
 // two floats -> packed bf16 pair, round to nearest even
@@ -145,7 +156,9 @@ static __device__ const uint16_t ft_zeros[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 // K and V rows of one sequence.  begin(kbase, wave) is called before the
 // addresses of a tile are asked for, with the wave (which moves the tile's
 // rows 16 wave .. + 15); rows past the last key repeat it (they are masked).
-// prefetch(kbase, wave) is called one tile ahead.
+// prefetch(kbase, wave) is called one tile ahead.  STRAIGHT sources also have
+// tiles (straight(kbase)) whose chunks lie at a scalar base per tile and wave
+// and at lane offsets, in bytes, that are the same for all of them.
 
 // In pages of any size; with a multiple of 16 a wave's rows lie in one page,
 // whose number was asked for one tile ahead, and the address is a scalar base
@@ -191,6 +204,16 @@ struct PagedRows {
   }
   // values past the width are not stored
   DEVINLINE const uint16_t* vp(int r, int c) const { return at(v, vw, r, c); }
+  static constexpr bool STRAIGHT = true;
+  DEVINLINE bool straight(int kbase) const {
+    return size % 16 == 0 && kbase + FT_BN <= kv_len;
+  }
+  DEVINLINE const uint16_t* k_base() const { return k + base * kw; }
+  DEVINLINE const uint16_t* v_base() const { return v + base * vw; }
+  DEVINLINE int k_off(int r, int c) const { return (r & 15) * kw * 2 + c * 16; }
+  DEVINLINE int v_off(int r, int c) const {
+    return (r & 15) * vw * 2 + (c * 8 < vw ? c * 16 : 0);
+  }
 };
 
 // Dense: k and v point to the sequence's first row, this head.  A tile's rows
@@ -215,12 +238,28 @@ struct DenseRows {
   DEVINLINE const uint16_t* vp(int r, int c) const {
     return vt + (uint32_t)(min(r, last) * v_rs + c * 8);
   }
+  static constexpr bool STRAIGHT = true;
+  DEVINLINE bool straight(int kbase) const { return kbase + FT_BN <= kv_len; }
+  DEVINLINE const uint16_t* k_base() const { return kt; }
+  DEVINLINE const uint16_t* v_base() const { return vt; }
+  DEVINLINE int k_off(int r, int c) const { return r * k_rs * 2 + c * 16; }
+  DEVINLINE int v_off(int r, int c) const { return r * v_rs * 2 + c * 16; }
 };
 
 // Swizzle of V's 16-byte chunks in row r.
 template <int NV>
 DEVINLINE int ft_vswz(int r) {
   return NV >= 128 ? (r & 3) << 2 : ((r >> 1) & 1) << 2;
+}
+
+// Swizzle of the 16-byte chunks of K row r, rows of NK entries: 256 bytes apart
+// in the banks' 256 (or a multiple), or 128 (with SHARED the transposing reads
+// of four neighbouring rows want bit 2 to tell rows 0 and 2 apart).  By r & 7
+// two rows met in a bank at every fragment.
+template <int NK>
+DEVINLINE int ft_kswz(int r) {
+  static_assert(NK % 64 == 0);
+  return NK % 128 == 0 ? r & 15 : (r & 2) << 1 | (r >> 2 & 3);
 }
 
 // Walks the tiles.  qf: the query row as B operand (dims 16 s + 8 half);
@@ -246,32 +285,69 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = lane >> 5, col = lane & 31;
 
-  auto stage = [&](int kbase, uint8_t* kd, uint8_t* vd) {
+  // rows and chunks of this lane's pieces
+  auto k_row = [&](int i) { return wave * RW + (i * 64 + lane) / CK; };
+  auto k_chunk = [&](int i) {
+    return ((i * 64 + lane) % CK) ^ ft_kswz<NK>(k_row(i));
+  };
+  constexpr int CV1 = CV > 0 ? CV : 1;
+  auto v_row = [&](int i) { return wave * RW + (i * 64 + lane) / CV1; };
+  auto v_chunk = [&](int i) {
+    return ((i * 64 + lane) % CV1) ^ ft_vswz<NV>(v_row(i));
+  };
+  // Addresses of whole tiles cost the vector units nothing: they are a scalar
+  // base and these offsets (64-bit sums per lane were a third of the vector
+  // instructions of a tile).
+  constexpr bool STRAIGHT = Rows::STRAIGHT && NK <= 256;
+  int ko[CK / 4], vo[CV / 4 + 1];
+  if constexpr (STRAIGHT) {
+#pragma unroll
+    for (int i = 0; i < CK / 4; ++i) ko[i] = rows.k_off(k_row(i), k_chunk(i));
+#pragma unroll
+    for (int i = 0; i < CV / 4; ++i) vo[i] = rows.v_off(v_row(i), v_chunk(i));
+  }
+  auto stage = [&](int kbase, uint8_t* kd, uint8_t* vd) FT_INLINE {
     rows.begin(kbase, wave);
-    auto keys = [&](auto pad) {
+    bool straight = false;
+    if constexpr (STRAIGHT) {
+      straight = rows.straight(kbase) && rows.key_width() >= NK;
+      if (straight) {
+        typedef __attribute__((address_space(3))) void lds_void;
+        const auto kr = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)rows.k_base(), 0, -1, 0x00020000);
+        const auto vr = __builtin_amdgcn_make_buffer_rsrc(
+            (void*)rows.v_base(), 0, -1, 0x00020000);
 #pragma unroll
-      for (int i = 0; i < CK / 4; ++i) {
-        const int r = wave * RW + (i * 64 + lane) / CK;
-        const int c = ((i * 64 + lane) % CK) ^ (r & 7);
-        __builtin_amdgcn_global_load_lds(
-            reinterpret_cast<const uint32_t*>(
-                rows.template kp<decltype(pad)::value>(r, c)),
-            reinterpret_cast<uint32_t*>(kd + (wave * (CK / 4) + i) * 1024),
-            16, 0, 0);
+        for (int i = 0; i < CK / 4; ++i)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              kr, (lds_void*)(kd + (wave * (CK / 4) + i) * 1024), 16, ko[i], 0,
+              0, 0);
+#pragma unroll
+        for (int i = 0; i < CV / 4; ++i)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              vr, (lds_void*)(vd + (wave * (CV / 4) + i) * 1024), 16, vo[i], 0,
+              0, 0);
       }
-    };
-    // where nothing is padded the address stays a scalar base and an offset
-    if (rows.key_width() < NK) keys(std::true_type{});
-    else keys(std::false_type{});
+    }
+    if (!straight) {
+      auto keys = [&](auto pad) {
 #pragma unroll
-    for (int i = 0; i < CV / 4; ++i) {
-      constexpr int C = CV > 0 ? CV : 1;
-      const int r = wave * RW + (i * 64 + lane) / C;
-      const int c = ((i * 64 + lane) % C) ^ ft_vswz<NV>(r);
-      __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const uint32_t*>(rows.vp(r, c)),
-          reinterpret_cast<uint32_t*>(vd + (wave * (CV / 4) + i) * 1024), 16,
-          0, 0);
+        for (int i = 0; i < CK / 4; ++i)
+          __builtin_amdgcn_global_load_lds(
+              reinterpret_cast<const uint32_t*>(
+                  rows.template kp<decltype(pad)::value>(k_row(i), k_chunk(i))),
+              reinterpret_cast<uint32_t*>(kd + (wave * (CK / 4) + i) * 1024),
+              16, 0, 0);
+      };
+      // where nothing is padded the address stays a scalar base and an offset
+      if (rows.key_width() < NK) keys(std::true_type{});
+      else keys(std::false_type{});
+#pragma unroll
+      for (int i = 0; i < CV / 4; ++i)
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const uint32_t*>(rows.vp(v_row(i), v_chunk(i))),
+            reinterpret_cast<uint32_t*>(vd + (wave * (CV / 4) + i) * 1024), 16,
+            0, 0);
     }
     rows.prefetch(span.next(kbase), wave);
   };
@@ -280,7 +356,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
   int koff[NK / 16];  // K row `col` (+ 32 per sub-tile), dims 16 s + 8 half
 #pragma unroll
   for (int s = 0; s < NK / 16; ++s)
-    koff[s] = col * (NK * 2) + (((2 * s + half) ^ (col & 7)) << 4);
+    koff[s] = col * (NK * 2) + (((2 * s + half) ^ ft_kswz<NK>(col)) << 4);
   int voff[VD / 32][2];  // V^T: dims 32 dt + 16 (lane bit 4), keys 4 half + 8 e
 #pragma unroll
   for (int dt = 0; dt < VD / 32; ++dt)
@@ -290,7 +366,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
       const int c =
           dim0 / 8 + 4 * dt + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
       voff[dt][e] = r * VROW +
-                    ((c ^ (SHARED ? r & 7 : ft_vswz<NV>(r))) << 4) +
+                    ((c ^ (SHARED ? ft_kswz<NK>(r) : ft_vswz<NV>(r))) << 4) +
                     8 * (i & 1);
     }
 
@@ -318,15 +394,33 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int i = 0; i < 16; ++i) s[t][i] = 0.0f;
+    // K fragments are read KD products ahead (left to itself the compiler reads
+    // a pair, waits for it and uses it)
+    constexpr int KD = NK / 16 < 4 ? NK / 16 : 4;
+    ft_bf16x8 kf[KD][2];
+    auto read_k = [&](int d) FT_INLINE {
 #pragma unroll
-    for (int d = 0; d < NK / 16; ++d)
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const ft_bf16x8 kf = *reinterpret_cast<const ft_bf16x8*>(
+      for (int t = 0; t < 2; ++t)
+        kf[d % KD][t] = *reinterpret_cast<const ft_bf16x8*>(
             kb + koff[d] + t * 32 * NK * 2);
-        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[d], s[t], 0, 0,
-                                                       0);
-      }
+    };
+#pragma unroll
+    for (int d = 0; d < KD; ++d) read_k(d);
+#pragma unroll
+    for (int d = 0; d < NK / 16; ++d) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+        s[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[d % KD][t], qf[d],
+                                                       s[t], 0, 0, 0);
+      if (d + KD < NK / 16) read_k(d + KD);
+    }
+    __builtin_amdgcn_sched_group_barrier(FT_DS_READ, 2 * KD, 0);
+#pragma unroll
+    for (int d = 0; d < NK / 16; ++d) {
+      __builtin_amdgcn_sched_group_barrier(FT_MFMA, 2, 0);
+      if (d + KD < NK / 16) __builtin_amdgcn_sched_group_barrier(FT_DS_READ, 2, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
 
     if (!PLAIN) {
       if (sc.cap > 0.0f) {
@@ -357,13 +451,16 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
     bool partly = kbase + BN - 1 > sc.wave_pos;
     if (!PLAIN) partly |= kbase < sc.wave_lo[1] && kbase + BN > sc.keep;
     if (partly) {
+      const int seen = min(sc.pos, span.kv_len - 1) - kbase - 4 * half;
+      const int lo = sc.lo - kbase - 4 * half;
+      const int keep = sc.keep - kbase - 4 * half;
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-          const int kpos = kbase + 32 * t + (i & 3) + 8 * (i >> 2) + 4 * half;
-          bool hide = kpos > sc.pos || kpos >= span.kv_len;
-          if (!PLAIN) hide |= kpos < sc.lo && kpos >= sc.keep;
+          const int key = 32 * t + (i & 3) + 8 * (i >> 2);
+          bool hide = key > seen;
+          if (!PLAIN) hide |= key < lo && key >= keep;
           if (hide) s[t][i] = -INFINITY;
         }
     }
@@ -391,47 +488,68 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
         for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
     }
     const float mc = m == -INFINITY ? 0.0f : m * c;
+    // Weights of 32 keys, and their products with V 16 keys at a time: those of
+    // the second 32 are computed between the products of the first, and V
+    // fragments are read one step of products ahead.
+    uint32_t p[2][8];
+    auto weigh = [&](int t) FT_INLINE {
+      float sum = 0.0f;
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i)
+      for (int i = 0; i < 16; ++i) {
         s[t][i] = __builtin_amdgcn_exp2f(PLAIN ? fmaf(s[t][i], c, -mc)
                                                : s[t][i] - mc);
-    float sum[2] = {0.0f, 0.0f};
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) sum[t] += s[t][i];
-    l += sum[0] + sum[1];
-
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        union {
-          uint32_t u[4];
-          ft_bf16x8 v;
-        } pf;
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          pf.u[e] = ft_pack_bf16(s[t][8 * ks + 2 * e],
-                                 s[t][8 * ks + 2 * e + 1]);
-#pragma unroll
-        for (int dt = 0; dt < VD / 32; ++dt) {
-          typedef __attribute__((address_space(3))) ft_short4 lds_short4;
-          union {
-            ft_short4 h[2];
-            ft_bf16x8 v;
-          } vf;
-#pragma unroll
-          for (int e = 0; e < 2; ++e)
-            vf.h[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                (lds_short4*)((SHARED ? kb : vb) + voff[dt][e] +
-                              (32 * t + 16 * ks) * VROW));
-          o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf.v, o[dt],
-                                                          0, 0, 0);
-        }
+        sum += s[t][i];
       }
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        p[t][i] = ft_pack_bf16(s[t][2 * i], s[t][2 * i + 1]);
+      return sum;
+    };
+    union {
+      ft_short4 h[2];
+      ft_bf16x8 v;
+    } vf[2][VD / 32];
+    auto read_v = [&](int j) FT_INLINE {
+      typedef __attribute__((address_space(3))) ft_short4 lds_short4;
+#pragma unroll
+      for (int dt = 0; dt < VD / 32; ++dt)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          vf[j & 1][dt].h[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+              (lds_short4*)((SHARED ? kb : vb) + voff[dt][e] + 16 * j * VROW));
+    };
+    __builtin_amdgcn_sched_barrier(0);
+    read_v(0);
+    const float sum0 = weigh(0);
+    __builtin_amdgcn_sched_barrier(0);
+    float sum1 = 0.0f;
+    __builtin_amdgcn_s_setprio(1);   // before the other wave's softmax
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (j < 3) read_v(j + 1);
+      if (j == 0) sum1 = weigh(1);
+      union {
+        uint32_t u[4];
+        ft_bf16x8 v;
+      } pf;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) pf.u[e] = p[j >> 1][(j & 1) * 4 + e];
+#pragma unroll
+      for (int dt = 0; dt < VD / 32; ++dt)
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[j & 1][dt].v, pf.v,
+                                                        o[dt], 0, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < VD / 8; ++i) {
+      __builtin_amdgcn_sched_group_barrier(FT_MFMA, 1, 0);
+      if (i < 3 * (VD / 32))
+        __builtin_amdgcn_sched_group_barrier(FT_DS_READ, 2, 0);
+      if (i < 2 * (VD / 32))
+        __builtin_amdgcn_sched_group_barrier(FT_VALU, 224 / VD * 4, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(0);
+    l += sum0 + sum1;
   };
 
   int kb = span.begin();

@@ -39,6 +39,7 @@ struct LatentRows {
     vt = v + (int64_t)kbase * v_rs;
     last = kv_len - 1 - kbase;
   }
+  static constexpr bool STRAIGHT = false;   // keys from two places
   DEVINLINE int key_width() const { return dk; }
   template <bool PAD>
   DEVINLINE const uint16_t* kp(int r, int c) const {
