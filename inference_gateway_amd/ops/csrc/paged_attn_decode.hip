@@ -3,23 +3,24 @@
 // Net-new engine scope (SURVEY.md §7 stage 3b): single-query attention over a
 // paged KV cache, GQA-aware. One workgroup per (sequence, kv_head); the GQA
 // group's G query heads ride along so each K/V byte is read exactly once per
-// step. Decode attention is HBM-bound; the kernel is built around coalesced
-// traffic and LATENCY HIDING (profiles/r01: the naive per-head loop was
-// latency-bound at 2.5 TB/s, 8x the per-iteration roofline):
+// step.  Bound by reading the cache; what a wave needs besides is kept small so
+// that its loads are always under way:
 //
-//   * cache layout [num_blocks, n_kv_heads, block_size=16, head_dim] gives a
-//     contiguous 16x128 bf16 tile (4 KiB) per (block, head);
-//   * K pass: 64 lanes x 64 B (4 lanes per token x 32-dim segment); all G
-//     head dot-products are computed back-to-back so their shfl reduction
-//     chains overlap (ILP across heads instead of serial per-head chains);
-//   * token-axis reductions use 4 shfl_xor steps (offsets 4,8,16,32 — the
-//     token index lives in lane bits 2..5), not a full 6-step wave reduce;
-//   * V rows for the CURRENT block and K rows for the NEXT block are issued
-//     before the softmax shfl chain, so HBM latency hides under it;
-//   * P values reach the V-pass lanes via ds_bpermute (no LDS round trip);
-//   * V pass: 16 lanes x 8 contiguous dims (b128 reads), 4 token subgroups,
-//     partials folded with 2 shfl_xor at the end;
-//   * waves stripe over cache blocks and merge via LDS once at the end
+//   * a wave takes two pages (32 tokens) at a time, K straight to the registers
+//     that the matrix instructions read it from, V by DMA to LDS, both one step
+//     ahead: 16 KB a wave, 128 KB a compute unit under way;
+//   * scores: S^T = K Q^T with mfma 16x16x32, the query heads in the columns
+//     (those past G are zero): 8 instructions for what took 256 dot products;
+//   * the result's token order follows from the layout of S^T and V is read from
+//     LDS in the same order (ds_read_b64_tr_b16), so weights stay in their
+//     lanes;
+//   * weights keep 16 bits of their mantissa: two bf16 parts, truncated part
+//     and rest, and two products (the matrix cores are idle otherwise).  The
+//     rest is never zero, so that an infinite value stays infinite;
+//   * addresses are a scalar base per page and fixed lane offsets; rows past a
+//     part's end lie past the buffer descriptor's and read as zeros, without a
+//     branch, so that the compiler knows which loads are under way;
+//   * waves stripe over pairs of pages and merge via LDS once at the end
 //     (flash-decoding style rescale);
 //   * a sequence's pages are split over up to nsplit workgroups when
 //     sequences x key/value heads alone do not fill the chip.  The split is
@@ -27,7 +28,13 @@
 //     stays right as contexts grow); the parts' unnormalised sums (fp32) are
 //     merged by a second kernel.
 //
-// Wavefront-64 throughout; no CUDA-isms, no Triton.
+// Measured, with dot products and fp32 multiply-adds on the vector units (450
+// instructions a page) and here (32 heads on 8, us): 1024 sequences of 554 to
+// 590 tokens 466 and 410 (5.9 TB/s), 300 of 3000 764 and 637, 61 of 200 to 4000
+// 134 and 104, 128 of 100 to 2000 159 and 109, 16 of 500 16.5 and 11.2; 64 heads
+// on 8, 64 of 400 to 4000 250 and 119.  One, two or eight waves a workgroup:
+// 691, 654, 635 for the 637, 120, 119, 108 for the 109, 114, 109, 114 for the
+// 104.
 
 #include <ATen/cuda/CUDAContext.h>
 #include <torch/extension.h>
@@ -36,39 +43,63 @@
 
 namespace igw {
 
-typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+typedef __attribute__((ext_vector_type(4))) short pd_short4;
+typedef __attribute__((ext_vector_type(8))) __bf16 pd_bf16x8;
+typedef __attribute__((ext_vector_type(4))) float pd_f32x4;
+typedef __attribute__((ext_vector_type(4))) uint32_t pd_u32x4;
 
-// xor-reduce over the token axis (lane bits 2..5); values stay replicated
-DEVINLINE float token_reduce_max(float x) {
-  x = fmaxf(x, __shfl_xor(x, 4, WAVE_SIZE));
-  x = fmaxf(x, __shfl_xor(x, 8, WAVE_SIZE));
-  x = fmaxf(x, __shfl_xor(x, 16, WAVE_SIZE));
-  x = fmaxf(x, __shfl_xor(x, 32, WAVE_SIZE));
-  return x;
+#define PD_INLINE __attribute__((always_inline))
+constexpr float PD_LOG2E = 1.44269504088896340736f;
+
+// x of lanes i and i ^ 16 (i ^ 32) in a and b of both.  Written out because the
+// compiler folds the builtins' two results into one when their operands are
+// equal; the s_nops are the waits that the swaps need.
+DEVINLINE void pd_both16(float x, float& a, float& b) {
+  a = b = x;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 0" : "+v"(a), "+v"(b));
+}
+DEVINLINE void pd_both32(float x, float& a, float& b) {
+  a = b = x;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 0" : "+v"(a), "+v"(b));
 }
 
-DEVINLINE float token_reduce_sum(float x) {
-  x += __shfl_xor(x, 4, WAVE_SIZE);
-  x += __shfl_xor(x, 8, WAVE_SIZE);
-  x += __shfl_xor(x, 16, WAVE_SIZE);
-  x += __shfl_xor(x, 32, WAVE_SIZE);
-  return x;
+// maximum and sum over the four lanes that share lane & 15
+DEVINLINE float pd_max(float x) {
+  float a, b;
+  pd_both16(x, a, b);
+  pd_both32(fmaxf(a, b), a, b);
+  return fmaxf(a, b);
+}
+DEVINLINE float pd_sum(float x) {
+  float a, b;
+  pd_both16(x, a, b);
+  pd_both32(a + b, a, b);
+  return a + b;
+}
+
+DEVINLINE uint32_t pd_pack(float a, float b) {
+  typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
+  const f32x2_t v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
 }
 
 // How a sequence of ctx tokens is cut for nsplit workgroups: `count` parts of
-// `blocks` pages, a part no shorter than min_blocks pages.
+// `blocks` pages, a part no shorter than min_blocks pages.  Up to 32 pages are
+// not cut: what a merge costs is not won back (1 sequence of 200 tokens 5.7 us
+// whole, 7.2 cut; of 500 8.0 and 8.2, of 700 9.8 and 9.1, of 1500 16.4 and 8.9).
 struct DecodeSplit {
   int blocks, count;
   DEVINLINE DecodeSplit(int ctx, int nsplit, int min_blocks) {
     const int n = (ctx + 15) / 16;
     blocks = max((n + nsplit - 1) / nsplit, min_blocks);
-    if (nsplit == 1) blocks = max(n, 1);
+    if (nsplit == 1 || n <= 32) blocks = max(n, 1);
     count = max((n + blocks - 1) / blocks, 1);
   }
 };
 
-template <int HD, int G, int NWAVES>
-__global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
+template <int G, int NWAVES>
+__global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel(
     uint16_t* __restrict__ out,          // [B, NQ, HD]
     const uint16_t* __restrict__ q,      // [B, NQ, HD]
     const uint16_t* __restrict__ kcache, // [NB, NKV, BS, HD]
@@ -77,221 +108,207 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
     const int32_t* __restrict__ ctx_lens,    // [B]
     int max_blocks, int nkv, float scale, int q_rs,
     float* __restrict__ part_o,   // [B, NQ, nsplit, HD] when nsplit > 1
-    float* __restrict__ part_ml,  // [B, NQ, nsplit, 2]: maximum, sum
+    float* __restrict__ part_ml,  // [B, NQ, nsplit, 2]: maximum (log2), sum
     int nsplit, int min_blocks) {
   // q_rs: q row stride in elements (q may be a view into the fused QKV
   // GEMM output — no .contiguous() copy on the decode hot path)
-  constexpr int BS = 16;  // tokens per cache block
+  constexpr int HD = 128, BS = 16, PAGE = BS * HD;  // tokens, entries of a page
+  static_assert(NWAVES * G <= 64, "a wave's results fit its V tiles");
+  // a wave's own V tiles, two pages each: nothing here waits for another wave.
+  // Two objects, so that reads of one do not wait for loads to the other.
+  __shared__ __attribute__((aligned(1024))) uint16_t v_s0[NWAVES][2 * PAGE];
+  __shared__ __attribute__((aligned(1024))) uint16_t v_s1[NWAVES][2 * PAGE];
+  __shared__ float m_lds[NWAVES][G];
+  __shared__ float l_lds[NWAVES][G];
   const int kvh = blockIdx.x;
   const int seq = blockIdx.y;
   const int nq = nkv * G;
-  const int ctx = ctx_lens[seq];
+  const int ctx = __builtin_amdgcn_readfirstlane(ctx_lens[seq]);
   const int split = blockIdx.z;
   const DecodeSplit part(ctx, nsplit, min_blocks);
   if (split >= part.count) return;
   const int block0 = split * part.blocks;
   const int nblocks = min((ctx + BS - 1) / BS, block0 + part.blocks);
+  const int limit = min(ctx, nblocks * BS);        // the part's tokens end here
+  const int pairs = (nblocks - block0 + 1) >> 1;   // wave, wave + NWAVES, ...
 
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE_SIZE - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-
-  __shared__ uint16_t q_lds[G][HD];
-  __shared__ float m_lds[NWAVES][G];
-  __shared__ float l_lds[NWAVES][G];
-  __shared__ float acc_lds[NWAVES][G][HD];
-
-  // stage Q into LDS (raw bf16; scale is applied to the scores so Q keeps
-  // full precision and the per-lane register image stays PACKED — an
-  // unpacked fp32 Q image is 128 VGPRs for G=4 and collapses occupancy)
-  for (int i = tid * 8; i < G * HD; i += NWAVES * WAVE_SIZE * 8) {
-    *reinterpret_cast<ushort8*>(&q_lds[0][0] + i) =
-        *reinterpret_cast<const ushort8*>(
-            q + (int64_t)seq * q_rs + (kvh * G) * HD + i);
-  }
-  __syncthreads();
-
-  const int tok = lane >> 2;        // K pass: 16 tokens per tile
-  const int seg = (lane & 3) * 32;  // 32-dim segment for the K dot
-  const int vlane = lane & 15;      // V pass: dims [vlane*8, vlane*8+8)
-  const int vtok = lane >> 4;       // V pass: tokens t = vtok + 4*t4
-
-  float m[G], l[G], acc[G][8];
-#pragma unroll
-  for (int j = 0; j < G; ++j) {
-    m[j] = -INFINITY;
-    l[j] = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) acc[j][e] = 0.0f;
-  }
-
-  const int64_t head_off = (int64_t)kvh * BS * HD;
+  const int r16 = lane & 15, quad = lane >> 4;
   const int32_t* bt_row = block_table + (int64_t)seq * max_blocks;
 
-  // raw (unconverted) K tile registers for the current block
-  ushort8 kraw[4];
-
-  // page numbers of this wave's next 64 pages, one per lane: a K address
-  // does not wait for a table entry, and its base is in scalar registers
-  const int b0 = block0 + wave;
+  // page numbers of this wave's next 32 pairs, one per lane: an address does
+  // not wait for a table entry, and its base is in scalar registers
   int ids = 0;
-  auto load_ids = [&](int b) {
-    const int i = b + lane * NWAVES;
-    ids = i < nblocks ? bt_row[i] : 0;
+  auto load_ids = [&](int u) PD_INLINE {
+    const int b = block0 + 2 * (u + (lane >> 1) * NWAVES) + (lane & 1);
+    ids = bt_row[min(b, nblocks - 1)];
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // here, not at every use
   };
-  auto page_of = [&](int b) {
-    return (int64_t)__builtin_amdgcn_readlane(ids, ((b - b0) / NWAVES) & 63);
-  };
-  load_ids(b0);
+  if (wave < pairs) load_ids(wave);
 
-  auto load_k = [&](int b, ushort8* dst) {
-    const uint16_t* kp = kcache + page_of(b) * nkv * BS * HD + head_off +
-                         (tok * HD + seg);
+  // the query heads as columns: head r16, dims 32 kk + 8 quad ..
+  pd_bf16x8 qf[4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      dst[c] = *reinterpret_cast<const ushort8*>(kp + c * 8);
-  };
-
-  if (b0 < nblocks) load_k(b0, kraw);
-
-  for (int b = b0; b < nblocks; b += NWAVES) {
-    // ---- scores for all G heads via v_dot2_f32_bf16: Q and K stay
-    //      PACKED (no bf16 unpack VALU — v3's unpack loop made the
-    //      kernel VALU-bound).  Q is re-read from LDS per head per block
-    //      with the head loop NOT unrolled and the source pointer made
-    //      opaque: a persistent (or unroll-duplicated) packed-Q image
-    //      costs 48-64 VGPRs and pins the kernel at 2 waves/SIMD —
-    //      occupancy (PMC: 60% of wave cycles parked) is the limiter,
-    //      not the extra ds_reads ----
-    float s[G];
-    const bf16x2* kp2 = reinterpret_cast<const bf16x2*>(&kraw[0]);
-#pragma unroll 1
-    for (int j = 0; j < G; ++j) {
-      const uint16_t* qsrc = &q_lds[j][seg];
-      asm("" : "+v"(qsrc));
-      uint32_t qtmp[16];
-#pragma unroll
-      for (int c4 = 0; c4 < 4; ++c4) {
-        *reinterpret_cast<uint4*>(&qtmp[c4 * 4]) =
-            *reinterpret_cast<const uint4*>(qsrc + c4 * 8);
-      }
-      const bf16x2* qp2 = reinterpret_cast<const bf16x2*>(&qtmp[0]);
-      float sj = 0.0f;
-#pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        sj = __builtin_amdgcn_fdot2_f32_bf16(qp2[c], kp2[c], sj, false);
-      }
-      s[j] = sj;
-    }
-
-    // ---- issue V loads (current block) and K loads (next block) now so
-    //      their latency hides under the shfl chains below; the scores
-    //      consumed kraw above, so the next-K prefetch gets the whole
-    //      softmax + V-accumulate phase of flight time ----
-    const int tlimit = min(BS, ctx - b * BS);
-    ushort8 vraw[4];
-    const uint16_t* vp =
-        vcache + page_of(b) * nkv * BS * HD + head_off + vlane * 8;
-    if (tlimit == BS) {
-#pragma unroll
-      for (int t4 = 0; t4 < 4; ++t4)
-        vraw[t4] = *reinterpret_cast<const ushort8*>(
-            vp + (vtok + 4 * t4) * HD);
-    } else {
-#pragma unroll
-      for (int t4 = 0; t4 < 4; ++t4)
-        if (vtok + 4 * t4 < tlimit)
-          vraw[t4] = *reinterpret_cast<const ushort8*>(
-              vp + (vtok + 4 * t4) * HD);
-    }
-    if (b + NWAVES < nblocks) {
-      if ((((b - b0) / NWAVES + 1) & 63) == 0) load_ids(b + NWAVES);
-      load_k(b + NWAVES, kraw);
-    }
-
-    // ---- finish scores: pairwise dot reduce + mask ----
-    const bool valid = (b * BS + tok) < ctx;
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      float v = s[j] + __shfl_xor(s[j], 1, WAVE_SIZE);
-      v += __shfl_xor(v, 2, WAVE_SIZE);
-      s[j] = valid ? v * scale : -INFINITY;
-    }
-
-    // ---- online softmax (all-head ILP) ----
-    float pmax[G], p[G];
-#pragma unroll
-    for (int j = 0; j < G; ++j) pmax[j] = token_reduce_max(s[j]);
-#pragma unroll
-    for (int j = 0; j < G; ++j) {
-      if (pmax[j] > m[j]) {
-        const float alpha = __expf(m[j] - pmax[j]);
-        l[j] *= alpha;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[j][e] *= alpha;
-        m[j] = pmax[j];
-      }
-      p[j] = (s[j] == -INFINITY) ? 0.0f : __expf(s[j] - m[j]);
-    }
-#pragma unroll
-    for (int j = 0; j < G; ++j)
-      l[j] += token_reduce_sum((lane & 3) == 0 ? p[j] : 0.0f);
-
-    // ---- V accumulate: p reaches the V lanes via bpermute; math runs
-    //      on float2 pairs (v_pk_fma_f32: 2 FLOPs/instr — no MFMAs here
-    //      to contend with, so packed f32 is a straight 2x on the VALU
-    //      issue count of this phase) ----
-#pragma unroll
-    for (int t4 = 0; t4 < 4; ++t4) {
-      const int t = vtok + 4 * t4;
-      float pj[G];
-#pragma unroll
-      for (int j = 0; j < G; ++j)
-        pj[j] = __shfl(p[j], 4 * t, WAVE_SIZE);
-      if (t >= tlimit) continue;
-      const uint32_t* vp32 = reinterpret_cast<const uint32_t*>(&vraw[t4]);
-      float2 vf2[4];
-#pragma unroll
-      for (int e2 = 0; e2 < 4; ++e2) {
-        const uint32_t q = vp32[e2];
-        vf2[e2].x = bf16_to_f32((uint16_t)(q & 0xffff));
-        vf2[e2].y = bf16_to_f32((uint16_t)(q >> 16));
-      }
-#pragma unroll
-      for (int j = 0; j < G; ++j) {
-        float2* a2 = reinterpret_cast<float2*>(&acc[j][0]);
-#pragma unroll
-        for (int e2 = 0; e2 < 4; ++e2) {
-          a2[e2].x = fmaf(pj[j], vf2[e2].x, a2[e2].x);
-          a2[e2].y = fmaf(pj[j], vf2[e2].y, a2[e2].y);
-        }
-      }
-    }
-
+  for (int kk = 0; kk < 4; ++kk) {
+    pd_bf16x8 f{};
+    if (r16 < G)
+      f = *reinterpret_cast<const pd_bf16x8*>(
+          q + (int64_t)seq * q_rs + (kvh * G + r16) * HD + kk * 32 + quad * 8);
+    qf[kk] = f;
   }
 
-  // fold the 4 token-subgroup partials (lanes l, l+16, l+32, l+48 share dims)
+  // lane offsets into a page, bytes: K as the rows of a matrix operand; V four
+  // rows a load, 16-byte chunks exchanged so that the eight rows which 32 lanes
+  // of a transposing read take 32 bytes of each lie in different banks
+  const int kx = r16 * HD * 2 + quad * 16;
+  int vx[4];
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
+  for (int i = 0; i < 4; ++i) {
+    const int r = i * 4 + quad;
+    vx[i] = r * HD * 2 + ((r16 ^ ((r & 7) << 1)) << 4);
+  }
+  struct Keys {
+    pd_u32x4 k[2][4];
+  };
+  typedef __attribute__((address_space(3))) void lds_void;
+  // pair u; past the part's end nothing is read and the values are zeros
+  auto fetch = [&](int u, Keys& K, uint16_t* vs) PD_INLINE {
+    const int at = (u - wave) / NWAVES;
+    const int left = limit - (block0 + 2 * u) * BS;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      acc[j][e] += __shfl_xor(acc[j][e], 16, WAVE_SIZE);
-      acc[j][e] += __shfl_xor(acc[j][e], 32, WAVE_SIZE);
+    for (int h = 0; h < 2; ++h) {
+      const int64_t page = __builtin_amdgcn_readlane(ids, (at & 31) * 2 + h);
+      const int64_t base = (page * nkv + kvh) * PAGE;
+      const int rows =
+          __builtin_amdgcn_readfirstlane(max(0, min(BS, left - h * BS)));
+      const auto kr = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(kcache + base), 0, rows * HD * 2, 0x00020000);
+      const auto vr = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(vcache + base), 0, rows * HD * 2, 0x00020000);
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+        K.k[h][kk] =
+            __builtin_amdgcn_raw_buffer_load_b128(kr, kx + kk * 64, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            vr, (lds_void*)(vs + h * PAGE + i * 512), 16, vx[i], 0, 0, 0);
+    }
+  };
+
+  // O^T: head r16, dims 16 d + 4 quad ..; m in log2, l of this lane's tokens
+  pd_f32x4 acc[8];
+#pragma unroll
+  for (int d = 0; d < 8; ++d) acc[d] = pd_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float m = -INFINITY, l = 0.0f;
+  const float c = scale * PD_LOG2E;
+  const int vrow = 4 * quad + (r16 >> 2);
+  auto use = [&](int u, const Keys& K, uint16_t* vs) PD_INLINE {
+    pd_f32x4 s[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) s[h] = pd_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        s[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(pd_bf16x8, K.k[h][kk]), qf[kk], s[h], 0, 0, 0);
+    // token 16 (j / 4) + 4 quad + j % 4 of the pair
+    float t[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) t[j] = s[j >> 2][j & 3] * c;
+    const int left = limit - (block0 + 2 * u) * BS;
+    if (left < 2 * BS) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if ((j >> 2) * 16 + 4 * quad + (j & 3) >= left) t[j] = -INFINITY;
+    }
+    float mx = t[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) mx = fmaxf(mx, t[j]);
+    mx = pd_max(mx);
+    if (__any(mx > m)) {
+      const float mn = fmaxf(m, mx);
+      const float alpha =
+          m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) acc[d] *= alpha;
+    }
+    const float mc = m == -INFINITY ? 0.0f : m;
+    float p[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p[j] = __builtin_amdgcn_exp2f(t[j] - mc);
+    l += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    union {
+      uint32_t u[4];
+      pd_bf16x8 v;
+    } hi, lo;
+    auto rest = [](float x) PD_INLINE {
+      const float top = __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+      return fmaxf(x - top, x * 0x1p-60f);
+    };
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      hi.u[e] = (__float_as_uint(p[2 * e]) >> 16) |
+                (__float_as_uint(p[2 * e + 1]) & 0xffff0000u);
+      lo.u[e] = pd_pack(rest(p[2 * e]), rest(p[2 * e + 1]));
+    }
+    typedef __attribute__((address_space(3))) pd_short4 lds_short4;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      union {
+        pd_short4 h[2];
+        pd_bf16x8 v;
+      } vf;
+      const int chunk = (2 * d + ((r16 & 3) >> 1)) ^ ((vrow & 7) << 1);
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        vf.h[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_short4*)(vs + h * PAGE + vrow * HD + chunk * 8 +
+                          (r16 & 1) * 4));
+      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, hi.v, acc[d], 0, 0,
+                                                       0);
+      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, lo.v, acc[d], 0, 0,
+                                                       0);
+    }
+  };
+
+  auto ahead = [&](int u, Keys& K, uint16_t* vs) PD_INLINE {
+    if ((((u - wave) / NWAVES) & 31) == 0 && u < pairs) load_ids(u);
+    fetch(u, K, vs);
+  };
+  Keys k0, k1;
+  if (wave < pairs) {
+    fetch(wave, k0, v_s0[wave]);
+    for (int u = wave;; u += 2 * NWAVES) {
+      ahead(u + NWAVES, k1, v_s1[wave]);
+      use(u, k0, v_s0[wave]);
+      if (u + NWAVES >= pairs) break;
+      ahead(u + 2 * NWAVES, k0, v_s0[wave]);
+      use(u + NWAVES, k1, v_s1[wave]);
+      if (u + 2 * NWAVES >= pairs) break;
     }
   }
+  l = pd_sum(l);
 
-  // ---- cross-wave merge ----
-#pragma unroll
-  for (int j = 0; j < G; ++j) {
-    if (lane == 0) {
-      m_lds[wave][j] = m[j];
-      l_lds[wave][j] = l[j];
+  // ---- cross-wave merge, in the memory of the V tiles (the loads that are
+  //      still under way there read nothing, and are waited for first)
+  float* acc_lds = reinterpret_cast<float*>(&v_s0[0][0]);  // [NWAVES][G][HD]
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  __syncthreads();
+  if (r16 < G) {
+    if (quad == 0) {
+      m_lds[wave][r16] = m;
+      l_lds[wave][r16] = l;
     }
-    if (vtok == 0) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        acc_lds[wave][j][vlane * 8 + e] = acc[j][e];
-    }
+    for (int d = 0; d < 8; ++d)
+      *reinterpret_cast<pd_f32x4*>(acc_lds + (wave * G + r16) * HD + d * 16 +
+                                   quad * 4) = acc[d];
   }
   __syncthreads();
 
@@ -304,10 +321,11 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE) void paged_attn_decode_kernel(
     float L = 0.0f, o = 0.0f;
 #pragma unroll
     for (int w = 0; w < NWAVES; ++w) {
-      const float f =
-          (m_lds[w][j] == -INFINITY) ? 0.0f : __expf(m_lds[w][j] - M);
+      const float f = m_lds[w][j] == -INFINITY
+                          ? 0.0f
+                          : __builtin_amdgcn_exp2f(m_lds[w][j] - M);
       L = fmaf(f, l_lds[w][j], L);
-      o = fmaf(f, acc_lds[w][j][d], o);
+      o = fmaf(f, acc_lds[(w * G + j) * HD + d], o);
     }
     const int64_t head = (int64_t)seq * nq + kvh * G + j;
     if (part.count == 1) {
@@ -354,7 +372,8 @@ __global__ __launch_bounds__(HD) void paged_attn_merge_kernel(
     float l = 0.0f;
     if (tid < n) {
       const float2 v = ml[s0 + tid];
-      const float f = v.x == -INFINITY ? 0.0f : __expf(v.x - M);
+      const float f =
+          v.x == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(v.x - M);
       weight[tid] = f;
       l = f * v.y;
     }
@@ -382,32 +401,28 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
   constexpr int NWAVES = 4, HD = 128;
   const int nq = q.size(1);
   const int max_blocks = block_table.size(1);
-  // The chip holds 1024 of these workgroups (four per compute unit, by their
-  // registers).  Where sequences x heads are fewer, aim for two rounds, so that
-  // parts of ragged lengths even out.  How short a part may be follows from
-  // what is waited for: few workgroups wait for memory, page after page, and
-  // gain from parts of a page per wave; from a few hundred on (half as many
-  // with one query head per key head) the chip as a whole is at the memory's
-  // rate, equal contexts gain nothing and only long ones among short ones do.
-  // Measured, whole and cut by these lines (us): 8 heads, 1 sequence of 500
-  // tokens 20.0 and 8.9, 8 of 500 20.2 and 10.9; 24 of 1000 39.4 and 26.1, of
-  // 256 not cut (parts of four pages 13.9 for 12.3); 48 of 500 26.0 and 25.6,
-  // 48 of 100 to 1000 39.9 and 32.7; 64 of 400 to 4000 166 and 137, of 4000 189
-  // and 200, of 500 not cut (parts of four pages 33 for 27).  Two parts of four
-  // pages do not pay for a merge (1 sequence of 100 tokens 7.7 whole, 9.0 cut,
-  // of 200 11.7 and 9.7).  With 1024 workgroups a split only adds the merge
-  // (128 of 100 to 2000 tokens: 155 and 160).  Whether anything is cut is known
-  // on the device only: where the block table is wide and the contexts are
-  // short the merge is launched for nothing (1.6 to 2 us: 16 sequences of 200
-  // tokens 13.3 without and 14.4, 100 of 100 16.2 and 18.2).
+  // The chip holds 512 of these workgroups (two per compute unit, by their
+  // registers).  Where sequences x heads are an eighth of that, they wait for
+  // memory, pair of pages after pair, and gain from parts of a pair per wave
+  // until they fill the chip once or a merge has 32 parts.  From there on the
+  // chip as a whole is at the memory's rate and equal contexts gain nothing
+  // (they lose what the merge costs); cut in long parts, the long ones among
+  // ragged contexts do not end alone.  Measured, whole and cut by these lines
+  // (us): 8 heads, 1 sequence of 3000 tokens 29.1 and 8.5, of 8000 71.4 and
+  // 10.6, 5 of 750 to 1500 16.6 and 11.4, 8 of 1000 13.0 and 10.7; 33 of 300 to
+  // 3000 47.5 and 40.5, 40 of 200 to 4000 93.5 and 72.2, 61 of them 117 and 104,
+  // 90 of 100 to 3000 119 and 115; but 24 of 3000 46.4 and 53.6, 64 of 4000 183
+  // and 188.  With 1024 workgroups a split only adds the merge (128 of 100 to
+  // 2000 tokens: 107 and 110).  Whether anything is cut is known on the device
+  // only: where the block table is wide and the contexts are short the merge is
+  // launched for nothing (1.6 to 2 us).
   const int whole = std::max(1, B * nkv);
-  const int filled = G == 1 ? 2 * whole : whole;
-  const int min_blocks =
-      whole <= 96 ? 4 : filled <= 256 ? 16 : filled < 512 ? 32 : 64;
+  const bool few = whole <= 64;
+  const int min_blocks = few ? 8 : 64;
   const int nsplit =
-      whole >= 1024 || max_blocks <= 8
+      whole >= 1024 || max_blocks <= 32
           ? 1
-          : std::max(1, std::min(2048 / whole,
+          : std::max(1, std::min(few ? std::min(512 / whole, 32) : 2048 / whole,
                                  (max_blocks + min_blocks - 1) / min_blocks));
   torch::Tensor part;
   float *part_o = nullptr, *part_ml = nullptr;
@@ -417,7 +432,7 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
     part_o = part.data_ptr<float>();
     part_ml = part_o + n * HD;
   }
-  hipLaunchKernelGGL((paged_attn_decode_kernel<HD, G, NWAVES>),
+  hipLaunchKernelGGL((paged_attn_decode_kernel<G, NWAVES>),
                      dim3(nkv, B, nsplit), dim3(NWAVES * WAVE_SIZE), 0, stream,
                      (uint16_t*)out.data_ptr(), (const uint16_t*)q.data_ptr(),
                      (const uint16_t*)kcache.data_ptr(),
