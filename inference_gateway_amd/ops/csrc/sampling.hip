@@ -24,6 +24,8 @@
 #include <ATen/cuda/CUDAContext.h>
 #include <torch/extension.h>
 
+#include <climits>
+
 #include "common.h"
 
 namespace igw {
@@ -584,35 +586,95 @@ __global__ __launch_bounds__(BLOCK) void sample_bf16_kernel(
 // read ONCE, 16 bytes a load, and every further pass runs on registers.
 //
 //   1. maximum, and for top-p the total mass Z;
+//      From there the row is kept as keys, whose order is the logits', so that
+//      the largest of a chunk of eight takes a few packed instructions and a
+//      wave goes past the chunks that no lane needs;
 //   2. thresholds: counts per exact bf16 value in LDS for the keys from the
-//      top down, first the 256 keys (two octaves) below the maximum, then
-//      windows of 4096, each starting at the highest key that is left.  The
-//      mass of a value is count * exp, so no exponential is taken per element
-//      here.  The first window that holds either threshold decides: the other
-//      one is lower and max(tau_k, tau_p) is wanted;
-//   3. kept mass per (chunk, wave) cell in index order, cells without a kept
-//      element skipped; the cell, the lane and the element of the draw.
+//      top down, first the 128 keys (an octave) below the maximum, then the 256
+//      after them, then windows of 4096, each starting at the highest key that
+//      is left.  The mass of a value is count * exp, so no exponential is taken
+//      per element here.  The first window that holds either threshold decides:
+//      the other one is lower and max(tau_k, tau_p) is wanted.  With more than
+//      eight chunks a thread, those with a key of the first window (commonly a
+//      few hundred of 16032) go to a list in LDS, and counts and draw are loops
+//      over it;
+//   3. the draw: listed chunks with a kept element, if they are at most as many
+//      as threads, are put in index order by counting, and one running sum finds
+//      the chunk.  Otherwise kept mass per (chunk, wave) cell in index order,
+//      cells without a kept element skipped; the cell, the lane, the element.
 //
 // Bound: the row's 256 KB arrive at HBM speed, then come passes over all its
-// elements on the vector units, one each for the mass, for every window of
-// counts, for the next key below a window and for the kept cells (the
-// exponentials themselves are about 3 us of a row of 128256); one row per
-// compute unit at a time.  Each of the four passes of sample_bf16_kernel reads
-// the row again and updates LDS bins for all elements: 1024 rows of 128256 took
-// 945 us, here 198 us (temperature, top-k and top-p on most rows; greedy rows
-// 62).  Rows of more than 8 * 512 * 40 logits keep that kernel: they would not
+// elements on the vector units, one for the mass, one for the keys and one for
+// every window or cell pass that is needed, at one row per compute unit at a time;
+// with the passes written out for up to 40 chunks also the 64 KB instruction
+// cache, which is why what is rare is a loop.  Each of the four passes of
+// sample_bf16_kernel reads the row again and updates LDS bins for all elements.
+// 1024 rows of 128256, greedy / top-k 50 and top-p / top-p 0.9 / top-k 40 / no
+// limits: 52, 117, 179, 90 and 103 us; with elements instead of keys, every pass
+// over all of them and the list's work in the cells 63, 152, 270, 122 and 138.
+// 1024 rows of 32064: 12.8, 36, 43, 29 and 22.5, before 14.4, 39, 65, 33 and 28
+// (the list there: 15, 38, 47, 35 and 26, hence the line at eight chunks).
+// Rows of more than 8 * 512 * 40 logits keep sample_bf16_kernel: they would not
 // leave registers for the arithmetic.  So do those of up to 4096, where its
 // passes are short (1000 logits, 300 rows, greedy / top-k and top-p / top-p:
-// 3.0, 15.9 and 15.0 us, here 7.5, 17.0 and 28.3; 4099 logits 3.9, 27.0 and
-// 24.7, here 3.8, 10.9 and 17.7).  There are as many sizes of the kernel as keep
-// rows without limits ahead of that one, which has few passes for them (300 rows
-// of 33000 29.7 us, here 35.3 with 16 chunks, 20.5 with 12; 66000 55.2, 64.7
+// 3.0, 15.9 and 15.0 us, here 7.5, 17.0 and 28.3 before; 4099 logits 3.9, 27.0
+// and 24.7, here 3.8, 10.9 and 17.7).  There are as many sizes of the kernel as
+// keep rows without limits ahead of that one, which has few passes for them (300
+// rows of 33000 29.7 us, here 35.3 with 16 chunks, 20.5 with 12; 66000 55.2, 64.7
 // with 32 and 50 with 24).
 // ---------------------------------------------------------------------------
 constexpr int SR_THREADS = 512;
 constexpr int SR_WAVES = SR_THREADS / WAVE_SIZE;
-constexpr int SR_FIRST = 256;    // keys of the first window
-constexpr int SR_WINDOW = 4096;  // keys of the others
+constexpr int SR_FIRST = 128;    // keys of the first window
+constexpr int SR_SECOND = 256;   // of the second
+constexpr int SR_WINDOW = 4096;  // of the others
+constexpr int SR_LIST = 2048;    // chunks of the first window that are listed
+
+// Sums, maxima and running sums over the wave by lane exchanges of the vector
+// units (one through LDS takes six round trips).  A lane without a partner gets
+// `none`.
+template <int CTRL, int ROWS = 0xf, class T>
+DEVINLINE T sr_lane(T x, T none) {
+  return __builtin_bit_cast(
+      T, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, none),
+                                     __builtin_bit_cast(int, x), CTRL, ROWS,
+                                     0xf, false));
+}
+DEVINLINE void sr_both16(float x, float& a, float& b) {
+  a = b = x;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 0" : "+v"(a), "+v"(b));
+}
+DEVINLINE void sr_both32(float x, float& a, float& b) {
+  a = b = x;
+  asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 0" : "+v"(a), "+v"(b));
+}
+template <class F>
+DEVINLINE float sr_reduce(float x, F f) {
+  x = f(x, sr_lane<0xb1>(x, x));    // lane ^ 1
+  x = f(x, sr_lane<0x4e>(x, x));    // lane ^ 2
+  x = f(x, sr_lane<0x141>(x, x));   // of 8, from the other end
+  x = f(x, sr_lane<0x140>(x, x));   // of 16, from the other end
+  float a, b;
+  sr_both16(x, a, b);
+  sr_both32(f(a, b), a, b);
+  return f(a, b);
+}
+DEVINLINE float sr_sum(float x) {
+  return sr_reduce(x, [](float a, float b) { return a + b; });
+}
+DEVINLINE float sr_max(float x) {
+  return sr_reduce(x, [](float a, float b) { return fmaxf(a, b); });
+}
+template <class T>
+DEVINLINE T sr_scan(T x) {
+  x += sr_lane<0x111>(x, T(0));        // the lane 1, 2, 4, 8 below in its 16
+  x += sr_lane<0x112>(x, T(0));
+  x += sr_lane<0x114>(x, T(0));
+  x += sr_lane<0x118>(x, T(0));
+  x += sr_lane<0x142, 0xa>(x, T(0));   // the last of the 16 below
+  x += sr_lane<0x143, 0xc>(x, T(0));   // the last of the lower half
+  return x;
+}
 
 // Constants that unpack a dword of two bf16.  Every pass asks for its own,
 // which the compiler cannot see to be the same: it would otherwise keep one
@@ -635,7 +697,42 @@ struct Unpack {
         __builtin_bit_cast(short2v, u) >> __builtin_bit_cast(short2v, sign);
     return u ^ (__builtin_bit_cast(uint32_t, neg) | 0x80008000u);
   }
+  // and back
+  DEVINLINE uint32_t bits(uint32_t k) const {
+    typedef __attribute__((ext_vector_type(2))) short short2v;
+    const short2v pos =
+        __builtin_bit_cast(short2v, k) >> __builtin_bit_cast(short2v, sign);
+    return k ^ (~__builtin_bit_cast(uint32_t, pos) | 0x80008000u);
+  }
+  // the halves of a pair of keys
+  DEVINLINE uint32_t first(uint32_t k) const { return k & ~high; }
+  DEVINLINE uint32_t second(uint32_t k) const { return k >> shift; }
 };
+
+// Largest of eight keys.  Written out so that a pass computes its own: the
+// compiler would keep all of them over the loop of the windows.
+DEVINLINE uint32_t largest_key(const uint32_t (&k)[4]) {
+  uint32_t m;
+  asm volatile(
+      "v_pk_max_u16 %0, %1, %2\n\tv_pk_max_u16 %0, %0, %3\n\t"
+      "v_pk_max_u16 %0, %0, %4"
+      : "=&v"(m)
+      : "v"(k[0]), "v"(k[1]), "v"(k[2]), "v"(k[3]));
+  return max(m & 0xffffu, m >> 16);
+}
+
+// Whether any of eight keys is one of two (each given twice in a dword).
+DEVINLINE bool has_key(const uint32_t (&k)[4], const uint32_t (&same)[2]) {
+  typedef __attribute__((ext_vector_type(2))) unsigned short ushort2v;
+  ushort2v m = {0xffff, 0xffff};
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      m = __builtin_elementwise_min(m,
+                                    __builtin_bit_cast(ushort2v, k[q] ^ same[i]));
+  return m.x == 0 || m.y == 0;
+}
 
 DEVINLINE float bf16_key_val(uint32_t key) {
   const uint32_t u = (key & 0x8000u) ? key ^ 0x8000u : key ^ 0xffffu;
@@ -653,7 +750,13 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
     const float* __restrict__ uniforms,    // [B]
     int V) {
   __shared__ float red[SR_WAVES];
-  __shared__ uint32_t bins[SR_WINDOW];
+  __shared__ uint32_t bins[SR_WINDOW + WAVE_SIZE];
+  __shared__ uint4 list_k[SR_LIST];    // chunks of the first window: keys
+  __shared__ int list_at[SR_LIST];     // and number
+  __shared__ __attribute__((aligned(16))) int kept_at[SR_THREADS];
+  __shared__ float kept_w[SR_THREADS], sorted_w[SR_THREADS];
+  __shared__ int kept_e[SR_THREADS], sorted_e[SR_THREADS];
+  __shared__ int s_list, s_kept, s_last;
   __shared__ uint32_t wave_n[SR_WAVES];
   __shared__ float wave_w[SR_WAVES];
   __shared__ int s_tau, s_top, s_cell;
@@ -670,23 +773,45 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
   const bool greedy = temp <= 0.0f;
   const float inv_t = greedy ? 1.0f : 1.0f / temp;
 
-  // element h of chunk j is logit (j * 512 + tid) * 8 + h; past the end -inf
+  // Element h of chunk j is logit (j * 512 + tid) * 8 + h; past the end -inf.
+  // The chunk that the row ends in is loaded once, for whichever it is: with a
+  // check in all of them the code of the loads alone was a third of the kernel,
+  // which then did not fit the instruction cache.
+  constexpr int CHUNK = SR_THREADS * 8;
+  const int whole = V / CHUNK;
   uint32_t d[NCH][4];
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    const int at = (j * SR_THREADS + tid) * 8;
+    if (j < whole) {
+      const uint4 v =
+          *reinterpret_cast<const uint4*>(row + (j * SR_THREADS + tid) * 8);
+      d[j][0] = v.x; d[j][1] = v.y; d[j][2] = v.z; d[j][3] = v.w;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) d[j][q] = 0xff80ff80u;
+    }
+  }
+  if (whole * CHUNK < V) {
+    const int at = (whole * SR_THREADS + tid) * 8;
+    uint32_t end[4];
     if (at + 8 <= V) {
       const uint4 v = *reinterpret_cast<const uint4*>(row + at);
-      d[j][0] = v.x; d[j][1] = v.y; d[j][2] = v.z; d[j][3] = v.w;
+      end[0] = v.x; end[1] = v.y; end[2] = v.z; end[3] = v.w;
     } else {
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int e = at + 2 * q;
         const uint32_t lo = e < V ? row[e] : 0xff80u;
         const uint32_t hi = e + 1 < V ? row[e + 1] : 0xff80u;
-        d[j][q] = lo | (hi << 16);
+        end[q] = lo | (hi << 16);
       }
     }
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+      if (j == whole) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[j][q] = end[q];
+      }
   }
   // ---- maximum ----
   float mx = -INFINITY;
@@ -698,7 +823,7 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
       for (int q = 0; q < 4; ++q)
         mx = fmaxf(fmaxf(mx, un.lo(d[j][q])), un.hi(d[j][q]));
   }
-  mx = wave_reduce_max(mx);
+  mx = sr_max(mx);
   if (lane == 0) red[wave] = mx;
   if (tid == 0) s_pick = 0xffffffffu;
   __syncthreads();
@@ -706,33 +831,14 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
 #pragma unroll
   for (int w = 1; w < SR_WAVES; ++w) M = fmaxf(M, red[w]);
 
-  // lowest index of the maximum (all threads call it)
-  auto first_max = [&]() {
-    const Unpack un;
-    uint32_t best = 0xffffffffu;
-#pragma unroll
-    for (int j = 0; j < NCH; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t at = (j * SR_THREADS + tid) * 8 + 2 * q;
-        if (un.hi(d[j][q]) == M && at + 1 < (uint32_t)V)
-          best = min(best, at + 1);
-        if (un.lo(d[j][q]) == M && at < (uint32_t)V) best = min(best, at);
-      }
-    if (best != 0xffffffffu) atomicMin(&s_pick, best);
-    __syncthreads();
-  };
-  if (greedy) {
-    first_max();
-    if (tid == 0) out[seq] = (int32_t)s_pick;
-    return;
-  }
-
   const int k = top_k[seq];
   const float p = top_p[seq];
   const bool do_k = k > 0 && k < V;
-  const bool do_p = p < 1.0f;
-  auto weight = [&](float x) { return __expf((x - M) * inv_t); };
+  const bool do_p = p < 1.0f && !greedy;
+  const float rate = inv_t * 1.44269504088896340736f;   // to powers of two
+  auto weight = [&](float x) {
+    return __builtin_amdgcn_exp2f((x - M) * rate);
+  };
 
   float target_p = 0.0f;
   if (do_p) {
@@ -743,7 +849,7 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
 #pragma unroll
       for (int q = 0; q < 4; ++q)
         z += weight(un.lo(d[j][q])) + weight(un.hi(d[j][q]));
-    z = wave_reduce_sum(z);
+    z = sr_sum(z);
     __syncthreads();  // red was read by everybody
     if (lane == 0) red[wave] = z;
     __syncthreads();
@@ -753,13 +859,75 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
     target_p = p * z;
   }
 
+  // From here on the row is kept as keys: a chunk's largest takes a few
+  // instructions, and a wave passes over the chunks of which none matters.
+  {
+    const Unpack un;
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) d[j][q] = un.keys(d[j][q]);
+  }
+  int max_key = 0x8000;  // key of the maximum (of +0 for either zero)
+  if (M != 0.0f)
+    max_key =
+        (int)bf16_key((uint16_t)(__builtin_bit_cast(uint32_t, M) >> 16));
+  // Lowest index of the maximum (all threads call it); -0 is as large as +0.
+  auto first_max = [&]() {
+    const uint32_t low = M == 0.0f ? 0x7fffu : (uint32_t)max_key;
+    const uint32_t same[2] = {(uint32_t)max_key * 0x10001u, low * 0x10001u};
+    uint32_t at = 0, e[4] = {0, 0, 0, 0};
+    bool any = false;
+#pragma unroll
+    for (int j = NCH - 1; j >= 0; --j)
+      if (largest_key(d[j]) >= low && has_key(d[j], same)) {
+        any = true;
+        at = (j * SR_THREADS + tid) * 8;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) e[q] = d[j][q];
+      }
+    if (any) {
+      uint32_t first = 8;
+#pragma unroll
+      for (int h = 7; h >= 0; --h) {
+        const uint32_t key = (h & 1) ? e[h >> 1] >> 16 : e[h >> 1] & 0xffffu;
+        if (key == low || key == (uint32_t)max_key) first = h;
+      }
+      atomicMin(&s_pick, at + first);
+    }
+    __syncthreads();
+    if (tid == 0)   // what is past the end is no logit
+      out[seq] = M == -INFINITY && !greedy ? 0
+                 : s_pick < (uint32_t)V    ? (int32_t)s_pick
+                                           : -1;
+  };
+  if (greedy) {
+    first_max();
+    return;
+  }
+
   // ---- thresholds ----
   int tau = 0;
+  int listed = -1;   // chunks in the list, when that is all that is kept
   if (do_k || do_p) {
-    int top = 0x8000;  // key of the maximum (of +0 for either zero)
-    if (M != 0.0f) {
-      const uint32_t u = __builtin_bit_cast(uint32_t, M) >> 16;
-      top = (int)bf16_key((uint16_t)u);
+    int top = max_key;
+    // The chunks with a key of the first window go to a list in LDS: they are
+    // few, and what is done with them is a loop and not the code of NCH chunks.
+    if constexpr (NCH > 8) {
+      if (tid == 0) s_list = 0;
+      __syncthreads();
+      const uint32_t low = (uint32_t)max(top - SR_FIRST + 1, 0);
+#pragma unroll
+      for (int j = 0; j < NCH; ++j)
+        if (largest_key(d[j]) >= low) {
+          const int at = atomicAdd(&s_list, 1);
+          if (at < SR_LIST) {
+            list_k[at] = make_uint4(d[j][0], d[j][1], d[j][2], d[j][3]);
+            list_at[at] = j * SR_THREADS + tid;
+          }
+        }
+      __syncthreads();
+      if (s_list <= SR_LIST) listed = s_list;
     }
     uint32_t seen_n = 0;   // above the window
     float seen_w = 0.0f;
@@ -771,17 +939,26 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
         s_top = -1;
       }
       __syncthreads();
-      {
+      // an element outside the window counts where nobody looks
+      const uint32_t spare = (uint32_t)(SR_WINDOW + lane);
+      auto count = [&](uint32_t k0, uint32_t k1) {
+        const uint32_t b0 = (uint32_t)top - k0, b1 = (uint32_t)top - k1;
+        atomicAdd(&bins[b0 < (uint32_t)width ? b0 : spare], 1u);
+        atomicAdd(&bins[b1 < (uint32_t)width ? b1 : spare], 1u);
+      };
+      if (NCH > 8 && width == SR_FIRST && listed >= 0) {
+        const uint32_t* list = reinterpret_cast<const uint32_t*>(list_k);
+        for (int e = tid; e < listed * 4; e += SR_THREADS)
+          count(list[e] & 0xffffu, list[e] >> 16);
+      } else {
         const Unpack un;
+        const uint32_t low = (uint32_t)max(top - width + 1, 0);
 #pragma unroll
         for (int j = 0; j < NCH; ++j)
+          if (largest_key(d[j]) >= low) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const uint32_t key = un.keys(d[j][q]);
-            const uint32_t b0 = (uint32_t)top - (key & 0xffffu);
-            const uint32_t b1 = (uint32_t)top - (key >> 16);
-            if (b0 < (uint32_t)width) atomicAdd(&bins[b0], 1u);
-            if (b1 < (uint32_t)width) atomicAdd(&bins[b1], 1u);
+            for (int q = 0; q < 4; ++q)
+              count(un.first(d[j][q]), un.second(d[j][q]));
           }
       }
       __syncthreads();
@@ -800,17 +977,8 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
           }
         }
       // inclusive sums over the wave, then over the waves before it
-      uint32_t sn = n;
-      float sw = w;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t tn = __shfl_up(sn, off, 64);
-        const float tw = __shfl_up(sw, off, 64);
-        if (lane >= off) {
-          sn += tn;
-          sw += tw;
-        }
-      }
+      const uint32_t sn = sr_scan(n);
+      const float sw = sr_scan(w);
       if (lane == 63) {
         wave_n[wave] = sn;
         wave_w[wave] = sw;
@@ -852,27 +1020,30 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
       __syncthreads();
       tau = s_tau;
       if (tau >= 0) break;
-      // the highest key below the window
-      const int lo = top - width + 1;
-      int next = -1;
-      {
+      if (width == SR_FIRST) {   // the second window follows the first
+        top -= SR_FIRST;
+      } else {
+        // the highest key below the window
+        const int lo = top - width + 1;
+        int next = -1;
         const Unpack un;
 #pragma unroll
         for (int j = 0; j < NCH; ++j)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            const uint32_t key = un.keys(d[j][q]);
-            const int k0 = (int)(key & 0xffffu), k1 = (int)(key >> 16);
+            const int k0 = (int)un.first(d[j][q]);
+            const int k1 = (int)un.second(d[j][q]);
             if (k0 < lo) next = max(next, k0);
             if (k1 < lo) next = max(next, k1);
           }
+        if (next >= 0) atomicMax(&s_top, next);
+        __syncthreads();
+        top = s_top;
       }
-      if (next >= 0) atomicMax(&s_top, next);
-      __syncthreads();
-      top = s_top;
+      listed = -1;
       seen_n = all_n;
       seen_w = all_w;
-      width = SR_WINDOW;
+      width = width < SR_SECOND ? SR_SECOND : SR_WINDOW;
       if (top < 0) {  // everything is kept (p * Z not reached by rounding)
         tau = 0;
         break;
@@ -881,27 +1052,111 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
     }
   }
 
-  // ---- kept mass of every (chunk, wave), in index order ----
   const uint32_t utau = (uint32_t)tau;
   auto kept = [&](uint32_t key) {
     return key >= utau ? weight(bf16_key_val(key)) : 0.0f;
   };
+  auto kept_sum = [&](const uint32_t* e) {
+    float sum = 0.0f;
+    for (int q = 0; q < 4; ++q) sum += kept(e[q] & 0xffffu) + kept(e[q] >> 16);
+    return sum;
+  };
+  // the element of a chunk at which the running sum passes, or the last with
+  // mass
+  auto element = [&](const uint32_t* e, float run, float target) {
+    int chosen = 0;
+    for (int h = 0; h < 8; ++h) {
+      const float w = kept((h & 1) ? e[h >> 1] >> 16 : e[h >> 1] & 0xffffu);
+      run += w;
+      if (w > 0.0f) chosen = h;
+      if (w > 0.0f && run > target) break;
+    }
+    return chosen;
+  };
+
+  // ---- listed: at most as many kept chunks as threads are put in order ----
+  if (NCH > 8 && listed >= 0) {
+    if (tid == 0) {
+      s_kept = 0;
+      s_cell = INT_MAX;
+      s_last = -1;
+    }
+    __syncthreads();
+    for (int e = tid; e < listed; e += SR_THREADS) {
+      const uint32_t* k = reinterpret_cast<const uint32_t*>(list_k + e);
+      uint32_t most = 0;
+      for (int q = 0; q < 4; ++q) most = max(most, max(k[q] & 0xffffu, k[q] >> 16));
+      if (most >= utau) {
+        const int at = atomicAdd(&s_kept, 1);
+        if (at < SR_THREADS) {
+          kept_at[at] = list_at[e];
+          kept_w[at] = kept_sum(k);
+          kept_e[at] = e;
+        }
+      }
+    }
+    __syncthreads();
+    const int n = s_kept;
+    if (n <= SR_THREADS) {
+      if (tid >= n) kept_at[tid] = INT_MAX;
+      __syncthreads();
+      if (tid < n) {
+        const int own = kept_at[tid];
+        int rank = 0;
+        for (int e = 0; e < n; e += 4) {
+          const int4 v = *reinterpret_cast<const int4*>(kept_at + e);
+          rank += (v.x < own) + (v.y < own) + (v.z < own) + (v.w < own);
+        }
+        sorted_w[rank] = kept_w[tid];
+        sorted_e[rank] = kept_e[tid];
+      }
+      __syncthreads();
+      const float w = tid < n ? sorted_w[tid] : 0.0f;
+      const float own = sr_scan(w);
+      if (lane == 63) wave_w[wave] = own;
+      __syncthreads();
+      float before = 0.0f, total = 0.0f;
+#pragma unroll
+      for (int v = 0; v < SR_WAVES; ++v) {
+        if (v == wave) before = total;
+        total += wave_w[v];
+      }
+      if (total > 0.0f) {
+        const float target = uniforms[seq] * total;
+        if (w > 0.0f) {
+          if (before + own > target) atomicMin(&s_cell, tid);
+          atomicMax(&s_last, tid);
+        }
+        __syncthreads();
+        const bool passed = s_cell != INT_MAX;
+        if (tid == (passed ? s_cell : s_last)) {
+          const int e = sorted_e[tid];
+          out[seq] = list_at[e] * 8 +
+                     element(reinterpret_cast<const uint32_t*>(list_k + e),
+                             before + own - w, passed ? target : INFINITY);
+        }
+      } else {   // as below
+        first_max();
+      }
+      return;
+    }
+    __syncthreads();   // s_cell is used again
+  }
+
+  // ---- kept mass of every (chunk, wave), in index order ----
   const Unpack un;
 #pragma unroll
   for (int j = 0; j < NCH; ++j) {
-    uint32_t e[4];
-    bool some = false;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      e[q] = un.keys(d[j][q]);
-      some |= (e[q] & 0xffffu) >= utau || (e[q] >> 16) >= utau;
-    }
     float sum = 0.0f;
-    if (__any(some)) {
+    if (__any(largest_key(d[j]) >= utau)) {
 #pragma unroll
-      for (int q = 0; q < 4; ++q)
-        sum += kept(e[q] & 0xffffu) + kept(e[q] >> 16);
-      sum = wave_reduce_sum(sum);
+      for (int q = 0; q < 4; ++q) {
+        const uint32_t v = un.bits(d[j][q]);
+        const float w0 = weight(un.lo(v)), w1 = weight(un.hi(v));
+        sum += (un.first(d[j][q]) >= utau ? w0 : 0.0f) +
+               (un.second(d[j][q]) >= utau ? w1 : 0.0f);
+      }
+      sum = sr_sum(sum);
     }
     if (lane == 0) cells[j * SR_WAVES + wave] = sum;
   }
@@ -915,12 +1170,7 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
       const int c = lane * PER + i;
       own += c < NCH * SR_WAVES ? cells[c] : 0.0f;
     }
-    float run = own;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const float t = __shfl_up(run, off, 64);
-      if (lane >= off) run += t;
-    }
+    float run = sr_scan(own);
     const float total = __shfl(run, 63, 64);
     const float target = uniforms[seq] * total;
     run -= own;
@@ -962,54 +1212,25 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
     // to draw from: the largest logit, the first one where none is above
     // minus infinity.
     first_max();
-    if (tid == 0) out[seq] = M == -INFINITY ? 0 : (int32_t)s_pick;
     return;
   }
   if (wave == cell % SR_WAVES) {
     uint32_t e[4] = {0, 0, 0, 0};
-    const Unpack un;
 #pragma unroll
     for (int j = 0; j < NCH; ++j)
       if (j == cell / SR_WAVES) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) e[q] = un.keys(d[j][q]);
+        for (int q = 0; q < 4; ++q) e[q] = d[j][q];
       }
-    float sum = 0.0f;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-      sum += kept(e[q] & 0xffffu) + kept(e[q] >> 16);
-    float run = sum;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const float t = __shfl_up(run, off, 64);
-      if (lane >= off) run += t;
-    }
+    const float sum = kept_sum(e);
+    const float run = sr_scan(sum);
     const float rest = s_base;
     const uint64_t past = __ballot(sum > 0.0f && run > rest);
     const uint64_t some = __ballot(sum > 0.0f);
     const int l = past ? __builtin_ctzll(past) : 63 - __builtin_clzll(some);
-    if (lane == l) {
-      float r = run - sum;
-      int chosen = 0;
-#pragma unroll
-      for (int h = 7; h >= 0; --h) {  // the last with mass, if none passes
-        const uint32_t key = (h & 1) ? e[h >> 1] >> 16 : e[h >> 1] & 0xffffu;
-        if (kept(key) > 0.0f) {
-          chosen = h;
-          break;
-        }
-      }
-      for (int h = 0; h < 8; ++h) {
-        const uint32_t q = h < 2 ? e[0] : h < 4 ? e[1] : h < 6 ? e[2] : e[3];
-        const float w = kept((h & 1) ? q >> 16 : q & 0xffffu);
-        r += w;
-        if (w > 0.0f && r > rest) {
-          chosen = h;
-          break;
-        }
-      }
-      out[seq] = ((cell / SR_WAVES) * SR_THREADS + tid) * 8 + chosen;
-    }
+    if (lane == l)
+      out[seq] = ((cell / SR_WAVES) * SR_THREADS + tid) * 8 +
+                 element(e, run - sum, rest);
   }
 }
 
