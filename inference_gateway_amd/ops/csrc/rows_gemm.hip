@@ -4,21 +4,28 @@
 // Bound by streaming W once from HBM.  A wave owns 16 rows of W and takes them
 // from memory straight to registers, 512 bytes of each per slice of K, two
 // slices on their way while one is multiplied; the slice's rows of x go
-// through LDS once for the eight waves of a workgroup.  Loads take whole
-// 128-byte lines, and workgroups start at different slices, waves at different
-// lines: rows of W lie a multiple of 4 KB apart and would meet in the same
-// memory channels (28672 x 4096, 16 rows: 52.0 us, with the starts apart 48.0,
-// with whole lines as well 47.1).  A workgroup draws about 28 KB a microsecond
-// whatever its depth, so the launch has to fill the compute units evenly.
+// through LDS once for the eight waves of a workgroup.
+//
+// Eight neighbouring lanes load a whole 128-byte line.  A matrix operand wants
+// neighbouring lanes in neighbouring rows, but a load laid out like that is 64
+// requests of 16 bytes to the compute unit's cache, which takes 65 cycles for
+// it: 28 KB a microsecond for a compute unit, even from L2.  In whole lines it is
+// 92, so the lines go through 2 KB of LDS of the wave's own to be turned.
+//
+// Workgroups start at different slices, waves at different lines: rows of W lie
+// a multiple of 4 KB apart and would meet in the same memory channels (28672 x
+// 4096, 16 rows, before the lines were turned: 52.0 us, with the starts apart
+// 48.0).
 //
 // SWIGLU: a wave's 16 rows are eight gate rows and the up rows of the same
 // outputs, and the result is silu(gate) * up of the fp32 sums.
 //
-// Measured, library and here (us, W cold; 16 / 32 / 48 / 64 rows): 28672 x 4096
-// 65 56 64 55 and 48 48 50 52 (5.0 TB/s at 32 rows), as SwiGLU with the
-// activation 70 58 70 58 and 47 48 50 52; 128256 x 4096 182 200 210 213 and
-// 190 193 198 204; 4096 x 14336 27 34 40 41 and 30 31 33 35; 5120 x 17920
-// 118 125 130 135 and 43 44 47 51.
+// Measured, here and with operands loaded as the matrix unit wants them (us, W
+// cold; 16 / 32 / 43 / 64 rows): 28672 x 4096 as SwiGLU 42.2 43.0 43.8 45.7 (5.1
+// TB/s) and 45.7 46.9 48.6 51.0; 28672 x 4096 at 32 / 43 / 64 rows 42.7 44.8 45.8
+// and 48.0 50.7 51.0; 128256 x 4096 178 182 189 (5.6 TB/s) and 188 193 201; 4096 x
+// 14336 27.7 29.5 32.7 and 29.9 31.2 34.1.  The library, 32 / 48 / 64 rows: 56 64
+// 55, 200 210 213 and 34 40 41.
 #include <ATen/cuda/CUDAContext.h>
 #include <c10/cuda/CUDAGuard.h>
 #include <torch/extension.h>
@@ -48,6 +55,7 @@ template <int MT, bool SWIGLU>
 __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
     RowsArgs a) {
   __shared__ __attribute__((aligned(1024))) uint16_t xs[3][MT * 16 * RG_BK];
+  __shared__ __attribute__((aligned(1024))) rg_u32x4 turned[RG_WAVES][2][128];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, quad = lane >> 4;
@@ -67,9 +75,18 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
                      a.K;
   };
   // A load takes whole 128-byte lines: eight rows, eight lanes a row.
-  const int piece = (quad + 4 * (r16 >> 3)) * 8;
-  const uint16_t* w_lo = w_row(r16 & 7) + piece;
-  const uint16_t* w_hi = w_row(8 + (r16 & 7)) + piece;
+  const int piece = (lane & 7) * 8;
+  const uint16_t* w_lo = w_row(lane >> 3) + piece;
+  const uint16_t* w_hi = w_row(8 + (lane >> 3)) + piece;
+  // The 16 lines of two loads, as they come and as operands: the 16-byte pieces
+  // of a row are permuted by it so that operands are read without conflicts.
+  auto perm = [](int row) __attribute__((always_inline)) {
+    return (row & 3) | ((row >> 3) & 1) << 2;
+  };
+  const int put = (lane >> 3) * 8 + ((lane & 7) ^ perm(lane >> 3));
+  const int put_hi = 64 + (lane >> 3) * 8 + ((lane & 7) ^ perm(8 + (lane >> 3)));
+  const int get = r16 * 8 + (quad ^ perm(r16));
+  const int get_hi = r16 * 8 + ((4 + quad) ^ perm(r16));
   // rows of x: 512 bytes of a row per 32 lanes, its 16-byte pieces permuted by
   // the row so that the 16 rows of a matrix operand lie in different banks
   constexpr int XR = MT * 8 / RG_WAVES;    // 16-byte pieces of x per lane
@@ -109,30 +126,31 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
   rg_f32x4 acc[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = rg_f32x4{0.f, 0.f, 0.f, 0.f};
-  // Two loads hold rows 0..7 and 8..15 of the same line, first half in lanes
-  // 0..7 of 16 and second half in 8..15; a matrix operand is one half of all
-  // 16 rows, so the inner quarters change places.
+  // Lines are turned one step ahead of their products, in two buffers in turn;
+  // a wave's LDS accesses keep their order.
   auto compute = [&](const rg_u32x4 (&wr)[8], const uint16_t* s) {
+    rg_u32x4 half[2][2];
+    auto turn = [&](int j) __attribute__((always_inline)) {
+      rg_u32x4* t = turned[wave][j & 1];
+      t[put] = wr[2 * j];
+      t[put_hi] = wr[2 * j + 1];
+      half[j & 1][0] = t[get];
+      half[j & 1][1] = t[get_hi];
+    };
+    turn(0);
 #pragma unroll
-    for (int j = 0; j < 8; j += 2) {
-      rg_u32x4 half[2];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        half[0][e] = __builtin_amdgcn_update_dpp(wr[j][e], wr[j + 1][e], 0x128,
-                                                 0xf, 0xc, false);
-        half[1][e] = __builtin_amdgcn_update_dpp(wr[j + 1][e], wr[j][e], 0x128,
-                                                 0xf, 0x3, false);
-      }
+    for (int j = 0; j < 4; ++j) {
+      if (j < 3) turn(j + 1);
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-          const int chunk =
-              (((j / 2 + wave) & 3) * 8 + h * 4 + quad) ^ r16;
+          const int chunk = (((j + wave) & 3) * 8 + h * 4 + quad) ^ r16;
           const rg_bf16x8 xv = *reinterpret_cast<const rg_bf16x8*>(
               s + (m * 16 + r16) * RG_BK + chunk * 8);
           acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(rg_bf16x8, half[h]), xv, acc[m], 0, 0, 0);
+              __builtin_bit_cast(rg_bf16x8, half[j & 1][h]), xv, acc[m], 0, 0,
+              0);
         }
     }
   };
