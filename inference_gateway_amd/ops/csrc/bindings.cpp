@@ -41,6 +41,11 @@ void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                bool swiglu, int64_t tile);
+void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> bias);
+bool few_rows_held(const torch::Tensor& x, const torch::Tensor& w,
+                   const c10::optional<torch::Tensor>& bias, bool swiglu,
+                   bool anywhere);
 int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
                        const c10::optional<torch::Tensor>& bias, bool swiglu,
                        bool anywhere);
@@ -108,10 +113,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("flash_prefill", &igw::flash_prefill,
         "varlen causal MFMA flash-attention prefill (bf16, gfx950)");
   m.def("few_rows", &igw::few_rows,
-        "x W^T by gemv, rows_gemm or wide_gemm, None: none of them takes it");
+        "x W^T by gemv, rows_gemm, held_gemm or wide_gemm, None: none of them "
+        "takes it");
   m.def("gemv", &igw::gemv,
         "x W^T for a few rows of x, optional bias or SwiGLU");
   m.def("rows_gemm", &igw::rows_gemm, "x W^T of tens of rows");
+  m.def("held_gemm", &igw::held_gemm,
+        "x W^T of tens of rows, x in registers", py::arg("out"), py::arg("x"),
+        py::arg("w"), py::arg("bias") = py::none());
+  m.def("few_rows_held", &igw::few_rows_held, "whether held_gemm takes it");
   m.def("wide_gemm", &igw::wide_gemm,
         "x W^T of hundreds to thousands of rows on a given tile");
   m.def("wide_gemm_tile", &igw::wide_gemm_tile,

@@ -1,5 +1,6 @@
 // Host side of ops.linear, ops.linear_silu_mul and ops.moe_few: which calls
-// the kernels for a few rows of x (gemv.hip, rows_gemm.hip) and for hundreds
+// the kernels for a few rows of x (gemv.hip), for tens of them (rows_gemm and
+// held_gemm in rows_gemm.hip) and for hundreds
 // and thousands of them (wide_gemm.hip) take.
 //
 // What they are handed is a pointer, so the tensors have to be what they seem:
@@ -19,6 +20,9 @@ bool gemv_fits(int64_t M, int64_t K, bool swiglu);
 bool gemv_ahead(int64_t M, int64_t N, int64_t K, bool swiglu);
 int64_t rows_gemm_splits(int64_t M, int64_t N, int64_t K, bool swiglu);
 bool rows_gemm_ahead(int64_t M, int64_t S, int64_t K, bool swiglu);
+bool held_gemm_takes(int64_t M, int64_t N, int64_t K);
+void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> bias);
 int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -54,11 +58,11 @@ static bool by16(const torch::Tensor& t) {
   return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
 
-// 0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm.  `anywhere`: also off the GPU (the rule
-// alone, nothing is launched).
-int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
-                       const c10::optional<torch::Tensor>& bias, bool swiglu,
-                       bool anywhere) {
+// 0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm, 4 (only asked for with
+// `held`): held_gemm, also in the place of 2 where that would split K.
+static int64_t pick(const torch::Tensor& x, const torch::Tensor& w,
+                    const c10::optional<torch::Tensor>& bias, bool swiglu,
+                    bool anywhere, bool held) {
   if (!(anywhere || x.is_cuda()) || x.dim() != 2 || w.dim() != 2 ||
       !call_is_plain() || !plain_bf16(x, x.device()) ||
       !plain_bf16(w, x.device()))
@@ -78,8 +82,24 @@ int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
                ? 3
                : 0;
   if (gemv_fits(M, K, swiglu)) return gemv_ahead(M, w.size(0), K, swiglu);
+  if (held && !swiglu && held_gemm_takes(M, N, K)) return 4;
   const int64_t S = rows_gemm_splits(M, N, K, swiglu);
   return S > 0 && rows_gemm_ahead(M, S, K, swiglu) ? 2 : 0;
+}
+
+// Which of the kernels that go over all of x for each row of W takes the call.
+// `anywhere`: also off the GPU (the rule alone, nothing is launched).
+int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
+                       const c10::optional<torch::Tensor>& bias, bool swiglu,
+                       bool anywhere) {
+  return pick(x, w, bias, swiglu, anywhere, false);
+}
+
+// Whether it is held_gemm that takes it.
+bool few_rows_held(const torch::Tensor& x, const torch::Tensor& w,
+                   const c10::optional<torch::Tensor>& bias, bool swiglu,
+                   bool anywhere) {
+  return pick(x, w, bias, swiglu, anywhere, true) == 4;
 }
 
 // The product, or nothing when none of the kernels takes it.
@@ -87,13 +107,15 @@ c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
                                       const torch::Tensor& w,
                                       const c10::optional<torch::Tensor>& bias,
                                       bool swiglu) {
-  const int64_t which = few_rows_takes(x, w, bias, swiglu, false);
+  const int64_t which = pick(x, w, bias, swiglu, false, true);
   if (which == 0) return c10::nullopt;
   auto out = torch::empty({x.size(0), swiglu ? w.size(0) / 2 : w.size(0)},
                           x.options());
   if (which == 3)
     wide_gemm(out, x, w, swiglu,
               wide_gemm_tile(x.size(0), out.size(1), x.size(1), swiglu));
+  else if (which == 4)
+    held_gemm(out, x, w, bias);
   else
     (which == 1 ? gemv : rows_gemm)(out, x, w, bias, swiglu);
   return out;

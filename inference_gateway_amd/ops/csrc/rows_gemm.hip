@@ -225,6 +225,163 @@ __global__ __launch_bounds__(256) void rows_gemm_sum_kernel(RowsArgs a,
   *reinterpret_cast<ushort4x*>(a.out + (int64_t)row * a.N + n) = o;
 }
 
+// The same product where the kernel above does not fill the chip: x stays in
+// registers.
+//
+// W is walked 16 rows at a time by a workgroup, an eighth of K (or of the
+// split's part of it) by each of its eight waves, up to 512 entries, whose 16 or
+// 32 rows of x lie in the wave's registers as operands from start to end.  So a
+// unit of work is 128 KB of W, often in one piece, instead of 1 MB; nothing
+// but the waves' sums goes through LDS, once a unit, and a wave refills the
+// registers of a line of W for the next unit when it has turned it.  More than
+// 32 rows are two halves, in workgroups of the same XCD at the same time: the
+// second finds W in L2.
+//
+// Bound by W's bytes, and by the start for small ones (x to registers, 256 KB a
+// workgroup, and the first lines: about 4 us).  Measured, library and here (us, W
+// cold, 8 / 16 / 32 / 40 / 64 rows): 4096 x 4096 15.6 15.8 13.3 13.7 15.1 and 8.8
+// 9.3 10.7 11.4 12.2; 6144 x 4096 14.6 14.4 15.5 17.3 18.0 and 11.3 12.0 13.7 14.0
+// 15.3; 1024 x 4096 12.8 12.9 10.7 13.2 13.9 and 5.4 5.7 7.4 7.2 7.4; 4096 x 14336,
+// 16 / 32 / 43 / 64 rows, the kernel above 26.1 27.7 29.5 32.7 and 24.5 25.9 29.3
+// 30.8.  x loaded in the operands' layout instead of whole lines (a note above):
+// 4 us more.
+template <int P, int MT>
+__global__ __launch_bounds__(64 * RG_WAVES, 2) void held_gemm_kernel(
+    RowsArgs a, int S, int halves) {
+  __shared__ __attribute__((aligned(16)))
+  rg_f32x4 sums[2][RG_WAVES][MT][WAVE_SIZE];
+  __shared__ __attribute__((aligned(1024))) rg_u32x4 turned[RG_WAVES][2][128];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, quad = lane >> 4;
+  // workgroups i and i + 8 are on the same XCD: the two halves of x
+  const int half = halves == 2 ? (blockIdx.x >> 3) & 1 : 0;
+  const int id = halves == 2 ? (blockIdx.x & 7) | (blockIdx.x >> 4) << 3
+                             : blockIdx.x;
+  const int split = id % S, step = gridDim.x / (S * halves);
+  const int units = (a.N + 15) >> 4;
+  int unit = id / S;
+  if (unit >= step || unit >= units) return;
+
+  // the wave's P lines of 64 entries, from another one on in each workgroup
+  const int k0 = (split * RG_WAVES + wave) * P * 64;
+  const int rot = ((id >> 3) + wave) % P;
+  auto line = [&](int j) __attribute__((always_inline)) {
+    return k0 + (j + rot >= P ? j + rot - P : j + rot) * 64;
+  };
+  const int r8 = lane >> 3, piece = (lane & 7) * 8;
+  rg_u32x4 xf[P][2][MT], w[P][2];
+#pragma unroll
+  for (int j = 0; j < P; ++j)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        xf[j][h][m] = *reinterpret_cast<const rg_u32x4*>(
+            a.x + min((half * MT + m) * 16 + h * 8 + r8, a.M - 1) * a.x_rs +
+            line(j) + piece);
+  asm volatile("" ::: "memory");
+  const uint16_t *lo, *hi;
+  auto rows_of = [&](int u) __attribute__((always_inline)) {
+    lo = a.w + (int64_t)min(u * 16 + r8, a.N - 1) * a.K + piece;
+    hi = a.w + (int64_t)min(u * 16 + 8 + r8, a.N - 1) * a.K + piece;
+  };
+  auto load = [&](int j) __attribute__((always_inline)) {
+    w[j][0] = *reinterpret_cast<const rg_u32x4*>(lo + line(j));
+    w[j][1] = *reinterpret_cast<const rg_u32x4*>(hi + line(j));
+    asm volatile("" ::: "memory");
+  };
+  rows_of(unit);
+#pragma unroll
+  for (int j = 0; j < P; ++j) load(j);
+
+  // lines to operands, as above
+  auto perm = [](int row) __attribute__((always_inline)) {
+    return (row & 3) | ((row >> 3) & 1) << 2;
+  };
+  const int put = r8 * 8 + ((lane & 7) ^ perm(r8));
+  const int put_hi = 64 + r8 * 8 + ((lane & 7) ^ perm(8 + r8));
+  const int get = r16 * 8 + (quad ^ perm(r16));
+  const int get_hi = r16 * 8 + ((4 + quad) ^ perm(r16));
+  auto turn = [&](int b, const rg_u32x4& in0, const rg_u32x4& in1,
+                  rg_u32x4& out0, rg_u32x4& out1)
+                  __attribute__((always_inline)) {
+    rg_u32x4* t = turned[wave][b & 1];
+    t[put] = in0;
+    t[put_hi] = in1;
+    out0 = t[get];
+    out1 = t[get_hi];
+  };
+#pragma unroll
+  for (int j = 0; j < P; ++j)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      turn(j * MT + m, xf[j][0][m], xf[j][1][m], xf[j][0][m], xf[j][1][m]);
+
+  rg_f32x4 acc[MT];
+  rg_u32x4 op[2][2];
+  auto product = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(rg_bf16x8, op[j & 1][h]),
+            __builtin_bit_cast(rg_bf16x8, xf[j][h][m]), acc[m], 0, 0, 0);
+  };
+  // Adds the waves' sums.  One barrier a unit: the buffer that the next unit
+  // writes was read before the barrier of this one.
+  int turns = 0;
+  auto finish = [&](int u) __attribute__((always_inline)) {
+    const int b = turns & 1;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) sums[b][wave][m][lane] = acc[m];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int m = (wave - turns * MT) & (RG_WAVES - 1);   // waves take turns
+    ++turns;
+    if (m >= MT) return;
+    rg_f32x4 y = sums[b][0][m][lane];
+#pragma unroll
+    for (int v = 1; v < RG_WAVES; ++v) y += sums[b][v][m][lane];
+    const int row = (half * MT + m) * 16 + r16, n = u * 16 + quad * 4;
+    if (row >= a.M || n >= a.N) return;
+    if (a.part) {
+      *reinterpret_cast<rg_f32x4*>(
+          a.part + ((int64_t)split * a.M + row) * a.N + n) = y;
+    } else {
+      ushort4x o;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        o.v[e] = f32_to_bf16(
+            y[e] + (a.bias ? bf16_to_f32(a.bias[n + e]) : 0.0f));
+      *reinterpret_cast<ushort4x*>(a.out + (int64_t)row * a.N + n) = o;
+    }
+  };
+  for (;; unit += step) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = rg_f32x4{0.f, 0.f, 0.f, 0.f};
+    if (unit + step >= units) break;
+    rows_of(unit + step);
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      turn(j, w[j][0], w[j][1], op[j & 1][0], op[j & 1][1]);
+      load(j);
+      if (j) product(j - 1);
+    }
+    product(P - 1);
+    finish(unit);
+  }
+#pragma unroll
+  for (int j = 0; j < P; ++j) {
+    turn(j, w[j][0], w[j][1], op[j & 1][0], op[j & 1][1]);
+    if (j) product(j - 1);
+  }
+  product(P - 1);
+  finish(unit);
+}
+
 // In how many parts K is split for M rows of x and N outputs; 0: cannot be
 // taken, or would not fill the chip.
 //
@@ -236,7 +393,9 @@ __global__ __launch_bounds__(256) void rows_gemm_sum_kernel(RowsArgs a,
 // 33.7 and 32.8, 8192 x 4096 22.8 and 18.8.  Up to 16 rows the library is
 // ahead on 128256 x 4096 (182 and 190) and 4096 x 14336 (27 and 30); with the
 // activation inside it is behind from 9 rows on (69 and 46).  Where both can
-// run, rows_gemm_ahead says which.
+// run, rows_gemm_ahead says which.  (Times of this kernel here and below are from
+// before W was loaded in whole lines, which took off a tenth and moved no line to
+// the library's side.)
 int64_t rows_gemm_splits(int64_t M, int64_t N, int64_t K, bool swiglu) {
   if (M < (swiglu ? 9 : 17) || M > 64 || K < RG_BK || K % RG_BK != 0 ||
       N <= 0 || N % 4 != 0)
@@ -314,6 +473,101 @@ void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   else LAUNCH_RG_M(4);
 #undef LAUNCH_RG_M
 #undef LAUNCH_RG
+  HIP_CHECK_KERNEL();
+  if (S > 1) {
+    hipLaunchKernelGGL(rows_gemm_sum_kernel, dim3((N / 4 + 255) / 256, M),
+                       dim3(256), 0, stream, a, (int)S);
+    HIP_CHECK_KERNEL();
+  }
+}
+
+// In how many parts held_gemm cuts K (a wave's part is four to eight lines of
+// 64 entries); 0: it cannot.
+static int64_t held_splits(int64_t M, int64_t N, int64_t K) {
+  if (M < 1 || M > 64 || N < 1 || N % 4 != 0 || N > (1 << 26) ||
+      K > (1 << 20))
+    return 0;
+  for (int64_t S = 1; S <= 8; ++S)
+    if (K % (RG_WAVES * 64 * S) == 0) {
+      const int64_t lines = K / (RG_WAVES * 64 * S);
+      if (lines >= 4 && lines <= 8) return S;
+    }
+  return 0;
+}
+
+// Whether held_gemm is ahead of the library (and of rows_gemm in parts); gemv
+// has up to six rows, rows_gemm what it takes whole (us, library and here).  With
+// one part, up to 32 rows, at all 60 measured sizes of 16 x 2048 to 10240 x 4096
+// (16 x 2048 5.2 and 3.3, 10240 x 4096 23.4 and 20.2); wider ones to 16 rows
+// (128256 x 3584 171 and 169, 20480 x 4096 75.6 and 37.2), to 32 from K = 2560 on
+// (28672 x 2560 31.5 and 30.5; 16384 x 2048 17.3 and 18.6, 65536 x 3584 83 and 86).
+// The two halves of more rows stream W at 4.5 TB/s: 10240 x 3584, 64 rows, 25.0 and
+// 22.3, 16384 x 3584 30.4 and 38.2.  Parts cost their sums, and a short K the
+// library has tiles for: up to 32 rows 10240 x 5120 33.2 and 27.5, 16384 x 5120 37.6
+// and 39.6, 256 x 8192 8.8 and 9.2, 4096 x 8192, 16 rows, 16.2 and 16.9, 6144 x 8192
+// 27.8 and 25.0; of 64 rows 6144 x 14336 63.6 and 58.4, 8192 x 8192 34.5 and 36.3.
+static bool held_ahead(int64_t M, int64_t N, int64_t K, int64_t S) {
+  if (M < 7) return false;
+  if (M > 32) return S == 1 ? N <= 10240 : N >= 1024 && N <= 6144;
+  if (S == 1) return N <= 10240 || M <= 16 || (K >= 2560 && N <= 32768);
+  if (S == 2 && K == 8192 && M <= 24 && N > 2048 && N <= 5120) return false;
+  return N <= 10240 && (M <= 16 || N >= 1024);
+}
+
+bool held_gemm_takes(int64_t M, int64_t N, int64_t K) {
+  const int64_t S = held_splits(M, N, K);
+  return S > 0 && held_ahead(M, N, K, S) &&
+         !(rows_gemm_splits(M, N, K, false) == 1 &&
+           rows_gemm_ahead(M, 1, K, false));
+}
+
+void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> bias) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 &&
+              x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
+              w.dim() == 2 && w.is_contiguous() && out.is_contiguous() &&
+              out.dtype() == x.dtype() && out.dim() == 2);
+  const int64_t M = x.size(0), K = x.size(1), N = out.size(1);
+  const int64_t S = held_splits(M, N, K);
+  TORCH_CHECK(S >= 1);
+  TORCH_CHECK(out.size(0) == M && w.size(1) == K && w.size(0) == N &&
+              x.stride(0) % 8 == 0);
+  TORCH_CHECK(w.device() == x.device() && out.device() == x.device(),
+              "tensors on different devices");
+  TORCH_CHECK((reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0 &&
+              (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15) == 0);
+  if (bias.has_value())
+    TORCH_CHECK(bias->dtype() == x.dtype() && bias->device() == x.device() &&
+                bias->is_contiguous() && bias->numel() == N);
+  const at::cuda::CUDAGuard guard(x.device());
+  hipStream_t stream = at::cuda::getCurrentCUDAStream();
+  torch::Tensor part;
+  if (S > 1)
+    part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
+  RowsArgs a{(uint16_t*)out.data_ptr(),
+             S > 1 ? part.data_ptr<float>() : nullptr,
+             (const uint16_t*)x.data_ptr(),
+             (const uint16_t*)w.data_ptr(),
+             bias.has_value() ? (const uint16_t*)bias->data_ptr() : nullptr,
+             (int)M, (int)N, (int)K, x.stride(0)};
+  const int halves = M > 32 ? 2 : 1;
+#define LAUNCH_HELD(P)                                                        \
+  case P:                                                                     \
+    if (M <= 16)                                                              \
+      hipLaunchKernelGGL((held_gemm_kernel<P, 1>), dim3(256),                 \
+                         dim3(64 * RG_WAVES), 0, stream, a, (int)S, halves);  \
+    else                                                                      \
+      hipLaunchKernelGGL((held_gemm_kernel<P, 2>), dim3(256),                 \
+                         dim3(64 * RG_WAVES), 0, stream, a, (int)S, halves);  \
+    break
+  switch (K / (RG_WAVES * 64 * S)) {
+    LAUNCH_HELD(4);
+    LAUNCH_HELD(5);
+    LAUNCH_HELD(6);
+    LAUNCH_HELD(7);
+    LAUNCH_HELD(8);
+  }
+#undef LAUNCH_HELD
   HIP_CHECK_KERNEL();
   if (S > 1) {
     hipLaunchKernelGGL(rows_gemm_sum_kernel, dim3((N / 4 + 255) / 256, M),

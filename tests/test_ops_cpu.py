@@ -244,6 +244,31 @@ def test_few_rows_lines(M, N, K, swiglu, want):
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,want", [
+    # rows of x in registers: from seven rows on, wide ones to 16 or 32
+    (6, 4096, 4096, False), (7, 4096, 4096, True), (64, 6144, 4096, True),
+    (65, 6144, 4096, False), (64, 10240, 3584, True), (33, 16384, 3584, False),
+    (32, 16384, 3584, True), (32, 16384, 2048, False), (16, 16384, 2048, True),
+    # rows_gemm's, as one part, not in parts
+    (17, 28672, 4096, False), (16, 28672, 4096, True), (24, 4096, 14336, True),
+    (64, 4096, 14336, True), (64, 8192, 8192, False), (32, 8192, 8192, True),
+    (16, 4096, 8192, False), (17, 512, 8192, False), (16, 16384, 5120, False),
+    # lines that do not come out even, short and long K
+    (32, 4096, 11008, False), (32, 4096, 1536, False), (32, 4096, 4352, False),
+    (32, 4094, 4096, False), (32, 4096, 36864, False)])
+def test_held_gemm_lines(M, N, K, want):
+    x = torch.empty(M, K, dtype=torch.bfloat16)
+    w = torch.empty(N, K, dtype=torch.bfloat16)
+    held = ops._kernels.few_rows_held
+    assert held(x, w, None, False, True) == want
+    assert not held(x, w, None, True, True)
+    for other in (x.float(), x[:, 1:], x.to("meta"), x.clone().requires_grad_()):
+        assert not held(other, w, None, False, True)
+    assert held(x, w, w.new_empty(N), False, True) == want
+    assert not held(x, w, w.new_empty(1), False, True)
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 @pytest.mark.parametrize("M,N,K,swiglu,tile", [
     # (rows of 16 in the tile, of W) for the library's side 0
     (1024, 28672, 4096, True, (8, 7)), (16000, 28672, 4096, True, (8, 8)),
