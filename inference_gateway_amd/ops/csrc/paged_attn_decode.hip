@@ -6,9 +6,14 @@
 // step.  Bound by reading the cache; what a wave needs besides is kept small so
 // that its loads are always under way:
 //
-//   * a wave takes two pages (32 tokens) at a time, K straight to the registers
-//     that the matrix instructions read it from, V by DMA to LDS, both one step
-//     ahead: 16 KB a wave, 128 KB a compute unit under way;
+//   * a wave takes two pages (32 tokens) at a time, K to registers, V by DMA to
+//     LDS, both one step ahead: 16 KB a wave, 128 KB a compute unit under way;
+//   * eight neighbouring lanes load a 128-byte line of K, and the lines become
+//     matrix operands through 2 KB of LDS of the wave's own.  Loaded as the matrix
+//     unit wants them, neighbouring lanes in neighbouring tokens, a load is 64
+//     requests of 16 bytes and takes the cache 65 cycles instead of 16 (61
+//     sequences of 200 to 4000 tokens 112 and 109 us, 16 of 500 10.5 and 8.4, 64 of
+//     100 to 2000 with a head each 54 and 52; 1024 of 570 the same);
 //   * scores: S^T = K Q^T with mfma 16x16x32, the query heads in the columns
 //     (those past G are zero): 8 instructions for what took 256 dot products;
 //   * the result's token order follows from the layout of S^T and V is read from
@@ -114,10 +119,12 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
   // GEMM output — no .contiguous() copy on the decode hot path)
   constexpr int HD = 128, BS = 16, PAGE = BS * HD;  // tokens, entries of a page
   static_assert(NWAVES * G <= 64, "a wave's results fit its V tiles");
-  // a wave's own V tiles, two pages each: nothing here waits for another wave.
+  // a wave's own V tiles, two pages each, and K lines: nothing here waits for
+  // another wave.
   // Two objects, so that reads of one do not wait for loads to the other.
   __shared__ __attribute__((aligned(1024))) uint16_t v_s0[NWAVES][2 * PAGE];
   __shared__ __attribute__((aligned(1024))) uint16_t v_s1[NWAVES][2 * PAGE];
+  __shared__ __attribute__((aligned(1024))) pd_u32x4 k_s[NWAVES][128];
   __shared__ float m_lds[NWAVES][G];
   __shared__ float l_lds[NWAVES][G];
   const int kvh = blockIdx.x;
@@ -159,10 +166,19 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
     qf[kk] = f;
   }
 
-  // lane offsets into a page, bytes: K as the rows of a matrix operand; V four
-  // rows a load, 16-byte chunks exchanged so that the eight rows which 32 lanes
+  // lane offsets into a page, bytes: K half a row of eight rows a load, turned
+  // with its 16-byte pieces permuted by the row (no bank conflicts); V four rows
+  // a load, 16-byte chunks exchanged so that the eight rows which 32 lanes
   // of a transposing read take 32 bytes of each lie in different banks
-  const int kx = r16 * HD * 2 + quad * 16;
+  const int kx = (lane >> 3) * HD * 2 + (lane & 7) * 16;
+  auto perm = [](int row) PD_INLINE {
+    return (row & 3) | ((row >> 3) & 1) << 2;
+  };
+  const int put = (lane >> 3) * 8 + ((lane & 7) ^ perm(lane >> 3));
+  const int put_hi =
+      64 + (lane >> 3) * 8 + ((lane & 7) ^ perm(8 + (lane >> 3)));
+  const int get = r16 * 8 + (quad ^ perm(r16));
+  const int get_hi = r16 * 8 + ((4 + quad) ^ perm(r16));
   int vx[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -190,7 +206,8 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk)
         K.k[h][kk] =
-            __builtin_amdgcn_raw_buffer_load_b128(kr, kx + kk * 64, 0, 0);
+            __builtin_amdgcn_raw_buffer_load_b128(
+                kr, kx + (kk >> 1) * 128 + (kk & 1) * 8 * HD * 2, 0, 0);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
@@ -209,12 +226,23 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
     pd_f32x4 s[2];
 #pragma unroll
     for (int h = 0; h < 2; ++h) s[h] = pd_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    pd_u32x4* ks = k_s[wave];
+    pd_u32x4 kf[2][4];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        ks[put] = K.k[h][2 * c];
+        ks[put_hi] = K.k[h][2 * c + 1];
+        kf[h][2 * c] = ks[get];
+        kf[h][2 * c + 1] = ks[get_hi];
+      }
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
         s[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-            __builtin_bit_cast(pd_bf16x8, K.k[h][kk]), qf[kk], s[h], 0, 0, 0);
+            __builtin_bit_cast(pd_bf16x8, kf[h][kk]), qf[kk], s[h], 0, 0, 0);
     // token 16 (j / 4) + 4 quad + j % 4 of the pair
     float t[8];
 #pragma unroll
