@@ -92,25 +92,26 @@ class LlamaAttention(nn.Module):
         if fb.is_prefill:
             P = fb.num_prefill_tokens if fb.is_mixed else T
             qv = q.view(T, self.nq, self.hd)
+            # prompt rows and decoded rows of a mixed round side by side
+            o = qv.new_empty((T, self.nq, self.hd))
             if fb.prefix_lens is not None:
                 # prefix-cache hit in the batch: q rows are suffixes;
                 # cached prefix + the just-appended suffix K/V are read
                 # back from the paged cache (ops/csrc/flash_prefill.hip)
-                o = ops.flash_prefill_paged(
+                ops.flash_prefill_paged(
                     qv[:P], kc, vc, fb.block_table,
-                    fb.prefix_lens, fb.cu_seqlens, fb.seq_lens, self.scale)
+                    fb.prefix_lens, fb.cu_seqlens, fb.seq_lens, self.scale,
+                    out=o[:P])
             else:
-                o = ops.flash_prefill(
+                ops.flash_prefill(
                     qv[:P], k3[:P], v3[:P], fb.cu_seqlens,
-                    fb.seq_lens, self.scale)
+                    fb.seq_lens, self.scale, out=o[:P])
             if fb.is_mixed:
                 # mixed round: rows [P, T) are one decode token per
                 # running sequence (engine._build_forward_batch)
-                od = ops.paged_attn_decode(
-                    qv[P:].contiguous(), kc, vc, fb.decode_block_table,
-                    fb.decode_ctx_lens, self.scale)
-                o = torch.cat([o.view(P, self.nq, self.hd),
-                               od.view(T - P, self.nq, self.hd)], 0)
+                ops.paged_attn_decode(
+                    qv[P:], kc, vc, fb.decode_block_table,
+                    fb.decode_ctx_lens, self.scale, out=o[P:])
         else:
             o = ops.paged_attn_decode(
                 q.view(T, self.nq, self.hd), kc, vc, fb.block_table,

@@ -163,48 +163,63 @@ def rope_append(positions, q, k, v, head_dim: int, cos_sin_cache, kcache,
     append_kv_cache(k.view(rows), v.view(rows), kcache, vcache, slot_mapping)
 
 
-def paged_attn_decode(q, kcache, vcache, block_table, ctx_lens, scale: float):
+def paged_attn_decode(q, kcache, vcache, block_table, ctx_lens, scale: float,
+                      out=None):
+    """One decoded token per row of q.  out: where the result goes, contiguous
+    (None: a new tensor)."""
     if q.is_cuda:
         _require_kernels()
-        out = torch.empty_like(q)
+        out = torch.empty_like(q) if out is None else _result_like(out, q)
         _kernels.paged_attn_decode(
             out, q, kcache, vcache, block_table, ctx_lens, scale
         )
         return out
-    return torch_ref.paged_attn_decode_ref(
+    y = torch_ref.paged_attn_decode_ref(
         q, kcache, vcache, block_table, ctx_lens, scale
     )
+    return y if out is None else _result_like(out, q).copy_(y)
 
 
-def flash_prefill(q, k, v, cu_seqlens, seq_lens, scale: float):
-    """Varlen causal prefill attention. seq_lens: python list of ints."""
+def _result_like(out, q):
+    if (out.shape != q.shape or out.dtype != q.dtype
+            or out.device != q.device or not out.is_contiguous()):
+        raise ValueError("out has to be contiguous and like q")
+    return out
+
+
+def flash_prefill(q, k, v, cu_seqlens, seq_lens, scale: float, out=None):
+    """Varlen causal prefill attention. seq_lens: python list of ints.  out:
+    where the result goes, contiguous (None: a new tensor)."""
     if q.is_cuda:
         _require_kernels()
-        out = torch.empty_like(q)
+        out = torch.empty_like(q) if out is None else _result_like(out, q)
         _kernels.flash_prefill(out, q, k, v, cu_seqlens, list(seq_lens),
                                scale)
         return out
-    return torch_ref.flash_prefill_ref(q, k, v, cu_seqlens, scale)
+    y = torch_ref.flash_prefill_ref(q, k, v, cu_seqlens, scale)
+    return y if out is None else _result_like(out, q).copy_(y)
 
 
 def flash_prefill_paged(q, kcache, vcache, block_table, prefix_lens,
-                        cu_seqlens, seq_lens, scale: float):
+                        cu_seqlens, seq_lens, scale: float, out=None):
     """Paged-EXTEND prefill (chunked-prefill / prefix-cache enabler):
     q rows are a per-seq CHUNK whose own K/V plus `prefix_lens` cached
     tokens before it are all in the paged cache; each q row attends over
     cache positions [0, prefix + row].  seq_lens: python ints (q rows
-    per sequence)."""
+    per sequence).  out: where the result goes, contiguous (None: a new
+    tensor)."""
     if q.is_cuda:
         _require_kernels()
-        out = torch.empty_like(q)
+        out = torch.empty_like(q) if out is None else _result_like(out, q)
         _kernels.flash_prefill_paged(
             out, q, kcache, vcache, block_table, prefix_lens, cu_seqlens,
             list(seq_lens), scale
         )
         return out
-    return torch_ref.flash_prefill_paged_ref(
+    y = torch_ref.flash_prefill_paged_ref(
         q, kcache, vcache, block_table, prefix_lens, cu_seqlens, scale
     )
+    return y if out is None else _result_like(out, q).copy_(y)
 
 
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
