@@ -498,9 +498,12 @@ static int64_t held_splits(int64_t M, int64_t N, int64_t K) {
 // Whether held_gemm is ahead of the library (and of rows_gemm in parts); gemv
 // has up to six rows, rows_gemm what it takes whole (us, library and here).  With
 // one part, up to 32 rows, at all 60 measured sizes of 16 x 2048 to 10240 x 4096
-// (16 x 2048 5.2 and 3.3, 10240 x 4096 23.4 and 20.2); wider ones to 16 rows
-// (128256 x 3584 171 and 169, 20480 x 4096 75.6 and 37.2), to 32 from K = 2560 on
-// (28672 x 2560 31.5 and 30.5; 16384 x 2048 17.3 and 18.6, 65536 x 3584 83 and 86).
+// (16 x 2048 5.2 and 3.3, 10240 x 4096 23.4 and 20.2), wider ones to 16 rows
+// (20480 x 4096 75.6 and 37.2, 32000 x 3584 46.1 and 41.2), to 32 from K = 2560 on
+// (20480 x 3584 40.9 and 31.3, but 32000 x 3584 41.4 and 43.1, 16384 x 2048 17.3 and
+// 18.6).  At a vocabulary's width what it gains alone is lost where it runs: 128256
+// x 4096, 16 rows, 187 and 182 one after the other, but 198 and 208 behind the
+// products of a prompt.
 // The two halves of more rows stream W at 4.5 TB/s: 10240 x 3584, 64 rows, 25.0 and
 // 22.3, 16384 x 3584 30.4 and 38.2.  Parts cost their sums, and a short K the
 // library has tiles for: up to 32 rows 10240 x 5120 33.2 and 27.5, 16384 x 5120 37.6
@@ -509,7 +512,8 @@ static int64_t held_splits(int64_t M, int64_t N, int64_t K) {
 static bool held_ahead(int64_t M, int64_t N, int64_t K, int64_t S) {
   if (M < 7) return false;
   if (M > 32) return S == 1 ? N <= 10240 : N >= 1024 && N <= 6144;
-  if (S == 1) return N <= 10240 || M <= 16 || (K >= 2560 && N <= 32768);
+  if (S == 1)
+    return N <= 10240 || (M <= 16 ? N <= 32768 : K >= 2560 && N <= 20480);
   if (S == 2 && K == 8192 && M <= 24 && N > 2048 && N <= 5120) return false;
   return N <= 10240 && (M <= 16 || N >= 1024);
 }

@@ -249,6 +249,7 @@ def test_few_rows_lines(M, N, K, swiglu, want):
     (6, 4096, 4096, False), (7, 4096, 4096, True), (64, 6144, 4096, True),
     (65, 6144, 4096, False), (64, 10240, 3584, True), (33, 16384, 3584, False),
     (32, 16384, 3584, True), (32, 16384, 2048, False), (16, 16384, 2048, True),
+    (16, 32768, 4096, True), (16, 32784, 4096, False), (32, 20496, 3584, False),
     # rows_gemm's, as one part, not in parts
     (17, 28672, 4096, False), (16, 28672, 4096, True), (24, 4096, 14336, True),
     (64, 4096, 14336, True), (64, 8192, 8192, False), (32, 8192, 8192, True),
