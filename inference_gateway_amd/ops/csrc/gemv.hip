@@ -32,8 +32,8 @@ constexpr int GV_WAVES = 8;
 constexpr int GV_ROWS = 2;              // of W per wave (SWIGLU: gate and up)
 constexpr int64_t GV_MAX_X = 64 * 1024; // entries of x: 128 KB of LDS
 
-// A wave's walk over the row groups first, first + stride, ... of W [N (or 2
-// N), K] against the M rows of x in LDS.  stage() puts x there, after the
+// A wave's walk over the row groups first, first + stride, ... below `groups`
+// of W [N (or 2 N), K] against the M rows of x in LDS.  stage() puts x there, after the
 // first rows of W have been asked for; store(n, sums of W row n, of its up
 // row) is called by lane 0.
 // U is the 16-byte loads in flight per row and lane: what 128 registers leave
@@ -42,12 +42,11 @@ constexpr int64_t GV_MAX_X = 64 * 1024; // entries of x: 128 KB of LDS
 template <int M, int R, int U, bool SWIGLU, bool TAIL, class Stage,
           class Store>
 DEVINLINE void gemv_walk(const uint16_t* xs, const uint16_t* __restrict__ w,
-                         int N, int K, int first, int stride, Stage stage,
-                         Store store) {
+                         int N, int K, int first, int groups, int stride,
+                         Stage stage, Store store) {
   const int lane = threadIdx.x & 63;
   const int chunks = (K + 511) >> 9;
   constexpr int STEP = SWIGLU ? R / 2 : R;   // output columns per group
-  const int groups = (N + STEP - 1) / STEP;
 
   uint4 buf[R][U];
   auto load = [&](int grp, int c0) {
@@ -139,8 +138,10 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
     int rows, int N, int K, int64_t x_rs) {
   extern __shared__ __attribute__((aligned(16))) uint16_t xs[];   // [M][K]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int STEP = SWIGLU ? R / 2 : R;
   gemv_walk<M, R, M <= 3 ? 8 : 4, SWIGLU, TAIL>(
-      xs, w, N, K, blockIdx.x * GV_WAVES + wave, gridDim.x * GV_WAVES,
+      xs, w, N, K, blockIdx.x * GV_WAVES + wave, (N + STEP - 1) / STEP,
+      gridDim.x * GV_WAVES,
       [&] {
         gemv_stage(xs, M * K, K,
                    [&](int m) { return x + min(m, rows - 1) * x_rs; });
@@ -159,8 +160,10 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
 
 // ---------------------------------------------------------------------------
 // Experts of a small decode step.  Assignment a = t K + k sends token t to
-// expert idx[a]; blockIdx.y is the expert, an expert without a token is not
-// read (a batched product over all experts reads every one of them).  The
+// expert idx[a]; an expert without a token is not read (a batched product over
+// all experts reads every one of them).  The row groups of the experts that have
+// one, one after the other, are cut evenly for as many workgroups as the chip
+// holds: which experts those are stands in the list on the device.  The
 // assignments of an expert are found from the list, in passes of as many rows
 // as LDS holds (more than one pass only where many tokens meet wide rows).
 //
@@ -169,9 +172,12 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
 //
 // Bound by streaming the chosen experts' weights.  Measured from the hidden
 // rows to the combined ones, 8 experts of 14336 x 4096 in bf16, two per token
-// (us; batched products over the padded rows of all experts, here): 1 token
-// 588 and 136, 2 589 and 259, 5 600 and 397 (six experts reached), 8 612 and
-// 489 (5.8 TB/s).
+// (us; batched products over the padded rows of all experts, a fixed number of
+// workgroups for each expert, and the even cut): 1 token 588, 120 and 113, 2 of
+// four experts 589, 235 and 216, 5 of six or seven 600, 375 / 405 and 324 / 376
+// (6.5 TB/s), 8 of eight 612, 470 and 430.  A fixed number leaves compute units idle
+// or with one workgroup too many.  Eight loads a row in flight instead of four do
+// not fit the registers beside the passes of up to eight rows (141 for the 113).
 constexpr int GV_ASSIGN = 64;   // assignments a step may have
 
 template <bool SWIGLU, bool TAIL>
@@ -179,51 +185,83 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void expert_gemv_kernel(
     uint16_t* __restrict__ out, float* __restrict__ sums,
     const uint16_t* __restrict__ in, const uint16_t* __restrict__ w,
     const int32_t* __restrict__ idx, const float* __restrict__ weight,
-    int assigned, int top_k, int N, int K, int64_t in_rs, int max_rows) {
+    int assigned, int experts, int top_k, int N, int K, int64_t in_rs,
+    int max_rows) {
   extern __shared__ __attribute__((aligned(16))) uint16_t xs[];
   __shared__ int list[GV_ASSIGN];
+  constexpr int STEP = SWIGLU ? GV_ROWS / 2 : GV_ROWS;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int e = blockIdx.y;
-  const bool mine = lane < assigned && idx[lane] == e;
-  const uint64_t all = __ballot(mine);
-  if (all == 0) return;
-  const int count = __popcll(all);
-  if (wave == 0 && mine)
-    list[__popcll(all & ((1ull << lane) - 1))] = lane;
-  __syncthreads();
-  w += (int64_t)e * (SWIGLU ? 2 * N : N) * K;
+  // the experts in the order of their first assignments
+  int own = lane < assigned ? idx[lane] : -1;
+  if (own >= experts) own = -1;   // nobody's
+  uint64_t firsts = 0;
+  for (int a = 0; a < assigned; ++a) {
+    const int e = __builtin_amdgcn_readlane(own, a);
+    if (__builtin_ctzll(__ballot(own == e)) == a && e >= 0) firsts |= 1ull << a;
+  }
+  // of expert e: its assignments, and the passes over its rows
+  auto tokens = [&](int e) { return __ballot(own == e); };
+  auto passes = [&](uint64_t all) {
+    return (__popcll(all) + max_rows - 1) / max_rows;
+  };
+  auto expert = [&](uint64_t left) {
+    return __builtin_amdgcn_readlane(own, __builtin_ctzll(left));
+  };
+  const int groups = (N + STEP - 1) / STEP;
+  int64_t total = 0;
+  for (uint64_t left = firsts; left; left &= left - 1)
+    total += (int64_t)passes(tokens(expert(left))) * groups;
+  // this workgroup's share of the row groups, each counted once a pass
+  int64_t from = total * blockIdx.x / gridDim.x;
+  int64_t to = total * (blockIdx.x + 1) / gridDim.x;
 
-  for (int at = 0; at < count; at += max_rows) {
-    const int rows = min(max_rows, count - at);
-    auto pass = [&](auto m_) {
-      constexpr int M = decltype(m_)::value;
-      gemv_walk<M, GV_ROWS, 4, SWIGLU, TAIL>(
-          xs, w, N, K, blockIdx.x * GV_WAVES + wave, gridDim.x * GV_WAVES,
-          [&] {
-            gemv_stage(xs, rows * K, K, [&](int m) {
-              const int a = list[at + m];
-              return in + (SWIGLU ? a / top_k : a) * in_rs;
-            });
-          },
-          [&](int n, const float* y, const float* up) {
+  for (uint64_t left = firsts; left && to > 0; left &= left - 1) {
+    const int e = expert(left);
+    const uint64_t all = tokens(e);
+    const int count = __popcll(all), p = passes(all);
+    const int first = (int)(min(max(from, (int64_t)0), (int64_t)groups * p) / p);
+    const int end = (int)(min(to, (int64_t)groups * p) / p);
+    from -= (int64_t)groups * p;
+    to -= (int64_t)groups * p;
+    if (first >= end) continue;
+    const bool mine = own == e;
+    if (wave == 0 && mine)
+      list[__popcll(all & ((1ull << lane) - 1))] = lane;
+    __syncthreads();
+    const uint16_t* we = w + (int64_t)e * (SWIGLU ? 2 * N : N) * K;
+
+    for (int at = 0; at < count; at += max_rows) {
+      const int rows = min(max_rows, count - at);
+      auto pass = [&](auto m_) {
+        constexpr int M = decltype(m_)::value;
+        gemv_walk<M, GV_ROWS, 4, SWIGLU, TAIL>(
+            xs, we, N, K, first + wave, end, GV_WAVES,
+            [&] {
+              gemv_stage(xs, rows * K, K, [&](int m) {
+                const int a = list[at + m];
+                return in + (SWIGLU ? a / top_k : a) * in_rs;
+              });
+            },
+            [&](int n, const float* y, const float* up) {
 #pragma unroll
-            for (int m = 0; m < M; ++m) {
-              if (m >= rows) break;
-              const int64_t a = list[at + m];
-              if (SWIGLU)
-                out[a * N + n] =
-                    f32_to_bf16(y[m] / (1.0f + __expf(-y[m])) * up[m]);
-              else
-                sums[a * N + n] = weight[a] * y[m];
-            }
-          });
-    };
-    if (rows == 1) pass(std::integral_constant<int, 1>{});
-    else if (rows == 2) pass(std::integral_constant<int, 2>{});
-    else if (rows <= 4) pass(std::integral_constant<int, 4>{});
-    else pass(std::integral_constant<int, 8>{});
-    __syncthreads();   // x is replaced by the next pass
+              for (int m = 0; m < M; ++m) {
+                if (m >= rows) break;
+                const int64_t a = list[at + m];
+                if (SWIGLU)
+                  out[a * N + n] =
+                      f32_to_bf16(y[m] / (1.0f + __expf(-y[m])) * up[m]);
+                else
+                  sums[a * N + n] = weight[a] * y[m];
+              }
+            });
+      };
+      if (rows == 1) pass(std::integral_constant<int, 1>{});
+      else if (rows == 2) pass(std::integral_constant<int, 2>{});
+      else if (rows <= 4) pass(std::integral_constant<int, 4>{});
+      else pass(std::integral_constant<int, 8>{});
+      __syncthreads();   // x and the list are replaced by the next pass
+    }
   }
 }
 
@@ -253,7 +291,7 @@ __global__ void expert_combine_kernel(uint16_t* __restrict__ out,
 // Most tokens that moe_few takes.  With more of them the experts that many
 // tokens share are read once per pass: at 16 tokens 540 us against 594 where
 // the router spreads them and 714 where it does not, at 8 it is ahead either
-// way (409 to 489 against 612).
+// way (426 to 460 against 612).
 constexpr int64_t GV_MOE_TOKENS = 8;
 
 bool moe_few_fits(int64_t T, int64_t top_k, int64_t D, int64_t F) {
@@ -287,10 +325,8 @@ void moe_few(torch::Tensor out, torch::Tensor x, torch::Tensor gate_up,
   auto act = torch::empty({n, F}, x.options());
   auto sums = torch::empty({n, D}, x.options().dtype(torch::kFloat32));
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
-  // two workgroups per compute unit for the experts that n draws are
-  // expected to reach
-  const double reached = E * (1.0 - std::pow(1.0 - 1.0 / E, (double)n));
-  const int64_t per = std::max<int64_t>(1, (int64_t)(512.0 / reached));
+  const int64_t cus =
+      at::cuda::getCurrentDeviceProperties()->multiProcessorCount;
   auto launch = [&](auto kern, int64_t K, int64_t cols, int64_t group,
                     const torch::Tensor& in, const torch::Tensor& w) {
     // a power of two, as the kernel rounds the rows of a pass up to one
@@ -303,14 +339,17 @@ void moe_few(torch::Tensor out, torch::Tensor x, torch::Tensor gate_up,
                       (const void*)kern,
                       hipFuncAttributeMaxDynamicSharedMemorySize,
                       (int)shmem) == hipSuccess);
-    const int64_t need = (cols / group + GV_WAVES) / GV_WAVES;
-    hipLaunchKernelGGL(kern, dim3(std::min(per, need), E),
+    // as many as are there at once, no more than there is work for
+    const int64_t need =
+        (cols / group + GV_WAVES) / GV_WAVES * std::min(E, n);
+    const int64_t fit = shmem > 80 * 1024 - 256 ? cus : 2 * cus;
+    hipLaunchKernelGGL(kern, dim3(std::min(fit, need)),
                        dim3(64 * GV_WAVES), shmem, stream,
                        (uint16_t*)act.data_ptr(), sums.data_ptr<float>(),
                        (const uint16_t*)in.data_ptr(),
                        (const uint16_t*)w.data_ptr(),
                        (const int32_t*)idx.data_ptr(),
-                       (const float*)weight.data_ptr(), (int)n, (int)top_k,
+                       (const float*)weight.data_ptr(), (int)n, (int)E, (int)top_k,
                        (int)cols, (int)K, K, (int)rows);
     HIP_CHECK_KERNEL();
   };
