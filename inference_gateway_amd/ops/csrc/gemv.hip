@@ -7,8 +7,8 @@
 // before the first is used.  Products and sums are fp32 (v_dot2_f32_bf16), a
 // row's sum is completed across the wave.  Workgroups of eight waves stay for
 // the whole of W, so x is staged 512 times at most; up to 80 KB of x two of
-// them share a compute unit and keep 128 to 256 KB in flight, well past HBM
-// latency times bandwidth, with more x one keeps half of that.
+// them share a compute unit and keep 128 KB in flight, well past HBM latency
+// times bandwidth, with more x one keeps half of that.
 //
 // SWIGLU: the rows of a wave are the same rows of the gate and of the up half
 // of W; the result is silu(gate) * up of the fp32 sums, one rounding where the
@@ -33,19 +33,20 @@ constexpr int GV_ROWS = 2;              // of W per wave (SWIGLU: gate and up)
 constexpr int64_t GV_MAX_X = 64 * 1024; // entries of x: 128 KB of LDS
 
 // A wave's walk over the row groups first, first + stride, ... below `groups`
-// of W [N (or 2 N), K] against the M rows of x in LDS.  stage() puts x there, after the
-// first rows of W have been asked for; store(n, sums of W row n, of its up
-// row) is called by lane 0.
-// U is the 16-byte loads in flight per row and lane: what 128 registers leave
-// room for (two workgroups per compute unit).  TAIL: K is not a multiple of the
-// 512 entries of a load, and lanes lie past a row's end.
-template <int M, int R, int U, bool SWIGLU, bool TAIL, class Stage,
-          class Store>
+// of W [N (or 2 N), K] against the M rows of x in LDS.  stage() puts x there,
+// after the first rows of W have been asked for; store(n, sums of W row n, of
+// its up row) is called by lane 0.
+// U is the 16-byte loads in flight per row and lane; eight for up to three rows
+// were 1 to 3 % slower (three rows: 4096 x 14336 23.2 us and 22.7, 28672 x 4096
+// with SwiGLU 38.5 and 37.6).  TAIL: K is not a multiple of the 512 entries of a
+// load, and lanes lie past a row's end.
+template <int M, int R, bool SWIGLU, bool TAIL, class Stage, class Store>
 DEVINLINE void gemv_walk(const uint16_t* xs, const uint16_t* __restrict__ w,
                          int N, int K, int first, int groups, int stride,
                          Stage stage, Store store) {
   const int lane = threadIdx.x & 63;
   const int chunks = (K + 511) >> 9;
+  constexpr int U = 4;
   constexpr int STEP = SWIGLU ? R / 2 : R;   // output columns per group
 
   uint4 buf[R][U];
@@ -139,7 +140,7 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
   extern __shared__ __attribute__((aligned(16))) uint16_t xs[];   // [M][K]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int STEP = SWIGLU ? R / 2 : R;
-  gemv_walk<M, R, M <= 3 ? 8 : 4, SWIGLU, TAIL>(
+  gemv_walk<M, R, SWIGLU, TAIL>(
       xs, w, N, K, blockIdx.x * GV_WAVES + wave, (N + STEP - 1) / STEP,
       gridDim.x * GV_WAVES,
       [&] {
@@ -235,7 +236,7 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void expert_gemv_kernel(
       const int rows = min(max_rows, count - at);
       auto pass = [&](auto m_) {
         constexpr int M = decltype(m_)::value;
-        gemv_walk<M, GV_ROWS, 4, SWIGLU, TAIL>(
+        gemv_walk<M, GV_ROWS, SWIGLU, TAIL>(
             xs, we, N, K, first + wave, end, GV_WAVES,
             [&] {
               gemv_stage(xs, rows * K, K, [&](int m) {
