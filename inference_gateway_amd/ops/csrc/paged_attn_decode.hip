@@ -21,7 +21,8 @@
 //     lanes;
 //   * weights keep 16 bits of their mantissa: two bf16 parts, truncated part
 //     and rest, and two products (the matrix cores are idle otherwise).  The
-//     rest is never zero, so that an infinite value stays infinite;
+//     rest is never below the smallest normal number, so that an infinite value
+//     stays infinite at every weight;
 //   * addresses are a scalar base per page and fixed lane offsets; rows past a
 //     part's end lie past the buffer descriptor's and read as zeros, without a
 //     branch, so that the compiler knows which loads are under way;
@@ -277,7 +278,7 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
     } hi, lo;
     auto rest = [](float x) PD_INLINE {
       const float top = __uint_as_float(__float_as_uint(x) & 0xffff0000u);
-      return fmaxf(x - top, x * 0x1p-60f);
+      return fmaxf(x - top, 0x1p-126f);
     };
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
