@@ -43,9 +43,6 @@ void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                bool swiglu, int64_t tile);
 void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias);
-bool few_rows_held(const torch::Tensor& x, const torch::Tensor& w,
-                   const c10::optional<torch::Tensor>& bias, bool swiglu,
-                   bool anywhere);
 int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
                        const c10::optional<torch::Tensor>& bias, bool swiglu,
                        bool anywhere);
@@ -121,13 +118,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("held_gemm", &igw::held_gemm,
         "x W^T of tens of rows, x in registers", py::arg("out"), py::arg("x"),
         py::arg("w"), py::arg("bias") = py::none());
-  m.def("few_rows_held", &igw::few_rows_held, "whether held_gemm takes it");
   m.def("wide_gemm", &igw::wide_gemm,
         "x W^T of hundreds to thousands of rows on a given tile");
   m.def("wide_gemm_tile", &igw::wide_gemm_tile,
         "its tile (16 MT + NT) for a product; 0: not ahead of the library");
   m.def("few_rows_takes", &igw::few_rows_takes,
-        "0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm");
+        "0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm, 4: held_gemm");
   m.def("moe_few", &igw::moe_few, "SwiGLU experts of a few tokens");
   m.def("moe_rows_takes", &igw::moe_rows_takes,
         "whether the grouped products take a step");

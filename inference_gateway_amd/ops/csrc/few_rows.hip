@@ -58,11 +58,12 @@ static bool by16(const torch::Tensor& t) {
   return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
 
-// 0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm, 4 (only asked for with
-// `held`): held_gemm, also in the place of 2 where that would split K.
-static int64_t pick(const torch::Tensor& x, const torch::Tensor& w,
-                    const c10::optional<torch::Tensor>& bias, bool swiglu,
-                    bool anywhere, bool held) {
+// Which kernel takes the call.  0: none of them, 1: gemv, 2: rows_gemm, 3:
+// wide_gemm, 4: held_gemm.  `anywhere`: also off the GPU (the rule alone, nothing
+// is launched).
+int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
+                       const c10::optional<torch::Tensor>& bias, bool swiglu,
+                       bool anywhere) {
   if (!(anywhere || x.is_cuda()) || x.dim() != 2 || w.dim() != 2 ||
       !call_is_plain() || !plain_bf16(x, x.device()) ||
       !plain_bf16(w, x.device()))
@@ -82,24 +83,9 @@ static int64_t pick(const torch::Tensor& x, const torch::Tensor& w,
                ? 3
                : 0;
   if (gemv_fits(M, K, swiglu)) return gemv_ahead(M, w.size(0), K, swiglu);
-  if (held && !swiglu && held_gemm_takes(M, N, K)) return 4;
+  if (!swiglu && held_gemm_takes(M, N, K)) return 4;
   const int64_t S = rows_gemm_splits(M, N, K, swiglu);
   return S > 0 && rows_gemm_ahead(M, S, K, swiglu) ? 2 : 0;
-}
-
-// Which of the kernels that go over all of x for each row of W takes the call.
-// `anywhere`: also off the GPU (the rule alone, nothing is launched).
-int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
-                       const c10::optional<torch::Tensor>& bias, bool swiglu,
-                       bool anywhere) {
-  return pick(x, w, bias, swiglu, anywhere, false);
-}
-
-// Whether it is held_gemm that takes it.
-bool few_rows_held(const torch::Tensor& x, const torch::Tensor& w,
-                   const c10::optional<torch::Tensor>& bias, bool swiglu,
-                   bool anywhere) {
-  return pick(x, w, bias, swiglu, anywhere, true) == 4;
 }
 
 // The product, or nothing when none of the kernels takes it.
@@ -107,7 +93,7 @@ c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
                                       const torch::Tensor& w,
                                       const c10::optional<torch::Tensor>& bias,
                                       bool swiglu) {
-  const int64_t which = pick(x, w, bias, swiglu, false, true);
+  const int64_t which = few_rows_takes(x, w, bias, swiglu, false);
   if (which == 0) return c10::nullopt;
   auto out = torch::empty({x.size(0), swiglu ? w.size(0) / 2 : w.size(0)},
                           x.options());

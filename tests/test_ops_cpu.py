@@ -228,15 +228,17 @@ def test_few_rows_takes(name):
     (1, 64, 64, False, 1), (2, 16384, 512, False, 1), (4, 512, 1024, False, 0),
     (4, 4096, 14336, False, 1), (4, 4096, 8192, False, 0),
     (6, 4096, 4096, False, 1), (6, 8192, 8192, False, 0),
-    (6, 2048, 1024, False, 0), (7, 4096, 4096, False, 0),
+    (6, 2048, 1024, False, 0), (7, 4096, 4096, False, 4),
     (1, 8192, 64, True, 1), (4, 16384, 256, True, 0),
     (8, 28672, 4096, True, 1), (8, 8192, 3072, True, 0),
     # tens of rows: rows of W a multiple of 4 KB apart, long or split K
     (33, 28672, 4096, False, 2), (33, 28672, 3072, False, 0),
     (33, 28672, 11008, False, 2), (64, 28672, 11008, False, 0),
-    (17, 4096, 14336, False, 0), (24, 4096, 14336, False, 2),
-    (17, 4096, 17920, False, 2), (33, 28672, 1024, True, 2),
-    (33, 6144, 4096, False, 0)])
+    (33, 28672, 1024, True, 2), (24, 4096, 36864, False, 2),
+    (17, 4096, 14080, False, 0), (24, 4096, 14080, False, 2),
+    # and x in registers
+    (17, 4096, 14336, False, 4), (24, 4096, 14336, False, 4),
+    (17, 4096, 17920, False, 4), (33, 6144, 4096, False, 4)])
 def test_few_rows_lines(M, N, K, swiglu, want):
     x = torch.empty(M, K, dtype=torch.bfloat16)
     w = torch.empty(N, K, dtype=torch.bfloat16)
@@ -260,13 +262,16 @@ def test_few_rows_lines(M, N, K, swiglu, want):
 def test_held_gemm_lines(M, N, K, want):
     x = torch.empty(M, K, dtype=torch.bfloat16)
     w = torch.empty(N, K, dtype=torch.bfloat16)
-    held = ops._kernels.few_rows_held
-    assert held(x, w, None, False, True) == want
-    assert not held(x, w, None, True, True)
+
+    def held(x, w, bias, swiglu):
+        return ops._kernels.few_rows_takes(x, w, bias, swiglu, True) == 4
+
+    assert held(x, w, None, False) == want
+    assert not held(x, w, None, True)
     for other in (x.float(), x[:, 1:], x.to("meta"), x.clone().requires_grad_()):
-        assert not held(other, w, None, False, True)
-    assert held(x, w, w.new_empty(N), False, True) == want
-    assert not held(x, w, w.new_empty(1), False, True)
+        assert not held(other, w, None, False)
+    assert held(x, w, w.new_empty(N), False) == want
+    assert not held(x, w, w.new_empty(1), False)
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
