@@ -77,13 +77,40 @@ class MixtralMoE(nn.Module):
         # K-major copies for the batched-GEMM path: hipBLASLt/Tensile on
         # ROCm 7.2 has a layout-dependent OOB read with a TRANSPOSED-VIEW
         # B at [8,512,4096]x[8,4096,28672] (memory faults, reproduced in
-        # isolation — gpurun_out/iso3); contiguous-B runs clean
-        self.gate_up_t = nn.Parameter(
-            self.gate_up.data.transpose(1, 2).contiguous(),
-            requires_grad=False)
-        self.down_t = nn.Parameter(
-            self.down.data.transpose(1, 2).contiguous(),
-            requires_grad=False)
+        # isolation — gpurun_out/iso3); contiguous-B runs clean.  Experts that
+        # ops.moe_rows takes do without (8 of 14336 x 4096: 2.8 GB a layer)
+        k_major = self.expert_parallel or not ops.moe_rows_fits(
+            self.gate_up.new_empty((1, h)), self.gate_up, self.down,
+            self.top_k)
+        for name in ("gate_up", "down"):
+            self.register_parameter(name + "_t", nn.Parameter(
+                getattr(self, name).data.transpose(1, 2).contiguous(),
+                requires_grad=False) if k_major else None)
+        self._register_load_state_dict_pre_hook(self._load_k_major)
+
+    def _load_k_major(self, state, prefix, *_):
+        """A state dict with or without the copies loads into either."""
+        for name in ("gate_up", "down"):
+            if getattr(self, name + "_t") is None:
+                state.pop(prefix + name + "_t", None)
+            elif prefix + name in state:
+                state.setdefault(prefix + name + "_t",
+                                 state[prefix + name].transpose(1, 2))
+
+    def sync_k_major(self) -> None:
+        """After gate_up and down were written in place."""
+        for name in ("gate_up", "down"):
+            t = getattr(self, name + "_t")
+            if t is not None:
+                t.data.copy_(getattr(self, name).data.transpose(1, 2))
+
+    def _products(self, x: torch.Tensor, name: str) -> torch.Tensor:
+        """x [E, C, k] by every expert's weights."""
+        t = getattr(self, name + "_t")
+        if t is not None:
+            return torch.bmm(x, t)
+        return torch.stack([F.linear(a, w)
+                            for a, w in zip(x, getattr(self, name))])
 
     def forward(self, x: torch.Tensor,
                 is_prefill: bool = False) -> torch.Tensor:
@@ -97,7 +124,7 @@ class MixtralMoE(nn.Module):
             return self._forward_expert_parallel_padded(x)
         if ops.moe_few_fits(x, self.gate_up, self.down, self.top_k):
             # a few tokens reach a part of the experts: read only those
-            # (5 tokens 397 us a layer, over all experts 600)
+            # (5 tokens on six experts 324 us a layer, over all eight 600)
             weights, _dst, idx, _counts = ops.moe_route(
                 self.router(x).float(), self.top_k, 64)
             out = ops.moe_few(x, self.gate_up, self.down, idx, weights)
@@ -292,17 +319,15 @@ class MixtralMoE(nn.Module):
             # kernel and padding-skipping SwiGLU
             buf = x.new_zeros((E * C, h))
             buf.index_copy_(0, dst, x[flat_token])
-            gu = torch.bmm(buf.view(E, C, h), self.gate_up_t)  # [E, C, 2s]
+            gu = self._products(buf.view(E, C, h), "gate_up")  # [E, C, 2s]
             act = ops.silu_mul_grouped(gu.view(E * C, -1), counts, C)
-            y = torch.bmm(act.view(E, C, -1),
-                          self.down_t).view(E * C, h)
+            y = self._products(act.view(E, C, -1), "down").view(E * C, h)
         else:
             buf = x.new_zeros((E * C, h))
             buf.index_copy_(0, dst, x[flat_token])
-            gu = torch.bmm(buf.view(E, C, h), self.gate_up_t)  # [E, C, 2s]
+            gu = self._products(buf.view(E, C, h), "gate_up")  # [E, C, 2s]
             act = ops.silu_mul(gu.view(E * C, -1))
-            y = torch.bmm(act.view(E, C, -1),
-                          self.down_t).view(E * C, h)
+            y = self._products(act.view(E, C, -1), "down").view(E * C, h)
         ys = y.index_select(0, dst)                           # [T*K, h]
         out = torch.zeros_like(x)
         out.index_add_(0, flat_token, ys * weights.reshape(-1, 1))
@@ -318,8 +343,13 @@ class MixtralMoE(nn.Module):
         weights = torch.softmax(weights, dim=-1)          # [T, K] fp32
         # the sort-by-expert dispatch is shared with the other
         # mixture-of-experts feed-forwards (models/moe_common.py)
-        return moe_common.experts_sorted(
-            x, weights, topk_idx, self.gate_up_t, self.down_t, ops.silu_mul)
+        # one expert at a time: a transposed view does where there is no copy
+        up_t, down_t = (
+            getattr(self, name).transpose(1, 2) if t is None else t
+            for name, t in (("gate_up", self.gate_up_t),
+                            ("down", self.down_t)))
+        return moe_common.experts_sorted(x, weights, topk_idx, up_t, down_t,
+                                         ops.silu_mul)
 
 
 class MixtralLayer(nn.Module):

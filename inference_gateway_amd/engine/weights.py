@@ -239,9 +239,7 @@ def load_mixtral_weights(model, path: str) -> int:
         _copy(moe.down, torch.stack(downs), f"l{i}.experts.down")
         # keep the K-major bmm copies in sync (mixtral.py: contiguous-B
         # is both the hipBLASLt fault fix and faster)
-        moe.gate_up_t.data.copy_(
-            moe.gate_up.data.transpose(1, 2).contiguous())
-        moe.down_t.data.copy_(moe.down.data.transpose(1, 2).contiguous())
+        moe.sync_k_major()
         _copy(layer.input_norm_w, sh.full(p + "input_layernorm.weight"),
               f"l{i}.in_norm")
         _copy(layer.post_norm_w,

@@ -165,6 +165,33 @@ def test_moe_padded_matches_sorted():
     assert torch.allclose(a, b, atol=1e-5, rtol=1e-4)
 
 
+def test_moe_without_k_major_copies():
+    """Experts that the GPU's kernels take keep one copy of their weights: what
+    other calls run then, and state dicts with and without the copies."""
+    from inference_gateway_amd.engine.models.mixtral import MixtralMoE
+
+    torch.manual_seed(5)
+    cfg = MODEL_PRESETS["tiny-moe"]
+    both, one = (MixtralMoE(cfg, layer=i, device="cpu", dtype=torch.float32)
+                 for i in range(2))
+    assert both.gate_up_t is not None and both.down_t is not None
+    one.gate_up_t = one.down_t = None
+    one.load_state_dict(both.state_dict())
+    x = torch.randn(13, cfg.hidden_size)
+    for name in ("_forward_padded", "_forward_sorted"):
+        torch.testing.assert_close(getattr(one, name)(x),
+                                   getattr(both, name)(x), atol=1e-5,
+                                   rtol=1e-4)
+    other = MixtralMoE(cfg, layer=2, device="cpu", dtype=torch.float32)
+    assert "gate_up_t" not in one.state_dict()
+    other.load_state_dict(one.state_dict())
+    for name, t in both.state_dict().items():
+        assert torch.equal(other.state_dict()[name], t)
+    other.gate_up.data.mul_(2)
+    other.sync_k_major()
+    assert torch.equal(other.gate_up_t, other.gate_up.transpose(1, 2))
+
+
 def test_moe_padded_every_expert_rank_unique():
     """Dispatch ranks must give every (token, k) pair a unique padded row."""
     from inference_gateway_amd.engine.models.mixtral import MixtralMoE
