@@ -16,6 +16,7 @@
 // One workgroup; per-expert counters live in LDS.  Decode-sized T only
 // (the prefill path uses the sorted per-expert torch route).
 #include <ATen/cuda/CUDAContext.h>
+#include <c10/cuda/CUDAGuard.h>
 #include <torch/extension.h>
 
 #include "common.h"
@@ -200,6 +201,7 @@ void moe_dispatch(torch::Tensor weights, torch::Tensor dst,
               start.is_contiguous() && start.numel() == E + 1);
   for (const auto* t : {&weights, &dst, &start})
     TORCH_CHECK(t->device() == logits.device(), "tensors on different devices");
+  const at::cuda::CUDAGuard guard(logits.device());
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
 #define LAUNCH_DISPATCH(L, KV)                                                \
   hipLaunchKernelGGL((moe_dispatch_kernel<L, KV>), dim3(1), dim3(1024), 0,    \

@@ -13,6 +13,8 @@
 // y nothing is updated and the input comes from X itself; X may repeat one
 // row for all streams (stream stride 0: the state after the embedding), in
 // which case the new streams go to a buffer of their own.
+#include <c10/cuda/CUDAGuard.h>
+
 #include "../csrc_hybrid/act_types.h"
 
 namespace igw {
@@ -287,6 +289,7 @@ void moe_scatter_rows(torch::Tensor buf, torch::Tensor x, torch::Tensor dst,
   TORCH_CHECK(K >= 1 && dst.dtype() == torch::kInt64 &&
               dst.is_contiguous() && dst.numel() == T * K);
   if (T == 0) return;
+  const at::cuda::CUDAGuard guard(x.device());
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
   const bool v4 = D % 4 == 0 && x.stride(0) % 4 == 0 &&
                   reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 == 0;
@@ -356,6 +359,7 @@ void moe_combine(torch::Tensor out, torch::Tensor y, torch::Tensor dst,
                 g->size(0) == T);
   }
   if (T == 0) return;
+  const at::cuda::CUDAGuard guard(y.device());
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
 #define MCB(V)                                                                \
   hipLaunchKernelGGL(                                                         \
