@@ -107,6 +107,41 @@ DEVINLINE float block_reduce_sum(float x, float* lds) {
   return lds[0];
 }
 
+// Lines of memory to operands of the 16x16x32 matrix instructions.
+//
+// A load takes whole 128-byte lines, eight lanes a line; a matrix operand wants
+// neighbouring lanes in neighbouring rows.  The 16 lines of two loads (rows 0-7
+// and 8-15, 64 bf16 of each) go through 2 KB of LDS of the wave's own and come
+// back as the operands of their first and second 32 entries.  The 16-byte pieces
+// of a row are permuted by it, so that neither access meets itself in a bank.
+// The wave's other lanes write what a lane reads: the fences keep the compiler
+// from moving an access past another, the LDS keeps a wave's order by itself.
+struct LineTurn {
+  typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+  int put, put_hi, get, get_hi;
+  static DEVINLINE int perm(int row) { return (row & 3) | ((row >> 3) & 1) << 2; }
+  DEVINLINE explicit LineTurn(int lane) {
+    const int r8 = lane >> 3, r16 = lane & 15, quad = lane >> 4;
+    put = r8 * 8 + ((lane & 7) ^ perm(r8));
+    put_hi = 64 + r8 * 8 + ((lane & 7) ^ perm(8 + r8));
+    get = r16 * 8 + (quad ^ perm(r16));
+    get_hi = r16 * 8 + ((4 + quad) ^ perm(r16));
+  }
+  static DEVINLINE void fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+  DEVINLINE void operator()(u32x4* t, const u32x4& in0, const u32x4& in1,
+                            u32x4& out0, u32x4& out1) const {
+    fence();
+    t[put] = in0;
+    t[put_hi] = in1;
+    fence();
+    out0 = t[get];
+    out1 = t[get_hi];
+  }
+};
+
 #define HIP_CHECK_KERNEL()                                                     \
   do {                                                                         \
     hipError_t err = hipGetLastError();                                        \

@@ -168,14 +168,7 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
   // a load, 16-byte chunks exchanged so that the eight rows which 32 lanes
   // of a transposing read take 32 bytes of each lie in different banks
   const int kx = (lane >> 3) * HD * 2 + (lane & 7) * 16;
-  auto perm = [](int row) PD_INLINE {
-    return (row & 3) | ((row >> 3) & 1) << 2;
-  };
-  const int put = (lane >> 3) * 8 + ((lane & 7) ^ perm(lane >> 3));
-  const int put_hi =
-      64 + (lane >> 3) * 8 + ((lane & 7) ^ perm(8 + (lane >> 3)));
-  const int get = r16 * 8 + (quad ^ perm(r16));
-  const int get_hi = r16 * 8 + ((4 + quad) ^ perm(r16));
+  const LineTurn turn(lane);
   int vx[4];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -231,12 +224,9 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        ks[put] = K.k[h][2 * c];
-        ks[put_hi] = K.k[h][2 * c + 1];
-        kf[h][2 * c] = ks[get];
-        kf[h][2 * c + 1] = ks[get_hi];
-      }
+      for (int h = 0; h < 2; ++h)
+        turn(ks, K.k[h][2 * c], K.k[h][2 * c + 1], kf[h][2 * c],
+             kf[h][2 * c + 1]);
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll

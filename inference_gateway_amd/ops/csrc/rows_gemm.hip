@@ -78,15 +78,7 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
   const int piece = (lane & 7) * 8;
   const uint16_t* w_lo = w_row(lane >> 3) + piece;
   const uint16_t* w_hi = w_row(8 + (lane >> 3)) + piece;
-  // The 16 lines of two loads, as they come and as operands: the 16-byte pieces
-  // of a row are permuted by it so that operands are read without conflicts.
-  auto perm = [](int row) __attribute__((always_inline)) {
-    return (row & 3) | ((row >> 3) & 1) << 2;
-  };
-  const int put = (lane >> 3) * 8 + ((lane & 7) ^ perm(lane >> 3));
-  const int put_hi = 64 + (lane >> 3) * 8 + ((lane & 7) ^ perm(8 + (lane >> 3)));
-  const int get = r16 * 8 + (quad ^ perm(r16));
-  const int get_hi = r16 * 8 + ((4 + quad) ^ perm(r16));
+  const LineTurn turn_lines(lane);
   // rows of x: 512 bytes of a row per 32 lanes, its 16-byte pieces permuted by
   // the row so that the 16 rows of a matrix operand lie in different banks
   constexpr int XR = MT * 8 / RG_WAVES;    // 16-byte pieces of x per lane
@@ -131,11 +123,8 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
   auto compute = [&](const rg_u32x4 (&wr)[8], const uint16_t* s) {
     rg_u32x4 half[2][2];
     auto turn = [&](int j) __attribute__((always_inline)) {
-      rg_u32x4* t = turned[wave][j & 1];
-      t[put] = wr[2 * j];
-      t[put_hi] = wr[2 * j + 1];
-      half[j & 1][0] = t[get];
-      half[j & 1][1] = t[get_hi];
+      turn_lines(turned[wave][j & 1], wr[2 * j], wr[2 * j + 1], half[j & 1][0],
+                 half[j & 1][1]);
     };
     turn(0);
 #pragma unroll
@@ -295,22 +284,11 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void held_gemm_kernel(
 #pragma unroll
   for (int j = 0; j < P; ++j) load(j);
 
-  // lines to operands, as above
-  auto perm = [](int row) __attribute__((always_inline)) {
-    return (row & 3) | ((row >> 3) & 1) << 2;
-  };
-  const int put = r8 * 8 + ((lane & 7) ^ perm(r8));
-  const int put_hi = 64 + r8 * 8 + ((lane & 7) ^ perm(8 + r8));
-  const int get = r16 * 8 + (quad ^ perm(r16));
-  const int get_hi = r16 * 8 + ((4 + quad) ^ perm(r16));
+  const LineTurn turn_lines(lane);
   auto turn = [&](int b, const rg_u32x4& in0, const rg_u32x4& in1,
                   rg_u32x4& out0, rg_u32x4& out1)
                   __attribute__((always_inline)) {
-    rg_u32x4* t = turned[wave][b & 1];
-    t[put] = in0;
-    t[put_hi] = in1;
-    out0 = t[get];
-    out1 = t[get_hi];
+    turn_lines(turned[wave][b & 1], in0, in1, out0, out1);
   };
 #pragma unroll
   for (int j = 0; j < P; ++j)
