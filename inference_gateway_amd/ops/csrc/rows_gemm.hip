@@ -369,9 +369,8 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void held_gemm_kernel(
 // 20480 x 4096 where it has 43 (40 rows).  Splitting K to get there pays for
 // the sums only over a long K: 4096 x 14336 32.2 and 39.4, but 8192 x 8192
 // 33.7 and 32.8, 8192 x 4096 22.8 and 18.8.  Up to 16 rows the library is
-// ahead on 128256 x 4096 (182 and 190) and 4096 x 14336 (27 and 30); with the
-// activation inside it is behind from 9 rows on (69 and 46).  Where both can
-// run, rows_gemm_ahead says which.  (Times of this kernel here and below are from
+// ahead on 128256 x 4096 (182 and 190); with the activation inside it is behind
+// from 9 rows on (69 and 46).  Where both can run, rows_gemm_ahead says which.  (Times of this kernel here and below are from
 // before W was loaded in whole lines, which took off a tenth and moved no line to
 // the library's side.)
 int64_t rows_gemm_splits(int64_t M, int64_t N, int64_t K, bool swiglu) {
@@ -485,14 +484,17 @@ static int64_t held_splits(int64_t M, int64_t N, int64_t K) {
 // The two halves of more rows stream W at 4.5 TB/s: 10240 x 3584, 64 rows, 25.0 and
 // 22.3, 16384 x 3584 30.4 and 38.2.  Parts cost their sums, and a short K the
 // library has tiles for: up to 32 rows 10240 x 5120 33.2 and 27.5, 16384 x 5120 37.6
-// and 39.6, 256 x 8192 8.8 and 9.2, 4096 x 8192, 16 rows, 16.2 and 16.9, 6144 x 8192
-// 27.8 and 25.0; of 64 rows 6144 x 14336 63.6 and 58.4, 8192 x 8192 34.5 and 36.3.
+// and 39.6, 256 x 8192 8.8 and 9.2; of 64 rows 6144 x 14336 63.6 and 58.4, 8192 x
+// 8192 34.5 and 36.3.  In two parts (1024 to 8192 x 5120 to 8192, 7 to 32 rows, 288
+// sizes) it takes 0.47 to 1.0 of the library's time, but around 16 rows of 2560 x
+// 5120 to 8192 and 3072 x 6144, and for 4096 x 7168 and 8192, 6144 x 8192 and 8192 x
+// 5120, where it is 2 to 8 % behind (4096 x 8192, 16 rows, 16.9 and 17.9; 5120 x 8192,
+// 17 rows, 25.9 and 21.8).
 static bool held_ahead(int64_t M, int64_t N, int64_t K, int64_t S) {
   if (M < 7) return false;
   if (M > 32) return S == 1 ? N <= 10240 : N >= 1024 && N <= 6144;
   if (S == 1)
     return N <= 10240 || (M <= 16 ? N <= 32768 : K >= 2560 && N <= 20480);
-  if (S == 2 && K == 8192 && M <= 24 && N > 2048 && N <= 5120) return false;
   return N <= 10240 && (M <= 16 || N >= 1024);
 }
 

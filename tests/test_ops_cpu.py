@@ -255,7 +255,10 @@ def test_few_rows_lines(M, N, K, swiglu, want):
     # rows_gemm's, as one part, not in parts
     (17, 28672, 4096, False), (16, 28672, 4096, True), (24, 4096, 14336, True),
     (64, 4096, 14336, True), (64, 8192, 8192, False), (32, 8192, 8192, True),
-    (16, 4096, 8192, False), (17, 512, 8192, False), (16, 16384, 5120, False),
+    (16, 4096, 8192, True), (17, 512, 8192, False), (16, 16384, 5120, False),
+    # the same over a range of K, not but for one size
+    (24, 4096, 7168, True), (24, 4096, 8192, True), (25, 4096, 8192, True),
+    (16, 3072, 8192, True), (17, 5120, 8192, True),
     # lines that do not come out even, short and long K
     (32, 4096, 11008, False), (32, 4096, 1536, False), (32, 4096, 4352, False),
     (32, 4094, 4096, False), (32, 4096, 36864, False)])
