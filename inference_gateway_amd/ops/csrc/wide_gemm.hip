@@ -376,9 +376,14 @@ static constexpr WideTile wide_tiles[] = {
 // 4096 37.7 and 44.2).  Over a long K the second launch weighs less: 2033 x
 // 7168 x 8192 167 and 172, 4096 x 57344 x 8192 2548 and 2591, but 1024 rows of
 // the latter 773 and 658.  As a plain product the library reaches 1.55 PFLOP/s
-// where its own tiles fill the rounds, this kernel 1.45; a vocabulary's width
-// is ahead here for 256 to 2048 rows (128256 x 4096: 384 rows 435 and 331,
-// 1024 856 and 755, 2048 1584 and 1501; 4096 2921 and 2993; 192 253 and 263).
+// where its own tiles fill the rounds, this kernel 1.45; ahead is a vocabulary's
+// width of hundreds of rows, from more of them on the longer K is (65536 to 262144
+// outputs x 512 to 8192; of the library's time at 257 to 320 rows 0.63 to 1.15 up to K
+// = 4096, 0.94 to 1.35 at 6144; 321 to 640 rows 0.47 to 1.19 up to 6144, 0.83 to 1.1 at
+// 8192; 641 to 1024 rows 0.53 to 1.08; 128256 x 4096 at 288, 384 and 1024 rows 0.80,
+// 0.75 and 0.87, 892 us and 776).  Of 256 rows and of more than 1024 it is as often
+// behind (65536 x 8192, 256 rows, 232 and 264; 98304 x 2048, 1500 rows, 11 %; 131072
+// x 4096, 2048 rows, 1 %, where 128256 is 6 % ahead).
 int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu) {
   if (M < 65 || K < 6 * WG_BK || K % (2 * WG_BK) != 0 || N < 8 || N % 8 != 0)
     return 0;
@@ -394,7 +399,8 @@ int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu) {
     }
   }
   if (swiglu) return tiles >= WG_BLOCKS / 2 && (K < 8192 || M <= 1536) ? best : 0;
-  return N >= 65536 && M >= 256 && M <= 2048 ? best : 0;
+  const int64_t from = K <= 4096 ? 257 : K <= 6144 ? 321 : 641;
+  return N >= 65536 && K <= 8192 && M >= from && M <= 1024 ? best : 0;
 }
 
 // Whether the kernel's 32-bit offsets reach everything: rows of x in a tile,

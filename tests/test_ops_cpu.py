@@ -286,8 +286,12 @@ def test_held_gemm_lines(M, N, K, want):
     (128, 28672, 4096, True, 0), (512, 7168, 4096, True, 0),
     (1536, 57344, 8192, True, (8, 7)), (1537, 57344, 8192, True, 0),
     (1024, 28672, 4160, True, 0), (1024, 28680, 4096, True, 0),
-    (1024, 128256, 4096, False, (8, 8)), (256, 65536, 4096, False, (8, 8)),
-    (255, 128256, 4096, False, 0), (2049, 128256, 4096, False, 0),
+    # a vocabulary's width, more rows the longer K is
+    (1024, 128256, 4096, False, (8, 8)), (257, 128256, 4096, False, (6, 8)),
+    (256, 128256, 4096, False, 0), (1025, 128256, 4096, False, 0),
+    (320, 65536, 6144, False, 0), (321, 65536, 6144, False, (6, 8)),
+    (640, 128256, 8192, False, 0), (641, 128256, 8192, False, (8, 8)),
+    (1024, 65528, 4096, False, 0), (1024, 65536, 8320, False, 0),
     (1024, 32000, 4096, False, 0), (1024, 128256, 256, False, 0),
     # offsets of 32 bits
     (256, 131072, 8192, True, 0)])
