@@ -6,10 +6,11 @@
 // the q rows are a chunk behind `prefix` cached tokens and row r sits at
 // position prefix + r; the chunk's own keys are already appended).
 //
-// Measured with 32 heads on 8 (cards differ by 10 %): one prompt of 16000
-// tokens 1948 us, 1077 TFLOP/s (64 x 64 tiles of 16x16x32 MFMAs with V
-// transposed by the stores and P through LDS: 12518 us); 16 prompts of 512 70
-// us, 490 TFLOP/s; 2000 rows behind 6000 cached ones 256 us, 900 TFLOP/s.
+// Measured with 32 heads on 8 (cards differ by 10 %), alone and between the other
+// kernels of a step: one prompt of 16000 tokens 1979 us, 1060 TFLOP/s, and 2130 (64
+// x 64 tiles of 16x16x32 MFMAs with V transposed by the stores and P through LDS:
+// 12518 us); 16 prompts of 512 71 us, 487 TFLOP/s, and 84; 2000 rows behind 6000
+// cached ones 236 us, 974 TFLOP/s, and 279.
 
 #include <ATen/cuda/CUDAContext.h>
 #include <torch/extension.h>

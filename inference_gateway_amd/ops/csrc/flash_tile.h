@@ -38,8 +38,9 @@
 // fragments four products ahead, V one step, the weights of the second 32 keys
 // between the products of the first.  Next to nothing is left of the addresses
 // of tiles that lie whole in one sequence.  One prompt of 16000 tokens, 32
-// heads on 8, before and after these: 2290 and 2148 us, of 4000 178 and 157,
-// 16 of 512 77 and 70, 2000 rows behind 6000 277 and 256.  Computing the next
+// heads on 8, before and after these, alone and on one card: 2290 and 2148 us, of
+// 4000 178 and 157, 16 of 512 77 and 70, 2000 rows behind 6000 277 and 256 (on
+// another card 1979, 146, 71 and 236 after them).  Computing the next
 // tile's scores beside this one's weights wants more registers than there are.
 #pragma once
 

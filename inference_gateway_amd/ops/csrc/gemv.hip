@@ -37,9 +37,9 @@ constexpr int64_t GV_MAX_X = 64 * 1024; // entries of x: 128 KB of LDS
 // after the first rows of W have been asked for; store(n, sums of W row n, of
 // its up row) is called by lane 0.
 // U is the 16-byte loads in flight per row and lane; eight for up to three rows
-// were 1 to 3 % slower (three rows: 4096 x 14336 23.2 us and 22.7, 28672 x 4096
-// with SwiGLU 38.5 and 37.6).  TAIL: K is not a multiple of the 512 entries of a
-// load, and lanes lie past a row's end.
+// were up to 3 % slower alone (three rows: 4096 x 14336 23.2 us and 22.7, 28672 x
+// 4096 with SwiGLU 38.5 and 37.6), within 1 % in a step of one row.  TAIL: K is
+// not a multiple of the 512 entries of a load, and lanes lie past a row's end.
 template <int M, int R, bool SWIGLU, bool TAIL, class Stage, class Store>
 DEVINLINE void gemv_walk(const uint16_t* xs, const uint16_t* __restrict__ w,
                          int N, int K, int first, int groups, int stride,

@@ -25,7 +25,9 @@
 // TB/s) and 45.7 46.9 48.6 51.0; 28672 x 4096 at 32 / 43 / 64 rows 42.7 44.8 45.8
 // and 48.0 50.7 51.0; 128256 x 4096 178 182 189 (5.6 TB/s) and 188 193 201; 4096 x
 // 14336 27.7 29.5 32.7 and 29.9 31.2 34.1.  The library, 32 / 48 / 64 rows: 56 64
-// 55, 200 210 213 and 34 40 41.
+// 55, 200 210 213 and 34 40 41.  These are one after the other on one card; on
+// another 45.3 46.0 46.3 48.8 as SwiGLU and 186 191 195 for 128256 x 4096, which takes
+// 196 to 199 between the other kernels of a step.
 #include <ATen/cuda/CUDAContext.h>
 #include <c10/cuda/CUDAGuard.h>
 #include <torch/extension.h>
@@ -370,9 +372,9 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void held_gemm_kernel(
 // the sums only over a long K: 4096 x 14336 32.2 and 39.4, but 8192 x 8192
 // 33.7 and 32.8, 8192 x 4096 22.8 and 18.8.  Up to 16 rows the library is
 // ahead on 128256 x 4096 (182 and 190); with the activation inside it is behind
-// from 9 rows on (69 and 46).  Where both can run, rows_gemm_ahead says which.  (Times of this kernel here and below are from
-// before W was loaded in whole lines, which took off a tenth and moved no line to
-// the library's side.)
+// from 9 rows on (69 and 46).  Where both can run, rows_gemm_ahead says which.
+// (These times of this kernel are from before W was loaded in whole lines, which
+// took off up to a tenth; 28672 x 4096 48.2 and 54.6 since.)
 int64_t rows_gemm_splits(int64_t M, int64_t N, int64_t K, bool swiglu) {
   if (M < (swiglu ? 9 : 17) || M > 64 || K < RG_BK || K % RG_BK != 0 ||
       N <= 0 || N % 4 != 0)
@@ -388,15 +390,17 @@ int64_t rows_gemm_splits(int64_t M, int64_t N, int64_t K, bool swiglu) {
 // Whether rows_gemm, where it has an answer, is ahead of the library.  As one
 // part it streams W at 4.9 to 5.7 TB/s whatever K is.  The library has 5.4 to
 // 5.7 where rows of W do not lie a multiple of 4 KB apart, and less where they
-// do (us, here and library, 33 rows: 28672 x 3072 38.7 and 34.2, 32064 x 5120
-// 63.6 and 58.7; 28672 x 4096 46.5 and 47.3, 65536 x 4096 100 and 122, 28672 x
-// 6144 67.5 and 78.7); over a long K it falls behind again up to 48 rows (28672
-// x 11008 114 and 133, x 17920 186 and 181, at 64 rows 206 and 184).  Below
-// 4096 this kernel's start and end weigh (65536 x 512 24.0 and 18.4).  A split
-// K is ahead from 24 rows on, more the longer K is (4096 x 14336: 17 rows 29.1
-// and 27.6, 33 rows 30.4 and 34.0; x 17920: 34.0 and 119).  With SwiGLU the
-// library has a second launch and is behind nearly everywhere (28672 x 1024, 17
-// rows: 15.9 and 20.4; x 17920, 64 rows: 203 and 184).
+// do (us, here and library, 33 rows: 28672 x 3072 37.9 and 36.6, 32064 x 5120
+// 66.4 and 63.8; 28672 x 4096 48.2 and 54.6, 65536 x 4096 100 and 125, 28672 x
+// 6144 68.7 and 80.5); over a long K it falls behind again up to 48 rows (28672
+// x 11008 117 and 139, x 17920 189 and 189, at 64 rows 204 and 193, but x 11008
+// 129 and 142, which the line leaves to the library).  Below 4096 this kernel's
+// start and end weigh (65536 x 512 21.4 and 19.5).  A split K, where held_gemm
+// does not take it, is ahead from 24 rows on and longer ones from 17 (4096 x 14080,
+// 24 rows 28.3 and 39.8, as at 17 rows, which the line leaves to the library; x
+// 17920 33.7 and 121).  With SwiGLU the library has a second launch and is behind
+// nearly everywhere (28672 x 1024, 17 rows: 14.5 and 22.2; x 17920, 64 rows: 213 and
+// 202).
 bool rows_gemm_ahead(int64_t M, int64_t S, int64_t K, bool swiglu) {
   if (swiglu) return true;
   if (S > 1) return M >= 24 || K > 16384;

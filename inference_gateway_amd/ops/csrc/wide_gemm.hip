@@ -19,9 +19,11 @@
 //     are under way while the results are stored;
 //   * tiles of fewer rows or columns where they fill the rounds better.
 //
-// Measured, library with silu_mul and here (us): 1024 x 28672 x 4096 197 and
-// 170, 8192 rows 1377 and 1319 (1.46 PFLOP/s), 16000 rows 2804 and 2590; with no
-// stores 1242, with every step from the caches 1256 at 8192 rows.
+// Measured alone, library with silu_mul and here (us): 1024 x 28672 x 4096 217 and
+// 176, 8192 rows 1524 and 1384 (1.39 PFLOP/s), 16000 rows 2869 and 2649; between the
+// other kernels of a step 193, 1443 and 2710.  On a cooler card 197 and 170, 1377 and
+// 1319 (1.46 PFLOP/s), 2804 and 2590; there, with no stores 1242, with every step
+// from the caches 1256 at 8192 rows.
 #include <ATen/cuda/CUDAContext.h>
 #include <c10/cuda/CUDAGuard.h>
 #include <torch/extension.h>
