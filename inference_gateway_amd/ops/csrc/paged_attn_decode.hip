@@ -14,18 +14,21 @@
 //     requests of 16 bytes and takes the cache 65 cycles instead of 16 (61
 //     sequences of 200 to 4000 tokens 112 and 109 us, 16 of 500 10.5 and 8.4, 64 of
 //     100 to 2000 with a head each 54 and 52; 1024 of 570 the same);
-//   * scores: S^T = K Q^T with mfma 16x16x32, the query heads in the columns
-//     (those past G are zero): 8 instructions for what took 256 dot products;
+//   * scores: S^T = K Q^T with mfma 16x16x32, the query heads in the columns,
+//     each once for every part of its weights: 8 instructions for what took 256 dot
+//     products;
 //   * the result's token order follows from the layout of S^T and V is read from
 //     LDS in the same order (ds_read_b64_tr_b16), so weights stay in their
 //     lanes;
 //   * weights keep all 24 bits of their mantissa: three bf16 parts, each the
-//     truncated rest of the ones before, and three products (the matrix cores are
-//     idle otherwise), the sums of the second and third apart.  No rest is below
-//     the smallest normal number, so that an infinite value stays infinite at
-//     every weight.  Results that are not the nearest bf16 to 64 bits (128
-//     sequences of 200 to 700 tokens, normal entries): 2.1e-4 of them with fp32
-//     multiply-adds, 1.5e-4 here, 3.7e-3 with two parts, which saved 0.5 %;
+//     truncated rest of the ones before.  Up to four heads leave columns for all
+//     three (one product for them, their sums added at the end), eight for two.
+//     No rest is below the smallest normal number, so that an infinite value stays
+//     infinite at every weight.  Results that are not the nearest bf16 to 64 bits
+//     (128 sequences of 200 to 700 tokens, normal entries): 2.1e-4 of them with fp32
+//     multiply-adds, 1.5e-4 here, 3.7e-3 with two parts (as products of their own the
+//     three took one sequence of 500 tokens 10.3 us, here 9.7, two parts 8.4; 1024 of
+//     570 the same);
 //   * addresses are a scalar base per page and fixed lane offsets; rows past a
 //     part's end lie past the buffer descriptor's and read as zeros, without a
 //     branch, so that the compiler knows which loads are under way;
@@ -47,6 +50,8 @@
 
 #include <ATen/cuda/CUDAContext.h>
 #include <torch/extension.h>
+
+#include <type_traits>
 
 #include "common.h"
 
@@ -115,7 +120,11 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
   // q_rs: q row stride in elements (q may be a view into the fused QKV
   // GEMM output — no .contiguous() copy on the decode hot path)
   constexpr int HD = 128, BS = 16, PAGE = BS * HD;  // tokens, entries of a page
-  static_assert(NWAVES * G <= 64, "a wave's results fit its V tiles");
+  // columns of the matrix products: the heads, once for each part of their
+  // weights (with eight heads the second column has the third part too)
+  constexpr int PARTS = G <= 4 ? 3 : 2, COLS = PARTS * G;
+  static_assert(COLS <= 16 && NWAVES * COLS <= 64,
+                "a wave's results fit its V tiles");
   // a wave's own V tiles, two pages each, and K lines: nothing here waits for
   // another wave.
   // Two objects, so that reads of one do not wait for loads to the other.
@@ -152,14 +161,15 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
   };
   if (wave < pairs) load_ids(wave);
 
-  // the query heads as columns: head r16, dims 32 kk + 8 quad ..
+  // the query heads as columns: head r16 % G, dims 32 kk + 8 quad ..
   pd_bf16x8 qf[4];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) {
     pd_bf16x8 f{};
-    if (r16 < G)
-      f = *reinterpret_cast<const pd_bf16x8*>(
-          q + (int64_t)seq * q_rs + (kvh * G + r16) * HD + kk * 32 + quad * 8);
+    if (r16 < COLS)
+      f = *reinterpret_cast<const pd_bf16x8*>(q + (int64_t)seq * q_rs +
+                                              (kvh * G + r16 % G) * HD +
+                                              kk * 32 + quad * 8);
     qf[kk] = f;
   }
 
@@ -205,13 +215,16 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
     }
   };
 
-  // O^T: head r16, dims 16 d + 4 quad ..; m in log2, l of this lane's tokens
-  // (low: what the second and third parts of the weights add, which would cost
-  // the sum a rounding each)
-  pd_f32x4 acc[8], low[8];
+  // O^T: column r16, dims 16 d + 4 quad ..; m in log2, l of this lane's tokens
+  pd_f32x4 acc[8];
 #pragma unroll
-  for (int d = 0; d < 8; ++d)
-    acc[d] = low[d] = pd_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int d = 0; d < 8; ++d) acc[d] = pd_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  // what this column's part leaves out of a weight
+  const int part_of = r16 / G;
+  constexpr uint32_t TOP = 0xffff0000u;
+  const uint32_t first = part_of > 0 ? TOP : 0, second = part_of > 1 ? TOP : 0;
+  const uint32_t third = part_of == 1 ? ~0u : 0;
+  const float least = part_of > 0 ? 0x1p-126f : 0.0f;
   float m = -INFINITY, l = 0.0f;
   const float c = scale * PD_LOG2E;
   const int vrow = 4 * quad + (r16 >> 2);
@@ -258,10 +271,7 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
       m = mn;
       l *= alpha;
 #pragma unroll
-      for (int d = 0; d < 8; ++d) {
-        acc[d] *= alpha;
-        low[d] *= alpha;
-      }
+      for (int d = 0; d < 8; ++d) acc[d] *= alpha;
     }
     const float mc = m == -INFINITY ? 0.0f : m;
     float p[8];
@@ -275,20 +285,30 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
     union {
       uint32_t u[4];
       pd_bf16x8 v;
-    } part[3];
-    constexpr uint32_t TOP = 0xffff0000u;
-    auto rest = [](float x) PD_INLINE {
-      return fmaxf(x - __uint_as_float(__float_as_uint(x) & TOP), 0x1p-126f);
+    } w, w3;
+    auto minus = [](float x, uint32_t mask) PD_INLINE {
+      return x - __uint_as_float(__float_as_uint(x) & mask);
+    };
+    auto pack = [](float a, float b) PD_INLINE {   // truncated
+      return (__float_as_uint(a) >> 16) | (__float_as_uint(b) & TOP);
     };
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      float a = p[2 * e], b = p[2 * e + 1];
+      float x[2];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        part[i].u[e] = (__float_as_uint(a) >> 16) | (__float_as_uint(b) & TOP);
-        a = rest(a);
-        b = rest(b);
+      for (int i = 0; i < 2; ++i) x[i] = minus(p[2 * e + i], first);
+      if (PARTS == 3) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) x[i] = minus(x[i], second);
+      } else {
+        float y[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          y[i] = fmaxf(__uint_as_float(__float_as_uint(minus(x[i], TOP)) & third),
+                       0x1p-126f);
+        w3.u[e] = pack(y[0], y[1]);
       }
+      w.u[e] = pack(fmaxf(x[0], least), fmaxf(x[1], least));
     }
     typedef __attribute__((address_space(3))) pd_short4 lds_short4;
 #pragma unroll
@@ -303,12 +323,11 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
         vf.h[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (lds_short4*)(vs + h * PAGE + vrow * HD + chunk * 8 +
                           (r16 & 1) * 4));
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        pd_f32x4& sum = i == 0 ? acc[d] : low[d];
-        sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, part[i].v, sum, 0,
-                                                      0, 0);
-      }
+      if (PARTS == 2)
+        acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, w3.v, acc[d], 0,
+                                                         0, 0);
+      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, w.v, acc[d], 0, 0,
+                                                       0);
     }
   };
 
@@ -332,47 +351,59 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
 
   // ---- cross-wave merge, in the memory of the V tiles (the loads that are
   //      still under way there read nothing, and are waited for first)
-  float* acc_lds = reinterpret_cast<float*>(&v_s0[0][0]);  // [NWAVES][G][HD]
+  // (up to four pages are the first or the first two waves')
+  const int waves = pairs <= 2 ? max(pairs, 1) : NWAVES;
+  float* acc_lds = reinterpret_cast<float*>(&v_s0[0][0]);  // [NWAVES][COLS][HD]
   __builtin_amdgcn_s_waitcnt(0x0f70);
   __syncthreads();
-  if (r16 < G) {
-    if (quad == 0) {
+  if (wave < waves && r16 < COLS) {
+    if (r16 < G && quad == 0) {
       m_lds[wave][r16] = m;
       l_lds[wave][r16] = l;
     }
 #pragma unroll
     for (int d = 0; d < 8; ++d)
-      *reinterpret_cast<pd_f32x4*>(acc_lds + (wave * G + r16) * HD + d * 16 +
-                                   quad * 4) = acc[d] + low[d];
+      *reinterpret_cast<pd_f32x4*>(acc_lds + (wave * COLS + r16) * HD + d * 16 +
+                                   quad * 4) = acc[d];
   }
   __syncthreads();
 
-  for (int i = tid; i < G * HD; i += NWAVES * WAVE_SIZE) {
-    const int j = i / HD;
-    const int d = i % HD;
-    float M = -INFINITY;
+  auto merge = [&](auto waves_) PD_INLINE {
+    constexpr int WAVES = decltype(waves_)::value;
+    for (int i = tid; i < G * HD; i += NWAVES * WAVE_SIZE) {
+      const int j = i / HD;
+      const int d = i % HD;
+      float M = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < NWAVES; ++w) M = fmaxf(M, m_lds[w][j]);
-    float L = 0.0f, o = 0.0f;
+      for (int w = 0; w < WAVES; ++w) M = fmaxf(M, m_lds[w][j]);
+      float L = 0.0f, o = 0.0f;
 #pragma unroll
-    for (int w = 0; w < NWAVES; ++w) {
-      const float f = m_lds[w][j] == -INFINITY
-                          ? 0.0f
-                          : __builtin_amdgcn_exp2f(m_lds[w][j] - M);
-      L = fmaf(f, l_lds[w][j], L);
-      o = fmaf(f, acc_lds[(w * G + j) * HD + d], o);
-    }
-    const int64_t head = (int64_t)seq * nq + kvh * G + j;
-    if (part.count == 1) {
-      out[head * HD + d] = f32_to_bf16(o / L);
-    } else {
-      part_o[(head * nsplit + split) * HD + d] = o;
-      if (d == 0) {
-        part_ml[(head * nsplit + split) * 2] = M;
-        part_ml[(head * nsplit + split) * 2 + 1] = L;
+      for (int w = 0; w < WAVES; ++w) {
+        const float f = m_lds[w][j] == -INFINITY
+                            ? 0.0f
+                            : __builtin_amdgcn_exp2f(m_lds[w][j] - M);
+        L = fmaf(f, l_lds[w][j], L);
+        float sum = 0.0f;   // of the parts, the smallest first
+#pragma unroll
+        for (int t = PARTS - 1; t >= 0; --t)
+          sum += acc_lds[(w * COLS + t * G + j) * HD + d];
+        o = fmaf(f, sum, o);
+      }
+      const int64_t head = (int64_t)seq * nq + kvh * G + j;
+      if (part.count == 1) {
+        out[head * HD + d] = f32_to_bf16(o / L);
+      } else {
+        part_o[(head * nsplit + split) * HD + d] = o;
+        if (d == 0) {
+          part_ml[(head * nsplit + split) * 2] = M;
+          part_ml[(head * nsplit + split) * 2 + 1] = L;
+        }
       }
     }
-  }
+  };
+  if (waves == 1) merge(std::integral_constant<int, 1>{});
+  else if (waves == 2) merge(std::integral_constant<int, 2>{});
+  else merge(std::integral_constant<int, NWAVES>{});
 }
 
 // Merges the parts of every (sequence, head) that has more than one: one
