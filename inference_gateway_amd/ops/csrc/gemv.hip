@@ -36,17 +36,15 @@ constexpr int64_t GV_MAX_X = 64 * 1024; // entries of x: 128 KB of LDS
 // of W [N (or 2 N), K] against the M rows of x in LDS.  stage() puts x there,
 // after the first rows of W have been asked for; store(n, sums of W row n, of
 // its up row) is called by lane 0.
-// U is the 16-byte loads in flight per row and lane; eight for up to three rows
-// were up to 3 % slower alone (three rows: 4096 x 14336 23.2 us and 22.7, 28672 x
-// 4096 with SwiGLU 38.5 and 37.6), within 1 % in a step of one row.  TAIL: K is
-// not a multiple of the 512 entries of a load, and lanes lie past a row's end.
-template <int M, int R, bool SWIGLU, bool TAIL, class Stage, class Store>
+// U is the 16-byte loads in flight per row and lane (gemv_deep says when eight).
+// TAIL: K is not a multiple of the 512 entries of a load, and lanes lie past a
+// row's end.
+template <int M, int R, bool SWIGLU, bool TAIL, int U, class Stage, class Store>
 DEVINLINE void gemv_walk(const uint16_t* xs, const uint16_t* __restrict__ w,
                          int N, int K, int first, int groups, int stride,
                          Stage stage, Store store) {
   const int lane = threadIdx.x & 63;
   const int chunks = (K + 511) >> 9;
-  constexpr int U = 4;
   constexpr int STEP = SWIGLU ? R / 2 : R;   // output columns per group
 
   uint4 buf[R][U];
@@ -132,7 +130,7 @@ DEVINLINE void gemv_stage(uint16_t* xs, int total, int K, Row row) {
   __syncthreads();
 }
 
-template <int M, int R, bool SWIGLU, bool TAIL>
+template <int M, int R, bool SWIGLU, bool TAIL, int U>
 __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
     const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
@@ -140,7 +138,7 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
   extern __shared__ __attribute__((aligned(16))) uint16_t xs[];   // [M][K]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int STEP = SWIGLU ? R / 2 : R;
-  gemv_walk<M, R, SWIGLU, TAIL>(
+  gemv_walk<M, R, SWIGLU, TAIL, U>(
       xs, w, N, K, blockIdx.x * GV_WAVES + wave, (N + STEP - 1) / STEP,
       gridDim.x * GV_WAVES,
       [&] {
@@ -236,7 +234,7 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void expert_gemv_kernel(
       const int rows = min(max_rows, count - at);
       auto pass = [&](auto m_) {
         constexpr int M = decltype(m_)::value;
-        gemv_walk<M, GV_ROWS, SWIGLU, TAIL>(
+        gemv_walk<M, GV_ROWS, SWIGLU, TAIL, 4>(
             xs, we, N, K, first + wave, end, GV_WAVES,
             [&] {
               gemv_stage(xs, rows * K, K, [&](int m) {
@@ -406,6 +404,17 @@ bool gemv_ahead(int64_t M, int64_t N, int64_t K, bool swiglu) {
          (N >= 512 && N <= 4096 && K >= (swiglu ? 1024 : 1536) && K <= 4096);
 }
 
+// Whether eight loads a row are in flight instead of four, for up to three rows of
+// x (more of them leave no registers).  Four are up to 8 % ahead at most sizes;
+// eight where five to seven make a whole row, and where rows of W lie a multiple of
+// 16 KB apart, of which fewer loads reach fewer of the memory channels (us, four and
+// eight, one row: 5120 x 5120 12.3 and 12.9, 7680 x 5120 14.4 and 15.2; 2560 wide 2
+// to 11 % apart, 8192 x 8192 29.4 and 26.8, 10240 x 8192 35.7 and 32.6, 16384 wide 1
+// to 17 %).  At 4096 wide up to 2048 outputs would want eight too (5.9 and 5.5).
+static bool gemv_deep(int64_t M, int64_t K) {
+  return M <= 3 && (K % 8192 == 0 || (K > 2048 && K <= 3584));
+}
+
 // out [M, N] = x [M, K] W^T (+ bias [N]); swiglu: W [2 N, K], out = silu(x
 // Wg^T) * (x Wu^T).  Rows of x and W 16-byte aligned.
 void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -436,12 +445,12 @@ void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   const int64_t step = swiglu ? GV_ROWS / 2 : GV_ROWS;
   const int64_t need = ((N + step - 1) / step + GV_WAVES - 1) / GV_WAVES;
   const dim3 grid(std::min<int64_t>(need, 512));
-#define LAUNCH_GV(MV)                                                         \
+#define LAUNCH_GV(MV, U)                                                      \
   do {                                                                        \
-    auto kern = K % 512 ? (swiglu ? gemv_kernel<MV, GV_ROWS, true, true>      \
-                                  : gemv_kernel<MV, GV_ROWS, false, true>)    \
-                        : (swiglu ? gemv_kernel<MV, GV_ROWS, true, false>     \
-                                  : gemv_kernel<MV, GV_ROWS, false, false>);  \
+    auto kern = K % 512 ? (swiglu ? gemv_kernel<MV, GV_ROWS, true, true, U>   \
+                                  : gemv_kernel<MV, GV_ROWS, false, true, U>) \
+                        : (swiglu ? gemv_kernel<MV, GV_ROWS, true, false, U>  \
+                                  : gemv_kernel<MV, GV_ROWS, false, false, U>); \
     if (shmem > 64 * 1024)                                                    \
       TORCH_CHECK(hipFuncSetAttribute(                                        \
                       (const void*)kern,                                      \
@@ -453,13 +462,23 @@ void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                        (const uint16_t*)w.data_ptr(), b, (int)M, (int)N,      \
                        (int)K, x.stride(0));                                  \
   } while (0)
+  const bool deep = gemv_deep(M, K);
   switch (mp) {
-    case 1: LAUNCH_GV(1); break;
-    case 2: LAUNCH_GV(2); break;
-    case 3: LAUNCH_GV(3); break;
-    case 4: LAUNCH_GV(4); break;
-    case 6: LAUNCH_GV(6); break;
-    default: LAUNCH_GV(8); break;
+    case 1:
+      if (deep) LAUNCH_GV(1, 8);
+      else LAUNCH_GV(1, 4);
+      break;
+    case 2:
+      if (deep) LAUNCH_GV(2, 8);
+      else LAUNCH_GV(2, 4);
+      break;
+    case 3:
+      if (deep) LAUNCH_GV(3, 8);
+      else LAUNCH_GV(3, 4);
+      break;
+    case 4: LAUNCH_GV(4, 4); break;
+    case 6: LAUNCH_GV(6, 4); break;
+    default: LAUNCH_GV(8, 4); break;
   }
 #undef LAUNCH_GV
   HIP_CHECK_KERNEL();
