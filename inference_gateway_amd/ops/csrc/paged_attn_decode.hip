@@ -123,8 +123,7 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
   // columns of the matrix products: the heads, once for each part of their
   // weights (with eight heads the second column has the third part too)
   constexpr int PARTS = G <= 4 ? 3 : 2, COLS = PARTS * G;
-  static_assert(COLS <= 16 && NWAVES * COLS <= 64,
-                "a wave's results fit its V tiles");
+  static_assert(COLS * HD * 4 <= 2 * PAGE * 2, "a wave's results fit its V tiles");
   // a wave's own V tiles, two pages each, and K lines: nothing here waits for
   // another wave.
   // Two objects, so that reads of one do not wait for loads to the other.
@@ -464,7 +463,7 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
                           hipStream_t stream) {
   const int B = q.size(0);
   const int nkv = kcache.size(1);
-  constexpr int NWAVES = 4, HD = 128;
+  constexpr int HD = 128;
   const int nq = q.size(1);
   const int max_blocks = block_table.size(1);
   // The chip holds 512 of these workgroups (two per compute unit, by their
@@ -498,15 +497,29 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
     part_o = part.data_ptr<float>();
     part_ml = part_o + n * HD;
   }
-  hipLaunchKernelGGL((paged_attn_decode_kernel<G, NWAVES>),
-                     dim3(nkv, B, nsplit), dim3(NWAVES * WAVE_SIZE), 0, stream,
-                     (uint16_t*)out.data_ptr(), (const uint16_t*)q.data_ptr(),
-                     (const uint16_t*)kcache.data_ptr(),
-                     (const uint16_t*)vcache.data_ptr(),
-                     (const int32_t*)block_table.data_ptr(),
-                     (const int32_t*)ctx_lens.data_ptr(), max_blocks, nkv,
-                     scale, (int)q.stride(0), part_o, part_ml, nsplit,
-                     min_blocks);
+  auto launch = [&](auto waves_) {
+    constexpr int NWAVES = decltype(waves_)::value;
+    hipLaunchKernelGGL((paged_attn_decode_kernel<G, NWAVES>),
+                       dim3(nkv, B, nsplit), dim3(NWAVES * WAVE_SIZE), 0,
+                       stream, (uint16_t*)out.data_ptr(),
+                       (const uint16_t*)q.data_ptr(),
+                       (const uint16_t*)kcache.data_ptr(),
+                       (const uint16_t*)vcache.data_ptr(),
+                       (const int32_t*)block_table.data_ptr(),
+                       (const int32_t*)ctx_lens.data_ptr(), max_blocks, nkv,
+                       scale, (int)q.stride(0), part_o, part_ml, nsplit,
+                       min_blocks);
+  };
+  // Four waves a workgroup, but two where one or two query heads share a key head and
+  // the chip is filled many times over: the bytes of a short context are few for its
+  // workgroup's start and end, and twice as many are there at a time (us, four and
+  // two: a head each, 256 sequences of 60 tokens 20.7 and 18.4, 1024 70.6 and 55, of
+  // 500 and more the same; 64 of 4000 189 and 200).  With more heads two are 3 %
+  // behind over long contexts.
+  if (G <= 2 && whole >= 1024)
+    launch(std::integral_constant<int, G <= 2 ? 2 : 4>{});
+  else
+    launch(std::integral_constant<int, 4>{});
   HIP_CHECK_KERNEL();
   if (nsplit > 1) {
     hipLaunchKernelGGL((paged_attn_merge_kernel<HD>), dim3(nq, B), dim3(HD), 0,
