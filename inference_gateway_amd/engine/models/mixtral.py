@@ -76,9 +76,9 @@ class MixtralMoE(nn.Module):
                                  requires_grad=False)
         # K-major copies for the batched-GEMM path: hipBLASLt/Tensile on
         # ROCm 7.2 has a layout-dependent OOB read with a TRANSPOSED-VIEW
-        # B at [8,512,4096]x[8,4096,28672] (memory faults, reproduced in
-        # isolation — gpurun_out/iso3); contiguous-B runs clean.  Experts that
-        # ops.moe_rows takes do without (8 of 14336 x 4096: 2.8 GB a layer)
+        # B at [8,512,4096]x[8,4096,28672] (memory faults); contiguous-B runs
+        # clean.  Experts that ops.moe_rows takes do without (8 of 14336 x
+        # 4096: 2.8 GB a layer)
         k_major = self.expert_parallel or not ops.moe_rows_fits(
             self.gate_up.new_empty((1, h)), self.gate_up, self.down,
             self.top_k)
@@ -203,8 +203,8 @@ class MixtralMoE(nn.Module):
 
     def _forward_expert_parallel_padded(self, x: torch.Tensor
                                         ) -> torch.Tensor:
-        """Sync-free EP for DECODE (the dynamic-split
-        EP path host-syncs on .tolist() and cannot be graph-captured).
+        """Sync-free EP for DECODE (the dynamic-split EP path host-syncs on
+        .tolist() and cannot be graph-captured).
         Every (src, dst) pair exchanges a STATIC capacity of
         cap = ceil(Tl)*K rows — the worst case, so routing is EXACT
         (zero token drops) — which makes both all-to-alls equal-split
