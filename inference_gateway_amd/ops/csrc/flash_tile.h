@@ -271,8 +271,12 @@ DEVINLINE int ft_kswz(int r) {
 // VD < NV: the four waves have the SAME 32 query rows and each the VD value
 // dims from dim0 on (decoded rows: the heads that share keys).
 // SHARED: the values are the first entries of the key rows, v0 and v1 unused.
+// ONCE: decoded rows, whose keys nobody else reads: loads are nontemporal and
+// leave nothing in the memory side's cache (a step of 48 sequences of 700 to 3500
+// keys, two latent and two windowed layers of 32 heads: 864 and 836 us, some of it
+// by the products' loads).
 template <int NK, int NV, bool PLAIN, class Rows, int VD = NV,
-          bool SHARED = false>
+          bool SHARED = false, bool ONCE = false>
 DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
                            const FlashScore& sc,
                            const ft_bf16x8 (&qf)[NK / 16], uint8_t* k0,
@@ -282,6 +286,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
   constexpr int BN = FT_BN, CK = NK / 8, CV = SHARED ? 0 : NV / 8;
   constexpr int VROW = SHARED ? NK * 2 : NV * 2;   // bytes of a V row
   constexpr int RW = BN / FT_WAVES;   // rows that a wave moves
+  constexpr int AUX = ONCE ? 2 : 0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int half = lane >> 5, col = lane & 31;
@@ -322,12 +327,12 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
         for (int i = 0; i < CK / 4; ++i)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
               kr, (lds_void*)(kd + (wave * (CK / 4) + i) * 1024), 16, ko[i], 0,
-              0, 0);
+              0, AUX);
 #pragma unroll
         for (int i = 0; i < CV / 4; ++i)
           __builtin_amdgcn_raw_ptr_buffer_load_lds(
               vr, (lds_void*)(vd + (wave * (CV / 4) + i) * 1024), 16, vo[i], 0,
-              0, 0);
+              0, AUX);
       }
     }
     if (!straight) {
@@ -338,7 +343,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
               reinterpret_cast<const uint32_t*>(
                   rows.template kp<decltype(pad)::value>(k_row(i), k_chunk(i))),
               reinterpret_cast<uint32_t*>(kd + (wave * (CK / 4) + i) * 1024),
-              16, 0, 0);
+              16, 0, AUX);
       };
       // where nothing is padded the address stays a scalar base and an offset
       if (rows.key_width() < NK) keys(std::true_type{});
@@ -348,7 +353,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
         __builtin_amdgcn_global_load_lds(
             reinterpret_cast<const uint32_t*>(rows.vp(v_row(i), v_chunk(i))),
             reinterpret_cast<uint32_t*>(vd + (wave * (CV / 4) + i) * 1024), 16,
-            0, 0);
+            0, AUX);
     }
     rows.prefetch(span.next(kbase), wave);
   };

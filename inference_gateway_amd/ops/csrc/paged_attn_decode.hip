@@ -41,7 +41,7 @@
 //     merged by a second kernel.
 //
 // Measured, with dot products and fp32 multiply-adds on the vector units (450
-// instructions a page) and here (32 heads on 8, us): 1024 sequences of 554 to
+// instructions a page) and here, before the loads were nontemporal (PD_ONCE) (32 heads on 8, us): 1024 sequences of 554 to
 // 590 tokens 466 and 410 (5.9 TB/s), 300 of 3000 764 and 637, 61 of 200 to 4000
 // 134 and 104, 128 of 100 to 2000 159 and 109, 16 of 500 16.5 and 11.2; 64 heads
 // on 8, 64 of 400 to 4000 250 and 119.  One, two or eight waves a workgroup:
@@ -76,6 +76,18 @@ DEVINLINE void pd_both32(float x, float& a, float& b) {
   a = b = x;
   asm("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 0" : "+v"(a), "+v"(b));
 }
+
+// From this many tokens x key heads on, a workgroup's own context for every
+// sequence of the step (40 MB of keys and values), the cache is read with
+// nontemporal loads.  What is read once a step and cannot wait for the next one in
+// the 256 MB memory-side cache is then not put there first: 1024 sequences of 570
+// tokens 5.8 and 6.5 TB/s.  Below, several layers' caches fit it together, and loads
+// that pass it by are the slower ones (us, 32 heads on 8, eight caches in turn,
+// plain and nontemporal: 9 of 500 10.5 and 12.1, of 700 12.2 and 14.1, of 1500 23.6
+// and 21.8; 16 of 500 11.4 and 12.4, of 700 16.6 and 14.8; 4 of 1500 14.8 and 14.7,
+// of 4000 21.7 and 19.5; 64 of 700 40.4 and 34.8, 128 of 700 75 and 63, 1024 of 500
+// 376 and 337; 33 of 16000 400 and 351).
+constexpr int64_t PD_ONCE = 80000;
 
 // maximum and sum over the four lanes that share lane & 15
 DEVINLINE float pd_max(float x) {
@@ -189,7 +201,8 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
   };
   typedef __attribute__((address_space(3))) void lds_void;
   // pair u; past the part's end nothing is read and the values are zeros
-  auto fetch = [&](int u, Keys& K, uint16_t* vs) PD_INLINE {
+  auto fetch = [&](auto once, int u, Keys& K, uint16_t* vs) PD_INLINE {
+    constexpr int NT = decltype(once)::value ? 2 : 0;   // bit 1: nontemporal
     const int at = (u - wave) / NWAVES;
     const int left = limit - (block0 + 2 * u) * BS;
 #pragma unroll
@@ -206,11 +219,11 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
       for (int kk = 0; kk < 4; ++kk)
         K.k[h][kk] =
             __builtin_amdgcn_raw_buffer_load_b128(
-                kr, kx + (kk >> 1) * 128 + (kk & 1) * 8 * HD * 2, 0, 0);
+                kr, kx + (kk >> 1) * 128 + (kk & 1) * 8 * HD * 2, 0, NT);
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            vr, (lds_void*)(vs + h * PAGE + i * 512), 16, vx[i], 0, 0, 0);
+            vr, (lds_void*)(vs + h * PAGE + i * 512), 16, vx[i], 0, 0, NT);
     }
   };
 
@@ -330,13 +343,13 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
     }
   };
 
-  auto ahead = [&](int u, Keys& K, uint16_t* vs) PD_INLINE {
-    if ((((u - wave) / NWAVES) & 31) == 0 && u < pairs) load_ids(u);
-    fetch(u, K, vs);
-  };
   Keys k0, k1;
-  if (wave < pairs) {
-    fetch(wave, k0, v_s0[wave]);
+  auto walk = [&](auto once) PD_INLINE {
+    auto ahead = [&](int u, Keys& K, uint16_t* vs) PD_INLINE {
+      if ((((u - wave) / NWAVES) & 31) == 0 && u < pairs) load_ids(u);
+      fetch(once, u, K, vs);
+    };
+    fetch(once, wave, k0, v_s0[wave]);
     for (int u = wave;; u += 2 * NWAVES) {
       ahead(u + NWAVES, k1, v_s1[wave]);
       use(u, k0, v_s0[wave]);
@@ -345,6 +358,10 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
       use(u + NWAVES, k1, v_s1[wave]);
       if (u + 2 * NWAVES >= pairs) break;
     }
+  };
+  if (wave < pairs) {
+    if ((int64_t)ctx * gridDim.y * nkv >= PD_ONCE) walk(std::true_type{});
+    else walk(std::false_type{});
   }
   l = pd_sum(l);
 

@@ -70,7 +70,7 @@ __global__ __launch_bounds__(64 * FT_WAVES, 1) void latent_decode_kernel(
                  a.size, R + a.RD, 0, pos + 1};
   ft_f32x16 o[VD / 32];
   float m, l;
-  flash_tiles<NK, R, false, PagedRows, VD, true>(
+  flash_tiles<NK, R, false, PagedRows, VD, true, true>(
       rows, span, sc, qf, k_s0, k_s1, nullptr, nullptr, o, m, l, wave * VD);
   if (head >= H) return;
   if (a.parts.nsplit > 1) {
