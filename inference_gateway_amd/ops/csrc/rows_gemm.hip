@@ -17,6 +17,14 @@
 // 4096, 16 rows, before the lines were turned: 52.0 us, with the starts apart
 // 48.0).
 //
+// W is read once a step, and by nontemporal loads: others leave it in the memory
+// side's cache, which has no room for a model, and that costs the memory a ninth of
+// its rate (loads alone, 128256 rows of 8 KB in this pattern, 183 and 157 us, 28672
+// of them 45.0 and 39.4; a row at a time, 1 KB a load, 168 and 150).  Of 49 rows and
+// more the kernel waits for other things, and between the others of a step plain
+// loads are as good (28672 x 4096 as SwiGLU 47.0 and 47.3 us, 43 rows 44.3 and 42.3;
+// 128256 x 4096, 61 rows, 194 and 199).
+//
 // SWIGLU: a wave's 16 rows are eight gate rows and the up rows of the same
 // outputs, and the result is silu(gate) * up of the fp32 sums.
 //
@@ -101,9 +109,11 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
       xr[i] = *reinterpret_cast<const rg_u32x4*>(xp[i] + k);
     asm volatile("" ::: "memory");
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
-      wr[j] = *reinterpret_cast<const rg_u32x4*>(
+    for (int j = 0; j < 8; ++j) {
+      const auto* p = reinterpret_cast<const rg_u32x4*>(
           (j & 1 ? w_hi : w_lo) + k + ((j / 2 + wave) & 3) * 64);
+      wr[j] = MT < 4 ? __builtin_nontemporal_load(p) : *p;
+    }
     asm volatile("" ::: "memory");
   };
   auto put_x = [&](const rg_u32x4 (&xr)[XR], uint16_t* s) {
@@ -236,9 +246,16 @@ __global__ __launch_bounds__(256) void rows_gemm_sum_kernel(RowsArgs a,
 // 16 / 32 / 43 / 64 rows, the kernel above 26.1 27.7 29.5 32.7 and 24.5 25.9 29.3
 // 30.8.  x loaded in the operands' layout instead of whole lines (a note above):
 // 4 us more.
-template <int P, int MT>
+//
+// ONCE: W is loaded past the caches of the memory's side (see above).  Not where a
+// second half wants it again, and not the few MB that may have stayed there since
+// the last step (HELD_ONCE: 1024 x 4096, 16 rows, 16 of them in turn, 5.7 us and
+// 6.6 so; 2560 x 5120 11.9 and 11.0, 4096 x 14336 27.0 and 24.8).
+constexpr int64_t HELD_ONCE = 12 << 20;   // entries of W
+
+template <int P, int MT, int halves, bool ONCE>
 __global__ __launch_bounds__(64 * RG_WAVES, 2) void held_gemm_kernel(
-    RowsArgs a, int S, int halves) {
+    RowsArgs a, int S) {
   __shared__ __attribute__((aligned(16)))
   rg_f32x4 sums[2][RG_WAVES][MT][WAVE_SIZE];
   __shared__ __attribute__((aligned(1024))) rg_u32x4 turned[RG_WAVES][2][128];
@@ -278,8 +295,12 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void held_gemm_kernel(
     hi = a.w + (int64_t)min(u * 16 + 8 + r8, a.N - 1) * a.K + piece;
   };
   auto load = [&](int j) __attribute__((always_inline)) {
-    w[j][0] = *reinterpret_cast<const rg_u32x4*>(lo + line(j));
-    w[j][1] = *reinterpret_cast<const rg_u32x4*>(hi + line(j));
+    auto of = [&](const uint16_t* p) __attribute__((always_inline)) {
+      const auto* q = reinterpret_cast<const rg_u32x4*>(p + line(j));
+      return ONCE ? __builtin_nontemporal_load(q) : *q;
+    };
+    w[j][0] = of(lo);
+    w[j][1] = of(hi);
     asm volatile("" ::: "memory");
   };
   rows_of(unit);
@@ -538,15 +559,17 @@ void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
              (const uint16_t*)w.data_ptr(),
              bias.has_value() ? (const uint16_t*)bias->data_ptr() : nullptr,
              (int)M, (int)N, (int)K, x.stride(0)};
-  const int halves = M > 32 ? 2 : 1;
+  const bool once = M <= 32 && N * K >= HELD_ONCE;
+#define LAUNCH_HELD_AS(...)                                                   \
+  hipLaunchKernelGGL((held_gemm_kernel<__VA_ARGS__>), dim3(256),              \
+                     dim3(64 * RG_WAVES), 0, stream, a, (int)S)
 #define LAUNCH_HELD(P)                                                        \
   case P:                                                                     \
-    if (M <= 16)                                                              \
-      hipLaunchKernelGGL((held_gemm_kernel<P, 1>), dim3(256),                 \
-                         dim3(64 * RG_WAVES), 0, stream, a, (int)S, halves);  \
-    else                                                                      \
-      hipLaunchKernelGGL((held_gemm_kernel<P, 2>), dim3(256),                 \
-                         dim3(64 * RG_WAVES), 0, stream, a, (int)S, halves);  \
+    if (M > 32) LAUNCH_HELD_AS(P, 2, 2, false);                               \
+    else if (M > 16 && once) LAUNCH_HELD_AS(P, 2, 1, true);                   \
+    else if (M > 16) LAUNCH_HELD_AS(P, 2, 1, false);                          \
+    else if (once) LAUNCH_HELD_AS(P, 1, 1, true);                             \
+    else LAUNCH_HELD_AS(P, 1, 1, false);                                      \
     break
   switch (K / (RG_WAVES * 64 * S)) {
     LAUNCH_HELD(4);
@@ -556,6 +579,7 @@ void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     LAUNCH_HELD(8);
   }
 #undef LAUNCH_HELD
+#undef LAUNCH_HELD_AS
   HIP_CHECK_KERNEL();
   if (S > 1) {
     hipLaunchKernelGGL(rows_gemm_sum_kernel, dim3((N / 4 + 255) / 256, M),
