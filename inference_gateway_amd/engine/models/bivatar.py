@@ -96,8 +96,8 @@ class GatedMLP(nn.Module):
                        spec.ff)
 
     def forward(self, h: torch.Tensor, fb: ForwardBatch) -> torch.Tensor:
-        return ops.linear(ops.gated_act(ops.linear(h, self.gate_up), self.mode),
-                        self.down)
+        return ops.linear(ops.linear_gated_act(h, self.gate_up, self.mode),
+                          self.down)
 
 
 class PostNormLayer(nn.Module):

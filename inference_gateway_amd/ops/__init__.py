@@ -236,28 +236,29 @@ def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
     return torch_ref.silu_mul_ref(gate_up)
 
 
-def _own_product(x, w, bias, swiglu: bool):
-    """x W^T by the kernels here (a few rows ops/csrc/gemv.hip, tens of them
-    ops/csrc/rows_gemm.hip, hundreds to thousands ops/csrc/wide_gemm.hip), or
-    None where they do not take the call (ops/csrc/few_rows.hip says which)."""
+def _own_product(x, w, bias, gate: int):
+    """x W^T (gate 0) or act(x Wg^T) * (x Wu^T) (1 SiLU, 2 GELU) by the kernels
+    here (a few rows ops/csrc/gemv.hip, tens of them ops/csrc/rows_gemm.hip,
+    hundreds to thousands ops/csrc/wide_gemm.hip), or None where they do not take
+    the call (ops/csrc/few_rows.hip says which)."""
     if (has_torch_function_variadic(x, w) or torch.compiler.is_compiling()
             or not (x.is_cuda and HAS_KERNELS)):
         return None
-    return _kernels.few_rows(x, w, bias, swiglu)
+    return _kernels.few_rows(x, w, bias, gate)
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     """x W^T (+ bias).  A few rows of bf16 run the weight-streaming kernels,
     hundreds of them over a vocabulary's width the tiled one, everything else
     the library's product."""
-    out = _own_product(x, w, bias, False)
+    out = _own_product(x, w, bias, 0)
     return torch.nn.functional.linear(x, w, bias) if out is None else out
 
 
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T) with w = [Wg; Wu]: one kernel for bf16 rows
     where it is ahead, else the product and silu_mul."""
-    out = _own_product(x, w, None, True)
+    out = _own_product(x, w, None, 1)
     return (silu_mul(torch.nn.functional.linear(x, w)) if out is None
             else out)
 
@@ -761,6 +762,15 @@ def gated_act(gate_up, mode: int, limit: float = 0.0, alpha: float = 1.0):
         _shared_ext("gated_act")(out, gate_up, mode, limit, alpha)
         return out
     return torch_ref.gated_act_ref(gate_up, mode, limit, alpha)
+
+
+def linear_gated_act(x: torch.Tensor, w: torch.Tensor, mode: int,
+                     limit: float = 0.0, alpha: float = 1.0) -> torch.Tensor:
+    """gated_act of x W^T, w = [Wg; Wu]: one kernel for bf16 rows where it is
+    ahead and mode is SiLU or GELU, else the product and gated_act."""
+    gate = {GATED_ACT_SILU: 1, GATED_ACT_GELU: 2}.get(mode)
+    out = None if gate is None else _own_product(x, w, None, gate)
+    return gated_act(linear(x, w), mode, limit, alpha) if out is None else out
 
 
 # ---------------------------------------------------------------------------

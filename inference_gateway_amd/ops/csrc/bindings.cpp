@@ -35,12 +35,12 @@ void flash_prefill_paged(torch::Tensor out, torch::Tensor q,
                          std::vector<int64_t> seq_lens, double scale);
 int64_t rows_gemm_splits(int64_t M, int64_t N, int64_t K, bool swiglu);
 void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-          c10::optional<torch::Tensor> bias, bool swiglu);
+          c10::optional<torch::Tensor> bias, int64_t gate);
 void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias, bool swiglu);
+               c10::optional<torch::Tensor> bias, int64_t gate);
 int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               bool swiglu, int64_t tile);
+               int64_t gate, int64_t tile);
 void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias);
 int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
@@ -49,7 +49,7 @@ int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
 c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
                                       const torch::Tensor& w,
                                       const c10::optional<torch::Tensor>& bias,
-                                      bool swiglu);
+                                      int64_t gate);
 bool moe_few_takes(const torch::Tensor& x, const torch::Tensor& gate_up,
                    const torch::Tensor& down, int64_t top_k, bool anywhere);
 bool moe_rows_takes(const torch::Tensor& x, const torch::Tensor& gate_up,

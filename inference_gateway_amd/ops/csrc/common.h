@@ -107,6 +107,17 @@ DEVINLINE float block_reduce_sum(float x, float* lds) {
   return lds[0];
 }
 
+// The gate of a gated activation, act(g): GATE 1 SiLU, 2 GELU by its tanh form
+// (0: the product has no activation), (1 + tanh(x)) / 2 being sigmoid(2 x).
+template <int GATE>
+DEVINLINE float gate_act(float g) {
+  if constexpr (GATE == 2)
+    return g / (1.0f + __expf(-1.5957691216057308f *
+                              (g + 0.044715f * g * g * g)));
+  else
+    return g / (1.0f + __expf(-g));
+}
+
 // Lines of memory to operands of the 16x16x32 matrix instructions.
 //
 // A load takes whole 128-byte lines, eight lanes a line; a matrix operand wants

@@ -1,7 +1,7 @@
-// Host side of ops.linear, ops.linear_silu_mul, ops.moe_few and ops.moe_rows:
-// which calls the kernels for a few rows of x (gemv.hip), for tens of them
-// (rows_gemm and held_gemm in rows_gemm.hip) and for hundreds and thousands of
-// them (wide_gemm.hip) take.
+// Host side of ops.linear, ops.linear_silu_mul, ops.linear_gated_act, ops.moe_few
+// and ops.moe_rows: which calls the kernels for a few rows of x (gemv.hip), for
+// tens of them (rows_gemm and held_gemm in rows_gemm.hip) and for hundreds and
+// thousands of them (wide_gemm.hip) take.
 //
 // What they are handed is a pointer, so the tensors have to be what they seem:
 // plain dense bf16 on one GPU, in a call that nothing but the product has to
@@ -26,12 +26,12 @@ void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               bool swiglu, int64_t tile);
+               int64_t gate, int64_t tile);
 bool moe_few_fits(int64_t T, int64_t top_k, int64_t D, int64_t F);
 void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-          c10::optional<torch::Tensor> bias, bool swiglu);
+          c10::optional<torch::Tensor> bias, int64_t gate);
 void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias, bool swiglu);
+               c10::optional<torch::Tensor> bias, int64_t gate);
 
 static bool call_is_plain() {
   using K = c10::DispatchKey;
@@ -88,22 +88,24 @@ int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
   return S > 0 && rows_gemm_ahead(M, S, K, swiglu) ? 2 : 0;
 }
 
-// The product, or nothing when none of the kernels takes it.
+// The product, or nothing when none of the kernels takes it.  gate: 0 none, else W
+// = [gate; up] and the result is SiLU(gate) * up (1) or GELU(gate) * up (2).
 c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
                                       const torch::Tensor& w,
                                       const c10::optional<torch::Tensor>& bias,
-                                      bool swiglu) {
+                                      int64_t gate) {
+  const bool swiglu = gate != 0;
   const int64_t which = few_rows_takes(x, w, bias, swiglu, false);
   if (which == 0) return c10::nullopt;
   auto out = torch::empty({x.size(0), swiglu ? w.size(0) / 2 : w.size(0)},
                           x.options());
   if (which == 3)
-    wide_gemm(out, x, w, swiglu,
+    wide_gemm(out, x, w, gate,
               wide_gemm_tile(x.size(0), out.size(1), x.size(1), swiglu));
   else if (which == 4)
     held_gemm(out, x, w, bias);
   else
-    (which == 1 ? gemv : rows_gemm)(out, x, w, bias, swiglu);
+    (which == 1 ? gemv : rows_gemm)(out, x, w, bias, gate);
   return out;
 }
 

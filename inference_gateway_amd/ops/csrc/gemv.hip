@@ -10,9 +10,9 @@
 // them share a compute unit and keep 128 KB in flight, well past HBM latency
 // times bandwidth, with more x one keeps half of that.
 //
-// SWIGLU: the rows of a wave are the same rows of the gate and of the up half
-// of W; the result is silu(gate) * up of the fp32 sums, one rounding where the
-// separate activation has two.
+// GATE: the rows of a wave are the same rows of the gate and of the up half of W;
+// the result is act(gate) * up of the fp32 sums, one rounding where the separate
+// activation has two.
 //
 // Measured, library and here (us; W cold, one row of x unless said): 6144 x
 // 4096 14.2 and 10.7, 4096 x 4096 14.9 and 8.0, 28672 x 4096 with SwiGLU 69.1
@@ -130,13 +130,14 @@ DEVINLINE void gemv_stage(uint16_t* xs, int total, int K, Row row) {
   __syncthreads();
 }
 
-template <int M, int R, bool SWIGLU, bool TAIL, int U>
+template <int M, int R, int GATE, bool TAIL, int U>
 __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
     uint16_t* __restrict__ out, const uint16_t* __restrict__ x,
     const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
     int rows, int N, int K, int64_t x_rs) {
   extern __shared__ __attribute__((aligned(16))) uint16_t xs[];   // [M][K]
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr bool SWIGLU = GATE != 0;
   constexpr int STEP = SWIGLU ? R / 2 : R;
   gemv_walk<M, R, SWIGLU, TAIL, U>(
       xs, w, N, K, blockIdx.x * GV_WAVES + wave, (N + STEP - 1) / STEP,
@@ -150,7 +151,7 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
         for (int m = 0; m < M; ++m) {
           if (m >= rows) break;
           float y = a[m];
-          if (SWIGLU) y = y / (1.0f + __expf(-y)) * up[m];
+          if (SWIGLU) y = gate_act<GATE>(y) * up[m];
           else if (bias) y += bf16_to_f32(bias[n]);
           out[(int64_t)m * N + n] = f32_to_bf16(y);
         }
@@ -249,7 +250,7 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void expert_gemv_kernel(
                 const int64_t a = list[at + m];
                 if (SWIGLU)
                   out[a * N + n] =
-                      f32_to_bf16(y[m] / (1.0f + __expf(-y[m])) * up[m]);
+                      f32_to_bf16(gate_act<1>(y[m]) * up[m]);
                 else
                   sums[a * N + n] = weight[a] * y[m];
               }
@@ -418,7 +419,9 @@ static bool gemv_deep(int64_t M, int64_t K) {
 // out [M, N] = x [M, K] W^T (+ bias [N]); swiglu: W [2 N, K], out = silu(x
 // Wg^T) * (x Wu^T).  Rows of x and W 16-byte aligned.
 void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-          c10::optional<torch::Tensor> bias, bool swiglu) {
+          c10::optional<torch::Tensor> bias, int64_t gate) {
+  const bool swiglu = gate != 0;
+  TORCH_CHECK(gate >= 0 && gate <= 2);
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 &&
               x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
               w.dim() == 2 && w.is_contiguous() && out.is_contiguous() &&
@@ -445,12 +448,13 @@ void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   const int64_t step = swiglu ? GV_ROWS / 2 : GV_ROWS;
   const int64_t need = ((N + step - 1) / step + GV_WAVES - 1) / GV_WAVES;
   const dim3 grid(std::min<int64_t>(need, 512));
+#define GV_KERNEL(MV, TAIL, U)                                                \
+  (gate == 2   ? gemv_kernel<MV, GV_ROWS, 2, TAIL, U>                         \
+   : gate == 1 ? gemv_kernel<MV, GV_ROWS, 1, TAIL, U>                         \
+               : gemv_kernel<MV, GV_ROWS, 0, TAIL, U>)
 #define LAUNCH_GV(MV, U)                                                      \
   do {                                                                        \
-    auto kern = K % 512 ? (swiglu ? gemv_kernel<MV, GV_ROWS, true, true, U>   \
-                                  : gemv_kernel<MV, GV_ROWS, false, true, U>) \
-                        : (swiglu ? gemv_kernel<MV, GV_ROWS, true, false, U>  \
-                                  : gemv_kernel<MV, GV_ROWS, false, false, U>); \
+    auto kern = K % 512 ? GV_KERNEL(MV, true, U) : GV_KERNEL(MV, false, U);   \
     if (shmem > 64 * 1024)                                                    \
       TORCH_CHECK(hipFuncSetAttribute(                                        \
                       (const void*)kern,                                      \
@@ -481,6 +485,7 @@ void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     default: LAUNCH_GV(8, 4); break;
   }
 #undef LAUNCH_GV
+#undef GV_KERNEL
   HIP_CHECK_KERNEL();
 }
 

@@ -25,8 +25,8 @@
 // loads are as good (28672 x 4096 as SwiGLU 47.0 and 47.3 us, 43 rows 44.3 and 42.3;
 // 128256 x 4096, 61 rows, 194 and 199).
 //
-// SWIGLU: a wave's 16 rows are eight gate rows and the up rows of the same
-// outputs, and the result is silu(gate) * up of the fp32 sums.
+// GATE: a wave's 16 rows are eight gate rows and the up rows of the same outputs,
+// and the result is act(gate) * up of the fp32 sums.
 //
 // Measured, here and with operands loaded as the matrix unit wants them (us, W
 // cold; 16 / 32 / 43 / 64 rows): 28672 x 4096 as SwiGLU 42.2 43.0 43.8 45.7 (5.1
@@ -61,7 +61,7 @@ struct RowsArgs {
   int64_t x_rs;
 };
 
-template <int MT, bool SWIGLU>
+template <int MT, int GATE>
 __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
     RowsArgs a) {
   __shared__ __attribute__((aligned(1024))) uint16_t xs[3][MT * 16 * RG_BK];
@@ -73,10 +73,11 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
   const int s0 = slices * blockIdx.y / gridDim.y;
   const int last = slices * (blockIdx.y + 1) / gridDim.y - 1;
   const int rot = (blockIdx.x + (blockIdx.x >> 3)) % (last + 1 - s0);
+  constexpr bool SWIGLU = GATE != 0;
   constexpr int COLS = SWIGLU ? 8 : 16;    // outputs of a wave
   const int n0 = (blockIdx.x * RG_WAVES + wave) * COLS;
 
-  // Matrix row r of a wave's tile is this row of W; with SWIGLU four of them
+  // Matrix row r of a wave's tile is this row of W; with a gate four of them
   // are two gate rows and the up rows of the same two outputs.
   auto w_row = [&](int r) {
     return a.w + (int64_t)(SWIGLU ? min(n0 + (r >> 2) * 2 + (r & 1), a.N - 1) +
@@ -185,8 +186,8 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
     if (SWIGLU) {
       const int n = n0 + quad * 2;
       if (n >= a.N) continue;
-      const uint32_t lo = f32_to_bf16(y[0] / (1.0f + __expf(-y[0])) * y[2]);
-      const uint32_t hi = f32_to_bf16(y[1] / (1.0f + __expf(-y[1])) * y[3]);
+      const uint32_t lo = f32_to_bf16(gate_act<GATE>(y[0]) * y[2]);
+      const uint32_t hi = f32_to_bf16(gate_act<GATE>(y[1]) * y[3]);
       *reinterpret_cast<uint32_t*>(a.out + (int64_t)row * a.N + n) =
           lo | hi << 16;
     } else {
@@ -429,7 +430,9 @@ bool rows_gemm_ahead(int64_t M, int64_t S, int64_t K, bool swiglu) {
 }
 
 void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias, bool swiglu) {
+               c10::optional<torch::Tensor> bias, int64_t gate) {
+  const bool swiglu = gate != 0;
+  TORCH_CHECK(gate >= 0 && gate <= 2);
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 &&
               x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
               w.dim() == 2 && w.is_contiguous() && out.is_contiguous() &&
@@ -466,10 +469,12 @@ void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                      0, stream, a)
 #define LAUNCH_RG_M(MT)                                                      \
   do {                                                                       \
-    if (swiglu) LAUNCH_RG(MT, true);                                         \
-    else LAUNCH_RG(MT, false);                                               \
+    if (gate == 2) LAUNCH_RG(MT, 2);                                         \
+    else if (gate == 1) LAUNCH_RG(MT, 1);                                    \
+    else LAUNCH_RG(MT, 0);                                                   \
   } while (0)
-  if (M <= 16) LAUNCH_RG(1, true);
+  if (M <= 16 && gate == 2) LAUNCH_RG(1, 2);   // with a gate only
+  else if (M <= 16) LAUNCH_RG(1, 1);
   else if (M <= 32) LAUNCH_RG_M(2);
   else if (M <= 48) LAUNCH_RG_M(3);
   else LAUNCH_RG_M(4);

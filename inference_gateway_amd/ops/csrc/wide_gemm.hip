@@ -1,6 +1,6 @@
 // y = x W^T for hundreds to thousands of rows of x, gfx950, bf16, products and
-// sums in fp32 (16x16x32 matrix instructions); with SWIGLU W = [gate; up] and
-// the result is silu(gate) * up of the fp32 sums.
+// sums in fp32 (16x16x32 matrix instructions); with a GATE W = [gate; up] and the
+// result is act(gate) * up of the fp32 sums.
 //
 // Bound by the matrix cores and, with them, by the card's power: the busier they
 // are the lower the clock (1.8 GHz at 74 % busy, 1.5 at 86).  So what counts is
@@ -23,7 +23,8 @@
 // 176, 8192 rows 1524 and 1384 (1.39 PFLOP/s), 16000 rows 2869 and 2649; between the
 // other kernels of a step 193, 1443 and 2710.  On a cooler card 197 and 170, 1377 and
 // 1319 (1.46 PFLOP/s), 2804 and 2590; there, with no stores 1242, with every step
-// from the caches 1256 at 8192 rows.
+// from the caches 1256 at 8192 rows.  With GELU, 5790 rows of 28672 x 4096 in a step
+// 1154 (library and gated_act) and 1048.
 #include <ATen/cuda/CUDAContext.h>
 #include <c10/cuda/CUDAGuard.h>
 #include <torch/extension.h>
@@ -88,8 +89,9 @@ DEVINLINE void wg_dma(wg_u32x4 buf, int lane_off, int off, uint32_t at) {
 // MT, NT: 16-row tiles of x and of W of one of the 2 x 2 waves.
 // GROUPED: rows start[e] .. start[e + 1] - 1 of x with the e-th of E <= 64
 // stacked W, known on the device only; an expert's tiles follow each other.
-template <int MT, int NT, bool SWIGLU, bool GROUPED>
+template <int MT, int NT, int GATE, bool GROUPED>
 __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
+  constexpr bool SWIGLU = GATE != 0;
   constexpr int XB = 32 * MT * WG_BK, WB = 32 * NT * WG_BK;  // of a K step
   constexpr int TM = 32 * MT, TN = SWIGLU ? 16 * NT : 32 * NT;
   __shared__ __attribute__((aligned(1024))) uint16_t lds[2 * XB + 3 * WB];
@@ -304,8 +306,7 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
       uint16_t* out = oc + (int64_t)row * a.N;
       if (SWIGLU) {
         auto act = [&](int t, int e) WG_INLINE {
-          const float g = acc[m][t][e];
-          return g / (1.0f + __expf(-g)) * acc[m][t][e + 2];
+          return gate_act<GATE>(acc[m][t][e]) * acc[m][t][e + 2];
         };
         auto pair = [&](int t) WG_INLINE {
           return wg_pack(act(t, 0), act(t, 1));
@@ -413,7 +414,9 @@ bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu) {
 }
 
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               bool swiglu, int64_t tile) {
+               int64_t gate, int64_t tile) {
+  const bool swiglu = gate != 0;
+  TORCH_CHECK(gate >= 0 && gate <= 2);
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 &&
               x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
               w.dim() == 2 && w.is_contiguous() && out.dim() == 2 &&
@@ -433,14 +436,14 @@ void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   const WideArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)x.data_ptr(),
                    (const uint16_t*)w.data_ptr(), (int)M, (int)N, (int)K,
                    x.stride(0), nullptr, 0};
+#define LAUNCH_WIDE_AS(...)                                                   \
+  hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__, false>), dim3(WG_BLOCKS), \
+                     dim3(256), 0, stream, a)
 #define LAUNCH_WIDE(MT, NT)                                                   \
   case MT * 16 + NT:                                                          \
-    if (swiglu)                                                               \
-      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, true, false>),             \
-                         dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
-    else                                                                      \
-      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, false, false>),            \
-                         dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
+    if (gate == 2) LAUNCH_WIDE_AS(MT, NT, 2);                                 \
+    else if (gate == 1) LAUNCH_WIDE_AS(MT, NT, 1);                            \
+    else LAUNCH_WIDE_AS(MT, NT, 0);                                           \
     break
   switch (tile) {
     LAUNCH_WIDE(8, 8);
@@ -451,6 +454,7 @@ void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     default: TORCH_CHECK(false, "no such tile: ", tile);
   }
 #undef LAUNCH_WIDE
+#undef LAUNCH_WIDE_AS
   HIP_CHECK_KERNEL();
 }
 
@@ -514,10 +518,10 @@ void grouped_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 #define LAUNCH_GROUPED(MT, NT)                                                \
   case MT * 16 + NT:                                                          \
     if (swiglu)                                                               \
-      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, true, true>),              \
+      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, 1, true>),              \
                          dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
     else                                                                      \
-      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, false, true>),             \
+      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, 0, true>),             \
                          dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
     break
   switch (tile > 0 ? tile : grouped_tile(R, E, N, swiglu)) {
