@@ -78,6 +78,12 @@ class LlamaAttention(nn.Module):
     def forward(self, x: torch.Tensor, fb: ForwardBatch,
                 kv_cache: Tuple[torch.Tensor, torch.Tensor],
                 cos_sin: torch.Tensor) -> torch.Tensor:
+        return self.o_proj(self.heads(x, fb, kv_cache, cos_sin))
+
+    def heads(self, x: torch.Tensor, fb: ForwardBatch,
+              kv_cache: Tuple[torch.Tensor, torch.Tensor],
+              cos_sin: torch.Tensor) -> torch.Tensor:
+        """What o_proj is applied to, [T, heads * head_dim]."""
         T = x.shape[0]
         qkv = ops.linear(x, self.qkv, self.qkv_b)
         # strided views into the fused QKV output — the HIP kernels take a
@@ -116,7 +122,7 @@ class LlamaAttention(nn.Module):
             o = ops.paged_attn_decode(
                 q.view(T, self.nq, self.hd), kc, vc, fb.block_table,
                 fb.ctx_lens, self.scale)
-        return self.o_proj(o.view(T, self.nq * self.hd))
+        return o.view(T, self.nq * self.hd)
 
 
 class LlamaMLP(nn.Module):
@@ -154,18 +160,15 @@ class LlamaLayer(nn.Module):
         self.mlp = LlamaMLP(cfg, layer, device, dtype)
         self.eps = cfg.norm_eps
 
-    def forward(self, x, residual, fb, kv_cache, cos_sin):
-        if residual is None:
-            residual = x.clone()
-            x = ops.rmsnorm(x, self.input_norm_w, self.eps)
-        else:
-            x, residual = ops.fused_add_rmsnorm(
-                x, residual, self.input_norm_w, self.eps)
-        x = self.attn(x, fb, kv_cache, cos_sin)
-        x, residual = ops.fused_add_rmsnorm(x, residual, self.post_norm_w,
-                                            self.eps)
-        x = self.mlp(x)
-        return x, residual
+    def forward(self, x, residual, fb, kv_cache, cos_sin, next_norm_w):
+        """x: the residual normed for this layer; returns it normed for what
+        follows, by next_norm_w, and the residual."""
+        x, residual = self.attn.o_proj.add_rmsnorm(
+            self.attn.heads(x, fb, kv_cache, cos_sin), residual,
+            self.post_norm_w, self.eps)
+        return self.mlp.down_proj.add_rmsnorm(
+            ops.linear_silu_mul(x, self.mlp.gate_up), residual, next_norm_w,
+            self.eps)
 
 
 class LlamaForCausalLM(nn.Module):
@@ -195,12 +198,12 @@ class LlamaForCausalLM(nn.Module):
     def forward(self, fb: ForwardBatch,
                 kv_caches: List[Tuple[torch.Tensor, torch.Tensor]]
                 ) -> torch.Tensor:
-        x = F.embedding(fb.token_ids, self.embed)
-        residual = None
+        residual = F.embedding(fb.token_ids, self.embed)
+        norms = [l.input_norm_w for l in self.layers] + [self.final_norm_w]
+        x = ops.rmsnorm(residual, norms[0], self.cfg.norm_eps)
         for i, layer in enumerate(self.layers):
-            x, residual = layer(x, residual, fb, kv_caches[i], self.cos_sin)
-        x, _ = ops.fused_add_rmsnorm(x, residual, self.final_norm_w,
-                                     self.cfg.norm_eps)
+            x, residual = layer(x, residual, fb, kv_caches[i], self.cos_sin,
+                                norms[i + 1])
         return x
 
     def compute_logits(self, hidden_last: torch.Tensor) -> torch.Tensor:

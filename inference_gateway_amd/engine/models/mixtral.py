@@ -367,14 +367,14 @@ class MixtralLayer(nn.Module):
 
     def forward(self, x, residual, fb, kv_cache, cos_sin):
         if residual is None:
-            residual = x.clone()
+            residual = x
             x = ops.rmsnorm(x, self.input_norm_w, self.eps)
         else:
             x, residual = ops.fused_add_rmsnorm(
                 x, residual, self.input_norm_w, self.eps)
-        x = self.attn(x, fb, kv_cache, cos_sin)
-        x, residual = ops.fused_add_rmsnorm(x, residual, self.post_norm_w,
-                                            self.eps)
+        x, residual = self.attn.o_proj.add_rmsnorm(
+            self.attn.heads(x, fb, kv_cache, cos_sin), residual,
+            self.post_norm_w, self.eps)
         x = self.moe(x, is_prefill=fb.is_prefill)
         return x, residual
 

@@ -249,10 +249,25 @@ def _own_product(x, w, bias, gate: int):
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     """x W^T (+ bias).  A few rows of bf16 run the weight-streaming kernels,
-    hundreds of them over a vocabulary's width the tiled one, everything else
-    the library's product."""
+    hundreds of them the tiled one over a vocabulary's width and, with K in parts,
+    where their tiles alone would leave the chip idle; everything else the
+    library's product."""
     out = _own_product(x, w, bias, 0)
     return torch.nn.functional.linear(x, w, bias) if out is None else out
+
+
+def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor,
+                       residual: torch.Tensor, weight: torch.Tensor,
+                       eps: float):
+    """fused_add_rmsnorm of x W^T: residual += x W^T in place; returns
+    (rmsnorm(residual) * weight, residual).  Where the product's K is in parts
+    (ops/csrc/few_rows.hip) the norm's kernel adds them."""
+    if (x.is_cuda and HAS_KERNELS and not torch.compiler.is_compiling()
+            and not has_torch_function_variadic(x, w, residual, weight)):
+        out = _kernels.linear_add_rmsnorm(x, w, residual, weight, eps)
+        if out is not None:
+            return out, residual
+    return fused_add_rmsnorm(linear(x, w), residual, weight, eps)
 
 
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:

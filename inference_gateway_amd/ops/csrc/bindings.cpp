@@ -41,6 +41,21 @@ void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                int64_t gate, int64_t tile);
+int64_t wide_split(int64_t M, int64_t N, int64_t K);
+torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
+                          int64_t tile, int64_t S);
+void sum_parts(torch::Tensor out, const torch::Tensor& part,
+               const c10::optional<torch::Tensor>& bias);
+void sum_add_rmsnorm(torch::Tensor out, torch::Tensor part,
+                     torch::Tensor residual, torch::Tensor weight, double eps);
+int64_t linear_norm_takes(const torch::Tensor& x, const torch::Tensor& w,
+                          const torch::Tensor& residual,
+                          const torch::Tensor& weight, bool anywhere);
+c10::optional<torch::Tensor> linear_add_rmsnorm(const torch::Tensor& x,
+                                                const torch::Tensor& w,
+                                                const torch::Tensor& residual,
+                                                const torch::Tensor& weight,
+                                                double eps);
 void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias);
 int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
@@ -118,12 +133,23 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("held_gemm", &igw::held_gemm,
         "x W^T of tens of rows, x in registers", py::arg("out"), py::arg("x"),
         py::arg("w"), py::arg("bias") = py::none());
+  m.def("wide_split", &igw::wide_split,
+        "256 x the tile + the parts of K of a product that leaves the chip idle");
+  m.def("split_parts", &igw::split_parts, "sums of the parts of K of x W^T");
+  m.def("sum_parts", &igw::sum_parts, "out = the parts' sum (+ bias)");
+  m.def("sum_add_rmsnorm", &igw::sum_add_rmsnorm,
+        "residual += the parts' sum, out = its norm");
+  m.def("linear_norm_takes", &igw::linear_norm_takes,
+        "as few_rows_takes, of a product in parts that a norm follows");
+  m.def("linear_add_rmsnorm", &igw::linear_add_rmsnorm,
+        "residual += x W^T and its norm, None: nothing done");
   m.def("wide_gemm", &igw::wide_gemm,
         "x W^T of hundreds to thousands of rows on a given tile");
   m.def("wide_gemm_tile", &igw::wide_gemm_tile,
         "its tile (16 MT + NT) for a product; 0: not ahead of the library");
   m.def("few_rows_takes", &igw::few_rows_takes,
-        "0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm, 4: held_gemm");
+        "0: none of them, 1: gemv, 2: rows_gemm, 3: wide_gemm, 4: held_gemm, "
+        "5: wide_gemm with K in parts");
   m.def("moe_few", &igw::moe_few, "SwiGLU experts of a few tokens");
   m.def("moe_rows_takes", &igw::moe_rows_takes,
         "whether the grouped products take a step");

@@ -21,12 +21,29 @@ bool gemv_ahead(int64_t M, int64_t N, int64_t K, bool swiglu);
 int64_t rows_gemm_splits(int64_t M, int64_t N, int64_t K, bool swiglu);
 bool rows_gemm_ahead(int64_t M, int64_t S, int64_t K, bool swiglu);
 bool held_gemm_takes(int64_t M, int64_t N, int64_t K);
+int64_t held_splits(int64_t M, int64_t N, int64_t K);
 void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias);
 int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                int64_t gate, int64_t tile);
+int64_t wide_split(int64_t M, int64_t N, int64_t K);
+bool wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm);
+torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
+                          int64_t tile, int64_t S);
+torch::Tensor rows_gemm_parts(const torch::Tensor& out, const torch::Tensor& x,
+                              const torch::Tensor& w,
+                              const c10::optional<torch::Tensor>& bias,
+                              int64_t gate);
+torch::Tensor held_gemm_parts(const torch::Tensor& out, const torch::Tensor& x,
+                              const torch::Tensor& w,
+                              const c10::optional<torch::Tensor>& bias);
+void sum_parts(torch::Tensor out, const torch::Tensor& part,
+               const c10::optional<torch::Tensor>& bias);
+bool sum_add_rmsnorm_fits(int64_t hidden);
+void sum_add_rmsnorm(torch::Tensor out, torch::Tensor part,
+                     torch::Tensor residual, torch::Tensor weight, double eps);
 bool moe_few_fits(int64_t T, int64_t top_k, int64_t D, int64_t F);
 void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
           c10::optional<torch::Tensor> bias, int64_t gate);
@@ -59,11 +76,11 @@ static bool by16(const torch::Tensor& t) {
 }
 
 // Which kernel takes the call.  0: none of them, 1: gemv, 2: rows_gemm, 3:
-// wide_gemm, 4: held_gemm.  `anywhere`: also off the GPU (the rule alone, nothing
-// is launched).
-int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
-                       const c10::optional<torch::Tensor>& bias, bool swiglu,
-                       bool anywhere) {
+// wide_gemm, 4: held_gemm, 5: wide_gemm with K in parts.  `anywhere`: also off the
+// GPU (the rule alone, nothing is launched).  norm: fused_add_rmsnorm follows.
+static int64_t which_takes(const torch::Tensor& x, const torch::Tensor& w,
+                           const c10::optional<torch::Tensor>& bias,
+                           bool swiglu, bool anywhere, bool norm) {
   if (!(anywhere || x.is_cuda()) || x.dim() != 2 || w.dim() != 2 ||
       !call_is_plain() || !plain_bf16(x, x.device()) ||
       !plain_bf16(w, x.device()))
@@ -77,15 +94,27 @@ int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
       !(!swiglu && plain_bf16(*bias, x.device()) && bias->dim() == 1 &&
         bias->size(0) == N && bias->is_contiguous()))
     return 0;
-  if (M > 64)
-    return !bias.has_value() && wide_gemm_tile(M, N, K, swiglu) > 0 &&
-                   wide_gemm_fits(x.stride(0), N, K, swiglu)
-               ? 3
-               : 0;
+  if (M > 64) {
+    if (!wide_gemm_fits(x.stride(0), N, K, swiglu)) return 0;
+    if (!bias.has_value() && wide_gemm_tile(M, N, K, swiglu) > 0) return 3;
+    return !swiglu && wide_split_ahead(M, N, K, norm) ? 5 : 0;
+  }
   if (gemv_fits(M, K, swiglu)) return gemv_ahead(M, w.size(0), K, swiglu);
   if (!swiglu && held_gemm_takes(M, N, K)) return 4;
   const int64_t S = rows_gemm_splits(M, N, K, swiglu);
   return S > 0 && rows_gemm_ahead(M, S, K, swiglu) ? 2 : 0;
+}
+
+int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
+                       const c10::optional<torch::Tensor>& bias, bool swiglu,
+                       bool anywhere) {
+  return which_takes(x, w, bias, swiglu, anywhere, false);
+}
+
+// The sums of the parts that wide_split cuts K into.
+static torch::Tensor wide_parts(const torch::Tensor& x, const torch::Tensor& w) {
+  const int64_t cut = wide_split(x.size(0), w.size(0), x.size(1));
+  return split_parts(x, w, cut >> 8, cut & 255);
 }
 
 // The product, or nothing when none of the kernels takes it.  gate: 0 none, else W
@@ -104,8 +133,48 @@ c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
               wide_gemm_tile(x.size(0), out.size(1), x.size(1), swiglu));
   else if (which == 4)
     held_gemm(out, x, w, bias);
+  else if (which == 5)
+    sum_parts(out, wide_parts(x, w), bias);
   else
     (which == 1 ? gemv : rows_gemm)(out, x, w, bias, gate);
+  return out;
+}
+
+// Which of the kernels takes a product that fused_add_rmsnorm follows, in parts
+// that the norm adds; 0: none.
+int64_t linear_norm_takes(const torch::Tensor& x, const torch::Tensor& w,
+                          const torch::Tensor& residual,
+                          const torch::Tensor& weight, bool anywhere) {
+  const int64_t which =
+      which_takes(x, w, c10::nullopt, false, anywhere, true);
+  if (which != 2 && which != 4 && which != 5) return 0;
+  const int64_t M = x.size(0), N = w.size(0);
+  if (!plain_bf16(residual, x.device()) || !plain_bf16(weight, x.device()) ||
+      residual.dim() != 2 || residual.size(0) != M || residual.size(1) != N ||
+      !residual.is_contiguous() || weight.dim() != 1 || weight.size(0) != N ||
+      !weight.is_contiguous() || !by16(residual) || !by16(weight) ||
+      !sum_add_rmsnorm_fits(N))
+    return 0;
+  if (which == 4 && held_splits(M, N, x.size(1)) < 2) return 0;
+  if (which == 2 && rows_gemm_splits(M, N, x.size(1), false) < 2) return 0;
+  return which;
+}
+
+// residual += x W^T in place and its norm, or nothing (and nothing done) when the
+// product does not come in parts.
+c10::optional<torch::Tensor> linear_add_rmsnorm(const torch::Tensor& x,
+                                                const torch::Tensor& w,
+                                                const torch::Tensor& residual,
+                                                const torch::Tensor& weight,
+                                                double eps) {
+  const int64_t which = linear_norm_takes(x, w, residual, weight, false);
+  if (which == 0) return c10::nullopt;
+  const torch::Tensor none;
+  const auto part = which == 5   ? wide_parts(x, w)
+                    : which == 4 ? held_gemm_parts(none, x, w, c10::nullopt)
+                                 : rows_gemm_parts(none, x, w, c10::nullopt, 0);
+  auto out = torch::empty_like(residual);
+  sum_add_rmsnorm(out, part, residual, weight, eps);
   return out;
 }
 

@@ -208,23 +208,38 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
   }
 }
 
-// sum of the splits' parts, with the bias
-__global__ __launch_bounds__(256) void rows_gemm_sum_kernel(RowsArgs a,
-                                                            int S) {
-  const int n = (blockIdx.x * 256 + threadIdx.x) * 4;
-  const int row = blockIdx.y;
-  if (n >= a.N) return;
-  const float* p = a.part + (int64_t)row * a.N + n;
-  const int64_t step = (int64_t)a.M * a.N;
+// sum of the parts of a split K, with the bias
+__global__ __launch_bounds__(256) void sum_parts_kernel(
+    uint16_t* __restrict__ out, const float* __restrict__ part,
+    const uint16_t* __restrict__ bias, int M, int N, int S) {
+  const int64_t step = (int64_t)M * N;
+  const int64_t at = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (at >= step) return;
   rg_f32x4 y = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
   for (int s = 0; s < S; ++s)
-    y += *reinterpret_cast<const rg_f32x4*>(p + s * step);
+    y += *reinterpret_cast<const rg_f32x4*>(part + s * step + at);
+  const int n = bias ? (int)(at % N) : 0;
   ushort4x o;
 #pragma unroll
   for (int e = 0; e < 4; ++e)
-    o.v[e] = f32_to_bf16(y[e] + (a.bias ? bf16_to_f32(a.bias[n + e]) : 0.0f));
-  *reinterpret_cast<ushort4x*>(a.out + (int64_t)row * a.N + n) = o;
+    o.v[e] = f32_to_bf16(y[e] + (bias ? bf16_to_f32(bias[n + e]) : 0.0f));
+  *reinterpret_cast<ushort4x*>(out + at) = o;
+}
+
+// out [M, N] = part [S, M, N] summed over S, plus the bias; N in fours
+void sum_parts(torch::Tensor out, const torch::Tensor& part,
+               const c10::optional<torch::Tensor>& bias) {
+  const int64_t S = part.size(0), M = part.size(1), N = part.size(2);
+  TORCH_CHECK(N % 4 == 0 && (M * N / 4 + 255) / 256 < (1LL << 31));
+  const at::cuda::CUDAGuard guard(part.device());
+  hipLaunchKernelGGL(sum_parts_kernel, dim3((M * N / 4 + 255) / 256), dim3(256),
+                     0, at::cuda::getCurrentCUDAStream(),
+                     (uint16_t*)out.data_ptr(), part.data_ptr<float>(),
+                     bias.has_value() ? (const uint16_t*)bias->data_ptr()
+                                      : nullptr,
+                     (int)M, (int)N, (int)S);
+  HIP_CHECK_KERNEL();
 }
 
 // The same product where the kernel above does not fill the chip: x stays in
@@ -429,21 +444,34 @@ bool rows_gemm_ahead(int64_t M, int64_t S, int64_t K, bool swiglu) {
   return (K >= 4096 && K % 2048 == 0) || (K >= 8192 && M <= 48);
 }
 
-void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias, int64_t gate) {
+// out [M, N] of a product, where it is written at once
+static void check_out(const torch::Tensor& out, const torch::Tensor& x,
+                      int64_t N) {
+  TORCH_CHECK(out.defined() && out.is_contiguous() && out.dim() == 2 &&
+              out.dtype() == x.dtype() && out.size(0) == x.size(0) &&
+              out.size(1) == N);
+  TORCH_CHECK(out.device() == x.device(), "tensors on different devices");
+}
+
+// Writes the product to out, or, where K is in parts, returns their sums [S, M, N]
+// (without the bias) and leaves out alone.
+torch::Tensor rows_gemm_parts(const torch::Tensor& out, const torch::Tensor& x,
+                              const torch::Tensor& w,
+                              const c10::optional<torch::Tensor>& bias,
+                              int64_t gate) {
   const bool swiglu = gate != 0;
   TORCH_CHECK(gate >= 0 && gate <= 2);
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 &&
               x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
-              w.dim() == 2 && w.is_contiguous() && out.is_contiguous() &&
-              out.dtype() == x.dtype());
-  const int64_t M = x.size(0), K = x.size(1), N = out.size(1);
+              w.dim() == 2 && w.is_contiguous());
+  const int64_t M = x.size(0), K = x.size(1);
+  const int64_t N = swiglu ? w.size(0) / 2 : w.size(0);
   const int64_t S = rows_gemm_splits(M, N, K, swiglu);
   TORCH_CHECK(S >= 1);
-  TORCH_CHECK(out.size(0) == M && w.size(1) == K &&
-              w.size(0) == (swiglu ? 2 * N : N) && x.stride(0) % 8 == 0);
-  TORCH_CHECK(w.device() == x.device() && out.device() == x.device(),
-              "tensors on different devices");
+  if (S == 1) check_out(out, x, N);
+  TORCH_CHECK(w.size(1) == K && w.size(0) == (swiglu ? 2 * N : N) &&
+              x.stride(0) % 8 == 0);
+  TORCH_CHECK(w.device() == x.device(), "tensors on different devices");
   TORCH_CHECK((reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0 &&
               (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15) == 0);
   if (bias.has_value())
@@ -457,7 +485,7 @@ void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   torch::Tensor part;
   if (S > 1)
     part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
-  RowsArgs a{(uint16_t*)out.data_ptr(),
+  RowsArgs a{S > 1 ? nullptr : (uint16_t*)out.data_ptr(),
              S > 1 ? part.data_ptr<float>() : nullptr,
              (const uint16_t*)x.data_ptr(),
              (const uint16_t*)w.data_ptr(),
@@ -481,16 +509,19 @@ void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 #undef LAUNCH_RG_M
 #undef LAUNCH_RG
   HIP_CHECK_KERNEL();
-  if (S > 1) {
-    hipLaunchKernelGGL(rows_gemm_sum_kernel, dim3((N / 4 + 255) / 256, M),
-                       dim3(256), 0, stream, a, (int)S);
-    HIP_CHECK_KERNEL();
-  }
+  return part;
+}
+
+void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> bias, int64_t gate) {
+  check_out(out, x, gate != 0 ? w.size(0) / 2 : w.size(0));
+  const auto part = rows_gemm_parts(out, x, w, bias, gate);
+  if (part.defined()) sum_parts(out, part, bias);
 }
 
 // In how many parts held_gemm cuts K (a wave's part is four to eight lines of
 // 64 entries); 0: it cannot.
-static int64_t held_splits(int64_t M, int64_t N, int64_t K) {
+int64_t held_splits(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || M > 64 || N < 1 || N % 4 != 0 || N > (1 << 26) ||
       K > (1 << 20))
     return 0;
@@ -535,19 +566,19 @@ bool held_gemm_takes(int64_t M, int64_t N, int64_t K) {
            rows_gemm_ahead(M, 1, K, false));
 }
 
-void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-               c10::optional<torch::Tensor> bias) {
+// The same with x in registers.
+torch::Tensor held_gemm_parts(const torch::Tensor& out, const torch::Tensor& x,
+                              const torch::Tensor& w,
+                              const c10::optional<torch::Tensor>& bias) {
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 &&
               x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
-              w.dim() == 2 && w.is_contiguous() && out.is_contiguous() &&
-              out.dtype() == x.dtype() && out.dim() == 2);
-  const int64_t M = x.size(0), K = x.size(1), N = out.size(1);
+              w.dim() == 2 && w.is_contiguous());
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
   const int64_t S = held_splits(M, N, K);
   TORCH_CHECK(S >= 1);
-  TORCH_CHECK(out.size(0) == M && w.size(1) == K && w.size(0) == N &&
-              x.stride(0) % 8 == 0);
-  TORCH_CHECK(w.device() == x.device() && out.device() == x.device(),
-              "tensors on different devices");
+  if (S == 1) check_out(out, x, N);
+  TORCH_CHECK(w.size(1) == K && x.stride(0) % 8 == 0);
+  TORCH_CHECK(w.device() == x.device(), "tensors on different devices");
   TORCH_CHECK((reinterpret_cast<uintptr_t>(x.data_ptr()) & 15) == 0 &&
               (reinterpret_cast<uintptr_t>(w.data_ptr()) & 15) == 0);
   if (bias.has_value())
@@ -558,7 +589,7 @@ void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   torch::Tensor part;
   if (S > 1)
     part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
-  RowsArgs a{(uint16_t*)out.data_ptr(),
+  RowsArgs a{S > 1 ? nullptr : (uint16_t*)out.data_ptr(),
              S > 1 ? part.data_ptr<float>() : nullptr,
              (const uint16_t*)x.data_ptr(),
              (const uint16_t*)w.data_ptr(),
@@ -586,11 +617,14 @@ void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 #undef LAUNCH_HELD
 #undef LAUNCH_HELD_AS
   HIP_CHECK_KERNEL();
-  if (S > 1) {
-    hipLaunchKernelGGL(rows_gemm_sum_kernel, dim3((N / 4 + 255) / 256, M),
-                       dim3(256), 0, stream, a, (int)S);
-    HIP_CHECK_KERNEL();
-  }
+  return part;
+}
+
+void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+               c10::optional<torch::Tensor> bias) {
+  check_out(out, x, w.size(0));
+  const auto part = held_gemm_parts(out, x, w, bias);
+  if (part.defined()) sum_parts(out, part, bias);
 }
 
 }  // namespace igw

@@ -52,6 +52,8 @@ struct WideArgs {
   int64_t x_rs;
   const int32_t* start;  // [E + 1]: first row of every expert (GROUPED)
   int E;
+  float* part;           // [S, M, N]: sums of the parts of K (SPLIT)
+  int S;
 };
 
 DEVINLINE uint32_t wg_pack(float a, float b) {
@@ -89,7 +91,9 @@ DEVINLINE void wg_dma(wg_u32x4 buf, int lane_off, int off, uint32_t at) {
 // MT, NT: 16-row tiles of x and of W of one of the 2 x 2 waves.
 // GROUPED: rows start[e] .. start[e + 1] - 1 of x with the e-th of E <= 64
 // stacked W, known on the device only; an expert's tiles follow each other.
-template <int MT, int NT, int GATE, bool GROUPED>
+// SPLIT: K in S parts of whole pairs of steps, as even as they go; a part of a tile
+// is an item like a tile and its sums go to `part`.
+template <int MT, int NT, int GATE, bool GROUPED, bool SPLIT = false>
 __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
   constexpr bool SWIGLU = GATE != 0;
   constexpr int XB = 32 * MT * WG_BK, WB = 32 * NT * WG_BK;  // of a K step
@@ -99,7 +103,8 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wr = wave >> 1, wc = wave & 1;
   const int r16 = lane & 15, quad = lane >> 4;
-  const int nt = (a.N + TN - 1) / TN, steps = a.K / WG_BK;
+  const int nt = (a.N + TN - 1) / TN;
+  int steps = a.K / WG_BK;
   // of this workgroup's tile: the matrix's first row in x and its row count; of
   // expert `lane`: its tiles, those up to it, its first row, its rows
   int base = 0, M = a.M, expert = 0;
@@ -117,8 +122,10 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
       if (lane >= d) upto += up;
     }
   }
+  const int whole = (a.M + TM - 1) / TM * nt;   // tiles of a part of K
   const int tiles = GROUPED ? __builtin_amdgcn_readlane(upto, 63)
-                            : (a.M + TM - 1) / TM * nt;
+                    : SPLIT ? whole * a.S
+                            : whole;
 
   // Tile of round r; -1: none.  A round's tiles are dealt to the XCDs in
   // stretches (ids go round-robin over the XCDs), and a stretch is a patch of
@@ -130,7 +137,17 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
     const int at = (blockIdx.x & 7) * per + slot;
     return slot < per && at < left ? r * WG_BLOCKS + at : -1;
   };
+  // the part of K of the tile that is loaded, its first entry and its steps
+  int part = 0, k0 = 0, own = 0;
   auto origin = [&](int tile, int* m0, int* n0) WG_INLINE {
+    if (SPLIT) {
+      part = tile / whole;
+      tile -= part * whole;
+      const int pairs = a.K / (2 * WG_BK);
+      const int from = pairs * part / a.S, to = pairs * (part + 1) / a.S;
+      k0 = from * 2 * WG_BK;
+      own = 2 * (to - from);
+    }
     if (GROUPED) {
       expert = __builtin_ctzll(__ballot(upto > tile));
       tile -= __builtin_amdgcn_readlane(upto - mine, expert);
@@ -152,16 +169,16 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
   wg_u32x4 xbuf, wbuf;
   int xo[MT], wo[NT];
   auto x_from = [&](int m0) WG_INLINE {
-    xbuf = wg_buffer(a.x + (base + m0) * a.x_rs,
-                     ((M - 1 - m0) * a.x_rs + a.K) * 2);
+    xbuf = wg_buffer(a.x + (base + m0) * a.x_rs + k0,
+                     ((M - 1 - m0) * a.x_rs + a.K - k0) * 2);
 #pragma unroll
     for (int i = 0; i < MT; ++i)
       xo[i] = min(i * 32 + prow, M - 1 - m0) * ((int)a.x_rs * 2) + pbyte;
   };
   auto w_from = [&](int n0) WG_INLINE {
     const int rows = SWIGLU ? 2 * a.N : a.N;
-    wbuf = wg_buffer(a.w + ((int64_t)expert * rows + n0) * a.K,
-                     (int64_t)(rows - n0) * a.K * 2);
+    wbuf = wg_buffer(a.w + ((int64_t)expert * rows + n0) * a.K + k0,
+                     ((int64_t)(rows - n0) * a.K - k0) * 2);
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const int r = i * 32 + prow, half = r >= 16 * NT, in = r - half * 16 * NT;
@@ -284,6 +301,8 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
     const int next = tile_of(++round);
     const int mc = m0, nc = n0, Mc = M;
     uint16_t* const oc = a.out + (int64_t)base * a.N;
+    float* const pc = SPLIT ? a.part + (int64_t)part * M * a.N : nullptr;
+    if (SPLIT) steps = own;
     origin(next < 0 ? tile : next, &m0, &n0);
     int k = 512;
     for (int t = 2; t < steps - 4; t += 2, k += 256) {
@@ -304,7 +323,16 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
     for (int m = 0; m < MT; ++m) {
       const int row = mc + (wr * MT + m) * 16 + r16;
       uint16_t* out = oc + (int64_t)row * a.N;
-      if (SWIGLU) {
+      if (SPLIT) {
+        static_assert(!SPLIT || (!SWIGLU && NT % 2 == 0));
+        float* sums = pc + (int64_t)row * a.N;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+          const int at = nc + wc * 16 * NT + t / 2 * 32 + quad * 8 + t % 2 * 4;
+          if (row < Mc && at < a.N)
+            *reinterpret_cast<wg_f32x4*>(sums + at) = acc[m][t];
+        }
+      } else if (SWIGLU) {
         auto act = [&](int t, int e) WG_INLINE {
           return gate_act<GATE>(acc[m][t][e]) * acc[m][t][e + 2];
         };
@@ -435,7 +463,7 @@ void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
   const WideArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)x.data_ptr(),
                    (const uint16_t*)w.data_ptr(), (int)M, (int)N, (int)K,
-                   x.stride(0), nullptr, 0};
+                   x.stride(0), nullptr, 0, nullptr, 1};
 #define LAUNCH_WIDE_AS(...)                                                   \
   hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__, false>), dim3(WG_BLOCKS), \
                      dim3(256), 0, stream, a)
@@ -456,6 +484,129 @@ void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 #undef LAUNCH_WIDE
 #undef LAUNCH_WIDE_AS
   HIP_CHECK_KERNEL();
+}
+
+// Products of rows that leave the chip idle, K in parts.
+//
+// Tiles of the kernel above with a part of K each, their fp32 sums to memory, and a
+// second kernel to add them (with the residual and the norm behind it where there is
+// one).  wide_split picks the tile and the parts by what they cost: rounds of 256
+// items at `step` us a K step of 64 and `start` to begin, against W from HBM, and
+// the sums' way to memory and back.  Of 768 measured pairs of a tile and parts the
+// model is off by 4 % on average, and its choice is 2 % behind the best.
+struct SplitTile {
+  int MT, NT;
+  double step;
+};
+static constexpr SplitTile split_tiles[] = {
+    {3, 4, 0.500}, {4, 4, 0.567}, {4, 6, 0.712}, {6, 4, 0.671}, {6, 6, 0.845},
+    {6, 8, 1.069}, {8, 4, 0.799}, {8, 6, 1.049}, {8, 8, 1.387}};
+
+// 256 times the tile (16 MT + NT) and the parts of K, at least two; 0: cannot be.
+int64_t wide_split(int64_t M, int64_t N, int64_t K) {
+  if (M < 65 || M > (1 << 16) || N < 8 || N % 8 != 0 || N > (1 << 20) ||
+      K % (2 * WG_BK) != 0 || K > (1 << 20))
+    return 0;
+  int64_t best = 0;
+  double least = 0.0;
+  const int64_t pairs = K / (2 * WG_BK);
+  for (const auto& c : split_tiles)
+    for (int64_t S = 2; S <= 16 && 3 * S <= pairs; ++S) {
+      const int64_t items = (M + 32 * c.MT - 1) / (32 * c.MT) *
+                            ((N + 32 * c.NT - 1) / (32 * c.NT)) * S;
+      const int64_t rounds = (items + WG_BLOCKS - 1) / WG_BLOCKS;
+      const double work =
+          rounds * (2 * ((pairs + S - 1) / S) * c.step + 0.11);
+      const double stream = N * K * 2e-6 / 4.6;
+      // about the longer of the two
+      const double a = work * work, b = stream * stream;
+      const double cost =
+          std::sqrt(std::sqrt(a * a + b * b)) + S * M * N * 4e-6 * 0.36;
+      if (best == 0 || cost < least) {
+        best = (c.MT * 16 + c.NT) * 256 + S;
+        least = cost;
+      }
+    }
+  return best;
+}
+
+// Whether that is ahead of the library; norm: where the norm that follows adds the
+// parts, of the library and fused_add_rmsnorm.  Measured at 19 sizes of W by 16 of
+// 65 to 2600 rows (us, library and here; then with the norm).  Over a long K the
+// library's tiles are few: 4096 x 14336, 65 / 128 / 256 / 512 / 1024 / 2033 rows 50.6
+// 76.5 63.8 90.9 134 204 and 36.1 38.9 49.3 65.7 108 185; 5120 x 17920, 65 / 256 / 1024
+// 148 222 249 and 45.8 65.1 158, but 2033 rows 291 and 320; 8192 x 28672, 512 / 640
+// rows 312 260 and 195 289.  Of squarer W the parts' way to memory weighs more: 4096 x
+// 4096, 128 / 256 / 512 / 1024 / 1600 rows 24.0 22.4 30.9 42.1 55.6 and 18.0 21.8 30.7
+// 43.4 66.9 (with the norm 27.2 25.9 36.0 48.9 65.4 and 19.1 23.1 32.6 46.1 70.2), 5120
+// x 5120, 256 / 640 / 1024 rows 50.8 51.3 62.7 and 30.7 47.5 60.7, 7680 x 5120, 128 /
+// 512 / 640 rows 34.9 52.1 58.0 and 28.0 51.0 63.6, 6144 x 4096, 128 / 160 / 200 rows
+// 26.5 29.1 26.5 and 23.8 26.1 30.0, 8192 x 8192, 65 / 128 rows 38.9 51.8 and 43.6
+// 46.6.  Small W and a short K pay for the second launch: 1024 x 4096, 128 rows, 10.3
+// and 11.9, 4096 x 2048 13.1 and 15.4, as do wide ones: 16384 x 4096 40.3 and 46.9.
+bool wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm) {
+  if (wide_split(M, N, K) == 0) return false;
+  const int64_t least = N > 7680 && K < 2 * N ? 128 : 65;
+  int64_t most;
+  if (norm) {
+    if (K < 3584 || N * K < (int64_t)12 << 20 || N > 16384) return false;
+    most = K >= 3 * N   ? N > 5120 ? 512 : N > 4096 ? 1600 : 2048
+           : K >= 2 * N ? N > 5120 ? 512 : 1600
+           : K >= N     ? N > 7680 ? 512 : 1024
+                        : 512;
+  } else {
+    if (K < 4096 || N * K < (int64_t)16 << 20 || N < 2048 || N > 10240)
+      return false;
+    most = K >= 3 * N   ? N > 5120 ? 512 : N > 4096 ? 1600 : 2048
+           : K >= 2 * N ? N > 5120 ? 512 : 1300
+           : K >= 5120  ? 512
+           : K >= N     ? 256
+                        : 160;
+  }
+  return M >= least && M <= most;
+}
+
+// The sums [S, M, N] of the parts that wide_split says.
+torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
+                          int64_t tile, int64_t S) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 &&
+              x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
+              w.dim() == 2 && w.is_contiguous());
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M >= 1 && N >= 8 && N % 8 == 0 && S >= 1 && S <= 64 &&
+              K / (2 * WG_BK) >= 3 * S && K % (2 * WG_BK) == 0 &&
+              M <= (1 << 20) && N <= (1 << 20) && K <= (1 << 20) &&
+              wide_gemm_fits(x.stride(0), N, K, false));
+  TORCH_CHECK(w.size(1) == K && x.stride(0) % 8 == 0);
+  TORCH_CHECK(w.device() == x.device(), "tensors on different devices");
+  for (const auto* t : {&x, &w})
+    TORCH_CHECK((reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) == 0);
+  const at::cuda::CUDAGuard guard(x.device());
+  hipStream_t stream = at::cuda::getCurrentCUDAStream();
+  auto part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
+  const WideArgs a{nullptr, (const uint16_t*)x.data_ptr(),
+                   (const uint16_t*)w.data_ptr(), (int)M, (int)N, (int)K,
+                   x.stride(0), nullptr, 0, part.data_ptr<float>(), (int)S};
+#define LAUNCH_SPLIT(MT, NT)                                                  \
+  case MT * 16 + NT:                                                          \
+    hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, 0, false, true>),            \
+                       dim3(WG_BLOCKS), dim3(256), 0, stream, a);             \
+    break
+  switch (tile) {
+    LAUNCH_SPLIT(3, 4);
+    LAUNCH_SPLIT(4, 4);
+    LAUNCH_SPLIT(4, 6);
+    LAUNCH_SPLIT(6, 4);
+    LAUNCH_SPLIT(6, 6);
+    LAUNCH_SPLIT(6, 8);
+    LAUNCH_SPLIT(8, 4);
+    LAUNCH_SPLIT(8, 6);
+    LAUNCH_SPLIT(8, 8);
+    default: TORCH_CHECK(false, "no such tile: ", tile);
+  }
+#undef LAUNCH_SPLIT
+  HIP_CHECK_KERNEL();
+  return part;
 }
 
 // Tiles of a grouped product and what a round of them costs (hundredths of one
@@ -514,7 +665,7 @@ void grouped_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
   const WideArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)x.data_ptr(),
                    (const uint16_t*)w.data_ptr(), (int)R, (int)N, (int)K, K,
-                   (const int32_t*)start.data_ptr(), (int)E};
+                   (const int32_t*)start.data_ptr(), (int)E, nullptr, 1};
 #define LAUNCH_GROUPED(MT, NT)                                                \
   case MT * 16 + NT:                                                          \
     if (swiglu)                                                               \

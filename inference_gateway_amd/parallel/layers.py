@@ -12,7 +12,8 @@ import torch
 import torch.nn as nn
 
 from .. import ops
-from .comm import row_parallel_matmul_allreduce, tp_all_reduce
+from .comm import (row_parallel_matmul_allreduce, tp_all_reduce,
+                   tp_world_size)
 
 
 def _init_weight(shape, device, dtype, seed: int) -> torch.Tensor:
@@ -61,6 +62,14 @@ class RowParallelLinear(nn.Module):
         # all-reduce (comm stream) with the next chunk's GEMM; decode
         # sizes go straight through (one-shot xGMI kernel when active)
         return row_parallel_matmul_allreduce(x, self.weight)
+
+    def add_rmsnorm(self, x: torch.Tensor, residual: torch.Tensor,
+                    norm_w: torch.Tensor, eps: float):
+        """residual += Y in place; returns its RMS norm and it."""
+        if tp_world_size() <= 1:
+            return ops.linear_add_rmsnorm(x, self.weight, residual, norm_w,
+                                          eps)
+        return ops.fused_add_rmsnorm(self(x), residual, norm_w, eps)
 
 
 class ReplicatedLinear(nn.Module):

@@ -307,6 +307,66 @@ def test_wide_gemm_lines(M, N, K, swiglu, tile):
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,linear,norm", [
+    # rows that a product in parts of K takes, alone and with a norm behind it
+    (64, 4096, 14336, 4, 4), (65, 4096, 14336, 5, 5), (2048, 4096, 14336, 5, 5),
+    (2049, 4096, 14336, 0, 0), (1600, 5120, 17920, 5, 5),
+    (1601, 5120, 17920, 0, 0), (513, 8192, 28672, 0, 0),
+    (256, 4096, 4096, 5, 5), (257, 4096, 4096, 0, 5), (1025, 4096, 4096, 0, 0),
+    (160, 6144, 4096, 5, 5), (161, 6144, 4096, 0, 5), (512, 7680, 5120, 5, 5),
+    (127, 8192, 8192, 0, 0), (128, 8192, 8192, 5, 5), (128, 1024, 4096, 0, 0),
+    (128, 4096, 2048, 0, 0), (128, 16384, 4096, 0, 5), (128, 12288, 4096, 0, 5),
+    (128, 4096, 4160, 0, 0), (128, 4100, 4096, 0, 0),
+    # in one part: nothing for the norm to add
+    (33, 4096, 4096, 4, 0), (5, 4096, 4096, 1, 0), (33, 28672, 4096, 2, 0)])
+def test_split_lines(M, N, K, linear, norm):
+    bf = torch.bfloat16
+    x, w = torch.empty(M, K, dtype=bf), torch.empty(N, K, dtype=bf)
+    r, nw = torch.empty(M, N, dtype=bf), torch.empty(N, dtype=bf)
+
+    def takes(x, w, r, nw):
+        return ops._kernels.linear_norm_takes(x, w, r, nw, True)
+
+    assert ops._kernels.few_rows_takes(x, w, None, False, True) == linear
+    assert ops._kernels.few_rows_takes(x, w, nw, False, True) == linear
+    assert takes(x, w, r, nw) == norm
+    for args in ((x, w, r.float(), nw), (x, w, r, nw.float()),
+                 (x, w, r[:, :8], nw), (x, w, r, nw[:8]), (x[:, 1:], w, r, nw),
+                 (x, w, torch.empty(N, M, dtype=bf).t(), nw),
+                 (x, w, torch.empty(M * N + 1, dtype=bf)[1:].view(M, N), nw),
+                 (x, w, r, torch.empty(N + 1, dtype=bf)[1:]),
+                 (x, w, r.to("meta"), nw), (x, w, r[None], nw),
+                 (x, w, r.clone().requires_grad_(), nw)):
+        assert takes(*args) == 0
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+def test_wide_split_parts():
+    """Every part of K has the three pairs of steps that the kernel needs."""
+    tiles = set()
+    for N in (8, 1024, 4096, 5120, 6144, 16384):
+        for K in (768, 896, 2048, 4096, 5120, 14336, 17920):
+            for M in (65, 96, 97, 200, 256, 700, 1024, 2033, 5000):
+                cut = ops._kernels.wide_split(M, N, K)
+                tiles.add(cut >> 8)
+                assert 2 <= cut & 255 and K // 128 // (cut & 255) >= 3
+    assert tiles <= {16 * m + n for m, n in (
+        (3, 4), (4, 4), (4, 6), (6, 4), (6, 6), (6, 8), (8, 4), (8, 6), (8, 8))}
+    for M, N, K in ((64, 4096, 4096), (65, 4096, 640), (65, 4100, 4096),
+                    (65, 4096, 4160), (65, 4, 4096)):
+        assert ops._kernels.wide_split(M, N, K) == 0
+
+
+def test_linear_add_rmsnorm_is_its_parts():
+    g = torch.Generator().manual_seed(0)
+    x, w = torch.randn(5, 24, generator=g), torch.randn(16, 24, generator=g)
+    r, nw = torch.randn(5, 16, generator=g), torch.randn(16, generator=g)
+    want, res = ops.fused_add_rmsnorm(ops.linear(x, w), r.clone(), nw, 1e-5)
+    got, same = ops.linear_add_rmsnorm(x, w, r, nw, 1e-5)
+    assert same is r and torch.equal(got, want) and torch.equal(r, res)
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 def test_wide_gemm_takes_plain_calls_only():
     bf = torch.bfloat16
     x, w = torch.empty(300, 520, dtype=bf), torch.empty(65536, 512, dtype=bf)
