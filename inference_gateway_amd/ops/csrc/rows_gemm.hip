@@ -40,6 +40,8 @@
 #include <c10/cuda/CUDAGuard.h>
 #include <torch/extension.h>
 
+#include <type_traits>
+
 #include "common.h"
 
 namespace igw {
@@ -251,8 +253,8 @@ void sum_parts(torch::Tensor out, const torch::Tensor& part,
 // unit of work is 128 KB of W, often in one piece, instead of 1 MB; nothing
 // but the waves' sums goes through LDS, once a unit, and a wave refills the
 // registers of a line of W for the next unit when it has turned it.  More than
-// 32 rows are two halves, in workgroups of the same XCD at the same time: the
-// second finds W in L2.
+// 32 rows are two halves, in workgroups of the same XCD at the same time (the second
+// finds W in L2), or ring_gemm's below.
 //
 // Bound by W's bytes, and by the start for small ones (x to registers, 256 KB a
 // workgroup, and the first lines: about 4 us).  Measured, library and here (us, W
@@ -399,6 +401,159 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void held_gemm_kernel(
   finish(unit);
 }
 
+// The same for 33 to 64 rows and a K in parts: three or four tiles of rows of x in
+// registers, which leaves none for W, whose lines wait in LDS.
+//
+// A wave has a ring of R lines (16 rows of W, 128 bytes each) that fill all of the
+// 160 KB that the waves' sums leave; a line goes from memory straight to its place,
+// its 16-byte pieces permuted as LineTurn has them, and its place is sent for again
+// as soon as it is read.  So W is streamed once, where two halves of x, in workgroups
+// of their own, stream it at 4.5 TB/s.  Measured, two halves and here, with the sum of
+// the parts (us, 43 and 61 rows): 4096 x 14336 30.8 32.2 and 27.4 30.9, 5120 x 17920
+// 48.7 50.1 and 40.4 42.4, 5120 x 5120 18.5 19.2 and 17.6 18.5.  In one part, where W
+// is short and x is most of what is loaded, it is behind (4096 x 4096 12.0 and 12.7);
+// with up to 32 rows, where x leaves registers for W, too (4096 x 14336, 16 rows, 23.3
+// and 25.4).
+DEVINLINE rg_u32x4 rg_buffer(const uint16_t* p, int64_t bytes) {
+  const uint64_t b = (uint64_t)p;
+  const int n = bytes > 0x7fffffff ? 0x7fffffff : (int)bytes;
+  return rg_u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)b),
+                  (uint32_t)__builtin_amdgcn_readfirstlane((int)(b >> 32)) &
+                      0xffffu,
+                  (uint32_t)__builtin_amdgcn_readfirstlane(n), 0x00020000u};
+}
+
+// 64 lanes x 16 bytes from memory straight to LDS, 1024 bytes from `at` on.
+DEVINLINE void rg_dma(rg_u32x4 buf, int lane_off, int off, uint32_t at) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+      "buffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(at),
+      "v"(lane_off), "s"(buf), "s"(off)
+      : "memory", "m0");
+}
+
+template <int P, int MT>
+__global__ __launch_bounds__(64 * RG_WAVES, 2) void ring_gemm_kernel(
+    RowsArgs a, int S) {
+  constexpr int R = 10 - MT;
+  __shared__ __attribute__((aligned(1024))) rg_u32x4 ring[RG_WAVES][R][128];
+  __shared__ __attribute__((aligned(16)))
+  rg_f32x4 sums[2][RG_WAVES][MT][WAVE_SIZE];
+  static_assert(sizeof(ring) + sizeof(sums) == 160 * 1024);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int r16 = lane & 15, quad = lane >> 4, r8 = lane >> 3;
+  const int split = blockIdx.x % S, step = gridDim.x / S;
+  const int units = (a.N + 15) >> 4;
+  int unit = blockIdx.x / S;
+  if (unit >= step || unit >= units) return;
+
+  const int k0 = (split * RG_WAVES + wave) * P * 64;
+  const int rot = ((blockIdx.x >> 3) + wave) % P;
+  auto line = [&](int j) __attribute__((always_inline)) {   // entries from k0 on
+    return (j + rot >= P ? j + rot - P : j + rot) * 64;
+  };
+  // x in whole lines, all of it on its way before the first of W
+  rg_u32x4 xf[P][2][MT];
+#pragma unroll
+  for (int j = 0; j < P; ++j)
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        xf[j][h][m] = *reinterpret_cast<const rg_u32x4*>(
+            a.x + min(m * 16 + h * 8 + r8, a.M - 1) * a.x_rs + k0 + line(j) +
+            (lane & 7) * 8);
+  asm volatile("" ::: "memory");
+
+  const int w0 = r8 * (a.K * 2) + ((lane & 7) ^ LineTurn::perm(r8)) * 16;
+  const int w1 = (8 + r8) * (a.K * 2) + ((lane & 7) ^ LineTurn::perm(8 + r8)) * 16;
+  const uint32_t lds0 =
+      (uint32_t)(uintptr_t)(__attribute__((address_space(3))) rg_u32x4*)
+          ring[wave];
+  rg_u32x4 wbuf;
+  int ahead = unit, jahead = 0, slot = 0;   // the line that is sent for next
+  auto w_from = [&](int u) __attribute__((always_inline)) {
+    // rows past N are zeros; past the last unit nothing is read
+    const int n0 = min(u, units - 1) * 16;
+    wbuf = rg_buffer(a.w + (int64_t)n0 * a.K + k0,
+                     u < units ? ((int64_t)(a.N - n0) * a.K - k0) * 2 : 0);
+  };
+  auto send = [&]() __attribute__((always_inline)) {
+    const int off = line(jahead) * 2;
+    rg_dma(wbuf, w0, off, lds0 + slot * 2048);
+    rg_dma(wbuf, w1, off, lds0 + slot * 2048 + 1024);
+    slot = slot + 1 == R ? 0 : slot + 1;
+    if (++jahead == P) {
+      jahead = 0;
+      ahead += step;
+      w_from(ahead);
+    }
+  };
+  w_from(unit);
+#pragma unroll
+  for (int i = 0; i < R; ++i) send();
+  // x becomes operands in the memory of the sums
+  const LineTurn turn_lines(lane);
+  rg_u32x4* const scratch =
+      reinterpret_cast<rg_u32x4*>(&sums[0][0][0][0]) + wave * 128;
+#pragma unroll
+  for (int j = 0; j < P; ++j)
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      turn_lines(scratch, xf[j][0][m], xf[j][1][m], xf[j][0][m], xf[j][1][m]);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+
+  int used = 0, turns = 0;    // the ring's next line; units done
+  for (; unit < units; unit += step, ++turns) {
+    rg_f32x4 acc[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[m] = rg_f32x4{0.f, 0.f, 0.f, 0.f};
+    rg_u32x4 op[2][2];
+    auto product = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(rg_bf16x8, op[j & 1][h]),
+              __builtin_bit_cast(rg_bf16x8, xf[j][h][m]), acc[m], 0, 0, 0);
+    };
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+      // the line has arrived when at most the R - 1 behind it are under way
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (R - 1)) : "memory");
+      op[j & 1][0] = ring[wave][used][turn_lines.get];
+      op[j & 1][1] = ring[wave][used][turn_lines.get_hi];
+      used = used + 1 == R ? 0 : used + 1;
+      if (j) product(j - 1);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      send();     // to where it was read
+    }
+    product(P - 1);
+    // adds the waves' sums; one barrier a unit, as above
+    const int b = turns & 1;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) sums[b][wave][m][lane] = acc[m];
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const int m = (wave - turns * MT) & (RG_WAVES - 1);   // waves take turns
+    if (m >= MT) continue;
+    rg_f32x4 y = sums[b][0][m][lane];
+#pragma unroll
+    for (int v = 1; v < RG_WAVES; ++v) y += sums[b][v][m][lane];
+    const int row = m * 16 + r16, n = unit * 16 + quad * 4;
+    if (row < a.M && n < a.N)
+      *reinterpret_cast<rg_f32x4*>(
+          a.part + ((int64_t)split * a.M + row) * a.N + n) = y;
+  }
+  // the last pieces land in LDS that is this workgroup's until it ends
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // In how many parts K is split for M rows of x and N outputs; 0: cannot be
 // taken, or would not fill the chip.
 //
@@ -525,11 +680,13 @@ int64_t held_splits(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || M > 64 || N < 1 || N % 4 != 0 || N > (1 << 26) ||
       K > (1 << 20))
     return 0;
-  for (int64_t S = 1; S <= 8; ++S)
-    if (K % (RG_WAVES * 64 * S) == 0) {
-      const int64_t lines = K / (RG_WAVES * 64 * S);
-      if (lines >= 4 && lines <= 8) return S;
-    }
+  // four tiles of rows leave registers for six lines, where it can be had so
+  for (const int64_t most : {M > 48 ? 6 : 8, 8})
+    for (int64_t S = 1; S <= 8; ++S)
+      if (K % (RG_WAVES * 64 * S) == 0) {
+        const int64_t lines = K / (RG_WAVES * 64 * S);
+        if (lines >= 4 && lines <= (S == 1 ? 8 : most)) return S;
+      }
   return 0;
 }
 
@@ -539,9 +696,8 @@ int64_t held_splits(int64_t M, int64_t N, int64_t K) {
 // (16 x 2048 5.2 and 3.3, 10240 x 4096 23.4 and 20.2), wider ones to 16 rows
 // (20480 x 4096 75.6 and 37.2, 32000 x 3584 46.1 and 41.2), to 32 from K = 2560 on
 // (20480 x 3584 40.9 and 31.3, but 32000 x 3584 41.4 and 43.1, 16384 x 2048 17.3 and
-// 18.6).  At a vocabulary's width what it gains alone is lost where it runs: 128256
-// x 4096, 16 rows, 187 and 182 one after the other, but 198 and 208 behind the
-// products of a prompt.
+// 18.6).  At a vocabulary's width it is ahead since its loads are nontemporal: 128256
+// x 4096, 8 and 16 rows, 190 183 and 169 171.
 // The two halves of more rows stream W at 4.5 TB/s: 10240 x 3584, 64 rows, 25.0 and
 // 22.3, 16384 x 3584 30.4 and 38.2.  Parts cost their sums, and a short K the
 // library has tiles for: up to 32 rows 10240 x 5120 33.2 and 27.5, 16384 x 5120 37.6
@@ -555,7 +711,8 @@ static bool held_ahead(int64_t M, int64_t N, int64_t K, int64_t S) {
   if (M < 7) return false;
   if (M > 32) return S == 1 ? N <= 10240 : N >= 1024 && N <= 6144;
   if (S == 1)
-    return N <= 10240 || (M <= 16 ? N <= 32768 : K >= 2560 && N <= 20480);
+    return N <= 10240 ||
+           (M <= 16 ? N <= 32768 || N >= 65536 : K >= 2560 && N <= 20480);
   return N <= 10240 && (M <= 16 || N >= 1024);
 }
 
@@ -596,6 +753,28 @@ torch::Tensor held_gemm_parts(const torch::Tensor& out, const torch::Tensor& x,
              bias.has_value() ? (const uint16_t*)bias->data_ptr() : nullptr,
              (int)M, (int)N, (int)K, x.stride(0)};
   const bool once = M <= 32 && N * K >= HELD_ONCE;
+  const int64_t lines = K / (RG_WAVES * 64 * S);
+#define LAUNCH_RING(P, MT)                                                    \
+  case MT * 16 + P:                                                           \
+    hipLaunchKernelGGL((ring_gemm_kernel<P, MT>), dim3(256),                  \
+                       dim3(64 * RG_WAVES), 0, stream, a, (int)S);            \
+    break
+  if (M > 32 && S > 1 && (M <= 48 || lines <= 6)) {
+    switch ((M > 48 ? 4 : 3) * 16 + lines) {
+      LAUNCH_RING(4, 3);
+      LAUNCH_RING(5, 3);
+      LAUNCH_RING(6, 3);
+      LAUNCH_RING(7, 3);
+      LAUNCH_RING(8, 3);
+      LAUNCH_RING(4, 4);
+      LAUNCH_RING(5, 4);
+      LAUNCH_RING(6, 4);
+      default: TORCH_CHECK(false, "no such parts: ", lines);
+    }
+    HIP_CHECK_KERNEL();
+    return part;
+  }
+#undef LAUNCH_RING
 #define LAUNCH_HELD_AS(...)                                                   \
   hipLaunchKernelGGL((held_gemm_kernel<__VA_ARGS__>), dim3(256),              \
                      dim3(64 * RG_WAVES), 0, stream, a, (int)S)
@@ -607,7 +786,7 @@ torch::Tensor held_gemm_parts(const torch::Tensor& out, const torch::Tensor& x,
     else if (once) LAUNCH_HELD_AS(P, 1, 1, true);                             \
     else LAUNCH_HELD_AS(P, 1, 1, false);                                      \
     break
-  switch (K / (RG_WAVES * 64 * S)) {
+  switch (lines) {
     LAUNCH_HELD(4);
     LAUNCH_HELD(5);
     LAUNCH_HELD(6);
