@@ -78,12 +78,20 @@ DEVINLINE wg_u32x4 wg_buffer(const uint16_t* p, int64_t bytes) {
 }
 
 // 64 lanes x 16 bytes from memory straight to LDS, 1024 bytes from `at` on.
+template <bool ONCE>
 DEVINLINE void wg_dma(wg_u32x4 buf, int lane_off, int off, uint32_t at) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
-      "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(at),
-      "v"(lane_off), "s"(buf), "s"(off)
-      : "memory", "m0");
+  if (ONCE)
+    asm volatile(
+        "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(at),
+        "v"(lane_off), "s"(buf), "s"(off)
+        : "memory", "m0");
+  else
+    asm volatile(
+        "s_mov_b32 m0, %0\n\ts_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(at),
+        "v"(lane_off), "s"(buf), "s"(off)
+        : "memory", "m0");
 }
 
 #define WG_INLINE __attribute__((always_inline))
@@ -93,7 +101,9 @@ DEVINLINE void wg_dma(wg_u32x4 buf, int lane_off, int off, uint32_t at) {
 // stacked W, known on the device only; an expert's tiles follow each other.
 // SPLIT: K in S parts of whole pairs of steps, as even as they go; a part of a tile
 // is an item like a tile and its sums go to `part`.
-template <int MT, int NT, int GATE, bool GROUPED, bool SPLIT = false>
+// ONCE: W is read by one patch of tiles and by nontemporal loads, which leave nothing
+// in the memory side's cache.
+template <int MT, int NT, int GATE, bool GROUPED, bool SPLIT, bool ONCE>
 __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
   constexpr bool SWIGLU = GATE != 0;
   constexpr int XB = 32 * MT * WG_BK, WB = 32 * NT * WG_BK;  // of a K step
@@ -202,10 +212,10 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)lds +
       wave * 8 * WG_BK * 2;
   auto load_x = [&](int i, int off, int buf) WG_INLINE {
-    wg_dma(xbuf, xo[i], off, lds0 + (buf + i * 32 * WG_BK) * 2);
+    wg_dma<false>(xbuf, xo[i], off, lds0 + (buf + i * 32 * WG_BK) * 2);
   };
   auto load_w = [&](int i, int off, int buf) WG_INLINE {
-    wg_dma(wbuf, wo[i], off, lds0 + (buf + i * 32 * WG_BK) * 2);
+    wg_dma<ONCE>(wbuf, wo[i], off, lds0 + (buf + i * 32 * WG_BK) * 2);
   };
   // a lane's 8 entries of the first half of a K step, and of the second
   const int f0 = r16 * WG_BK + ((quad ^ wg_swz(r16)) << 3), f1 = f0 ^ 32;
@@ -441,6 +451,12 @@ bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu) {
          (!swiglu || 2 * N * K < (int64_t)1 << 30);
 }
 
+// Up to this many rows a gated product reads W once and by nontemporal loads (us, plain
+// and so: 28672 x 4096, 200 / 256 / 384 / 512 rows 70.4 73.3 82.9 96.7 and 66.8 69.4 80.2
+// 94.1, 35840 x 5120 103 113 153 169 and 98.4 100 160 165; 8192 rows, where W comes
+// back from the caches for every patch of tiles, 1 % behind).
+constexpr int64_t WIDE_ONCE = 256;
+
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                int64_t gate, int64_t tile) {
   const bool swiglu = gate != 0;
@@ -464,14 +480,22 @@ void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   const WideArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)x.data_ptr(),
                    (const uint16_t*)w.data_ptr(), (int)M, (int)N, (int)K,
                    x.stride(0), nullptr, 0, nullptr, 1};
+  const bool once = M <= WIDE_ONCE;
 #define LAUNCH_WIDE_AS(...)                                                   \
-  hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__, false>), dim3(WG_BLOCKS), \
+  hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__>), dim3(WG_BLOCKS),        \
                      dim3(256), 0, stream, a)
 #define LAUNCH_WIDE(MT, NT)                                                   \
   case MT * 16 + NT:                                                          \
-    if (gate == 2) LAUNCH_WIDE_AS(MT, NT, 2);                                 \
-    else if (gate == 1) LAUNCH_WIDE_AS(MT, NT, 1);                            \
-    else LAUNCH_WIDE_AS(MT, NT, 0);                                           \
+    if (gate == 2 && once)                                                    \
+      LAUNCH_WIDE_AS(MT, NT, 2, false, false, true);                          \
+    else if (gate == 2)                                                       \
+      LAUNCH_WIDE_AS(MT, NT, 2, false, false, false);                         \
+    else if (gate == 1 && once)                                               \
+      LAUNCH_WIDE_AS(MT, NT, 1, false, false, true);                          \
+    else if (gate == 1)                                                       \
+      LAUNCH_WIDE_AS(MT, NT, 1, false, false, false);                         \
+    else                                                                      \
+      LAUNCH_WIDE_AS(MT, NT, 0, false, false, false);                         \
     break
   switch (tile) {
     LAUNCH_WIDE(8, 8);
@@ -587,10 +611,15 @@ torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
   const WideArgs a{nullptr, (const uint16_t*)x.data_ptr(),
                    (const uint16_t*)w.data_ptr(), (int)M, (int)N, (int)K,
                    x.stride(0), nullptr, 0, part.data_ptr<float>(), (int)S};
+  // nontemporal where one patch of tiles has all rows (8192 x 28672, 65 / 256 / 1024
+  // rows 107 154 347 and 91 131 337)
+#define LAUNCH_SPLIT_AS(...)                                                  \
+  hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__>), dim3(WG_BLOCKS),        \
+                     dim3(256), 0, stream, a)
 #define LAUNCH_SPLIT(MT, NT)                                                  \
   case MT * 16 + NT:                                                          \
-    hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, 0, false, true>),            \
-                       dim3(WG_BLOCKS), dim3(256), 0, stream, a);             \
+    if (M <= 4 * 32 * MT) LAUNCH_SPLIT_AS(MT, NT, 0, false, true, true);      \
+    else LAUNCH_SPLIT_AS(MT, NT, 0, false, true, false);                      \
     break
   switch (tile) {
     LAUNCH_SPLIT(3, 4);
@@ -605,6 +634,7 @@ torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
     default: TORCH_CHECK(false, "no such tile: ", tile);
   }
 #undef LAUNCH_SPLIT
+#undef LAUNCH_SPLIT_AS
   HIP_CHECK_KERNEL();
   return part;
 }
@@ -666,14 +696,21 @@ void grouped_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   const WideArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)x.data_ptr(),
                    (const uint16_t*)w.data_ptr(), (int)R, (int)N, (int)K, K,
                    (const int32_t*)start.data_ptr(), (int)E, nullptr, 1};
+  // nontemporal W where one patch of tiles has an expert's rows (three prompts of
+  // 560 to 700 tokens on eight experts of 14336 x 4096: a step 1442 and 1330 us)
+#define LAUNCH_GROUPED_AS(...)                                                \
+  hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__>), dim3(WG_BLOCKS),        \
+                     dim3(256), 0, stream, a)
 #define LAUNCH_GROUPED(MT, NT)                                                \
   case MT * 16 + NT:                                                          \
-    if (swiglu)                                                               \
-      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, 1, true>),              \
-                         dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
+    if (swiglu && R <= E * 4 * 32 * MT)                                       \
+      LAUNCH_GROUPED_AS(MT, NT, 1, true, false, true);                        \
+    else if (swiglu)                                                          \
+      LAUNCH_GROUPED_AS(MT, NT, 1, true, false, false);                       \
+    else if (R <= E * 4 * 32 * MT)                                            \
+      LAUNCH_GROUPED_AS(MT, NT, 0, true, false, true);                        \
     else                                                                      \
-      hipLaunchKernelGGL((wide_gemm_kernel<MT, NT, 0, true>),             \
-                         dim3(WG_BLOCKS), dim3(256), 0, stream, a);           \
+      LAUNCH_GROUPED_AS(MT, NT, 0, true, false, false);                       \
     break
   switch (tile > 0 ? tile : grouped_tile(R, E, N, swiglu)) {
     LAUNCH_GROUPED(8, 8);
@@ -685,6 +722,7 @@ void grouped_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     default: TORCH_CHECK(false, "no such tile: ", tile);
   }
 #undef LAUNCH_GROUPED
+#undef LAUNCH_GROUPED_AS
   HIP_CHECK_KERNEL();
 }
 
