@@ -24,6 +24,11 @@ from ..config import ModelConfig
 from .batch import ForwardBatch
 
 
+# rows whose products norm for themselves (ops.norm_linear); from seven on the
+# products come in parts that the norm adds (ops.linear_add_rmsnorm)
+FEW_ROWS = 6
+
+
 def _seed(name: str) -> int:
     # deterministic ACROSS PROCESSES: python's hash() is salted per process,
     # which would give each TP rank different weights (caught by the gloo
@@ -84,8 +89,13 @@ class LlamaAttention(nn.Module):
               kv_cache: Tuple[torch.Tensor, torch.Tensor],
               cos_sin: torch.Tensor) -> torch.Tensor:
         """What o_proj is applied to, [T, heads * head_dim]."""
-        T = x.shape[0]
-        qkv = ops.linear(x, self.qkv, self.qkv_b)
+        return self.attend(ops.linear(x, self.qkv, self.qkv_b), fb, kv_cache,
+                           cos_sin)
+
+    def attend(self, qkv: torch.Tensor, fb: ForwardBatch,
+               kv_cache: Tuple[torch.Tensor, torch.Tensor],
+               cos_sin: torch.Tensor) -> torch.Tensor:
+        T = qkv.shape[0]
         # strided views into the fused QKV output — the HIP kernels take a
         # row stride, so there are no .contiguous() copies on the hot path
         q, k, v = qkv.split(
@@ -171,6 +181,19 @@ class LlamaLayer(nn.Module):
             self.eps)
 
 
+    def few_rows(self, delta, residual, fb, kv_cache, cos_sin):
+        """The layer for a few rows, whose products norm for themselves.  delta:
+        what the residual still lacks (None: nothing); returns both."""
+        qkv, residual = ops.norm_linear(
+            delta, residual, self.input_norm_w, self.eps, self.attn.qkv,
+            self.attn.qkv_b)
+        delta = self.attn.o_proj(self.attn.attend(qkv, fb, kv_cache, cos_sin))
+        act, residual = ops.norm_linear(
+            delta, residual, self.post_norm_w, self.eps, self.mlp.gate_up,
+            silu=True)
+        return self.mlp.down_proj(act), residual
+
+
 class LlamaForCausalLM(nn.Module):
     def __init__(self, cfg: ModelConfig, device, dtype=torch.bfloat16):
         super().__init__()
@@ -199,6 +222,13 @@ class LlamaForCausalLM(nn.Module):
                 kv_caches: List[Tuple[torch.Tensor, torch.Tensor]]
                 ) -> torch.Tensor:
         residual = F.embedding(fb.token_ids, self.embed)
+        if residual.shape[0] <= FEW_ROWS:
+            delta = None
+            for i, layer in enumerate(self.layers):
+                delta, residual = layer.few_rows(
+                    delta, residual, fb, kv_caches[i], self.cos_sin)
+            return ops.fused_add_rmsnorm(delta, residual, self.final_norm_w,
+                                         self.cfg.norm_eps)[0]
         norms = [l.input_norm_w for l in self.layers] + [self.final_norm_w]
         x = ops.rmsnorm(residual, norms[0], self.cfg.norm_eps)
         for i, layer in enumerate(self.layers):

@@ -270,6 +270,25 @@ def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor,
     return fused_add_rmsnorm(linear(x, w), residual, weight, eps)
 
 
+def norm_linear(delta, residual: torch.Tensor, weight: torch.Tensor,
+                eps: float, w: torch.Tensor, bias=None, silu: bool = False):
+    """linear (silu: linear_silu_mul) of rmsnorm(residual + delta) * weight;
+    delta may be None.  Returns the product and residual + delta, which may or may
+    not be residual's memory.  A few rows run as one kernel."""
+    if (residual.is_cuda and HAS_KERNELS
+            and not torch.compiler.is_compiling()
+            and not has_torch_function_variadic(residual, weight, w)):
+        got = _kernels.norm_linear(delta, residual, weight, eps, w, bias,
+                                   int(silu))
+        if got is not None:
+            return got
+    if delta is None:
+        x = rmsnorm(residual, weight, eps)
+    else:
+        x, residual = fused_add_rmsnorm(delta, residual, weight, eps)
+    return (linear_silu_mul(x, w) if silu else linear(x, w, bias)), residual
+
+
 def linear_silu_mul(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """silu(x Wg^T) * (x Wu^T) with w = [Wg; Wu]: one kernel for bf16 rows
     where it is ahead, else the product and silu_mul."""

@@ -41,6 +41,15 @@ void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                int64_t gate, int64_t tile);
+bool norm_linear_takes(const c10::optional<torch::Tensor>& delta,
+                       const torch::Tensor& residual,
+                       const torch::Tensor& weight, const torch::Tensor& w,
+                       const c10::optional<torch::Tensor>& bias, bool swiglu,
+                       bool anywhere);
+c10::optional<std::tuple<torch::Tensor, torch::Tensor>> norm_linear(
+    const c10::optional<torch::Tensor>& delta, const torch::Tensor& residual,
+    const torch::Tensor& weight, double eps, const torch::Tensor& w,
+    const c10::optional<torch::Tensor>& bias, int64_t gate);
 int64_t wide_split(int64_t M, int64_t N, int64_t K);
 torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
                           int64_t tile, int64_t S);
@@ -133,6 +142,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("held_gemm", &igw::held_gemm,
         "x W^T of tens of rows, x in registers", py::arg("out"), py::arg("x"),
         py::arg("w"), py::arg("bias") = py::none());
+  m.def("norm_linear_takes", &igw::norm_linear_takes,
+        "whether gemv has the norm before it inside");
+  m.def("norm_linear", &igw::norm_linear,
+        "rmsnorm(residual + delta) W^T and residual + delta, None: nothing done");
   m.def("wide_split", &igw::wide_split,
         "256 x the tile + the parts of K of a product that leaves the chip idle");
   m.def("split_parts", &igw::split_parts, "sums of the parts of K of x W^T");

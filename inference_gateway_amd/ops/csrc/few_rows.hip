@@ -44,6 +44,11 @@ void sum_parts(torch::Tensor out, const torch::Tensor& part,
 bool sum_add_rmsnorm_fits(int64_t hidden);
 void sum_add_rmsnorm(torch::Tensor out, torch::Tensor part,
                      torch::Tensor residual, torch::Tensor weight, double eps);
+bool gemv_norm_fits(int64_t M, int64_t K, bool swiglu);
+void gemv_norm(torch::Tensor out, torch::Tensor sum, torch::Tensor delta,
+               torch::Tensor residual, torch::Tensor weight, double eps,
+               torch::Tensor w, c10::optional<torch::Tensor> bias,
+               int64_t gate);
 bool moe_few_fits(int64_t T, int64_t top_k, int64_t D, int64_t F);
 void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
           c10::optional<torch::Tensor> bias, int64_t gate);
@@ -176,6 +181,43 @@ c10::optional<torch::Tensor> linear_add_rmsnorm(const torch::Tensor& x,
   auto out = torch::empty_like(residual);
   sum_add_rmsnorm(out, part, residual, weight, eps);
   return out;
+}
+
+// Whether gemv takes the product of x = rmsnorm(residual + delta) with the norm in
+// it.
+bool norm_linear_takes(const c10::optional<torch::Tensor>& delta,
+                       const torch::Tensor& residual,
+                       const torch::Tensor& weight, const torch::Tensor& w,
+                       const c10::optional<torch::Tensor>& bias, bool swiglu,
+                       bool anywhere) {
+  if (few_rows_takes(residual, w, bias, swiglu, anywhere) != 1) return false;
+  const int64_t M = residual.size(0), K = residual.size(1);
+  if (!gemv_norm_fits(M, K, swiglu) || !residual.is_contiguous() ||
+      !plain_bf16(weight, residual.device()) || weight.dim() != 1 ||
+      weight.size(0) != K || !weight.is_contiguous() || !by16(weight))
+    return false;
+  return !delta.has_value() ||
+         (plain_bf16(*delta, residual.device()) && delta->dim() == 2 &&
+          delta->size(0) == M && delta->size(1) == K &&
+          delta->is_contiguous() && by16(*delta));
+}
+
+// The product and residual + delta (in memory of its own; without a delta the
+// residual itself), or nothing.
+c10::optional<std::tuple<torch::Tensor, torch::Tensor>> norm_linear(
+    const c10::optional<torch::Tensor>& delta, const torch::Tensor& residual,
+    const torch::Tensor& weight, double eps, const torch::Tensor& w,
+    const c10::optional<torch::Tensor>& bias, int64_t gate) {
+  if (!norm_linear_takes(delta, residual, weight, w, bias, gate != 0, false))
+    return c10::nullopt;
+  auto out = torch::empty(
+      {residual.size(0), gate != 0 ? w.size(0) / 2 : w.size(0)},
+      residual.options());
+  torch::Tensor sum, none;
+  if (delta.has_value()) sum = torch::empty_like(residual);
+  gemv_norm(out, sum, delta.has_value() ? *delta : none, residual, weight, eps,
+            w, bias, gate);
+  return std::make_tuple(out, delta.has_value() ? sum : residual);
 }
 
 // Whether moe_few takes a step: x [T, D], gate_up [E, 2 F, D], down [E, D, F].

@@ -34,15 +34,16 @@ constexpr int64_t GV_MAX_X = 64 * 1024; // entries of x: 128 KB of LDS
 
 // A wave's walk over the row groups first, first + stride, ... below `groups`
 // of W [N (or 2 N), K] against the M rows of x in LDS.  stage() puts x there,
-// after the first rows of W have been asked for; store(n, sums of W row n, of
-// its up row) is called by lane 0.
+// after the first rows of W have been asked for (ahead() is called before); store(n,
+// sums of W row n, of its up row) is called by lane 0.
 // U is the 16-byte loads in flight per row and lane (gemv_deep says when eight).
 // TAIL: K is not a multiple of the 512 entries of a load, and lanes lie past a
 // row's end.
-template <int M, int R, bool SWIGLU, bool TAIL, int U, class Stage, class Store>
+template <int M, int R, bool SWIGLU, bool TAIL, int U, class Stage, class Store,
+          class Ahead>
 DEVINLINE void gemv_walk(const uint16_t* xs, const uint16_t* __restrict__ w,
                          int N, int K, int first, int groups, int stride,
-                         Stage stage, Store store) {
+                         Stage stage, Store store, Ahead ahead) {
   const int lane = threadIdx.x & 63;
   const int chunks = (K + 511) >> 9;
   constexpr int STEP = SWIGLU ? R / 2 : R;   // output columns per group
@@ -68,6 +69,7 @@ DEVINLINE void gemv_walk(const uint16_t* xs, const uint16_t* __restrict__ w,
       }
     }
   };
+  ahead();
   if (first < groups) load(first, 0);
   stage();
 
@@ -155,7 +157,129 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_kernel(
           else if (bias) y += bf16_to_f32(bias[n]);
           out[(int64_t)m * N + n] = f32_to_bf16(y);
         }
-      });
+      },
+      [] {});
+}
+
+// The same with the norm before it: x = rmsnorm(residual + delta) * weight, rows of
+// K entries.  Every workgroup norms for itself (24 KB a row from L2, 512 times) while
+// its first rows of W are on their way, which takes longer; a launch of the norm's
+// own is 2.5 to 3 us of a decode step, twice a layer.  The first workgroup writes the
+// new residual, to other memory, as the others still read the old one.
+// A thread has 8 entries of a row in each of IT turns; sums wait in LDS.
+struct GemvNorm {
+  const uint16_t *delta, *residual, *weight;   // delta may be null
+  uint16_t* sum;                               // residual + delta, where there is one
+  float eps;
+};
+
+template <int M, int R, int GATE, int IT, int U>
+__global__ __launch_bounds__(64 * GV_WAVES, 4) void gemv_norm_kernel(
+    uint16_t* __restrict__ out, GemvNorm g, const uint16_t* __restrict__ w,
+    const uint16_t* __restrict__ bias, int rows, int N, int K) {
+  extern __shared__ __attribute__((aligned(16))) uint16_t xs[];   // [M][K]
+  __shared__ float red[GV_WAVES][M];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr bool SWIGLU = GATE != 0;
+  constexpr int STEP = SWIGLU ? R / 2 : R;
+  // Loads return in order: what the norm needs is asked for before W where it fits
+  // the registers, else two or three rows at a time behind it.
+  constexpr bool AHEAD = M * IT <= 4;
+  constexpr int G = M <= 4 && (AHEAD || M == 3) ? M : 2, TURNS = AHEAD ? IT : 1;
+  static_assert(M % G == 0);
+  ushort8 s[TURNS][G], d[TURNS][G];
+  auto fetch = [&](int it, int m0, int t) {
+    const int i = (it * 64 * GV_WAVES + threadIdx.x) * 8;
+    if (i >= K) return;
+#pragma unroll
+    for (int m = 0; m < G; ++m) {
+      const int64_t at = (int64_t)min(m0 + m, rows - 1) * K + i;
+      s[t][m] = *reinterpret_cast<const ushort8*>(g.residual + at);
+      if (g.delta) d[t][m] = *reinterpret_cast<const ushort8*>(g.delta + at);
+    }
+  };
+  auto ahead = [&] {
+    if (!AHEAD) return;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) fetch(it, 0, it);
+    asm volatile("" ::: "memory");
+  };
+  auto stage = [&] {
+    float ss[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) ss[m] = 0.0f;
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int i = (it * 64 * GV_WAVES + threadIdx.x) * 8;
+#pragma unroll
+      for (int m0 = 0; m0 < M; m0 += G) {
+        const int t = AHEAD ? it : 0;
+        if (!AHEAD) fetch(it, m0, 0);
+        if (i < K) {
+#pragma unroll
+          for (int m = 0; m < G; ++m) {
+            ushort8& v = s[t][m];
+            if (g.delta) {
+#pragma unroll
+              for (int j = 0; j < 8; ++j)
+                v.v[j] = f32_to_bf16(bf16_to_f32(d[t][m].v[j]) +
+                                     bf16_to_f32(v.v[j]));
+              if (blockIdx.x == 0 && m0 + m < rows)
+                *reinterpret_cast<ushort8*>(g.sum + (int64_t)(m0 + m) * K + i) =
+                    v;
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+              const float f = bf16_to_f32(v.v[j]);
+              ss[m0 + m] += f * f;
+            }
+            *reinterpret_cast<ushort8*>(xs + (m0 + m) * K + i) = v;
+          }
+        }
+        asm volatile("" ::: "memory");
+      }
+    }
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      ss[m] = wave_reduce_sum(ss[m]);
+      if (lane == 0) red[wave][m] = ss[m];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      const int i = (it * 64 * GV_WAVES + threadIdx.x) * 8;
+      if (i >= K) continue;
+      const ushort8 wv = *reinterpret_cast<const ushort8*>(g.weight + i);
+#pragma unroll 2
+      for (int m = 0; m < M; ++m) {
+        float all = 0.0f;
+#pragma unroll
+        for (int v = 0; v < GV_WAVES; ++v) all += red[v][m];
+        const float inv = rsqrtf(all / K + g.eps);
+        ushort8 o = *reinterpret_cast<const ushort8*>(xs + m * K + i);
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          o.v[j] = f32_to_bf16(bf16_to_f32(o.v[j]) * inv *
+                               bf16_to_f32(wv.v[j]));
+        *reinterpret_cast<ushort8*>(xs + m * K + i) = o;
+      }
+    }
+    __syncthreads();
+  };
+  gemv_walk<M, R, SWIGLU, false, U>(
+      xs, w, N, K, blockIdx.x * GV_WAVES + wave, (N + STEP - 1) / STEP,
+      gridDim.x * GV_WAVES, stage, [&](int n, const float* a, const float* up) {
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          if (m >= rows) break;
+          float y = a[m];
+          if (SWIGLU) y = gate_act<GATE>(y) * up[m];
+          else if (bias) y += bf16_to_f32(bias[n]);
+          out[(int64_t)m * N + n] = f32_to_bf16(y);
+        }
+      },
+      ahead);
 }
 
 // ---------------------------------------------------------------------------
@@ -254,7 +378,8 @@ __global__ __launch_bounds__(64 * GV_WAVES, 4) void expert_gemv_kernel(
                 else
                   sums[a * N + n] = weight[a] * y[m];
               }
-            });
+            },
+            [] {});
       };
       if (rows == 1) pass(std::integral_constant<int, 1>{});
       else if (rows == 2) pass(std::integral_constant<int, 2>{});
@@ -487,6 +612,96 @@ void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 #undef LAUNCH_GV
 #undef GV_KERNEL
   HIP_CHECK_KERNEL();
+}
+
+// Whether gemv_norm can take M rows of K entries where gemv does.
+bool gemv_norm_fits(int64_t M, int64_t K, bool swiglu) {
+  return gemv_fits(M, K, swiglu) && K % 512 == 0 && K <= 2 * 64 * GV_WAVES * 8;
+}
+
+// out = rmsnorm(residual + delta) W^T (+ bias), or with a gate as gemv; sum takes
+// residual + delta (delta undefined: residual alone, and no sum).
+void gemv_norm(torch::Tensor out, torch::Tensor sum, torch::Tensor delta,
+               torch::Tensor residual, torch::Tensor weight, double eps,
+               torch::Tensor w, c10::optional<torch::Tensor> bias,
+               int64_t gate) {
+  const bool swiglu = gate != 0;
+  TORCH_CHECK(gate >= 0 && gate <= 1);
+  TORCH_CHECK(residual.is_cuda() && residual.dim() == 2 && w.dim() == 2);
+  const int64_t M = residual.size(0), K = residual.size(1);
+  const int64_t N = swiglu ? w.size(0) / 2 : w.size(0);
+  TORCH_CHECK(gemv_norm_fits(M, K, swiglu) && N >= 1 &&
+              delta.defined() == sum.defined());
+  auto check = [&](const torch::Tensor& t, int64_t n) {
+    TORCH_CHECK(t.device() == residual.device(), "tensors on different devices");
+    TORCH_CHECK(t.dtype() == torch::kBFloat16 && t.is_contiguous() &&
+                t.numel() == n);
+  };
+  auto check16 = [&](const torch::Tensor& t, int64_t n) {
+    check(t, n);
+    TORCH_CHECK((reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0);
+  };
+  check16(residual, M * K);
+  check16(weight, K);
+  check16(w, (swiglu ? 2 * N : N) * K);
+  check(out, M * N);
+  if (delta.defined()) {
+    check16(delta, M * K);
+    check16(sum, M * K);
+  }
+  if (bias.has_value()) {
+    TORCH_CHECK(!swiglu);
+    check(*bias, N);
+  }
+  const at::cuda::CUDAGuard guard(residual.device());
+  hipStream_t stream = at::cuda::getCurrentCUDAStream();
+  const int64_t mp = M <= 4 ? M : M <= 6 ? 6 : 8;
+  const size_t shmem = (size_t)mp * K * 2;
+  const int64_t step = swiglu ? GV_ROWS / 2 : GV_ROWS;
+  const int64_t need = ((N + step - 1) / step + GV_WAVES - 1) / GV_WAVES;
+  const dim3 grid(std::min<int64_t>(need, 512));
+  const GemvNorm g{
+      delta.defined() ? (const uint16_t*)delta.data_ptr() : nullptr,
+      (const uint16_t*)residual.data_ptr(), (const uint16_t*)weight.data_ptr(),
+      sum.defined() ? (uint16_t*)sum.data_ptr() : nullptr, (float)eps};
+  const uint16_t* b =
+      bias.has_value() ? (const uint16_t*)bias->data_ptr() : nullptr;
+  auto launch = [&](auto kern) {
+    if (shmem > 64 * 1024)
+      TORCH_CHECK(hipFuncSetAttribute(
+                      (const void*)kern,
+                      hipFuncAttributeMaxDynamicSharedMemorySize,
+                      (int)shmem) == hipSuccess);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * GV_WAVES), shmem, stream,
+                       (uint16_t*)out.data_ptr(), g,
+                       (const uint16_t*)w.data_ptr(), b, (int)M, (int)N,
+                       (int)K);
+    HIP_CHECK_KERNEL();
+  };
+  const bool deep = gemv_deep(M, K), twice = K > 64 * GV_WAVES * 8;
+#define LAUNCH_GVN_G(MV, GATE)                                                \
+  do {                                                                        \
+    constexpr int DEEP = MV <= 3 ? 8 : 4;                                     \
+    if (deep && twice) launch(gemv_norm_kernel<MV, GV_ROWS, GATE, 2, DEEP>);  \
+    else if (deep) launch(gemv_norm_kernel<MV, GV_ROWS, GATE, 1, DEEP>);      \
+    else if (twice) launch(gemv_norm_kernel<MV, GV_ROWS, GATE, 2, 4>);        \
+    else launch(gemv_norm_kernel<MV, GV_ROWS, GATE, 1, 4>);                   \
+  } while (0)
+#define LAUNCH_GVN(MV)                                                        \
+  case MV:                                                                    \
+    if (swiglu) LAUNCH_GVN_G(MV, 1);                                          \
+    else LAUNCH_GVN_G(MV, 0);                                                 \
+    break
+  switch (mp) {
+    LAUNCH_GVN(1);
+    LAUNCH_GVN(2);
+    LAUNCH_GVN(3);
+    LAUNCH_GVN(4);
+    LAUNCH_GVN(6);
+    default: LAUNCH_GVN_G(8, 1); break;
+  }
+#undef LAUNCH_GVN
+#undef LAUNCH_GVN_G
 }
 
 }  // namespace igw
