@@ -50,6 +50,11 @@ c10::optional<std::tuple<torch::Tensor, torch::Tensor>> norm_linear(
     const c10::optional<torch::Tensor>& delta, const torch::Tensor& residual,
     const torch::Tensor& weight, double eps, const torch::Tensor& w,
     const c10::optional<torch::Tensor>& bias, int64_t gate);
+int64_t narrow_takes(const torch::Tensor& x, const torch::Tensor& w,
+                     const c10::optional<torch::Tensor>& bias, bool swiglu,
+                     bool anywhere);
+void narrow_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                 int64_t gate, int64_t tile);
 int64_t wide_split(int64_t M, int64_t N, int64_t K);
 torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
                           int64_t tile, int64_t S);
@@ -146,6 +151,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "whether gemv has the norm before it inside");
   m.def("norm_linear", &igw::norm_linear,
         "rmsnorm(residual + delta) W^T and residual + delta, None: nothing done");
+  m.def("narrow_takes", &igw::narrow_takes,
+        "narrow_gemm's tile of a call that it takes, 0: it does not");
+  m.def("narrow_gemm", &igw::narrow_gemm, "x W^T on tiles of few columns");
   m.def("wide_split", &igw::wide_split,
         "256 x the tile + the parts of K of a product that leaves the chip idle");
   m.def("split_parts", &igw::split_parts, "sums of the parts of K of x W^T");

@@ -1,7 +1,7 @@
 // Host side of ops.linear, ops.linear_silu_mul, ops.linear_gated_act, ops.moe_few
 // and ops.moe_rows: which calls the kernels for a few rows of x (gemv.hip), for
 // tens of them (rows_gemm and held_gemm in rows_gemm.hip) and for hundreds and
-// thousands of them (wide_gemm.hip) take.
+// thousands of them (narrow_gemm.hip, wide_gemm.hip) take.
 //
 // What they are handed is a pointer, so the tensors have to be what they seem:
 // plain dense bf16 on one GPU, in a call that nothing but the product has to
@@ -28,6 +28,9 @@ int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                int64_t gate, int64_t tile);
+int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated);
+void narrow_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                 int64_t gate, int64_t tile);
 int64_t wide_split(int64_t M, int64_t N, int64_t K);
 bool wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm);
 torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
@@ -80,25 +83,45 @@ static bool by16(const torch::Tensor& t) {
   return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;
 }
 
+// Whether the kernels can be handed the call at all.
+static bool call_fits(const torch::Tensor& x, const torch::Tensor& w,
+                      const c10::optional<torch::Tensor>& bias, bool swiglu,
+                      bool anywhere) {
+  if (!(anywhere || x.is_cuda()) || x.dim() != 2 || w.dim() != 2 ||
+      !call_is_plain() || !plain_bf16(x, x.device()) ||
+      !plain_bf16(w, x.device()))
+    return false;
+  const int64_t K = x.size(1);
+  const int64_t N = swiglu ? w.size(0) / 2 : w.size(0);
+  if (w.size(1) != K || (swiglu && w.size(0) % 2 != 0) || !w.is_contiguous() ||
+      x.stride(1) != 1 || x.stride(0) % 8 != 0 || !by16(x) || !by16(w))
+    return false;
+  return !bias.has_value() ||
+         (!swiglu && plain_bf16(*bias, x.device()) && bias->dim() == 1 &&
+          bias->size(0) == N && bias->is_contiguous());
+}
+
+// The tile of narrow_gemm for a call that it takes (it is asked before the others),
+// or 0.
+int64_t narrow_takes(const torch::Tensor& x, const torch::Tensor& w,
+                     const c10::optional<torch::Tensor>& bias, bool swiglu,
+                     bool anywhere) {
+  if (bias.has_value() || !call_fits(x, w, bias, swiglu, anywhere)) return 0;
+  const int64_t N = swiglu ? w.size(0) / 2 : w.size(0), K = x.size(1);
+  return wide_gemm_fits(x.stride(0), N, K, swiglu)
+             ? narrow_tile(x.size(0), N, K, swiglu)
+             : 0;
+}
+
 // Which kernel takes the call.  0: none of them, 1: gemv, 2: rows_gemm, 3:
 // wide_gemm, 4: held_gemm, 5: wide_gemm with K in parts.  `anywhere`: also off the
 // GPU (the rule alone, nothing is launched).  norm: fused_add_rmsnorm follows.
 static int64_t which_takes(const torch::Tensor& x, const torch::Tensor& w,
                            const c10::optional<torch::Tensor>& bias,
                            bool swiglu, bool anywhere, bool norm) {
-  if (!(anywhere || x.is_cuda()) || x.dim() != 2 || w.dim() != 2 ||
-      !call_is_plain() || !plain_bf16(x, x.device()) ||
-      !plain_bf16(w, x.device()))
-    return 0;
+  if (!call_fits(x, w, bias, swiglu, anywhere)) return 0;
   const int64_t M = x.size(0), K = x.size(1);
   const int64_t N = swiglu ? w.size(0) / 2 : w.size(0);
-  if (w.size(1) != K || (swiglu && w.size(0) % 2 != 0) || !w.is_contiguous() ||
-      x.stride(1) != 1 || x.stride(0) % 8 != 0 || !by16(x) || !by16(w))
-    return 0;
-  if (bias.has_value() &&
-      !(!swiglu && plain_bf16(*bias, x.device()) && bias->dim() == 1 &&
-        bias->size(0) == N && bias->is_contiguous()))
-    return 0;
   if (M > 64) {
     if (!wide_gemm_fits(x.stride(0), N, K, swiglu)) return 0;
     if (!bias.has_value() && wide_gemm_tile(M, N, K, swiglu) > 0) return 3;
@@ -129,11 +152,15 @@ c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
                                       const c10::optional<torch::Tensor>& bias,
                                       int64_t gate) {
   const bool swiglu = gate != 0;
-  const int64_t which = few_rows_takes(x, w, bias, swiglu, false);
-  if (which == 0) return c10::nullopt;
+  const int64_t tile = narrow_takes(x, w, bias, swiglu, false);
+  const int64_t which =
+      tile > 0 ? 0 : few_rows_takes(x, w, bias, swiglu, false);
+  if (tile == 0 && which == 0) return c10::nullopt;
   auto out = torch::empty({x.size(0), swiglu ? w.size(0) / 2 : w.size(0)},
                           x.options());
-  if (which == 3)
+  if (tile > 0)
+    narrow_gemm(out, x, w, gate, tile);
+  else if (which == 3)
     wide_gemm(out, x, w, gate,
               wide_gemm_tile(x.size(0), out.size(1), x.size(1), swiglu));
   else if (which == 4)

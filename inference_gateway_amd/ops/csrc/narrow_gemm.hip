@@ -1,0 +1,264 @@
+// Products of tens to hundreds of rows on the tiles of wide_tile.h: with K in parts,
+// or on tiles of fewer columns, where the whole K of wide tiles would leave compute
+// units without one.
+#include <ATen/cuda/CUDAContext.h>
+#include <c10/cuda/CUDAGuard.h>
+#include <torch/extension.h>
+
+#include <cmath>
+
+#include "wide_tile.h"
+
+namespace igw {
+
+bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu);
+
+// Products of rows that leave the chip idle, K in parts.
+//
+// Tiles with a part of K each, their fp32 sums to memory, and a
+// second kernel to add them (with the residual and the norm behind it where there is
+// one).  wide_split picks the tile and the parts by what they cost: rounds of 256
+// items at `step` us a K step of 64, against W from HBM, and the sums' way to memory and back.  Of 768 measured pairs of a tile and parts the
+// model is off by 4 % on average, and its choice is 2 % behind the best.
+struct SplitTile {
+  int MT, NT;
+  double step;
+};
+// us for `work` us of steps beside `mb` MB of W from HBM: about the longer of the two
+static double split_cost(double work, double mb) {
+  const double stream = mb / 4.6, a = work * work, b = stream * stream;
+  return std::sqrt(std::sqrt(a * a + b * b));
+}
+static constexpr SplitTile split_tiles[] = {
+    {3, 4, 0.500}, {4, 4, 0.567}, {4, 6, 0.712}, {6, 4, 0.671}, {6, 6, 0.845},
+    {6, 8, 1.069}, {8, 4, 0.799}, {8, 6, 1.049}, {8, 8, 1.387}};
+
+// 256 times the tile (16 MT + NT) and the parts of K, at least two; 0: cannot be.
+int64_t wide_split(int64_t M, int64_t N, int64_t K) {
+  if (M < 65 || M > (1 << 16) || N < 8 || N % 8 != 0 || N > (1 << 20) ||
+      K % (2 * WG_BK) != 0 || K > (1 << 20))
+    return 0;
+  int64_t best = 0;
+  double least = 0.0;
+  const int64_t pairs = K / (2 * WG_BK);
+  for (const auto& c : split_tiles)
+    for (int64_t S = 2; S <= 16 && 3 * S <= pairs; ++S) {
+      const int64_t items = (M + 32 * c.MT - 1) / (32 * c.MT) *
+                            ((N + 32 * c.NT - 1) / (32 * c.NT)) * S;
+      const int64_t rounds = (items + WG_BLOCKS - 1) / WG_BLOCKS;
+      const double work =
+          rounds * (2 * ((pairs + S - 1) / S) * c.step + 0.11);
+      const double cost =
+          split_cost(work, N * K * 2e-6) + S * M * N * 4e-6 * 0.36;
+      if (best == 0 || cost < least) {
+        best = (c.MT * 16 + c.NT) * 256 + S;
+        least = cost;
+      }
+    }
+  return best;
+}
+
+// Whether that is ahead of the library; norm: where the norm that follows adds the
+// parts, of the library and fused_add_rmsnorm.  Measured at 19 sizes of W by 16 of
+// 65 to 2600 rows (us, library and here; then with the norm).  Over a long K the
+// library's tiles are few: 4096 x 14336, 65 / 128 / 256 / 512 / 1024 / 2033 rows 50.6
+// 76.5 63.8 90.9 134 204 and 36.1 38.9 49.3 65.7 108 185; 5120 x 17920, 65 / 256 / 1024
+// 148 222 249 and 45.8 65.1 158, but 2033 rows 291 and 320; 8192 x 28672, 512 / 640
+// rows 312 260 and 195 289.  Of squarer W the parts' way to memory weighs more: 4096 x
+// 4096, 128 / 256 / 512 / 1024 / 1600 rows 24.0 22.4 30.9 42.1 55.6 and 18.0 21.8 30.7
+// 43.4 66.9 (with the norm 27.2 25.9 36.0 48.9 65.4 and 19.1 23.1 32.6 46.1 70.2), 5120
+// x 5120, 256 / 640 / 1024 rows 50.8 51.3 62.7 and 30.7 47.5 60.7, 7680 x 5120, 128 /
+// 512 / 640 rows 34.9 52.1 58.0 and 28.0 51.0 63.6, 6144 x 4096, 128 / 160 / 200 rows
+// 26.5 29.1 26.5 and 23.8 26.1 30.0, 8192 x 8192, 65 / 128 rows 38.9 51.8 and 43.6
+// 46.6.  Small W and a short K pay for the second launch: 1024 x 4096, 128 rows, 10.3
+// and 11.9, 4096 x 2048 13.1 and 15.4, as do wide ones: 16384 x 4096 40.3 and 46.9.
+bool wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm) {
+  if (wide_split(M, N, K) == 0) return false;
+  const int64_t least = N > 7680 && K < 2 * N ? 128 : 65;
+  int64_t most;
+  if (norm) {
+    if (K < 3584 || N * K < (int64_t)12 << 20 || N > 16384) return false;
+    most = K >= 3 * N   ? N > 5120 ? 512 : N > 4096 ? 1600 : 2048
+           : K >= 2 * N ? N > 5120 ? 512 : 1600
+           : K >= N     ? N > 7680 ? 512 : 1024
+                        : 512;
+  } else {
+    if (K < 4096 || N * K < (int64_t)16 << 20 || N < 2048 || N > 10240)
+      return false;
+    most = K >= 3 * N   ? N > 5120 ? 512 : N > 4096 ? 1600 : 2048
+           : K >= 2 * N ? N > 5120 ? 512 : 1300
+           : K >= 5120  ? 512
+           : K >= N     ? 256
+                        : 160;
+  }
+  return M >= least && M <= most;
+}
+
+// The sums [S, M, N] of the parts that wide_split says.
+torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
+                          int64_t tile, int64_t S) {
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 &&
+              x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
+              w.dim() == 2 && w.is_contiguous());
+  const int64_t M = x.size(0), K = x.size(1), N = w.size(0);
+  TORCH_CHECK(M >= 1 && N >= 8 && N % 8 == 0 && S >= 1 && S <= 64 &&
+              K / (2 * WG_BK) >= 3 * S && K % (2 * WG_BK) == 0 &&
+              M <= (1 << 20) && N <= (1 << 20) && K <= (1 << 20) &&
+              wide_gemm_fits(x.stride(0), N, K, false));
+  TORCH_CHECK(w.size(1) == K && x.stride(0) % 8 == 0);
+  TORCH_CHECK(w.device() == x.device(), "tensors on different devices");
+  for (const auto* t : {&x, &w})
+    TORCH_CHECK((reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) == 0);
+  const at::cuda::CUDAGuard guard(x.device());
+  hipStream_t stream = at::cuda::getCurrentCUDAStream();
+  auto part = torch::empty({S, M, N}, x.options().dtype(torch::kFloat32));
+  const WideArgs a{nullptr, (const uint16_t*)x.data_ptr(),
+                   (const uint16_t*)w.data_ptr(), (int)M, (int)N, (int)K,
+                   x.stride(0), nullptr, 0, part.data_ptr<float>(), (int)S};
+  // nontemporal where one patch of tiles has all rows (8192 x 28672, 65 / 256 / 1024
+  // rows 107 154 347 and 91 131 337)
+#define LAUNCH_SPLIT_AS(...)                                                  \
+  hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__>), dim3(WG_BLOCKS),        \
+                     dim3(256), 0, stream, a)
+#define LAUNCH_SPLIT(MT, NT)                                                  \
+  case MT * 16 + NT:                                                          \
+    if (M <= 4 * 32 * MT) LAUNCH_SPLIT_AS(MT, NT, 0, false, true, true);      \
+    else LAUNCH_SPLIT_AS(MT, NT, 0, false, true, false);                      \
+    break
+  switch (tile) {
+    LAUNCH_SPLIT(3, 4);
+    LAUNCH_SPLIT(4, 4);
+    LAUNCH_SPLIT(4, 6);
+    LAUNCH_SPLIT(6, 4);
+    LAUNCH_SPLIT(6, 6);
+    LAUNCH_SPLIT(6, 8);
+    LAUNCH_SPLIT(8, 4);
+    LAUNCH_SPLIT(8, 6);
+    LAUNCH_SPLIT(8, 8);
+    default: TORCH_CHECK(false, "no such tile: ", tile);
+  }
+#undef LAUNCH_SPLIT
+#undef LAUNCH_SPLIT_AS
+  HIP_CHECK_KERNEL();
+  return part;
+}
+
+// Gated products of up to 384 rows, and plain ones of a vocabulary's width of up to
+// 256, on tiles of 64 to 128 columns.
+//
+// So few rows are bound by streaming W, and wider tiles leave compute units without
+// one: 28672 rows of W are 112 tiles of 256 and 224 of 128.  Measured, before (the
+// library with silu_mul, or the tiles of wide_gemm_tile) and here (us): 28672 x 4096
+// as SwiGLU, 65 / 128 / 200 / 256 rows 60.1 60.5 65.4 68.5 and 48.4 52.2 62.1 62.6;
+// 35840 x 5120, 65 / 128 / 256 / 384 rows 90.4 86.6 99 160 and 68.0 71.8 86.4 136; 57344
+// x 8192, 160 / 256 rows 227 244 and 211 231; 14336 x 4096, 160 / 256 rows 44.0 56.5 and
+// 39.4 44.8, but 96 rows, with 112 tiles, 39.9 and 44.1; 128256 x 4096, 65 / 128 / 200 /
+// 256 rows 232 240 304 302 and 226 236 258 262; 32064 x 5120 70.5 73.9 91.3 94.2 and
+// 60.7 73.2 80.2 81.5.
+static constexpr SplitTile narrow_tiles[] = {
+    {3, 4, 0.500}, {4, 4, 0.567}, {3, 5, 0.560}, {4, 5, 0.640}, {6, 4, 0.671},
+    {6, 5, 0.758}, {8, 4, 0.799}, {8, 5, 0.920}};
+static constexpr SplitTile few_wide_tiles[] = {
+    {3, 4, 0.500}, {4, 4, 0.567}, {6, 4, 0.671}, {8, 4, 0.799}, {3, 8, 0.769},
+    {4, 8, 0.864}, {6, 6, 0.845}, {8, 6, 1.049}};
+// the tiles that a gated product would have else
+static constexpr SplitTile gated_tiles[] = {
+    {4, 8, 0.864}, {6, 8, 1.069}, {8, 6, 1.049}, {8, 7, 1.220}, {8, 8, 1.387}};
+
+// 16 MT + NT of the tile, or 0.
+int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated) {
+  if (M < 65 || M > (gated ? 384 : 256) || N < 8 || N % 8 != 0 ||
+      N > (1 << 24) || K < 2048 || K > 8192 || K % (2 * WG_BK) != 0 ||
+      (!gated && N < 32000))
+    return 0;
+  auto price = [&](const SplitTile& c, int64_t* items) {
+    const int64_t tn = (gated ? 16 : 32) * c.NT;
+    *items = (M + 32 * c.MT - 1) / (32 * c.MT) * ((N + tn - 1) / tn);
+    const int64_t rounds = (*items + WG_BLOCKS - 1) / WG_BLOCKS;
+    return split_cost(rounds * (K / WG_BK) * c.step,
+                      (gated ? 2 : 1) * N * K * 2e-6);
+  };
+  int64_t best = 0, tiles = 0, items = 0;
+  double least = 0.0;
+  for (int i = 0; i < 8; ++i) {
+    const auto& c = gated ? narrow_tiles[i] : few_wide_tiles[i];
+    const double cost = price(c, &items);
+    if (best == 0 || cost < least) {
+      best = c.MT * 16 + c.NT;
+      least = cost;
+      tiles = items;
+    }
+  }
+  if (!gated) return best;
+  for (const auto& c : gated_tiles)
+    if (price(c, &items) <= least) return 0;
+  return tiles >= WG_BLOCKS * 3 / 4 ? best : 0;
+}
+
+void narrow_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
+                 int64_t gate, int64_t tile) {
+  const bool swiglu = gate != 0;
+  TORCH_CHECK(gate >= 0 && gate <= 2);
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1 &&
+              x.dtype() == torch::kBFloat16 && w.dtype() == x.dtype() &&
+              w.dim() == 2 && w.is_contiguous() && out.dim() == 2 &&
+              out.is_contiguous() && out.dtype() == x.dtype());
+  const int64_t M = x.size(0), K = x.size(1), N = out.size(1);
+  TORCH_CHECK(M >= 1 && N >= 8 && N % 8 == 0 && K >= 6 * WG_BK &&
+              K % (2 * WG_BK) == 0 && M <= (1 << 20) && N <= (1 << 24) &&
+              wide_gemm_fits(x.stride(0), N, K, swiglu));
+  TORCH_CHECK(out.size(0) == M && w.size(1) == K &&
+              w.size(0) == (swiglu ? 2 * N : N) && x.stride(0) % 8 == 0);
+  TORCH_CHECK(w.device() == x.device() && out.device() == x.device(),
+              "tensors on different devices");
+  for (const auto* t : {&out, &x, &w})
+    TORCH_CHECK((reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) == 0);
+  const at::cuda::CUDAGuard guard(x.device());
+  hipStream_t stream = at::cuda::getCurrentCUDAStream();
+  const WideArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)x.data_ptr(),
+                   (const uint16_t*)w.data_ptr(), (int)M, (int)N, (int)K,
+                   x.stride(0), nullptr, 0, nullptr, 1};
+#define LAUNCH_NARROW_AS(...)                                                 \
+  hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__, false, false, true>),     \
+                     dim3(WG_BLOCKS), dim3(256), 0, stream, a)
+#define LAUNCH_GATED(MT, NT)                                                  \
+  case MT * 16 + NT:                                                          \
+    if (gate == 2) LAUNCH_NARROW_AS(MT, NT, 2);                               \
+    else LAUNCH_NARROW_AS(MT, NT, 1);                                         \
+    break
+#define LAUNCH_PLAIN(MT, NT)                                                  \
+  case MT * 16 + NT:                                                          \
+    LAUNCH_NARROW_AS(MT, NT, 0);                                              \
+    break
+  if (swiglu) {
+    switch (tile) {
+      LAUNCH_GATED(3, 4);
+      LAUNCH_GATED(4, 4);
+      LAUNCH_GATED(3, 5);
+      LAUNCH_GATED(4, 5);
+      LAUNCH_GATED(6, 4);
+      LAUNCH_GATED(6, 5);
+      LAUNCH_GATED(8, 4);
+      LAUNCH_GATED(8, 5);
+      default: TORCH_CHECK(false, "no such tile: ", tile);
+    }
+  } else {
+    switch (tile) {
+      LAUNCH_PLAIN(3, 4);
+      LAUNCH_PLAIN(4, 4);
+      LAUNCH_PLAIN(6, 4);
+      LAUNCH_PLAIN(8, 4);
+      LAUNCH_PLAIN(3, 8);
+      LAUNCH_PLAIN(4, 8);
+      LAUNCH_PLAIN(6, 6);
+      LAUNCH_PLAIN(8, 6);
+      default: TORCH_CHECK(false, "no such tile: ", tile);
+    }
+  }
+#undef LAUNCH_PLAIN
+#undef LAUNCH_GATED
+#undef LAUNCH_NARROW_AS
+  HIP_CHECK_KERNEL();
+}
+
+}  // namespace igw

@@ -341,6 +341,33 @@ def test_split_lines(M, N, K, linear, norm):
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,gated,tile", [
+    (64, 28672, 4096, True, 0), (65, 28672, 4096, True, (3, 4)),
+    (128, 28672, 4096, True, (4, 4)), (160, 28672, 4096, True, (6, 4)),
+    (256, 28672, 4096, True, (8, 4)), (257, 28672, 4096, True, 0),
+    (96, 35840, 5120, True, (3, 5)), (256, 35840, 5120, True, (8, 5)),
+    (384, 35840, 5120, True, (6, 5)), (385, 35840, 5120, True, 0),
+    (96, 14336, 4096, True, 0), (160, 14336, 4096, True, (3, 4)),
+    (128, 7168, 8192, True, 0), (128, 28672, 8320, True, 0),
+    (128, 28672, 4160, True, 0), (128, 28680, 4096, True, 0),
+    (65, 128256, 4096, False, (3, 8)), (256, 128256, 4096, False, (8, 6)),
+    (257, 128256, 4096, False, 0), (128, 32064, 5120, False, (4, 4)),
+    (128, 31992, 5120, False, 0)])
+def test_narrow_lines(M, N, K, gated, tile):
+    bf = torch.bfloat16
+    x, w = torch.empty(M, K, dtype=bf), torch.empty(N, K, dtype=bf)
+
+    def takes(x, w, b=None):
+        return ops._kernels.narrow_takes(x, w, b, gated, True)
+
+    assert takes(x, w) == (tile and tile[0] * 16 + tile[1])
+    for args in ((x.float(), w), (x[:, 1:], w), (x.to("meta"), w),
+                 (x.clone().requires_grad_(), w), (x, w[::2]), (x[0], w),
+                 (x, w, torch.empty(N, dtype=bf))):
+        assert takes(*args) == 0
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 def test_wide_split_parts():
     """Every part of K has the three pairs of steps that the kernel needs."""
     tiles = set()
