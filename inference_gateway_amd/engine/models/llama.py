@@ -101,37 +101,37 @@ class LlamaAttention(nn.Module):
         q, k, v = qkv.split(
             [self.nq * self.hd, self.nkv * self.hd, self.nkv * self.hd], dim=-1)
         kc, vc = kv_cache
+        if not fb.is_prefill:
+            o = ops.rope_paged_attn_decode(
+                fb.positions, q, k, v, cos_sin, kc, vc, fb.slot_mapping,
+                fb.block_table, fb.ctx_lens, self.scale)
+            return o.view(T, self.nq * self.hd)
         ops.rope_append(fb.positions, q, k, v, self.hd, cos_sin, kc, vc,
                         fb.slot_mapping)
         k3 = k.view(T, self.nkv, self.hd)
         v3 = v.view(T, self.nkv, self.hd)
-        if fb.is_prefill:
-            P = fb.num_prefill_tokens if fb.is_mixed else T
-            qv = q.view(T, self.nq, self.hd)
-            # prompt rows and decoded rows of a mixed round side by side
-            o = qv.new_empty((T, self.nq, self.hd))
-            if fb.prefix_lens is not None:
-                # prefix-cache hit in the batch: q rows are suffixes;
-                # cached prefix + the just-appended suffix K/V are read
-                # back from the paged cache (ops/csrc/flash_prefill.hip)
-                ops.flash_prefill_paged(
-                    qv[:P], kc, vc, fb.block_table,
-                    fb.prefix_lens, fb.cu_seqlens, fb.seq_lens, self.scale,
-                    out=o[:P])
-            else:
-                ops.flash_prefill(
-                    qv[:P], k3[:P], v3[:P], fb.cu_seqlens,
-                    fb.seq_lens, self.scale, out=o[:P])
-            if fb.is_mixed:
-                # mixed round: rows [P, T) are one decode token per
-                # running sequence (engine._build_forward_batch)
-                ops.paged_attn_decode(
-                    qv[P:], kc, vc, fb.decode_block_table,
-                    fb.decode_ctx_lens, self.scale, out=o[P:])
+        P = fb.num_prefill_tokens if fb.is_mixed else T
+        qv = q.view(T, self.nq, self.hd)
+        # prompt rows and decoded rows of a mixed round side by side
+        o = qv.new_empty((T, self.nq, self.hd))
+        if fb.prefix_lens is not None:
+            # prefix-cache hit in the batch: q rows are suffixes;
+            # cached prefix + the just-appended suffix K/V are read
+            # back from the paged cache (ops/csrc/flash_prefill.hip)
+            ops.flash_prefill_paged(
+                qv[:P], kc, vc, fb.block_table,
+                fb.prefix_lens, fb.cu_seqlens, fb.seq_lens, self.scale,
+                out=o[:P])
         else:
-            o = ops.paged_attn_decode(
-                q.view(T, self.nq, self.hd), kc, vc, fb.block_table,
-                fb.ctx_lens, self.scale)
+            ops.flash_prefill(
+                qv[:P], k3[:P], v3[:P], fb.cu_seqlens,
+                fb.seq_lens, self.scale, out=o[:P])
+        if fb.is_mixed:
+            # mixed round: rows [P, T) are one decode token per
+            # running sequence (engine._build_forward_batch)
+            ops.paged_attn_decode(
+                qv[P:], kc, vc, fb.decode_block_table,
+                fb.decode_ctx_lens, self.scale, out=o[P:])
         return o.view(T, self.nq * self.hd)
 
 

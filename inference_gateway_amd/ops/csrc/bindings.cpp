@@ -21,6 +21,12 @@ void rope_append(torch::Tensor positions, torch::Tensor q, torch::Tensor k,
                  torch::Tensor slot_mapping);
 void append_kv_cache(torch::Tensor k, torch::Tensor v, torch::Tensor kcache,
                      torch::Tensor vcache, torch::Tensor slot_mapping);
+void rope_paged_attn_decode(torch::Tensor out, torch::Tensor positions,
+                            torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                            torch::Tensor cos_sin_cache, torch::Tensor kcache,
+                            torch::Tensor vcache, torch::Tensor slot_mapping,
+                            torch::Tensor block_table, torch::Tensor ctx_lens,
+                            double scale);
 void paged_attn_decode(torch::Tensor out, torch::Tensor q,
                        torch::Tensor kcache, torch::Tensor vcache,
                        torch::Tensor block_table, torch::Tensor ctx_lens,
@@ -134,6 +140,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "RoPE of q and k, k and v into the paged cache");
   m.def("append_kv_cache", &igw::append_kv_cache,
         "scatter step K/V into the paged cache (bf16, gfx950)");
+  m.def("rope_paged_attn_decode", &igw::rope_paged_attn_decode,
+        "rope_append and paged_attn_decode in one launch");
   m.def("paged_attn_decode", &igw::paged_attn_decode,
         "GQA paged-attention decode (bf16, gfx950)");
   m.def("flash_prefill", &igw::flash_prefill,

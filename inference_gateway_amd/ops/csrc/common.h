@@ -107,6 +107,14 @@ DEVINLINE float block_reduce_sum(float x, float* lds) {
   return lds[0];
 }
 
+// A rotated pair (x1, x2) of NeoX RoPE, rounded.  Written out, so that every kernel
+// has the same bits.
+DEVINLINE void rope_pair(uint16_t& x1, uint16_t& x2, float cos, float sin) {
+  const float a = bf16_to_f32(x1), b = bf16_to_f32(x2);
+  x1 = f32_to_bf16(fmaf(a, cos, -(b * sin)));
+  x2 = f32_to_bf16(fmaf(b, cos, a * sin));
+}
+
 // The gate of a gated activation, act(g): GATE 1 SiLU, 2 GELU by its tanh form
 // (0: the product has no activation), (1 + tanh(x)) / 2 being sigmoid(2 x).
 template <int GATE>

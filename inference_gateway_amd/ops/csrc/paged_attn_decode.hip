@@ -117,18 +117,32 @@ struct DecodeSplit {
   }
 };
 
-template <int G, int NWAVES>
+// What rope_append would have done before: queries are rotated as they are loaded,
+// and the new key and value go to the cache from the wave that reads their page,
+// before it does (a wave's accesses to memory keep their order).  No other workgroup
+// reads that page's key head: a sequence has one new token, and what sequences share
+// is not written.  As a launch of its own it takes 2 to 3 us of a small step's layer;
+// ops.rope_paged_attn_decode says up to where this is ahead.
+struct DecodeRope {
+  const int32_t* positions;   // [B]
+  const int32_t* slots;       // [B]: page * 16 + offset, < 0: not stored
+  const float* cos_sin;       // [positions, HD]
+  const uint16_t *k, *v;      // [B, NKV * HD], row strides k_rs and v_rs
+  int64_t k_rs, v_rs;
+};
+
+template <int G, int NWAVES, bool ROPE>
 __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel(
     uint16_t* __restrict__ out,          // [B, NQ, HD]
     const uint16_t* __restrict__ q,      // [B, NQ, HD]
-    const uint16_t* __restrict__ kcache, // [NB, NKV, BS, HD]
-    const uint16_t* __restrict__ vcache, // [NB, NKV, BS, HD]
+    uint16_t* kcache,                    // [NB, NKV, BS, HD]
+    uint16_t* vcache,                    // [NB, NKV, BS, HD]
     const int32_t* __restrict__ block_table, // [B, max_blocks]
     const int32_t* __restrict__ ctx_lens,    // [B]
     int max_blocks, int nkv, float scale, int q_rs,
     float* __restrict__ part_o,   // [B, NQ, nsplit, HD] when nsplit > 1
     float* __restrict__ part_ml,  // [B, NQ, nsplit, 2]: maximum (log2), sum
-    int nsplit, int min_blocks) {
+    int nsplit, int min_blocks, DecodeRope rope) {
   // q_rs: q row stride in elements (q may be a view into the fused QKV
   // GEMM output — no .contiguous() copy on the decode hot path)
   constexpr int HD = 128, BS = 16, PAGE = BS * HD;  // tokens, entries of a page
@@ -182,6 +196,45 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
                                               (kvh * G + r16 % G) * HD +
                                               kk * 32 + quad * 8);
     qf[kk] = f;
+  }
+  if (ROPE) {
+    const float* cs = rope.cos_sin + (int64_t)rope.positions[seq] * HD;
+    auto turned = [&](ushort8& a, ushort8& b, int d) PD_INLINE {
+      const float4* c = reinterpret_cast<const float4*>(cs + d);
+      const float4* s = reinterpret_cast<const float4*>(cs + HD / 2 + d);
+      const float4 c0 = c[0], c1 = c[1], s0 = s[0], s1 = s[1];
+      const float cv[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
+      const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+#pragma unroll
+      for (int j = 0; j < 8; ++j) rope_pair(a.v[j], b.v[j], cv[j], sv[j]);
+    };
+    const int slot = rope.slots[seq];
+    if (split == part.count - 1 && slot >= 0 &&
+        wave == (pairs > 0 ? (pairs - 1) % NWAVES : 0)) {
+      const int64_t cell =
+          ((int64_t)(slot / BS * nkv + kvh) * BS + slot % BS) * HD;
+      if (lane < 8) {
+        const uint16_t* k = rope.k + seq * rope.k_rs + kvh * HD + lane * 8;
+        ushort8 a = *reinterpret_cast<const ushort8*>(k);
+        ushort8 b = *reinterpret_cast<const ushort8*>(k + HD / 2);
+        turned(a, b, lane * 8);
+        *reinterpret_cast<ushort8*>(kcache + cell + lane * 8) = a;
+        *reinterpret_cast<ushort8*>(kcache + cell + HD / 2 + lane * 8) = b;
+      } else if (lane >= 16 && lane < 32) {
+        *reinterpret_cast<ushort8*>(vcache + cell + (lane - 16) * 8) =
+            *reinterpret_cast<const ushort8*>(rope.v + seq * rope.v_rs +
+                                              kvh * HD + (lane - 16) * 8);
+      }
+      asm volatile("" ::: "memory");
+    }
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      ushort8 a = __builtin_bit_cast(ushort8, qf[kk]);
+      ushort8 b = __builtin_bit_cast(ushort8, qf[kk + 2]);
+      turned(a, b, kk * 32 + quad * 8);
+      qf[kk] = __builtin_bit_cast(pd_bf16x8, a);
+      qf[kk + 2] = __builtin_bit_cast(pd_bf16x8, b);
+    }
   }
 
   // lane offsets into a page, bytes: K half a row of eight rows a load, turned
@@ -477,7 +530,7 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
                           const torch::Tensor& vcache,
                           const torch::Tensor& block_table,
                           const torch::Tensor& ctx_lens, float scale,
-                          hipStream_t stream) {
+                          const DecodeRope* rope, hipStream_t stream) {
   const int B = q.size(0);
   const int nkv = kcache.size(1);
   constexpr int HD = 128;
@@ -516,16 +569,17 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
   }
   auto launch = [&](auto waves_) {
     constexpr int NWAVES = decltype(waves_)::value;
-    hipLaunchKernelGGL((paged_attn_decode_kernel<G, NWAVES>),
-                       dim3(nkv, B, nsplit), dim3(NWAVES * WAVE_SIZE), 0,
+    auto kern = rope ? paged_attn_decode_kernel<G, NWAVES, true>
+                     : paged_attn_decode_kernel<G, NWAVES, false>;
+    hipLaunchKernelGGL(kern, dim3(nkv, B, nsplit), dim3(NWAVES * WAVE_SIZE), 0,
                        stream, (uint16_t*)out.data_ptr(),
                        (const uint16_t*)q.data_ptr(),
-                       (const uint16_t*)kcache.data_ptr(),
-                       (const uint16_t*)vcache.data_ptr(),
+                       (uint16_t*)kcache.data_ptr(),
+                       (uint16_t*)vcache.data_ptr(),
                        (const int32_t*)block_table.data_ptr(),
                        (const int32_t*)ctx_lens.data_ptr(), max_blocks, nkv,
                        scale, (int)q.stride(0), part_o, part_ml, nsplit,
-                       min_blocks);
+                       min_blocks, rope ? *rope : DecodeRope{});
   };
   // Four waves a workgroup, but two where one or two query heads share a key head and
   // the chip is filled many times over: the bytes of a short context are few for its
@@ -547,10 +601,11 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
   }
 }
 
-void paged_attn_decode(torch::Tensor out, torch::Tensor q,
-                       torch::Tensor kcache, torch::Tensor vcache,
-                       torch::Tensor block_table, torch::Tensor ctx_lens,
-                       double scale) {
+static void decode(torch::Tensor& out, const torch::Tensor& q,
+                   const torch::Tensor& kcache, const torch::Tensor& vcache,
+                   const torch::Tensor& block_table,
+                   const torch::Tensor& ctx_lens, double scale,
+                   const DecodeRope* rope) {
   TORCH_CHECK(q.is_cuda() && q.dtype() == torch::kBFloat16);
   TORCH_CHECK(q.stride(-1) == 1 && q.stride(1) == q.size(2));
   TORCH_CHECK(out.is_contiguous());
@@ -566,23 +621,70 @@ void paged_attn_decode(torch::Tensor out, torch::Tensor q,
   switch (G) {
     case 1:
       launch_decode<1>(out, q, kcache, vcache, block_table, ctx_lens,
-                       (float)scale, stream);
+                       (float)scale, rope, stream);
       break;
     case 2:
       launch_decode<2>(out, q, kcache, vcache, block_table, ctx_lens,
-                       (float)scale, stream);
+                       (float)scale, rope, stream);
       break;
     case 4:
       launch_decode<4>(out, q, kcache, vcache, block_table, ctx_lens,
-                       (float)scale, stream);
+                       (float)scale, rope, stream);
       break;
     case 8:
       launch_decode<8>(out, q, kcache, vcache, block_table, ctx_lens,
-                       (float)scale, stream);
+                       (float)scale, rope, stream);
       break;
     default:
       TORCH_CHECK(false, "unsupported GQA group size: ", G);
   }
+}
+
+void paged_attn_decode(torch::Tensor out, torch::Tensor q,
+                       torch::Tensor kcache, torch::Tensor vcache,
+                       torch::Tensor block_table, torch::Tensor ctx_lens,
+                       double scale) {
+  decode(out, q, kcache, vcache, block_table, ctx_lens, scale, nullptr);
+}
+
+// rope_append of q, k and v (q and k are left as they are), then
+// paged_attn_decode of the rotated q [B, NQ * HD].
+void rope_paged_attn_decode(torch::Tensor out, torch::Tensor positions,
+                            torch::Tensor q, torch::Tensor k, torch::Tensor v,
+                            torch::Tensor cos_sin_cache, torch::Tensor kcache,
+                            torch::Tensor vcache, torch::Tensor slot_mapping,
+                            torch::Tensor block_table, torch::Tensor ctx_lens,
+                            double scale) {
+  TORCH_CHECK(q.is_cuda() && q.dim() == 2 && k.dim() == 2 && v.dim() == 2 &&
+              q.dtype() == torch::kBFloat16 && k.dtype() == q.dtype() &&
+              v.dtype() == q.dtype() && kcache.dtype() == q.dtype() &&
+              vcache.dtype() == q.dtype());
+  TORCH_CHECK(positions.dtype() == torch::kInt32 &&
+              slot_mapping.dtype() == torch::kInt32 &&
+              positions.is_contiguous() && slot_mapping.is_contiguous());
+  TORCH_CHECK(cos_sin_cache.dtype() == torch::kFloat32 &&
+              cos_sin_cache.is_contiguous() && cos_sin_cache.size(-1) == 128);
+  TORCH_CHECK(kcache.dim() == 4 && kcache.is_contiguous() &&
+              vcache.is_contiguous() && vcache.sizes() == kcache.sizes() &&
+              kcache.size(3) == 128);
+  const int64_t B = q.size(0), nkv = kcache.size(1);
+  TORCH_CHECK(positions.numel() == B && slot_mapping.numel() == B &&
+              k.size(0) == B && v.size(0) == B && k.size(1) == nkv * 128 &&
+              v.size(1) == nkv * 128 && q.size(1) % (nkv * 128) == 0);
+  for (const auto* t : {&q, &k, &v})
+    TORCH_CHECK(t->stride(1) == 1 && t->stride(0) % 8 == 0 &&
+                (reinterpret_cast<uintptr_t>(t->data_ptr()) & 15) == 0);
+  for (const auto* t : {&out, &positions, &k, &v, &cos_sin_cache, &kcache,
+                        &vcache, &slot_mapping, &block_table, &ctx_lens})
+    TORCH_CHECK(t->device() == q.device(), "tensors on different devices");
+  const DecodeRope rope{(const int32_t*)positions.data_ptr(),
+                        (const int32_t*)slot_mapping.data_ptr(),
+                        (const float*)cos_sin_cache.data_ptr(),
+                        (const uint16_t*)k.data_ptr(),
+                        (const uint16_t*)v.data_ptr(), k.stride(0),
+                        v.stride(0)};
+  decode(out, q.unflatten(1, {-1, 128}), kcache, vcache, block_table, ctx_lens,
+         scale, &rope);
 }
 
 }  // namespace igw

@@ -61,14 +61,9 @@ __global__ void rope_kernel(uint16_t* __restrict__ q, uint16_t* __restrict__ k,
     const float4 s1 = *reinterpret_cast<const float4*>(cs + half + d0 + 4);
     const float cv[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
     const float sv[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
-    ushort8 o1, o2;
+    ushort8 o1 = v1, o2 = v2;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float x1 = bf16_to_f32(v1.v[j]);
-      const float x2 = bf16_to_f32(v2.v[j]);
-      o1.v[j] = f32_to_bf16(x1 * cv[j] - x2 * sv[j]);
-      o2.v[j] = f32_to_bf16(x2 * cv[j] + x1 * sv[j]);
-    }
+    for (int j = 0; j < 8; ++j) rope_pair(o1.v[j], o2.v[j], cv[j], sv[j]);
     *reinterpret_cast<ushort8*>(base + d0) = o1;
     *reinterpret_cast<ushort8*>(base + half + d0) = o2;
     if (APPEND && slot >= 0 && h >= nq) {
