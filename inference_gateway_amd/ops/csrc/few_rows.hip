@@ -101,18 +101,6 @@ static bool call_fits(const torch::Tensor& x, const torch::Tensor& w,
           bias->size(0) == N && bias->is_contiguous());
 }
 
-// The tile of narrow_gemm for a call that it takes (it is asked before the others),
-// or 0.
-int64_t narrow_takes(const torch::Tensor& x, const torch::Tensor& w,
-                     const c10::optional<torch::Tensor>& bias, bool swiglu,
-                     bool anywhere) {
-  if (bias.has_value() || !call_fits(x, w, bias, swiglu, anywhere)) return 0;
-  const int64_t N = swiglu ? w.size(0) / 2 : w.size(0), K = x.size(1);
-  return wide_gemm_fits(x.stride(0), N, K, swiglu)
-             ? narrow_tile(x.size(0), N, K, swiglu)
-             : 0;
-}
-
 // Which kernel takes the call.  0: none of them, 1: gemv, 2: rows_gemm, 3:
 // wide_gemm, 4: held_gemm, 5: wide_gemm with K in parts.  `anywhere`: also off the
 // GPU (the rule alone, nothing is launched).  norm: fused_add_rmsnorm follows.
@@ -137,6 +125,24 @@ int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
                        const c10::optional<torch::Tensor>& bias, bool swiglu,
                        bool anywhere) {
   return which_takes(x, w, bias, swiglu, anywhere, false);
+}
+
+// The tile of narrow_gemm for a call that it takes (it is asked before the others),
+// or 0.  Up to 48 rows of fewer than 65536 outputs, and 16 of a K below 4096, the other
+// kernels keep what they take, where they are as fast or faster (see narrow_gemm.hip).
+int64_t narrow_takes(const torch::Tensor& x, const torch::Tensor& w,
+                     const c10::optional<torch::Tensor>& bias, bool swiglu,
+                     bool anywhere) {
+  if (bias.has_value() || !call_fits(x, w, bias, swiglu, anywhere)) return 0;
+  const int64_t M = x.size(0), K = x.size(1);
+  const int64_t N = swiglu ? w.size(0) / 2 : w.size(0);
+  if (!wide_gemm_fits(x.stride(0), N, K, swiglu)) return 0;
+  if (M <= 64) {
+    const int64_t other = few_rows_takes(x, w, bias, swiglu, anywhere);
+    if (other == 1 || (other != 0 && M <= 48 && (N < 65536 || (M <= 16 && K < 4096))))
+      return 0;
+  }
+  return narrow_tile(M, N, K, swiglu);
 }
 
 // The sums of the parts that wide_split cuts K into.

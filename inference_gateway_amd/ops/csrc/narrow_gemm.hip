@@ -1,4 +1,4 @@
-// Products of tens to hundreds of rows on the tiles of wide_tile.h: with K in parts,
+// Products of a few to hundreds of rows on the tiles of wide_tile.h: with K in parts,
 // or on tiles of fewer columns, where the whole K of wide tiles would leave compute
 // units without one.
 #include <ATen/cuda/CUDAContext.h>
@@ -143,33 +143,39 @@ torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
   return part;
 }
 
-// Gated products of up to 384 rows, and plain ones of a vocabulary's width of up to
-// 256, on tiles of 64 to 128 columns.
+// Gated products of up to 384 rows, and plain ones of many outputs of up to 256, on
+// tiles of 64 to 128 columns.
 //
 // So few rows are bound by streaming W, and wider tiles leave compute units without
 // one: 28672 rows of W are 112 tiles of 256 and 224 of 128.  Measured, before (the
-// library with silu_mul, or the tiles of wide_gemm_tile) and here (us): 28672 x 4096
-// as SwiGLU, 65 / 128 / 200 / 256 rows 60.1 60.5 65.4 68.5 and 48.4 52.2 62.1 62.6;
-// 35840 x 5120, 65 / 128 / 256 / 384 rows 90.4 86.6 99 160 and 68.0 71.8 86.4 136; 57344
-// x 8192, 160 / 256 rows 227 244 and 211 231; 14336 x 4096, 160 / 256 rows 44.0 56.5 and
-// 39.4 44.8, but 96 rows, with 112 tiles, 39.9 and 44.1; 128256 x 4096, 65 / 128 / 200 /
-// 256 rows 232 240 304 302 and 226 236 258 262; 32064 x 5120 70.5 73.9 91.3 94.2 and
-// 60.7 73.2 80.2 81.5.
+// library with silu_mul, rows_gemm, held_gemm or the tiles of wide_gemm_tile) and here
+// (us): 28672 x 4096 as SwiGLU, 61 / 65 / 128 / 200 / 256 rows 46.1 60.1 60.5 65.4 68.5
+// and 42.3 44.0 52 63.5 64; 35840 x 5120, 16 / 48 / 65 / 128 / 256 / 384 rows 93 92 90.4
+// 86.6 99 160 and 63 65 68.0 71.8 86.4 136; 57344 x 8192, 61 / 160 / 256 rows 169 227 244
+// and 144 211 231; 14336 x 4096, 160 / 256 rows 44.0 56.5 and 39.4 44.8, but 96 rows,
+// with 112 tiles, 39.9 and 44.1; 128256 x 4096, 9 / 32 / 61 / 65 / 128 / 256 rows 164
+// 175 190 232 240 302 and 159 164 169 176 178 247; 32064 x 5120, 16 / 48 / 65 / 256 rows
+// 73.4 81.5 70.5 94.2 and 57 57 60.7 81.5; 28672 x 4096, 61 rows 46.6 and 42.1, but 24 to
+// 48 rows the same; 24576 x 5120, with 192 tiles, 64 rows 56.5 and 59.6
+// (as SwiGLU 24576 x 4096 52.6 and 43); 65536 x 2048 and
+// 152064 x 3584, 16 rows 48.7 182.8 and 50.1 179, 32 rows 62.7 261 and 50.6 191.
+static constexpr SplitTile two_tiles[] = {
+    {2, 4, 0.450}, {2, 5, 0.500}, {2, 8, 0.850}};  // up to 64 rows
 static constexpr SplitTile narrow_tiles[] = {
     {3, 4, 0.500}, {4, 4, 0.567}, {3, 5, 0.560}, {4, 5, 0.640}, {6, 4, 0.671},
     {6, 5, 0.758}, {8, 4, 0.799}, {8, 5, 0.920}};
 static constexpr SplitTile few_wide_tiles[] = {
     {3, 4, 0.500}, {4, 4, 0.567}, {6, 4, 0.671}, {8, 4, 0.799}, {3, 8, 0.769},
     {4, 8, 0.864}, {6, 6, 0.845}, {8, 6, 1.049}};
-// the tiles that a gated product would have else
+// the tiles that a gated product of more than 64 rows would have else
 static constexpr SplitTile gated_tiles[] = {
     {4, 8, 0.864}, {6, 8, 1.069}, {8, 6, 1.049}, {8, 7, 1.220}, {8, 8, 1.387}};
 
 // 16 MT + NT of the tile, or 0.
 int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated) {
-  if (M < 65 || M > (gated ? 384 : 256) || N < 8 || N % 8 != 0 ||
+  if (M < 7 || M > (gated ? 384 : 256) || N < 8 || N % 8 != 0 ||
       N > (1 << 24) || K < 2048 || K > 8192 || K % (2 * WG_BK) != 0 ||
-      (!gated && N < 32000))
+      (!gated && M > 64 && N < 32000))
     return 0;
   auto price = [&](const SplitTile& c, int64_t* items) {
     const int64_t tn = (gated ? 16 : 32) * c.NT;
@@ -180,8 +186,9 @@ int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated) {
   };
   int64_t best = 0, tiles = 0, items = 0;
   double least = 0.0;
-  for (int i = 0; i < 8; ++i) {
-    const auto& c = gated ? narrow_tiles[i] : few_wide_tiles[i];
+  for (int i = 0; i < (M <= 64 ? 3 : 8); ++i) {
+    const auto& c = M <= 64 ? two_tiles[i] : gated ? narrow_tiles[i] : few_wide_tiles[i];
+    if (!gated && c.NT % 2 != 0) continue;
     const double cost = price(c, &items);
     if (best == 0 || cost < least) {
       best = c.MT * 16 + c.NT;
@@ -189,10 +196,11 @@ int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated) {
       tiles = items;
     }
   }
-  if (!gated) return best;
-  for (const auto& c : gated_tiles)
-    if (price(c, &items) <= least) return 0;
-  return tiles >= WG_BLOCKS * 3 / 4 ? best : 0;
+  if (!gated && M > 64) return best;
+  if (M > 64)
+    for (const auto& c : gated_tiles)
+      if (price(c, &items) <= least) return 0;
+  return tiles >= WG_BLOCKS * (gated ? 6 : 7) / 8 ? best : 0;
 }
 
 void narrow_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -232,6 +240,9 @@ void narrow_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     break
   if (swiglu) {
     switch (tile) {
+      LAUNCH_GATED(2, 4);
+      LAUNCH_GATED(2, 5);
+      LAUNCH_GATED(2, 8);
       LAUNCH_GATED(3, 4);
       LAUNCH_GATED(4, 4);
       LAUNCH_GATED(3, 5);
@@ -244,6 +255,8 @@ void narrow_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
     }
   } else {
     switch (tile) {
+      LAUNCH_PLAIN(2, 4);
+      LAUNCH_PLAIN(2, 8);
       LAUNCH_PLAIN(3, 4);
       LAUNCH_PLAIN(4, 4);
       LAUNCH_PLAIN(6, 4);

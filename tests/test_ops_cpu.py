@@ -342,17 +342,26 @@ def test_split_lines(M, N, K, linear, norm):
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 @pytest.mark.parametrize("M,N,K,gated,tile", [
-    (64, 28672, 4096, True, 0), (65, 28672, 4096, True, (3, 4)),
-    (128, 28672, 4096, True, (4, 4)), (160, 28672, 4096, True, (6, 4)),
-    (256, 28672, 4096, True, (8, 4)), (257, 28672, 4096, True, 0),
-    (96, 35840, 5120, True, (3, 5)), (256, 35840, 5120, True, (8, 5)),
-    (384, 35840, 5120, True, (6, 5)), (385, 35840, 5120, True, 0),
-    (96, 14336, 4096, True, 0), (160, 14336, 4096, True, (3, 4)),
-    (128, 7168, 8192, True, 0), (128, 28672, 8320, True, 0),
-    (128, 28672, 4160, True, 0), (128, 28680, 4096, True, 0),
-    (65, 128256, 4096, False, (3, 8)), (256, 128256, 4096, False, (8, 6)),
-    (257, 128256, 4096, False, 0), (128, 32064, 5120, False, (4, 4)),
-    (128, 31992, 5120, False, 0)])
+    # up to 48 rows what the others do not take, or a vocabulary
+    (48, 28672, 4096, True, 0), (49, 28672, 4096, True, (2, 4)),
+    (6, 35840, 5120, True, 0), (16, 35840, 5120, True, (2, 5)), (64, 35840, 5120, True, (2, 5)),
+    (48, 28672, 4096, False, 0), (64, 28672, 4096, False, (2, 4)),
+    (6, 128256, 4096, False, 0), (7, 128256, 4096, False, (2, 8)),
+    (16, 32064, 5120, False, (2, 4)), (16, 28544, 5120, False, 0), (16, 24576, 4096, True, (2, 4)),
+    (16, 24448, 4096, True, 0),
+    (16, 65536, 2048, False, 0), (17, 65536, 2048, False, (2, 8)),
+    (32, 152064, 3584, False, (2, 4)),
+    # hundreds
+    (65, 28672, 4096, True, (3, 4)), (128, 28672, 4096, True, (4, 4)),
+    (160, 28672, 4096, True, (6, 4)), (256, 28672, 4096, True, (8, 4)),
+    (257, 28672, 4096, True, 0), (96, 35840, 5120, True, (3, 5)),
+    (256, 35840, 5120, True, (8, 5)), (384, 35840, 5120, True, (6, 5)),
+    (385, 35840, 5120, True, 0), (96, 14336, 4096, True, 0),
+    (160, 14336, 4096, True, (3, 4)), (128, 7168, 8192, True, 0),
+    (128, 28672, 8320, True, 0), (128, 28672, 4160, True, 0),
+    (128, 28680, 4096, True, 0), (65, 128256, 4096, False, (3, 8)),
+    (256, 128256, 4096, False, (8, 6)), (257, 128256, 4096, False, 0),
+    (128, 32064, 5120, False, (4, 4))])
 def test_narrow_lines(M, N, K, gated, tile):
     bf = torch.bfloat16
     x, w = torch.empty(M, K, dtype=bf), torch.empty(N, K, dtype=bf)
