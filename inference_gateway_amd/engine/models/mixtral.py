@@ -125,8 +125,7 @@ class MixtralMoE(nn.Module):
         if ops.moe_few_fits(x, self.gate_up, self.down, self.top_k):
             # a few tokens reach a part of the experts: read only those
             # (5 tokens on six experts 324 us a layer, over all eight 600)
-            weights, _dst, idx, _counts = ops.moe_route(
-                self.router(x).float(), self.top_k, 64)
+            weights, idx = ops.moe_pick(x, self.router.weight, self.top_k)
             out = ops.moe_few(x, self.gate_up, self.down, idx, weights)
         elif ops.moe_rows_fits(x, self.gate_up, self.down, self.top_k):
             out = ops.moe_rows(x, self.router(x).contiguous(), self.gate_up,

@@ -379,6 +379,18 @@ def moe_grouped_gemm(a: torch.Tensor, w: torch.Tensor,
     return torch_ref.moe_grouped_gemm_ref(a, w, counts, capacity)
 
 
+def moe_pick(x: torch.Tensor, w: torch.Tensor, top_k: int):
+    """moe_route of the logits x w^T for a few tokens: (weights [T, K] fp32,
+    topk_idx [T, K] int32), in one launch."""
+    if (x.is_cuda and HAS_KERNELS and not torch.compiler.is_compiling()
+            and not has_torch_function_variadic(x, w)):
+        got = _kernels.moe_pick(x, w, top_k)
+        if got is not None:
+            return got
+    weights, _dst, idx, _counts = moe_route(linear(x, w).float(), top_k, 64)
+    return weights, idx
+
+
 def moe_few_fits(x: torch.Tensor, gate_up: torch.Tensor,
                  down: torch.Tensor, top_k: int) -> bool:
     """Whether moe_few takes this step: a few bf16 tokens on the GPU, a top_k

@@ -47,6 +47,10 @@ void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                int64_t gate, int64_t tile);
+bool moe_pick_takes(const torch::Tensor& x, const torch::Tensor& w, int64_t top_k,
+                    bool anywhere);
+c10::optional<std::tuple<torch::Tensor, torch::Tensor>> moe_pick(
+    torch::Tensor x, torch::Tensor w, int64_t top_k);
 bool norm_linear_takes(const c10::optional<torch::Tensor>& delta,
                        const torch::Tensor& residual,
                        const torch::Tensor& weight, const torch::Tensor& w,
@@ -155,6 +159,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("held_gemm", &igw::held_gemm,
         "x W^T of tens of rows, x in registers", py::arg("out"), py::arg("x"),
         py::arg("w"), py::arg("bias") = py::none());
+  m.def("moe_pick_takes", &igw::moe_pick_takes,
+        "whether moe_pick takes the call");
+  m.def("moe_pick", &igw::moe_pick,
+        "router product and the chosen experts of a few tokens, or None");
   m.def("norm_linear_takes", &igw::norm_linear_takes,
         "whether gemv has the norm before it inside");
   m.def("norm_linear", &igw::norm_linear,

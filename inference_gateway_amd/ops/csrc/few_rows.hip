@@ -29,6 +29,8 @@ bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu);
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                int64_t gate, int64_t tile);
 int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated);
+void moe_pick_rows(torch::Tensor weights, torch::Tensor topk_idx,
+                   const torch::Tensor& x, const torch::Tensor& w);
 void narrow_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                  int64_t gate, int64_t tile);
 int64_t wide_split(int64_t M, int64_t N, int64_t K);
@@ -268,6 +270,27 @@ bool moe_few_takes(const torch::Tensor& x, const torch::Tensor& gate_up,
   return gate_up.size(1) == 2 * F && gate_up.size(2) == D &&
          down.size(0) == E && down.size(1) == D &&
          moe_few_fits(x.size(0), top_k, D, F);
+}
+
+// Whether moe_pick takes the router's product of these tokens.
+bool moe_pick_takes(const torch::Tensor& x, const torch::Tensor& w, int64_t top_k,
+                    bool anywhere) {
+  return call_fits(x, w, c10::nullopt, false, anywhere) && x.size(0) <= 64 &&
+         x.size(1) % 8 == 0 && x.size(1) <= (1 << 20) && w.size(0) <= 64 &&
+         top_k <= w.size(0) &&
+         (top_k == 1 || top_k == 2 || top_k == 4 || top_k == 8);
+}
+
+// Weights and indices of the top_k experts of each token; None where it does not
+// take the call.
+c10::optional<std::tuple<torch::Tensor, torch::Tensor>> moe_pick(
+    torch::Tensor x, torch::Tensor w, int64_t top_k) {
+  if (!moe_pick_takes(x, w, top_k, false)) return c10::nullopt;
+  const c10::cuda::CUDAGuard guard(x.device());
+  auto weights = torch::empty({x.size(0), top_k}, x.options().dtype(torch::kFloat32));
+  auto idx = torch::empty({x.size(0), top_k}, x.options().dtype(torch::kInt32));
+  moe_pick_rows(weights, idx, x, w);
+  return std::make_tuple(weights, idx);
 }
 
 // Whether the grouped products take a step of any number of tokens.

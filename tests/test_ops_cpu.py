@@ -482,3 +482,20 @@ def test_linear_is_the_library_under_a_symbolic_trace():
     assert torch.equal(torch.fx.symbolic_trace(m)(x), m(x))
     torch.testing.assert_close(
         torch.vmap(m)(x[None])[0], x @ m.w.t())
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+def test_moe_pick_takes():
+    bf = torch.bfloat16
+    x, w = torch.empty(5, 64, dtype=bf), torch.empty(8, 64, dtype=bf)
+
+    def takes(x, w, k=2):
+        return ops._kernels.moe_pick_takes(x, w, k, True)
+
+    assert takes(x, w) and takes(torch.empty(64, 64, dtype=bf), w)
+    for args in ((torch.empty(65, 64, dtype=bf), w), (x.float(), w),
+                 (x, w, 3), (x, w[:1]), (x[:, 4:], w[:, 4:]),
+                 (x, torch.empty(65, 64, dtype=bf)), (x[0], w),
+                 (x, w.clone().requires_grad_()), (x, w.float()),
+                 (x[:, :60], w[:, :60].contiguous())):
+        assert not takes(*args)
