@@ -156,9 +156,13 @@ torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
 // with 112 tiles, 39.9 and 44.1; 128256 x 4096, 9 / 32 / 61 / 65 / 128 / 256 rows 164
 // 175 190 232 240 302 and 159 164 169 176 178 247; 32064 x 5120, 16 / 48 / 65 / 256 rows
 // 73.4 81.5 70.5 94.2 and 57 57 60.7 81.5; 28672 x 4096, 61 rows 46.6 and 42.1, but 24 to
-// 48 rows the same; 24576 x 5120, with 192 tiles, 64 rows 56.5 and 59.6
-// (as SwiGLU 24576 x 4096 52.6 and 43); 65536 x 2048 and
-// 152064 x 3584, 16 rows 48.7 182.8 and 50.1 179, 32 rows 62.7 261 and 50.6 191.
+// 48 rows the same; 24576 x 5120, with 192 tiles, 64 rows 56.5 and 59.6 (as SwiGLU 24576
+// x 4096 52.6 and 43); 65536 x 2048 and 152064 x 3584, 16 rows 48.7 182.8 and 50.1 179, 32
+// rows 62.7 261 and 50.6 191; 49152 x 6144, 65 / 160 / 256 rows 156 168 203 and 111 114
+// 129; 32768 x 8192 127 140 170 and 90 108 127; 128256 x 8192 426 463 546 and 339 398 467.
+// Of more than 192 rows of a long K the library is ahead where its tiles, 256 wide,
+// fill one round: 65536 x 8192, 200 / 256 rows, 211 237 and 235 243; 57344 x 8192 225 237
+// and 227 236; but 98304 x 8192 396 417 and 344 335.
 static constexpr SplitTile two_tiles[] = {
     {2, 4, 0.450}, {2, 5, 0.500}, {2, 8, 0.850}};  // up to 64 rows
 static constexpr SplitTile narrow_tiles[] = {
@@ -196,7 +200,10 @@ int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated) {
       tiles = items;
     }
   }
-  if (!gated && M > 64) return best;
+  if (!gated && M > 64) {
+    const int64_t its = (N + 255) / 256;   // the library's tiles
+    return M > 192 && K > 6144 && its >= WG_BLOCKS * 7 / 8 && its <= WG_BLOCKS ? 0 : best;
+  }
   if (M > 64)
     for (const auto& c : gated_tiles)
       if (price(c, &items) <= least) return 0;

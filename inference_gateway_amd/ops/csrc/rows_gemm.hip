@@ -34,8 +34,8 @@
 // and 48.0 50.7 51.0; 128256 x 4096 178 182 189 (5.6 TB/s) and 188 193 201; 4096 x
 // 14336 27.7 29.5 32.7 and 29.9 31.2 34.1.  The library, 32 / 48 / 64 rows: 56 64
 // 55, 200 210 213 and 34 40 41.  These are one after the other on one card; on
-// another 45.3 46.0 46.3 48.8 as SwiGLU and 186 191 195 for 128256 x 4096, which takes
-// 196 to 199 between the other kernels of a step.
+// another 45.3 46.0 46.3 48.8 as SwiGLU and 186 191 195 for 128256 x 4096.  narrow_gemm,
+// asked first, takes more than 48 rows of the former and the latter.
 #include <ATen/cuda/CUDAContext.h>
 #include <c10/cuda/CUDAGuard.h>
 #include <torch/extension.h>
@@ -697,7 +697,8 @@ int64_t held_splits(int64_t M, int64_t N, int64_t K) {
 // (20480 x 4096 75.6 and 37.2, 32000 x 3584 46.1 and 41.2), to 32 from K = 2560 on
 // (20480 x 3584 40.9 and 31.3, but 32000 x 3584 41.4 and 43.1, 16384 x 2048 17.3 and
 // 18.6).  At a vocabulary's width it is ahead since its loads are nontemporal: 128256
-// x 4096, 8 and 16 rows, 190 183 and 169 171.
+// x 4096, 8 and 16 rows, 190 183 and 169 171 (narrow_gemm, asked first, takes those
+// from K = 4096 on).
 // The two halves of more rows stream W at 4.5 TB/s: 10240 x 3584, 64 rows, 25.0 and
 // 22.3, 16384 x 3584 30.4 and 38.2.  Parts cost their sums, and a short K the
 // library has tiles for: up to 32 rows 10240 x 5120 33.2 and 27.5, 16384 x 5120 37.6

@@ -361,7 +361,8 @@ def test_split_lines(M, N, K, linear, norm):
     (128, 28672, 8320, True, 0), (128, 28672, 4160, True, 0),
     (128, 28680, 4096, True, 0), (65, 128256, 4096, False, (3, 8)),
     (256, 128256, 4096, False, (8, 6)), (257, 128256, 4096, False, 0),
-    (128, 32064, 5120, False, (4, 4))])
+    (128, 32064, 5120, False, (4, 4)), (160, 65536, 8192, False, (6, 4)),
+    (193, 65536, 8192, False, 0), (256, 98304, 8192, False, (8, 6))])
 def test_narrow_lines(M, N, K, gated, tile):
     bf = torch.bfloat16
     x, w = torch.empty(M, K, dtype=bf), torch.empty(N, K, dtype=bf)
