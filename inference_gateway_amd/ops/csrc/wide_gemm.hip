@@ -181,18 +181,19 @@ void grouped_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   const WideArgs a{(uint16_t*)out.data_ptr(), (const uint16_t*)x.data_ptr(),
                    (const uint16_t*)w.data_ptr(), (int)R, (int)N, (int)K, K,
                    (const int32_t*)start.data_ptr(), (int)E, nullptr, 1};
-  // nontemporal W where one patch of tiles has an expert's rows (three prompts of
-  // 560 to 700 tokens on eight experts of 14336 x 4096: a step 1442 and 1330 us)
+  // nontemporal W where half a patch of tiles has an expert's rows: three prompts of
+  // 560 to 700 tokens on eight experts of 14336 x 4096, a step 1442 and 1330 us; with 790
+  // rows an expert, some of which have more than a patch, 2484 and 2522
 #define LAUNCH_GROUPED_AS(...)                                                \
   hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__>), dim3(WG_BLOCKS),        \
                      dim3(256), 0, stream, a)
 #define LAUNCH_GROUPED(MT, NT)                                                \
   case MT * 16 + NT:                                                          \
-    if (swiglu && R <= E * 4 * 32 * MT)                                       \
+    if (swiglu && R <= E * 2 * 32 * MT)                                       \
       LAUNCH_GROUPED_AS(MT, NT, 1, true, false, true);                        \
     else if (swiglu)                                                          \
       LAUNCH_GROUPED_AS(MT, NT, 1, true, false, false);                       \
-    else if (R <= E * 4 * 32 * MT)                                            \
+    else if (R <= E * 2 * 32 * MT)                                            \
       LAUNCH_GROUPED_AS(MT, NT, 0, true, false, true);                        \
     else                                                                      \
       LAUNCH_GROUPED_AS(MT, NT, 0, true, false, false);                       \
