@@ -19,7 +19,8 @@ import torch.nn.functional as F
 from ... import ops
 from ...parallel.comm import tp_rank, tp_world_size
 from ...parallel.layers import (ColumnParallelLinear, ReplicatedLinear,
-                                RowParallelLinear, _init_weight)
+                                RowParallelLinear, _init_weight,
+                                calls_plainly)
 from ..config import ModelConfig
 from .batch import ForwardBatch
 
@@ -170,7 +171,30 @@ class LlamaLayer(nn.Module):
         self.mlp = LlamaMLP(cfg, layer, device, dtype)
         self.eps = cfg.norm_eps
 
-    def forward(self, x, residual, fb, kv_cache, cos_sin, next_norm_w):
+    def forward(self, x, residual, fb, kv_cache, cos_sin):
+        if residual is None:
+            residual = x.clone()
+            x = ops.rmsnorm(x, self.input_norm_w, self.eps)
+        else:
+            x, residual = ops.fused_add_rmsnorm(
+                x, residual, self.input_norm_w, self.eps)
+        x = self.attn(x, fb, kv_cache, cos_sin)
+        x, residual = ops.fused_add_rmsnorm(x, residual, self.post_norm_w,
+                                            self.eps)
+        x = self.mlp(x)
+        return x, residual
+
+    def opens(self) -> bool:
+        """Whether normed and few_rows, which call none of the modules that they
+        stand for, do what calls of them would."""
+        attn, mlp = self.attn, self.mlp
+        return (calls_plainly(self, LlamaLayer)
+                and calls_plainly(attn, LlamaAttention)
+                and calls_plainly(attn.o_proj, RowParallelLinear)
+                and calls_plainly(mlp, LlamaMLP)
+                and calls_plainly(mlp.down_proj, RowParallelLinear))
+
+    def normed(self, x, residual, fb, kv_cache, cos_sin, next_norm_w):
         """x: the residual normed for this layer; returns it normed for what
         follows, by next_norm_w, and the residual."""
         x, residual = self.attn.o_proj.add_rmsnorm(
@@ -179,7 +203,6 @@ class LlamaLayer(nn.Module):
         return self.mlp.down_proj.add_rmsnorm(
             ops.linear_silu_mul(x, self.mlp.gate_up), residual, next_norm_w,
             self.eps)
-
 
     def few_rows(self, delta, residual, fb, kv_cache, cos_sin):
         """The layer for a few rows, whose products norm for themselves.  delta:
@@ -222,6 +245,13 @@ class LlamaForCausalLM(nn.Module):
                 kv_caches: List[Tuple[torch.Tensor, torch.Tensor]]
                 ) -> torch.Tensor:
         residual = F.embedding(fb.token_ids, self.embed)
+        if not all(layer.opens() for layer in self.layers):
+            x, residual = residual, None
+            for i, layer in enumerate(self.layers):
+                x, residual = layer(x, residual, fb, kv_caches[i],
+                                    self.cos_sin)
+            return ops.fused_add_rmsnorm(x, residual, self.final_norm_w,
+                                         self.cfg.norm_eps)[0]
         if residual.shape[0] <= FEW_ROWS:
             delta = None
             for i, layer in enumerate(self.layers):
@@ -232,8 +262,8 @@ class LlamaForCausalLM(nn.Module):
         norms = [l.input_norm_w for l in self.layers] + [self.final_norm_w]
         x = ops.rmsnorm(residual, norms[0], self.cfg.norm_eps)
         for i, layer in enumerate(self.layers):
-            x, residual = layer(x, residual, fb, kv_caches[i], self.cos_sin,
-                                norms[i + 1])
+            x, residual = layer.normed(x, residual, fb, kv_caches[i],
+                                       self.cos_sin, norms[i + 1])
         return x
 
     def compute_logits(self, hidden_last: torch.Tensor) -> torch.Tensor:

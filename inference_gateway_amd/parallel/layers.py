@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
+from torch.nn.modules.module import _has_any_global_hook
 
 from .. import ops
 from .comm import (row_parallel_matmul_allreduce, tp_all_reduce,
@@ -27,6 +28,16 @@ def _init_weight(shape, device, dtype, seed: int) -> torch.Tensor:
     g = torch.Generator(device=dev).manual_seed(seed & 0x7FFFFFFF)
     w = torch.randn(shape, generator=g, device=dev, dtype=torch.float32) * 0.02
     return w.to(dtype)
+
+
+def calls_plainly(m: nn.Module, cls) -> bool:
+    """Whether a call of m is cls.forward and nothing else (no hook, no other
+    class, no compiled call), so that its caller may do the work itself."""
+    own = m.__dict__
+    return (type(m) is cls and "forward" not in own
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"]
+                     or own["_backward_hooks"] or own["_backward_pre_hooks"])
+            and m._compiled_call_impl is None and not _has_any_global_hook())
 
 
 class ColumnParallelLinear(nn.Module):

@@ -1503,3 +1503,77 @@ def test_finished_requests_are_evicted_from_bookkeeping(monkeypatch):
     assert len(eng._seqs) <= 8
     assert rids[0] not in eng._seqs            # oldest evicted
     assert rids[-1] in eng._seqs               # recent retained
+
+
+def _prompt_batch(eng, rows):
+    from inference_gateway_amd.engine.models.batch import ForwardBatch
+
+    pos = torch.arange(rows, dtype=torch.int32)
+    return ForwardBatch(token_ids=torch.arange(rows) + 1, positions=pos,
+                        slot_mapping=pos + 16, is_prefill=True,
+                        cu_seqlens=torch.tensor([0, rows], dtype=torch.int32),
+                        seq_lens=[rows])
+
+
+@pytest.mark.parametrize("rows", [3, 9])
+def test_llama_modules_are_called(rows):
+    """A hook on any module of a layer runs, a module put in another's place is
+    the one that is used, and what comes out is the same: the layers do without
+    calls of their modules only where nobody can tell."""
+    eng = _engine()
+    model, fb = eng.model, _prompt_batch(eng, rows)
+    want = model(fb, eng.kv_caches)
+    layer = model.layers[1]
+    for m in (layer, layer.attn, layer.attn.o_proj, layer.mlp,
+              layer.mlp.down_proj):
+        seen = []
+        handles = (m.register_forward_hook(lambda *a: seen.append("after")),
+                   m.register_forward_pre_hook(lambda *a: seen.append("to")))
+        assert torch.equal(model(fb, eng.kv_caches), want)
+        assert seen == ["to", "after"]
+        for h in handles:
+            h.remove()
+    seen = []
+    handle = torch.nn.modules.module.register_module_forward_hook(
+        lambda m, *a: seen.append(m))
+    assert torch.equal(model(fb, eng.kv_caches), want)
+    handle.remove()
+    assert {id(layer.mlp), id(layer.attn.o_proj), id(model.layers[0])} <= {
+        id(m) for m in seen}
+
+    class Negated(torch.nn.Module):
+        def __init__(self, m):
+            super().__init__()
+            self.m = m
+
+        def forward(self, *a):
+            return -self.m(*a)
+
+    for owner, name in ((layer.attn, "o_proj"), (layer, "mlp"),
+                        (layer, "attn"), (layer.mlp, "down_proj")):
+        m = getattr(owner, name)
+        setattr(owner, name, Negated(m))
+        other = model(fb, eng.kv_caches)
+        setattr(owner, name, Negated(Negated(m)))
+        assert torch.equal(model(fb, eng.kv_caches), want)
+        setattr(owner, name, m)
+        assert not torch.equal(other, want)
+    assert torch.equal(model(fb, eng.kv_caches), want)
+
+
+def test_llama_layers_one_by_one():
+    """A layer called by itself: what the residual lacks and the residual, its
+    input left as it was."""
+    from inference_gateway_amd import ops
+
+    eng = _engine()
+    model, fb = eng.model, _prompt_batch(eng, 5)
+    want = model(fb, eng.kv_caches)
+    x = torch.nn.functional.embedding(fb.token_ids, model.embed)
+    kept, first, residual = x.clone(), x, None
+    for layer, kv in zip(model.layers, eng.kv_caches):
+        x, residual = layer(x, residual, fb, kv, model.cos_sin)
+    assert torch.equal(first, kept)
+    got, _ = ops.fused_add_rmsnorm(x, residual, model.final_norm_w,
+                                   model.cfg.norm_eps)
+    assert torch.equal(got, want)
