@@ -24,7 +24,8 @@ import torch.nn.functional as F
 from ... import ops
 from ...parallel.comm import tp_rank, tp_world_size
 from ...parallel.layers import (ColumnParallelLinear, ReplicatedLinear,
-                                RowParallelLinear, _init_weight)
+                                RowParallelLinear, _init_weight,
+                                calls_plainly)
 from ..config import ModelConfig
 from .batch import ForwardBatch
 from .llama import LlamaAttention, _seed
@@ -125,7 +126,11 @@ class MixtralMoE(nn.Module):
         if ops.moe_few_fits(x, self.gate_up, self.down, self.top_k):
             # a few tokens reach a part of the experts: read only those
             # (5 tokens on six experts 324 us a layer, over all eight 600)
-            weights, idx = ops.moe_pick(x, self.router.weight, self.top_k)
+            if calls_plainly(self.router, ReplicatedLinear):
+                weights, idx = ops.moe_pick(x, self.router.weight, self.top_k)
+            else:
+                weights, _dst, idx, _counts = ops.moe_route(
+                    self.router(x).float(), self.top_k, 64)
             out = ops.moe_few(x, self.gate_up, self.down, idx, weights)
         elif ops.moe_rows_fits(x, self.gate_up, self.down, self.top_k):
             out = ops.moe_rows(x, self.router(x).contiguous(), self.gate_up,
@@ -371,9 +376,15 @@ class MixtralLayer(nn.Module):
         else:
             x, residual = ops.fused_add_rmsnorm(
                 x, residual, self.input_norm_w, self.eps)
-        x, residual = self.attn.o_proj.add_rmsnorm(
-            self.attn.heads(x, fb, kv_cache, cos_sin), residual,
-            self.post_norm_w, self.eps)
+        if (calls_plainly(self.attn, LlamaAttention)
+                and calls_plainly(self.attn.o_proj, RowParallelLinear)):
+            x, residual = self.attn.o_proj.add_rmsnorm(
+                self.attn.heads(x, fb, kv_cache, cos_sin), residual,
+                self.post_norm_w, self.eps)
+        else:
+            x = self.attn(x, fb, kv_cache, cos_sin)
+            x, residual = ops.fused_add_rmsnorm(x, residual, self.post_norm_w,
+                                                self.eps)
         x = self.moe(x, is_prefill=fb.is_prefill)
         return x, residual
 

@@ -1515,6 +1515,15 @@ def _prompt_batch(eng, rows):
                         seq_lens=[rows])
 
 
+class Negated(torch.nn.Module):
+    def __init__(self, m):
+        super().__init__()
+        self.m = m
+
+    def forward(self, *a, **kw):
+        return -self.m(*a, **kw)
+
+
 @pytest.mark.parametrize("rows", [3, 9])
 def test_llama_modules_are_called(rows):
     """A hook on any module of a layer runs, a module put in another's place is
@@ -1540,14 +1549,6 @@ def test_llama_modules_are_called(rows):
     handle.remove()
     assert {id(layer.mlp), id(layer.attn.o_proj), id(model.layers[0])} <= {
         id(m) for m in seen}
-
-    class Negated(torch.nn.Module):
-        def __init__(self, m):
-            super().__init__()
-            self.m = m
-
-        def forward(self, *a):
-            return -self.m(*a)
 
     for owner, name in ((layer.attn, "o_proj"), (layer, "mlp"),
                         (layer, "attn"), (layer.mlp, "down_proj")):
@@ -1577,3 +1578,40 @@ def test_llama_layers_one_by_one():
     got, _ = ops.fused_add_rmsnorm(x, residual, model.final_norm_w,
                                    model.cfg.norm_eps)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows", [3, 9])
+def test_mixtral_modules_are_called(rows, monkeypatch):
+    """As above; few: the route of a few tokens, which reads the router's weight."""
+    from inference_gateway_amd import ops
+
+    eng = LLMEngine(EngineConfig.tiny_moe(), device="cpu")
+    model, fb = eng.model, _prompt_batch(eng, rows)
+    layer = model.layers[1]
+
+    def few(x, gate_up, down, idx, weights):
+        y = torch.zeros_like(x, dtype=torch.float32)
+        for t in range(x.shape[0]):
+            for e, w in zip(idx[t].tolist(), weights[t]):
+                y[t] += w * (ops.linear_silu_mul(x[t:t + 1], gate_up[e])
+                             @ down[e].t())[0].float()
+        return y.to(x.dtype)
+
+    for fits in (False, True):
+        monkeypatch.setattr(ops, "moe_few_fits", lambda *a: fits)
+        monkeypatch.setattr(ops, "moe_few", few)
+        want = model(fb, eng.kv_caches)
+        for m in (layer, layer.attn, layer.attn.o_proj, layer.moe,
+                  layer.moe.router):
+            seen = []
+            handle = m.register_forward_hook(lambda *a: seen.append(1))
+            assert torch.equal(model(fb, eng.kv_caches), want)
+            handle.remove()
+            assert seen == [1]
+        for owner, name in ((layer.attn, "o_proj"), (layer, "attn"),
+                            (layer.moe, "router")):
+            m = getattr(owner, name)
+            setattr(owner, name, Negated(m))
+            other = model(fb, eng.kv_caches)
+            setattr(owner, name, m)
+            assert not torch.equal(other, want)
