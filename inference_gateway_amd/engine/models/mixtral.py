@@ -371,11 +371,16 @@ class MixtralLayer(nn.Module):
 
     def forward(self, x, residual, fb, kv_cache, cos_sin):
         if residual is None:
-            residual = x
+            residual = x.clone()
             x = ops.rmsnorm(x, self.input_norm_w, self.eps)
         else:
             x, residual = ops.fused_add_rmsnorm(
                 x, residual, self.input_norm_w, self.eps)
+        return self.normed(x, residual, fb, kv_cache, cos_sin)
+
+    def normed(self, x, residual, fb, kv_cache, cos_sin):
+        """x: the residual normed for this layer; the residual is added to in
+        place."""
         if (calls_plainly(self.attn, LlamaAttention)
                 and calls_plainly(self.attn.o_proj, RowParallelLinear)):
             x, residual = self.attn.o_proj.add_rmsnorm(
@@ -414,7 +419,14 @@ class MixtralForCausalLM(nn.Module):
         x = F.embedding(fb.token_ids, self.embed)
         residual = None
         for i, layer in enumerate(self.layers):
-            x, residual = layer(x, residual, fb, kv_caches[i], self.cos_sin)
+            if residual is None and calls_plainly(layer, MixtralLayer):
+                # the embedding's rows become the residual, without a copy
+                x, residual = layer.normed(
+                    ops.rmsnorm(x, layer.input_norm_w, layer.eps), x, fb,
+                    kv_caches[i], self.cos_sin)
+            else:
+                x, residual = layer(x, residual, fb, kv_caches[i],
+                                    self.cos_sin)
         x, _ = ops.fused_add_rmsnorm(x, residual, self.final_norm_w,
                                      self.cfg.norm_eps)
         return x

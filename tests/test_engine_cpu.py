@@ -1562,12 +1562,13 @@ def test_llama_modules_are_called(rows):
     assert torch.equal(model(fb, eng.kv_caches), want)
 
 
-def test_llama_layers_one_by_one():
+@pytest.mark.parametrize("preset", ["tiny_llama", "tiny_moe"])
+def test_layers_one_by_one(preset):
     """A layer called by itself: what the residual lacks and the residual, its
     input left as it was."""
     from inference_gateway_amd import ops
 
-    eng = _engine()
+    eng = LLMEngine(getattr(EngineConfig, preset)(), device="cpu")
     model, fb = eng.model, _prompt_batch(eng, 5)
     want = model(fb, eng.kv_caches)
     x = torch.nn.functional.embedding(fb.token_ids, model.embed)
