@@ -22,8 +22,9 @@ host's per-step device interaction is O(1) kernel launches.
 
 Padding rows (B < bucket) point at a dedicated pad slot whose position is
 0 and whose block-table row is all zeros, so they run a 1-token attention
-against reserved scratch block 0 and write their dummy KV there
-(BlockManager never hands out block 0).
+against reserved scratch block 0 (BlockManager never hands out block 0).
+Nothing is written for them: they share that block, and a row's append is
+ordered before its own reads only.
 """
 from __future__ import annotations
 
@@ -146,6 +147,7 @@ class DecodeGraphRunner:
         posl = pos.to(torch.int64)
         blk = bt.gather(1, (posl // bs).unsqueeze(1)).squeeze(1)
         slot_map = (blk * bs + (pos % bs)).to(torch.int32)
+        slot_map.masked_fill_(idx == self.pad_slot, -1)
         fb = ForwardBatch(
             token_ids=tokens,
             positions=pos,

@@ -1616,3 +1616,23 @@ def test_mixtral_modules_are_called(rows, monkeypatch):
             other = model(fb, eng.kv_caches)
             setattr(owner, name, m)
             assert not torch.equal(other, want)
+
+
+def test_graph_padding_rows_write_nothing():
+    """The rows that fill a captured batch all read page 0: none of them is
+    written, also where they outnumber the sequences."""
+    from inference_gateway_amd.engine.graph_runner import DecodeGraphRunner
+
+    run = object.__new__(DecodeGraphRunner)
+    run.cfg, run.pad_slot = EngineConfig.tiny_llama(), 4
+    run.in_slot_idx = torch.tensor([2, 0, 4, 4, 4])
+    run.slot_token = torch.tensor([11, 12, 13, 14, 0])
+    run.slot_pos = torch.tensor([17, 0, 5, 0, 0], dtype=torch.int32)
+    run.bt_slots = torch.tensor([[3, 7], [0, 0], [9, 0], [0, 0], [0, 0]],
+                                dtype=torch.int32)
+    for bucket in (2, 5):
+        fb = run._build_fb(bucket)
+        assert fb.slot_mapping.dtype == torch.int32
+        assert fb.slot_mapping.tolist() == [9 * 16 + 5, 7 * 16 + 1,
+                                            -1, -1, -1][:bucket]
+        assert fb.ctx_lens.tolist() == [6, 18, 1, 1, 1][:bucket]
