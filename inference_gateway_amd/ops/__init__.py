@@ -184,7 +184,9 @@ def rope_paged_attn_decode(positions, q, k, v, cos_sin_cache, kcache, vcache,
                            slot_mapping, block_table, ctx_lens, scale: float):
     """rope_append of one new token per sequence, then paged_attn_decode of its
     rotated queries; q [B, NQ*HD], k and v [B, NKV*HD].  Which of q and k are
-    rotated in place is not said.  No sequence may read another's new token.
+    rotated in place is not said.  The slot of a sequence's token (below 0: not
+    stored) is on a page that no other sequence of the call reads or writes: one
+    that does sees its content of before or after, or a mixture.
 
     One launch up to 1024 sequences x key heads.  Beyond, many workgroups follow
     each other on a compute unit and each waits for its angles (us, 32 heads on 8,

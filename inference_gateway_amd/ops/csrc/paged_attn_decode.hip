@@ -118,11 +118,13 @@ struct DecodeSplit {
 };
 
 // What rope_append would have done before: queries are rotated as they are loaded,
-// and the new key and value go to the cache from the wave that reads their page,
-// before it does (a wave's accesses to memory keep their order).  No other workgroup
-// reads that page's key head: a sequence has one new token, and what sequences share
-// is not written.  As a launch of its own it takes 2 to 3 us of a small step's layer;
-// ops.rope_paged_attn_decode says up to where this is ahead.
+// and a sequence's new key and value go to the cache from the wave that reads their
+// page, before it does (a wave's accesses to memory keep their order).  That is the
+// last page of the context, or else every wave looks its own pages through and each
+// that has the slot's writes it, the same bytes, and the last wave in any case.  What
+// other sequences read must not be written: a sequence that reads another's slot sees
+// it as it was or as it becomes.  As a launch of its own it takes 2 to 3 us of a small
+// step's layer; ops.rope_paged_attn_decode says up to where this is ahead.
 struct DecodeRope {
   const int32_t* positions;   // [B]
   const int32_t* slots;       // [B]: page * 16 + offset, < 0: not stored
@@ -209,8 +211,17 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
       for (int j = 0; j < 8; ++j) rope_pair(a.v[j], b.v[j], cv[j], sv[j]);
     };
     const int slot = rope.slots[seq];
-    if (split == part.count - 1 && slot >= 0 &&
-        wave == (pairs > 0 ? (pairs - 1) % NWAVES : 0)) {
+    bool write = split == part.count - 1 && slot >= 0 &&
+                 wave == (pairs > 0 ? (pairs - 1) % NWAVES : 0);
+    if (slot >= 0 && ctx > 0 && slot / BS != bt_row[(ctx - 1) / BS]) {
+      bool here = false;
+      for (int u = wave; u < pairs; u += 32 * NWAVES) {
+        const int b = block0 + 2 * (u + (lane >> 1) * NWAVES) + (lane & 1);
+        here |= b < nblocks && bt_row[min(b, nblocks - 1)] == slot / BS;
+      }
+      write |= __ballot(here) != 0;
+    }
+    if (write) {
       const int64_t cell =
           ((int64_t)(slot / BS * nkv + kvh) * BS + slot % BS) * HD;
       if (lane < 8) {
