@@ -232,8 +232,22 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(
 // out [M, N] = part [S, M, N] summed over S, plus the bias; N in fours
 void sum_parts(torch::Tensor out, const torch::Tensor& part,
                const c10::optional<torch::Tensor>& bias) {
+  TORCH_CHECK(part.is_cuda() && part.dim() == 3 && part.is_contiguous() &&
+              part.dtype() == torch::kFloat32);
   const int64_t S = part.size(0), M = part.size(1), N = part.size(2);
-  TORCH_CHECK(N % 4 == 0 && (M * N / 4 + 255) / 256 < (1LL << 31));
+  TORCH_CHECK(S < (1LL << 31) && M < (1LL << 31) && N < (1LL << 31) &&
+              N % 4 == 0 && (M * N / 4 + 255) / 256 < (1LL << 31));
+  TORCH_CHECK(out.dim() == 2 && out.size(0) == M && out.size(1) == N &&
+              out.is_contiguous() && out.dtype() == torch::kBFloat16 &&
+              (reinterpret_cast<uintptr_t>(out.data_ptr()) & 7) == 0 &&
+              (reinterpret_cast<uintptr_t>(part.data_ptr()) & 15) == 0);
+  TORCH_CHECK(out.device() == part.device() &&
+                  (!bias.has_value() || bias->device() == part.device()),
+              "tensors on different devices");
+  if (bias.has_value())
+    TORCH_CHECK(bias->dtype() == torch::kBFloat16 && bias->dim() == 1 &&
+                bias->size(0) == N && bias->is_contiguous());
+  if (M * N == 0) return;
   const at::cuda::CUDAGuard guard(part.device());
   hipLaunchKernelGGL(sum_parts_kernel, dim3((M * N / 4 + 255) / 256), dim3(256),
                      0, at::cuda::getCurrentCUDAStream(),
