@@ -33,8 +33,7 @@ void moe_pick_rows(torch::Tensor weights, torch::Tensor topk_idx,
                    const torch::Tensor& x, const torch::Tensor& w);
 void narrow_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                  int64_t gate, int64_t tile);
-int64_t wide_split(int64_t M, int64_t N, int64_t K);
-bool wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm);
+int64_t wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm);
 torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
                           int64_t tile, int64_t S);
 torch::Tensor rows_gemm_parts(const torch::Tensor& out, const torch::Tensor& x,
@@ -103,54 +102,81 @@ static bool call_fits(const torch::Tensor& x, const torch::Tensor& w,
           bias->size(0) == N && bias->is_contiguous());
 }
 
-// Which kernel takes the call.  0: none of them, 1: gemv, 2: rows_gemm, 3:
-// wide_gemm, 4: held_gemm, 5: wide_gemm with K in parts.  `anywhere`: also off the
-// GPU (the rule alone, nothing is launched).  norm: fused_add_rmsnorm follows.
-static int64_t which_takes(const torch::Tensor& x, const torch::Tensor& w,
-                           const c10::optional<torch::Tensor>& bias,
-                           bool swiglu, bool anywhere, bool norm) {
-  if (!call_fits(x, w, bias, swiglu, anywhere)) return 0;
+// A kernel and what it is launched with: the tile, with K in parts 256 times the
+// tile and the parts.
+struct Route {
+  int64_t kernel = 0, how = 0;
+};
+
+// The kernel of a call, narrow_gemm aside.  0: none of them, 1: gemv, 2: rows_gemm,
+// 3: wide_gemm, 4: held_gemm, 5: wide_gemm with K in parts.  `anywhere`: also off
+// the GPU (the rule alone, nothing is launched).  norm: fused_add_rmsnorm follows.
+static Route route_of(const torch::Tensor& x, const torch::Tensor& w,
+                      const c10::optional<torch::Tensor>& bias, bool swiglu,
+                      bool norm) {
   const int64_t M = x.size(0), K = x.size(1);
   const int64_t N = swiglu ? w.size(0) / 2 : w.size(0);
   if (M > 64) {
-    if (!wide_gemm_fits(x.stride(0), N, K, swiglu)) return 0;
-    if (!bias.has_value() && wide_gemm_tile(M, N, K, swiglu) > 0) return 3;
-    return !swiglu && wide_split_ahead(M, N, K, norm) ? 5 : 0;
+    if (!wide_gemm_fits(x.stride(0), N, K, swiglu)) return {};
+    const int64_t tile = bias.has_value() ? 0 : wide_gemm_tile(M, N, K, swiglu);
+    if (tile > 0) return {3, tile};
+    const int64_t cut = swiglu ? 0 : wide_split_ahead(M, N, K, norm);
+    return cut > 0 ? Route{5, cut} : Route{};
   }
-  if (gemv_fits(M, K, swiglu)) return gemv_ahead(M, w.size(0), K, swiglu);
-  if (!swiglu && held_gemm_takes(M, N, K)) return 4;
+  if (gemv_fits(M, K, swiglu)) return {gemv_ahead(M, w.size(0), K, swiglu)};
+  if (!swiglu && held_gemm_takes(M, N, K)) return {4};
   const int64_t S = rows_gemm_splits(M, N, K, swiglu);
-  return S > 0 && rows_gemm_ahead(M, S, K, swiglu) ? 2 : 0;
+  return {S > 0 && rows_gemm_ahead(M, S, K, swiglu) ? 2 : 0};
 }
 
-int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
-                       const c10::optional<torch::Tensor>& bias, bool swiglu,
-                       bool anywhere) {
-  return which_takes(x, w, bias, swiglu, anywhere, false);
-}
-
-// The tile of narrow_gemm for a call that it takes (it is asked before the others),
-// or 0.  Up to 48 rows of fewer than 65536 outputs, and 16 of a K below 4096, the other
-// kernels keep what they take, where they are as fast or faster (see narrow_gemm.hip).
-int64_t narrow_takes(const torch::Tensor& x, const torch::Tensor& w,
-                     const c10::optional<torch::Tensor>& bias, bool swiglu,
-                     bool anywhere) {
-  if (bias.has_value() || !call_fits(x, w, bias, swiglu, anywhere)) return 0;
+// narrow_gemm's tile for a call that it takes before `other`, or 0.  Up to 48 rows
+// of fewer than 65536 outputs, and 16 of a K below 4096, the other kernels keep what
+// they take, where they are as fast or faster (see narrow_gemm.hip).
+static int64_t narrow_before(const Route& other, const torch::Tensor& x,
+                             const torch::Tensor& w,
+                             const c10::optional<torch::Tensor>& bias,
+                             bool swiglu) {
   const int64_t M = x.size(0), K = x.size(1);
   const int64_t N = swiglu ? w.size(0) / 2 : w.size(0);
-  if (!wide_gemm_fits(x.stride(0), N, K, swiglu)) return 0;
-  if (M <= 64) {
-    const int64_t other = few_rows_takes(x, w, bias, swiglu, anywhere);
-    if (other == 1 || (other != 0 && M <= 48 && (N < 65536 || (M <= 16 && K < 4096))))
-      return 0;
-  }
+  if (bias.has_value() || other.kernel == 1 ||
+      !wide_gemm_fits(x.stride(0), N, K, swiglu))
+    return 0;
+  if (other.kernel != 0 && M <= 48 && (N < 65536 || (M <= 16 && K < 4096)))
+    return 0;
   return narrow_tile(M, N, K, swiglu);
 }
 
-// The sums of the parts that wide_split cuts K into.
-static torch::Tensor wide_parts(const torch::Tensor& x, const torch::Tensor& w) {
-  const int64_t cut = wide_split(x.size(0), w.size(0), x.size(1));
-  return split_parts(x, w, cut >> 8, cut & 255);
+// What runs the call: as above, 6: narrow_gemm.
+static Route product_route(const torch::Tensor& x, const torch::Tensor& w,
+                           const c10::optional<torch::Tensor>& bias,
+                           bool swiglu, bool anywhere) {
+  if (!call_fits(x, w, bias, swiglu, anywhere)) return {};
+  const Route other = route_of(x, w, bias, swiglu, false);
+  const int64_t tile = narrow_before(other, x, w, bias, swiglu);
+  return tile > 0 ? Route{6, tile} : other;
+}
+
+int64_t product_kernel(const torch::Tensor& x, const torch::Tensor& w,
+                       const c10::optional<torch::Tensor>& bias, bool swiglu,
+                       bool anywhere) {
+  return product_route(x, w, bias, swiglu, anywhere).kernel;
+}
+
+// As product_kernel, were narrow_gemm not there.
+int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
+                       const c10::optional<torch::Tensor>& bias, bool swiglu,
+                       bool anywhere) {
+  return call_fits(x, w, bias, swiglu, anywhere)
+             ? route_of(x, w, bias, swiglu, false).kernel
+             : 0;
+}
+
+// The tile of narrow_gemm for a call that it takes, or 0.
+int64_t narrow_takes(const torch::Tensor& x, const torch::Tensor& w,
+                     const c10::optional<torch::Tensor>& bias, bool swiglu,
+                     bool anywhere) {
+  const Route r = product_route(x, w, bias, swiglu, anywhere);
+  return r.kernel == 6 ? r.how : 0;
 }
 
 // The product, or nothing when none of the kernels takes it.  gate: 0 none, else W
@@ -159,45 +185,47 @@ c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
                                       const torch::Tensor& w,
                                       const c10::optional<torch::Tensor>& bias,
                                       int64_t gate) {
-  const bool swiglu = gate != 0;
-  const int64_t tile = narrow_takes(x, w, bias, swiglu, false);
-  const int64_t which =
-      tile > 0 ? 0 : few_rows_takes(x, w, bias, swiglu, false);
-  if (tile == 0 && which == 0) return c10::nullopt;
-  auto out = torch::empty({x.size(0), swiglu ? w.size(0) / 2 : w.size(0)},
+  const Route r = product_route(x, w, bias, gate != 0, false);
+  if (r.kernel == 0) return c10::nullopt;
+  auto out = torch::empty({x.size(0), gate != 0 ? w.size(0) / 2 : w.size(0)},
                           x.options());
-  if (tile > 0)
-    narrow_gemm(out, x, w, gate, tile);
-  else if (which == 3)
-    wide_gemm(out, x, w, gate,
-              wide_gemm_tile(x.size(0), out.size(1), x.size(1), swiglu));
-  else if (which == 4)
-    held_gemm(out, x, w, bias);
-  else if (which == 5)
-    sum_parts(out, wide_parts(x, w), bias);
-  else
-    (which == 1 ? gemv : rows_gemm)(out, x, w, bias, gate);
+  switch (r.kernel) {
+    case 1: gemv(out, x, w, bias, gate); break;
+    case 2: rows_gemm(out, x, w, bias, gate); break;
+    case 3: wide_gemm(out, x, w, gate, r.how); break;
+    case 4: held_gemm(out, x, w, bias); break;
+    case 5:
+      sum_parts(out, split_parts(x, w, r.how >> 8, r.how & 255), bias);
+      break;
+    default: narrow_gemm(out, x, w, gate, r.how);
+  }
   return out;
 }
 
 // Which of the kernels takes a product that fused_add_rmsnorm follows, in parts
 // that the norm adds; 0: none.
-int64_t linear_norm_takes(const torch::Tensor& x, const torch::Tensor& w,
-                          const torch::Tensor& residual,
-                          const torch::Tensor& weight, bool anywhere) {
-  const int64_t which =
-      which_takes(x, w, c10::nullopt, false, anywhere, true);
-  if (which != 2 && which != 4 && which != 5) return 0;
+static Route norm_route(const torch::Tensor& x, const torch::Tensor& w,
+                        const torch::Tensor& residual,
+                        const torch::Tensor& weight, bool anywhere) {
+  if (!call_fits(x, w, c10::nullopt, false, anywhere)) return {};
+  const Route r = route_of(x, w, c10::nullopt, false, true);
+  if (r.kernel != 2 && r.kernel != 4 && r.kernel != 5) return {};
   const int64_t M = x.size(0), N = w.size(0);
   if (!plain_bf16(residual, x.device()) || !plain_bf16(weight, x.device()) ||
       residual.dim() != 2 || residual.size(0) != M || residual.size(1) != N ||
       !residual.is_contiguous() || weight.dim() != 1 || weight.size(0) != N ||
       !weight.is_contiguous() || !by16(residual) || !by16(weight) ||
       !sum_add_rmsnorm_fits(N))
-    return 0;
-  if (which == 4 && held_splits(M, N, x.size(1)) < 2) return 0;
-  if (which == 2 && rows_gemm_splits(M, N, x.size(1), false) < 2) return 0;
-  return which;
+    return {};
+  if (r.kernel == 4 && held_splits(M, N, x.size(1)) < 2) return {};
+  if (r.kernel == 2 && rows_gemm_splits(M, N, x.size(1), false) < 2) return {};
+  return r;
+}
+
+int64_t linear_norm_takes(const torch::Tensor& x, const torch::Tensor& w,
+                          const torch::Tensor& residual,
+                          const torch::Tensor& weight, bool anywhere) {
+  return norm_route(x, w, residual, weight, anywhere).kernel;
 }
 
 // residual += x W^T in place and its norm, or nothing (and nothing done) when the
@@ -207,12 +235,13 @@ c10::optional<torch::Tensor> linear_add_rmsnorm(const torch::Tensor& x,
                                                 const torch::Tensor& residual,
                                                 const torch::Tensor& weight,
                                                 double eps) {
-  const int64_t which = linear_norm_takes(x, w, residual, weight, false);
-  if (which == 0) return c10::nullopt;
+  const Route r = norm_route(x, w, residual, weight, false);
+  if (r.kernel == 0) return c10::nullopt;
   const torch::Tensor none;
-  const auto part = which == 5   ? wide_parts(x, w)
-                    : which == 4 ? held_gemm_parts(none, x, w, c10::nullopt)
-                                 : rows_gemm_parts(none, x, w, c10::nullopt, 0);
+  const auto part =
+      r.kernel == 5   ? split_parts(x, w, r.how >> 8, r.how & 255)
+      : r.kernel == 4 ? held_gemm_parts(none, x, w, c10::nullopt)
+                      : rows_gemm_parts(none, x, w, c10::nullopt, 0);
   auto out = torch::empty_like(residual);
   sum_add_rmsnorm(out, part, residual, weight, eps);
   return out;

@@ -58,7 +58,7 @@ int64_t wide_split(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
-// Whether that is ahead of the library; norm: where the norm that follows adds the
+// What wide_split says where that is ahead of the library, else 0; norm: where the norm that follows adds the
 // parts, of the library and fused_add_rmsnorm.  Measured at 19 sizes of W by 16 of
 // 65 to 2600 rows (us, library and here; then with the norm).  Over a long K the
 // library's tiles are few: 4096 x 14336, 65 / 128 / 256 / 512 / 1024 / 2033 rows 50.6
@@ -72,26 +72,24 @@ int64_t wide_split(int64_t M, int64_t N, int64_t K) {
 // 26.5 29.1 26.5 and 23.8 26.1 30.0, 8192 x 8192, 65 / 128 rows 38.9 51.8 and 43.6
 // 46.6.  Small W and a short K pay for the second launch: 1024 x 4096, 128 rows, 10.3
 // and 11.9, 4096 x 2048 13.1 and 15.4, as do wide ones: 16384 x 4096 40.3 and 46.9.
-bool wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm) {
-  if (wide_split(M, N, K) == 0) return false;
+int64_t wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm) {
   const int64_t least = N > 7680 && K < 2 * N ? 128 : 65;
   int64_t most;
   if (norm) {
-    if (K < 3584 || N * K < (int64_t)12 << 20 || N > 16384) return false;
+    if (K < 3584 || N * K < (int64_t)12 << 20 || N > 16384) return 0;
     most = K >= 3 * N   ? N > 5120 ? 512 : N > 4096 ? 1600 : 2048
            : K >= 2 * N ? N > 5120 ? 512 : 1600
            : K >= N     ? N > 7680 ? 512 : 1024
                         : 512;
   } else {
-    if (K < 4096 || N * K < (int64_t)16 << 20 || N < 2048 || N > 10240)
-      return false;
+    if (K < 4096 || N * K < (int64_t)16 << 20 || N < 2048 || N > 10240) return 0;
     most = K >= 3 * N   ? N > 5120 ? 512 : N > 4096 ? 1600 : 2048
            : K >= 2 * N ? N > 5120 ? 512 : 1300
            : K >= 5120  ? 512
            : K >= N     ? 256
                         : 160;
   }
-  return M >= least && M <= most;
+  return M >= least && M <= most ? wide_split(M, N, K) : 0;
 }
 
 // The sums [S, M, N] of the parts that wide_split says.

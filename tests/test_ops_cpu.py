@@ -378,6 +378,40 @@ def test_narrow_lines(M, N, K, gated, tile):
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,gated,want", [
+    # each kernel, narrow_gemm beside those that it is asked before
+    (5, 4096, 4096, False, 1), (8, 28672, 4096, True, 1),
+    (33, 28672, 4096, False, 2), (33, 28672, 1024, True, 2),
+    (300, 128256, 4096, False, 3), (300, 28672, 4096, True, 3),
+    (33, 6144, 4096, False, 4), (16, 28672, 4096, False, 4),
+    (65, 4096, 14336, False, 5), (128, 4096, 4096, False, 5),
+    (64, 28672, 4096, False, 6), (64, 28672, 4096, True, 6),
+    (7, 128256, 4096, False, 6), (16, 128256, 4096, False, 6),
+    (64, 128256, 4096, False, 6), (256, 28672, 4096, True, 6),
+    (65, 35840, 5120, True, 6), (256, 128256, 4096, False, 6),
+    (513, 8192, 28672, False, 0), (65, 4100, 4096, False, 0)])
+def test_product_kernel(M, N, K, gated, want):
+    """One answer for what runs; with a bias or a call that none of them takes,
+    never narrow_gemm."""
+    bf = torch.bfloat16
+    x, w = torch.empty(M, K, dtype=bf), torch.empty(N, K, dtype=bf)
+
+    def which(f, x, w, b=None):
+        return f(x, w, b, gated, True)
+
+    k = ops._kernels
+    assert which(k.product_kernel, x, w) == want
+    assert (which(k.narrow_takes, x, w) > 0) == (want == 6)
+    if want != 6:
+        assert which(k.few_rows_takes, x, w) == want
+    b = torch.empty(N, dtype=bf)
+    assert which(k.product_kernel, x, w, b) == which(k.few_rows_takes, x, w, b)
+    for args in ((x.float(), w), (x[:, 1:], w), (x.to("meta"), w),
+                 (x.clone().requires_grad_(), w), (x, w[::2]), (x[0], w)):
+        assert which(k.product_kernel, *args) == 0
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 def test_wide_split_parts():
     """Every part of K has the three pairs of steps that the kernel needs."""
     tiles = set()
