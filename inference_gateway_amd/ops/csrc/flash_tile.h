@@ -271,10 +271,8 @@ DEVINLINE int ft_kswz(int r) {
 // VD < NV: the four waves have the SAME 32 query rows and each the VD value
 // dims from dim0 on (decoded rows: the heads that share keys).
 // SHARED: the values are the first entries of the key rows, v0 and v1 unused.
-// ONCE: decoded rows, whose keys nobody else reads: loads are nontemporal and
-// leave nothing in the memory side's cache (a step of 48 sequences of 700 to 3500
-// keys, two latent and two windowed layers of 32 heads: 864 and 836 us, some of it
-// by the products' loads).
+// ONCE: decoded rows, whose keys nobody reads again soon: loads are nontemporal and
+// leave nothing in the memory side's cache.
 template <int NK, int NV, bool PLAIN, class Rows, int VD = NV,
           bool SHARED = false, bool ONCE = false>
 DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,

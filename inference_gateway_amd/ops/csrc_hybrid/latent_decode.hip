@@ -33,7 +33,18 @@ struct LatentDecodeArgs {
   FlashParts parts;
 };
 
-template <int NK, int R>
+// From this many bytes of rows on (as if every context were the longest) they are
+// read with nontemporal loads: the memory side's cache, of this size, holds them
+// neither for the next step nor beside other layers' (us, eight caches in turn, plain
+// and nontemporal: 256 tokens of 2048, rank 512, 32 / 64 / 128 heads 147.4 291 573 and
+// 146.2 286 567, rank 256, 16 / 64 heads 89.5 172.6 and 85.8 168.0).  Smaller ones are
+// as fast with plain loads or faster, above all where groups of heads read the rows
+// again (16 of 2000, rank 512, 32 / 64 / 128 heads 28.7 32.3 45.5 and 30.2 36.0 49.5;
+// 48 of 2000 46.2 71.0 121.8 and 47.6 73.3 123.2; of 700 to 3500 59.1 102.8 and 59.0
+// 103.6; 512 of 300 64.8 120.1 and 64.3 123.5, but rank 256, 16 heads, 36.6 and 35.2).
+constexpr int64_t LD_ONCE = 256 << 20;
+
+template <int NK, int R, bool ONCE>
 __global__ __launch_bounds__(64 * FT_WAVES, 1) void latent_decode_kernel(
     LatentDecodeArgs a) {
   constexpr int VD = R / FT_WAVES;
@@ -70,7 +81,7 @@ __global__ __launch_bounds__(64 * FT_WAVES, 1) void latent_decode_kernel(
                  a.size, R + a.RD, 0, pos + 1};
   ft_f32x16 o[VD / 32];
   float m, l;
-  flash_tiles<NK, R, false, PagedRows, VD, true, true>(
+  flash_tiles<NK, R, false, PagedRows, VD, true, ONCE>(
       rows, span, sc, qf, k_s0, k_s1, nullptr, nullptr, o, m, l, wave * VD);
   if (head >= H) return;
   if (a.parts.nsplit > 1) {
@@ -147,12 +158,12 @@ bool latent_decode(torch::Tensor out, torch::Tensor q_abs,
   }
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
   const dim3 grid(T, groups, nsplit), block(64 * FT_WAVES);
-  if (R == 512)
-    hipLaunchKernelGGL((latent_decode_kernel<576, 512>), grid, block, 0,
-                       stream, a);
-  else
-    hipLaunchKernelGGL((latent_decode_kernel<320, 256>), grid, block, 0,
-                       stream, a);
+  const bool once = T * max_keys * (R + RD) * 2 >= LD_ONCE;
+  auto* kern = R == 512 ? once ? latent_decode_kernel<576, 512, true>
+                               : latent_decode_kernel<576, 512, false>
+               : once   ? latent_decode_kernel<320, 256, true>
+                        : latent_decode_kernel<320, 256, false>;
+  hipLaunchKernelGGL(kern, grid, block, 0, stream, a);
   HIP_CHECK_KERNEL();
   if (nsplit > 1) {
     hipLaunchKernelGGL(flash_merge_kernel, dim3(T * H), dim3(R / 4), 0, stream,

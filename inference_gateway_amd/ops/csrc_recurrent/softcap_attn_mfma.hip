@@ -443,7 +443,13 @@ __global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_prompt_kernel(
 // workgroup) are the 32 query rows of all four waves, which take a quarter of
 // the value dims each; no probabilities are exchanged, and scoring four times
 // costs less than HBM takes to deliver the keys.
-template <int NP>
+// ONCE: nontemporal loads, where one workgroup reads a key head's rows (us, eight
+// caches in turn, plain and so: 32 heads on 8, 16 of 500 tokens 14.4 and 14.5, of 2000
+// 31.2 and 28.1, 48 of 700 to 3500 95.3 and 89.9, 256 of 2048 374 and 335; 32 on 4, the
+// last 512 keys, 48 of 2000 19.6 and 18.2).  Of more heads several do, and find them in
+// the memory side's cache (64 on 1, 48 of 2000 25.0 and 25.7, 128 of 700 24.6 and 25.6,
+// 256 of 2048 79.5 and 80.8).
+template <int NP, bool ONCE>
 __global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_decode_kernel(
     SoftcapArgs a, FlashClose close, FlashParts parts) {
   constexpr int PP = 128, VD = PP / FT_WAVES;
@@ -491,9 +497,8 @@ __global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_decode_kernel(
                  a.N, a.P, pos + 1};
   ft_f32x16 o[VD / 32];
   float m, l;
-  flash_tiles<NP, PP, false, PagedRows, VD, false, true>(
-      rows, span, sc, qf, k_s0, k_s1,
-                                            v_s0, v_s1, o, m, l, wave * VD);
+  flash_tiles<NP, PP, false, PagedRows, VD, false, ONCE>(
+      rows, span, sc, qf, k_s0, k_s1, v_s0, v_s1, o, m, l, wave * VD);
   if (!real) return;
   if (parts.nsplit > 1) {
     flash_store_part<VD>(parts, (int64_t)blockIdx.x * a.H + head, blockIdx.z,
@@ -621,12 +626,12 @@ bool softcap_attention_mfma(torch::Tensor out, torch::Tensor q,
       parts.ml = parts.o + slots * P;
     }
     const dim3 grid(ndec, groups, nsplit), block(64 * FT_WAVES);
-    if (N <= 64)
-      hipLaunchKernelGGL(softcap_decode_kernel<64>, grid, block, 0, stream, a,
-                         close, parts);
-    else
-      hipLaunchKernelGGL(softcap_decode_kernel<128>, grid, block, 0, stream, a,
-                         close, parts);
+    const bool once = H / G <= 32;
+    auto* kern = N <= 64 ? once ? softcap_decode_kernel<64, true>
+                                : softcap_decode_kernel<64, false>
+                 : once  ? softcap_decode_kernel<128, true>
+                         : softcap_decode_kernel<128, false>;
+    hipLaunchKernelGGL(kern, grid, block, 0, stream, a, close, parts);
     HIP_CHECK_KERNEL();
     if (nsplit > 1) {
       hipLaunchKernelGGL(flash_merge_kernel, dim3((int64_t)ndec * H),
