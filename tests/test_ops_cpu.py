@@ -534,3 +534,65 @@ def test_moe_pick_takes():
                  (x, w.clone().requires_grad_()), (x, w.float()),
                  (x[:, :60], w[:, :60].contiguous())):
         assert not takes(*args)
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,silu,want", [
+    (1, 6144, 4096, False, True), (6, 4096, 4096, False, True),
+    (7, 4096, 4096, False, False), (8, 28672, 4096, True, True),
+    (9, 28672, 4096, True, False), (2, 4096, 8192, False, True),
+    (2, 4096, 8704, False, False), (8, 22016, 8192, True, True),
+    # not ahead of the library, no whole lines of 512
+    (6, 8192, 8192, False, False), (2, 4096, 4104, False, False)])
+def test_norm_linear_takes(M, N, K, silu, want):
+    bf = torch.bfloat16
+    d, r = torch.empty(M, K, dtype=bf), torch.empty(M, K, dtype=bf)
+    nw, w = torch.empty(K, dtype=bf), torch.empty(N, K, dtype=bf)
+    b = torch.empty(N, dtype=bf)
+
+    def takes(d, r, nw, w, b=None):
+        return ops._kernels.norm_linear_takes(d, r, nw, w, b, silu, True)
+
+    assert takes(d, r, nw, w) == takes(None, r, nw, w) == want
+    assert takes(d, r, nw, w, b) == (want and not silu)
+    wide = torch.empty(M, K + 8, dtype=bf)
+
+    def shifted(*shape):
+        n = torch.Size(shape).numel()
+        return torch.empty(n + 1, dtype=bf)[1:].view(shape)
+
+    def grad(t):
+        return t.clone().requires_grad_()
+
+    if M > 1:      # one row is contiguous whatever its stride
+        assert not takes(wide[:, :K], r, nw, w)
+        assert not takes(d, wide[:, :K], nw, w)
+    for args in ((d.float(), r, nw, w), (d[:, :8], r, nw, w), (torch.empty(M + 1, K, dtype=bf), r, nw, w),
+                 (d[None], r, nw, w), (d.to("meta"), r, nw, w),
+                 (shifted(M, K), r, nw, w), (grad(d), r, nw, w),
+                 (d, r.float(), nw, w),
+                 (d, r[0], nw, w), (d, shifted(M, K), nw, w), (d, grad(r), nw, w),
+                 (d, r, nw.float(), w), (d, r, nw[:8], w), (d, r, nw[None], w),
+                 (d, r, torch.empty(2 * K, dtype=bf)[::2], w),
+                 (d, r, shifted(K), w), (d, r, nw.to("meta"), w),
+                 (d, r, grad(nw), w), (d, r, nw, w.float()),
+                 (d, r, nw, w[::2]), (d, r, nw, w[:, :K - 8].contiguous()),
+                 (d, r, nw, grad(w)), (d, r, nw, w, b[:4]),
+                 (d, r, nw, w, b.float()), (d, r, nw, w, grad(b))):
+        assert not takes(*args)
+
+
+def test_norm_linear_is_its_parts():
+    g = torch.Generator().manual_seed(0)
+    d, r = torch.randn(2, 3, 24, generator=g)
+    nw, w = torch.randn(24, generator=g), torch.randn(16, 24, generator=g)
+    b, gu = torch.randn(16, generator=g), torch.randn(32, 24, generator=g)
+    x, want = ops.fused_add_rmsnorm(d.clone(), r.clone(), nw, 1e-5)
+    y, res = ops.norm_linear(d.clone(), r.clone(), nw, 1e-5, w, b)
+    assert torch.equal(y, ops.linear(x, w, b)) and torch.equal(res, want)
+    y, res = ops.norm_linear(d.clone(), r.clone(), nw, 1e-5, gu, silu=True)
+    assert torch.equal(y, ops.linear_silu_mul(x, gu)) and torch.equal(res, want)
+    kept = r.clone()
+    y, res = ops.norm_linear(None, r, nw, 1e-5, w)
+    assert torch.equal(y, ops.linear(ops.rmsnorm(r, nw, 1e-5), w))
+    assert torch.equal(res, kept)
