@@ -25,9 +25,14 @@ from ..config import ModelConfig
 from .batch import ForwardBatch
 
 
-# rows whose products norm for themselves (ops.norm_linear); from seven on the
-# products come in parts that the norm adds (ops.linear_add_rmsnorm)
-FEW_ROWS = 6
+# Rows whose products norm for themselves (ops.norm_linear).  Every workgroup does
+# so, which from four rows on takes longer than a launch of the norm's own (us, norm
+# and product, apart and as one, K = 4096: 1 / 2 / 3 / 4 / 5 rows of 6144 outputs 12.0
+# 13.0 14.0 15.0 16.5 and 10.7 12.9 15.0 16.8 19.8, of 28672 as SwiGLU 39.8 40.3 40.5
+# 41.2 42.4 and 37.8 39.1 40.5 42.4 47.9; steps of four such layers, 700 tokens each, 3 /
+# 4 / 6 sequences 583.9 604.4 650.8 and 582.1 610.8 675.2).  From seven on products may
+# come in parts that the norm adds (ops.linear_add_rmsnorm).
+FEW_ROWS = 3
 
 
 def _seed(name: str) -> int:

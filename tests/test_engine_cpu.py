@@ -1636,3 +1636,17 @@ def test_graph_padding_rows_write_nothing():
         assert fb.slot_mapping.tolist() == [9 * 16 + 5, 7 * 16 + 1,
                                             -1, -1, -1][:bucket]
         assert fb.ctx_lens.tolist() == [6, 18, 1, 1, 1][:bucket]
+
+
+@pytest.mark.parametrize("rows,inside", [(1, True), (3, True), (4, False),
+                                         (6, False), (7, False)])
+def test_llama_rows_that_norm_inside_the_product(rows, inside, monkeypatch):
+    """The norm runs inside the product that follows it where that is the faster
+    way, up to three rows."""
+    from inference_gateway_amd import ops
+
+    eng, seen, real = _engine(), [], ops.norm_linear
+    monkeypatch.setattr(ops, "norm_linear",
+                        lambda *a, **kw: seen.append(1) or real(*a, **kw))
+    eng.model(_prompt_batch(eng, rows), eng.kv_caches)
+    assert len(seen) == (2 * len(eng.model.layers) if inside else 0)
