@@ -144,7 +144,7 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
     int max_blocks, int nkv, float scale, int q_rs,
     float* __restrict__ part_o,   // [B, NQ, nsplit, HD] when nsplit > 1
     float* __restrict__ part_ml,  // [B, NQ, nsplit, 2]: maximum (log2), sum
-    int nsplit, int min_blocks, DecodeRope rope) {
+    int nsplit, int min_blocks, int once_ctx, DecodeRope rope) {
   // q_rs: q row stride in elements (q may be a view into the fused QKV
   // GEMM output — no .contiguous() copy on the decode hot path)
   constexpr int HD = 128, BS = 16, PAGE = BS * HD;  // tokens, entries of a page
@@ -424,7 +424,7 @@ __global__ __launch_bounds__(NWAVES* WAVE_SIZE, 2) void paged_attn_decode_kernel
     }
   };
   if (wave < pairs) {
-    if ((int64_t)ctx * gridDim.y * nkv >= PD_ONCE) walk(std::true_type{});
+    if (ctx >= once_ctx) walk(std::true_type{});   // PD_ONCE
     else walk(std::false_type{});
   }
   l = pd_sum(l);
@@ -578,6 +578,7 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
     part_o = part.data_ptr<float>();
     part_ml = part_o + n * HD;
   }
+  const int once_ctx = (int)((PD_ONCE + whole - 1) / whole);
   auto launch = [&](auto waves_) {
     constexpr int NWAVES = decltype(waves_)::value;
     auto kern = rope ? paged_attn_decode_kernel<G, NWAVES, true>
@@ -590,7 +591,7 @@ static void launch_decode(torch::Tensor& out, const torch::Tensor& q,
                        (const int32_t*)block_table.data_ptr(),
                        (const int32_t*)ctx_lens.data_ptr(), max_blocks, nkv,
                        scale, (int)q.stride(0), part_o, part_ml, nsplit,
-                       min_blocks, rope ? *rope : DecodeRope{});
+                       min_blocks, once_ctx, rope ? *rope : DecodeRope{});
   };
   // Four waves a workgroup, but two where one or two query heads share a key head and
   // the chip is filled many times over: the bytes of a short context are few for its
