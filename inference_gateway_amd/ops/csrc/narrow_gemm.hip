@@ -92,6 +92,15 @@ int64_t wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm) {
   return M >= least && M <= most ? wide_split(M, N, K) : 0;
 }
 
+// W from this many entries on is read by nontemporal loads where one patch of tiles
+// has all rows (us, plain and so: 8192 x 28672, 65 / 256 / 512 rows 105.3 148.6 201
+// and 88.0 119.5 187.5; 4096 x 14336, 65 / 128 rows 35.2 39.4 and 30.4 36.4, most of it
+// the turned K, 256 rows 47.5 and 48.6; 12288 x 4096, 128 / 256 rows 34.7 41.7 and 33.6
+// 42.0).  Less of it is slower so: 4096 x 4096, 65 / 128 / 256 rows 15.4 17.6 21.3 and
+// 16.2 19.2 25.5; 7680 x 5120, 128 / 256 rows 27.1 38.4 and 29.8 39.9; 4096 x 8192 25.0
+// 32.1 and 27.0 32.6.
+constexpr int64_t SPLIT_ONCE = 48 << 20;
+
 // The sums [S, M, N] of the parts that wide_split says.
 torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
                           int64_t tile, int64_t S) {
@@ -113,15 +122,16 @@ torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
   const WideArgs a{nullptr, (const uint16_t*)x.data_ptr(),
                    (const uint16_t*)w.data_ptr(), (int)M, (int)N, (int)K,
                    x.stride(0), nullptr, 0, part.data_ptr<float>(), (int)S};
-  // nontemporal where one patch of tiles has all rows (8192 x 28672, 65 / 256 / 1024
-  // rows 107 154 347 and 91 131 337)
+  const bool once = N * K >= SPLIT_ONCE;
 #define LAUNCH_SPLIT_AS(...)                                                  \
   hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__>), dim3(WG_BLOCKS),        \
                      dim3(256), 0, stream, a)
 #define LAUNCH_SPLIT(MT, NT)                                                  \
   case MT * 16 + NT:                                                          \
-    if (M <= 4 * 32 * MT) LAUNCH_SPLIT_AS(MT, NT, 0, false, true, true);      \
-    else LAUNCH_SPLIT_AS(MT, NT, 0, false, true, false);                      \
+    if (once && M <= 4 * 32 * MT)                                             \
+      LAUNCH_SPLIT_AS(MT, NT, 0, false, true, true);                          \
+    else                                                                      \
+      LAUNCH_SPLIT_AS(MT, NT, 0, false, true, false);                         \
     break
   switch (tile) {
     LAUNCH_SPLIT(3, 4);
