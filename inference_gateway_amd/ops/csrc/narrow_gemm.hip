@@ -15,11 +15,13 @@ bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu);
 
 // Products of rows that leave the chip idle, K in parts.
 //
-// Tiles with a part of K each, their fp32 sums to memory, and a
-// second kernel to add them (with the residual and the norm behind it where there is
-// one).  wide_split picks the tile and the parts by what they cost: rounds of 256
-// items at `step` us a K step of 64, against W from HBM, and the sums' way to memory and back.  Of 768 measured pairs of a tile and parts the
-// model is off by 4 % on average, and its choice is 2 % behind the best.
+// Tiles with a part of K each, their fp32 sums to memory, and a second kernel to add
+// them (with the residual and the norm behind it where there is one).  wide_split picks
+// the tile and the parts by what they cost: rounds of 256 items at `step` us a K step of
+// 64, against W from HBM, and the sums' way to memory and back.  Of 1044 measured pairs
+// of a tile and parts the model is off by 12 % on average (10 % too low: it leaves out
+// what a launch costs whatever its size), and its choice is 1 % behind the best, 7 % at
+// worst.
 struct SplitTile {
   int MT, NT;
   double step;
@@ -58,22 +60,27 @@ int64_t wide_split(int64_t M, int64_t N, int64_t K) {
   return best;
 }
 
-// What wide_split says where that is ahead of the library, else 0; norm: where the norm that follows adds the
-// parts, of the library and fused_add_rmsnorm.  Measured at 19 sizes of W by 16 of
-// 65 to 2600 rows (us, library and here; then with the norm).  Over a long K the
-// library's tiles are few: 4096 x 14336, 65 / 128 / 256 / 512 / 1024 / 2033 rows 50.6
-// 76.5 63.8 90.9 134 204 and 36.1 38.9 49.3 65.7 108 185; 5120 x 17920, 65 / 256 / 1024
-// 148 222 249 and 45.8 65.1 158, but 2033 rows 291 and 320; 8192 x 28672, 512 / 640
-// rows 312 260 and 195 289.  Of squarer W the parts' way to memory weighs more: 4096 x
-// 4096, 128 / 256 / 512 / 1024 / 1600 rows 24.0 22.4 30.9 42.1 55.6 and 18.0 21.8 30.7
-// 43.4 66.9 (with the norm 27.2 25.9 36.0 48.9 65.4 and 19.1 23.1 32.6 46.1 70.2), 5120
-// x 5120, 256 / 640 / 1024 rows 50.8 51.3 62.7 and 30.7 47.5 60.7, 7680 x 5120, 128 /
-// 512 / 640 rows 34.9 52.1 58.0 and 28.0 51.0 63.6, 6144 x 4096, 128 / 160 / 200 rows
-// 26.5 29.1 26.5 and 23.8 26.1 30.0, 8192 x 8192, 65 / 128 rows 38.9 51.8 and 43.6
-// 46.6.  Small W and a short K pay for the second launch: 1024 x 4096, 128 rows, 10.3
-// and 11.9, 4096 x 2048 13.1 and 15.4, as do wide ones: 16384 x 4096 40.3 and 46.9.
+// What wide_split says where that is ahead of the library, else 0; norm: where the
+// norm that follows adds the parts, of the library and fused_add_rmsnorm.  Measured at
+// 29 sizes of W by 24 of 65 to 2048 rows (us, library and here; then with the norm).
+// Over a long K the library's tiles are few: 4096 x 14336, 65 / 128 / 256 / 512 / 1024 /
+// 2033 rows 47.7 75.0 61.2 88.2 130 205 and 30.3 37.3 48.2 61.9 108 181; 5120 x 17920,
+// 65 / 256 / 1024 rows 145 220 246 and 42.9 60.8 156, but 2033 rows 290 and 311; 8192 x
+// 28672, 512 / 640 rows 312 265 and 183 271.  Of squarer W the parts' way to memory
+// weighs more: 4096 x 4096, 128 / 256 / 512 / 1024 / 1600 rows 24.2 22.4 29.2 40.7 54.0
+// and 17.8 21.3 29.7 41.7 64.1 (with the norm 27.3 25.9 33.8 46.9 62.6 and 19.0 22.5 31.6
+// 44.3 68.1), 5120 x 5120, 256 / 640 / 1024 rows 49.6 50.4 62.1 and 29.0 45.7 58.9, 7680
+// x 5120, 128 / 512 / 640 rows 33.4 52.1 58.2 and 27.3 50.1 60.1, 6144 x 4096, 128 / 160
+// / 200 rows 25.4 27.8 25.4 and 21.0 23.7 25.2, 8192 x 8192, 128 rows 47.4 and 36.1 (65
+// rows, which the line leaves to the library, 36.9 and 32.8).  Small W and a short K pay
+// for the second launch: 1024 x 4096, 128 rows, 11.8 and 12.2, 4096 x 2048 14.6 and 15.4,
+// as do wide ones: 16384 x 4096 36.8 and 38.1.  Without the norm the library is ahead
+// where its tiles come out even: 5120 x 4096, 65 / 80 rows 16.5 16.9 and 18.3 17.4; 9216
+// x 6144, 257 / 384 rows 49.9 60.0 and 59.8 66.3, 10240 x 5120, 257 rows 43.6 and 49.9.
 int64_t wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm) {
-  const int64_t least = N > 7680 && K < 2 * N ? 128 : 65;
+  const int64_t least = N > 7680 && K < 2 * N            ? 128
+                        : !norm && N <= 5120 && K < N ? 81
+                                                      : 65;
   int64_t most;
   if (norm) {
     if (K < 3584 || N * K < (int64_t)12 << 20 || N > 16384) return 0;
@@ -85,7 +92,7 @@ int64_t wide_split_ahead(int64_t M, int64_t N, int64_t K, bool norm) {
     if (K < 4096 || N * K < (int64_t)16 << 20 || N < 2048 || N > 10240) return 0;
     most = K >= 3 * N   ? N > 5120 ? 512 : N > 4096 ? 1600 : 2048
            : K >= 2 * N ? N > 5120 ? 512 : 1300
-           : K >= 5120  ? 512
+           : K >= 5120  ? N > 7680 && K < 8192 ? 256 : 512
            : K >= N     ? 256
                         : 160;
   }

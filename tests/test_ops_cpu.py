@@ -378,6 +378,20 @@ def test_narrow_lines(M, N, K, gated, tile):
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,linear,norm", [
+    # where the library's own tiles come out even
+    (80, 5120, 4096, 0, 5), (81, 5120, 4096, 5, 5), (65, 5376, 4608, 5, 5),
+    (65, 5120, 5120, 5, 5), (256, 9216, 6144, 5, 5), (257, 9216, 6144, 0, 5),
+    (257, 10240, 5120, 0, 5), (257, 7680, 5120, 5, 5), (257, 10240, 8192, 5, 5)])
+def test_split_lines_of_the_product_alone(M, N, K, linear, norm):
+    bf = torch.bfloat16
+    x, w = torch.empty(M, K, dtype=bf), torch.empty(N, K, dtype=bf)
+    r, nw = torch.empty(M, N, dtype=bf), torch.empty(N, dtype=bf)
+    assert ops._kernels.product_kernel(x, w, None, False, True) == linear
+    assert ops._kernels.linear_norm_takes(x, w, r, nw, True) == norm
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 @pytest.mark.parametrize("M,N,K,gated,want", [
     # each kernel, narrow_gemm beside those that it is asked before
     (5, 4096, 4096, False, 1), (8, 28672, 4096, True, 1),
