@@ -688,6 +688,21 @@ void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   if (part.defined()) sum_parts(out, part, bias);
 }
 
+// Whether ring_gemm takes a held product whose K is in parts.  It streams W once, but a
+// workgroup's start, with all of x, is longer than that of two halves, and few outputs
+// share it (us, two halves and ring_gemm, 43 and 61 rows or 64: 1024 x 5120 8.9 9.1 and
+// 10.0 10.6, 2560 x 6144 13.4 14.2 and 14.1 15.3, 3072 x 8192 16.5 18.1 and 17.5 18.3,
+// 1536 x 10240 13.0 13.8 and 13.4 14.6; 4096 x 6144 16.0 16.8 and 15.5 17.1, 2048 x 10240
+// 15.0 15.8 and 14.4 15.3, 1024 x 12288 13.9 15.1 and 13.2 13.9, 4096 x 14336 30.2 31.5
+// and 26.3 29.9).
+static bool ring_takes(int64_t M, int64_t N, int64_t K) {
+  const int64_t least = K >= 12288   ? 1024
+                        : K >= 10240 ? 2048
+                        : M <= 48    ? 4096
+                                     : 5120;
+  return M > 32 && N >= least;
+}
+
 // In how many parts held_gemm cuts K (a wave's part is four to eight lines of
 // 64 entries); 0: it cannot.
 int64_t held_splits(int64_t M, int64_t N, int64_t K) {
@@ -695,7 +710,7 @@ int64_t held_splits(int64_t M, int64_t N, int64_t K) {
       K > (1 << 20))
     return 0;
   // four tiles of rows leave registers for six lines, where it can be had so
-  for (const int64_t most : {M > 48 ? 6 : 8, 8})
+  for (const int64_t most : {M > 48 && ring_takes(M, N, K) ? 6 : 8, 8})
     for (int64_t S = 1; S <= 8; ++S)
       if (K % (RG_WAVES * 64 * S) == 0) {
         const int64_t lines = K / (RG_WAVES * 64 * S);
@@ -774,9 +789,8 @@ torch::Tensor held_gemm_parts(const torch::Tensor& out, const torch::Tensor& x,
     hipLaunchKernelGGL((ring_gemm_kernel<P, MT>), dim3(256),                  \
                        dim3(64 * RG_WAVES), 0, stream, a, (int)S);            \
     break
-  if (M > 32 && S > 1 && (M <= 48 || lines <= 6)) {
-    switch ((M > 48 ? 4 : 3) * 16 + lines) {
-      LAUNCH_RING(4, 3);
+  if (S > 1 && ring_takes(M, N, K) && (M <= 48 || lines <= 6)) {
+    switch ((M > 48 ? 4 : 3) * 16 + lines) {   // four lines only of four tiles
       LAUNCH_RING(5, 3);
       LAUNCH_RING(6, 3);
       LAUNCH_RING(7, 3);
