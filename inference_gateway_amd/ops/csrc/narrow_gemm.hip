@@ -175,9 +175,13 @@ torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
 // x 4096 52.6 and 43); 65536 x 2048 and 152064 x 3584, 16 rows 48.7 182.8 and 50.1 179, 32
 // rows 62.7 261 and 50.6 191; 49152 x 6144, 65 / 160 / 256 rows 156 168 203 and 111 114
 // 129; 32768 x 8192 127 140 170 and 90 108 127; 128256 x 8192 426 463 546 and 339 398 467.
-// Of more than 192 rows of a long K the library is ahead where its tiles, 256 wide,
-// fill one round: 65536 x 8192, 200 / 256 rows, 211 237 and 235 243; 57344 x 8192 225 237
-// and 227 236; but 98304 x 8192 396 417 and 344 335.
+// Of more than 128 rows the library is ahead where its tiles, 256 wide, are one round,
+// ours of 192 more, and rows of W do not lie a multiple of 4 KB apart (57344 x 3584, 129 / 160 / 256 rows 90.4
+// 90.0 95.3 and 97.5 100 111; 65536 x 2560 77 77 83 and 83 84 93; but 65536 x 4096 151 138
+// 149 and 107 110 125), of more than 192 also where they do, over a long K or where they
+// leave a part of the round (65536 x 8192, 200 / 256 rows, 211 237 and 235 243; 57344 x
+// 4096, 193 / 256 rows 111 113 and 117 121; but 98304 x 8192, 200 / 256 rows 396 417 and
+// 344 335).
 static constexpr SplitTile two_tiles[] = {
     {2, 4, 0.450}, {2, 5, 0.500}, {2, 8, 0.850}};  // up to 64 rows
 static constexpr SplitTile narrow_tiles[] = {
@@ -217,7 +221,10 @@ int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated) {
   }
   if (!gated && M > 64) {
     const int64_t its = (N + 255) / 256;   // the library's tiles
-    return M > 192 && K > 6144 && its >= WG_BLOCKS * 7 / 8 && its <= WG_BLOCKS ? 0 : best;
+    const bool round = N > 192 * WG_BLOCKS && its <= WG_BLOCKS;
+    const bool even = K % 2048 == 0 &&
+                      (M <= 192 || (K <= 6144 && its > WG_BLOCKS * 15 / 16));
+    return M > 128 && round && !even ? 0 : best;
   }
   if (M > 64)
     for (const auto& c : gated_tiles)

@@ -378,6 +378,21 @@ def test_narrow_lines(M, N, K, gated, tile):
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,tile", [
+    # one round of the library's tiles, rows of W a multiple of 4 KB apart and not
+    (128, 57344, 3584, (4, 8)), (129, 57344, 3584, 0), (256, 65536, 2560, 0),
+    (129, 65536, 4096, (6, 4)), (256, 65536, 4096, (8, 4)),
+    (192, 57344, 4096, (6, 4)), (193, 57344, 4096, 0), (193, 65536, 6144, (8, 4)),
+    (129, 49152, 3584, (6, 6)), (129, 49160, 3584, 0),
+    (256, 65536, 3584, 0), (256, 65544, 3584, (8, 6))])
+def test_narrow_lines_of_one_round(M, N, K, tile):
+    bf = torch.bfloat16
+    x, w = torch.empty(M, K, dtype=bf), torch.empty(N, K, dtype=bf)
+    got = ops._kernels.narrow_takes(x, w, None, False, True)
+    assert got == (tile and tile[0] * 16 + tile[1])
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 @pytest.mark.parametrize("M,N,K,linear,norm", [
     # where the library's own tiles come out even
     (80, 5120, 4096, 0, 5), (81, 5120, 4096, 5, 5), (65, 5376, 4608, 5, 5),
