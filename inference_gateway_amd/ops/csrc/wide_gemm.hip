@@ -156,6 +156,14 @@ int64_t grouped_tile(int64_t rows, int64_t E, int64_t N, bool swiglu) {
   return best;
 }
 
+// From this many entries of W, in rows of 4 KB and more, a grouped product of few rows
+// an expert reads it by nontemporal loads and from turned starts (us, without and so; 2
+// / 64 rows an expert: 8 x 4096 x 2048 as SwiGLU 32.5 37.1 and 26.4 30.1, 8 x 4096 x 4096
+// 58 69 and 49 55).  Smaller W gains nothing (8 x 2048 x 2048 24.0 27.1 and 23.5 26.6; 4 x
+// 4096 x 1024, 13.3 15.1 and 14.2 15.9), nor do shorter rows (64 x 1024 x 1024 as SwiGLU, 8
+// rows, 28.8 and 32.1, 8 x 8192 x 1024 29.1 and 32.4).
+constexpr int64_t GROUPED_ONCE = 48 << 20;
+
 // out[r] = x[r] W_e^T for the rows start[e] .. start[e + 1] - 1 of every expert
 // e, w [E, N or 2 N, K]; rows past start[E] are left alone.
 void grouped_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
@@ -184,16 +192,17 @@ void grouped_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   // nontemporal W where half a patch of tiles has an expert's rows: three prompts of
   // 560 to 700 tokens on eight experts of 14336 x 4096, a step 1442 and 1330 us; with 790
   // rows an expert, some of which have more than a patch, 2484 and 2522
+  const bool once = K >= 2048 && w.numel() >= GROUPED_ONCE;
 #define LAUNCH_GROUPED_AS(...)                                                \
   hipLaunchKernelGGL((wide_gemm_kernel<__VA_ARGS__>), dim3(WG_BLOCKS),        \
                      dim3(256), 0, stream, a)
 #define LAUNCH_GROUPED(MT, NT)                                                \
   case MT * 16 + NT:                                                          \
-    if (swiglu && R <= E * 2 * 32 * MT)                                       \
+    if (swiglu && once && R <= E * 2 * 32 * MT)                               \
       LAUNCH_GROUPED_AS(MT, NT, 1, true, false, true);                        \
     else if (swiglu)                                                          \
       LAUNCH_GROUPED_AS(MT, NT, 1, true, false, false);                       \
-    else if (R <= E * 2 * 32 * MT)                                            \
+    else if (once && R <= E * 2 * 32 * MT)                                    \
       LAUNCH_GROUPED_AS(MT, NT, 0, true, false, true);                        \
     else                                                                      \
       LAUNCH_GROUPED_AS(MT, NT, 0, true, false, false);                       \
