@@ -17,13 +17,14 @@
 // 4096, 16 rows, before the lines were turned: 52.0 us, with the starts apart
 // 48.0).
 //
-// W is read once a step, and by nontemporal loads: others leave it in the memory
-// side's cache, which has no room for a model, and that costs the memory a ninth of
-// its rate (loads alone, 128256 rows of 8 KB in this pattern, 183 and 157 us, 28672
-// of them 45.0 and 39.4; a row at a time, 1 KB a load, 168 and 150).  Of 49 rows and
-// more the kernel waits for other things, and between the others of a step plain
-// loads are as good (28672 x 4096 as SwiGLU 47.0 and 47.3 us, 43 rows 44.3 and 42.3;
-// 128256 x 4096, 61 rows, 194 and 199).
+// W is read once a step, and in rows of 4 KB and more by nontemporal loads (RG_ONCE):
+// others leave it in the memory side's cache, which has no room for a model, and that
+// costs the memory a ninth of its rate (loads alone, 128256 rows of 8 KB in this pattern,
+// 183 and 157 us, 28672 of them 45.0 and 39.4; a row at a time, 1 KB a load, 168 and 150).
+// Shorter rows are slower so (28672 x 1024 as SwiGLU, 9 / 17 / 33 rows, plain and so, 12.9
+// 13.4 13.8 and 13.9 14.0 14.2).  Of 49 rows and more the kernel waits for other things,
+// and between the others of a step plain loads are as good (28672 x 4096 as SwiGLU 47.0
+// and 47.3 us, 43 rows 44.3 and 42.3; 128256 x 4096, 61 rows, 194 and 199).
 //
 // GATE: a wave's 16 rows are eight gate rows and the up rows of the same outputs,
 // and the result is act(gate) * up of the fp32 sums.
@@ -51,6 +52,7 @@ typedef __attribute__((ext_vector_type(4))) float rg_f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t rg_u32x4;
 
 constexpr int RG_BK = 256;     // entries of a K slice
+constexpr int64_t RG_ONCE = 2048;   // entries of a row of W, nontemporal from there on
 constexpr int RG_WAVES = 8;
 
 struct RowsArgs {
@@ -63,7 +65,7 @@ struct RowsArgs {
   int64_t x_rs;
 };
 
-template <int MT, int GATE>
+template <int MT, int GATE, bool ONCE>
 __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
     RowsArgs a) {
   __shared__ __attribute__((aligned(1024))) uint16_t xs[3][MT * 16 * RG_BK];
@@ -115,7 +117,7 @@ __global__ __launch_bounds__(64 * RG_WAVES, 2) void rows_gemm_kernel(
     for (int j = 0; j < 8; ++j) {
       const auto* p = reinterpret_cast<const rg_u32x4*>(
           (j & 1 ? w_hi : w_lo) + k + ((j / 2 + wave) & 3) * 64);
-      wr[j] = MT < 4 ? __builtin_nontemporal_load(p) : *p;
+      wr[j] = ONCE ? __builtin_nontemporal_load(p) : *p;
     }
     asm volatile("" ::: "memory");
   };
@@ -661,21 +663,30 @@ torch::Tensor rows_gemm_parts(const torch::Tensor& out, const torch::Tensor& x,
              bias.has_value() ? (const uint16_t*)bias->data_ptr() : nullptr,
              (int)M, (int)N, (int)K, x.stride(0)};
   const dim3 grid(blocks, S);
-#define LAUNCH_RG(MT, SW)                                                    \
-  hipLaunchKernelGGL((rows_gemm_kernel<MT, SW>), grid, dim3(64 * RG_WAVES),  \
-                     0, stream, a)
+  const bool once = K >= RG_ONCE;
+#define LAUNCH_RG(...)                                                       \
+  hipLaunchKernelGGL((rows_gemm_kernel<__VA_ARGS__>), grid,                  \
+                     dim3(64 * RG_WAVES), 0, stream, a)
+#define LAUNCH_RG_G(MT, ONCE)                                                \
+  do {                                                                       \
+    if (gate == 2) LAUNCH_RG(MT, 2, ONCE);                                   \
+    else if (gate == 1) LAUNCH_RG(MT, 1, ONCE);                              \
+    else LAUNCH_RG(MT, 0, ONCE);                                             \
+  } while (0)
 #define LAUNCH_RG_M(MT)                                                      \
   do {                                                                       \
-    if (gate == 2) LAUNCH_RG(MT, 2);                                         \
-    else if (gate == 1) LAUNCH_RG(MT, 1);                                    \
-    else LAUNCH_RG(MT, 0);                                                   \
+    if (once) LAUNCH_RG_G(MT, true);                                         \
+    else LAUNCH_RG_G(MT, false);                                             \
   } while (0)
-  if (M <= 16 && gate == 2) LAUNCH_RG(1, 2);   // with a gate only
-  else if (M <= 16) LAUNCH_RG(1, 1);
+  if (M <= 16 && gate == 2 && once) LAUNCH_RG(1, 2, true);   // with a gate only
+  else if (M <= 16 && gate == 2) LAUNCH_RG(1, 2, false);
+  else if (M <= 16 && once) LAUNCH_RG(1, 1, true);
+  else if (M <= 16) LAUNCH_RG(1, 1, false);
   else if (M <= 32) LAUNCH_RG_M(2);
   else if (M <= 48) LAUNCH_RG_M(3);
-  else LAUNCH_RG_M(4);
+  else LAUNCH_RG_G(4, false);
 #undef LAUNCH_RG_M
+#undef LAUNCH_RG_G
 #undef LAUNCH_RG
   HIP_CHECK_KERNEL();
   return part;
