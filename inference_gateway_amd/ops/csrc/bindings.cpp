@@ -83,7 +83,7 @@ c10::optional<torch::Tensor> linear_add_rmsnorm(const torch::Tensor& x,
 void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias);
 int64_t product_kernel(const torch::Tensor& x, const torch::Tensor& w,
-                       const c10::optional<torch::Tensor>& bias, bool swiglu,
+                       const c10::optional<torch::Tensor>& bias, int64_t gate,
                        bool anywhere);
 int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
                        const c10::optional<torch::Tensor>& bias, bool swiglu,
@@ -188,11 +188,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("wide_gemm_tile", &igw::wide_gemm_tile,
         "its tile (16 MT + NT) for a product; 0: not ahead of the library");
   m.def("product_kernel", &igw::product_kernel,
-        "what runs x W^T, plain or gated.  0: none of them, 1: gemv, 2: "
+        "what runs x W^T, plain or gated (gate 1 SiLU, 2 GELU).  0: none of "
+        "them, 1: gemv, 2: "
         "rows_gemm, 3: wide_gemm, 4: held_gemm, 5: wide_gemm with K in parts, "
         "6: narrow_gemm");
   m.def("few_rows_takes", &igw::few_rows_takes,
-        "as product_kernel, were narrow_gemm not there");
+        "as product_kernel of gate 0 or 1, were narrow_gemm not there");
   m.def("moe_few", &igw::moe_few, "SwiGLU experts of a few tokens");
   m.def("moe_rows_takes", &igw::moe_rows_takes,
         "whether the grouped products take a step");

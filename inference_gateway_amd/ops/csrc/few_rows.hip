@@ -108,22 +108,42 @@ struct Route {
   int64_t kernel = 0, how = 0;
 };
 
+// Where GELU inside is ahead of the product (gemv, held_gemm or the library's) and
+// gated_act.  SwiGLU's lines are against the library and silu_mul (us, apart and inside:
+// gemv, 3 rows 64128 x 512 18.3 and 21.8, 4 rows 68736 x 512 21.8 and 27.5, 7 rows 15360 x
+// 2560 17.9 and 23.1, 8 rows 14592 x 3072 19.2 and 24.9, 3712 x 2560 8.6 and 9.9, but
+// 28672 x 8192 in 0.77 of the time; tiles that leave a half of the compute units idle, or
+// of a long K, 8192 x 3584, 440 rows, 42.0 and 49.6, 4096 x 8192, 1000 rows, 83.4 and 94.6,
+// 16384 x 11008, 131 rows, 107 and 181, 32768 x 14336, 288 rows, 279 and 326, but 28672 x
+// 4096, 320 to 3000 rows, in 0.86 to 0.96 of the time).
+static bool gelu_gemv_ahead(int64_t M, int64_t rows, int64_t K) {
+  return M <= 2 || (M <= 6 ? K >= 1024 : rows >= 28672 || K > 4096);
+}
+static bool gelu_wide_ahead(int64_t M, int64_t N, int64_t K, int64_t tile) {
+  const int64_t tm = 32 * (tile >> 4), tn = 16 * (tile & 15);
+  return K <= 8192 && (M + tm - 1) / tm * ((N + tn - 1) / tn) >= 192;
+}
+
 // The kernel of a call, narrow_gemm aside.  0: none of them, 1: gemv, 2: rows_gemm,
 // 3: wide_gemm, 4: held_gemm, 5: wide_gemm with K in parts.  `anywhere`: also off
 // the GPU (the rule alone, nothing is launched).  norm: fused_add_rmsnorm follows.
 static Route route_of(const torch::Tensor& x, const torch::Tensor& w,
-                      const c10::optional<torch::Tensor>& bias, bool swiglu,
+                      const c10::optional<torch::Tensor>& bias, int64_t gate,
                       bool norm) {
+  const bool swiglu = gate != 0;
   const int64_t M = x.size(0), K = x.size(1);
   const int64_t N = swiglu ? w.size(0) / 2 : w.size(0);
   if (M > 64) {
     if (!wide_gemm_fits(x.stride(0), N, K, swiglu)) return {};
     const int64_t tile = bias.has_value() ? 0 : wide_gemm_tile(M, N, K, swiglu);
-    if (tile > 0) return {3, tile};
+    if (tile > 0)
+      return gate != 2 || gelu_wide_ahead(M, N, K, tile) ? Route{3, tile} : Route{};
     const int64_t cut = swiglu ? 0 : wide_split_ahead(M, N, K, norm);
     return cut > 0 ? Route{5, cut} : Route{};
   }
-  if (gemv_fits(M, K, swiglu)) return {gemv_ahead(M, w.size(0), K, swiglu)};
+  if (gemv_fits(M, K, swiglu))
+    return {gemv_ahead(M, w.size(0), K, swiglu) &&
+            (gate != 2 || gelu_gemv_ahead(M, w.size(0), K))};
   if (!swiglu && held_gemm_takes(M, N, K)) return {4};
   const int64_t S = rows_gemm_splits(M, N, K, swiglu);
   return {S > 0 && rows_gemm_ahead(M, S, K, swiglu) ? 2 : 0};
@@ -146,23 +166,23 @@ static int64_t narrow_before(const Route& other, const torch::Tensor& x,
   return narrow_tile(M, N, K, swiglu);
 }
 
-// What runs the call: as above, 6: narrow_gemm.
+// What runs the call: as above, 6: narrow_gemm.  gate: 0 none, 1 SiLU, 2 GELU.
 static Route product_route(const torch::Tensor& x, const torch::Tensor& w,
                            const c10::optional<torch::Tensor>& bias,
-                           bool swiglu, bool anywhere) {
-  if (!call_fits(x, w, bias, swiglu, anywhere)) return {};
-  const Route other = route_of(x, w, bias, swiglu, false);
-  const int64_t tile = narrow_before(other, x, w, bias, swiglu);
+                           int64_t gate, bool anywhere) {
+  if (!call_fits(x, w, bias, gate != 0, anywhere)) return {};
+  const Route other = route_of(x, w, bias, gate, false);
+  const int64_t tile = narrow_before(other, x, w, bias, gate != 0);
   return tile > 0 ? Route{6, tile} : other;
 }
 
 int64_t product_kernel(const torch::Tensor& x, const torch::Tensor& w,
-                       const c10::optional<torch::Tensor>& bias, bool swiglu,
+                       const c10::optional<torch::Tensor>& bias, int64_t gate,
                        bool anywhere) {
-  return product_route(x, w, bias, swiglu, anywhere).kernel;
+  return product_route(x, w, bias, gate, anywhere).kernel;
 }
 
-// As product_kernel, were narrow_gemm not there.
+// As product_kernel of gate 0 or 1, were narrow_gemm not there.
 int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
                        const c10::optional<torch::Tensor>& bias, bool swiglu,
                        bool anywhere) {
@@ -171,7 +191,7 @@ int64_t few_rows_takes(const torch::Tensor& x, const torch::Tensor& w,
              : 0;
 }
 
-// The tile of narrow_gemm for a call that it takes, or 0.
+// The tile of narrow_gemm for a call of gate 0 or 1 that it takes, or 0.
 int64_t narrow_takes(const torch::Tensor& x, const torch::Tensor& w,
                      const c10::optional<torch::Tensor>& bias, bool swiglu,
                      bool anywhere) {
@@ -185,7 +205,7 @@ c10::optional<torch::Tensor> few_rows(const torch::Tensor& x,
                                       const torch::Tensor& w,
                                       const c10::optional<torch::Tensor>& bias,
                                       int64_t gate) {
-  const Route r = product_route(x, w, bias, gate != 0, false);
+  const Route r = product_route(x, w, bias, gate, false);
   if (r.kernel == 0) return c10::nullopt;
   auto out = torch::empty({x.size(0), gate != 0 ? w.size(0) / 2 : w.size(0)},
                           x.options());
@@ -208,7 +228,7 @@ static Route norm_route(const torch::Tensor& x, const torch::Tensor& w,
                         const torch::Tensor& residual,
                         const torch::Tensor& weight, bool anywhere) {
   if (!call_fits(x, w, c10::nullopt, false, anywhere)) return {};
-  const Route r = route_of(x, w, c10::nullopt, false, true);
+  const Route r = route_of(x, w, c10::nullopt, 0, true);
   if (r.kernel != 2 && r.kernel != 4 && r.kernel != 5) return {};
   const int64_t M = x.size(0), N = w.size(0);
   if (!plain_bf16(residual, x.device()) || !plain_bf16(weight, x.device()) ||

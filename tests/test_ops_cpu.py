@@ -441,6 +441,23 @@ def test_product_kernel(M, N, K, gated, want):
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,silu,gelu", [
+    # a few rows: short K, and seven and eight rows of fewer outputs
+    (2, 65536, 512, 1, 1), (3, 65536, 1024, 1, 1), (3, 8192, 768, 1, 0),
+    (7, 28672, 2048, 1, 1), (7, 24064, 2048, 1, 0), (8, 24064, 4608, 1, 1),
+    (9, 28672, 4096, 2, 2), (64, 28672, 4096, 6, 6),
+    # tiles of less than three quarters of the compute units, a long K
+    (440, 8192, 3584, 3, 0), (700, 8192, 4096, 3, 3), (1000, 4096, 8192, 3, 0),
+    (320, 28672, 4096, 3, 3), (6000, 28672, 4096, 3, 3),
+    (512, 28672, 8192, 3, 3), (512, 28672, 8320, 3, 0), (256, 28672, 4096, 6, 6)])
+def test_gelu_lines(M, N, K, silu, gelu):
+    x = torch.empty(M, K, dtype=torch.bfloat16)
+    w = torch.empty(N, K, dtype=torch.bfloat16)
+    for gate, want in ((1, silu), (2, gelu)):
+        assert ops._kernels.product_kernel(x, w, None, gate, True) == want
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 def test_wide_split_parts():
     """Every part of K has the three pairs of steps that the kernel needs."""
     tiles = set()
