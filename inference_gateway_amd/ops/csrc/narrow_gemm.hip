@@ -12,6 +12,7 @@
 namespace igw {
 
 bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu);
+int64_t wide_gemm_tile(int64_t M, int64_t N, int64_t K, bool swiglu);
 
 // Products of rows that leave the chip idle, K in parts.
 //
@@ -194,6 +195,23 @@ static constexpr SplitTile few_wide_tiles[] = {
 static constexpr SplitTile gated_tiles[] = {
     {4, 8, 0.864}, {6, 8, 1.069}, {8, 6, 1.049}, {8, 7, 1.220}, {8, 8, 1.387}};
 
+// Gated products of a K above 2048 that the library would have else (wide_gemm_tile does
+// not take them): it is ahead where the second row of tiles is filled to a third, or the
+// third to a half, as W is read again for it (us, library with silu_mul and here: 16384 x
+// 5120, 107 rows, 47.7 and 53.4, 12288 x 8192 59.4 and 64.9; 8192 x 5120, 200 rows, 40.0
+// and 44.3, 12288 x 6144, 239 rows, 64.0 and 68.8; but 16384 x 6144, whose rows of W lie a
+// multiple of 4 KB apart, 107 rows, 0.98 of the library's time, and 10240 x 5120, whose
+// tiles fill a round, 193 and 239 rows, 0.93 and 0.89).
+static bool mostly_empty(int64_t M, int64_t N, int64_t K, int64_t tile,
+                         int64_t tiles) {
+  const int64_t tm = 32 * (tile >> 4), last = (M - 1) % tm + 1;
+  if (K <= 2048) return false;
+  if (M > tm && M <= 2 * tm)
+    return 3 * last <= tm && (K % 2048 != 0 || N < 8192);
+  return M > 2 * tm && M <= 3 * tm && 2 * last <= tm &&
+         tiles < WG_BLOCKS * 15 / 16;
+}
+
 // 16 MT + NT of the tile, or 0.
 int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated) {
   if (M < 7 || M > (gated ? 384 : 256) || N < 8 || N % 8 != 0 ||
@@ -229,6 +247,8 @@ int64_t narrow_tile(int64_t M, int64_t N, int64_t K, bool gated) {
   if (M > 64)
     for (const auto& c : gated_tiles)
       if (price(c, &items) <= least) return 0;
+  if (M > 64 && wide_gemm_tile(M, N, K, true) == 0 && mostly_empty(M, N, K, best, tiles))
+    return 0;
   return tiles >= WG_BLOCKS * (gated ? 6 : 7) / 8 ? best : 0;
 }
 

@@ -441,6 +441,21 @@ def test_product_kernel(M, N, K, gated, want):
 
 
 @pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
+@pytest.mark.parametrize("M,N,K,tile", [
+    # the second row of tiles filled to a third, the third to a half
+    (128, 16384, 5120, 0), (129, 16384, 5120, (3, 4)), (128, 16384, 2048, (3, 4)),
+    (128, 16384, 6144, (3, 4)), (128, 14336, 6144, 0), (129, 14336, 6144, (3, 4)),
+    (240, 8192, 4096, 0), (241, 8192, 4096, (3, 4)), (200, 8192, 2048, (3, 4)),
+    (200, 10240, 5120, (3, 4)), (240, 12288, 4096, 0), (241, 12288, 4096, (3, 5)),
+    (107, 24576, 5120, (4, 4)), (200, 16384, 5120, (4, 4))])
+def test_narrow_lines_of_part_tiles(M, N, K, tile):
+    x = torch.empty(M, K, dtype=torch.bfloat16)
+    w = torch.empty(N, K, dtype=torch.bfloat16)
+    got = ops._kernels.narrow_takes(x, w, None, True, True)
+    assert got == (tile and tile[0] * 16 + tile[1])
+
+
+@pytest.mark.skipif(not ops.HAS_KERNELS, reason="extension not built")
 @pytest.mark.parametrize("M,N,K,silu,gelu", [
     # a few rows: short K, and seven and eight rows of fewer outputs
     (2, 65536, 512, 1, 1), (3, 65536, 1024, 1, 1), (3, 8192, 768, 1, 0),
