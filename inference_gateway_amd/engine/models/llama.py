@@ -192,12 +192,14 @@ class LlamaLayer(nn.Module):
     def opens(self) -> bool:
         """Whether normed and few_rows, which call none of the modules that they
         stand for, do what calls of them would."""
-        attn, mlp = self.attn, self.mlp
+        attn, mlp = self._modules.get("attn"), self._modules.get("mlp")
         return (calls_plainly(self, LlamaLayer)
                 and calls_plainly(attn, LlamaAttention)
-                and calls_plainly(attn.o_proj, RowParallelLinear)
                 and calls_plainly(mlp, LlamaMLP)
-                and calls_plainly(mlp.down_proj, RowParallelLinear))
+                and calls_plainly(attn._modules.get("o_proj"),
+                                  RowParallelLinear)
+                and calls_plainly(mlp._modules.get("down_proj"),
+                                  RowParallelLinear))
 
     def normed(self, x, residual, fb, kv_cache, cos_sin, next_norm_w):
         """x: the residual normed for this layer; returns it normed for what

@@ -30,13 +30,12 @@ def _init_weight(shape, device, dtype, seed: int) -> torch.Tensor:
     return w.to(dtype)
 
 
-def calls_plainly(m: nn.Module, cls) -> bool:
+def calls_plainly(m, cls) -> bool:
     """Whether a call of m is cls.forward and nothing else (no hook, no other
     class, no compiled call), so that its caller may do the work itself."""
-    own = m.__dict__
-    return (type(m) is cls and "forward" not in own
-            and not (own["_forward_hooks"] or own["_forward_pre_hooks"]
-                     or own["_backward_hooks"] or own["_backward_pre_hooks"])
+    return (type(m) is cls and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks
+                     or m._backward_hooks or m._backward_pre_hooks)
             and m._compiled_call_impl is None and not _has_any_global_hook())
 
 
