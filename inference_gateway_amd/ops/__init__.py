@@ -303,7 +303,8 @@ def norm_linear(delta, residual: torch.Tensor, weight: torch.Tensor,
                 eps: float, w: torch.Tensor, bias=None, silu: bool = False):
     """linear (silu: linear_silu_mul) of rmsnorm(residual + delta) * weight;
     delta may be None.  Returns the product and residual + delta, which may or may
-    not be residual's memory.  A few rows run as one kernel."""
+    not be residual's memory.  A few rows run as one kernel, which is ahead of the
+    two up to three rows (one row of 4096 x 6144 10.7 and 12.0 us, four 16.8 and 15.0)."""
     if (residual.is_cuda and HAS_KERNELS
             and not torch.compiler.is_compiling()
             and not has_torch_function_variadic(residual, weight, w)):
@@ -842,7 +843,8 @@ def gated_act(gate_up, mode: int, limit: float = 0.0, alpha: float = 1.0):
 def linear_gated_act(x: torch.Tensor, w: torch.Tensor, mode: int,
                      limit: float = 0.0, alpha: float = 1.0) -> torch.Tensor:
     """gated_act of x W^T, w = [Wg; Wu]: one kernel for bf16 rows where it is
-    ahead and mode is SiLU or GELU, else the product and gated_act."""
+    ahead and mode is SiLU or GELU, each by its own lines, else the product and
+    gated_act."""
     gate = {GATED_ACT_SILU: 1, GATED_ACT_GELU: 2}.get(mode)
     out = None if gate is None else _own_product(x, w, None, gate)
     return gated_act(linear(x, w), mode, limit, alpha) if out is None else out

@@ -1,7 +1,8 @@
 // Host side of ops.linear, ops.linear_silu_mul, ops.linear_gated_act, ops.moe_few
 // and ops.moe_rows: which calls the kernels for a few rows of x (gemv.hip), for
 // tens of them (rows_gemm and held_gemm in rows_gemm.hip) and for hundreds and
-// thousands of them (narrow_gemm.hip, wide_gemm.hip) take.
+// thousands of them (narrow_gemm.hip, wide_gemm.hip) take.  product_route is the
+// rule that the launch goes by.
 //
 // What they are handed is a pointer, so the tensors have to be what they seem:
 // plain dense bf16 on one GPU, in a call that nothing but the product has to

@@ -120,8 +120,9 @@ void moe_route(torch::Tensor weights, torch::Tensor dst,
 
 // The router's product of a few tokens with the choice of their experts: a workgroup
 // per token, a wave per expert, logits rounded to bf16 like those of a product of its
-// own.  Bound by latency: 5 tokens of 8 experts x 4096 take
-// 5.8 us; the library's product, the conversion and moe_route took 19.7.
+// own, but summed in another order: a logit, and between near ties the expert, can
+// differ.  Bound by latency: 5 tokens of 8 experts x 4096 take 5.8 us; the library's
+// product, the conversion and moe_route took 19.7.
 template <int K>
 __global__ __launch_bounds__(512) void moe_pick_kernel(
     float* __restrict__ weights,       // [T, K] softmax over the chosen

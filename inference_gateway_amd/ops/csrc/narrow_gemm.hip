@@ -27,7 +27,9 @@ struct SplitTile {
   int MT, NT;
   double step;
 };
-// us for `work` us of steps beside `mb` MB of W from HBM: about the longer of the two
+// us for `work` us of steps beside `mb` MB of W from HBM: about the longer of the two.
+// 4.6 TB/s was fitted with plain loads; read once by nontemporal ones W comes at up to
+// 6.4 (128256 x 4096, 16 rows), for which the choices here are priced too high alike.
 static double split_cost(double work, double mb) {
   const double stream = mb / 4.6, a = work * work, b = stream * stream;
   return std::sqrt(std::sqrt(a * a + b * b));
@@ -163,26 +165,28 @@ torch::Tensor split_parts(const torch::Tensor& x, const torch::Tensor& w,
 // tiles of 64 to 128 columns.
 //
 // So few rows are bound by streaming W, and wider tiles leave compute units without
-// one: 28672 rows of W are 112 tiles of 256 and 224 of 128.  Measured, before (the
-// library with silu_mul, rows_gemm, held_gemm or the tiles of wide_gemm_tile) and here
-// (us): 28672 x 4096 as SwiGLU, 61 / 65 / 128 / 200 / 256 rows 46.1 60.1 60.5 65.4 68.5
-// and 42.3 44.0 52 63.5 64; 35840 x 5120, 16 / 48 / 65 / 128 / 256 / 384 rows 93 92 90.4
-// 86.6 99 160 and 63 65 68.0 71.8 86.4 136; 57344 x 8192, 61 / 160 / 256 rows 169 227 244
-// and 144 211 231; 14336 x 4096, 160 / 256 rows 44.0 56.5 and 39.4 44.8, but 96 rows,
-// with 112 tiles, 39.9 and 44.1; 128256 x 4096, 9 / 32 / 61 / 65 / 128 / 256 rows 164
-// 175 190 232 240 302 and 159 164 169 176 178 247; 32064 x 5120, 16 / 48 / 65 / 256 rows
-// 73.4 81.5 70.5 94.2 and 57 57 60.7 81.5; 28672 x 4096, 61 rows 46.6 and 42.1, but 24 to
-// 48 rows the same; 24576 x 5120, with 192 tiles, 64 rows 56.5 and 59.6 (as SwiGLU 24576
-// x 4096 52.6 and 43); 65536 x 2048 and 152064 x 3584, 16 rows 48.7 182.8 and 50.1 179, 32
-// rows 62.7 261 and 50.6 191; 49152 x 6144, 65 / 160 / 256 rows 156 168 203 and 111 114
-// 129; 32768 x 8192 127 140 170 and 90 108 127; 128256 x 8192 426 463 546 and 339 398 467.
+// one: 28672 rows of W are 112 tiles of 256 and 224 of 128.  Measured, what a call would
+// have else (the library with silu_mul, rows_gemm, held_gemm or the tiles of
+// wide_gemm_tile) and here (us): 28672 x 4096 as SwiGLU, 61 / 65 / 128 / 200 / 256 rows
+// 44.8 60.6 61.1 64.9 66.3 and 41.5 42.9 48.6 59.7 60.8; 35840 x 5120, 16 / 48 / 65 / 128 /
+// 256 / 384 rows 91.2 98.1 80.5 86.8 93.1 154 and 62.1 66.6 64.8 72.8 86.1 138; 57344 x
+// 8192, 61 rows, 174 and 153, but 160 and 256, which wide_gemm_tile's tiles keep, 162 190
+// and 206 231; 14336 x 4096, 160 / 256 rows 42.8 54.9 and 37.8 42.8, but 96 rows, with 112
+// tiles, 36.4 and 39.3; 128256 x 4096, 9 / 32 / 61 / 65 / 128 / 256 rows 167 180 194 230
+// 237 302 and 164 171 176 172 169 242; 32064 x 5120, 16 / 48 / 65 / 256 rows 69.1 80.7 68.8
+// 94.6 and 53.6 55.2 57.9 84.9; 28672 x 4096, 61 rows 45.7 and 43.5, but 24 and 48 rows
+// 39.6 41.0 and 41.6 42.6; 24576 x 5120, with 192 tiles, 64 rows 51.4 and 52.0 (as SwiGLU
+// 24576 x 4096 53.8 and 39.3); 65536 x 2048 and 152064 x 3584, 32 rows 67.3 262 and 44.7
+// 190, and 16 rows, which held_gemm keeps, 48.5 186 and 43.9 180; 49152 x 6144, 65 / 160 /
+// 256 rows 151 163 200 and 107 107 136; 32768 x 8192 126 134 158 and 88.7 103 123; 128256 x
+// 8192 425 457 546 and 339 391 474.
 // Of more than 128 rows the library is ahead where its tiles, 256 wide, are one round,
-// ours of 192 more, and rows of W do not lie a multiple of 4 KB apart (57344 x 3584, 129 / 160 / 256 rows 90.4
-// 90.0 95.3 and 97.5 100 111; 65536 x 2560 77 77 83 and 83 84 93; but 65536 x 4096 151 138
-// 149 and 107 110 125), of more than 192 also where they do, over a long K or where they
-// leave a part of the round (65536 x 8192, 200 / 256 rows, 211 237 and 235 243; 57344 x
-// 4096, 193 / 256 rows 111 113 and 117 121; but 98304 x 8192, 200 / 256 rows 396 417 and
-// 344 335).
+// ours of 192 more, and rows of W do not lie a multiple of 4 KB apart (57344 x 3584, 129 /
+// 160 / 256 rows 90.4 90.0 95.3 and 97.5 100 111; 65536 x 2560 77 77 83 and 83 84 93; but
+// 65536 x 4096 151 138 149 and 107 110 125), of more than 192 also where they do, over a
+// long K or where they leave a part of the round (65536 x 8192, 200 / 256 rows, 224 246 and
+// 247 245; 57344 x 4096, 193 / 256 rows 111 113 and 117 121; but 98304 x 8192, 200 / 256
+// rows 403 410 and 347 352).
 static constexpr SplitTile two_tiles[] = {
     {2, 4, 0.450}, {2, 5, 0.500}, {2, 8, 0.850}};  // up to 64 rows
 static constexpr SplitTile narrow_tiles[] = {

@@ -67,10 +67,10 @@ bool wide_gemm_fits(int64_t x_rs, int64_t N, int64_t K, bool swiglu) {
 
 // Up to this many rows, and entries of a row of W, a gated product reads W once and by
 // nontemporal loads (us, plain and so: 28672 x 4096, 200 / 256 rows 70.4 73.3 and 66.8
-// 69.4, 35840 x 5120 103 113 and 98.4 100).  384 and 512 rows gain there or lose (82.9 96.7 and
-// 80.2 94.1, 153 169 and 160 165), 8192 do not, where W comes back from the caches for
-// every patch of tiles (1 % behind); longer rows of W are slower so (28672 x 14336, 134
-// rows, 218 and 257, 18560 x 11008, 138 rows, 154 and 179).
+// 69.4, 35840 x 5120 103 113 and 98.4 100).  384 and 512 rows gain or lose (28672 x 4096
+// 82.9 96.7 and 80.2 94.1, 35840 x 5120 153 169 and 160 165), 8192 do not, where W comes
+// back from the caches for every patch of tiles (1 % behind); longer rows of W are slower
+// so (28672 x 14336, 134 rows, 218 and 257, 18560 x 11008, 138 rows, 154 and 179).
 constexpr int64_t WIDE_ONCE = 256, WIDE_ONCE_K = 8192;
 
 void wide_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,

@@ -184,15 +184,15 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
   // With ONCE the workgroups of an XCD start their walks over K (over their part of
   // it) two steps apart and the XCDs eight, and go on from its beginning.  Rows lie a
   // multiple of 4 KB apart, so that a step's lines meet in a sixteenth of the memory
-  // channels, and with them those of every workgroup at the same step (us, together and
-  // apart: 128256 x 4096, 16 / 61 / 128 / 256 rows, 213 227 239 268 and 165 175 177 241;
-  // 28672 x 4096 as SwiGLU, 64 / 65 / 128 rows, 49.6 50.0 56.0 and 44.5 46.6 52.4; Mixtral's
-  // experts, 176 tokens, a step 769 and 678; 4096 x 14336 in parts, 65 / 96 / 128 rows,
-  // 31.4 33.6 36.6 and 27.3 30.5 34.5, but short parts and 200 rows 1 to 4 % slower; rows of
-  // 10 KB the same).  With every XCD's first at the same step 32768 x 4096, whose XCDs
-  // lie 16 MB apart, took 75 us at 64 rows, and takes 44.  Rows of tiles that share W
-  // start together.  (By the column of tiles, two steps each, 28672 x 4096 took 59 us:
-  // its address and the start cancel out in the channel.)
+  // channels, and with them those of every workgroup at the same step (us, together
+  // and apart: 128256 x 4096, 16 / 61 / 128 / 256 rows, 213 227 239 268 and 165 175 177
+  // 241; 28672 x 4096 as SwiGLU, 64 / 65 / 128 rows, 49.6 50.0 56.0 and 44.5 46.6 52.4;
+  // Mixtral's experts, 176 tokens, a step 769 and 678; 4096 x 14336 in parts, 65 / 96 /
+  // 128 rows, 31.4 33.6 36.6 and 27.3 30.5 34.5, but short parts and 200 rows 1 to 4 %
+  // slower; rows of 10 KB the same).  With every XCD's first at the same step 32768 x
+  // 4096, whose XCDs lie 16 MB apart, took 75 us at 64 rows, and takes 44.  Rows of
+  // tiles that share W start together.  (By the column of tiles, two steps each, 28672
+  // x 4096 took 59 us: its address and the start cancel out in the channel.)
   int xturn = 0, wturn = 0, xwrap = 0, wwrap = 0;   // bytes
   auto turned = [&](int k, int by, int wrap) WG_INLINE {
     const int r = k + by;
@@ -240,10 +240,12 @@ __global__ __launch_bounds__(256, 1) void wide_gemm_kernel(WideArgs a) {
       (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint16_t*)lds +
       wave * 8 * WG_BK * 2;
   auto load_x = [&](int i, int off, int buf) WG_INLINE {
-    wg_dma<false>(xbuf, xo[i], turned(off, xturn, xwrap), lds0 + (buf + i * 32 * WG_BK) * 2);
+    wg_dma<false>(xbuf, xo[i], turned(off, xturn, xwrap),
+                  lds0 + (buf + i * 32 * WG_BK) * 2);
   };
   auto load_w = [&](int i, int off, int buf) WG_INLINE {
-    wg_dma<ONCE>(wbuf, wo[i], turned(off, wturn, wwrap), lds0 + (buf + i * 32 * WG_BK) * 2);
+    wg_dma<ONCE>(wbuf, wo[i], turned(off, wturn, wwrap),
+                 lds0 + (buf + i * 32 * WG_BK) * 2);
   };
   // a lane's 8 entries of the first half of a K step, and of the second
   const int f0 = r16 * WG_BK + ((quad ^ wg_swz(r16)) << 3), f1 = f0 ^ 32;
