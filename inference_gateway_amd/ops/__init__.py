@@ -307,7 +307,8 @@ def norm_linear(delta, residual: torch.Tensor, weight: torch.Tensor,
     two up to three rows (one row of 4096 x 6144 10.7 and 12.0 us, four 16.8 and 15.0)."""
     if (residual.is_cuda and HAS_KERNELS
             and not torch.compiler.is_compiling()
-            and not has_torch_function_variadic(residual, weight, w)):
+            and not has_torch_function_variadic(delta, residual, weight, w,
+                                                bias)):
         got = _kernels.norm_linear(delta, residual, weight, eps, w, bias,
                                    int(silu))
         if got is not None:

@@ -657,3 +657,32 @@ def test_norm_linear_is_its_parts():
     y, res = ops.norm_linear(None, r, nw, 1e-5, w)
     assert torch.equal(y, ops.linear(ops.rmsnorm(r, nw, 1e-5), w))
     assert torch.equal(res, kept)
+
+
+@pytest.mark.parametrize("which", range(5))
+def test_norm_linear_sees_overrides(which, monkeypatch):
+    """Any operand whose type overrides torch functions keeps the call from the
+    kernel, whose pointers would pass the override by."""
+    class Own(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, args=(), kwargs=None):
+            return super().__torch_function__(func, types, args, kwargs or {})
+
+    class Kernels:
+        @staticmethod
+        def norm_linear(*args):
+            raise AssertionError("the kernel was asked")
+
+    d, r = torch.randn(2, 3, 24)
+    args = [d, r, torch.randn(24), torch.randn(16, 24), torch.randn(16)]
+    monkeypatch.setattr(ops, "_kernels", Kernels)
+    monkeypatch.setattr(ops, "HAS_KERNELS", True)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    with pytest.raises(AssertionError, match="the kernel was asked"):
+        ops.norm_linear(*args[:3], 1e-5, *args[3:])
+    args[which] = args[which].as_subclass(Own)
+    monkeypatch.setattr(ops, "rmsnorm", torch_ref.rmsnorm_ref)
+    monkeypatch.setattr(ops, "fused_add_rmsnorm", torch_ref.fused_add_rmsnorm_ref)
+    monkeypatch.setattr(ops, "linear", torch.nn.functional.linear)
+    y, _ = ops.norm_linear(*args[:3], 1e-5, *args[3:])
+    assert y.shape == (3, 16)
