@@ -43,10 +43,10 @@
 // Measured, with dot products and fp32 multiply-adds on the vector units (450
 // instructions a page) and here, before the loads were nontemporal (PD_ONCE; 32 heads
 // on 8, us): 1024 sequences of 554 to 590 tokens 466 and 410 (5.9 TB/s), 300 of 3000
-// 764 and 637, 61 of 200 to 4000 134 and 104, 128 of 100 to 2000 159 and 109, 16 of 500 16.5 and 11.2; 64 heads
-// on 8, 64 of 400 to 4000 250 and 119.  One, two or eight waves a workgroup:
-// 691, 654, 635 for the 637, 120, 119, 108 for the 109, 114, 109, 114 for the
-// 104.
+// 764 and 637, 61 of 200 to 4000 134 and 104, 128 of 100 to 2000 159 and 109, 16 of
+// 500 16.5 and 11.2; 64 heads on 8, 64 of 400 to 4000 250 and 119.  One, two or eight
+// waves a workgroup: 691, 654, 635 for the 637, 120, 119, 108 for the 109, 114, 109, 114
+// for the 104.
 
 #include <ATen/cuda/CUDAContext.h>
 #include <torch/extension.h>
