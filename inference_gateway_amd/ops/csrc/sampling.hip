@@ -583,8 +583,8 @@ __global__ __launch_bounds__(BLOCK) void sample_bf16_kernel(
 
 // ---------------------------------------------------------------------------
 // bf16 rows that fit a workgroup's registers (V <= 8 * 512 * NCH): the row is
-// read ONCE, 16 bytes a load, past the memory side's cache (1024 rows of 128256, mixed
-// requests, 141 and 138 us), and every further pass runs on registers.
+// read ONCE, 16 bytes a load, past the memory side's cache, and every further pass
+// runs on registers.
 //
 //   1. maximum, and for top-p the total mass Z;
 //      From there the row is kept as keys, whose order is the logits', so that
@@ -597,32 +597,30 @@ __global__ __launch_bounds__(BLOCK) void sample_bf16_kernel(
 //      per element here.  The first window that holds either threshold decides:
 //      the other one is lower and max(tau_k, tau_p) is wanted.  With more than
 //      eight chunks a thread, those with a key of the first window (commonly a
-//      few hundred of 16032) go to a list in LDS, and counts and draw are loops
+//      few hundred of 8192) go to a list in LDS, and counts and draw are loops
 //      over it;
 //   3. the draw: listed chunks with a kept element, if they are at most as many
 //      as threads, are put in index order by counting, and one running sum finds
 //      the chunk.  Otherwise kept mass per (chunk, wave) cell in index order,
 //      cells without a kept element skipped; the cell, the lane, the element.
 //
-// Bound: the row's 256 KB arrive at HBM speed, then come passes over all its
+// Bound: the row's 64 KB to 128 KB arrive at HBM speed, then come passes over all its
 // elements on the vector units, one for the mass, one for the keys and one for
-// every window or cell pass that is needed, at one row per compute unit at a time;
-// with the passes written out for up to 40 chunks also the 64 KB instruction
+// every window or cell pass that is needed, with two to four rows on a compute unit;
+// with the passes written out for up to 16 chunks also the 64 KB instruction
 // cache, which is why what is rare is a loop.  Each of the four passes of
 // sample_bf16_kernel reads the row again and updates LDS bins for all elements.
-// 1024 rows of 128256, greedy / top-k 50 and top-p / top-p 0.9 / top-k 40 / no
-// limits: 52, 117, 179, 90 and 103 us; with elements instead of keys, every pass
-// over all of them and the list's work in the cells 63, 152, 270, 122 and 138.
-// 1024 rows of 32064: 12.8, 36, 43, 29 and 22.5, before 14.4, 39, 65, 33 and 28
+// 1024 rows of 32064, greedy / top-k 50 and top-p / top-p 0.9 / top-k 40 / no
+// limits: 12.8, 36, 43, 29 and 22.5 us; with elements instead of keys, every pass
+// over all of them and the list's work in the cells 14.4, 39, 65, 33 and 28
 // (the list there: 15, 38, 47, 35 and 26, hence the line at eight chunks).
-// Rows of more than 8 * 512 * 40 logits keep sample_bf16_kernel: they would not
-// leave registers for the arithmetic.  So do those of up to 4096, where its
-// passes are short (1000 logits, 300 rows, greedy / top-k and top-p / top-p:
-// 3.0, 15.9 and 15.0 us, here 7.5, 17.0 and 28.3 before; 4099 logits 3.9, 27.0
-// and 24.7, here 3.8, 10.9 and 17.7).  There are as many sizes of the kernel as
+// Rows of more than 8 * 512 * 16 logits go to sample_bf16_stream_kernel: they leave
+// registers for one row a compute unit only.  Those of up to 4096 keep
+// sample_bf16_kernel, where its passes are short (1000 logits, 300 rows, greedy /
+// top-k and top-p / top-p: 3.0, 15.9 and 15.0 us, here 7.5, 17.0 and 28.3 before;
+// 4099 logits 3.9, 27.0 and 24.7, here 3.8, 10.9 and 17.7).  There are as many sizes of the kernel as
 // keep rows without limits ahead of that one, which has few passes for them (300
-// rows of 33000 29.7 us, here 35.3 with 16 chunks, 20.5 with 12; 66000 55.2, 64.7
-// with 32 and 50 with 24).
+// rows of 33000 29.7 us, here 35.3 with 16 chunks, 20.5 with 12).
 // ---------------------------------------------------------------------------
 constexpr int SR_THREADS = 512;
 constexpr int SR_WAVES = SR_THREADS / WAVE_SIZE;
@@ -1236,6 +1234,882 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------
+// bf16 rows of more than 65536 logits (up to 262144): one pass over the row, a
+// wave at a time 2048 logits that lie together (a unit), the next unit's loads under
+// way, so that rows of several workgroups and their arithmetic overlap.  The pass
+// leaves
+//
+//   * the largest logit of every lane;
+//   * where top-p or no limit needs them, the mass of every unit, each with its own
+//     largest as reference (scaled to the row's maximum afterwards: one rounding);
+//   * a list of the chunks of eight that can hold a kept logit.  With top-k these
+//     are the ones at or above a bound: every wave knows the ceil(k / waves)-th of
+//     its lanes' maxima, at least k logits are at or above the least of those.
+//     With top-p alone: an octave below the largest so far, where the logits of the
+//     first step that are listed hold p of that step's mass;
+//   * otherwise (a flat top-p, a k of more than 32 a wave) the counts of all keys in
+//     a window around the first step's maximum.
+//
+// Thresholds come from the counts as in the resident kernel; those of a short
+// list every wave finds for itself, and up to 64 kept chunks one wave puts in order.
+// A row without limits is drawn from the units' masses, of which one is read
+// again; so is a row whose list does not hold all that is kept, by another pass for
+// the kept masses.  Whatever else can be met (a threshold below the window, a
+// sum that is not a number) is done by further passes over memory from the top
+// key down: rare, and written as loops.
+//
+// Bound: HBM with greedy rows (1024 of 128256: 41.6 us, 6.3 TB/s) and with sampled
+// ones without limits (50 us); an exponential is four cycles a logit of the 7 us a
+// row's arithmetic takes; then the serial end of a row, four barriers.
+// 1024 rows of 128256, greedy / top-k 50 and top-p / top-p 0.9 / top-k 40 / no limits /
+// mixed: 41.6, 62, 124, 54, 50 and 89 us; held in registers, one row a compute unit
+// whose passes follow its loads, 54, 123, 185, 99, 103 and 144.  64 rows mixed 39.9 for
+// 42.5; 1024 of 66000, mixed, 60 for 98.  Up to 65536 logits the register kernel has
+// two rows on a unit and is ahead (1024 of 49000, mixed, 49.3, here 50.7; of 32000 36.3
+// and 43).
+// ---------------------------------------------------------------------------
+constexpr int SS_U = 4;                  // chunks of eight a lane in a unit
+constexpr int SS_UNIT = SS_U * 512;      // logits
+constexpr int SS_UNITS = 128;            // of a row at most
+constexpr int SS_WINDOW = 4096;          // keys that are counted at a time
+constexpr int SS_OCTAVE = 128;           // keys of an octave
+constexpr int SS_ABOVE = 512;            // of the window, above the first maximum
+constexpr int SS_NARROW = 512;           // keys that a wave looks through alone
+
+// Not fmaxf, which would quiet each operand first; rows with a NaN are found by
+// their bits or their mass and done again.
+DEVINLINE float ss_max3(float a, float b, float c) {
+  float m;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(a), "v"(b), "v"(c));
+  return m;
+}
+DEVINLINE uint32_t ss_pk_max(uint32_t a, uint32_t b) {
+  uint32_t m;
+  asm("v_pk_max_u16 %0, %1, %2" : "=v"(m) : "v"(a), "v"(b));
+  return m;
+}
+
+// Two bins of a window of SS_WINDOW keys from `top` down, `spare` outside of it.
+DEVINLINE uint32_t ss_bins(uint32_t keys, uint32_t top, uint32_t spare) {
+  typedef __attribute__((ext_vector_type(2))) unsigned short ushort2v;
+  const ushort2v b = __builtin_bit_cast(ushort2v, top) -
+                     __builtin_bit_cast(ushort2v, keys);
+  return __builtin_bit_cast(
+      uint32_t,
+      __builtin_elementwise_min(b, __builtin_bit_cast(ushort2v, spare)));
+}
+
+template <int SS_THREADS>
+__global__ __launch_bounds__(SS_THREADS, 4) void sample_bf16_stream_kernel(
+    int32_t* __restrict__ out,             // [B]
+    const uint16_t* __restrict__ logits,   // [B, V] bf16 bits
+    const float* __restrict__ temperature, // [B]
+    const int32_t* __restrict__ top_k,     // [B] (<=0 => disabled)
+    const float* __restrict__ top_p,       // [B] (>=1 => disabled)
+    const float* __restrict__ uniforms,    // [B]
+    int V) {
+  constexpr int SS_WAVES = SS_THREADS / WAVE_SIZE;
+  constexpr int SS_LIST = SS_THREADS == 512 ? 3072 : 4096;   // as the LDS takes
+  constexpr int U = SS_U, UNIT = SS_UNIT;
+  __shared__ __attribute__((aligned(16))) uint32_t
+      bins[SS_WINDOW + WAVE_SIZE > 4 * SS_THREADS ? SS_WINDOW + WAVE_SIZE
+                                                 : 4 * SS_THREADS];
+  __shared__ __attribute__((aligned(16))) int kept_at[SS_THREADS];
+  __shared__ uint4 list_k[SS_LIST];    // listed chunks: logits
+  __shared__ int list_at[SS_LIST];     // and number
+  // behind the counts, where they were
+  int* const kept_e = reinterpret_cast<int*>(bins);
+  int* const sorted_e = kept_e + SS_THREADS;
+  float* const kept_w = reinterpret_cast<float*>(sorted_e + SS_THREADS);
+  float* const sorted_w = kept_w + SS_THREADS;
+  __shared__ float cells[SS_UNITS], cell_c[SS_UNITS];
+  __shared__ float red[SS_WAVES];
+  __shared__ uint32_t bound[SS_WAVES], bound0[SS_WAVES];
+  __shared__ uint32_t wave_n[SS_WAVES];
+  __shared__ float wave_w[SS_WAVES];
+  __shared__ int s_list, s_bad, s_kept, s_last, s_tau, s_top, s_cell;
+  __shared__ uint32_t s_pick;
+
+  const int seq = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint16_t* row = logits + (int64_t)seq * V;
+  const float temp = temperature[seq];
+  const bool greedy = temp <= 0.0f;
+  const float inv_t = greedy ? 1.0f : 1.0f / temp;
+  const float rate = inv_t * 1.44269504088896340736f;   // to powers of two
+  const int k = top_k[seq];
+  const float p = top_p[seq];
+  const bool do_k = k > 0 && k < V && !greedy;
+  const bool do_p = p < 1.0f && !greedy;
+  const bool do_z = !greedy && (do_p || !do_k);   // exponentials of all
+  const bool do_list = do_k || do_p;
+  const int units = (V + UNIT - 1) / UNIT;
+
+  typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+  // chunk of eight logits at `at`, past the end -inf
+  auto load_chunk = [&](int at, uint32_t (&d)[4]) {
+    if (at + 8 <= V) {
+      const u32x4 v =
+          __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(row + at));
+      d[0] = v.x; d[1] = v.y; d[2] = v.z; d[3] = v.w;
+    } else {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int e = at + 2 * q;
+        const uint32_t lo = e < V ? row[e] : 0xff80u;
+        const uint32_t hi = e + 1 < V ? row[e + 1] : 0xff80u;
+        d[q] = lo | (hi << 16);
+      }
+    }
+  };
+  auto load = [&](int unit, uint32_t (&d)[U][4]) {
+    const int at = unit * UNIT + lane * 8;
+    if ((unit + 1) * UNIT <= V) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const u32x4* from = reinterpret_cast<const u32x4*>(row + at + u * 512);
+        const u32x4 v = __builtin_nontemporal_load(from);
+        d[u][0] = v.x; d[u][1] = v.y; d[u][2] = v.z; d[u][3] = v.w;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) load_chunk(at + u * 512, d[u]);
+    }
+  };
+  // f(unit, logits) of this wave's units, the next one's loads under way
+  auto for_units = [&](auto&& f) {
+    uint32_t d[U][4], e[U][4];
+    int unit = wave;
+    if (unit < units) load(unit, d);
+    while (unit < units) {
+      if (unit + SS_WAVES < units) load(unit + SS_WAVES, e);
+      f(unit, d);
+      unit += SS_WAVES;
+      if (unit >= units) break;
+      if (unit + SS_WAVES < units) load(unit + SS_WAVES, d);
+      f(unit, e);
+      unit += SS_WAVES;
+    }
+  };
+
+  // ---- the row, once: largest, mass, list ----
+  const int active = min(SS_WAVES, units);
+  // lanes of a wave at or above its bound; of its largest, if that is wanted
+  const int share = do_k ? (k + active - 1) / active : 1;
+  const bool octave = !do_k || share > 32;
+  const int need = octave ? 1 : share;
+  float best = -INFINITY;   // of this lane
+  int best_at = 0;          // the unit it came with
+  uint32_t odd = 0;         // largest bits without the sign, both halves
+  int anchor = -1;          // key of the first bin, where all are counted
+  if (do_list) {
+    for (int b = tid; b < SS_WINDOW; b += SS_THREADS) bins[b] = 0;
+    kept_at[tid] = INT_MAX;
+  }
+  if (tid == 0) {
+    s_list = 0;
+    s_bad = 0;
+    s_kept = 0;
+    s_tau = -1;
+    s_top = -1;
+    s_cell = INT_MAX;
+    s_last = -1;
+    s_pick = 0xffffffffu;
+  }
+  const float u01 = uniforms[seq];
+  auto take = [&](int unit, const uint32_t (&d)[U][4], bool first) {
+    float most[U];
+    const Unpack un;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const float a = ss_max3(un.lo(d[u][0]), un.hi(d[u][0]), un.lo(d[u][1]));
+      const float b = ss_max3(un.hi(d[u][1]), un.lo(d[u][2]), un.hi(d[u][2]));
+      most[u] = ss_max3(ss_max3(un.lo(d[u][3]), un.hi(d[u][3]), a), b, b);
+    }
+    float all = most[0];
+#pragma unroll
+    for (int u = 1; u < U; ++u) all = ss_max3(all, most[u], most[u]);
+    if (all > best) {
+      best = all;
+      best_at = unit;
+    }
+    if (do_z) {
+      const float ref = sr_max(all);
+      const float c = ref == -INFINITY ? 0.0f : -(ref * rate);
+      float z0 = 0.0f, z1 = 0.0f;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          z0 += __builtin_amdgcn_exp2f(fmaf(un.lo(d[u][q]), rate, c));
+          z1 += __builtin_amdgcn_exp2f(fmaf(un.hi(d[u][q]), rate, c));
+        }
+      const float z = sr_sum(z0 + z1);
+      if (lane == 0 && unit < units) {
+        cells[unit] = z;
+        cell_c[unit] = c;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) odd = ss_pk_max(odd, d[u][q] & 0x7fff7fffu);
+    }
+    if (do_list) {
+      const uint32_t own =
+          bf16_key((uint16_t)(__builtin_bit_cast(uint32_t, best) >> 16));
+      const int step = unit / SS_WAVES;
+      if ((step & (step + 1)) == 0) {   // the bound rises with the logarithm
+        uint32_t t = 0;
+#pragma unroll
+        for (int bit = 15; bit >= 0; --bit) {
+          const uint32_t c = t | (1u << bit);
+          if (__popcll(__ballot(own >= c)) >= need) t = c;
+        }
+        if (lane == 0) {
+          if (first) bound0[wave] = t;
+          __hip_atomic_store(&bound[wave], t, __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+      }
+      if (first) {
+        __syncthreads();
+        if (octave) {
+          int top = 0;
+          for (int w = 0; w < active; ++w) top = max(top, (int)bound0[w]);
+          bool flat = do_k;
+          if (!do_k) {
+            // mass of what would be listed, and of all, of the logits so far
+            const float m = bf16_key_val(max(top, 0x007f));
+            const float from = bf16_key_val(max(top - SS_OCTAVE + 1, 0x007f));
+            const float c = -(m * rate);
+            float above = 0.0f;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+              for (int q = 0; q < 4; ++q) {
+                const float lo = un.lo(d[u][q]), hi = un.hi(d[u][q]);
+                const float w0 = __builtin_amdgcn_exp2f(fmaf(lo, rate, c));
+                const float w1 = __builtin_amdgcn_exp2f(fmaf(hi, rate, c));
+                above += (lo >= from ? w0 : 0.0f) + (hi >= from ? w1 : 0.0f);
+              }
+            above = sr_sum(above);
+            if (lane == 0) wave_w[wave] = above;
+            __syncthreads();
+            above = sr_sum(lane < active ? wave_w[lane] : 0.0f);
+            const float z = sr_sum(
+                lane < active && cells[lane] > 0.0f
+                    ? cells[lane] * __builtin_amdgcn_exp2f(
+                                        fmaf(-m, rate, -cell_c[lane]))
+                    : 0.0f);
+            flat = !(above >= p * z);
+          }
+          if (flat) anchor = min(top + SS_ABOVE, 0xff80);
+        }
+      }
+      if (anchor >= 0 && unit < units) {
+        const uint32_t top = (uint32_t)anchor * 0x10001u;
+        // an element outside the window counts where nobody looks
+        const uint32_t spare = (uint32_t)(SS_WINDOW + lane) * 0x10001u;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const uint32_t b = ss_bins(un.keys(d[u][q]), top, spare);
+            atomicAdd(&bins[b & 0xffffu], 1u);
+            atomicAdd(&bins[b >> 16], 1u);
+          }
+      }
+      uint32_t low = octave ? 0 : 0xffffffffu;
+      for (int w = 0; w < active; ++w) {
+        const uint32_t b = __hip_atomic_load(&bound[w], __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_WORKGROUP);
+        low = octave ? max(low, b) : min(low, b);
+      }
+      if (octave) low = (uint32_t)max((int)low - SS_OCTAVE + 1, 0);
+      const float from = bf16_key_val(max(low, 0x007fu));
+      if (anchor < 0 && unit < units && __any(all >= from)) {
+        uint64_t at[U];
+        int n = 0;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          at[u] = __ballot(most[u] >= from);
+          n += __popcll(at[u]);
+        }
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&s_list, n);
+        base = __builtin_amdgcn_readfirstlane(base);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int to = base + __builtin_amdgcn_mbcnt_hi(
+                                    (uint32_t)(at[u] >> 32),
+                                    __builtin_amdgcn_mbcnt_lo((uint32_t)at[u], 0));
+          if ((at[u] >> lane & 1) && to < SS_LIST) {
+            list_k[to] = make_uint4(d[u][0], d[u][1], d[u][2], d[u][3]);
+            list_at[to] = unit * (UNIT / 8) + u * 64 + lane;
+          }
+          base += __popcll(at[u]);
+        }
+      }
+    }
+  };
+  {
+    uint32_t d[U][4], e[U][4];
+    int unit = wave;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) d[u][q] = 0xff80ff80u;
+    if (unit < units) load(unit, d);
+    __syncthreads();   // s_list
+    bool first = true;
+    while (true) {
+      if (unit + SS_WAVES < units) load(unit + SS_WAVES, e);
+      take(unit, d, first);
+      first = false;
+      unit += SS_WAVES;
+      if (unit >= units) break;
+      if (unit + SS_WAVES < units) load(unit + SS_WAVES, d);
+      take(unit, e, false);
+      unit += SS_WAVES;
+      if (unit >= units) break;
+    }
+  }
+  if (__any((odd & 0xffffu) > 0x7f80u || (odd >> 16) > 0x7f80u) && lane == 0)
+    s_bad = 1;
+  {
+    const float m = sr_max(best);
+    if (lane == 0) red[wave] = m;
+  }
+  __syncthreads();
+  float M = red[0];
+#pragma unroll
+  for (int w = 1; w < SS_WAVES; ++w) M = fmaxf(M, red[w]);
+  bool bad = s_bad;
+
+  // Mass of a unit with M's weight 1 (0 stays: its own scale may be infinite).
+  auto cell = [&](int c) {
+    const float z = c < units ? cells[c] : 0.0f;
+    return z > 0.0f
+               ? z * __builtin_amdgcn_exp2f(fmaf(-M, rate, -cell_c[c]))
+               : z;
+  };
+  float Z = 0.0f;
+  if (do_z) {
+#pragma unroll
+    for (int i = 0; i < SS_UNITS / 64; ++i) Z += cell(i * 64 + lane);
+    Z = sr_sum(Z);
+    bad = !(Z > 0.0f && Z < INFINITY);
+  }
+  bad = bad || M == -INFINITY;
+
+  // Lowest index of the largest logit that is a number (all threads call it).
+  auto first_max = [&]() {
+    for (int at = tid * 8; at < V; at += SS_THREADS * 8) {
+      uint32_t d[4];
+      load_chunk(at, d);
+      const Unpack un;
+      uint32_t h = 8;
+#pragma unroll
+      for (int q = 3; q >= 0; --q) {
+        if (un.hi(d[q]) == M) h = 2 * q + 1;
+        if (un.lo(d[q]) == M) h = 2 * q;
+      }
+      if (h < 8) {
+        atomicMin(&s_pick, at + h);
+        break;
+      }
+    }
+    __syncthreads();
+    if (tid == 0)   // what is past the end is no logit
+      out[seq] = M == -INFINITY && !greedy ? 0
+                 : s_pick < (uint32_t)V    ? (int32_t)s_pick
+                                           : -1;
+  };
+  if (bad) {   // the maximum of the numbers, by comparisons that pass over others
+    float m = -INFINITY;
+    for (int at = tid * 8; at < V; at += SS_THREADS * 8) {
+      uint32_t d[4];
+      load_chunk(at, d);
+      const Unpack un;
+      for (int q = 0; q < 4; ++q) {
+        const float lo = un.lo(d[q]), hi = un.hi(d[q]);
+        m = lo > m ? lo : m;
+        m = hi > m ? hi : m;
+      }
+    }
+    m = sr_max(m);
+    __syncthreads();   // red was read by everybody
+    if (lane == 0) red[wave] = m;
+    __syncthreads();
+    M = red[0];
+#pragma unroll
+    for (int w = 1; w < SS_WAVES; ++w) M = fmaxf(M, red[w]);
+  }
+  if (greedy) {
+    if (bad) {
+      first_max();
+      return;
+    }
+    if (best == M) {
+      uint32_t d[U][4];
+      load(best_at, d);
+      const Unpack un;
+      uint32_t h = 0;
+#pragma unroll
+      for (int u = U - 1; u >= 0; --u)
+#pragma unroll
+        for (int q = 3; q >= 0; --q) {
+          if (un.hi(d[u][q]) == M) h = u * 512 + 2 * q + 1;
+          if (un.lo(d[u][q]) == M) h = u * 512 + 2 * q;
+        }
+      atomicMin(&s_pick, (uint32_t)(best_at * UNIT + lane * 8) + h);
+    }
+    __syncthreads();
+    if (tid == 0) out[seq] = (int32_t)s_pick;
+    return;
+  }
+
+  auto weight = [&](float x) {
+    return __builtin_amdgcn_exp2f((x - M) * rate);
+  };
+  if (bad && do_p) {
+    float z = 0.0f;
+    for (int at = tid * 8; at < V; at += SS_THREADS * 8) {
+      uint32_t d[4];
+      load_chunk(at, d);
+      const Unpack un;
+      for (int q = 0; q < 4; ++q) z += weight(un.lo(d[q])) + weight(un.hi(d[q]));
+    }
+    z = sr_sum(z);
+    __syncthreads();   // red was read by everybody
+    if (lane == 0) red[wave] = z;
+    __syncthreads();
+    Z = 0.0f;
+#pragma unroll
+    for (int w = 0; w < SS_WAVES; ++w) Z += red[w];
+  }
+  const float target_p = p * Z;
+  int max_key = 0x8000;  // key of the maximum (of +0 for either zero)
+  if (M != 0.0f)
+    max_key =
+        (int)bf16_key((uint16_t)(__builtin_bit_cast(uint32_t, M) >> 16));
+
+  // ---- thresholds ----
+  int tau = 0;
+  int listed = -1;   // chunks in the list, when it holds all that is kept
+  if (do_list) {
+    uint32_t low = octave ? 0 : 0xffffffffu;
+    for (int w = 0; w < active; ++w)
+      low = octave ? max(low, bound[w]) : min(low, bound[w]);
+    if (octave) low = (uint32_t)max((int)low - SS_OCTAVE + 1, 0);
+    // whether all from `low` on is listed
+    const bool whole = !bad && anchor < 0 && s_list <= SS_LIST;
+    int top = max_key, width = SS_WINDOW;
+    // whether the bins hold the counts: of all logits, or of the listed ones
+    bool counted = false, some = false;
+    if (!bad && max_key <= anchor) {
+      counted = true;
+      top = anchor;
+    } else if (whole && top - (int)low < SS_WINDOW) {
+      counted = some = true;
+      width = max(top - (int)low + 1, 1);
+      const Unpack un;
+      const uint32_t* list = reinterpret_cast<const uint32_t*>(list_k);
+      for (int e = tid; e < s_list * 4; e += SS_THREADS) {
+        const uint32_t b =
+            ss_bins(un.keys(list[e]), (uint32_t)top * 0x10001u,
+                    (uint32_t)(SS_WINDOW + lane) * 0x10001u);
+        atomicAdd(&bins[b & 0xffffu], 1u);
+        atomicAdd(&bins[b >> 16], 1u);
+      }
+      __syncthreads();
+    }
+    if (some && width <= SS_NARROW) {
+      // every wave for itself: lane l takes the keys top - (8 l + i), in order
+      constexpr int PER = SS_NARROW / 64;
+      uint32_t c[PER], n = 0;
+      float m[PER], w = 0.0f;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int b = lane * PER + i;
+        c[i] = b < width ? bins[b] : 0;
+        m[i] = c[i] ? (float)c[i] * weight(bf16_key_val((uint32_t)(top - b)))
+                    : 0.0f;
+        n += c[i];
+        w += m[i];
+      }
+      const uint32_t sn = sr_scan(n);
+      const float sw = sr_scan(w);
+      const uint64_t ends = __ballot(n && ((do_k && sn >= (uint32_t)k) ||
+                                           (do_p && sw >= target_p)));
+      if (ends) {
+        // the first key, from the top, at which either is reached; the sums
+        // in this order may end a rounding step below the scanned ones: then
+        // the last key with a logit
+        uint32_t cn = sn - n;
+        float cw = sw - w;
+        int reached = -1;
+        bool done = false;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+          cn += c[i];
+          cw += m[i];
+          if (c[i] && !done) {
+            reached = top - (lane * PER + i);
+            done = (do_k && cn >= (uint32_t)k) || (do_p && cw >= target_p);
+          }
+        }
+        tau = __builtin_amdgcn_readlane(reached, __builtin_ctzll(ends));
+        listed = s_list;
+      } else {
+        __syncthreads();   // the bins were read by everybody
+        counted = some = false;
+        width = SS_WINDOW;
+      }
+    }
+    uint32_t seen_n = 0;   // above the window
+    float seen_w = 0.0f;
+    while (listed < 0) {
+      if (!counted) {
+        for (int b = tid; b < width; b += SS_THREADS) bins[b] = 0;
+        if (tid == 0) {
+          s_tau = -1;
+          s_top = -1;
+        }
+        __syncthreads();
+        const uint32_t top2 = (uint32_t)top * 0x10001u;
+        const uint32_t spare = (uint32_t)(SS_WINDOW + lane) * 0x10001u;
+        for_units([&](int, const uint32_t(&d)[U][4]) {
+          const Unpack un;
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              const uint32_t b = ss_bins(un.keys(d[u][q]), top2, spare);
+              atomicAdd(&bins[b & 0xffffu], 1u);
+              atomicAdd(&bins[b >> 16], 1u);
+            }
+        });
+        __syncthreads();
+      }
+      // thread t takes the keys top - (per t + i), i < per, in order
+      const int per = (width + SS_THREADS - 1) / SS_THREADS;
+      const int b0 = min(tid * per, width), b1 = min(b0 + per, width);
+      uint32_t n = 0;
+      float w = 0.0f;
+      for (int b = b0; b < b1; ++b) {
+        const uint32_t c = bins[b];
+        if (c) {
+          n += c;
+          w += (float)c * weight(bf16_key_val((uint32_t)(top - b)));
+        }
+      }
+      // inclusive sums over the wave, then over the waves before it
+      const uint32_t sn = sr_scan(n);
+      const float sw = sr_scan(w);
+      if (lane == 63) {
+        wave_n[wave] = sn;
+        wave_w[wave] = sw;
+      }
+      __syncthreads();
+      uint32_t all_n = seen_n, base_n = 0;
+      float all_w = seen_w, base_w = 0.0f;
+#pragma unroll
+      for (int v = 0; v < SS_WAVES; ++v) {
+        if (v == wave) {
+          base_n = all_n;
+          base_w = all_w;
+        }
+        all_n += wave_n[v];
+        all_w += wave_w[v];
+      }
+      {
+        uint32_t cn = base_n + sn - n;
+        float cw = base_w + sw - w;
+        const bool end_k = do_k && cn + n >= (uint32_t)k;
+        const bool end_p = do_p && base_w + sw >= target_p;
+        if (n && (end_k || end_p)) {   // as above
+          int reached = -1;
+          for (int b = b0; b < b1; ++b) {
+            const uint32_t c = bins[b];
+            if (!c) continue;
+            cn += c;
+            cw += (float)c * weight(bf16_key_val((uint32_t)(top - b)));
+            reached = top - b;
+            if ((do_k && cn >= (uint32_t)k) || (do_p && cw >= target_p)) break;
+          }
+          atomicMax(&s_tau, reached);
+        }
+      }
+      __syncthreads();
+      tau = s_tau;
+      if (tau >= 0) {
+        if (some) listed = s_list;
+        break;
+      }
+      if (counted) {   // below what was counted: from the top, all logits
+        counted = some = false;
+        top = max_key;
+        width = SS_WINDOW;
+        __syncthreads();
+        continue;
+      }
+      // the highest key below the window
+      const int lo = top - width + 1;
+      int next = -1;
+      for (int at = tid * 8; at < V; at += SS_THREADS * 8) {
+        uint32_t d[4];
+        load_chunk(at, d);
+        const Unpack un;
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t key = un.keys(d[q]);
+          const int k0 = (int)un.first(key), k1 = (int)un.second(key);
+          if (k0 < lo) next = max(next, k0);
+          if (k1 < lo) next = max(next, k1);
+        }
+      }
+      if (next >= 0) atomicMax(&s_top, next);
+      __syncthreads();
+      top = s_top;
+      seen_n = all_n;
+      seen_w = all_w;
+      if (top < 0) {  // everything is kept (p * Z not reached by rounding)
+        tau = 0;
+        break;
+      }
+      __syncthreads();  // s_top and the bins are reset above
+    }
+  }
+
+  const uint32_t utau = (uint32_t)tau;
+  auto kept = [&](uint32_t key) {
+    return key >= utau ? weight(bf16_key_val(key)) : 0.0f;
+  };
+  auto kept_sum = [&](const uint32_t* e) {
+    float sum = 0.0f;
+    for (int q = 0; q < 4; ++q) sum += kept(e[q] & 0xffffu) + kept(e[q] >> 16);
+    return sum;
+  };
+  // the element of a chunk at which the running sum passes, or the last with
+  // mass
+  auto element = [&](const uint32_t* e, float run, float target) {
+    int chosen = 0;
+    for (int h = 0; h < 8; ++h) {
+      const float w = kept((h & 1) ? e[h >> 1] >> 16 : e[h >> 1] & 0xffffu);
+      run += w;
+      if (w > 0.0f) chosen = h;
+      if (w > 0.0f && run > target) break;
+    }
+    return chosen;
+  };
+
+  // ---- listed: at most as many kept chunks as threads are put in order ----
+  if (listed >= 0) {
+    const Unpack un;
+    auto keys_of = [&](int e, uint32_t (&l)[4]) {
+      const uint4 v = list_k[e];
+      l[0] = un.keys(v.x); l[1] = un.keys(v.y);
+      l[2] = un.keys(v.z); l[3] = un.keys(v.w);
+    };
+    // kept_e and kept_w lie where counts were: nobody reads them any more
+    __syncthreads();
+    for (int e = tid; e < listed; e += SS_THREADS) {
+      uint32_t l[4];
+      keys_of(e, l);
+      if (largest_key(l) >= utau) {
+        const int at = atomicAdd(&s_kept, 1);
+        if (at < SS_THREADS) {
+          kept_at[at] = list_at[e];
+          kept_w[at] = kept_sum(l);
+          kept_e[at] = e;
+        }
+      }
+    }
+    __syncthreads();
+    const int n = s_kept;
+    auto rank_of = [&](int own) {
+      int rank = 0;
+      for (int e = 0; e < n; e += 4) {
+        const int4 v = *reinterpret_cast<const int4*>(kept_at + e);
+        rank += (v.x < own) + (v.y < own) + (v.z < own) + (v.w < own);
+      }
+      return rank;
+    };
+    auto draw = [&](int e, float run, float target) {
+      uint32_t l[4];
+      keys_of(e, l);
+      out[seq] = list_at[e] * 8 + element(l, run, target);
+    };
+    if (n <= 64) {   // one wave
+      if (wave == 0) {
+        if (lane < n) {
+          const int rank = rank_of(kept_at[lane]);
+          sorted_w[rank] = kept_w[lane];
+          sorted_e[rank] = kept_e[lane];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        __builtin_amdgcn_wave_barrier();
+        const float w = lane < n ? sorted_w[lane] : 0.0f;
+        const float own = sr_scan(w);
+        const float total =
+            __builtin_bit_cast(float, __builtin_amdgcn_readlane(
+                                          __builtin_bit_cast(int, own), 63));
+        if (total > 0.0f) {
+          const float target = u01 * total;
+          const uint64_t past = __ballot(w > 0.0f && own > target);
+          const uint64_t any = __ballot(w > 0.0f);
+          const int l = past ? __builtin_ctzll(past) : 63 - __builtin_clzll(any);
+          if (lane == l)
+            draw(sorted_e[lane], own - w, past ? target : INFINITY);
+        } else if (lane == 0) {
+          s_last = 1;   // nothing to draw from
+        }
+      }
+      __syncthreads();
+      if (s_last == 1) first_max();
+      return;
+    }
+    if (n <= SS_THREADS) {
+      if (tid < n) {
+        const int rank = rank_of(kept_at[tid]);
+        sorted_w[rank] = kept_w[tid];
+        sorted_e[rank] = kept_e[tid];
+      }
+      __syncthreads();
+      const float w = tid < n ? sorted_w[tid] : 0.0f;
+      const float own = sr_scan(w);
+      if (lane == 63) wave_w[wave] = own;
+      __syncthreads();
+      float before = 0.0f, total = 0.0f;
+#pragma unroll
+      for (int v = 0; v < SS_WAVES; ++v) {
+        if (v == wave) before = total;
+        total += wave_w[v];
+      }
+      if (total > 0.0f) {
+        const float target = u01 * total;
+        if (w > 0.0f) {
+          if (before + own > target) atomicMin(&s_cell, tid);
+          atomicMax(&s_last, tid);
+        }
+        __syncthreads();
+        const bool passed = s_cell != INT_MAX;
+        if (tid == (passed ? s_cell : s_last))
+          draw(sorted_e[tid], before + own - w, passed ? target : INFINITY);
+      } else {   // as below
+        first_max();
+      }
+      return;
+    }
+  }
+
+  // ---- kept mass of every unit, in index order ----
+  if (do_list || bad) {
+    for_units([&](int unit, const uint32_t(&d)[U][4]) {
+      const Unpack un;
+      float sum = 0.0f;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const uint32_t key = un.keys(d[u][q]);
+          const float w0 = weight(un.lo(d[u][q])), w1 = weight(un.hi(d[u][q]));
+          sum += (un.first(key) >= utau ? w0 : 0.0f) +
+                 (un.second(key) >= utau ? w1 : 0.0f);
+        }
+      sum = sr_sum(sum);
+      if (lane == 0) {
+        cells[unit] = sum;
+        cell_c[unit] = 0.0f;
+      }
+    });
+    __syncthreads();
+  }
+  // every wave: the first unit whose running sum passes u * total
+  constexpr int PER = SS_UNITS / 64;
+  float mass[PER], own = 0.0f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int c = lane * PER + i;
+    mass[i] = do_list || bad ? (c < units ? cells[c] : 0.0f) : cell(c);
+    own += mass[i];
+  }
+  float run = sr_scan(own);
+  const float total = __shfl(run, 63, 64);
+  const float target = u01 * total;
+  run -= own;
+  int at = -1;         // first that passes the target
+  int last = -1;       // last with any mass
+  float base = 0.0f;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int c = lane * PER + i;
+    const float w = mass[i];
+    if (w > 0.0f) last = c;
+    if (at < 0 && w > 0.0f && run + w > target) {
+      at = c;
+      base = run;
+    }
+    run += w;
+  }
+  const uint64_t found = __ballot(at >= 0), some = __ballot(last >= 0);
+  float rest = INFINITY;   // mass into the unit; infinite: its last element
+  int pick = -1;
+  if (!(total > 0.0f)) {
+    // nothing that could be drawn from: the largest logit
+  } else if (found) {
+    const int l = __builtin_ctzll(found);
+    pick = __shfl(at, l, 64);
+    rest = target - __shfl(base, l, 64);
+  } else if (some) {
+    pick = __shfl(last, 63 - __builtin_clzll(some), 64);
+  }
+  if (pick < 0) {
+    // A kept logit that is not a number, or an infinite one, leaves no mass
+    // to draw from: the largest logit, the first one where none is above
+    // minus infinity.
+    first_max();
+    return;
+  }
+  if (wave != 0) return;
+  uint32_t d[U][4];
+  load(pick, d);
+  float before = 0.0f, at_run = 0.0f;
+  int chunk = -1, at_lane = 0;
+  bool passed = false;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) d[u][q] = Unpack().keys(d[u][q]);
+    const float sum = kept_sum(d[u]);
+    const float to = before + sr_scan(sum);
+    const uint64_t past = __ballot(sum > 0.0f && to > rest);
+    const uint64_t any = __ballot(sum > 0.0f);
+    if (!passed && any) {
+      passed = past != 0;
+      chunk = u;
+      at_lane = past ? __builtin_ctzll(past) : 63 - __builtin_clzll(any);
+      at_run = to - sum;
+    }
+    before = __shfl(to, 63, 64);
+  }
+  if (lane == at_lane) {
+    uint32_t e[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u == chunk) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) e[q] = d[u][q];
+      }
+    out[seq] = pick * UNIT + chunk * 512 + lane * 8 +
+               element(e, at_run, passed ? rest : INFINITY);
+  }
+}
+
 void sample(torch::Tensor out, torch::Tensor logits, torch::Tensor temperature,
             torch::Tensor top_k, torch::Tensor top_p, torch::Tensor uniforms) {
   TORCH_CHECK(logits.is_cuda());
@@ -1255,17 +2129,33 @@ void sample(torch::Tensor out, torch::Tensor logits, torch::Tensor temperature,
                      (const int32_t*)top_k.data_ptr(),                        \
                      (const float*)top_p.data_ptr(),                          \
                      (const float*)uniforms.data_ptr(), V)
+    // Longer rows than the resident kernel is ahead for (its line: see there), up
+    // to what `cells` holds.  Up to a row per compute unit, 1024 threads a row: 64
+    // and 400 rows of 128256, mixed requests, 39.9 and 61.8 us, with 512 threads
+    // and two rows on a unit 42.3 and 57.8.
+    if (V > 16 * 8 * SR_THREADS && V <= SS_UNITS * SS_UNIT) {
+#define LAUNCH_STREAM(T)                                                      \
+  hipLaunchKernelGGL((sample_bf16_stream_kernel<T>), dim3(B), dim3(T), 0,     \
+                     stream, (int32_t*)out.data_ptr(),                        \
+                     (const uint16_t*)logits.data_ptr(),                      \
+                     (const float*)temperature.data_ptr(),                    \
+                     (const int32_t*)top_k.data_ptr(),                        \
+                     (const float*)top_p.data_ptr(),                          \
+                     (const float*)uniforms.data_ptr(), V)
+      if (B <= 256) LAUNCH_STREAM(1024);
+      else LAUNCH_STREAM(512);
+#undef LAUNCH_STREAM
+      HIP_CHECK_KERNEL();
+      return;
+    }
     const int chunks = (V + 8 * SR_THREADS - 1) / (8 * SR_THREADS);
-    if (V > 8 * SR_THREADS && chunks <= 40) {
+    if (V > 8 * SR_THREADS && chunks <= 16) {
       if (chunks <= 2) LAUNCH_RESIDENT(2);
       else if (chunks <= 4) LAUNCH_RESIDENT(4);
       else if (chunks <= 6) LAUNCH_RESIDENT(6);
       else if (chunks <= 8) LAUNCH_RESIDENT(8);
       else if (chunks <= 12) LAUNCH_RESIDENT(12);
-      else if (chunks <= 16) LAUNCH_RESIDENT(16);
-      else if (chunks <= 24) LAUNCH_RESIDENT(24);
-      else if (chunks <= 32) LAUNCH_RESIDENT(32);
-      else LAUNCH_RESIDENT(40);
+      else LAUNCH_RESIDENT(16);
       HIP_CHECK_KERNEL();
       return;
     }
