@@ -182,6 +182,135 @@ __global__ __launch_bounds__(256) void qk_norm_rope_append_kernel(
   }
 }
 
+// The same for bf16 heads of 64, 128 or 256 entries whose rows lie on 16 bytes: a
+// thread takes 16-byte chunks of the row, NC of them with all loads sent before the
+// first is used, and a head's N / 8 lanes exchange its sum (and, where halves turn,
+// its chunks) among themselves.
+//
+// Bound by one pass over the rows; few rows by the latency of one load, one exchange
+// and one store: a row is cut over workgroups until a thread has one chunk.  Waves
+// that took a row's heads in turn, a pair of entries a lane, and here (us; 32 heads on
+// 8 of 128, normed, not rotated): 1 row 9.9 and 2.4, 48 rows 10.3 and 2.6, 400 rows 11.4
+// and 5.2, 1303 rows 19.7 and 9.3, 5790 rows 58.5 and 27.0 (5.3 TB/s).
+template <int NC>
+__global__ __launch_bounds__(256) void qk_norm_rope_append_chunks_kernel(
+    uint16_t* __restrict__ qout, const uint16_t* __restrict__ proj,
+    int64_t proj_rs, const int32_t* __restrict__ positions,
+    const int32_t* __restrict__ slot_mapping, uint16_t* __restrict__ kcache,
+    uint16_t* __restrict__ vcache, const float* __restrict__ qnorm_w,
+    const float* __restrict__ knorm_w, const float* __restrict__ inv_freq,
+    int R, float mag, float eps, int H, int G, int N, int P, int BS, int tied,
+    int half) {
+  extern __shared__ float cs_lds[];
+  const int t = blockIdx.x, tid = threadIdx.x;
+  const uint16_t* row = proj + (int64_t)t * proj_rs;
+  const int lph = N / 8;                  // lanes of a head
+  const int qk = (H + G) * lph;           // chunks of queries and keys
+  const int all = qk + (tied ? 0 : G * P / 8);
+  const int c0 = blockIdx.y * NC * 256 + tid;
+  uint4 raw[NC];
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int c = c0 + i * 256;
+    if (c < all) raw[i] = *reinterpret_cast<const uint4*>(row + c * 8);
+  }
+  const int slot = slot_mapping[t];
+  const int64_t blk = slot / BS, off = slot % BS;
+  if (R > 0) {
+    const float pos = (float)positions[t];
+    for (int i = tid; i < R; i += 256) {
+      const float ang = pos * inv_freq[i];
+      cs_lds[i] = cosf(ang) * mag;
+      cs_lds[R + i] = sinf(ang) * mag;
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < NC; ++i) {
+    const int c = c0 + i * 256;
+    if (c >= all) break;
+    if (c >= qk) {
+      const int d = (c - qk) * 8, g = d / P;
+      *reinterpret_cast<uint4*>(vcache + ((blk * G + g) * BS + off) * P +
+                                (d - g * P)) = raw[i];
+      continue;
+    }
+    // from here on a head's lanes are here together
+    const int head = c / lph, l = c - head * lph, d0 = l * 8;
+    const uint32_t* u = reinterpret_cast<const uint32_t*>(&raw[i]);
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      x[2 * e] = bf16_to_f32((uint16_t)(u[e] & 0xffffu));
+      x[2 * e + 1] = bf16_to_f32((uint16_t)(u[e] >> 16));
+    }
+    if (head >= H && tied)
+      *reinterpret_cast<uint4*>(
+          vcache + ((blk * G + (head - H)) * BS + off) * P + d0) = raw[i];
+    const float* w = head < H ? qnorm_w : knorm_w;
+    float scale = 1.0f;
+    if (w) {
+      float ss = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ss += x[e] * x[e];
+      for (int o = lph >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+      scale = 1.0f / sqrtf(ss / (float)N + eps);
+    }
+    // entries d .. d + 7 of the head, of bits v
+    auto normed = [&](const float (&v)[8], int d, float (&y)[8]) {
+      float g[8] = {1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f, 1.0f};
+      if (w) {
+        *reinterpret_cast<float4*>(g) = *reinterpret_cast<const float4*>(w + d);
+        *reinterpret_cast<float4*>(g + 4) =
+            *reinterpret_cast<const float4*>(w + d + 4);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = v[e] * scale * g[e];
+    };
+    float y[8];
+    normed(x, d0, y);
+    if (R > 0 && half) {
+      // entries R away are another lane's; R is a multiple of 8
+      const int r = R / 8, m = l < r ? l + r : l < 2 * r ? l - r : l;
+      const int from = (int)(threadIdx.x & 63) - l + m;
+      float v[8], z[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t b = __shfl((int)u[e], from, 64);
+        v[2 * e] = bf16_to_f32((uint16_t)(b & 0xffffu));
+        v[2 * e + 1] = bf16_to_f32((uint16_t)(b >> 16));
+      }
+      normed(v, m * 8, z);
+      if (l < 2 * r) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int a = (l < r ? d0 : d0 - R) + e;
+          const float cs = cs_lds[a], sn = cs_lds[R + a];
+          y[e] = l < r ? y[e] * cs - z[e] * sn : y[e] * cs + z[e] * sn;
+        }
+      }
+    } else if (d0 < 2 * R) {   // R is a multiple of 4
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float cs = cs_lds[d0 / 2 + e], sn = cs_lds[R + d0 / 2 + e];
+        const float a = y[2 * e], b = y[2 * e + 1];
+        y[2 * e] = a * cs - b * sn;
+        y[2 * e + 1] = b * cs + a * sn;
+      }
+    }
+    uint4 out;
+    uint32_t* o = reinterpret_cast<uint32_t*>(&out);
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      o[e] = (uint32_t)f32_to_bf16(y[2 * e]) |
+             ((uint32_t)f32_to_bf16(y[2 * e + 1]) << 16);
+    uint16_t* dst = head < H
+                        ? qout + ((int64_t)t * H + head) * N + d0
+                        : kcache + ((blk * G + (head - H)) * BS + off) * N + d0;
+    *reinterpret_cast<uint4*>(dst) = out;
+  }
+}
+
 void qk_norm_rope_append(torch::Tensor qout, torch::Tensor proj,
                          torch::Tensor positions, torch::Tensor slot_mapping,
                          torch::Tensor kcache, torch::Tensor vcache,
@@ -223,6 +352,42 @@ void qk_norm_rope_append(torch::Tensor qout, torch::Tensor proj,
   }
   if (T == 0) return;
   hipStream_t stream = at::cuda::getCurrentCUDAStream();
+  // 16-byte chunks: heads that a wave holds whole, everything on 16 bytes
+  auto on16 = [](const void* p) {
+    return (reinterpret_cast<uintptr_t>(p) & 15) == 0;
+  };
+  if (proj.scalar_type() == torch::kBFloat16 &&
+      (N == 64 || N == 128 || N == 256) && P % 8 == 0 &&
+      R % (half ? 8 : 4) == 0 && proj.stride(0) % 8 == 0 &&
+      on16(proj.data_ptr()) && on16(qout.data_ptr()) &&
+      on16(kcache.data_ptr()) && on16(vcache.data_ptr()) &&
+      (!qnorm_w.has_value() ||
+       (on16(qnorm_w->data_ptr()) && on16(knorm_w->data_ptr())))) {
+    const int64_t per =
+        ((int64_t)(H + G) * N + (tied ? 0 : (int64_t)G * P) + 2047) / 2048;
+    // a thread has one chunk up to four workgroups a compute unit, then its row's
+    const int nc = T * per <= 1024 ? 1 : (int)std::min<int64_t>(per, 4);
+#define LAUNCH_QKC(NC)                                                        \
+  hipLaunchKernelGGL(                                                         \
+      (qk_norm_rope_append_chunks_kernel<NC>),                                \
+      dim3(T, (unsigned)((per + NC - 1) / NC)), dim3(256),                    \
+      (size_t)(2 * R) * sizeof(float), stream, (uint16_t*)qout.data_ptr(),    \
+      (const uint16_t*)proj.data_ptr(), (int64_t)proj.stride(0),              \
+      (const int32_t*)positions.data_ptr(),                                   \
+      (const int32_t*)slot_mapping.data_ptr(), (uint16_t*)kcache.data_ptr(),  \
+      (uint16_t*)vcache.data_ptr(),                                           \
+      qnorm_w.has_value() ? (const float*)qnorm_w->data_ptr() : nullptr,      \
+      knorm_w.has_value() ? (const float*)knorm_w->data_ptr() : nullptr,      \
+      R ? (const float*)inv_freq->data_ptr() : nullptr, R, (float)mag,        \
+      (float)eps, H, G, N, P, BS, tied ? 1 : 0, half ? 1 : 0)
+    if (nc == 1) LAUNCH_QKC(1);
+    else if (nc == 2) LAUNCH_QKC(2);
+    else if (nc == 3) LAUNCH_QKC(3);
+    else LAUNCH_QKC(4);
+#undef LAUNCH_QKC
+    HIP_CHECK_KERNEL();
+    return;
+  }
   // pair accesses need even sizes and an aligned start of every row
   const int64_t es = proj.element_size();
   const bool paired =
