@@ -1263,9 +1263,11 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
 // ones without limits (50 us); an exponential is four cycles a logit of the 7 us a
 // row's arithmetic takes; then the serial end of a row, four barriers.
 // 1024 rows of 128256, greedy / top-k 50 and top-p / top-p 0.9 / top-k 40 / no limits /
-// mixed: 41.6, 62, 124, 54, 50 and 89 us; held in registers, one row a compute unit
-// whose passes follow its loads, 54, 123, 185, 99, 103 and 144.  64 rows mixed 39.9 for
-// 42.5; 1024 of 66000, mixed, 60 for 98.  Up to 65536 logits the register kernel has
+// mixed: 41.6, 62, 124, 54, 50 and 77 us; held in registers, one row a compute unit
+// whose passes follow its loads, 54, 123, 185, 99, 103 and 140.  64 rows mixed 39.9 for
+// 42.5.  A flat top-p row takes twice as long as another: of more rows than are on
+// the chip at once (two a compute unit) those start first, which costs a
+// microsecond a row (1024 mixed rows in the order of the call 92 us, so 77).  Up to 65536 logits the register kernel has
 // two rows on a unit and is ahead (1024 of 49000, mixed, 49.3, here 50.7; of 32000 36.3
 // and 43).
 // ---------------------------------------------------------------------------
@@ -1276,6 +1278,7 @@ constexpr int SS_WINDOW = 4096;          // keys that are counted at a time
 constexpr int SS_OCTAVE = 128;           // keys of an octave
 constexpr int SS_ABOVE = 512;            // of the window, above the first maximum
 constexpr int SS_NARROW = 512;           // keys that a wave looks through alone
+constexpr int SS_ORDERED = 4096;         // rows that are put in order: 64 words
 
 // Not fmaxf, which would quiet each operand first; rows with a NaN are found by
 // their bits or their mass and done again.
@@ -1300,6 +1303,44 @@ DEVINLINE uint32_t ss_bins(uint32_t keys, uint32_t top, uint32_t spare) {
       __builtin_elementwise_min(b, __builtin_bit_cast(ushort2v, spare)));
 }
 
+// Row of a workgroup when those that can take another pass (top-p without a top-k
+// that its list serves) start first.  Every wave finds it for itself from
+// the rows' settings, 64 rows in a word of `words`, which is free again behind the
+// next barrier.
+template <int WAVES>
+DEVINLINE int ss_long_first(uint64_t* words, int wave, int V,
+                            const float* temperature, const int32_t* top_k,
+                            const float* top_p) {
+  const int lane = threadIdx.x & 63, B = gridDim.x;
+  const int groups = (B + 63) / 64;
+  for (int g = wave; g < groups; g += WAVES) {
+    const int r = min(g * 64 + lane, B - 1);
+    const int k = top_k[r];
+    const bool later = temperature[r] <= 0.0f || !(top_p[r] < 1.0f) ||
+                       (k > 0 && k < V && k <= 32 * WAVES);
+    const uint64_t word = __ballot(!later && g * 64 + lane < B);
+    if (lane == 0) words[g] = word;
+  }
+  __syncthreads();
+  uint64_t own = lane < groups ? words[lane] : 0;
+  const int first = __builtin_amdgcn_readlane(sr_scan(__popcll(own)), 63);
+  int at = blockIdx.x;
+  if (at >= first) {   // among the others
+    at -= first;
+    const int n = min(max(B - lane * 64, 0), 64);
+    own = ~own & (n == 64 ? ~0ull : (1ull << n) - 1);
+  }
+  const int n = __popcll(own), to = sr_scan(n);
+  const int g = __builtin_ctzll(__ballot(to > at));
+  at -= __builtin_amdgcn_readlane(to - n, g);
+  const uint64_t word =
+      (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(own >> 32), g) << 32 |
+      (uint32_t)__builtin_amdgcn_readlane((int)own, g);
+  const bool mine = (word >> lane & 1) &&
+                    __popcll(word & ((1ull << lane) - 1)) == at;
+  return g * 64 + __builtin_ctzll(__ballot(mine));
+}
+
 template <int SS_THREADS>
 __global__ __launch_bounds__(SS_THREADS, 4) void sample_bf16_stream_kernel(
     int32_t* __restrict__ out,             // [B]
@@ -1308,7 +1349,7 @@ __global__ __launch_bounds__(SS_THREADS, 4) void sample_bf16_stream_kernel(
     const int32_t* __restrict__ top_k,     // [B] (<=0 => disabled)
     const float* __restrict__ top_p,       // [B] (>=1 => disabled)
     const float* __restrict__ uniforms,    // [B]
-    int V) {
+    int V, bool ordered) {
   constexpr int SS_WAVES = SS_THREADS / WAVE_SIZE;
   constexpr int SS_LIST = SS_THREADS == 512 ? 3072 : 4096;   // as the LDS takes
   constexpr int U = SS_U, UNIT = SS_UNIT;
@@ -1331,10 +1372,13 @@ __global__ __launch_bounds__(SS_THREADS, 4) void sample_bf16_stream_kernel(
   __shared__ int s_list, s_bad, s_kept, s_last, s_tau, s_top, s_cell;
   __shared__ uint32_t s_pick;
 
-  const int seq = blockIdx.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int seq =
+      ordered ? ss_long_first<SS_WAVES>(reinterpret_cast<uint64_t*>(cells), wave,
+                                        V, temperature, top_k, top_p)
+              : blockIdx.x;
   const uint16_t* row = logits + (int64_t)seq * V;
   const float temp = temperature[seq];
   const bool greedy = temp <= 0.0f;
@@ -2141,7 +2185,8 @@ void sample(torch::Tensor out, torch::Tensor logits, torch::Tensor temperature,
                      (const float*)temperature.data_ptr(),                    \
                      (const int32_t*)top_k.data_ptr(),                        \
                      (const float*)top_p.data_ptr(),                          \
-                     (const float*)uniforms.data_ptr(), V)
+                     (const float*)uniforms.data_ptr(), V,                    \
+                     B > 512 && B <= SS_ORDERED)
       if (B <= 256) LAUNCH_STREAM(1024);
       else LAUNCH_STREAM(512);
 #undef LAUNCH_STREAM
