@@ -254,7 +254,7 @@ DEVINLINE int ft_vswz(int r) {
 }
 
 // Swizzle of the 16-byte chunks of K row r, rows of NK entries: 256 bytes apart
-// in the banks' 256 (or a multiple), or 128 (with SHARED the transposing reads
+// in the banks' 256 (or a multiple), or 128 (latent_decode's transposing reads
 // of four neighbouring rows want bit 2 to tell rows 0 and 2 apart).  By r & 7
 // two rows met in a bank at every fragment.
 template <int NK>
@@ -270,19 +270,18 @@ DEVINLINE int ft_kswz(int r) {
 // PLAIN: causal only, the maximum is of raw scores.
 // VD < NV: the four waves have the SAME 32 query rows and each the VD value
 // dims from dim0 on (decoded rows: the heads that share keys).
-// SHARED: the values are the first entries of the key rows, v0 and v1 unused.
 // ONCE: decoded rows, whose keys nobody reads again soon: loads are nontemporal and
 // leave nothing in the memory side's cache.
 template <int NK, int NV, bool PLAIN, class Rows, int VD = NV,
-          bool SHARED = false, bool ONCE = false>
+          bool ONCE = false>
 DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
                            const FlashScore& sc,
                            const ft_bf16x8 (&qf)[NK / 16], uint8_t* k0,
                            uint8_t* k1, uint8_t* v0, uint8_t* v1,
                            ft_f32x16 (&o)[VD / 32], float& m, float& l,
                            int dim0 = 0) {
-  constexpr int BN = FT_BN, CK = NK / 8, CV = SHARED ? 0 : NV / 8;
-  constexpr int VROW = SHARED ? NK * 2 : NV * 2;   // bytes of a V row
+  constexpr int BN = FT_BN, CK = NK / 8, CV = NV / 8;
+  constexpr int VROW = NV * 2;        // bytes of a V row
   constexpr int RW = BN / FT_WAVES;   // rows that a wave moves
   constexpr int AUX = ONCE ? 2 : 0;
   const int lane = threadIdx.x & 63;
@@ -294,16 +293,15 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
   auto k_chunk = [&](int i) {
     return ((i * 64 + lane) % CK) ^ ft_kswz<NK>(k_row(i));
   };
-  constexpr int CV1 = CV > 0 ? CV : 1;
-  auto v_row = [&](int i) { return wave * RW + (i * 64 + lane) / CV1; };
+  auto v_row = [&](int i) { return wave * RW + (i * 64 + lane) / CV; };
   auto v_chunk = [&](int i) {
-    return ((i * 64 + lane) % CV1) ^ ft_vswz<NV>(v_row(i));
+    return ((i * 64 + lane) % CV) ^ ft_vswz<NV>(v_row(i));
   };
   // Addresses of whole tiles cost the vector units nothing: they are a scalar
   // base and these offsets (64-bit sums per lane were a third of the vector
   // instructions of a tile).
   constexpr bool STRAIGHT = Rows::STRAIGHT && NK <= 256;
-  int ko[CK / 4], vo[CV / 4 + 1];
+  int ko[CK / 4], vo[CV / 4];
   if constexpr (STRAIGHT) {
 #pragma unroll
     for (int i = 0; i < CK / 4; ++i) ko[i] = rows.k_off(k_row(i), k_chunk(i));
@@ -370,7 +368,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
       const int c =
           dim0 / 8 + 4 * dt + 2 * ((lane >> 4) & 1) + ((i & 3) >> 1);
       voff[dt][e] = r * VROW +
-                    ((c ^ (SHARED ? ft_kswz<NK>(r) : ft_vswz<NV>(r))) << 4) +
+                    ((c ^ ft_vswz<NV>(r)) << 4) +
                     8 * (i & 1);
     }
 
@@ -520,7 +518,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
 #pragma unroll
         for (int e = 0; e < 2; ++e)
           vf[j & 1][dt].h[e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-              (lds_short4*)((SHARED ? kb : vb) + voff[dt][e] + 16 * j * VROW));
+              (lds_short4*)(vb + voff[dt][e] + 16 * j * VROW));
     };
     __builtin_amdgcn_sched_barrier(0);
     read_v(0);

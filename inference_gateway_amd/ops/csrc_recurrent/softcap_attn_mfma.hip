@@ -497,7 +497,7 @@ __global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_decode_kernel(
                  a.N, a.P, pos + 1};
   ft_f32x16 o[VD / 32];
   float m, l;
-  flash_tiles<NP, PP, false, PagedRows, VD, false, ONCE>(
+  flash_tiles<NP, PP, false, PagedRows, VD, ONCE>(
       rows, span, sc, qf, k_s0, k_s1, v_s0, v_s1, o, m, l, wave * VD);
   if (!real) return;
   if (parts.nsplit > 1) {
