@@ -207,10 +207,13 @@ class LatentAttention(nn.Module):
                 self.kvnorm_w, self.inv_freq, self.eps, sp.q_rank,
                 sp.kv_rank, rd, H, sp.rot_half, self.mag)
             q = ops.linear(cq, self.uq).view(T, H, dn + rd)
-            ops.rope_pairs_(q, fb.positions, self.inv_freq, dn, sp.rot_half,
-                            self.mag)
         v = torch.empty((T, H, sp.vdim), dtype=h.dtype, device=h.device)
         P = self._expanded_rows(q, fb)
+        # queries without rows to write out are turned where they are absorbed
+        turn = not self.direct and not P
+        if P and not self.direct:
+            ops.rope_pairs_(q, fb.positions, self.inv_freq, dn, sp.rot_half,
+                            self.mag)
         out, row_seq, positions, slots = \
             v, fb.row_seq, fb.positions, fb.slot_mapping
         chunk_rows, lens, whole = fb.num_chunk_rows, fb.seq_lens, None
@@ -233,14 +236,17 @@ class LatentAttention(nn.Module):
         if P < T:
             if P and gate is not None:
                 gate = gate[P:]
-            q_abs = torch.bmm(q[:, :, :dn].transpose(0, 1), self.uk)
+            if turn:
+                q_abs = ops.turned_head_products(
+                    q, self.uk, positions, self.inv_freq, sp.rot_half,
+                    self.mag)
+            else:
+                q_abs = ops.head_products(q[:, :, :dn], self.uk)
             o_lat = ops.latent_attention(
-                q_abs.transpose(0, 1), q[:, :, dn:], cache,
+                q_abs, q[:, :, dn:], cache,
                 fb.seq_block_table, row_seq, positions, self.sink, sp.scale,
                 sp.window, chunk_rows, lens, fb.max_context, gate)
-            # the batched product writes head-major rows [T, H, vd] in place
-            torch.bmm(o_lat.transpose(0, 1), self.uv_t,
-                      out=out.transpose(0, 1))
+            ops.head_products(o_lat, self.uv_t, out)
         return ops.linear(v.view(T, H * sp.vdim), self.o)
 
 

@@ -653,6 +653,35 @@ def latent_attention(q_abs, q_rot, cache, block_table, row_seq, positions,
         window, gate)
 
 
+def head_products(x, w, out=None):
+    """x [T, H, K] times a matrix per head, w [H, K, N]: [T, H, N] (`out` when
+    given; strided views ok).  A few rows of bf16 run one kernel
+    (ops/csrc_hybrid/head_products.hip), everything else the library's batched
+    product."""
+    if out is None:
+        out = x.new_empty((x.shape[0], x.shape[1], w.shape[2]))
+    if not (x.is_cuda and _shared_ext("head_products")(
+            out, x, w, None, None, None, False, 1.0)):
+        torch.bmm(x.transpose(0, 1), w, out=out.transpose(0, 1))
+    return out
+
+
+def turned_head_products(q, w, positions, inv_freq, half: bool = False,
+                         mag: float = 1.0):
+    """head_products of the first w.shape[1] entries of every head of q, whose
+    others are rotated in place (rope_pairs_); in one launch for a few rows of
+    bf16."""
+    K = w.shape[1]
+    x = q[:, :, :K]
+    if q.is_cuda and q.shape[2] == K + 2 * inv_freq.numel():
+        out = q.new_empty((q.shape[0], q.shape[1], w.shape[2]))
+        if _shared_ext("head_products")(out, x, w, q[:, :, K:], positions,
+                                        inv_freq, half, mag):
+            return out
+    rope_pairs_(q, positions, inv_freq, K, half, mag)
+    return head_products(x, w)
+
+
 def latent_prompt_fits(q, rot_dim: int, vdim: int, kv_rank: int = 0) -> bool:
     """Whether latent_prompt_attention takes queries q [P, H, dim + rot_dim],
     values of vdim entries and rotated keys that stand behind kv_rank entries

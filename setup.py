@@ -40,7 +40,7 @@ recurrent_sources = [str(REC / "bindings.cpp")] + _hip_sources(REC) + [str(HYB /
 # attention and row kernels that its models launch
 PN = ROOT / "inference_gateway_amd" / "ops" / "csrc_postnorm"
 postnorm_sources = [str(PN / "bindings.cpp")] + [
-    str(HYB / f) for f in ("hybrid_ops.hip", "latent_attn.hip",
+    str(HYB / f) for f in ("head_products.hip", "hybrid_ops.hip", "latent_attn.hip",
                            "latent_attn_mfma.hip", "latent_decode.hip",
                            "latent_prompt.hip",
                            "parallel_ops.hip")] + [
@@ -50,7 +50,7 @@ postnorm_sources = [str(PN / "bindings.cpp")] + [
 # the multi-stream extension: its own kernels plus the attention, row and
 # router kernels its models launch
 streams_sources = [str(STR / "bindings.cpp")] + _hip_sources(STR) + [
-    str(HYB / f) for f in ("hybrid_ops.hip", "latent_attn.hip",
+    str(HYB / f) for f in ("head_products.hip", "hybrid_ops.hip", "latent_attn.hip",
                            "latent_attn_mfma.hip", "latent_decode.hip",
                            "latent_prompt.hip",
                            "parallel_ops.hip")] + [
