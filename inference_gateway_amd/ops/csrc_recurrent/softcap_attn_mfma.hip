@@ -512,6 +512,302 @@ __global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_decode_kernel(
                   });
 }
 
+// Decoded rows of keys and values of 128 entries in pages of 16 tokens, up to eight
+// heads on a key head: every wave walks pages of its own, two at a time, K to
+// registers in whole lines (LineTurn), V by DMA to LDS, both one step ahead, as in
+// the engine's own decode attention: nothing waits for another wave until the
+// end, and 128 KB are under way on a compute unit where the tiles above have 64.
+// S^T = K Q^T with the heads in the columns of mfma 16x16x32; the order of its
+// rows is the one that V is read in (ds_read_b64_tr_b16), so weights stay in their
+// lanes.  The waves' sums meet in LDS once.
+//
+// Bound by the cache's bytes where there are workgroups for the chip, else by a walk's
+// latency.  Measured, the tiles above and this (us, eight caches in turn, 32 heads
+// on 8, distance bias and head gate): 48 of 700 to 3500, the last 1024 and the first
+// 16 keys, 49.7 and 38.2, all 94.5 and 83.6, of 2000 with a score cap 93.6 and 70.2,
+// 128 of 100 to 1000 77.2 and 57.3, 256 of 2048 356 and 336 (6.4 TB/s), 700 of 200
+// 178 and 112, one of 3000 15.5 and 13.3, 64 of 20 10.7 and 6.6; 32 on 4, the last
+// 512, 48 of 2000 21.0 and 19.2.  With 16 on 1, where a page's bytes are a 32nd of
+// a workgroup's, they are behind (48 of 2000 21.4 and 22.5).
+constexpr int SD_HD = 128, SD_BS = 16, SD_PAGE = SD_HD * SD_BS;
+
+DEVINLINE float sd_quads(float x, bool max) {   // of lanes l, l ^ 16, l ^ 32
+  float a = x, b = x;
+  asm("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 0" : "+v"(a), "+v"(b));
+  x = max ? fmaxf(a, b) : a + b;
+  ft_both_halves(x, a, b);
+  return max ? fmaxf(a, b) : a + b;
+}
+
+DEVINLINE void softcap_pages_body(const SoftcapArgs& a, const FlashClose& close,
+                                  const FlashParts& parts) {
+  typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+  constexpr int HD = SD_HD, BS = SD_BS, PAGE = SD_PAGE, WAVES = FT_WAVES;
+  // two objects, so that reads of one do not wait for loads to the other
+  __shared__ __attribute__((aligned(1024))) uint16_t v_s0[WAVES][2 * PAGE];
+  __shared__ __attribute__((aligned(1024))) uint16_t v_s1[WAVES][2 * PAGE];
+  __shared__ __attribute__((aligned(1024))) u32x4 k_s[WAVES][128];
+  __shared__ float m_s[WAVES][16], l_s[WAVES][16];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, quad = lane >> 4;
+  const int row = blockIdx.x, seq = a.nprompt + row;
+  const int rep = a.H / a.G, kvh = blockIdx.y;
+  const int64_t tok = a.seq_cu[seq];
+  const int pos = __builtin_amdgcn_readfirstlane(a.seq_start[seq]);
+
+  // visible pages: the kept ones, then from the window's first on; this part's
+  int lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
+  if (a.chunk > 0) lo = max(lo, pos / a.chunk * a.chunk);
+  const int first = lo / BS;
+  const int kept = a.keep > 0 ? min((a.keep + BS - 1) / BS, first) : 0;
+  const int pages = kept + pos / BS + 1 - first;
+  const int per = ((pages + parts.nsplit - 1) / parts.nsplit + 1) & ~1;
+  const int page0 = blockIdx.z * per, page1 = min(page0 + per, pages);
+  const int pairs = (page1 - page0 + 1) >> 1;   // wave, wave + WAVES, ...
+  auto page_at = [&](int i) FT_INLINE { return i < kept ? i : first + i - kept; };
+
+  // page numbers of this wave's next 32 pairs, one per lane
+  const int32_t* table = a.block_table + (int64_t)seq * a.max_blocks;
+  int ids = 0;
+  auto load_ids = [&](int u) FT_INLINE {
+    const int i = page0 + 2 * (u + (lane >> 1) * WAVES) + (lane & 1);
+    ids = table[page_at(min(i, page1 - 1))];
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // here, not at every use
+  };
+  if (wave < pairs) load_ids(wave);
+
+  // the heads as columns, dims 32 kk + 8 quad ..; past the last the first one's
+  const int head = kvh * rep + (r16 < rep ? r16 : 0);
+  ft_bf16x8 qf[4];
+  const uint16_t* qp = a.q + tok * a.q_rs + (int64_t)head * HD + quad * 8;
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk)
+    qf[kk] = *reinterpret_cast<const ft_bf16x8*>(qp + kk * 32);
+  const float c =
+      a.scale * FT_LOG2E *
+      (1.0f + a.temp_coef * logf((float)((pos + 1) / a.temp_every) + 1.0f));
+  const float cap = a.softcap > 0.0f ? a.softcap * FT_LOG2E : 0.0f;
+  // tanh by exp2: cap - 2 cap / (1 + 2^(cap_k s))
+  const float cap_k = cap > 0.0f ? 2.0f * FT_LOG2E * c / cap : 0.0f;
+  const float slope = a.slopes ? a.slopes[head] * FT_LOG2E : 0.0f;
+
+  // lane offsets into a page, bytes: K half a row of eight rows a load; V four rows
+  // a load, 16-byte chunks exchanged so that the eight rows which 32 lanes
+  // of a transposing read take 32 bytes of each lie in different banks
+  const int kx = (lane >> 3) * HD * 2 + (lane & 7) * 16;
+  const LineTurn turn(lane);
+  int vx[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = i * 4 + quad;
+    vx[i] = r * HD * 2 + ((r16 ^ ((r & 7) << 1)) << 4);
+  }
+  struct Keys {
+    u32x4 k[2][4];
+  };
+  typedef __attribute__((address_space(3))) void lds_void;
+  // pair u; rows past the part's end or the row's position read as zeros
+  auto fetch = [&](int u, Keys& K, uint16_t* vs) FT_INLINE {
+    const int at = (u - wave) / WAVES;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int i = page0 + 2 * u + h;
+      const int64_t id = __builtin_amdgcn_readlane(ids, (at & 31) * 2 + h);
+      const int64_t base = (id * a.G + kvh) * PAGE;
+      const int rows = __builtin_amdgcn_readfirstlane(
+          i < page1 ? max(0, min(BS, pos + 1 - page_at(i) * BS)) : 0);
+      const auto kr = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(a.kcache + base), 0, rows * HD * 2, 0x00020000);
+      const auto vr = __builtin_amdgcn_make_buffer_rsrc(
+          (void*)(a.vcache + base), 0, rows * HD * 2, 0x00020000);
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+        K.k[h][kk] = __builtin_amdgcn_raw_buffer_load_b128(
+            kr, kx + (kk >> 1) * 128 + (kk & 1) * 8 * HD * 2, 0, 2);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            vr, (lds_void*)(vs + h * PAGE + j * 512), 16, vx[j], 0, 0, 2);
+    }
+  };
+
+  // O^T: column r16, dims 16 d + 4 quad ..; m in log2, l of this lane's tokens
+  typedef __attribute__((ext_vector_type(4))) float f32x4;
+  f32x4 acc[8];
+#pragma unroll
+  for (int d = 0; d < 8; ++d) acc[d] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  float m = -INFINITY, l = 0.0f;
+  // V's rows as operands: dims 16 d + r16, tokens 4 quad ..
+  const int vrow = 4 * quad + (r16 >> 2);
+  const int vat = vrow * HD + ((r16 & 3) >> 1) * 8 + (r16 & 1) * 4;
+  auto use = [&](int u, const Keys& K, uint16_t* vs) FT_INLINE {
+    f32x4 s[2];
+    u32x4 kf[2][4];
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        turn(k_s[wave], K.k[h][2 * e], K.k[h][2 * e + 1], kf[h][2 * e],
+             kf[h][2 * e + 1]);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) s[h] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        s[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            __builtin_bit_cast(ft_bf16x8, kf[h][kk]), qf[kk], s[h], 0, 0, 0);
+    // token 4 quad + j % 4 of page j / 4
+    float t[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) t[j] = s[j >> 2][j & 3];
+    if (cap > 0.0f) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        t[j] = fmaf(-2.0f * cap,
+                    __builtin_amdgcn_rcpf(
+                        1.0f + __builtin_amdgcn_exp2f(t[j] * cap_k)),
+                    cap);
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) t[j] *= c;
+    }
+    const int i = page0 + 2 * u;
+    const int key0 = page_at(i) * BS, key1 = page_at(i + 1) * BS;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      t[j] = fmaf((float)((j < 4 ? key0 : key1) + 4 * quad + (j & 3) - pos),
+                  slope, t[j]);
+    if (i + 1 >= page1 || key1 + BS > pos + 1 || key0 < lo || key1 < lo) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int key = (j < 4 ? key0 : key1) + 4 * quad + (j & 3);
+        if ((j >= 4 && i + 1 >= page1) || key > pos ||
+            (key < lo && key >= a.keep))
+          t[j] = -INFINITY;
+      }
+    }
+    float mx = t[0];
+#pragma unroll
+    for (int j = 1; j < 8; ++j) mx = fmaxf(mx, t[j]);
+    mx = sd_quads(mx, true);
+    if (__any(mx > m)) {
+      const float mn = fmaxf(m, mx);
+      const float alpha =
+          m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
+      m = mn;
+      l *= alpha;
+#pragma unroll
+      for (int d = 0; d < 8; ++d) acc[d] *= alpha;
+    }
+    const float mc = m == -INFINITY ? 0.0f : m;
+    float p[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) p[j] = __builtin_amdgcn_exp2f(t[j] - mc);
+    l += ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+    union {
+      uint32_t u[4];
+      ft_bf16x8 v;
+    } w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) w.u[e] = ft_pack_bf16(p[2 * e], p[2 * e + 1]);
+    typedef __attribute__((address_space(3))) ft_short4 lds_short4;
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      union {
+        ft_short4 h[2];
+        ft_bf16x8 v;
+      } vf;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        vf.h[h] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+            (lds_short4*)(vs + h * PAGE + vat + ((d ^ (vrow & 7)) << 4)));
+      acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, w.v, acc[d], 0, 0,
+                                                       0);
+    }
+  };
+
+  Keys k0, k1;
+  auto ahead = [&](int u, Keys& K, uint16_t* vs) FT_INLINE {
+    if ((((u - wave) / WAVES) & 31) == 0 && u < pairs) load_ids(u);
+    fetch(u, K, vs);
+  };
+  if (wave < pairs) {
+    fetch(wave, k0, v_s0[wave]);
+    for (int u = wave;; u += 2 * WAVES) {
+      ahead(u + WAVES, k1, v_s1[wave]);
+      use(u, k0, v_s0[wave]);
+      if (u + WAVES >= pairs) break;
+      ahead(u + 2 * WAVES, k0, v_s0[wave]);
+      use(u + WAVES, k1, v_s1[wave]);
+      if (u + 2 * WAVES >= pairs) break;
+    }
+  }
+  l = sd_quads(l, false);
+
+  // the waves' sums meet in the memory of the V tiles (loads that are still
+  // under way there read nothing, and are waited for first)
+  float* sums = reinterpret_cast<float*>(&v_s0[0][0]);   // [WAVES][16][HD]
+  static_assert(sizeof(v_s0) == WAVES * 16 * HD * sizeof(float));
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  __syncthreads();
+  if (quad == 0) {
+    m_s[wave][r16] = m;
+    l_s[wave][r16] = l;
+  }
+  if (r16 < rep) {
+#pragma unroll
+    for (int d = 0; d < 8; ++d)
+      *reinterpret_cast<f32x4*>(sums + (wave * 16 + r16) * HD + d * 16 +
+                                quad * 4) = acc[d];
+  }
+  __syncthreads();
+  for (int i = tid; i < rep * (HD / 4); i += 64 * WAVES) {
+    const int j = i / (HD / 4), d = i % (HD / 4) * 4;
+    float M = m_s[0][j], L = 0.0f;
+#pragma unroll
+    for (int w = 1; w < WAVES; ++w) M = fmaxf(M, m_s[w][j]);
+    float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = m_s[w][j] == -INFINITY
+                          ? 0.0f
+                          : __builtin_amdgcn_exp2f(m_s[w][j] - M);
+      const float4 x =
+          *reinterpret_cast<const float4*>(sums + (w * 16 + j) * HD + d);
+      L = fmaf(f, l_s[w][j], L);
+      o.x = fmaf(f, x.x, o.x);
+      o.y = fmaf(f, x.y, o.y);
+      o.z = fmaf(f, x.z, o.z);
+      o.w = fmaf(f, x.w, o.w);
+    }
+    const int at = kvh * rep + j;
+    if (parts.nsplit > 1) {
+      const int64_t slot =
+          ((int64_t)row * a.H + at) * parts.nsplit + blockIdx.z;
+      *reinterpret_cast<float4*>(parts.o + slot * HD + d) = o;
+      if (d == 0) {
+        parts.ml[2 * slot] = M;
+        parts.ml[2 * slot + 1] = L;
+      }
+    } else {
+      const float inv = 1.0f / close.sum(at, M, L);
+      uint2 y;
+      y.x = ft_pack_bf16(o.x * (inv * close.factor(tok, at, d)),
+                         o.y * (inv * close.factor(tok, at, d + 1)));
+      y.y = ft_pack_bf16(o.z * (inv * close.factor(tok, at, d + 2)),
+                         o.w * (inv * close.factor(tok, at, d + 3)));
+      *reinterpret_cast<uint2*>(a.out + (tok * a.H + at) * HD + d) = y;
+    }
+  }
+}
+
+__global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_pages_kernel(
+    SoftcapArgs a, FlashClose close, FlashParts parts) {
+  softcap_pages_body(a, close, parts);
+}
+
 // prompt_rows: row counts of the first sequences of the batch; the other
 // sequences bring one decoded row each.  Returns false when the sizes do not
 // fit the tile kernels.
@@ -627,10 +923,12 @@ bool softcap_attention_mfma(torch::Tensor out, torch::Tensor q,
     }
     const dim3 grid(ndec, groups, nsplit), block(64 * FT_WAVES);
     const bool once = H / G <= 32;
-    auto* kern = N <= 64 ? once ? softcap_decode_kernel<64, true>
-                                : softcap_decode_kernel<64, false>
-                 : once  ? softcap_decode_kernel<128, true>
-                         : softcap_decode_kernel<128, false>;
+    const bool in_pages = N == SD_HD && P == SD_HD && BS == SD_BS && H / G <= 8;
+    auto* kern = in_pages  ? softcap_pages_kernel
+                 : N <= 64 ? once ? softcap_decode_kernel<64, true>
+                                  : softcap_decode_kernel<64, false>
+                 : once    ? softcap_decode_kernel<128, true>
+                           : softcap_decode_kernel<128, false>;
     hipLaunchKernelGGL(kern, grid, block, 0, stream, a, close, parts);
     HIP_CHECK_KERNEL();
     if (nsplit > 1) {
