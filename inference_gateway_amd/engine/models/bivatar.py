@@ -33,6 +33,7 @@ import torch.nn.functional as F
 
 from ... import ops
 from ...parallel.comm import tp_world_size
+from ...parallel.layers import calls_plainly
 from ..config import BivatarConfig, GatedFFSpec, WindowAttentionSpec
 from .batch import ForwardBatch
 from .bozolorn import _norm_w, _w
@@ -129,13 +130,23 @@ class PostNormLayer(nn.Module):
         sublayer's output and the weight of its norm, added inside this
         sublayer's fused residual kernel.  Returns this layer's last
         un-added pair."""
+        return self.step(residual, delta, w_post, fb, cache, False)
+
+    def step(self, residual, delta, w_post, fb, cache, parts: bool):
+        """forward; with `parts` the delta that it returns may be parts of a
+        product for add_normed_rmsnorm to add (ops.linear_parts)."""
         x = ops.add_normed_rmsnorm(residual, delta, w_post, None, self.eps,
                                    self.dtype, self.mult)
         delta, w_post = self.mixer(x, fb, cache), self.norm1_w
         if self.mlp is not None:
             x = ops.add_normed_rmsnorm(residual, delta, w_post, None,
                                        self.eps, self.dtype, self.mult)
-            delta, w_post = self.mlp(x, fb), self.norm2_w
+            mlp, w_post = self.mlp, self.norm2_w
+            if parts and calls_plainly(mlp, GatedMLP):
+                delta = ops.linear_parts(
+                    ops.linear_gated_act(x, mlp.gate_up, mlp.mode), mlp.down)
+            else:
+                delta = mlp(x, fb)
         return delta, w_post
 
 
@@ -176,7 +187,11 @@ class BivatarForCausalLM(nn.Module):
         delta = w_post = None
         for i, layer in enumerate(self.layers):
             cache = caches[layer.kv_from if layer.kv_from >= 0 else i]
-            delta, w_post = layer(residual, delta, w_post, fb, cache)
+            if self.tap is None and calls_plainly(layer, PostNormLayer):
+                delta, w_post = layer.step(residual, delta, w_post, fb, cache,
+                                           True)
+            else:
+                delta, w_post = layer(residual, delta, w_post, fb, cache)
             if self.tap is not None:
                 d = delta.float()
                 self.tap(i, residual + cfg.residual_mult * d * torch.rsqrt(

@@ -285,6 +285,19 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias=None) -> torch.Tensor:
     return torch.nn.functional.linear(x, w, bias) if out is None else out
 
 
+def linear_parts(x: torch.Tensor, w: torch.Tensor):
+    """linear(x, w) for add_normed_rmsnorm: where the product's K is in parts
+    (ops/csrc/few_rows.hip) and a row stays in that kernel's registers, their fp32
+    sums [S, M, N], which it adds; else the product."""
+    if (x.is_cuda and HAS_KERNELS and not torch.compiler.is_compiling()
+            and not has_torch_function_variadic(x, w)
+            and w.shape[0] <= 8192 and w.shape[0] % 4 == 0):
+        out = _kernels.linear_parts(x, w)
+        if out is not None:
+            return out
+    return linear(x, w)
+
+
 def linear_add_rmsnorm(x: torch.Tensor, w: torch.Tensor,
                        residual: torch.Tensor, weight: torch.Tensor,
                        eps: float):
@@ -1184,8 +1197,9 @@ def add_normed_rmsnorm(residual, delta, w_post, w_pre, eps: float,
                        out_dtype, mult: float = 1.0):
     """Step of a layer that norms its sublayers' outputs: residual [T, D]
     fp32 += mult * rmsnorm(delta) * w_post (in place; delta None = nothing
-    added), then returns rmsnorm(residual) * w_pre in out_dtype (w_pre
-    None: the residual itself in out_dtype).  Weights fp32 [D]."""
+    added; [S, T, D] fp32 = the sum of S parts), then returns
+    rmsnorm(residual) * w_pre in out_dtype (w_pre None: the residual itself in
+    out_dtype).  Weights fp32 [D]."""
     if residual.is_cuda:
         out = torch.empty(residual.shape, dtype=out_dtype,
                           device=residual.device)

@@ -80,6 +80,8 @@ c10::optional<torch::Tensor> linear_add_rmsnorm(const torch::Tensor& x,
                                                 const torch::Tensor& residual,
                                                 const torch::Tensor& weight,
                                                 double eps);
+c10::optional<torch::Tensor> linear_parts(const torch::Tensor& x,
+                                          const torch::Tensor& w);
 void held_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias);
 int64_t product_kernel(const torch::Tensor& x, const torch::Tensor& w,
@@ -183,6 +185,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "as few_rows_takes, of a product in parts that a norm follows");
   m.def("linear_add_rmsnorm", &igw::linear_add_rmsnorm,
         "residual += x W^T and its norm, None: nothing done");
+  m.def("linear_parts", &igw::linear_parts,
+        "the sums of the parts of K of x W^T, None: not in parts");
   m.def("wide_gemm", &igw::wide_gemm,
         "x W^T of hundreds to thousands of rows on a given tile");
   m.def("wide_gemm_tile", &igw::wide_gemm_tile,

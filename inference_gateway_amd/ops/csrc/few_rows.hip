@@ -268,6 +268,21 @@ c10::optional<torch::Tensor> linear_add_rmsnorm(const torch::Tensor& x,
   return out;
 }
 
+// The product that few_rows would make of parts of K (gate 0, no bias) as those parts,
+// fp32 [S, M, N], for a kernel that adds them as it reads; nothing where it has none.
+c10::optional<torch::Tensor> linear_parts(const torch::Tensor& x,
+                                          const torch::Tensor& w) {
+  const Route r = product_route(x, w, c10::nullopt, 0, false);
+  const int64_t M = x.dim() == 2 ? x.size(0) : 0;
+  const torch::Tensor none;
+  if (r.kernel == 5) return split_parts(x, w, r.how >> 8, r.how & 255);
+  if (r.kernel == 4 && held_splits(M, w.size(0), x.size(1)) >= 2)
+    return held_gemm_parts(none, x, w, c10::nullopt);
+  if (r.kernel == 2 && rows_gemm_splits(M, w.size(0), x.size(1), false) >= 2)
+    return rows_gemm_parts(none, x, w, c10::nullopt, 0);
+  return c10::nullopt;
+}
+
 // Whether gemv takes the product of x = rmsnorm(residual + delta) with the norm in
 // it.
 bool norm_linear_takes(const c10::optional<torch::Tensor>& delta,

@@ -14,7 +14,9 @@
 // their loads issued before the first is used; longer, odd or misaligned rows
 // are read again after each statistic.  Measured, rows read again and kept
 // (us): 6000 rows of 4096 71.0 and 47.4 (6.2 TB/s), of 8192 188 and 122; 48
-// rows of 4096 9.3 and 5.9.
+// rows of 4096 9.3 and 5.9.  A delta of several parts (a product's sums over parts of
+// its K) is added as it is read: a sum of its own takes another 4.5 us of 48 rows
+// (Bivatar's decode of 48 sequences, four such sums, 698 and 688).
 #include "../csrc_hybrid/act_types.h"
 
 namespace igw {
@@ -91,13 +93,14 @@ DEVINLINE float square4(float4 v) {
   return v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
 }
 
-// D <= 1024 NC, D % 4 == 0, rows and weights aligned to four entries
-template <typename TD, typename TO, int NC>
+// D <= 1024 NC, D % 4 == 0, rows and weights aligned to four entries.  PARTS: delta
+// is the sum of `parts` of them, part_stride entries apart.
+template <typename TD, typename TO, int NC, bool PARTS = false>
 __global__ __launch_bounds__(256) void add_normed_rmsnorm_row_kernel(
     TO* __restrict__ out, float* __restrict__ residual,
     const TD* __restrict__ delta, int64_t delta_rs,
     const float* __restrict__ w_post, const float* __restrict__ w_pre, int D,
-    float eps, float mult) {
+    float eps, float mult, int parts, int64_t part_stride) {
   __shared__ float red[8];
   const int t = blockIdx.x, tid = threadIdx.x;
   float* res = residual + (int64_t)t * D;
@@ -117,6 +120,21 @@ __global__ __launch_bounds__(256) void add_normed_rmsnorm_row_kernel(
     for (int c = 0; c < NC; ++c) {
       const int d = (c * 256 + tid) * 4;
       y[c] = d < D ? load4(dl + d) : zero;
+    }
+    if constexpr (PARTS) {
+#pragma unroll 4
+      for (int p = 1; p < parts; ++p) {
+        dl += part_stride;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          const int d = (c * 256 + tid) * 4;
+          const float4 v = d < D ? load4(dl + d) : zero;
+          y[c].x += v.x;
+          y[c].y += v.y;
+          y[c].z += v.z;
+          y[c].w += v.w;
+        }
+      }
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) sd += square4(y[c]);
@@ -166,6 +184,15 @@ void add_normed_rmsnorm(torch::Tensor out, torch::Tensor residual,
               residual.is_contiguous() && residual.dim() == 2);
   const int T = residual.size(0), D = residual.size(1);
   TORCH_CHECK(out.is_contiguous() && out.numel() == residual.numel());
+  int parts = 1;
+  int64_t part_stride = 0;
+  if (delta.has_value() && delta->dim() == 3) {
+    TORCH_CHECK(delta->dtype() == torch::kFloat32 && delta->is_contiguous() &&
+                delta->size(0) >= 1 && delta->size(0) < (1 << 16));
+    parts = (int)delta->size(0);
+    part_stride = delta->stride(0);
+    delta = delta->select(0, 0);
+  }
   if (delta.has_value()) {
     TORCH_CHECK(delta->dim() == 2 && delta->size(0) == T &&
                 delta->size(1) == D && delta->stride(1) == 1);
@@ -192,14 +219,24 @@ void add_normed_rmsnorm(torch::Tensor out, torch::Tensor residual,
       by4(residual.data_ptr(), 4) &&
       by4(out.data_ptr(), out.element_size()) &&
       (!delta.has_value() || by4(delta->data_ptr(), delta->element_size()));
-#define LAUNCH_ANR_K(KERN, TD, TO)                                            \
+  TORCH_CHECK(parts == 1 || in_regs,
+              "a delta in parts wants rows that stay in registers");
+#define LAUNCH_ANR_K(KERN, TD, TO, ...)                                       \
   hipLaunchKernelGGL((KERN), dim3(T), dim3(256), 0, stream,                   \
                      (TO*)out.data_ptr(), (float*)residual.data_ptr(),        \
                      delta.has_value() ? (const TD*)delta->data_ptr()         \
                                        : nullptr,                             \
-                     drs, wp, wn, D, (float)eps, (float)mult)
+                     drs, wp, wn, D, (float)eps, (float)mult __VA_ARGS__)
 #define LAUNCH_ANR_ROW(TD, TO, NC)                                            \
-  LAUNCH_ANR_K((add_normed_rmsnorm_row_kernel<TD, TO, NC>), TD, TO)
+  do {                                                                        \
+    if (sizeof(TD) == 4 && parts > 1)                                         \
+      LAUNCH_ANR_K((add_normed_rmsnorm_row_kernel<TD, TO, NC,                 \
+                                                  sizeof(TD) == 4>),          \
+                   TD, TO, , parts, part_stride);                             \
+    else                                                                      \
+      LAUNCH_ANR_K((add_normed_rmsnorm_row_kernel<TD, TO, NC>), TD, TO, , 1,  \
+                   0);                                                        \
+  } while (0)
 #define LAUNCH_ANR(TD, TO)                                                    \
   do {                                                                        \
     if (!in_regs)                                                             \

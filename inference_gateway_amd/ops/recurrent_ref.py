@@ -372,10 +372,11 @@ def moe_group_route_ref(logits, correction, top, groups, keep):
 def add_normed_rmsnorm_ref(residual, delta, w_post, w_pre, eps, out_dtype,
                            mult=1.0):
     """residual [T, D] fp32 += mult * rmsnorm(delta) * w_post (in place; delta
-    None = nothing added); returns rmsnorm(residual) * w_pre in
-    out_dtype, or the residual itself in out_dtype when w_pre is None."""
+    None = nothing added, [S, T, D] = the sum of parts); returns
+    rmsnorm(residual) * w_pre in out_dtype, or the residual itself in out_dtype
+    when w_pre is None."""
     if delta is not None:
-        d = delta.float()
+        d = delta.float() if delta.dim() == 2 else delta.sum(0)
         residual += d * (mult * torch.rsqrt(
             (d * d).mean(-1, keepdim=True) + eps)) * w_post
     if w_pre is None:
