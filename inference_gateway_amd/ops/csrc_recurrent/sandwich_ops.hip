@@ -6,7 +6,7 @@
 //                        itself in the activation type when w_pre is absent
 //   gelu_mul_rows        gelu_tanh(z) * table[token, col0 : col0 + W]
 //
-// One 256-thread block per row; both statistics are fp32 block reductions.
+// One block per row (256 threads, of few rows 1024); both statistics are fp32 block reductions.
 //
 // add_normed_rmsnorm is bound by one pass over the row: residual read and
 // written, delta read, out written.  Rows of up to 8192 entries that allow
@@ -14,7 +14,7 @@
 // their loads issued before the first is used; longer, odd or misaligned rows
 // are read again after each statistic.  Measured, rows read again and kept
 // (us): 6000 rows of 4096 71.0 and 47.4 (6.2 TB/s), of 8192 188 and 122; 48
-// rows of 4096 9.3 and 5.9.  A delta of several parts (a product's sums over parts of
+// rows of 4096 9.3 and 5.9 (3.3 with 1024 threads).  A delta of several parts (a product's sums over parts of
 // its K) is added as it is read: a sum of its own takes another 4.5 us of 48 rows
 // (Bivatar's decode of 48 sequences, four such sums, 698 and 688).
 #include "../csrc_hybrid/act_types.h"
@@ -93,15 +93,16 @@ DEVINLINE float square4(float4 v) {
   return v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
 }
 
-// D <= 1024 NC, D % 4 == 0, rows and weights aligned to four entries.  PARTS: delta
+// D <= 4 BLOCK NC, D % 4 == 0, rows and weights aligned to four entries.  PARTS: delta
 // is the sum of `parts` of them, part_stride entries apart.
-template <typename TD, typename TO, int NC, bool PARTS = false>
-__global__ __launch_bounds__(256) void add_normed_rmsnorm_row_kernel(
+template <typename TD, typename TO, int NC, int BLOCK = 256,
+          bool PARTS = false>
+__global__ __launch_bounds__(BLOCK) void add_normed_rmsnorm_row_kernel(
     TO* __restrict__ out, float* __restrict__ residual,
     const TD* __restrict__ delta, int64_t delta_rs,
     const float* __restrict__ w_post, const float* __restrict__ w_pre, int D,
     float eps, float mult, int parts, int64_t part_stride) {
-  __shared__ float red[8];
+  __shared__ float red[BLOCK / WAVE_SIZE];
   const int t = blockIdx.x, tid = threadIdx.x;
   float* res = residual + (int64_t)t * D;
   TO* o = out + (int64_t)t * D;
@@ -109,7 +110,7 @@ __global__ __launch_bounds__(256) void add_normed_rmsnorm_row_kernel(
   float4 x[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int d = (c * 256 + tid) * 4;
+    const int d = (c * BLOCK + tid) * 4;
     x[c] = d < D ? load4(res + d) : zero;
   }
   if (delta) {
@@ -118,7 +119,7 @@ __global__ __launch_bounds__(256) void add_normed_rmsnorm_row_kernel(
     float sd = 0.0f;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      const int d = (c * 256 + tid) * 4;
+      const int d = (c * BLOCK + tid) * 4;
       y[c] = d < D ? load4(dl + d) : zero;
     }
     if constexpr (PARTS) {
@@ -127,7 +128,7 @@ __global__ __launch_bounds__(256) void add_normed_rmsnorm_row_kernel(
         dl += part_stride;
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
-          const int d = (c * 256 + tid) * 4;
+          const int d = (c * BLOCK + tid) * 4;
           const float4 v = d < D ? load4(dl + d) : zero;
           y[c].x += v.x;
           y[c].y += v.y;
@@ -138,12 +139,12 @@ __global__ __launch_bounds__(256) void add_normed_rmsnorm_row_kernel(
     }
 #pragma unroll
     for (int c = 0; c < NC; ++c) sd += square4(y[c]);
-    sd = block_reduce_sum<256>(sd, red);
+    sd = block_reduce_sum<BLOCK>(sd, red);
     const float r1 = mult / sqrtf(sd / (float)D + eps);
     __syncthreads();
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      const int d = (c * 256 + tid) * 4;
+      const int d = (c * BLOCK + tid) * 4;
       if (d >= D) break;
       const float4 w = load4(w_post + d);
       x[c].x += y[c].x * r1 * w.x;
@@ -158,12 +159,12 @@ __global__ __launch_bounds__(256) void add_normed_rmsnorm_row_kernel(
     float ss = 0.0f;
 #pragma unroll
     for (int c = 0; c < NC; ++c) ss += square4(x[c]);
-    ss = block_reduce_sum<256>(ss, red);
+    ss = block_reduce_sum<BLOCK>(ss, red);
     r2 = 1.0f / sqrtf(ss / (float)D + eps);
   }
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    const int d = (c * 256 + tid) * 4;
+    const int d = (c * BLOCK + tid) * 4;
     if (d >= D) break;
     float4 v = x[c];
     if (w_pre) {
@@ -221,30 +222,37 @@ void add_normed_rmsnorm(torch::Tensor out, torch::Tensor residual,
       (!delta.has_value() || by4(delta->data_ptr(), delta->element_size()));
   TORCH_CHECK(parts == 1 || in_regs,
               "a delta in parts wants rows that stay in registers");
-#define LAUNCH_ANR_K(KERN, TD, TO, ...)                                       \
-  hipLaunchKernelGGL((KERN), dim3(T), dim3(256), 0, stream,                   \
+#define LAUNCH_ANR_K(KERN, BLOCK, TD, TO, ...)                                \
+  hipLaunchKernelGGL((KERN), dim3(T), dim3(BLOCK), 0, stream,                 \
                      (TO*)out.data_ptr(), (float*)residual.data_ptr(),        \
                      delta.has_value() ? (const TD*)delta->data_ptr()         \
                                        : nullptr,                             \
                      drs, wp, wn, D, (float)eps, (float)mult __VA_ARGS__)
-#define LAUNCH_ANR_ROW(TD, TO, NC)                                            \
+#define LAUNCH_ANR_ROW(TD, TO, NC, BLOCK)                                     \
   do {                                                                        \
     if (sizeof(TD) == 4 && parts > 1)                                         \
-      LAUNCH_ANR_K((add_normed_rmsnorm_row_kernel<TD, TO, NC,                 \
+      LAUNCH_ANR_K((add_normed_rmsnorm_row_kernel<TD, TO, NC, BLOCK,          \
                                                   sizeof(TD) == 4>),          \
-                   TD, TO, , parts, part_stride);                             \
+                   BLOCK, TD, TO, , parts, part_stride);                      \
     else                                                                      \
-      LAUNCH_ANR_K((add_normed_rmsnorm_row_kernel<TD, TO, NC>), TD, TO, , 1,  \
-                   0);                                                        \
+      LAUNCH_ANR_K((add_normed_rmsnorm_row_kernel<TD, TO, NC, BLOCK>), BLOCK, \
+                   TD, TO, , 1, 0);                                           \
   } while (0)
+  // Few rows wait for their own loads, of which 1024 threads have a quarter each; of
+  // many, workgroups wait beside each other (us, 256 threads and 1024, 1 / 48 / 256 /
+  // 512 rows: 4096 entries 3.7 4.0 5.7 7.5 and 3.2 3.3 4.8 6.8, 8192 5.2 5.7 9.1 11.9
+  // and 3.6 4.0 7.0 10.5).
+  const bool few = T <= 512;
 #define LAUNCH_ANR(TD, TO)                                                    \
   do {                                                                        \
     if (!in_regs)                                                             \
-      LAUNCH_ANR_K((add_normed_rmsnorm_kernel<TD, TO>), TD, TO);              \
-    else if (D <= 1024) LAUNCH_ANR_ROW(TD, TO, 1);                            \
-    else if (D <= 2048) LAUNCH_ANR_ROW(TD, TO, 2);                            \
-    else if (D <= 4096) LAUNCH_ANR_ROW(TD, TO, 4);                            \
-    else LAUNCH_ANR_ROW(TD, TO, 8);                                           \
+      LAUNCH_ANR_K((add_normed_rmsnorm_kernel<TD, TO>), 256, TD, TO);         \
+    else if (D <= 1024) LAUNCH_ANR_ROW(TD, TO, 1, 256);                       \
+    else if (D <= 2048) LAUNCH_ANR_ROW(TD, TO, 2, 256);                       \
+    else if (D <= 4096 && few) LAUNCH_ANR_ROW(TD, TO, 1, 1024);               \
+    else if (D <= 4096) LAUNCH_ANR_ROW(TD, TO, 4, 256);                       \
+    else if (few) LAUNCH_ANR_ROW(TD, TO, 2, 1024);                            \
+    else LAUNCH_ANR_ROW(TD, TO, 8, 256);                                      \
   } while (0)
   if (delta.has_value())
     TORCH_CHECK(d16 || delta->scalar_type() == torch::kFloat32,
