@@ -14,9 +14,8 @@
 // gives too few workgroups, one behind the other along K with their sums added
 // through LDS in fp32.
 //
-// Measured, the library's batched product and here (us): 48 tokens, 32 heads, 128 x
-// 512 13.2 and, with the rotation, 4.1 us of its own before, 6.1; 512 x 128 7.3 and
-// 5.8.
+// Measured in a step of 48 tokens, 32 heads, W cold (us): 128 x 512 with the rotation
+// 13.2 and 4.1 as two launches, 6.1 here; 512 x 128 7.3 and 5.8.
 #include "../csrc/flash_tile.h"
 #include "act_types.h"
 

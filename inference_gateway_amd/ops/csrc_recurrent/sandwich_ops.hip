@@ -6,7 +6,8 @@
 //                        itself in the activation type when w_pre is absent
 //   gelu_mul_rows        gelu_tanh(z) * table[token, col0 : col0 + W]
 //
-// One block per row (256 threads, of few rows 1024); both statistics are fp32 block reductions.
+// One block per row (256 threads, of few rows 1024); both statistics are fp32
+// block reductions.
 //
 // add_normed_rmsnorm is bound by one pass over the row: residual read and
 // written, delta read, out written.  Rows of up to 8192 entries that allow
@@ -14,9 +15,10 @@
 // their loads issued before the first is used; longer, odd or misaligned rows
 // are read again after each statistic.  Measured, rows read again and kept
 // (us): 6000 rows of 4096 71.0 and 47.4 (6.2 TB/s), of 8192 188 and 122; 48
-// rows of 4096 9.3 and 5.9 (3.3 with 1024 threads).  A delta of several parts (a product's sums over parts of
-// its K) is added as it is read: a sum of its own takes another 4.5 us of 48 rows
-// (Bivatar's decode of 48 sequences, four such sums, 698 and 688).
+// rows of 4096 9.3 and 5.9 (with 1024 threads two thirds of that).  A delta of
+// several parts (a product's sums over parts of its K) is added as it is read: a
+// sum of its own takes another 4.5 us of 48 rows (Bivatar's decode of 48 sequences,
+// four such sums, 698 and 688).
 #include "../csrc_hybrid/act_types.h"
 
 namespace igw {
