@@ -130,11 +130,12 @@ class PostNormLayer(nn.Module):
         sublayer's output and the weight of its norm, added inside this
         sublayer's fused residual kernel.  Returns this layer's last
         un-added pair."""
-        return self.step(residual, delta, w_post, fb, cache, False)
+        return self.step(residual, delta, w_post, fb, cache, lambda: False)
 
-    def step(self, residual, delta, w_post, fb, cache, parts: bool):
-        """forward; with `parts` the delta that it returns may be parts of a
-        product for add_normed_rmsnorm to add (ops.linear_parts)."""
+    def step(self, residual, delta, w_post, fb, cache, adds_parts):
+        """forward; where adds_parts() the delta that it returns may be parts of
+        a product for add_normed_rmsnorm to add (ops.linear_parts).  It is
+        asked when the mixer, which may have hooks, has run."""
         x = ops.add_normed_rmsnorm(residual, delta, w_post, None, self.eps,
                                    self.dtype, self.mult)
         delta, w_post = self.mixer(x, fb, cache), self.norm1_w
@@ -142,7 +143,7 @@ class PostNormLayer(nn.Module):
             x = ops.add_normed_rmsnorm(residual, delta, w_post, None,
                                        self.eps, self.dtype, self.mult)
             mlp, w_post = self.mlp, self.norm2_w
-            if parts and calls_plainly(mlp, GatedMLP):
+            if calls_plainly(mlp, GatedMLP) and adds_parts():
                 delta = ops.linear_parts(
                     ops.linear_gated_act(x, mlp.gate_up, mlp.mode), mlp.down)
             else:
@@ -185,11 +186,19 @@ class BivatarForCausalLM(nn.Module):
         if cfg.embed_scale != 1.0:
             residual.mul_(cfg.embed_scale)
         delta = w_post = None
+
+        def plain(i):
+            """Whether what follows layer i - 1 adds its delta in this
+            file and nobody else sees it: a layer or the final norm."""
+            return self.tap is None and (
+                i == len(self.layers)
+                or calls_plainly(self.layers[i], PostNormLayer))
+
         for i, layer in enumerate(self.layers):
             cache = caches[layer.kv_from if layer.kv_from >= 0 else i]
-            if self.tap is None and calls_plainly(layer, PostNormLayer):
+            if plain(i):
                 delta, w_post = layer.step(residual, delta, w_post, fb, cache,
-                                           True)
+                                           lambda: plain(i + 1))
             else:
                 delta, w_post = layer(residual, delta, w_post, fb, cache)
             if self.tap is not None:

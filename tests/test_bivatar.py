@@ -701,6 +701,84 @@ def test_borrowed_latents_follow_the_source_layer(tmp_path, device):
     close(replay_all(eng2, t, [45]), ref2, 2e-4)
 
 
+class Through(torch.nn.Module):
+    """A layer put in another's place, which reads its delta itself."""
+
+    def __init__(self, m, seen):
+        super().__init__()
+        self.m, self.seen, self.kv_from = m, seen, m.kv_from
+
+    def forward(self, residual, delta, w_post, fb, cache):
+        self.seen.append(tuple(delta.shape))
+        return self.m(residual, delta, w_post, fb, cache)
+
+
+def test_layers_that_are_called_get_whole_deltas(tmp_path, monkeypatch):
+    """A delta in parts goes only to a norm that adds parts: a layer with a
+    pre-hook (there before the step, or registered while the layer before it runs)
+    and one of another class get [rows, hidden], and the logits are those of a
+    model without parts."""
+    cfg = cfg_small()
+    eng = make_engine(tmp_path, cfg, oracle.random_weights(cfg, 61), "cpu")
+    t = toks(9, cfg["vocab"], 62)
+    layers, asked = eng.model.layers, []
+
+    def parts(x, w):
+        y = ops.linear(x, w)
+        asked.append(y.shape[0])
+        return torch.stack([y, torch.zeros_like(y)])
+
+    def both():
+        """Logits without and with parts."""
+        whole = replay_all(eng, t, [6, 3])
+        asked.clear()
+        with monkeypatch.context() as m:
+            m.setattr(ops, "linear_parts", parts)
+            return whole, replay_all(eng, t, [6, 3])
+
+    want, got = both()
+    assert torch.equal(got, want)
+    # every layer with a feed-forward, both portions
+    assert len(asked) == 2 * sum(l.mlp is not None for l in layers)
+
+    seen = []
+
+    def add(m, args):
+        seen.append(tuple(args[1].shape))
+        return (args[0], args[1] + 0.5, *args[2:])
+
+    shapes = 2 * [(6, cfg["width"]), (3, cfg["width"])]
+    for i in range(1, len(layers)):
+        seen.clear()
+        handle = layers[i].register_forward_pre_hook(add)
+        a, b = both()
+        handle.remove()
+        assert seen == shapes
+        assert torch.equal(a, b) and not torch.equal(a, want)
+
+        seen.clear()
+        handles = []
+        outer = layers[i - 1].mixer.register_forward_hook(
+            lambda *a, i=i: handles.append(
+                layers[i].register_forward_pre_hook(add)))
+        with monkeypatch.context() as m:
+            m.setattr(ops, "linear_parts", parts)
+            replay_all(eng, t, [9])
+        outer.remove()
+        for h in handles:
+            h.remove()
+        assert seen == [(9, cfg["width"])]
+
+        seen.clear()
+        kept = layers[i]
+        layers[i] = Through(kept, seen)
+        a, b = both()
+        layers[i] = kept
+        assert seen == shapes
+        assert torch.equal(a, want) and torch.equal(b, want)
+    assert torch.equal(both()[1], want)
+
+
 @pytest.mark.parametrize("device", DEVICES)
 def test_bfloat16_mode(tmp_path, device):
     cfg = cfg_small()
