@@ -23,12 +23,13 @@
 
 namespace igw {
 
-template <typename TD, typename TO>
+// PARTS: delta is the sum of `parts` of them, part_stride entries apart.
+template <typename TD, typename TO, bool PARTS = false>
 __global__ __launch_bounds__(256) void add_normed_rmsnorm_kernel(
     TO* __restrict__ out, float* __restrict__ residual,
     const TD* __restrict__ delta, int64_t delta_rs,
     const float* __restrict__ w_post, const float* __restrict__ w_pre, int D,
-    float eps, float mult) {
+    float eps, float mult, int parts, int64_t part_stride) {
   __shared__ float red[8];
   const int t = blockIdx.x, tid = threadIdx.x;
   float* res = residual + (int64_t)t * D;
@@ -36,16 +37,22 @@ __global__ __launch_bounds__(256) void add_normed_rmsnorm_kernel(
   float ss = 0.0f;
   if (delta) {
     const TD* dl = delta + (int64_t)t * delta_rs;
+    auto entry = [&](int d) {
+      float x = Act<TD>::ld(dl + d);
+      if constexpr (PARTS)
+        for (int p = 1; p < parts; ++p) x += Act<TD>::ld(dl + p * part_stride + d);
+      return x;
+    };
     float sd = 0.0f;
     for (int d = tid; d < D; d += 256) {
-      const float x = Act<TD>::ld(dl + d);
+      const float x = entry(d);
       sd += x * x;
     }
     sd = block_reduce_sum<256>(sd, red);
     const float r1 = mult / sqrtf(sd / (float)D + eps);
     __syncthreads();
     for (int d = tid; d < D; d += 256) {
-      const float x = res[d] + Act<TD>::ld(dl + d) * r1 * w_post[d];
+      const float x = res[d] + entry(d) * r1 * w_post[d];
       res[d] = x;
       ss += x * x;
     }
@@ -95,8 +102,8 @@ DEVINLINE float square4(float4 v) {
   return v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
 }
 
-// D <= 4 BLOCK NC, D % 4 == 0, rows and weights aligned to four entries.  PARTS: delta
-// is the sum of `parts` of them, part_stride entries apart.
+// D <= 4 BLOCK NC, D % 4 == 0, rows and weights aligned to four entries.  PARTS as
+// above.
 template <typename TD, typename TO, int NC, int BLOCK = 256,
           bool PARTS = false>
 __global__ __launch_bounds__(BLOCK) void add_normed_rmsnorm_row_kernel(
@@ -222,23 +229,31 @@ void add_normed_rmsnorm(torch::Tensor out, torch::Tensor residual,
       by4(residual.data_ptr(), 4) &&
       by4(out.data_ptr(), out.element_size()) &&
       (!delta.has_value() || by4(delta->data_ptr(), delta->element_size()));
-  TORCH_CHECK(parts == 1 || in_regs,
-              "a delta in parts wants rows that stay in registers");
-#define LAUNCH_ANR_K(KERN, BLOCK, TD, TO, ...)                                \
+#define LAUNCH_ANR_K(KERN, BLOCK, TD, TO)                                     \
   hipLaunchKernelGGL((KERN), dim3(T), dim3(BLOCK), 0, stream,                 \
                      (TO*)out.data_ptr(), (float*)residual.data_ptr(),        \
                      delta.has_value() ? (const TD*)delta->data_ptr()         \
                                        : nullptr,                             \
-                     drs, wp, wn, D, (float)eps, (float)mult __VA_ARGS__)
+                     drs, wp, wn, D, (float)eps, (float)mult, parts,          \
+                     part_stride)
+// parts come in fp32
+#define LAUNCH_ANR_ALL(TD, TO)                                                \
+  do {                                                                        \
+    if (sizeof(TD) == 4 && parts > 1)                                         \
+      LAUNCH_ANR_K((add_normed_rmsnorm_kernel<TD, TO, sizeof(TD) == 4>), 256, \
+                   TD, TO);                                                   \
+    else                                                                      \
+      LAUNCH_ANR_K((add_normed_rmsnorm_kernel<TD, TO>), 256, TD, TO);         \
+  } while (0)
 #define LAUNCH_ANR_ROW(TD, TO, NC, BLOCK)                                     \
   do {                                                                        \
     if (sizeof(TD) == 4 && parts > 1)                                         \
       LAUNCH_ANR_K((add_normed_rmsnorm_row_kernel<TD, TO, NC, BLOCK,          \
                                                   sizeof(TD) == 4>),          \
-                   BLOCK, TD, TO, , parts, part_stride);                      \
+                   BLOCK, TD, TO);                                            \
     else                                                                      \
       LAUNCH_ANR_K((add_normed_rmsnorm_row_kernel<TD, TO, NC, BLOCK>), BLOCK, \
-                   TD, TO, , 1, 0);                                           \
+                   TD, TO);                                                   \
   } while (0)
   // Few rows wait for their own loads, of which 1024 threads have a quarter each; of
   // many, workgroups wait beside each other (us, 256 threads and 1024, 1 / 48 / 256 /
@@ -247,8 +262,7 @@ void add_normed_rmsnorm(torch::Tensor out, torch::Tensor residual,
   const bool few = T <= 512;
 #define LAUNCH_ANR(TD, TO)                                                    \
   do {                                                                        \
-    if (!in_regs)                                                             \
-      LAUNCH_ANR_K((add_normed_rmsnorm_kernel<TD, TO>), 256, TD, TO);         \
+    if (!in_regs) LAUNCH_ANR_ALL(TD, TO);                                     \
     else if (D <= 1024) LAUNCH_ANR_ROW(TD, TO, 1, 256);                       \
     else if (D <= 2048) LAUNCH_ANR_ROW(TD, TO, 2, 256);                       \
     else if (D <= 4096 && few) LAUNCH_ANR_ROW(TD, TO, 1, 1024);               \
@@ -265,6 +279,7 @@ void add_normed_rmsnorm(torch::Tensor out, torch::Tensor residual,
   });
 #undef LAUNCH_ANR
 #undef LAUNCH_ANR_ROW
+#undef LAUNCH_ANR_ALL
 #undef LAUNCH_ANR_K
   HIP_CHECK_KERNEL();
 }
