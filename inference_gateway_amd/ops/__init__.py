@@ -686,13 +686,15 @@ def turned_head_products(q, w, positions, inv_freq, half: bool = False,
     bf16."""
     K = w.shape[1]
     x = q[:, :, :K]
-    if q.is_cuda and q.shape[2] == K + 2 * inv_freq.numel():
-        out = q.new_empty((q.shape[0], q.shape[1], w.shape[2]))
-        if _shared_ext("head_products")(out, x, w, q[:, :, K:], positions,
+    if not q.is_cuda or q.shape[2] != K + 2 * inv_freq.numel():
+        rope_pairs_(q, positions, inv_freq, K, half, mag)
+        return head_products(x, w)
+    out = q.new_empty((q.shape[0], q.shape[1], w.shape[2]))
+    if not _shared_ext("head_products")(out, x, w, q[:, :, K:], positions,
                                         inv_freq, half, mag):
-            return out
-    rope_pairs_(q, positions, inv_freq, K, half, mag)
-    return head_products(x, w)
+        rope_pairs_(q, positions, inv_freq, K, half, mag)
+        torch.bmm(x.transpose(0, 1), w, out=out.transpose(0, 1))
+    return out
 
 
 def latent_prompt_fits(q, rot_dim: int, vdim: int, kv_rank: int = 0) -> bool:
