@@ -666,16 +666,25 @@ def latent_attention(q_abs, q_rot, cache, block_table, row_seq, positions,
         window, gate)
 
 
+def _own_head_products(out, x, w, *turned):
+    """head_products by the kernel, or None where it does not take the call."""
+    if (not x.is_cuda or torch.compiler.is_compiling()
+            or has_torch_function_variadic(x, w)):
+        return None
+    return _shared_ext("head_products")(out, x, w, *turned)
+
+
 def head_products(x, w, out=None):
     """x [T, H, K] times a matrix per head, w [H, K, N]: [T, H, N] (`out` when
     given; strided views ok).  A few rows of bf16 run one kernel
     (ops/csrc_hybrid/head_products.hip), everything else the library's batched
     product."""
+    got = _own_head_products(out, x, w, None, None, None, False, 1.0)
+    if got is not None:
+        return got
     if out is None:
-        out = x.new_empty((x.shape[0], x.shape[1], w.shape[2]))
-    if not (x.is_cuda and _shared_ext("head_products")(
-            out, x, w, None, None, None, False, 1.0)):
-        torch.bmm(x.transpose(0, 1), w, out=out.transpose(0, 1))
+        return torch.bmm(x.transpose(0, 1), w).transpose(0, 1)
+    torch.bmm(x.transpose(0, 1), w, out=out.transpose(0, 1))
     return out
 
 
@@ -686,15 +695,15 @@ def turned_head_products(q, w, positions, inv_freq, half: bool = False,
     bf16."""
     K = w.shape[1]
     x = q[:, :, :K]
-    if not q.is_cuda or q.shape[2] != K + 2 * inv_freq.numel():
+    if q.shape[2] != K + 2 * inv_freq.numel():
         rope_pairs_(q, positions, inv_freq, K, half, mag)
         return head_products(x, w)
-    out = q.new_empty((q.shape[0], q.shape[1], w.shape[2]))
-    if not _shared_ext("head_products")(out, x, w, q[:, :, K:], positions,
-                                        inv_freq, half, mag):
+    got = _own_head_products(None, x, w, q[:, :, K:], positions, inv_freq, half,
+                             mag)
+    if got is None:
         rope_pairs_(q, positions, inv_freq, K, half, mag)
-        torch.bmm(x.transpose(0, 1), w, out=out.transpose(0, 1))
-    return out
+        got = torch.bmm(x.transpose(0, 1), w).transpose(0, 1)
+    return got
 
 
 def latent_prompt_fits(q, rot_dim: int, vdim: int, kv_rank: int = 0) -> bool:

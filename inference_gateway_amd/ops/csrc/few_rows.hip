@@ -9,11 +9,11 @@
 // see.  Everything else (weights elsewhere, autograd in either mode, vmap, a
 // trace, a dispatch mode, autocast, other types and layouts) is the library's
 // product, with its results and its errors.
-#include <ATen/autocast_mode.h>
 #include <ATen/cuda/CUDAContext.h>
-#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/cuda/CUDAGuard.h>
 #include <torch/extension.h>
+
+#include "plain_call.h"
 
 namespace igw {
 
@@ -59,27 +59,6 @@ void gemv(torch::Tensor out, torch::Tensor x, torch::Tensor w,
           c10::optional<torch::Tensor> bias, int64_t gate);
 void rows_gemm(torch::Tensor out, torch::Tensor x, torch::Tensor w,
                c10::optional<torch::Tensor> bias, int64_t gate);
-
-static bool call_is_plain() {
-  using K = c10::DispatchKey;
-  const auto seen = c10::impl::tls_local_dispatch_key_set().included_;
-  return !seen.has_any(c10::DispatchKeySet(
-             {K::Python, K::PythonTLSSnapshot, K::FuncTorchVmapMode,
-              K::FuncTorchDynamicLayerFrontMode, K::FuncTorchBatched,
-              K::Functionalize, K::Tracer})) &&
-         !at::autocast::is_autocast_enabled(at::kCUDA);
-}
-
-static bool plain_bf16(const torch::Tensor& t, c10::Device where) {
-  using K = c10::DispatchKey;
-  return t.defined() && t.scalar_type() == torch::kBFloat16 &&
-         t.layout() == torch::kStrided && t.device() == where &&
-         !t.key_set().has_any(c10::DispatchKeySet(
-             {K::Python, K::FuncTorchBatched, K::FuncTorchGradWrapper,
-              K::Functionalize, K::ZeroTensor, K::NestedTensor})) &&
-         !(at::GradMode::is_enabled() && t.requires_grad()) &&
-         !t._fw_grad(0).defined();
-}
 
 static bool by16(const torch::Tensor& t) {
   return (reinterpret_cast<uintptr_t>(t.data_ptr()) & 15) == 0;

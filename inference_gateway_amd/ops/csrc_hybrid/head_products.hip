@@ -17,6 +17,7 @@
 // Measured in a step of 48 tokens, 32 heads, W cold (us): 128 x 512 with the rotation
 // 13.2 and 4.1 as two launches, 6.1 here; 512 x 128 7.3 and 5.8.
 #include "../csrc/flash_tile.h"
+#include "../csrc/plain_call.h"
 #include "act_types.h"
 
 namespace igw {
@@ -157,23 +158,24 @@ __global__ __launch_bounds__(64 * FT_WAVES, 1) void head_products_kernel(
   }
 }
 
-// out [T, H, N] = x [T, H, K] W [H, K, N] per head; with `turn` [T, H, 2 pairs] (the
-// same strides as x) its rotation in place, as rope_pairs does it.  False, and
-// nothing done, when the sizes do not fit: the caller then runs the library's
-// batched product.
-bool head_products(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-                   c10::optional<torch::Tensor> turn,
-                   c10::optional<torch::Tensor> positions,
-                   c10::optional<torch::Tensor> inv_freq, bool half,
-                   double mag) {
-  if (!x.is_cuda() || x.scalar_type() != torch::kBFloat16 ||
-      w.scalar_type() != torch::kBFloat16 ||
-      out.scalar_type() != torch::kBFloat16 || x.dim() != 3 || w.dim() != 3 ||
-      out.dim() != 3 || x.device() != w.device() || x.device() != out.device())
-    return false;
+// x [T, H, K] times W [H, K, N] per head, in `out` [T, H, N] where it is given; with
+// `turn` [T, H, 2 pairs] (the same strides as x) its rotation in place, as
+// rope_pairs does it.  Nothing, and nothing done, when the call does not fit: the
+// caller then runs the library's batched product.
+c10::optional<torch::Tensor> head_products(
+    c10::optional<torch::Tensor> given, torch::Tensor x, torch::Tensor w,
+    c10::optional<torch::Tensor> turn, c10::optional<torch::Tensor> positions,
+    c10::optional<torch::Tensor> inv_freq, bool half, double mag) {
+  if (!x.is_cuda() || !call_is_plain() || !plain_bf16(x, x.device()) ||
+      !plain_bf16(w, x.device()) || x.dim() != 3 || w.dim() != 3 ||
+      (given.has_value() &&
+       (!plain_bf16(*given, x.device()) || given->dim() != 3)))
+    return c10::nullopt;
   const int64_t T = x.size(0), H = x.size(1), K = x.size(2), N = w.size(2);
-  TORCH_CHECK(w.size(0) == H && w.size(1) == K && out.size(0) == T &&
-                  out.size(1) == H && out.size(2) == N,
+  TORCH_CHECK(w.size(0) == H && w.size(1) == K &&
+                  (!given.has_value() ||
+                   (given->size(0) == T && given->size(1) == H &&
+                    given->size(2) == N)),
               "head_products: sizes");
   auto on = [](const torch::Tensor& t, int64_t bytes) {
     return reinterpret_cast<uintptr_t>(t.data_ptr()) % bytes == 0 &&
@@ -182,8 +184,8 @@ bool head_products(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   };
   if (T < 1 || T > HP_ROWS || H < 1 || K < 64 || K > 1024 || N < 128 ||
       N > 4096 || N % 128 || K % 64 || !w.is_contiguous() || !on(x, 16) ||
-      !on(w, 16) || !on(out, 8))
-    return false;
+      !on(w, 16) || (given.has_value() && !on(*given, 8)))
+    return c10::nullopt;
   // By columns where a wave can have all of K at once; longer ones are cut over the
   // waves.  Up to where the library is ahead (us, it and this: 128 x 512, 32 heads,
   // 1 / 32 / 48 / 64 / 96 tokens 4.4 4.2 5.1 4.9 5.5 and 3.0 4.0 4.9 5.6 7.6, whose
@@ -192,9 +194,11 @@ bool head_products(torch::Tensor out, torch::Tensor x, torch::Tensor w,
   // 64 / 96 9.6 10.8 and 9.0 14.5).
   const bool by_k = K > 128;
   if (by_k ? T * H > 8192 : T * N > (turn.has_value() ? 96 : 48) * 512)
-    return false;
+    return c10::nullopt;
   const int64_t kper = by_k ? K / FT_WAVES : K;
-  if (kper * (by_k ? FT_WAVES : 1) != K || kper % 64) return false;
+  if (kper * (by_k ? FT_WAVES : 1) != K || kper % 64) return c10::nullopt;
+  const torch::Tensor out =
+      given.has_value() ? *given : torch::empty({T, H, N}, x.options());
   HeadProducts a{(uint16_t*)out.data_ptr(), out.stride(0), out.stride(1),
                  (const uint16_t*)x.data_ptr(), x.stride(0), x.stride(1),
                  (const uint16_t*)w.data_ptr(), (int)T, (int)H, (int)K, (int)N,
@@ -236,7 +240,7 @@ bool head_products(torch::Tensor out, torch::Tensor x, torch::Tensor w,
 #undef LAUNCH_HP_NT
 #undef LAUNCH_HP
   HIP_CHECK_KERNEL();
-  return true;
+  return out;
 }
 
 }  // namespace igw

@@ -36,11 +36,10 @@ bool latent_attention_mfma(torch::Tensor out, torch::Tensor q_abs,
                            int64_t window, int64_t max_keys,
                            c10::optional<torch::Tensor> gate);
 int64_t latent_attention_tile_rows(int64_t H);
-bool head_products(torch::Tensor out, torch::Tensor x, torch::Tensor w,
-                   c10::optional<torch::Tensor> turn,
-                   c10::optional<torch::Tensor> positions,
-                   c10::optional<torch::Tensor> inv_freq, bool half,
-                   double mag);
+c10::optional<torch::Tensor> head_products(
+    c10::optional<torch::Tensor> given, torch::Tensor x, torch::Tensor w,
+    c10::optional<torch::Tensor> turn, c10::optional<torch::Tensor> positions,
+    c10::optional<torch::Tensor> inv_freq, bool half, double mag);
 bool latent_prompt_fits(int64_t dn, int64_t rd, int64_t vd);
 void latent_prompt(torch::Tensor out, torch::Tensor q, torch::Tensor kn,
                    torch::Tensor kr, torch::Tensor v, torch::Tensor cu,
@@ -102,7 +101,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "token rows per MFMA tile for a head count");
   m.def("head_products", &igw::head_products,
         "a few rows times a matrix per head, and the rotation beside it; "
-        "false = sizes do not fit");
+        "None: the call does not fit");
   m.def("softcap_attention", &igw::softcap_attention,
         "causal paged softmax attention with a tanh score cap");
   m.def("softcap_attention_mfma", &igw::softcap_attention_mfma,
