@@ -158,6 +158,40 @@ __global__ __launch_bounds__(64 * FT_WAVES, 1) void head_products_kernel(
   }
 }
 
+// Whether the kernel is ahead of the library's batched product (and, of `pairs`
+// turned pairs, of that and rope_pairs).  It sends a wave's loads once, tokens with
+// them: its time grows with the tokens a wave has, and with the rounds of workgroups,
+// where the library's hardly does (us, it and this):
+//  * by columns, 1 / 32 / 48 / 64 / 96 tokens of 32 heads: 64 x 128 4.9 4.2 4.7 4.5
+//    4.9 and 2.4 2.9 3.8 4.0 5.2, 128 x 128 5.6 4.7 5.3 5.1 5.6 and 2.7 3.7 4.7 5.1
+//    7.0, 128 x 256 5.3 5.7 6.7 6.4 8.2 and 3.2 4.0 5.0 5.5 7.5, 64 x 512 6.9 4.5 4.9
+//    and 3.0 3.5 4.1, 128 x 512 of four heads 3.8 3.9 4.0 and 2.6 3.7 4.6, of 128
+//    heads, 16 / 32 tokens 7.4 7.9 and 6.8 8.3;
+//  * with 32 pairs a head turned, 32 heads, 48 / 64 / 96 / 128 tokens: 128 x 128 8.0
+//    7.8 8.3 8.8 and 4.8 5.2 7.0 8.1, 128 x 512 8.3 8.3 8.8 and 5.3 5.8 7.7, of four
+//    heads 6.1 6.6 6.4 and 4.7 5.1 6.9, 128 x 256 of 128 heads 12.4 12.3 14.2 14.2 and
+//    7.6 8.9 13.1 17.4.  One workgroup turns a head, which takes 8 us of 4096 pairs;
+//  * cut by K, 1 / 32 / 64 / 128 tokens: 512 x 128, 32 heads 9.9 8.8 9.1 10.7 and 3.6
+//    4.2 5.4 8.2, 128 heads 12.7 12.1 12.5 and 6.2 7.6 10.3, 768 x 128, 128 heads 12.4
+//    11.5 12.1 and 7.2 9.4 13.5, 1024 x 128, 16 heads 6.3 6.5 6.7 8.6 and 4.6 5.8 8.0
+//    12.5, 512 x 256, 128 heads, 1 / 32 / 48 tokens 13.7 13.7 14.7 and 8.8 11.7 14.8.
+//    Of wider ones the library is ahead early (512 x 512, 64 heads, 16 tokens 10.5 and
+//    10.7, 1024 x 1024, 16 heads, one token 10.3 and 11.4);
+//  * of more than 128 heads the library is ahead early (128 x 256, 160 heads, 32 / 64
+//    tokens 7.5 7.5 and 6.9 9.4).
+static bool hp_ahead(int64_t T, int64_t H, int64_t K, int64_t N,
+                     int64_t pairs) {
+  if (T * pairs > 3072 || H > 128) return false;
+  if (K > 128)
+    return N <= 256 && K * N <= 131072 && (K <= 768 || T <= 32) &&
+           T * H * N * std::max<int64_t>(K, 512) <= (int64_t)1 << 29;
+  if (pairs > 0) return T * N <= 49152 && T <= (N > 256 ? 64 : 96);
+  if (N > 256)
+    return T * N <= 24576 &&
+           T <= (K <= 64 ? 48 : H * N < 65536 ? 32 : 16);
+  return T <= 96 && (N > 128 || (T <= 64 && T * K <= 6144));
+}
+
 // x [T, H, K] times W [H, K, N] per head, in `out` [T, H, N] where it is given; with
 // `turn` [T, H, 2 pairs] (the same strides as x) its rotation in place, as
 // rope_pairs does it.  Nothing, and nothing done, when the call does not fit: the
@@ -187,13 +221,9 @@ c10::optional<torch::Tensor> head_products(
       !on(w, 16) || (given.has_value() && !on(*given, 8)))
     return c10::nullopt;
   // By columns where a wave can have all of K at once; longer ones are cut over the
-  // waves.  Up to where the library is ahead (us, it and this: 128 x 512, 32 heads,
-  // 1 / 32 / 48 / 64 / 96 tokens 4.4 4.2 5.1 4.9 5.5 and 3.0 4.0 4.9 5.6 7.6, whose
-  // rotation takes another 3 to 4; 64 x 256, 16 heads, 96 tokens 7.0 and 5.3;
-  // 512 x 128, 32 heads, 1 / 48 / 128 tokens 9.8 9.0 10.6 and 3.6 5.0 7.8, 128 heads,
-  // 64 / 96 9.6 10.8 and 9.0 14.5).
+  // waves.
   const bool by_k = K > 128;
-  if (by_k ? T * H > 8192 : T * N > (turn.has_value() ? 96 : 48) * 512)
+  if (!hp_ahead(T, H, K, N, turn.has_value() ? turn->size(2) / 2 : 0))
     return c10::nullopt;
   const int64_t kper = by_k ? K / FT_WAVES : K;
   if (kper * (by_k ? FT_WAVES : 1) != K || kper % 64) return c10::nullopt;
