@@ -1267,7 +1267,9 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
 // whose passes follow its loads, 54, 123, 185, 99, 103 and 140.  64 rows mixed 39.9 for
 // 42.5.  A flat top-p row takes twice as long as another: of more rows than are on
 // the chip at once (two a compute unit) those start first, which costs a
-// microsecond a row (1024 mixed rows in the order of the call 92 us, so 77).  Up to 65536 logits the register kernel has
+// microsecond a row (1024 mixed rows in the order of the call 92 us, so 77); so do
+// rows of a top-k that no list serves (a tenth of k = 500 among others of top-k 50 and
+// top-p, 600 / 1024 / 2000 rows 69.9 90.6 154, so 51.4 76.5 134).  Up to 65536 logits the register kernel has
 // two rows on a unit and is ahead (1024 of 49000, mixed, 49.3, here 50.7; of 32000 36.3
 // and 43).
 // ---------------------------------------------------------------------------
@@ -1303,8 +1305,8 @@ DEVINLINE uint32_t ss_bins(uint32_t keys, uint32_t top, uint32_t spare) {
       __builtin_elementwise_min(b, __builtin_bit_cast(ushort2v, spare)));
 }
 
-// Row of a workgroup when those that can take another pass (top-p without a top-k
-// that its list serves) start first.  Every wave finds it for itself from
+// Row of a workgroup when those that can take another pass (a top-k that no list
+// serves, top-p without a top-k) start first.  Every wave finds it for itself from
 // the rows' settings, 64 rows in a word of `words`, which is free again behind the
 // next barrier.
 template <int WAVES>
@@ -1316,8 +1318,9 @@ DEVINLINE int ss_long_first(uint64_t* words, int wave, int V,
   for (int g = wave; g < groups; g += WAVES) {
     const int r = min(g * 64 + lane, B - 1);
     const int k = top_k[r];
-    const bool later = temperature[r] <= 0.0f || !(top_p[r] < 1.0f) ||
-                       (k > 0 && k < V && k <= 32 * WAVES);
+    const bool later =
+        temperature[r] <= 0.0f ||
+        (k > 0 && k < V ? k <= 32 * WAVES : !(top_p[r] < 1.0f));
     const uint64_t word = __ballot(!later && g * 64 + lane < B);
     if (lane == 0) words[g] = word;
   }
@@ -1364,7 +1367,8 @@ __global__ __launch_bounds__(SS_THREADS, 4) void sample_bf16_stream_kernel(
   int* const sorted_e = kept_e + SS_THREADS;
   float* const kept_w = reinterpret_cast<float*>(sorted_e + SS_THREADS);
   float* const sorted_w = kept_w + SS_THREADS;
-  __shared__ float cells[SS_UNITS], cell_c[SS_UNITS];
+  // cells: before them the words of ss_long_first
+  __shared__ __attribute__((aligned(16))) float cells[SS_UNITS], cell_c[SS_UNITS];
   __shared__ float red[SS_WAVES];
   __shared__ uint32_t bound[SS_WAVES], bound0[SS_WAVES];
   __shared__ uint32_t wave_n[SS_WAVES];
