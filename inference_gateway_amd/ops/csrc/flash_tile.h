@@ -300,7 +300,7 @@ DEVINLINE void flash_tiles(Rows& rows, const FlashSpan& span,
   // Addresses of whole tiles cost the vector units nothing: they are a scalar
   // base and these offsets (64-bit sums per lane were a third of the vector
   // instructions of a tile).
-  constexpr bool STRAIGHT = Rows::STRAIGHT && NK <= 256;
+  constexpr bool STRAIGHT = Rows::STRAIGHT;
   int ko[CK / 4], vo[CV / 4];
   if constexpr (STRAIGHT) {
 #pragma unroll
