@@ -1271,7 +1271,16 @@ __launch_bounds__(SR_THREADS, NCH > 8 ? 2 : 4) void sample_bf16_resident_kernel(
 // rows of a top-k that no list serves (a tenth of k = 500 among others of top-k 50 and
 // top-p, 600 / 1024 / 2000 rows 69.9 90.6 154, so 51.4 76.5 134).  Up to 65536 logits the register kernel has
 // two rows on a unit and is ahead (1024 of 49000, mixed, 49.3, here 50.7; of 32000 36.3
-// and 43).
+// and 43).  Just beyond, held in registers and here, 256 rows of 65544: top-k 50 and
+// top-p 26.9 and 18.9, top-k 40 22.1 and 16.8, no limits 20.5 and 14.0, greedy 10.9 and
+// 10.1, mixed 31.0 and 31.1, but rows that are read again are behind there, top-p 0.9
+// 31.7 and 33.8, k = 500 27.5 and 29.8 (64 rows 29.9 29.8 and 25.7 27.6; 300 rows 57.4
+// 41.0 and 48.3 35.5; 256 rows of 128256 53.3 47.8 and 41.4 36.8, one of k = 500 27.0 and
+// 29.8).  That second read is not it: plain loads in the first pass of such rows, for
+// the caches to keep them, change nothing at any of these sizes.
+//
+// Thresholds, ordered draw and `element` repeat the resident kernel's on another
+// list: what is mended in one is looked for in the other.
 // ---------------------------------------------------------------------------
 constexpr int SS_U = 4;                  // chunks of eight a lane in a unit
 constexpr int SS_UNIT = SS_U * 512;      // logits

@@ -12,11 +12,13 @@
 //   v -> vcache [blocks, G, block, P] at slot (copied); TIED: v is the key
 //   as projected, before norm and rotation, and proj has no value block
 //
-// One 256-thread workgroup per row; its four waves take the row's units in
-// turn: the H query heads, then the G key heads, then the G value heads.
-// Lanes own entry pairs (one 4- or 8-byte access per pair when the layout
-// allows); norms, angles and the rotation are fp32 (cosf / sinf with full
-// range reduction, evaluated once per row and shared through LDS).
+// Norms, angles and the rotation are fp32 (cosf / sinf with full range reduction,
+// evaluated once per workgroup and shared through LDS).  bf16 heads of 64, 128 or 256
+// entries that lie on 16 bytes run qk_norm_rope_append_chunks_kernel, everything else
+// qk_norm_rope_append_kernel: one 256-thread workgroup per row, whose four waves take
+// the row's units in turn (the H query heads, then the G key heads, then the G value
+// heads), lanes own entry pairs (one 4- or 8-byte access per pair when the layout
+// allows).
 #include "../csrc_hybrid/act_types.h"
 
 namespace igw {

@@ -14,11 +14,10 @@
 // loads of four entries stay in registers between the two statistics, all
 // their loads issued before the first is used; longer, odd or misaligned rows
 // are read again after each statistic.  Measured, rows read again and kept
-// (us): 6000 rows of 4096 71.0 and 47.4 (6.2 TB/s), of 8192 188 and 122; 48
-// rows of 4096 9.3 and 5.9 (with 1024 threads two thirds of that).  A delta of
-// several parts (a product's sums over parts of its K) is added as it is read: a
-// sum of its own takes another 4.5 us of 48 rows (Bivatar's decode of 48 sequences,
-// four such sums, 698 and 688).
+// (us): 6000 rows of 4096 71.0 and 47.4 (6.2 TB/s), of 8192 188 and 122; few rows are
+// at the launch.  A delta of several parts (a product's sums over parts of its K) is
+// added as it is read: a sum of its own takes another 4.5 us of 48 rows (Bivatar's
+// decode of 48 sequences, four such sums, 698 and 688).
 #include "../csrc_hybrid/act_types.h"
 
 namespace igw {
@@ -256,9 +255,12 @@ void add_normed_rmsnorm(torch::Tensor out, torch::Tensor residual,
                    TD, TO);                                                   \
   } while (0)
   // Few rows wait for their own loads, of which 1024 threads have a quarter each; of
-  // many, workgroups wait beside each other (us, 256 threads and 1024, 1 / 48 / 256 /
-  // 512 rows: 4096 entries 3.7 4.0 5.7 7.5 and 3.2 3.3 4.8 6.8, 8192 5.2 5.7 9.1 11.9
-  // and 3.6 4.0 7.0 10.5).
+  // many, workgroups wait beside each other (us, bf16 deltas, rows in the caches, 256
+  // threads and 1024, 1 / 48 / 256 / 512 rows: 2052 entries, where half the threads
+  // have none, 3.3 3.8 4.1 5.3 and 2.7 3.3 3.7 4.9, 3072 3.5 3.7 4.6 6.3 and 2.8 3.1
+  // 3.9 5.7, 4096 3.7 4.0 5.7 7.5 and 2.9 3.3 4.8 6.8, 8192 5.2 5.7 9.1 11.9 and 3.6
+  // 4.0 7.0 10.4; with a norm behind it 512 rows of 2052 / 4096 / 8192 6.3 8.7 13.7
+  // and 6.5 8.4 11.7).
   const bool few = T <= 512;
 #define LAUNCH_ANR(TD, TO)                                                    \
   do {                                                                        \

@@ -16,7 +16,8 @@
 //
 // Values of at most 128 entries run the tile walk of flash_tile.h
 // (softcap_prompt_kernel: 128 rows of one head; softcap_decode_kernel: the
-// heads that share a key/value head).  Wider ones, whose accumulators do not
+// heads that share a key/value head), decoded rows of 128 entries in pages of 16
+// softcap_pages_kernel.  Wider ones, whose accumulators do not
 // fit two waves per SIMD there, run softcap_attention_mfma_kernel: 64 rows x
 // 64 keys, 4 waves of 16 rows, mfma_f32_16x16x32_bf16, K staged row-major and
 // V transposed in swizzled LDS, probabilities through a per-wave LDS tile.  Its
@@ -28,9 +29,10 @@
 // Measured (32 heads on 8, N = P = 128), 64-row tiles for all and the tile
 // walk: prompts of 3000 and 2790 tokens, window 1024 with 16 kept tokens,
 // distance bias and head gate 563 and 156 us; 4 prompts of 2048, causal, with
-// a sink 1293 and 197 us, with a score cap 1412 and 227 us; decoded, 256
-// tokens of 2048 keys 863 and 388 us (5.5 TB/s), 48 of 700 to 3500 with that
-// window 103 and 51, one of 3000 181 and 17 (split over workgroups).
+// a sink 1293 and 197 us, with a score cap 1412 and 227 us; decoded, on pages of a
+// size that softcap_pages_kernel does not take, 256 tokens of 2048 keys 863 and 388 us
+// (5.5 TB/s), 48 of 700 to 3500 with that window 103 and 51, one of 3000 181 and 17
+// (split over workgroups).
 //
 // Everything is read from the paged cache; a row's own key is already
 // appended.  Sequence s has rows [seq_cu[s], seq_cu[s+1]) whose first sits
@@ -515,7 +517,8 @@ __global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_decode_kernel(
 // Decoded rows of keys and values of 128 entries in pages of 16 tokens, up to eight
 // heads on a key head: every wave walks pages of its own, two at a time, K to
 // registers in whole lines (LineTurn), V by DMA to LDS, both one step ahead, as in
-// the engine's own decode attention: nothing waits for another wave until the
+// the engine's own decode attention (csrc/paged_attn_decode.hip, whose walk this
+// repeats: what is mended in one is looked for in the other): nothing waits for another wave until the
 // end, and 128 KB are under way on a compute unit where the tiles above have 64.
 // S^T = K Q^T with the heads in the columns of mfma 16x16x32; the order of its
 // rows is the one that V is read in (ds_read_b64_tr_b16), so weights stay in their
