@@ -515,14 +515,23 @@ bool latent_decode(torch::Tensor out, torch::Tensor q_abs,
   // 19.3 us; 16 of 2000 27.0 and 29.6).  Up to 128 tokens share the slots by their
   // contexts' lengths, which is found on the device (32 heads, rank 512, in equal
   // numbers of parts and so: 48 of 700 to 3500 49.2 and 42.4, of 2000 each 40.4 and
-  // 40.8).
-  const bool shared = T > 1 && T <= 64 * LD_SETS;
+  // 40.8).  Up to four tokens of rank 256 whose parts, as many as there can be, are
+  // one round have them in equal numbers, of which each counts a quarter of a tile in
+  // the merge (us, in equal numbers of the tile walk before, shared without that, and
+  // so: 32 heads, 2 / 4 tokens of 4000 21.7 22.3, 22.8 24.8 and 19.4 20.3, of 8000 23.8
+  // 24.8, 25.7 28.1 and 24.7 25.7, of 600 19.8 19.8, 13.5 13.7 and 12.8 13.1); of rank
+  // 512 shared ones are ahead in a window and where lengths differ (4 tokens, 3000 and
+  // three of 30, 64 heads 24.6 and 26.2).
+  const bool one_round =
+      R == 256 && T <= 4 && T * groups * LD_PARTS <= cus;
+  const bool shared = T > 1 && T <= 64 * LD_SETS && !one_round;
   const int64_t shortest = T <= 4 ? 2 : 4;
   int64_t slots = 0, each = 0;
-  int64_t least = (T * groups + cus - 1) / cus * (tiles + 2);
+  int64_t least = (T * groups + cus - 1) / cus * (tiles + 2) * 4;
   for (int64_t n = 2; n <= std::min<int64_t>(LD_PARTS, tiles / shortest); ++n) {
     const int64_t rounds = (T * groups * n + cus - 1) / cus;
-    const int64_t cost = rounds * ((tiles + n - 1) / n + 2);
+    const int64_t cost = rounds * ((tiles + n - 1) / n + 2) * 4 +
+                         (one_round ? n : 0);
     if (cost < least) {
       least = cost;
       each = shared ? 0 : n;
