@@ -530,7 +530,10 @@ __global__ __launch_bounds__(64 * FT_WAVES, 2) void softcap_decode_kernel(
 // 16 keys, 49.7 and 38.2, all 94.5 and 83.6, of 2000 with a score cap 93.6 and 70.2,
 // 128 of 100 to 1000 77.2 and 57.3, 256 of 2048 356 and 336 (6.4 TB/s), 700 of 200
 // 178 and 112, one of 3000 15.5 and 13.3, 64 of 20 10.7 and 6.6; 32 on 4, the last
-// 512, 48 of 2000 21.0 and 19.2.  With 16 on 1, where a page's bytes are a 32nd of
+// 512, 48 of 2000 21.0 and 19.2.  Of 2700 mixes of 1 to 600 tokens of 20 to 4000 keys,
+// one to eight heads a key head, whole, windowed or in chunks, the tiles are ahead only
+// where few parts of 1000 keys are one round (16 of 1000, 40 on 8 20.4 and 21.6; 64 of
+// 1000, 16 on 2 21.2 and 22.4).  With 16 on 1, where a page's bytes are a 32nd of
 // a workgroup's, they are behind (48 of 2000 21.4 and 22.5).
 constexpr int SD_HD = 128, SD_BS = 16, SD_PAGE = SD_HD * SD_BS;
 
